@@ -1,0 +1,51 @@
+"""Verify steps and draft blocks: requests with more than 16 query columns per kv head (two column
+tiles per workgroup, several tiles per request) on the balanced plan, at the edges of halves, units,
+pieces and entry groups; against the oracle at the contract bound."""
+import numpy as np
+import pytest
+
+import oracle
+from oracle import DT_BF16, DT_F16, FMT_BF16, FMT_FP16, FMT_FP8, FMT_Q8_0, XF_IDENTITY, XF_WHT256
+from test_gpu_attention import _check
+
+pytestmark = pytest.mark.gpu
+
+SCRATCH = 64 << 20
+ROWS = [(FMT_BF16, DT_BF16), (FMT_FP16, DT_F16), (FMT_FP8, DT_F16), (FMT_Q8_0, DT_BF16)]
+
+
+@pytest.mark.parametrize("fmt,dtype", ROWS)
+@pytest.mark.parametrize("seq,q", [([4], [4]), ([16, 17, 33], [4, 3, 4]), ([700, 31, 2500, 48, 900], [4, 4, 3, 1, 2]),
+                                   ([5000, 64], [4, 4]), ([130, 900, 70], [9, 16, 5])])
+def test_rows_verify_column_tiles(fmt, dtype, seq, q):
+    """One to four tiles per request, pieces that end inside a unit, requests shorter than a half."""
+    _check(fmt, dtype, 16, seq, q, 411, scratch=SCRATCH, q_heads=16)
+
+
+@pytest.mark.parametrize("mask_mode", [0, 1])
+@pytest.mark.parametrize("seq,q", [([16], [16]), ([300, 41, 1000], [16, 16, 8]), ([2100, 90], [16, 9])])
+def test_rows_draft_blocks_head_dim_128(mask_mode, seq, q):
+    """Blocks of up to sixteen tokens at head dimension 128, causal and seeing each other both ways."""
+    _check(FMT_BF16, DT_BF16, 16, seq, q, 412, scratch=SCRATCH, q_heads=16, kv_heads=4, head_dim=128, mask_mode=mask_mode)
+
+
+@pytest.mark.parametrize("fmt,dtype", [(FMT_Q8_0, DT_F16), (FMT_BF16, DT_BF16)])
+@pytest.mark.parametrize("n", [17, 33, 70])
+def test_rows_verify_many_requests(fmt, dtype, n):
+    """More entries than are cut into pieces of their own, and more than one group of 64."""
+    seq = [20 + 37 * ((i * 7) % 11) for i in range(n)]
+    _check(fmt, dtype, 64, seq, [1 + (i % 6) for i in range(n)], 413, scratch=SCRATCH, q_heads=16)
+
+
+@pytest.mark.parametrize("scratch", [2 << 20, 8 << 20])
+def test_rows_verify_small_scratch(scratch):
+    """Fewer pieces where the scratch cannot hold the records of all of them, or the plain form."""
+    _check(FMT_FP8, DT_F16, 64, [3000, 900, 2000], [4, 4, 4], 414, scratch=scratch, q_heads=16)
+
+
+@pytest.mark.parametrize("fmt", [FMT_FP8, FMT_Q8_0])
+def test_rows_verify_rotated_keys_or_values(fmt):
+    """Rotated 8-bit rows: one column tile, several tiles per request; keys alone rotated: two."""
+    _check(fmt, DT_F16, 16, [300, 45, 800], [4, 2, 3], 415, scratch=SCRATCH, q_heads=16, xf=XF_WHT256, plain_excess=4e-4)
+    _check(fmt, DT_F16, 16, [300, 45, 800], [4, 2, 3], 416, scratch=SCRATCH, q_heads=16, xf=XF_WHT256, v_xf=XF_IDENTITY,
+           plain_excess=4e-4)

@@ -103,7 +103,12 @@ struct AttnParams {
     int rot_q;             // K rows are stored rotated (WHT-256 transform): rotate the query rows
     int rot_out;           // V rows are stored rotated: rotate the output back
     int32_t* bal_table;    // balanced decode: per query token {first partial slot, pieces, token of the tile, -}
+    int bal_tiles;         // balanced decode: tiles per request (a bound; the plan's entries are request x tile)
+    int bal_aligned;       // balanced decode: no piece boundary inside a workgroup's share (few entries)
+    int piece_cost;        // balanced decode: what starting a piece costs, in units
+    int bal_cols;          // columns of a partial slot: 16 x column tiles of the kernel
     uint32_t block_magic;  // floor(2^32 / block_size), see div_block
+    uint32_t q_group_magic;  // see div_q_group
     const uint16_t* gate;  // fp16 [tokens, q heads, 256] or null: out = fp16(out) * sigmoid(gate)
     // chunk geometry of a tile whose keys are exactly [0, max_seq_len): worked out on the host, so a
     // request that is as long as the host's bound needs no division on the device
@@ -158,14 +163,14 @@ __device__ __forceinline__ constexpr int unit_token(int s, int b, int i) {
 // one correction step makes it exact.  A runtime integer division costs ~40 dependent
 // instructions on this hardware, and the prologue and the per-unit address arithmetic
 // divide by block sizes and group sizes that only the descriptors know.
-__device__ __forceinline__ int fast_div(int a, int b) {
-    if (a >= (1 << 21)) return a / b;
+__device__ __forceinline__ int small_div(int a, int b) {  // a < 2^21
     int q = (int)((float)a * __builtin_amdgcn_rcpf((float)b));
     const int r = a - q * b;
     q += r >= b ? 1 : 0;
     q -= r < 0 ? 1 : 0;
     return q;
 }
+__device__ __forceinline__ int fast_div(int a, int b) { return a >= (1 << 21) ? a / b : small_div(a, b); }
 
 // pos / block_size for 0 <= pos < 2^31 without a branch: the high word of pos * floor(2^32 / b)
 // is the quotient or one less, one compare settles it.  The inner loops divide a token position
@@ -178,6 +183,13 @@ __device__ __forceinline__ int div_block(int pos, const AttnParams& P) {
 __host__ inline uint32_t block_magic_for(int block_size) {
     return block_size <= 1 ? 0xFFFFFFFFu : (uint32_t)((1ull << 32) / (uint32_t)block_size);
 }
+
+// column / q_group for the columns of a workgroup (at most 128, q_group at most 16): exact with
+// ceil(2^16 / q_group), whose excess over 2^16 / q_group adds less than 128 * 16 / 2^16 of a group
+__device__ __forceinline__ int div_q_group(int col, const AttnParams& P) {
+    return (int)(((uint32_t)col * P.q_group_magic) >> 16);
+}
+__host__ inline uint32_t q_group_magic_for(int q_group) { return (65536u + (uint32_t)q_group - 1u) / (uint32_t)q_group; }
 
 struct ChunkGeom {
     int u_first, n_units, upc, n_chunks;
@@ -257,6 +269,16 @@ __device__ __forceinline__ void split_h2(float a, float b, uint32_t& hi, uint32_
     asm("v_fma_mixhi_f16 %0, %1, 1.0, -%2 op_sel:[0,0,1] op_sel_hi:[0,0,1]" : "+v"(l) : "v"(b), "v"(hi));
     lo = l;
 }
+// An MFMA may read a register two wait states after a vector instruction has written it.  The compiler
+// keeps that distance for its own instructions but does not see through an assembly statement, so
+// the low-order operands pass through settle() on their way to the MFMAs.
+__device__ __forceinline__ void settle(u4& a, u4& b) { asm("s_nop 1" : "+v"(a), "+v"(b)); }
+__device__ __forceinline__ void settle(u4& a, u4& b, u4& c, u4& d) {
+    asm("s_nop 1" : "+v"(a), "+v"(b), "+v"(c), "+v"(d));
+}
+__device__ __forceinline__ void settle(u2v (&a)[8]) {
+    asm("s_nop 1" : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]), "+v"(a[4]), "+v"(a[5]), "+v"(a[6]), "+v"(a[7]));
+}
 // a * (fp16 half of w) as one mixed-precision FMA that reads the half in place (v_fma_mix_f32 with
 // a zero addend; written as an fma so that the compiler forms it and places the wait states that
 // separate it from the instruction that produced a).  A product of -0 comes out as +0.
@@ -328,65 +350,81 @@ constexpr int kMergeGroups = 16;
 constexpr int kMergeMaxPerGroup = 16;  // at most 256 partials per row
 
 // ---- balanced decode ----------------------------------------------------------------------------
-// A decode batch (at most one tile per request, no window, no token mask) is cut into equal
-// shares of 32-token units, one share per workgroup, whatever the lengths of the requests: the
-// units of all requests are laid end to end and workgroup x owns units [x S, (x + 1) S).  A share
-// that crosses a request boundary is worked off piece by piece.  Piece (x, r) gets partial slot
-// x + r: both grow along the pieces, so the slots are unique and those of one request are
-// consecutive, first_wg(r) + r .. last_wg(r) + r.  The workgroup that owns a request's first
-// piece records {first slot, number of pieces, token of the tile} for each of the request's
-// query tokens in a per-token table for the merge kernel; the tokens of requests without work
+// A decode or verify batch (no window, no token mask) is cut into equal shares of 32-token units,
+// one share per workgroup, whatever the lengths of the requests.  A request with more query tokens
+// than a tile holds has several tiles; entry e of the plan is tile e % T of request e / T, T =
+// P.bal_tiles (1 for a decode step; tiles a request does not have are entries without units).
+// The units of all entries are laid end to end and workgroup x owns units [x S, (x + 1) S).  A share
+// that crosses an entry boundary is worked off piece by piece.  Piece (x, e) gets partial slot
+// x + e: both grow along the pieces, so the slots are unique and those of one entry are
+// consecutive, first_wg(e) + e .. last_wg(e) + e.  The workgroup that owns an entry's first
+// piece records {first slot, number of pieces, token of the tile} for each of the tile's
+// query tokens in a per-token table for the merge kernel; the tokens of entries without work
 // are recorded by workgroup (0, 0): pieces = 0 for a live request without visible keys (output
 // zeros), -1 for a masked one and for tokens behind the last request (output untouched).
+// Few entries (P.bal_aligned): every entry is cut into equal pieces of its own, no workgroup has two
+// pieces.  The start of a piece is a chain of memory round trips and its end a merge of the waves,
+// together more than a workgroup's streaming when the batch is small, and the call lasts as long as
+// the workgroup that goes through it twice.  With n entries on G workgroups rounding to whole pieces
+// costs about n / 2G of the streaming, so for many entries the shares that cross boundaries are
+// better.  Slot of a piece: its workgroup.
 // Starting a piece (table, query rotation, first loads, merge of the waves) costs about as much
-// as kBalPieceCost units of streaming, so every request is charged that many extra units in
-// front of its real ones: a share that contains request boundaries gets fewer keys.
-constexpr int kBalPieceCost = 32;
-__host__ __device__ __forceinline__ size_t bal_partial_row(int slot, int kv_subs, int kv_sub, int col) {
-    return ((size_t)slot * kv_subs + kv_sub) * 16 + col;
+// as P.piece_cost units of streaming, so every entry is charged that many extra units in
+// front of its real ones: a share that contains entry boundaries gets fewer keys.
+__host__ __device__ __forceinline__ size_t bal_partial_row(int slot, int kv_subs, int kv_sub, int cols, int col) {
+    return ((size_t)slot * kv_subs + kv_sub) * cols + col;
 }
 
-struct BalReq {  // request base + lane of a 64-request group
-    int lo, hi, sa, cb, units;
-    int cost;  // units + kBalPieceCost, 0 for a request without work
+struct BalReq {  // entry base + lane of a group of 64
+    int lo, hi;          // query tokens of the request
+    int t_lo, t_hi;      // query tokens of the tile
+    int sa, cb, units;
+    int cost;  // units + P.piece_cost, 0 for an entry without work
     int live;  // has query tokens and is not masked
 };
-__device__ __forceinline__ BalReq bal_load_req(const AttnParams& P, int r) {
+__device__ __forceinline__ BalReq bal_load_req(const AttnParams& P, int e) {
     const warp34_attention_batch& B = P.B;
-    BalReq q{0, 0, 0, 0, 0, 0, 0};
+    BalReq q{0, 0, 0, 0, 0, 0, 0, 0, 0};
+    const int r = P.bal_tiles == 1 ? e : small_div(e, P.bal_tiles);
     if (r >= B.num_reqs) return q;
     q.lo = B.query_start_loc[r];
     q.hi = B.query_start_loc[r + 1];
     q.sa = B.seq_lens_after[r];
     const int q_len = q.hi - q.lo;
     q.cb = B.context_lens_before != nullptr ? B.context_lens_before[r] : q.sa - q_len;
-    const bool live = q_len > 0 && (B.valid_req_mask == nullptr || B.valid_req_mask[r] != 0);
-    int last = (B.mask_mode == WARP34_ATTN_MASK_NONCAUSAL_WINDOW) ? q.sa - 1 : q.cb + min(q_len, P.tok_tile) - 1;
+    const int first = (e - r * P.bal_tiles) * P.tok_tile;  // the tile's first token inside the request
+    q.t_lo = min(q.lo + first, max(q.lo, q.hi));
+    q.t_hi = min(q.lo + first + P.tok_tile, max(q.lo, q.hi));
+    const bool live = q.t_hi > q.t_lo && (B.valid_req_mask == nullptr || B.valid_req_mask[r] != 0);
+    int last = (B.mask_mode == WARP34_ATTN_MASK_NONCAUSAL_WINDOW) ? q.sa - 1 : q.cb + (q.t_hi - q.lo) - 1;
     if (last >= q.sa) last = q.sa - 1;
     q.units = (live && last >= 0) ? (last >> 5) + 1 : 0;
-    q.cost = q.units > 0 ? q.units + kBalPieceCost : 0;
+    q.cost = q.units > 0 ? q.units + P.piece_cost : 0;
     q.live = live ? 1 : 0;
     return q;
 }
-__device__ __forceinline__ int wave_incl_scan(int v, int lane) {
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-        const int up = __shfl_up(v, off, 64);
-        if (lane >= off) v += up;
-    }
+// inclusive prefix sum over the wave: four row shifts, then the totals of the rows before (DPP moves;
+// lanes without a source add 0)
+__device__ __forceinline__ int wave_incl_scan(int v) {
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, false);  // row_shr:1
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, false);  // row_shr:2
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, false);  // row_shr:4
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, false);  // row_shr:8
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xA, 0xF, false);  // row_bcast:15 into rows 1 and 3
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, false);  // row_bcast:31 into rows 2 and 3
     return v;
 }
 // units per share for a batch of `total` units over `groups` workgroups
 __device__ __forceinline__ int bal_share(int total, int groups, int min_share) {
-    int s = (total + groups - 1) / groups;
+    const int s = fast_div(total + groups - 1, groups);
     return s < min_share ? min_share : s;
 }
 
-// One piece of work of the balanced decode kernel: units [u_begin, u_end) of request `req`,
-// the piece number `slot` (partials of a request occupy consecutive slots) and the number of
-// pieces the request is cut into.
+// One piece of work of the balanced decode kernel: units [u_begin, u_end) of tile `tile` of request
+// `req`, the piece number `slot` (partials of a tile occupy consecutive slots) and the number of
+// pieces the tile is cut into.
 struct BalItem {
-    int req, rq_start, rq_end, seq_after, ctx_before;
+    int req, tile, rq_start, rq_end, seq_after, ctx_before;
     int u_begin, u_end, n_chunks, slot;
 };
 
@@ -528,7 +566,7 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
     // with a prefix sum over the requests' tile counts.
     const int tile_z = BAL ? item.req : (int)blockIdx.z;
     const int kv_sub = (int)blockIdx.y;
-    const int kv_head = fast_div(kv_sub, P.q_subgroups);
+    const int kv_head = small_div(kv_sub, P.q_subgroups);
     const int q_head_base = kv_head * P.gqa + (kv_sub - kv_head * P.q_subgroups) * P.q_group;
     const int chunk = BAL ? 0 : (int)blockIdx.x;
 
@@ -544,6 +582,7 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
         rq_end = item.rq_end;
         seq_after = item.seq_after;
         ctx_before = item.ctx_before;
+        tile_in_req = item.tile;
         req_hit = true;
         // the piece's first unit is known: its block-table slice is requested together with the
         // query rows
@@ -582,7 +621,7 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
     // While the request's lengths are on their way: the raw query rows of this wave's columns and
     // the table.  The first token of the tile is guessed (exact when every request has a whole
     // number of tiles); a wrong guess is corrected after the lookup.
-    const int tok_guess = BAL ? item.rq_start
+    const int tok_guess = BAL ? item.rq_start + item.tile * P.tok_tile
                               : min(P.tiles_by_request ? tile_z : tile_z * P.tok_tile, B.total_tokens - 1);
     constexpr int kColsPerWave = (16 + kWaves - 1) / kWaves;
     uint2 q_raw[kColsPerWave];
@@ -590,7 +629,7 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
 #pragma unroll
         for (int c = 0; c < kColsPerWave; ++c) {
             const int col = wave + c * kWaves;
-            const int t = fast_div(col, P.q_group);
+            const int t = div_q_group(col, P);
             const int a = col - t * P.q_group;
             q_raw[c] = uint2{0u, 0u};
             if (col < 16 && tokbase + t < B.total_tokens) {
@@ -604,7 +643,7 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
     // validity of the token of this lane's column
     bool tok_ok;
     auto load_tok_ok_col = [&](int tokbase, int column) {
-        const int tok = tokbase + fast_div(column, P.q_group);
+        const int tok = tokbase + div_q_group(column, P);
         tok_ok = tok < B.total_tokens &&
                  (B.valid_token_mask == nullptr || B.valid_token_mask[min(tok, B.total_tokens - 1)] != 0);
     };
@@ -670,7 +709,7 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
     int key_floor = 0;
     if constexpr (SP) key_floor = __builtin_amdgcn_readfirstlane(*P.key_floor);
     auto column_info = [&](bool accumulate) {
-        const int t = fast_div(ncol, P.q_group);
+        const int t = div_q_group(ncol, P);
         const int tok = tok0 + t;
         const bool ok = t < tile_tokens && tok_ok;
         const int q_off = tok - rq_start;
@@ -1136,6 +1175,7 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
                 hi[h][k] = ((wa >> 4) & 0x0F0F0F0Fu) | (wb & 0xF0F0F0F0u);
             }
         }
+        settle(ph[0], ph[1], pl[0], pl[1]);
         // four batches of four value tiles (16 table reads, eight MFMAs), pipelined like the QK batches
         u4 va[2][4];
         auto pv_reads = [&](int bt, u4 (&a)[4]) {
@@ -1309,12 +1349,12 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
             float v[4];
 #pragma unroll
             for (int k = 0; k < 4; ++k) v[k] = tbuf[merge_slot[k]];
-            const int t = fast_div(col, P.q_group);
+            const int t = div_q_group(col, P);
             const int a = col - t * P.q_group;
             const size_t row = (size_t)(tok0 + t) * P.num_q_heads + (size_t)(q_head_base + a);
             if (BAL ? item.n_chunks > 1 : P.max_chunks > 1) {
                 // un-normalised, rotated, still carrying the table gain; the merge kernel finishes
-                const size_t prow = BAL ? bal_partial_row(item.slot, (int)gridDim.y, kv_sub, col)
+                const size_t prow = BAL ? bal_partial_row(item.slot, (int)gridDim.y, kv_sub, 16, col)
                                         : row * (SP ? P.part_stride : P.max_chunks) + chunk;
                 float* dst = P.part_acc + prow * kHeadDim;
                 *reinterpret_cast<f4*>(dst + 4 * lane) = f4{v[0], v[1], v[2], v[3]};
@@ -1359,42 +1399,81 @@ __global__ __launch_bounds__(kTq4Waves * 64, 1) void paged_attn_tq4_kernel(const
 template <typename TileFn>
 __device__ __forceinline__ void bal_for_each_piece(const AttnParams& P, TileFn&& tile) {
     const int lane = (int)threadIdx.x & 63;
-    const int num_reqs = P.B.num_reqs;
-    // the first 64 requests are loaded once: their lane values serve the total and the search for
-    // the first piece (most workgroups have exactly one piece, most batches at most 64 requests)
+    const int entries = P.B.num_reqs * P.bal_tiles;
+    // the first 64 entries are loaded once: their lane values serve the total and the search for
+    // the first piece (most workgroups have exactly one piece, most batches at most 64 entries)
     const BalReq q0 = bal_load_req(P, lane);
-    const int incl0 = wave_incl_scan(q0.cost, lane);
+    const int incl0 = wave_incl_scan(q0.cost);
     int total = __builtin_amdgcn_readlane(incl0, 63);
-    // wave 0 of workgroup (0, 0) records the requests no workgroup will work on
+    // wave 0 of workgroup (0, 0) records the tokens no workgroup will work on
     const bool recorder = blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x < 64;
-    auto record_idle = [&](const BalReq& q, int r) {
-        if (!recorder || r >= num_reqs) return;
+    auto record_idle = [&](const BalReq& q, int e) {
+        if (!recorder || e >= entries) return;
         if (q.units == 0) {
-            for (int t = q.lo; t < q.hi && t < P.B.total_tokens; ++t)
-                *reinterpret_cast<int4*>(P.bal_table + 4 * (size_t)t) = int4{0, q.live ? 0 : -1, t - q.lo, 0};
+            for (int t = q.t_lo; t < q.t_hi && t < P.B.total_tokens; ++t)
+                *reinterpret_cast<int4*>(P.bal_table + 4 * (size_t)t) = int4{0, q.live ? 0 : -1, t - q.t_lo, 0};
         }
-        if (r == num_reqs - 1) {
+        if (e == entries - 1) {
             for (int t = max(q.hi, 0); t < P.B.total_tokens; ++t)
                 *reinterpret_cast<int4*>(P.bal_table + 4 * (size_t)t) = int4{0, -1, 0, 0};
         }
     };
     record_idle(q0, lane);
-    for (int base = 64; base < num_reqs; base += 64) {
+    for (int base = 64; base < entries; base += 64) {
         const BalReq q = bal_load_req(P, base + lane);
         record_idle(q, base + lane);
-        total += __builtin_amdgcn_readlane(wave_incl_scan(q.cost, lane), 63);
+        total += __builtin_amdgcn_readlane(wave_incl_scan(q.cost), 63);
     }
-    const int share = bal_share(total, (int)gridDim.x, P.min_upc + kBalPieceCost);
-    const int my_begin = (int)blockIdx.x * share;
-    int my_end = my_begin + share;
-    if (my_end > total) my_end = total;
-    if (my_begin >= total) return;
+    BalItem it{};
+    int my_begin = 0, my_end = 0, piece_end = 0;  // (aligned: the one piece ends the share)
+    int share = 1;
+    if (P.bal_aligned) {  // uniform for the grid; at most 64 entries
+        // Units per piece: the smallest count found by a few steps from below for which the pieces fit
+        // the grid.  (Every wave of the chip computes the same numbers.)
+        const int groups = (int)gridDim.x;
+        const int units = __builtin_amdgcn_readlane(wave_incl_scan(q0.units), 63);
+        int pieces, incl;
+        share = bal_share(units, groups, P.min_upc);
+        for (;;) {
+            pieces = q0.units > 0 ? fast_div(q0.units + share - 1, share) : 0;
+            incl = wave_incl_scan(pieces);
+            const int n = __builtin_amdgcn_readlane(incl, 63);
+            if (n <= groups) break;
+            share += fast_div(share * (n - groups), groups) + 1;
+        }
+        const unsigned long long hits = __ballot(pieces > 0 && (int)blockIdx.x < incl);
+        if (hits == 0ull) return;
+        const int src = __builtin_ctzll(hits);
+        const int n_pieces = __builtin_amdgcn_readlane(pieces, src);
+        const int first = __builtin_amdgcn_readlane(incl, src) - n_pieces;
+        const int e_units = __builtin_amdgcn_readlane(q0.units, src);
+        const int per_piece = fast_div(e_units + n_pieces - 1, n_pieces);
+        it.req = P.bal_tiles == 1 ? src : small_div(src, P.bal_tiles);
+        it.tile = src - it.req * P.bal_tiles;
+        it.rq_start = __builtin_amdgcn_readlane(q0.lo, src);
+        it.rq_end = __builtin_amdgcn_readlane(q0.hi, src);
+        it.seq_after = __builtin_amdgcn_readlane(q0.sa, src);
+        it.ctx_before = __builtin_amdgcn_readlane(q0.cb, src);
+        // (equal pieces; rounding up may leave the last ones without units, they still write a record)
+        it.u_begin = min(((int)blockIdx.x - first) * per_piece, e_units);
+        it.u_end = min(it.u_begin + per_piece, e_units);
+        it.n_chunks = n_pieces;
+        it.slot = (int)blockIdx.x;
+        const int tok = __builtin_amdgcn_readlane(q0.t_lo, src) + (int)threadIdx.x;
+        if ((int)blockIdx.x == first && blockIdx.y == 0 && tok < __builtin_amdgcn_readlane(q0.t_hi, src) &&
+            tok < P.B.total_tokens) {
+            *reinterpret_cast<int4*>(P.bal_table + 4 * (size_t)tok) = int4{first, n_pieces, (int)threadIdx.x, 0};
+        }
+    } else {
+        share = bal_share(total, (int)gridDim.x, P.min_upc + P.piece_cost);
+        my_begin = (int)blockIdx.x * share;
+        my_end = min(my_begin + share, total);
+        if (my_begin >= total) return;
+    }
 
     // The pieces of this share, in order.  Nothing but a few scalars stays live across a tile:
     // the 64-request group that holds the next piece is loaded and scanned again after each one.
     int base = 0, before = 0, taken = 0;  // group, units before it, pieces of it already done
-    BalItem it{};
-    int piece_end = 0;
     // next piece inside the group whose lane values are (q, incl); false: the group has none left
     auto scan_group = [&](const BalReq& q, int incl) -> bool {
         const int start = before + incl - q.units;  // of the real units, behind the charge
@@ -1409,32 +1488,34 @@ __device__ __forceinline__ void bal_for_each_piece(const AttnParams& P, TileFn&&
         const int src = __builtin_ctzll(hits);
         const int r_start = __builtin_amdgcn_readlane(start, src);
         const int r_units = __builtin_amdgcn_readlane(q.units, src);
-        it.req = base + src;
+        const int entry = base + src;
+        it.req = P.bal_tiles == 1 ? entry : small_div(entry, P.bal_tiles);
+        it.tile = entry - it.req * P.bal_tiles;
         it.rq_start = __builtin_amdgcn_readlane(q.lo, src);
         it.rq_end = __builtin_amdgcn_readlane(q.hi, src);
         it.seq_after = __builtin_amdgcn_readlane(q.sa, src);
         it.ctx_before = __builtin_amdgcn_readlane(q.cb, src);
         it.u_begin = max(my_begin, r_start) - r_start;
         it.u_end = min(my_end, r_start + r_units) - r_start;
-        it.n_chunks = (r_start + r_units - 1) / share - r_start / share + 1;
-        it.slot = (int)blockIdx.x + it.req;
+        it.n_chunks = fast_div(r_start + r_units - 1, share) - fast_div(r_start, share) + 1;
+        it.slot = (int)blockIdx.x + entry;
         piece_end = r_start + it.u_end;
-        if (it.u_begin == 0 && blockIdx.y == 0 && (int)threadIdx.x < it.rq_end - it.rq_start &&
-            it.rq_start + (int)threadIdx.x < P.B.total_tokens) {  // first piece: one entry per query token
-            *reinterpret_cast<int4*>(P.bal_table + 4 * (size_t)(it.rq_start + (int)threadIdx.x)) =
-                int4{it.slot, it.n_chunks, (int)threadIdx.x, 0};
+        const int tok = __builtin_amdgcn_readlane(q.t_lo, src) + (int)threadIdx.x;
+        if (it.u_begin == 0 && blockIdx.y == 0 && tok < __builtin_amdgcn_readlane(q.t_hi, src) &&
+            tok < P.B.total_tokens) {  // first piece: one entry per query token
+            *reinterpret_cast<int4*>(P.bal_table + 4 * (size_t)tok) = int4{it.slot, it.n_chunks, (int)threadIdx.x, 0};
         }
         ++taken;
         return true;
     };
     auto find_next = [&]() -> bool {
-        while (base < num_reqs && before < my_end) {
+        while (base < entries && before < my_end) {
             const BalReq q = bal_load_req(P, base + lane);
-            if (scan_group(q, wave_incl_scan(q.cost, lane))) return true;
+            if (scan_group(q, wave_incl_scan(q.cost))) return true;
         }
         return false;
     };
-    bool have = scan_group(q0, incl0);
+    bool have = P.bal_aligned || scan_group(q0, incl0);
     if (!have) have = find_next();
     while (have) {
         tile(it);
@@ -1455,42 +1536,48 @@ __global__ __launch_bounds__(kTq4Waves * 64, 1) void paged_attn_tq4_balanced_ker
     });
 }
 
-// Merge for the balanced decode kernel: one workgroup of 1024 threads per (token, q head) row.
-// The token's table entry says where its partials are; rows whose request was not cut (one
-// piece) were finished by the attention kernel, rows of live requests without visible keys are
-// zero, rows of masked requests stay untouched.
-template <typename TQ>
-__global__ __launch_bounds__(1024) void balanced_merge_kernel(const AttnParams P, int kv_subs, float out_scale,
-                                                              int rotate) {
-    __shared__ f4 s_acc[kMergeGroups][64];
-    __shared__ f4 s_rec[256];
-    __shared__ float s_red[kMergeGroups];
+// Merge for the balanced decode kernel: one workgroup of GROUPS waves per (token, q head) row; wave g
+// sums the partials g, g + GROUPS, ... and the first wave adds up the waves.  The token's table entry
+// says where the partials are; rows whose tile was not cut (one piece) were finished by the attention
+// kernel, rows of live requests without visible keys are zero, rows of masked requests stay untouched.
+// GROUPS: see merge_small_groups.
+template <typename TQ, int HD, int GROUPS>
+__global__ __launch_bounds__(GROUPS * 64) void balanced_merge_kernel(const AttnParams P, int kv_subs, float out_scale,
+                                                                     int rotate) {
+    constexpr int kSlots = kMergeGroups * kMergeMaxPerGroup;  // partials of a row at most
+    static_assert(GROUPS * 64 >= kSlots, "one record per thread");
+    __shared__ f4 s_acc[GROUPS][64];
+    __shared__ f4 s_rec[kSlots];
+    __shared__ float s_red[GROUPS];
     const int tid = (int)threadIdx.x;
     const int lane = tid & 63;
-    const int grp = tid >> 6;
-    const long long row = (long long)blockIdx.x;
-    const int tok = (int)(row / P.num_q_heads);
-    const int head = (int)(row - (long long)tok * P.num_q_heads);
+    const int grp = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int head = (int)blockIdx.x, tok = (int)blockIdx.y;
+    const size_t row = (size_t)tok * P.num_q_heads + head;
     const int4 entry = *reinterpret_cast<const int4*>(P.bal_table + 4 * (size_t)tok);  // same address in every lane
-    const int n_chunks = entry.y;
+    const int n_chunks = __builtin_amdgcn_readfirstlane(entry.y);
     if (n_chunks < 0 || n_chunks == 1) return;  // masked, or finished by the attention kernel
     if (n_chunks == 0) {                        // no visible key: zeros
         const float zero[4] = {0.f, 0.f, 0.f, 0.f};
-        if (grp == 0) store_out_row<TQ>(P, (size_t)row, lane, zero);
+        if (grp == 0) store_out_row<TQ, HD>(P, row, lane, zero);
         return;
     }
-    const int col = entry.z * P.q_group + head % P.q_group;
-    const int kv_sub = head / P.q_group;  // = kv_head * q_subgroups + subgroup
-    const size_t prow0 = bal_partial_row(entry.x, kv_subs, kv_sub, col);
-    const size_t pstride = (size_t)kv_subs * 16;  // partial rows between consecutive slots
-    if (tid < n_chunks && tid < 256) s_rec[tid] = *reinterpret_cast<const f4*>(P.part_ml + (prow0 + tid * pstride) * 4);
+    const int kv_sub = small_div(head, P.q_group);  // = kv_head * q_subgroups + subgroup
+    const int col = entry.z * P.q_group + (head - kv_sub * P.q_group);
+    const size_t prow0 = bal_partial_row(entry.x, kv_subs, kv_sub, P.bal_cols, col);
+    const size_t pstride = (size_t)kv_subs * P.bal_cols;  // partial rows between consecutive slots
+    if (tid < n_chunks && tid < kSlots) s_rec[tid] = *reinterpret_cast<const f4*>(P.part_ml + (prow0 + tid * pstride) * 4);
     f4 a[kMergeMaxPerGroup];
+    auto load_slices = [&](int first) {
 #pragma unroll
-    for (int k = 0; k < kMergeMaxPerGroup; ++k) {
-        const int s = grp + k * kMergeGroups;
-        a[k] = f4{0.f, 0.f, 0.f, 0.f};
-        if (s < n_chunks) a[k] = *reinterpret_cast<const f4*>(P.part_acc + (prow0 + s * pstride) * kHeadDim + 4 * lane);
-    }
+        for (int k = 0; k < kMergeMaxPerGroup; ++k) {
+            const int s = first + grp + k * GROUPS;
+            a[k] = f4{0.f, 0.f, 0.f, 0.f};
+            if (s < n_chunks && (HD == 256 || 4 * lane < HD))
+                a[k] = *reinterpret_cast<const f4*>(P.part_acc + (prow0 + s * pstride) * kHeadDim + 4 * lane);
+        }
+    };
+    load_slices(0);
     __syncthreads();
     float m_tot = kNegBig;
     for (int s = lane; s < n_chunks; s += 64) {
@@ -1505,17 +1592,22 @@ __global__ __launch_bounds__(1024) void balanced_merge_kernel(const AttnParams P
     m_tot = fmaxf(m_tot, lane_xor<32>(m_tot, lane));
     f4 v = {0.f, 0.f, 0.f, 0.f};
     float l_part = 0.f;
+    for (int first = 0;;) {
 #pragma unroll
-    for (int k = 0; k < kMergeMaxPerGroup; ++k) {
-        const int s = grp + k * kMergeGroups;
-        if (s < n_chunks) {
-            const f4 r = s_rec[s];
-            if (r[1] > 0.f) {
-                const float w = __builtin_amdgcn_exp2f(r[0] - m_tot);
-                l_part += r[1] * w;
-                v += a[k] * w;
+        for (int k = 0; k < kMergeMaxPerGroup; ++k) {
+            const int s = first + grp + k * GROUPS;
+            if (s < n_chunks) {
+                const f4 r = s_rec[s];
+                if (r[1] > 0.f) {
+                    const float w = __builtin_amdgcn_exp2f(r[0] - m_tot);
+                    l_part += r[1] * w;
+                    v += a[k] * w;
+                }
             }
         }
+        first += kMergeMaxPerGroup * GROUPS;
+        if (GROUPS == kMergeGroups || first >= n_chunks) break;
+        load_slices(first);
     }
     s_acc[grp][lane] = v;
     if (lane == 0) s_red[grp] = l_part;
@@ -1524,7 +1616,7 @@ __global__ __launch_bounds__(1024) void balanced_merge_kernel(const AttnParams P
     float l_tot = 0.f;
     f4 tot = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int k = 0; k < kMergeGroups; ++k) {
+    for (int k = 0; k < GROUPS; ++k) {
         tot += s_acc[k][lane];
         l_tot += s_red[k];
     }
@@ -1535,48 +1627,53 @@ __global__ __launch_bounds__(1024) void balanced_merge_kernel(const AttnParams P
 #pragma unroll
         for (int k = 0; k < 4; ++k) o[k] = apply_sign(o[k], 4 * lane + k);
     }
-    store_out_row<TQ>(P, (size_t)row, lane, o);
+    store_out_row<TQ, HD>(P, row, lane, o);
 }
 
 // Merge of the split-K partials (op_paged_attn.cu:1132-1218): m_tot = max m_s,
 // w_s = 2^(m_s - m_tot), out = sum acc_s w_s / sum l_s w_s, then one inverse rotation.
-// One workgroup of 1024 threads per (token, q head) row: 16 groups of 64 threads stride the
-// chunks, each thread owns 4 of the 256 columns; the groups are summed through LDS.
+// One workgroup of GROUPS waves per (token, q head) row: the waves stride the chunks, each thread
+// owns 4 of the 256 columns; the waves are summed through LDS.
 // Everything the row needs (validity, chunk records, accumulators) is requested in ONE memory
-// round trip: records and accumulators of all max_chunks slots are loaded speculatively and
-// the slots beyond the row's chunk count are discarded with selects.
-template <typename TQ, bool SP = false, int HD = kHeadDim>
-__global__ __launch_bounds__(1024) void split_merge_kernel(const float* part_acc_in, const float* part_ml_in,
-                                                           int max_chunks_in, const AttnParams P,
-                                                           float out_scale, int rotate) {
-    __shared__ f4 s_acc[kMergeGroups][64];
-    __shared__ f4 s_rec[256];
-    __shared__ float s_red[kMergeGroups];
+// round trip: records and accumulators of all max_chunks slots (the first 16 GROUPS of them) are
+// loaded speculatively and the slots beyond the row's chunk count are discarded with selects.
+template <typename TQ, bool SP, int HD, int GROUPS>
+__global__ __launch_bounds__(GROUPS * 64) void split_merge_kernel(const float* part_acc_in, const float* part_ml_in,
+                                                                  int max_chunks_in, int num_q_heads_in, const AttnParams P,
+                                                                  float out_scale, int rotate) {
+    constexpr int kSlots = kMergeGroups * kMergeMaxPerGroup;
+    static_assert(GROUPS * 64 >= kSlots, "one record per thread");
+    __shared__ f4 s_acc[GROUPS][64];
+    __shared__ f4 s_rec[kSlots];
+    __shared__ float s_red[GROUPS];
     __shared__ int s_valid;
     const int tid = (int)threadIdx.x;
     const int lane = tid & 63;
-    const int grp = tid >> 6;
-    const long long row = (long long)blockIdx.x;
-    const int tok = (int)(row / P.num_q_heads);
+    const int grp = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int tok = (int)blockIdx.y;
     const warp34_attention_batch& B = P.B;
-    // the leading arguments repeat P.part_acc / P.part_ml / P.max_chunks: they are preloaded into
-    // scalar registers at wave launch, so the speculative loads below do not wait for the
-    // kernel-argument fetch
-    const float* ml = part_ml_in + (size_t)row * max_chunks_in * 4;
-    const float* acc = part_acc_in + (size_t)row * max_chunks_in * kHeadDim;
+    // the leading arguments repeat P.part_acc / P.part_ml / P.max_chunks / P.num_q_heads: they are
+    // preloaded into scalar registers at wave launch, so the speculative loads below do not wait for
+    // the kernel-argument fetch
+    const size_t row = (size_t)tok * num_q_heads_in + blockIdx.x;
+    const float* ml = part_ml_in + row * max_chunks_in * 4;
+    const float* acc = part_acc_in + row * max_chunks_in * kHeadDim;
 
     // speculative loads: chunk records (one per thread) and this thread's accumulator slices
     f4 rec = {kNegBig, 0.f, 0.f, 0.f};
     if (tid < max_chunks_in) rec = *reinterpret_cast<const f4*>(ml + 4 * tid);
     f4 a[kMergeMaxPerGroup];
+    auto load_slices = [&](int first) {
 #pragma unroll
-    for (int k = 0; k < kMergeMaxPerGroup; ++k) {
-        const int s = grp + k * kMergeGroups;
-        a[k] = f4{0.f, 0.f, 0.f, 0.f};
-        // (records keep a 256-float stride at every head dimension; lanes beyond the row load nothing)
-        if (s < max_chunks_in && (HD == 256 || 4 * lane < HD))
-            a[k] = *reinterpret_cast<const f4*>(acc + (size_t)s * kHeadDim + 4 * lane);
-    }
+        for (int k = 0; k < kMergeMaxPerGroup; ++k) {
+            const int s = first + grp + k * GROUPS;
+            a[k] = f4{0.f, 0.f, 0.f, 0.f};
+            // (records keep a 256-float stride at every head dimension; lanes beyond the row load nothing)
+            if (s < max_chunks_in && (HD == 256 || 4 * lane < HD))
+                a[k] = *reinterpret_cast<const f4*>(acc + (size_t)s * kHeadDim + 4 * lane);
+        }
+    };
+    load_slices(0);
     // row validity (wave 0): token mask and owning request, first match wins
     if (grp == 0) {
         bool ok = B.valid_token_mask == nullptr || B.valid_token_mask[tok] != 0;
@@ -1595,7 +1692,7 @@ __global__ __launch_bounds__(1024) void split_merge_kernel(const float* part_acc
         }
         if (lane == 0) s_valid = (ok && found) ? 1 : 0;
     }
-    if (tid < 256) s_rec[tid] = rec;
+    if (tid < kSlots) s_rec[tid] = rec;
     __syncthreads();
     if (!s_valid) return;  // masked row: output untouched (uniform for the block)
     int n_chunks = (int)s_rec[0][2];
@@ -1605,7 +1702,7 @@ __global__ __launch_bounds__(1024) void split_merge_kernel(const float* part_acc
         if constexpr (SP) return s < n_chunks || (s >= P.pf_slot_base && s < P.pf_slot_base + P.pf_split);
         return s < n_chunks;
     };
-    const int n_slots = SP ? max_chunks_in : n_chunks;
+    const int n_slots = __builtin_amdgcn_readfirstlane(SP ? max_chunks_in : n_chunks);
 
     // global maximum of m over chunks with l > 0 (every thread scans the LDS copy)
     float m_tot = kNegBig;
@@ -1623,17 +1720,22 @@ __global__ __launch_bounds__(1024) void split_merge_kernel(const float* part_acc
 
     f4 v = {0.f, 0.f, 0.f, 0.f};
     float l_part = 0.f;
+    for (int first = 0;;) {
 #pragma unroll
-    for (int k = 0; k < kMergeMaxPerGroup; ++k) {
-        const int s = grp + k * kMergeGroups;
-        if (s < n_slots && live_slot(s)) {
-            const f4 r = s_rec[s];
-            if (r[1] > 0.f) {
-                const float w = __builtin_amdgcn_exp2f(r[0] - m_tot);
-                l_part += r[1] * w;
-                v += a[k] * w;
+        for (int k = 0; k < kMergeMaxPerGroup; ++k) {
+            const int s = first + grp + k * GROUPS;
+            if (s < n_slots && live_slot(s)) {
+                const f4 r = s_rec[s];
+                if (r[1] > 0.f) {
+                    const float w = __builtin_amdgcn_exp2f(r[0] - m_tot);
+                    l_part += r[1] * w;
+                    v += a[k] * w;
+                }
             }
         }
+        first += kMergeMaxPerGroup * GROUPS;
+        if (GROUPS == kMergeGroups || first >= n_slots) break;
+        load_slices(first);
     }
     s_acc[grp][lane] = v;
     if (lane == 0) s_red[grp] = l_part;
@@ -1642,7 +1744,7 @@ __global__ __launch_bounds__(1024) void split_merge_kernel(const float* part_acc
     float l_tot = 0.f;
     f4 tot = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int k = 0; k < kMergeGroups; ++k) {
+    for (int k = 0; k < GROUPS; ++k) {
         tot += s_acc[k][lane];
         l_tot += s_red[k];
     }
@@ -1653,7 +1755,7 @@ __global__ __launch_bounds__(1024) void split_merge_kernel(const float* part_acc
 #pragma unroll
         for (int k = 0; k < 4; ++k) o[k] = apply_sign(o[k], 4 * lane + k);
     }
-    store_out_row<TQ, HD>(P, (size_t)row, lane, o);
+    store_out_row<TQ, HD>(P, row, lane, o);
 }
 
 }  // namespace w34
@@ -1669,6 +1771,13 @@ namespace w34 {
 constexpr int kMaxChunksCap = 256;
 // 256 tokens, one unit per wave: 7 to 12 % faster than 16 at 16K-32K keys, same as 4
 constexpr int kMinUnitsPerChunk = 8;
+// Cost of starting a piece of a balanced batch, in units of streaming: TQ4 builds its table and
+// rotates the queries first.
+constexpr int kTq4PieceCost = 32;
+constexpr int kRowsPieceCost = 16;
+// Pieces of more than one column tile leave more records and longer merges: four draft blocks of sixteen
+// tokens (head dimension 128, four kv heads) 25.5 us with pieces from 10 units on, 20.7 from 16, 24.2 from 24.
+constexpr int kMinUnitsPerWidePiece = 16;
 // Split geometry is sized for the layout the path is built for, two kv heads per device: 128
 // chunks (or shares) per kv head.  The counts below depend on the batch and on gqa only, never
 // on local_kv_heads: a rank that holds one kv head of a sharded model computes every row with
@@ -1743,13 +1852,52 @@ static int ensure_dynamic_lds(KernelT kernel, int bytes, bool lds_base_zero = fa
 static bool balanced_decode_applicable(const warp34_exec* ex, const warp34_attention_batch* batch,
                                        int tiles_by_request, int force_single) {
     return tiles_by_request && batch->num_reqs >= 2 && !force_single && batch->sliding_window <= 0 &&
-           batch->valid_token_mask == nullptr && ex->scratch_ptr != 0 && (ex->scratch_ptr & 15u) == 0u;
+           batch->valid_token_mask == nullptr && batch->total_tokens <= 65535 && ex->scratch_ptr != 0 && (ex->scratch_ptr & 15u) == 0u;
 }
 // shares of a balanced decode batch per (kv head, q subgroup): a function of gqa only
 static int balanced_groups(int q_subgroups) {
     int groups = kTargetWorkgroupsPerHead / (q_subgroups > 0 ? q_subgroups : 1);
     if (groups > kMergeGroups * kMergeMaxPerGroup - 1) groups = kMergeGroups * kMergeMaxPerGroup - 1;
     return groups < 1 ? 1 : groups;
+}
+
+// Entries that are cut into pieces of their own, see the plan.  Up to one entry per eight workgroups:
+// five requests of 3K to 21K keys (10 entries on 128) 29.7 -> 28.7 us; 32 requests of 1K to 64K keys
+// 136 -> 149 us, they keep the shares that cross boundaries.
+static int balanced_aligned(long long entries, int groups) {
+    return entries <= 64 && entries * 8 <= groups ? 1 : 0;
+}
+
+// The second launch of a split batch: one workgroup per row.  Sixteen waves per row have all partials of
+// a long sequence in flight at once; from 32 rows per kv head on the workgroups are many and the
+// partials of a row few, and four waves per row start sooner (two kv heads, 80 rows of 25 partials: 6.9 ->
+// 5.2 us; 512 rows: 8.9 -> 5.8; four kv heads, 1 024 rows of ten: 11.5 -> 4.9; but 16 rows of 128
+// partials: 5.2 -> 6.8).  Rows per kv head, not rows: a rank with one kv head adds in the same order.
+static bool merge_small_groups(const AttnParams& P) { return (long long)P.B.total_tokens * P.gqa >= 32; }
+
+template <typename TQ, int HD>
+static int launch_balanced_merge(const AttnParams& P, int kv_subs, float out_scale, hipStream_t stream) {
+    const dim3 grid((unsigned)P.num_q_heads, (unsigned)P.B.total_tokens);
+    if (merge_small_groups(P)) {
+        hipLaunchKernelGGL((balanced_merge_kernel<TQ, HD, 4>), grid, dim3(4 * 64), 0, stream, P, kv_subs, out_scale, P.rot_out);
+    } else {
+        hipLaunchKernelGGL((balanced_merge_kernel<TQ, HD, kMergeGroups>), grid, dim3(kMergeGroups * 64), 0, stream, P, kv_subs,
+                           out_scale, P.rot_out);
+    }
+    return (int)hipGetLastError();
+}
+
+template <typename TQ, bool SP, int HD>
+static int launch_split_merge(const AttnParams& P, int slots, float out_scale, hipStream_t stream) {
+    const dim3 grid((unsigned)P.num_q_heads, (unsigned)P.B.total_tokens);
+    if (merge_small_groups(P)) {
+        hipLaunchKernelGGL((split_merge_kernel<TQ, SP, HD, 4>), grid, dim3(4 * 64), 0, stream, (const float*)P.part_acc,
+                           (const float*)P.part_ml, slots, P.num_q_heads, P, out_scale, P.rot_out);
+    } else {
+        hipLaunchKernelGGL((split_merge_kernel<TQ, SP, HD, kMergeGroups>), grid, dim3(kMergeGroups * 64), 0, stream,
+                           (const float*)P.part_acc, (const float*)P.part_ml, slots, P.num_q_heads, P, out_scale, P.rot_out);
+    }
+    return (int)hipGetLastError();
 }
 
 // P.spec_* = chunk_geom(0, max_seq_len - 1, P.max_chunks, P.min_upc), worked out on the host
@@ -1874,6 +2022,7 @@ static int launch_tq4(const warp34_exec* ex, const warp34_kv_layer_layout* layou
             }
     }
     P.q_group = q_group;
+    P.q_group_magic = q_group_magic_for(q_group);
     P.q_subgroups = P.gqa / q_group;
     // One N tile (16 query columns) per workgroup, also for verify batches: the two-tile variant
     // (4 waves, 32 columns) halves the key reads but runs at half the occupancy and measured
@@ -1957,31 +2106,30 @@ static int launch_tq4(const warp34_exec* ex, const warp34_kv_layer_layout* layou
                                stream, P);
             rc = (int)hipGetLastError();
             if (rc) return rc;
-            hipLaunchKernelGGL((split_merge_kernel<TQ, true>), dim3((unsigned)rows), dim3(1024), 0, stream,
-                               (const float*)P.part_acc, (const float*)P.part_ml, stride, P, kLutInvGain, P.rot_out);
-            return (int)hipGetLastError();
+            return launch_split_merge<TQ, true, kHeadDim>(P, stride, kLutInvGain, stream);
         }
     }
     // Decode batches of several requests: equal shares of the batch's units per workgroup
     // instead of per-request chunks (the requests' lengths are unknown to the host and differ).
     if (balanced_decode_applicable(ex, batch, P.tiles_by_request, force_single)) {
         const int groups = balanced_groups(P.q_subgroups);
-        const size_t prows = bal_partial_row(groups + batch->num_reqs, kv_subs, 0, 0);
+        const size_t prows = bal_partial_row(groups + batch->num_reqs, kv_subs, 0, 16, 0);
         if (partial_bytes((long long)prows, 1) + (size_t)batch->total_tokens * 16 <= ex->scratch_size) {
             P.part_acc = reinterpret_cast<float*>((uintptr_t)ex->scratch_ptr);
             P.part_ml = P.part_acc + prows * kHeadDim;
             P.bal_table = reinterpret_cast<int32_t*>(P.part_ml + prows * 4);
             P.max_chunks = groups + 1;
+            P.bal_tiles = 1;
+            P.bal_cols = 16;
+            P.piece_cost = kTq4PieceCost;
+            P.bal_aligned = balanced_aligned(batch->num_reqs, groups);
             rc = ensure_dynamic_lds(paged_attn_tq4_balanced_kernel<TQ>, smem_bytes_for(1), true);
             if (rc) return rc;
             hipLaunchKernelGGL((paged_attn_tq4_balanced_kernel<TQ>), dim3((unsigned)groups, (unsigned)kv_subs),
                                dim3(waves_for(1) * 64), smem_bytes_for(1), stream, P);
             rc = (int)hipGetLastError();
             if (rc) return rc;
-            hipLaunchKernelGGL((balanced_merge_kernel<TQ>),
-                               dim3((unsigned)rows), dim3(1024), 0, stream, P,
-                               kv_subs, kLutInvGain, P.rot_out);
-            return (int)hipGetLastError();
+            return launch_balanced_merge<TQ, kHeadDim>(P, kv_subs, kLutInvGain, stream);
         }
     }
     rc = ensure_dynamic_lds(paged_attn_tq4_kernel<TQ, 1>, smem_bytes_for(1), true);
@@ -1989,12 +2137,73 @@ static int launch_tq4(const warp34_exec* ex, const warp34_kv_layer_layout* layou
     hipLaunchKernelGGL((paged_attn_tq4_kernel<TQ, 1>), grid, dim3(waves_for(1) * 64), smem_bytes_for(1), stream, P);
     rc = (int)hipGetLastError();
     if (rc) return rc;
-    if (P.max_chunks > 1) {
-        hipLaunchKernelGGL((split_merge_kernel<TQ>), dim3((unsigned)rows), dim3(1024), 0, stream,
-                           (const float*)P.part_acc, (const float*)P.part_ml, P.max_chunks, P, kLutInvGain, P.rot_out);
+    return P.max_chunks > 1 ? launch_split_merge<TQ, false, kHeadDim>(P, P.max_chunks, kLutInvGain, stream) : 0;
+}
+
+// Most tiles per request that the balanced plan takes: with more, the 128-row tile kernel or one
+// workgroup per tile is the better shape.
+constexpr int kBalMaxTiles = 16;
+// Column tiles per workgroup (nt) and tiles per request of a balanced batch whose requests have up to
+// q_len query tokens: as many column tiles as a request's query columns fill, up to max_nt.
+struct BalShape {
+    int nt, tok_tile, tiles;
+};
+static BalShape balanced_shape(int q_len, int q_group, int max_nt) {
+    const long long cols = (long long)q_len * q_group;
+    BalShape s;
+    s.nt = cols > 16 && max_nt >= 2 ? 2 : 1;
+    s.tok_tile = 16 * s.nt / q_group;
+    s.tiles = (q_len + s.tok_tile - 1) / s.tok_tile;
+    return s;
+}
+
+// Balanced decode / verify over row-format pages; -1: the batch is not for it.
+// Two column tiles where a request has more than 16 query columns; rotated 8-bit values (a second value
+// operand) stay with one (accumulator registers).
+template <typename TQ, int KVF, bool VRES, int HD>
+static int launch_rows_balanced(const warp34_exec* ex, const warp34_attention_batch* batch, AttnParams P, int kv_subs,
+                                int force_single, hipStream_t stream) {
+    if (force_single || batch->max_q_len <= 0 || batch->sliding_window > 0 || batch->valid_token_mask != nullptr ||
+        ex->scratch_ptr == 0 || (ex->scratch_ptr & 15u) != 0u || batch->total_tokens > 65535)
+        return -1;
+    const BalShape shape = balanced_shape(batch->max_q_len, P.q_group, VRES ? 1 : 2);
+    const int nt = shape.nt, tiles = shape.tiles;
+    P.tok_tile = shape.tok_tile;
+    if (tiles > kBalMaxTiles || (batch->num_reqs == 1 && nt == 1 && tiles == 1)) return -1;
+    // fewer shares where the scratch cannot hold the records of all of them
+    const long long entries = (long long)batch->num_reqs * tiles;
+    const size_t slot_bytes = partial_bytes((long long)kv_subs * 16 * nt, 1), table_bytes = (size_t)batch->total_tokens * 16;
+    if (ex->scratch_size < table_bytes) return -1;
+    const long long room = (long long)((ex->scratch_size - table_bytes) / slot_bytes) - entries;
+    const int groups = (int)(room < balanced_groups(P.q_subgroups) ? room : balanced_groups(P.q_subgroups));
+    if (groups < 16) return -1;
+    const size_t prows = (size_t)(groups + entries) * kv_subs * 16 * nt;
+    P.piece_cost = kRowsPieceCost;
+    if (nt * tiles > 1) P.min_upc = kMinUnitsPerWidePiece;
+    P.part_acc = reinterpret_cast<float*>((uintptr_t)ex->scratch_ptr);
+    P.part_ml = P.part_acc + prows * kHeadDim;
+    P.bal_table = reinterpret_cast<int32_t*>(P.part_ml + prows * 4);
+    P.max_chunks = groups + 1;
+    P.bal_tiles = tiles;
+    P.bal_cols = 16 * nt;
+    P.bal_aligned = balanced_aligned(entries, groups);
+    const auto launch = [&](auto column_tiles) -> int {
+        constexpr int NT = decltype(column_tiles)::value;
+        constexpr int smem = rows_smem_bytes<KVF, HD>(NT);
+        // every key is read by one workgroup only when no request has two tiles: streaming loads
+        const auto kernel = tiles == 1 && P.q_subgroups == 1 ? paged_attn_rows_balanced_kernel<TQ, NT, KVF, VRES, true, HD>
+                                                             : paged_attn_rows_balanced_kernel<TQ, NT, KVF, VRES, false, HD>;
+        int rc = ensure_dynamic_lds(kernel, smem, true);
+        if (rc) return rc;
+        hipLaunchKernelGGL(kernel, dim3((unsigned)groups, (unsigned)kv_subs), dim3(kKv16Waves * 64), smem, stream, P);
         rc = (int)hipGetLastError();
+        if (rc) return rc;
+        return launch_balanced_merge<TQ, HD>(P, kv_subs, 1.0f, stream);
+    };
+    if constexpr (!VRES) {
+        if (nt == 2) return launch(std::integral_constant<int, 2>{});
     }
-    return rc;
+    return launch(std::integral_constant<int, 1>{});
 }
 
 // VRES: value rows stored rotated in an 8-bit format (residual operand, see rows_tile)
@@ -2020,6 +2229,7 @@ static int launch_rows(const warp34_exec* ex, const warp34_kv_layer_layout* layo
             }
     }
     P.q_group = q_group;
+    P.q_group_magic = q_group_magic_for(q_group);
     P.q_subgroups = P.gqa / q_group;
     P.tok_tile = 16 / q_group;  // one N tile
     if (P.tok_tile < 1) P.tok_tile = 1;
@@ -2054,37 +2264,15 @@ static int launch_rows(const warp34_exec* ex, const warp34_kv_layer_layout* layo
     const dim3 grid((unsigned)grid_x, (unsigned)kv_subs, (unsigned)grid_z);
     hipStream_t stream = (hipStream_t)ex->stream;
     int rc;
-    if (HD == kHeadDim && balanced_decode_applicable(ex, batch, P.tiles_by_request, force_single)) {
-        const int groups = balanced_groups(P.q_subgroups);
-        const size_t prows = bal_partial_row(groups + batch->num_reqs, kv_subs, 0, 0);
-        if (partial_bytes((long long)prows, 1) + (size_t)batch->total_tokens * 16 <= ex->scratch_size) {
-            P.part_acc = reinterpret_cast<float*>((uintptr_t)ex->scratch_ptr);
-            P.part_ml = P.part_acc + prows * kHeadDim;
-            P.bal_table = reinterpret_cast<int32_t*>(P.part_ml + prows * 4);
-            P.max_chunks = groups + 1;
-            rc = ensure_dynamic_lds(paged_attn_rows_balanced_kernel<TQ, KVF, VRES>, kv16_smem_bytes(1));
-            if (rc) return rc;
-            hipLaunchKernelGGL((paged_attn_rows_balanced_kernel<TQ, KVF, VRES>), dim3((unsigned)groups, (unsigned)kv_subs),
-                               dim3(kKv16Waves * 64), kv16_smem_bytes(1), stream, P);
-            rc = (int)hipGetLastError();
-            if (rc) return rc;
-            hipLaunchKernelGGL((balanced_merge_kernel<TQ>),
-                               dim3((unsigned)rows), dim3(1024), 0, stream, P,
-                               kv_subs, 1.0f, P.rot_out);
-            return (int)hipGetLastError();
-        }
-    }
-    rc = ensure_dynamic_lds(paged_attn_rows_kernel<TQ, 1, KVF, VRES, HD>, kv16_smem_bytes(1));
+    rc = launch_rows_balanced<TQ, KVF, VRES, HD>(ex, batch, P, kv_subs, force_single, stream);
+    if (rc >= 0) return rc;
+    constexpr int smem = rows_smem_bytes<KVF, HD>(1);
+    rc = ensure_dynamic_lds(paged_attn_rows_kernel<TQ, KVF, VRES, HD>, smem, true);
     if (rc) return rc;
-    hipLaunchKernelGGL((paged_attn_rows_kernel<TQ, 1, KVF, VRES, HD>), grid, dim3(kKv16Waves * 64), kv16_smem_bytes(1), stream, P);
+    hipLaunchKernelGGL((paged_attn_rows_kernel<TQ, KVF, VRES, HD>), grid, dim3(kKv16Waves * 64), smem, stream, P);
     rc = (int)hipGetLastError();
     if (rc) return rc;
-    if (P.max_chunks > 1) {
-        hipLaunchKernelGGL((split_merge_kernel<TQ, false, HD>), dim3((unsigned)rows), dim3(1024), 0, stream,
-                           (const float*)P.part_acc, (const float*)P.part_ml, P.max_chunks, P, 1.0f, P.rot_out);
-        rc = (int)hipGetLastError();
-    }
-    return rc;
+    return P.max_chunks > 1 ? launch_split_merge<TQ, false, HD>(P, P.max_chunks, 1.0f, stream) : 0;
 }
 
 // Chunked prefill over TQ4 pages: one workgroup per (128-row query tile, kv head x q subgroup,
@@ -2127,6 +2315,7 @@ static int launch_prefill_tq4(const warp34_exec* ex, const warp34_kv_layer_layou
             }
     }
     P.q_group = q_group;
+    P.q_group_magic = q_group_magic_for(q_group);
     P.q_subgroups = P.gqa / q_group;
     P.tok_tile = kPfRows / q_group;
     P.max_chunks = 1;
@@ -2508,7 +2697,16 @@ static size_t scratch_bytes_for(int local_kv_heads, int total_tokens, int num_re
     // (only batches in which no request has more than one tile take it; max_q_len <= 0: not known)
     if (num_reqs < 0 || num_reqs > total_tokens) num_reqs = total_tokens;
     if (num_reqs >= 2 && max_q_len <= tok_tile) {
-        const size_t prows = bal_partial_row(balanced_groups(q_subgroups) + num_reqs, kv_subs, 0, 0);
+        const size_t prows = bal_partial_row(balanced_groups(q_subgroups) + num_reqs, kv_subs, 0, 16, 0);
+        const size_t bal = partial_bytes((long long)prows, 1) + (size_t)total_tokens * 16;
+        if (bal > bytes) bytes = bal;
+    }
+    // verify batches: several column tiles per workgroup, several tiles per request (the query tokens
+    // taken as spread evenly over the requests)
+    const int q_len = max_q_len > 0 ? max_q_len : (total_tokens + num_reqs - 1) / num_reqs;
+    const BalShape shape = balanced_shape(q_len, q_group, 2);
+    if (shape.tiles <= kBalMaxTiles) {
+        const size_t prows = bal_partial_row(balanced_groups(q_subgroups) + num_reqs * shape.tiles, kv_subs, 0, 16 * shape.nt, 0);
         const size_t bal = partial_bytes((long long)prows, 1) + (size_t)total_tokens * 16;
         if (bal > bytes) bytes = bal;
     }

@@ -2,10 +2,9 @@
 // (FP16 or BF16 storage, identity transform) and the 8-bit rows FP8-E4M3-256 and Q8_0-64, for
 // gfx950.  Same work decomposition, chunk geometry, wave merge and split-K partial format as
 // the TQ4 kernel in paged_attn.hip (which includes this file); only the per-unit body differs:
-//   * a 32-token unit is processed as two 16-token halves; the wave copies the 16 K rows and
-//     16 V rows of a half into its private LDS area.  16-bit rows (512 B) get a row stride of
-//     544 bytes (keys) or 576 bytes (values), the strides at which their 128-bit operand reads
-//     are conflict-free; 8-bit rows (264 B / 272 B, codes and their fp32 block scales) 272 bytes;
+//   * the keys are dealt to the waves in halves of 16 tokens; the 16 K rows and 16 V rows of a half
+//     go straight from the pages into the wave's private LDS area (LDS-direct loads, one half
+//     ahead), laid out so that the operand reads do not conflict (RowsLds);
 //   * S^T = K Q^T: A operand = 16 K rows read from LDS, B operand = the query rows, loaded
 //     once in MFMA layout.  8-bit codes are widened to fp16 in registers (exact) and the fp32
 //     block scales are applied to per-block partial scores, so K is never rounded;
@@ -27,7 +26,7 @@ typedef short s4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
 
 constexpr int kKv16Waves = 8;
-// LDS row strides of 16-bit rows (512 B).  The key operand reads are 128 bits at (row n, piece b)
+// The sparse kernel (qsa_sparse_rows.h) copies its rows through registers.  LDS row strides of 16-bit rows (512 B).  The key operand reads are 128 bits at (row n, piece b)
 // for 16 rows x 4 pieces per instruction, the value reads 128 bits at (row 4 b + i, piece n): a
 // probe of those two patterns measures the rate of a contiguous read at 544 / 608 / 672 bytes for
 // the first and at 576 bytes for the second, 40 % less at 528.
@@ -92,9 +91,79 @@ __device__ __forceinline__ f4 mfma_x16(u2v a, u2v b, f4 c) {
     }
 }
 
+// Staging area of one wave: the K half (16 rows), then the V half, as LDS-direct loads leave them.
+//   16-bit rows: an instruction moves 1024 bytes = 2 rows (4 at head dimension 128).  Keys: the LDS
+//     address advances by 64 (128) bytes more than that, and inside an instruction the 16-byte
+//     pieces of row r are exchanged by r -- piece c of the row lies at c ^ 2 (r & 1) (c ^ 2 (r & 3)) --,
+//     which the lanes do by loading from the exchanged address.  The 128-bit operand reads of 16 rows
+//     then touch the banks in the same pattern as rows 544 bytes apart do.  Values: contiguous (a
+//     read takes the same 256 bytes of four rows whose distance is a multiple of 256 bytes).
+//   8-bit rows: contiguous, 272 (Q8_0) or 264 (FP8) bytes per row.
+template <int KVF, int HD>
+struct RowsLds {
+    static constexpr bool kFp8 = KVF == WARP34_KV_FORMAT_FP8_E4M3;
+    static constexpr bool k8 = kFp8 || KVF == WARP34_KV_FORMAT_Q8_0;
+    static constexpr int kRowBytes = k8 ? (kFp8 ? 264 : 272) : 2 * HD;  // in memory
+    static constexpr int kHalf = 16 * kRowBytes;                        // a half: 16 rows, contiguous in a page
+    static constexpr int kLoads = (kHalf + 1023) / 1024;                // instructions per half
+    static constexpr int kRowsPerLoad = k8 ? 0 : 1024 / kRowBytes;
+    static constexpr int kKeyPad = k8 ? 0 : (HD == 256 ? 64 : 128);     // per instruction
+    static constexpr int kKeyBytes = k8 ? (kHalf + 15) / 16 * 16 : kLoads * (1024 + kKeyPad);
+    // after the loop the area holds the wave's merge region (16 columns) and 1 KB for transposing
+    static constexpr int kColStride = HD + 8;                           // dwords, see kMergeColStride
+    static constexpr int kRegion = 16 * kColStride * 4;
+    static constexpr int kLoop = kKeyBytes + kHalf;
+    static constexpr int kStage = kLoop > kRegion + 1024 ? kLoop : kRegion + 1024;
+    static_assert(kStage % 16 == 0 && (kColStride * 4) % 256 == 32, "alignment, bank pattern of the merge reads");
+};
+// LDS of a workgroup with NT column tiles: [staging areas][query operands][(m, l) tables]
+template <int KVF, int HD>
+__host__ __device__ constexpr int rows_q_offset() {
+    return kKv16Waves * RowsLds<KVF, HD>::kStage;
+}
+template <int KVF, int HD>
+__host__ __device__ constexpr int rows_ml_offset(int nt) {
+    return rows_q_offset<KVF, HD>() + nt * (HD / 32) * 1024;
+}
+template <int KVF, int HD>
+__host__ __device__ constexpr int rows_smem_bytes(int nt) {
+    return rows_ml_offset<KVF, HD>(nt) + kKv16Waves * nt * 16 * 2 * 4;
+}
+
+// One LDS-direct load instruction: lane l's 16 bytes from base + voffset + IMM to lds_addr + IMM + 16 l.
+template <bool STREAM, int IMM>
+__device__ __forceinline__ void lds_load_piece(uint32_t voffset, const uint8_t* sbase, uint32_t lds_addr) {
+    if constexpr (STREAM) {
+        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 offset:%3 nt"
+                     : : "v"(voffset), "s"(sbase), "s"(lds_addr), "n"(IMM) : "memory");
+    } else {
+        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 offset:%3"
+                     : : "v"(voffset), "s"(sbase), "s"(lds_addr), "n"(IMM) : "memory");
+    }
+}
+// One half (16 rows): instruction i moves bytes 1024 i .. 1024 i + 1023 to lds_addr + (1024 + PAD) i.
+template <bool STREAM, int BYTES, int PAD, int I = 0>
+__device__ __forceinline__ void lds_load_half(uint32_t voffset, const uint8_t* sbase, uint32_t lds_addr, int lane) {
+    if constexpr (1024 * I < BYTES) {
+        constexpr int kImm = 1024 * (I & 3), kBase = 1024 * (I & ~3);  // the immediate holds 12 bits
+        if (BYTES - 1024 * I >= 1024 || lane < (BYTES - 1024 * I) / 16)
+            lds_load_piece<STREAM, kImm>(voffset, sbase + kBase, lds_addr + (uint32_t)(kBase + PAD * I));
+        lds_load_half<STREAM, BYTES, PAD, I + 1>(voffset, sbase, lds_addr, lane);
+    }
+}
+
 // KVF is the storage format of both slabs.  16-bit pages: TQ doubles as the storage type (F16
 // query/output over FP16 pages, BF16 over BF16 pages).  8-bit pages: the MFMAs run in fp16 and
 // a BF16 query is converted once.
+// NT: 16-column tiles per workgroup.  A verify step or a draft block has more than 16 query columns
+// per kv head; with two tiles the keys are read, and 8-bit codes widened, once for 32 columns.  The
+// accumulators take 64 NT registers at head dimension 256 (32 NT at 128), so the query operands stay in
+// LDS for NT = 2 and are read again for every half.  (Four tiles at head dimension 128: the merge of
+// the eight waves, 2 us per tile, outweighs the keys read once more: 24.8 against 20.7 us for four draft
+// blocks of sixteen tokens over 1K to 9K keys.)
+// Bound: one workgroup per CU streams about 20 bytes per ns, what the memory delivers; below some 100 MB the
+// launch is the chain arguments - plan - block table - first rows (7 us to the first product), the
+// streaming, and the merge of the waves (2.3 us per tile).
 // BAL: the tile and its unit range come from `item` (balanced decode, see bal_for_each_piece)
 // instead of blockIdx.
 // VRES (8-bit rows stored rotated): the value operand fp16(d * code) is followed by a second
@@ -108,19 +177,18 @@ __device__ __forceinline__ f4 mfma_x16(u2v a, u2v b, f4 c) {
 template <typename TQ, int NT, int KVF, bool BAL, bool VRES = false, bool STREAM = BAL, int HD = kHeadDim>
 __device__ __forceinline__ void rows_tile(const AttnParams& P, uint8_t* smem, const BalItem& item) {
     static_assert(!VRES || KVF == WARP34_KV_FORMAT_FP8_E4M3 || KVF == WARP34_KV_FORMAT_Q8_0, "residual operand: 8-bit rows");
-    constexpr bool K8 = KVF == WARP34_KV_FORMAT_FP8_E4M3 || KVF == WARP34_KV_FORMAT_Q8_0;
+    using M = RowsLds<KVF, HD>;
+    constexpr bool K8 = M::k8;
+    constexpr bool FP8 = M::kFp8;
     static_assert(HD == 256 || (HD == 128 && !K8), "head dimension 128: 16-bit rows only");
+    static_assert(NT == 1 || BAL, "several column tiles: balanced form only");
     constexpr int kM = HD / 32;   // QK operands (32 elements each) per row
     constexpr int kH = HD / 128;  // 128-element halves of a row
-    constexpr bool FP8 = KVF == WARP34_KV_FORMAT_FP8_E4M3;
     static_assert(K8 || KVF == TQ::kStorageFormat, "16-bit pages are read in the query type");
     constexpr bool IS_BF16 = !K8 && TQ::kStorageFormat == WARP34_KV_FORMAT_BF16;
     constexpr bool Q_BF16 = TQ::kStorageFormat == WARP34_KV_FORMAT_BF16;
     constexpr int kWaves = kKv16Waves;
-    // LDS row strides (16-bit rows of 256 bytes: the row plus 32 / 64 bytes, the same bank pattern as 544 / 576)
-    constexpr int kRowStride = K8 ? kKv8RowStride : (HD == 256 ? kKv16RowStride : 2 * HD + 32);    // key rows
-    constexpr int kVRowStride = K8 ? kKv8RowStride : (HD == 256 ? kKv16VRowStride : 2 * HD + 64);  // value rows
-    constexpr int kRowBytes = K8 ? (FP8 ? 264 : 272) : 2 * HD;       // row in memory
+    constexpr int kRowBytes = M::kRowBytes;
 
     const int tid = (int)threadIdx.x;
     const int lane = tid & 63;
@@ -132,62 +200,33 @@ __device__ __forceinline__ void rows_tile(const AttnParams& P, uint8_t* smem, co
 
     const int tile_z = BAL ? item.req : (int)blockIdx.z;  // tile index (see locate_tile)
     const int kv_sub = (int)blockIdx.y;
-    const int kv_head = fast_div(kv_sub, P.q_subgroups);
+    const int kv_head = small_div(kv_sub, P.q_subgroups);
     const int q_head_base = kv_head * P.gqa + (kv_sub - kv_head * P.q_subgroups) * P.q_group;
     const int chunk = BAL ? 0 : (int)blockIdx.x;
 
-    // query rows in MFMA B layout straight from global memory: lane (n, b) holds
-    // Q[column n][32 m + 8 b .. + 7] for m = 0..7 (dead columns are zeroed below).  The first
-    // token of the tile is guessed so that these loads overlap the lookup; a wrong guess is
-    // corrected after it.
-    const int tok_guess = BAL ? item.rq_start
-                              : min(P.tiles_by_request ? tile_z : tile_z * P.tok_tile, B.total_tokens - 1);
-    u4 bq[NT][kM];
-    auto load_q = [&](int tokbase) {
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt) {
-            const int col = nt * 16 + n;
-            const int t = fast_div(col, P.q_group);
-            const int a = col - t * P.q_group;
-            const int tok = min(tokbase + t, B.total_tokens - 1);
-            const uint16_t* qrow = P.q + ((size_t)tok * P.num_q_heads + (size_t)(q_head_base + a)) * HD;
-#pragma unroll
-            for (int m = 0; m < kM; ++m) bq[nt][m] = *reinterpret_cast<const u4*>(qrow + 32 * m + 8 * b);
-        }
-    };
-    // Rotated K rows: the query rows go through sign + WHT256 first (one row per wave at a time,
-    // element e = 4 lane + k), are staged as fp16 in the still unused staging area and read
-    // back in MFMA layout.
-    constexpr int kQStride = 264;  // halves
-    auto load_q_rotated = [&](int tokbase) {
-        if constexpr (HD != 256) return;
-        _Float16* qlds = reinterpret_cast<_Float16*>(smem);
-        for (int col = wave; col < 16 * NT; col += kWaves) {
-            const int t = fast_div(col, P.q_group);
-            const int a = col - t * P.q_group;
-            const int tok = min(tokbase + t, B.total_tokens - 1);
-            const uint16_t* qrow = P.q + ((size_t)tok * P.num_q_heads + (size_t)(q_head_base + a)) * kHeadDim;
-            const uint2 raw = *reinterpret_cast<const uint2*>(qrow + 4 * lane);
-            float v[4] = {TQ::to_f32((uint16_t)(raw.x & 0xFFFFu)), TQ::to_f32((uint16_t)(raw.x >> 16)),
-                          TQ::to_f32((uint16_t)(raw.y & 0xFFFFu)), TQ::to_f32((uint16_t)(raw.y >> 16))};
-#pragma unroll
-            for (int k = 0; k < 4; ++k) v[k] = apply_sign(v[k], 4 * lane + k);
-            wht256_wave(v, lane);
-            uint2 packed;
-            packed.x = pack_h2(v[0], v[1]);
-            packed.y = pack_h2(v[2], v[3]);
-            *reinterpret_cast<uint2*>(qlds + col * kQStride + 4 * lane) = packed;
-        }
-        __syncthreads();
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-            for (int m = 0; m < kM; ++m)
-                bq[nt][m] = *reinterpret_cast<const u4*>(qlds + (nt * 16 + n) * kQStride + 32 * m + 8 * b);
-        __syncthreads();  // the staging area is reused by the K/V rows
-    };
+    // Query rows in MFMA B layout: lane (n, b) holds Q[column n][32 m + 8 b .. + 7] for m = 0..kM-1.
+    // One tile of un-rotated queries comes straight from global memory into registers; the first
+    // token of the tile is guessed so that these loads overlap the lookup, a wrong guess is corrected
+    // after it.  Rotated queries and several tiles go through the LDS table below.
     const bool rot_q = K8 && P.rot_q != 0;  // workgroup-uniform
-    if (!rot_q) load_q(tok_guess);
+    const bool q_direct = NT == 1 && !rot_q;
+    const int tok_guess = BAL ? item.rq_start + item.tile * P.tok_tile
+                              : min(P.tiles_by_request ? tile_z : tile_z * P.tok_tile, B.total_tokens - 1);
+    u4 bq[kM];
+    auto load_q = [&](int tokbase) {
+        const int t = div_q_group(n, P);
+        const int a = n - t * P.q_group;
+        const int tok = min(tokbase + t, B.total_tokens - 1);
+        const uint16_t* qrow = P.q + ((size_t)tok * P.num_q_heads + (size_t)(q_head_base + a)) * HD;
+#pragma unroll
+        for (int m = 0; m < kM; ++m) bq[m] = *reinterpret_cast<const u4*>(qrow + 32 * m + 8 * b);
+    };
+    if (q_direct) {
+        load_q(tok_guess);
+    } else {
+#pragma unroll
+        for (int m = 0; m < kM; ++m) bq[m] = u4{0u, 0u, 0u, 0u};
+    }
 
     // Speculative block-table load, in flight together with the lookup: it assumes that the
     // request's length is the host's bound max_seq_len.  A wrong guess is fetched again below,
@@ -206,7 +245,7 @@ __device__ __forceinline__ void rows_tile(const AttnParams& P, uint8_t* smem, co
     }
     TileInfo ti;
     if constexpr (BAL) {
-        ti = TileInfo{true, item.req, item.rq_start, item.rq_end, item.seq_after, item.ctx_before, 0};
+        ti = TileInfo{true, item.req, item.rq_start, item.rq_end, item.seq_after, item.ctx_before, item.tile};
     } else {
         ti = locate_tile(P, tile_z, lane);
     }
@@ -214,26 +253,22 @@ __device__ __forceinline__ void rows_tile(const AttnParams& P, uint8_t* smem, co
     const int req = ti.req, rq_start = ti.rq_start, rq_end = ti.rq_end;
     const int seq_after = ti.seq_after, ctx_before = ti.ctx_before;
     const int tok0 = rq_start + ti.tile_in_req * P.tok_tile;
-    if (rot_q) {
-        load_q_rotated(tok0);  // every wave of the workgroup takes the same path up to here
-    } else {
+    if (q_direct) {
         if (tok0 != tok_guess) load_q(tok0);  // wave-uniform, rare
         if constexpr (K8 && Q_BF16) {
 #pragma unroll
-            for (int nt = 0; nt < NT; ++nt)
+            for (int m = 0; m < kM; ++m)
 #pragma unroll
-                for (int m = 0; m < kM; ++m)
-#pragma unroll
-                    for (int k = 0; k < 4; ++k) {
-                        const uint32_t w = bq[nt][m][k];
-                        bq[nt][m][k] = pack_h2(BF16::to_f32((uint16_t)(w & 0xFFFFu)), BF16::to_f32((uint16_t)(w >> 16)));
-                    }
+                for (int k = 0; k < 4; ++k) {
+                    const uint32_t w = bq[m][k];
+                    bq[m][k] = pack_h2(BF16::to_f32((uint16_t)(w & 0xFFFFu)), BF16::to_f32((uint16_t)(w >> 16)));
+                }
         }
     }
     bool tok_ok[NT];
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
-        const int tok = tok0 + fast_div(nt * 16 + n, P.q_group);
+        const int tok = tok0 + div_q_group(nt * 16 + n, P);
         tok_ok[nt] = tok < B.total_tokens &&
                      (B.valid_token_mask == nullptr || B.valid_token_mask[min(tok, B.total_tokens - 1)] != 0);
     }
@@ -260,7 +295,7 @@ __device__ __forceinline__ void rows_tile(const AttnParams& P, uint8_t* smem, co
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) {
             const int col = nt * 16 + n;
-            const int t = fast_div(col, P.q_group);
+            const int t = div_q_group(col, P);
             const int tok = tok0 + t;
             const bool ok = t < tile_tokens && tok_ok[nt];
             const int q_off = tok - rq_start;
@@ -280,9 +315,9 @@ __device__ __forceinline__ void rows_tile(const AttnParams& P, uint8_t* smem, co
                         u_hi = max(u_hi, mx);
                     }
                 }
-            } else {
+            } else if (NT == 1) {
 #pragma unroll
-                for (int m = 0; m < kM; ++m) bq[nt][m] = u4{0u, 0u, 0u, 0u};
+                for (int m = 0; m < kM; ++m) bq[m] = u4{0u, 0u, 0u, 0u};
             }
             ok_mask[nt] = (uint32_t)(__ballot(ok) & 0xFFFFull);
         }
@@ -338,100 +373,63 @@ __device__ __forceinline__ void rows_tile(const AttnParams& P, uint8_t* smem, co
         if (cu_end > g.u_first + g.n_units) cu_end = g.u_first + g.n_units;
     }
 
+    // ---- staging: LDS-direct loads of half units, K and V one half ahead ------------------------------
     const uint8_t* k_base = reinterpret_cast<const uint8_t*>((uintptr_t)L.k_base) +
                             (size_t)kv_head * L.k_head_stride_bytes;
     const uint8_t* v_base = reinterpret_cast<const uint8_t*>((uintptr_t)L.v_base) +
                             (size_t)kv_head * L.v_head_stride_bytes;
-    uint8_t* stage = smem + wave * kKv16Stage;  // [K rows 0..15][V rows 0..15], kRowStride each
+    uint8_t* stage = smem + wave * M::kStage;
+    const uint8_t* k_rows = stage;
+    const uint8_t* v_rows = stage + M::kKeyBytes;
+    // (the dynamic LDS block starts at LDS address 0: the kernel has no static LDS, checked on the host)
+    const uint32_t k_lds = (uint32_t)(wave * M::kStage), v_lds = k_lds + (uint32_t)M::kKeyBytes;
     const int32_t* req_blocks = B.block_tables + (size_t)req * B.max_blocks_per_req;
     int slot_base = div_block(cu_first * kUnit, P);
     int page_vec;
+    // (one assembly statement with its own wait, see the TQ4 kernel: a compiler load here would put a
+    // vmcnt(0) in front of every half)
     auto load_page_vec = [&]() {
         const int slot = slot_base + lane;
-        page_vec = slot < B.max_blocks_per_req ? req_blocks[slot] : -1;
+        int32_t ids = -1;
+        if (slot < B.max_blocks_per_req) {
+            const int32_t* src = req_blocks + slot;
+            asm volatile("global_load_dword %0, %1, off\n\ts_waitcnt vmcnt(0)" : "=v"(ids) : "v"(src) : "memory");
+        }
+        page_vec = ids;
     };
-
-    // A half = 16 consecutive tokens: 16 K rows and 16 V rows, each run contiguous inside one
-    // page (8 KiB of 16-bit rows, 4224 B of FP8 rows, 4352 B of Q8_0 rows).  It is fetched as
-    // 16-byte pieces c = lane + 64 i.
-    constexpr int kPieces = 16 * kRowBytes / 16;        // 512, 264 or 272 (256 at head dimension 128)
-    constexpr int kLoads = (kPieces + 63) / 64;         // 8 or 5 (4)
-    u4 pf[2 * kLoads];
-    auto issue_half = [&](int hidx) {  // hidx = 2 * unit + half
+    // lane l of a load instruction fetches piece l of the 64 it moves; key rows of 16-bit pages with
+    // their pieces exchanged (see RowsLds)
+    uint32_t k_off = (uint32_t)lane * 16u;
+    const uint32_t v_off = (uint32_t)lane * 16u;
+    if constexpr (!K8) {
+        constexpr int kPieces = kRowBytes / 16;
+        const int r = lane / kPieces, c = lane % kPieces;
+        k_off = (uint32_t)(r * kRowBytes + 16 * (c ^ (2 * (r & (M::kRowsPerLoad - 1)))));
+    }
+    const uint8_t* next_k;
+    const uint8_t* next_v;
+    // rows of the half with index hidx (16 tokens); halves outside the visible range read page 0
+    auto locate_half = [&](int hidx) {
         const int pos = hidx * 16;
         const int page_slot = div_block(pos, P);
         const int in_page = pos - page_slot * L.block_size;
         int rel = page_slot - slot_base;
-        if (rel >= 64) {
+        if (rel >= 64) {  // wave-uniform, at most once per 64 slots
             slot_base = page_slot;
             load_page_vec();
             rel = 0;
         }
         const int32_t pg = __builtin_amdgcn_readlane(page_vec, rel);
         const bool live = pos <= u_hi && pos + 15 >= u_lo && pg >= 0;
-        const uint8_t* kp = k_base + (live ? (size_t)pg * L.k_page_stride_bytes + (size_t)in_page * L.k_token_stride_bytes : 0);
-        const uint8_t* vp = v_base + (live ? (size_t)pg * L.v_page_stride_bytes + (size_t)in_page * L.v_token_stride_bytes : 0);
-        // STREAM: every key is read by exactly one workgroup (decode steps: no request has more
-        // than one tile), and the loads carry the non-temporal hint, which is worth 8 to 13 % on a
-        // plain streaming read of HBM and 3 to 8 % here.  Tiles that share a request's keys
-        // (verify, prefill through this kernel) keep ordinary loads: with the hint their batches
-        // measure 7 to 22 % slower, the lines are gone when the next tile asks for them.
-#pragma unroll
-        for (int i = 0; i < kLoads; ++i) {
-            // pieces beyond the run (last, partial round of the 8-bit formats) re-read piece 0
-            const int c = (kPieces % 64 == 0 || lane + 64 * i < kPieces) ? lane + 64 * i : 0;
-            if constexpr (STREAM) {
-                pf[i] = __builtin_nontemporal_load((global_cu4*)(kp + 16 * c));
-                pf[kLoads + i] = __builtin_nontemporal_load((global_cu4*)(vp + 16 * c));
-            } else {
-                pf[i] = *(global_cu4*)(kp + 16 * c);
-                pf[kLoads + i] = *(global_cu4*)(vp + 16 * c);
-            }
-        }
+        next_k = k_base + (live ? (size_t)pg * L.k_page_stride_bytes + (size_t)in_page * L.k_token_stride_bytes : 0);
+        next_v = v_base + (live ? (size_t)pg * L.v_page_stride_bytes + (size_t)in_page * L.v_token_stride_bytes : 0);
     };
-    // rows outside [u_lo, u_hi] are stored as zeros: unwritten pool memory may hold NaN
-    // patterns, and 0 * NaN would poison the P V product
-    auto commit_half = [&](int hidx) {
-        const int pos0 = hidx * 16;
-        const bool edge = pos0 < u_lo || pos0 + 15 > u_hi;
-        uint8_t* k_rows = stage;
-        uint8_t* v_rows = stage + 16 * kRowStride;
-#pragma unroll
-        for (int i = 0; i < kLoads; ++i) {
-            const int c = lane + 64 * i;
-            if (kPieces % 64 != 0 && c >= kPieces) break;
-            u4 kv = pf[i], vv = pf[kLoads + i];
-            if constexpr (FP8) {
-                // 264-byte rows: the two 8-byte halves of a piece may belong to different rows
-#pragma unroll
-                for (int hf = 0; hf < 2; ++hf) {
-                    const unsigned sub = 2u * (unsigned)c + hf;
-                    const unsigned row = sub / 33u, col = sub - row * 33u;
-                    u2v k8 = hf ? u2v{kv[2], kv[3]} : u2v{kv[0], kv[1]};
-                    u2v v8 = hf ? u2v{vv[2], vv[3]} : u2v{vv[0], vv[1]};
-                    if (edge && !(pos0 + (int)row >= u_lo && pos0 + (int)row <= u_hi)) {
-                        k8 = u2v{0u, 0u};
-                        v8 = u2v{0u, 0u};
-                    }
-                    *reinterpret_cast<u2v*>(k_rows + row * kRowStride + 8 * col) = k8;
-                    *reinterpret_cast<u2v*>(v_rows + row * kVRowStride + 8 * col) = v8;
-                }
-            } else {
-                constexpr int kPiecesPerRow = kRowBytes / 16;  // 32 or 17
-                const int row = (int)((unsigned)c / (unsigned)kPiecesPerRow);
-                const int col = c - row * kPiecesPerRow;
-                if (edge) {
-                    const bool vis = pos0 + row >= u_lo && pos0 + row <= u_hi;
-                    if (!vis) {
-                        kv = u4{0u, 0u, 0u, 0u};
-                        vv = u4{0u, 0u, 0u, 0u};
-                    }
-                }
-                *reinterpret_cast<u4*>(k_rows + row * kRowStride + 16 * col) = kv;
-                *reinterpret_cast<u4*>(v_rows + row * kVRowStride + 16 * col) = vv;
-            }
-        }
-    };
+    // STREAM: every key is read by exactly one workgroup (no request has more than one tile), and
+    // the loads carry the non-temporal hint, which is worth 8 to 13 % on a plain streaming read of
+    // HBM.  Tiles that share a request's keys keep ordinary loads: with the hint the lines are gone
+    // when the next tile asks for them.
+    auto issue_k = [&]() { lds_load_half<STREAM, M::kHalf, M::kKeyPad>(k_off, next_k, k_lds, lane); };
+    auto issue_v = [&]() { lds_load_half<STREAM, M::kHalf, 0>(v_off, next_v, v_lds, lane); };
 
     f4 o_acc[NT][kH][8];
     float m_run[NT], l_run[NT];
@@ -445,115 +443,145 @@ __device__ __forceinline__ void rows_tile(const AttnParams& P, uint8_t* smem, co
             for (int j = 0; j < 8; ++j) o_acc[nt][h][j] = f4{0.f, 0.f, 0.f, 0.f};
     }
     const float score_scale = B.sm_scale * kLog2e;
+    // query operands of tile nt, step m: 1 KB each, lane l's 16 bytes at 16 l
+    uint8_t* qtab = smem + rows_q_offset<KVF, HD>();
+    auto q_operand = [&](int nt, int m) -> u4 {
+        if constexpr (NT == 1) return bq[m];
+        else return *reinterpret_cast<const u4*>(qtab + (nt * kM + m) * 1024 + 16 * lane);
+    };
+    // where this lane reads its key operands (row n, piece 4 m + b): the exchange of the pieces
+    // touches bit 1 of the piece number (in b) and, at head dimension 128, bit 2 (in m)
+    const uint8_t* ka_even = k_rows;
+    const uint8_t* ka_odd = k_rows;
+    if constexpr (!K8) {
+        constexpr int kRpl = M::kRowsPerLoad;
+        const uint8_t* row = k_rows + (n / kRpl) * (1024 + M::kKeyPad) + (n % kRpl) * kRowBytes;
+        if constexpr (kRpl == 2) {
+            ka_even = ka_odd = row + 16 * (b ^ (2 * (n & 1)));
+        } else {
+            const int swap = (n >> 1) & 1;
+            ka_even = row + 16 * (b ^ (2 * (n & 1))) + 64 * swap;
+            ka_odd = row + 16 * (b ^ (2 * (n & 1))) - 64 * swap;
+        }
+    }
 
-    auto process_half = [&](int pos0, const bool MASKED) {
-        const uint8_t* k_rows = stage;
-        const uint8_t* v_rows = stage + 16 * kRowStride;
-        // ---- S^T = K Q^T: A row n = token n of the half ----
+    // One 16-token half.  MASKED = false (wave-uniform): every token is visible to every live column.
+    auto process_half = [&](int pos0, const bool MASKED, const bool HAS_NEXT) {
+        wait_vm<M::kLoads>();  // this half's keys have landed, its values may still be in flight
         f4 s_acc[NT];
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) s_acc[nt] = f4{0.f, 0.f, 0.f, 0.f};
-        // V operands of the 16 P V MFMAs: a_v[h][j] = element 128 h + 8 n + j of tokens 4b..4b+3
-        u2v a_v[kH][8];
-        u2v a_vr[VRES ? 2 : 1][VRES ? 8 : 1];  // residuals of a_v
-        if constexpr (K8 && HD == 256) {
+        u4 ka[kM];
+        if constexpr (K8) {
             // Codes of row n, elements 32 m + 8 b .. + 7, widened to fp16; one partial score per
             // scale block (FP8: 2 blocks of 128 = m / 4; Q8_0: 4 blocks of 64 = m / 2), combined
             // with the fp32 scales of this lane's 4 tokens.
             constexpr int kBlocks = FP8 ? 2 : 4;
             constexpr int kMPerBlock = 8 / kBlocks;
-            u4 ka[8];
+            uint32_t kc[8][2];
 #pragma unroll
             for (int m = 0; m < 8; ++m) {
                 const int off = FP8 ? 32 * m + 8 * b : 68 * (m >> 1) + 4 + 32 * (m & 1) + 8 * b;
-                const uint32_t* src = reinterpret_cast<const uint32_t*>(k_rows + n * kRowStride + off);
-                const uint32_t w0 = src[0], w1 = src[1];
-                uint32_t h0, h1, h2_, h3;
-                if constexpr (FP8) {
-                    fp8x4_to_h4(w0, h0, h1);
-                    fp8x4_to_h4(w1, h2_, h3);
-                } else {
-                    i8x4_to_h4(w0, h0, h1);
-                    i8x4_to_h4(w1, h2_, h3);
-                }
-                ka[m] = u4{h0, h1, h2_, h3};
+                const uint32_t* src = reinterpret_cast<const uint32_t*>(k_rows + n * kRowBytes + off);
+                kc[m][0] = src[0];
+                kc[m][1] = src[1];
             }
             float dk[4][kBlocks];
 #pragma unroll
             for (int i = 0; i < 4; ++i)
 #pragma unroll
                 for (int kb = 0; kb < kBlocks; ++kb)
-                    dk[i][kb] = *reinterpret_cast<const float*>(k_rows + (4 * b + i) * kRowStride +
+                    dk[i][kb] = *reinterpret_cast<const float*>(k_rows + (4 * b + i) * kRowBytes +
                                                                 (FP8 ? 256 + 4 * kb : 68 * kb));
+            wait_lds_reads();
+            if (HAS_NEXT) issue_k();  // located by the caller
 #pragma unroll
-            for (int nt = 0; nt < NT; ++nt) {
+            for (int kb = 0; kb < kBlocks; ++kb) {
+                f4 part[NT];
 #pragma unroll
-                for (int kb = 0; kb < kBlocks; ++kb) {
-                    f4 part = f4{0.f, 0.f, 0.f, 0.f};
+                for (int nt = 0; nt < NT; ++nt) part[nt] = f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                    for (int mm = 0; mm < kMPerBlock; ++mm)
-                        part = mfma_x32<false>(ka[kb * kMPerBlock + mm], bq[nt][kb * kMPerBlock + mm], part);
+                for (int mm = 0; mm < kMPerBlock; ++mm) {
+                    const int m = kb * kMPerBlock + mm;
+                    uint32_t h0, h1, h2_, h3;
+                    if constexpr (FP8) {
+                        fp8x4_to_h4(kc[m][0], h0, h1);
+                        fp8x4_to_h4(kc[m][1], h2_, h3);
+                    } else {
+                        i8x4_to_h4(kc[m][0], h0, h1);
+                        i8x4_to_h4(kc[m][1], h2_, h3);
+                    }
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) s_acc[nt][i] += dk[i][kb] * part[i];
+                    for (int nt = 0; nt < NT; ++nt)
+                        part[nt] = mfma_x32<false>(u4{h0, h1, h2_, h3}, q_operand(nt, m), part[nt]);
                 }
-            }
-            // V: fp16(d * code), the value the reference stages (op_paged_attn.cu:59-105)
 #pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                float vf[4][8];
+                for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) s_acc[nt][i] += dk[i][kb] * part[nt][i];
+            }
+        } else {
+#pragma unroll
+            for (int m = 0; m < kM; ++m)
+                ka[m] = *reinterpret_cast<const u4*>(((m & 1) ? ka_odd : ka_even) + 64 * m);
+            wait_lds_reads();
+            if (HAS_NEXT) issue_k();
+#pragma unroll
+            for (int m = 0; m < kM; ++m)
+#pragma unroll
+                for (int nt = 0; nt < NT; ++nt) s_acc[nt] = mfma_x32<IS_BF16>(ka[m], q_operand(nt, m), s_acc[nt]);
+        }
+
+        // ---- raw value rows of this lane's tokens 4b .. 4b + 3 ----
+        if (HAS_NEXT) {
+            wait_vm<M::kLoads>();  // the values have landed, the next half's keys may be in flight
+        } else {
+            wait_vm<0>();
+        }
+        u4 vr[K8 ? 1 : kH][4];
+        uint32_t vc[K8 ? 2 : 1][4][2];
+        float vd[K8 ? 2 : 1][4];
+        if constexpr (K8) {
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    const uint8_t* vrow = v_rows + (4 * b + i) * kVRowStride;
+                    const uint8_t* vrow = v_rows + (4 * b + i) * kRowBytes;
                     const int blk = 2 * h + (n >> 3);  // Q8_0 block of element 128 h + 8 n
                     const int off = FP8 ? 128 * h + 8 * n : 68 * blk + 4 + 8 * (n & 7);
                     const uint32_t* src = reinterpret_cast<const uint32_t*>(vrow + off);
-                    const float d = *reinterpret_cast<const float*>(vrow + (FP8 ? 256 + 4 * h : 68 * blk));
-                    float f0[4], f1[4];
-                    codes4_to_f32<FP8>(src[0], f0);
-                    codes4_to_f32<FP8>(src[1], f1);
-#pragma unroll
-                    for (int k = 0; k < 4; ++k) {
-                        vf[i][k] = d * f0[k];
-                        vf[i][4 + k] = d * f1[k];
-                    }
+                    vc[h][i][0] = src[0];
+                    vc[h][i][1] = src[1];
+                    vd[h][i] = *reinterpret_cast<const float*>(vrow + (FP8 ? 256 + 4 * h : 68 * blk));
                 }
-#pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    if constexpr (VRES) {
-                        uint32_t hi0, lo0, hi1, lo1;
-                        split_h2(vf[0][j], vf[1][j], hi0, lo0);
-                        split_h2(vf[2][j], vf[3][j], hi1, lo1);
-                        a_v[h][j] = u2v{hi0, hi1};
-                        a_vr[h][j] = u2v{lo0, lo1};
-                    } else {
-                        a_v[h][j] = u2v{pack_h2(vf[0][j], vf[1][j]), pack_h2(vf[2][j], vf[3][j])};
-                    }
-                }
-            }
         } else {
-            u4 ka[kM];
 #pragma unroll
-            for (int m = 0; m < kM; ++m)
-                ka[m] = *reinterpret_cast<const u4*>(k_rows + n * kRowStride + 64 * m + 16 * b);
-#pragma unroll
-            for (int m = 0; m < kM; ++m)
-#pragma unroll
-                for (int nt = 0; nt < NT; ++nt) s_acc[nt] = mfma_x32<IS_BF16>(ka[m], bq[nt][m], s_acc[nt]);
-
-            // V slices of this lane's 4 tokens (rows 4b..4b+3), both halves of the head dim; the
-            // 4x8 block of 16-bit values is transposed in registers
-#pragma unroll
-            for (int h = 0; h < kH; ++h) {
-                u4 vr[4];
+            for (int h = 0; h < kH; ++h)
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
-                    vr[i] = *reinterpret_cast<const u4*>(v_rows + (4 * b + i) * kVRowStride + 256 * h + 16 * n);
+                    vr[h][i] = *reinterpret_cast<const u4*>(v_rows + (4 * b + i) * kRowBytes + 256 * h + 16 * n);
+        }
+        wait_lds_reads();
+        if (HAS_NEXT) issue_v();
+        // rows outside [u_lo, u_hi] count as zeros: unwritten pool memory may hold NaN patterns,
+        // and 0 * NaN would poison the P V product
+        if (MASKED) {
 #pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    // 16-bit element j of the four token slices -> (t0,t1), (t2,t3)
-                    const uint32_t sel = (j & 1) ? 0x07060302u : 0x05040100u;
-                    a_v[h][j] = u2v{__builtin_amdgcn_perm(vr[1][j >> 1], vr[0][j >> 1], sel),
-                                    __builtin_amdgcn_perm(vr[3][j >> 1], vr[2][j >> 1], sel)};
+            for (int i = 0; i < 4; ++i) {
+                const int pos = pos0 + 4 * b + i;
+                const bool row_ok = pos >= u_lo && pos <= u_hi;
+                if constexpr (K8) {
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {
+                        vc[h][i][0] = row_ok ? vc[h][i][0] : 0u;
+                        vc[h][i][1] = row_ok ? vc[h][i][1] : 0u;
+                        vd[h][i] = row_ok ? vd[h][i] : 0.f;
+                    }
+                } else {
+#pragma unroll
+                    for (int h = 0; h < kH; ++h)
+#pragma unroll
+                        for (int k = 0; k < 4; ++k) vr[h][i][k] = row_ok ? vr[h][i][k] : 0u;
                 }
             }
         }
@@ -611,82 +639,164 @@ __device__ __forceinline__ void rows_tile(const AttnParams& P, uint8_t* smem, co
             }
         }
 
-        // ---- O^T += V^T P^T: row r = n of MFMA (h, j) is head dimension 128 h + 8 n + j ----
+        // ---- O^T += V^T P^T: row r = n of MFMA (h, j) is head dimension 128 h + 8 n + j; its operand
+        // holds that element of tokens 4b .. 4b + 3 ----
 #pragma unroll
         for (int h = 0; h < kH; ++h) {
+            u2v a_v[8];
+            u2v a_vr[VRES ? 8 : 1];  // residuals of a_v
+            if constexpr (K8) {
+                // fp16(d * code), the value the reference stages (op_paged_attn.cu:59-105)
+                float vf[4][8];
 #pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const u2v a = a_v[h][j];
+                for (int i = 0; i < 4; ++i) {
+                    float f0[4], f1[4];
+                    codes4_to_f32<FP8>(vc[h][i][0], f0);
+                    codes4_to_f32<FP8>(vc[h][i][1], f1);
 #pragma unroll
-                for (int nt = 0; nt < NT; ++nt) {
-                    o_acc[nt][h][j] = mfma_x16<IS_BF16>(a, pb_hi[nt], o_acc[nt][h][j]);
-                    if constexpr (IS_BF16) o_acc[nt][h][j] = mfma_x16<IS_BF16>(a, pb_lo[nt], o_acc[nt][h][j]);
+                    for (int k = 0; k < 4; ++k) {
+                        vf[i][k] = vd[h][i] * f0[k];
+                        vf[i][4 + k] = vd[h][i] * f1[k];
+                    }
                 }
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    if constexpr (VRES) {
+                        uint32_t hi0, lo0, hi1, lo1;
+                        split_h2(vf[0][j], vf[1][j], hi0, lo0);
+                        split_h2(vf[2][j], vf[3][j], hi1, lo1);
+                        a_v[j] = u2v{hi0, hi1};
+                        a_vr[j] = u2v{lo0, lo1};
+                    } else {
+                        a_v[j] = u2v{pack_h2(vf[0][j], vf[1][j]), pack_h2(vf[2][j], vf[3][j])};
+                    }
+                }
+            } else {
+                // the 4x8 block of 16-bit values is transposed in registers
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    // 16-bit element j of the four token slices -> (t0,t1), (t2,t3)
+                    const uint32_t sel = (j & 1) ? 0x07060302u : 0x05040100u;
+                    a_v[j] = u2v{__builtin_amdgcn_perm(vr[h][1][j >> 1], vr[h][0][j >> 1], sel),
+                                 __builtin_amdgcn_perm(vr[h][3][j >> 1], vr[h][2][j >> 1], sel)};
+                }
+            }
+            if constexpr (VRES) settle(a_vr);
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+#pragma unroll
+                for (int nt = 0; nt < NT; ++nt) o_acc[nt][h][j] = mfma_x16<IS_BF16>(a_v[j], pb_hi[nt], o_acc[nt][h][j]);
+            if constexpr (IS_BF16) {
+#pragma unroll
+                for (int j = 0; j < 8; ++j)
+#pragma unroll
+                    for (int nt = 0; nt < NT; ++nt) o_acc[nt][h][j] = mfma_x16<true>(a_v[j], pb_lo[nt], o_acc[nt][h][j]);
             }
             if constexpr (VRES) {
 #pragma unroll
                 for (int j = 0; j < 8; ++j)
 #pragma unroll
                     for (int nt = 0; nt < NT; ++nt)
-                        o_acc[nt][h][j] = mfma_x16<false>(a_vr[h][j], pb_hi[nt], o_acc[nt][h][j]);
+                        o_acc[nt][h][j] = mfma_x16<false>(a_vr[j], pb_hi[nt], o_acc[nt][h][j]);
             }
         }
     };
 
-    // halves of this wave's units, in order; the next half is in flight while one is processed
-    int unit = cu_first + wave;
+    // Halves are dealt to the waves round robin, a fixed rule (the result must not depend on timing).
+    const int h_end = min(2 * cu_end, (u_hi >> 4) + 1);  // (the last unit may end with an invisible half)
+    int hidx = 2 * cu_first + wave;
     if (slot_base == spec_slot_base) {
         page_vec = spec_vec;
     } else {
         load_page_vec();
     }
-    // Units are dealt by a fixed rule (the result must not depend on timing): round robin with
-    // one extra unit for waves 0-3 after every eight rounds, because each SIMD serves its older
-    // wave first (see the TQ4 kernel).
-    auto nth_unit = [&](int j) -> int {
-        if (wave < 4) {
-            const int g = j / 9, k = j - 9 * g;
-            return cu_first + 68 * g + (k < 8 ? 8 * k + wave : 64 + wave);
-        }
-        return cu_first + 68 * (j >> 3) + 8 * (j & 7) + wave;
-    };
-    static_assert(kWaves == 8, "unit deal assumes two waves per SIMD");
-    int hidx = 2 * unit, unit_no = 0;
     // The query operands are touched again after the first rows have been requested (dead columns
     // are zeroed).  Loads return in order: a wait for them placed behind the row loads would wait
     // for the rows too, so the compiler is made to finish them here, where they have long landed.
+    // (On every path: the compiler does not connect this test of q_direct with the one at the loads,
+    // and would otherwise wait for them once more inside the loop.)
+    if constexpr (NT == 1) {
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-        for (int m = 0; m < kM; ++m)
-            asm volatile("" ::"v"(bq[nt][m][0]), "v"(bq[nt][m][1]), "v"(bq[nt][m][2]), "v"(bq[nt][m][3]));
-    issue_half(hidx);
-    if (simple) column_info(false);
-    while (unit < cu_end) {
-        commit_half(hidx);
-        int next_h = hidx + 1, next_unit = unit;
-        if (next_h & 1) {
-            // second half of the same unit
-        } else {
-            next_unit = nth_unit(++unit_no);
-            next_h = 2 * next_unit;
-        }
-        if (next_unit < cu_end) issue_half(next_h);
-        const int pos0 = hidx * 16;
-        if (pos0 <= u_hi) process_half(pos0, !(pos0 >= i_lo && pos0 + 15 <= i_hi));
-        hidx = next_h;
-        unit = next_unit;
+        for (int m = 0; m < kM; ++m) asm volatile("" : "+v"(bq[m]));
     }
+    asm volatile("" ::"v"(page_vec));
+    auto first_rows = [&]() {
+        if (hidx < h_end) {
+            locate_half(hidx);
+            issue_k();
+            issue_v();
+        }
+    };
+    if (q_direct) {
+        first_rows();
+        if (simple) column_info(false);
+    } else {
+        // The query table: one column per wave at a time, lane l holds elements 4 l .. 4 l + 3 =
+        // one half of operand (m = l / 8, k-block (l / 2) % 4).  (The rows are requested behind the
+        // query loads: a wait for those would wait for the rows as well.)
+        if (simple) column_info(false);
+        constexpr int kCols = 16 * NT / kWaves;
+        uint2 raw[kCols];
+#pragma unroll
+        for (int c = 0; c < kCols; ++c) {
+            const int col = wave + c * kWaves;
+            const int t = div_q_group(col, P);
+            const int a = col - t * P.q_group;
+            raw[c] = uint2{0u, 0u};
+            if (4 * lane < HD && t < tile_tokens) {
+                const int tok = min(tok0 + t, B.total_tokens - 1);
+                raw[c] = *reinterpret_cast<const uint2*>(P.q + ((size_t)tok * P.num_q_heads + (size_t)(q_head_base + a)) * HD +
+                                                         4 * lane);
+            }
+        }
+#pragma unroll
+        for (int c = 0; c < kCols; ++c) asm volatile("" ::"v"(raw[c].x), "v"(raw[c].y));
+        first_rows();
+#pragma unroll
+        for (int c = 0; c < kCols; ++c) {
+            const int col = wave + c * kWaves;
+            uint2 packed = raw[c];
+            if constexpr (K8) {
+                float v[4] = {TQ::to_f32((uint16_t)(raw[c].x & 0xFFFFu)), TQ::to_f32((uint16_t)(raw[c].x >> 16)),
+                              TQ::to_f32((uint16_t)(raw[c].y & 0xFFFFu)), TQ::to_f32((uint16_t)(raw[c].y >> 16))};
+                if (rot_q) {
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) v[k] = apply_sign(v[k], 4 * lane + k);
+                    wht256_wave(v, lane);
+                }
+                packed.x = pack_h2(v[0], v[1]);
+                packed.y = pack_h2(v[2], v[3]);
+            }
+            if (4 * lane < HD)
+                *reinterpret_cast<uint2*>(qtab + ((col >> 4) * kM + (lane >> 3)) * 1024 +
+                                          16 * (16 * ((lane >> 1) & 3) + (col & 15)) + 8 * (lane & 1)) = packed;
+        }
+        __syncthreads();
+        if constexpr (NT == 1) {
+#pragma unroll
+            for (int m = 0; m < kM; ++m) bq[m] = *reinterpret_cast<const u4*>(qtab + m * 1024 + 16 * lane);
+        }
+    }
+    while (hidx < h_end) {
+        const int next_h = hidx + kWaves;
+        const bool has_next = next_h < h_end;
+        if (has_next) locate_half(next_h);
+        const int pos0 = hidx * 16;
+        process_half(pos0, !(pos0 >= i_lo && pos0 + 15 <= i_hi), has_next);
+        hidx = next_h;
+    }
+    wait_vm<0>();  // nothing of this wave may still be on its way into LDS when the areas are reused
 
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) l_run[nt] = sum_over_rows(l_run[nt]);
 
     // ---- merge of the waves' states (same scheme and region layout as the TQ4 kernel) ----
-    constexpr int kColStride = kKv16ColStride;
-    constexpr int kRegion = NT * 16 * kColStride;
-    float* mlbuf = reinterpret_cast<float*>(smem + kv16_ml_offset(NT));
-    static_assert(kv16_ml_offset(NT) >= kWaves * kRegion * 4 && kv16_ml_offset(NT) >= kWaves * kKv16Stage,
-                  "(m, l) table must not alias live LDS");
+    // A wave stores one tile of its O as it stands in its own staging area, which nobody else
+    // touches; after a barrier wave c adds up column c (and c + 8) of the eight regions, each weighted
+    // by 2^(m_w - m_tot), one 128-bit piece per lane and region, and brings the sums into element
+    // order through the 1 KB its staging area has left behind the region.
+    constexpr int kColStride = M::kColStride;
+    float* mlbuf = reinterpret_cast<float*>(smem + rows_ml_offset<KVF, HD>(NT));
     if (b == 0) {
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) {
@@ -704,11 +814,11 @@ __device__ __forceinline__ void rows_tile(const AttnParams& P, uint8_t* smem, co
     }
     // finishes column `col` from its sums v (element order of the head dimension) and its state
     auto finish_column = [&](int col, float (&v)[4], float m_col, float l_col) {
-        const int t = fast_div(col, P.q_group);
+        const int t = div_q_group(col, P);
         const int a = col - t * P.q_group;
         const size_t row = (size_t)(tok0 + t) * P.num_q_heads + (size_t)(q_head_base + a);
         if (BAL ? item.n_chunks > 1 : P.max_chunks > 1) {
-            const size_t prow = BAL ? bal_partial_row(item.slot, (int)gridDim.y, kv_sub, col)
+            const size_t prow = BAL ? bal_partial_row(item.slot, (int)gridDim.y, kv_sub, 16 * NT, col)
                                     : row * P.max_chunks + chunk;
             float* dst = P.part_acc + prow * kHeadDim;
             if (4 * lane < HD) *reinterpret_cast<f4*>(dst + 4 * lane) = f4{v[0], v[1], v[2], v[3]};
@@ -727,29 +837,34 @@ __device__ __forceinline__ void rows_tile(const AttnParams& P, uint8_t* smem, co
             store_out_row<TQ, HD>(P, row, lane, v);
         }
     };
-    {
-        static_assert(NT == 1, "the merge below is the one-tile form");
-        // One 16-column tile: a wave's region fits its own staging area, which nobody else touches.
-        // The wave stores its O as it stands, before the barrier; the adding wave weights the eight
-        // regions by 2^(m_w - m_tot), reads one 128-bit piece per lane and region, and brings the
-        // sums into element order through the 1 KB its staging area has left behind the region.
-        static_assert(kRegion * 4 + 1024 <= kKv16Stage, "region and transposition buffer inside the staging area");
-        float* region = reinterpret_cast<float*>(stage);
-        float* tbuf = region + kRegion;
-        if (col_ok[0]) {
-            float* c = region + n * kColStride;
+    float* region = reinterpret_cast<float*>(stage);
+    float* tbuf = region + 16 * kColStride;
+    // (rolled loops: this code runs once per workgroup, and a workgroup of a small batch waits for its
+    // instructions to come from memory)
+#pragma unroll 1
+    for (int nt = 0; nt < NT; ++nt) {
+        if (nt > 0) __syncthreads();  // the previous tile's regions have been read
+        uint32_t live = 0;
 #pragma unroll
-            for (int h = 0; h < kH; ++h)
+        for (int k = 0; k < NT; ++k) {
+            if (k != nt) continue;  // wave-uniform
+            live = ok_mask[k];
+            if (col_ok[k]) {
+                float* c = region + n * kColStride;
 #pragma unroll
-                for (int j = 0; j < 8; ++j) *reinterpret_cast<f4*>(c + ((h * 8 + j) * 4 + b) * 4) = o_acc[0][h][j];
+                for (int h = 0; h < kH; ++h)
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) *reinterpret_cast<f4*>(c + ((h * 8 + j) * 4 + b) * 4) = o_acc[k][h][j];
+            }
         }
         __syncthreads();
+#pragma unroll 1
         for (int col = wave; col < 16; col += kWaves) {
-            if (!((ok_mask[0] >> col) & 1u)) continue;
+            if (!((live >> col) & 1u)) continue;
             float mw[kWaves], lw[kWaves];
 #pragma unroll
             for (int w = 0; w < kWaves; ++w) {
-                const f2 r = *reinterpret_cast<const f2*>(mlbuf + (w * 16 + col) * 2);
+                const f2 r = *reinterpret_cast<const f2*>(mlbuf + (w * NT * 16 + nt * 16 + col) * 2);
                 mw[w] = r[0];
                 lw[w] = r[1];
             }
@@ -762,33 +877,33 @@ __device__ __forceinline__ void rows_tile(const AttnParams& P, uint8_t* smem, co
                 const float wgt = __builtin_amdgcn_exp2f(mw[w] - m_col);
                 l_col += lw[w] * wgt;
                 // (head dimension 128: the upper lanes read what the lower ones read and drop it)
-                tot += *reinterpret_cast<const f4*>(smem + w * kKv16Stage + (col * kColStride + ((4 * lane) & (HD - 1))) * 4) * wgt;
+                tot += *reinterpret_cast<const f4*>(smem + w * M::kStage + (col * kColStride + ((4 * lane) & (HD - 1))) * 4) * wgt;
             }
             *reinterpret_cast<f4*>(tbuf + 4 * lane) = tot;
             float v[4];  // the reads follow the write of the same wave in LDS order
 #pragma unroll
             for (int k = 0; k < 4; ++k) v[k] = tbuf[merge_slot[k]];
-            finish_column(col, v, m_col, l_col);
+            finish_column(nt * 16 + col, v, m_col, l_col);
         }
     }
 }
 
-template <typename TQ, int NT, int KVF, bool VRES, int HD = kHeadDim>
+template <typename TQ, int KVF, bool VRES, int HD = kHeadDim>
 __global__ __launch_bounds__(kKv16Waves * 64, 1) void paged_attn_rows_kernel(const AttnParams P) {
     extern __shared__ __align__(16) uint8_t smem[];
     // (one body per kind of load: a branch around the loads themselves keeps the compiler from
     // scheduling them freely and loses what the hint gains)
     if (P.tiles_by_request != 0 && P.q_subgroups == 1) {  // uniform for the grid
-        rows_tile<TQ, NT, KVF, false, VRES, true, HD>(P, smem, BalItem{});
+        rows_tile<TQ, 1, KVF, false, VRES, true, HD>(P, smem, BalItem{});
     } else {
-        rows_tile<TQ, NT, KVF, false, VRES, false, HD>(P, smem, BalItem{});
+        rows_tile<TQ, 1, KVF, false, VRES, false, HD>(P, smem, BalItem{});
     }
 }
 
-template <typename TQ, int KVF, bool VRES>
+template <typename TQ, int NT, int KVF, bool VRES, bool STREAM, int HD = kHeadDim>
 __global__ __launch_bounds__(kKv16Waves * 64, 1) void paged_attn_rows_balanced_kernel(const AttnParams P) {
     extern __shared__ __align__(16) uint8_t smem[];
-    bal_for_each_piece(P, [&](const BalItem& it) { rows_tile<TQ, 1, KVF, true, VRES>(P, smem, it); });
+    bal_for_each_piece(P, [&](const BalItem& it) { rows_tile<TQ, NT, KVF, true, VRES, STREAM, HD>(P, smem, it); });
 }
 
 }  // namespace w34

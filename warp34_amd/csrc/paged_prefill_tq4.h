@@ -159,7 +159,7 @@ __global__ __launch_bounds__((PC ? 12 : kPfWaves) * 64, 1) void paged_prefill_tq
     }
 
     const int my_col = 16 * wave + n;
-    const int my_t = fast_div(my_col, P.q_group);
+    const int my_t = div_q_group(my_col, P);
     const int my_tok = tok0 + my_t;
     const bool col_ok = my_t < tile_tokens &&
                         (B.valid_token_mask == nullptr || B.valid_token_mask[min(my_tok, B.total_tokens - 1)] != 0);
@@ -186,7 +186,7 @@ __global__ __launch_bounds__((PC ? 12 : kPfWaves) * 64, 1) void paged_prefill_tq
 #pragma unroll
         for (int c = 0; c < 16; ++c) {
             const int col = 16 * wave + c;
-            const int t = fast_div(col, P.q_group);
+            const int t = div_q_group(col, P);
             const int a = col - t * P.q_group;
             const int tok = min(tok0 + t, B.total_tokens - 1);
             const uint16_t* qrow = P.q + ((size_t)tok * P.num_q_heads + (size_t)(q_head_base + a)) * kHeadDim;
@@ -746,6 +746,7 @@ __global__ __launch_bounds__((PC ? 12 : kPfWaves) * 64, 1) void paged_prefill_tq
                     pq_lo[blk][k] = wlo;
                 }
             }
+            settle(pq_lo[0], pq_lo[1], pq_lo[2], pq_lo[3]);
         } else {
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
@@ -769,6 +770,7 @@ __global__ __launch_bounds__((PC ? 12 : kPfWaves) * 64, 1) void paged_prefill_tq
                     pb_l2[h][k] = wlo;
                 }
             }
+            settle(pb_l2[0], pb_l2[1]);
         }
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
@@ -894,7 +896,7 @@ __global__ __launch_bounds__((PC ? 12 : kPfWaves) * 64, 1) void paged_prefill_tq
     for (int c = 0; c < 16; ++c) {
         if (!((ok_mask >> c) & 1u)) continue;
         const int col = 16 * wave + c;
-        const int t = fast_div(col, P.q_group);
+        const int t = div_q_group(col, P);
         const int a = col - t * P.q_group;
         const f4 x = *reinterpret_cast<const f4*>(reg + c * 260 + 4 * lane);
         float o[4] = {x[0], x[1], x[2], x[3]};

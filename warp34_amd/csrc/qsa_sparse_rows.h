@@ -277,6 +277,7 @@ __global__ __launch_bounds__(kKv16Waves * 64, 1) void qsa_sparse_rows_kernel(con
                         a_v[h][j] = u2v{pack_h2(vf[0][j], vf[1][j]), pack_h2(vf[2][j], vf[3][j])};
                     }
                 }
+                if constexpr (VRES) settle(a_vr[h]);
             }
         } else {
             u4 ka[8];

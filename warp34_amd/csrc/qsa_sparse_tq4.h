@@ -427,8 +427,9 @@ __global__ __launch_bounds__(kQsaWaves * 64, 1) void qsa_sparse_tq4_kernel(const
                 }
             }
             __builtin_amdgcn_sched_barrier(0);
-            const u4 ph = {pb_hi[0], pb_hi[1], pb_hi[2], pb_hi[3]};
-            const u4 pl = {pb_lo[0], pb_lo[1], pb_lo[2], pb_lo[3]};
+            u4 ph = {pb_hi[0], pb_hi[1], pb_hi[2], pb_hi[3]};
+            u4 pl = {pb_lo[0], pb_lo[1], pb_lo[2], pb_lo[3]};
+            settle(ph, pl);
 #pragma unroll
             for (int j = 0; j < 8; ++j)
                 o_acc[h][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, a[j]),
