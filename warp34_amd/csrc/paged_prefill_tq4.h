@@ -63,6 +63,55 @@ __device__ __forceinline__ f4 pf_mfma32(h8 a, h8 b, f4 c) {
     }
 }
 
+// Which tile a workgroup takes: the n-th longest of the batch.  A causal tile's length is known up to a
+// tile as (context / tile_tok) + its index in the request; the host knows neither the requests'
+// contexts nor their numbers of new tokens.  In launch order -- requests one after the other, short
+// tiles first -- a batch of 1 to 2 tiles per CU ended with long tiles started late: three requests of
+// 1365, 722 and 1214 new tokens on 1 600 to 1 700 of context (416 tiles of 52 to 94 units, 115 per CU)
+// needed the time of 176 units.  Tiles of equal length go round the requests, which
+// also puts the requests of an even batch on XCDs of their own.  Lane r holds request r: at most 64.
+struct PfTile {
+    int req, tile;
+};
+__device__ __forceinline__ PfTile pf_longest_first(const AttnParams& P, int lane, int rank) {
+    const warp34_attention_batch& B = P.B;
+    int first = 0, count = 0;  // the request's tiles have the lengths first .. first + count - 1
+    if (lane < B.num_reqs && (B.valid_req_mask == nullptr || B.valid_req_mask[lane] != 0)) {
+        const int q_len = B.query_start_loc[lane + 1] - B.query_start_loc[lane];
+        const int ctx = B.context_lens_before != nullptr ? B.context_lens_before[lane] : B.seq_lens_after[lane] - q_len;
+        count = q_len > 0 ? (q_len + P.tok_tile - 1) / P.tok_tile : 0;
+        first = ctx > 0 ? ctx / P.tok_tile : 0;
+    }
+    auto wave_sum = [&](int x) {
+#pragma unroll
+        for (int off = 32; off >= 1; off >>= 1) x += __shfl_xor(x, off, 64);
+        return __builtin_amdgcn_readfirstlane(x);
+    };
+    auto longer = [&](int length) {  // tiles of at least this length
+        return wave_sum(max(0, min(count, first + count - length)));
+    };
+    int lo = 0, hi = first + count;  // longer(lo) > rank, longer(hi) <= rank
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) hi = max(hi, __shfl_xor(hi, off, 64));
+    hi = __builtin_amdgcn_readfirstlane(hi);
+    if (longer(0) <= rank) return PfTile{-1, 0};
+    while (hi - lo > 1) {
+        const int mid = (lo + hi) >> 1;
+        if (longer(mid) > rank) {
+            lo = mid;
+        } else {
+            hi = mid;
+        }
+    }
+    // the (rank - longer(hi))-th request that has a tile of length lo
+    const unsigned long long has = __ballot(first <= lo && lo < first + count);
+    const int nth = rank - longer(hi);
+    const int before = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(has >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)has, 0u));
+    const unsigned long long mine = __ballot(((has >> lane) & 1ull) != 0 && before == nth);
+    const int req = (int)__builtin_ctzll(mine);
+    return PfTile{req, lo - __builtin_amdgcn_readlane(first, req)};
+}
+
 // VF (8-bit rows stored rotated): the value tile holds the codes themselves (exact in fp16) and
 // the block scales go into the probabilities as a high and a low fp16 operand, as for TQ4 rows.
 // fp16(d * code) rounds partly alike across a scale block that holds few distinct codes, and the
@@ -106,9 +155,22 @@ __global__ __launch_bounds__((PC ? 12 : kPfWaves) * 64, 1) void paged_prefill_tq
     const warp34_kv_layer_layout& L = P.L;
     const warp34_attention_batch& B = P.B;
 
-    // ---- tile identification: blockIdx = (tile of the request, kv head x q subgroup, request) ----
-    const int req = (int)blockIdx.z;
-    const int kv_sub = (int)blockIdx.y;
+    // ---- tile identification ----
+    // SPLIT: blockIdx = (tile x part, kv head x q subgroup, 0).  Else the grid holds (tiles of a request, kv
+    // heads x q subgroups, requests) workgroups; taken in launch order they get the tiles longest first,
+    // the heads of a tile next to each other.  More than 64 requests: in grid order.
+    int req = (int)blockIdx.z, kv_sub = (int)blockIdx.y;
+    int tile_x = SPLIT ? (int)blockIdx.x / P.pf_split : (int)(gridDim.x - 1 - blockIdx.x);
+    const int part_x = SPLIT ? (int)blockIdx.x - tile_x * P.pf_split : 0;
+    if (!SPLIT && B.num_reqs <= 64) {
+        const uint32_t at = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
+        const uint32_t rank = at / gridDim.y;
+        kv_sub = (int)(at - rank * gridDim.y);
+        const PfTile t = pf_longest_first(P, lane, (int)rank);
+        if (t.req < 0) return;
+        req = t.req;
+        tile_x = t.tile;
+    }
     const int kv_head = fast_div(kv_sub, P.q_subgroups);
     const int q_head_base = kv_head * P.gqa + (kv_sub - kv_head * P.q_subgroups) * P.q_group;
     if (B.valid_req_mask != nullptr && B.valid_req_mask[req] == 0) return;
@@ -118,8 +180,6 @@ __global__ __launch_bounds__((PC ? 12 : kPfWaves) * 64, 1) void paged_prefill_tq
     const int ctx_before = B.context_lens_before != nullptr ? B.context_lens_before[req]
                                                             : seq_after - (rq_end - rq_start);
     const int tile_tok = P.tok_tile;  // 128 / q_group
-    const int tile_x = SPLIT ? (int)blockIdx.x / P.pf_split : (int)blockIdx.x;
-    const int part_x = SPLIT ? (int)blockIdx.x - tile_x * P.pf_split : 0;
     const int tok0 = rq_start + tile_x * tile_tok;
     if (tok0 >= rq_end || tok0 >= B.total_tokens) return;
     int tile_tokens = rq_end - tok0;
