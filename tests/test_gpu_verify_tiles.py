@@ -49,3 +49,12 @@ def test_rows_verify_rotated_keys_or_values(fmt):
     _check(fmt, DT_F16, 16, [300, 45, 800], [4, 2, 3], 415, scratch=SCRATCH, q_heads=16, xf=XF_WHT256, plain_excess=4e-4)
     _check(fmt, DT_F16, 16, [300, 45, 800], [4, 2, 3], 416, scratch=SCRATCH, q_heads=16, xf=XF_WHT256, v_xf=XF_IDENTITY,
            plain_excess=4e-4)
+
+
+@pytest.mark.parametrize("fmt,dtype", [(FMT_BF16, DT_BF16), (FMT_Q8_0, DT_F16)])
+@pytest.mark.parametrize("n", [4, 5])
+def test_rows_verify_either_side_of_the_grid_rule(fmt, dtype, n):
+    """Four requests of four tokens (8 tiles per kv head) run on the chunk grid, five on the plan; short and
+    longer requests, for which the plan cuts pieces of 4 units and of more."""
+    for seq in ([130, 40, 300, 90, 17][:n], [2600, 900, 4000, 31, 1500][:n]):
+        _check(fmt, dtype, 16, seq, [4] * n, 417, scratch=SCRATCH, q_heads=16)

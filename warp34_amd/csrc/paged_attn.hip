@@ -1775,9 +1775,19 @@ constexpr int kMinUnitsPerChunk = 8;
 // rotates the queries first.
 constexpr int kTq4PieceCost = 32;
 constexpr int kRowsPieceCost = 16;
-// Pieces of more than one column tile leave more records and longer merges: four draft blocks of sixteen
-// tokens (head dimension 128, four kv heads) 25.5 us with pieces from 10 units on, 20.7 from 16, 24.2 from 24.
-constexpr int kMinUnitsPerWidePiece = 16;
+// Smallest piece where a request has several tiles or column tiles.  It counts for short requests only: a
+// layer's step of 12 requests x 4 tokens on 270 to 800 keys (Q8_0) 34.8 us with 16, 28.6 with 8, 26.8 with 4
+// (31.3 on the chunk grid of one-tile workgroups before); at 7K to 19K keys the same.
+constexpr int kMinUnitsPerWidePiece = 4;
+// A batch whose requests have several tiles goes to the chunk grid instead while it has no more 16-column
+// tiles than this per kv head: the plan, the table and the merge of wider pieces cost 4 to 9 us of a call,
+// which reading the keys once for two tiles repays from there on.  Layer steps over Q8_0 pages, chunk
+// grid against plan: 4 requests x 4 tokens (8 tiles) on 2000 keys 23.0 against 26.8 us, on 16000 keys 35.5 against 36.8;
+// 5 x 4 (10 tiles) on 7K to 19K keys 46.2 against 40.2; 12 x 4 on 800 keys 23.4 against 26.8, on 3000 (16 x 4) the same.
+// At head dimension 128 every such batch does: half the bytes per tile.  Three draft blocks of 8 tokens on 2000 keys 17.4
+// against 24.2 us, eight of 16 on 4000 39.7 against 44.2, but four of 16 on 2K to 5K keys 31.8 against 30.9 and
+// twelve of 8 on 8000 55.0 against 50.2.  (Counts of tiles, not lengths: results do not depend on max_seq_len.)
+constexpr int kRowsGridTiles = 8;
 // Split geometry is sized for the layout the path is built for, two kv heads per device: 128
 // chunks (or shares) per kv head.  The counts below depend on the batch and on gqa only, never
 // on local_kv_heads: a rank that holds one kv head of a sharded model computes every row with
@@ -2170,6 +2180,10 @@ static int launch_rows_balanced(const warp34_exec* ex, const warp34_attention_ba
     const int nt = shape.nt, tiles = shape.tiles;
     P.tok_tile = shape.tok_tile;
     if (tiles > kBalMaxTiles || (batch->num_reqs == 1 && nt == 1 && tiles == 1)) return -1;
+    if (nt * tiles > 1) {
+        const long long tiles16 = ((long long)batch->total_tokens * P.q_group + 15) / 16 * P.q_subgroups;
+        if (HD != kHeadDim || tiles16 <= kRowsGridTiles) return -1;
+    }
     // fewer shares where the scratch cannot hold the records of all of them
     const long long entries = (long long)batch->num_reqs * tiles;
     const size_t slot_bytes = partial_bytes((long long)kv_subs * 16 * nt, 1), table_bytes = (size_t)batch->total_tokens * 16;
@@ -2200,7 +2214,7 @@ static int launch_rows_balanced(const warp34_exec* ex, const warp34_attention_ba
         if (rc) return rc;
         return launch_balanced_merge<TQ, HD>(P, kv_subs, 1.0f, stream);
     };
-    if constexpr (!VRES) {
+    if constexpr (!VRES && HD == kHeadDim) {
         if (nt == 2) return launch(std::integral_constant<int, 2>{});
     }
     return launch(std::integral_constant<int, 1>{});

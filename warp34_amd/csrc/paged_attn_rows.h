@@ -155,12 +155,11 @@ __device__ __forceinline__ void lds_load_half(uint32_t voffset, const uint8_t* s
 // KVF is the storage format of both slabs.  16-bit pages: TQ doubles as the storage type (F16
 // query/output over FP16 pages, BF16 over BF16 pages).  8-bit pages: the MFMAs run in fp16 and
 // a BF16 query is converted once.
-// NT: 16-column tiles per workgroup.  A verify step or a draft block has more than 16 query columns
-// per kv head; with two tiles the keys are read, and 8-bit codes widened, once for 32 columns.  The
-// accumulators take 64 NT registers at head dimension 256 (32 NT at 128), so the query operands stay in
-// LDS for NT = 2 and are read again for every half.  (Four tiles at head dimension 128: the merge of
-// the eight waves, 2 us per tile, outweighs the keys read once more: 24.8 against 20.7 us for four draft
-// blocks of sixteen tokens over 1K to 9K keys.)
+// NT: 16-column tiles per workgroup.  A verify step has more than 16 query columns per kv head; with two
+// tiles the keys are read, and 8-bit codes widened, once for 32 columns.  The accumulators take 64 NT
+// registers, so the query operands stay in LDS for NT = 2 and are read again for every half.  Head
+// dimension 256 only: at 128 the merge of the waves (2 us per tile) outweighs the keys read once more
+// (launch_rows_balanced).
 // Bound: one workgroup per CU streams about 20 bytes per ns, what the memory delivers; below some 100 MB the
 // launch is the chain arguments - plan - block table - first rows (7 us to the first product), the
 // streaming, and the merge of the waves (2.3 us per tile).
@@ -181,7 +180,7 @@ __device__ __forceinline__ void rows_tile(const AttnParams& P, uint8_t* smem, co
     constexpr bool K8 = M::k8;
     constexpr bool FP8 = M::kFp8;
     static_assert(HD == 256 || (HD == 128 && !K8), "head dimension 128: 16-bit rows only");
-    static_assert(NT == 1 || BAL, "several column tiles: balanced form only");
+    static_assert(NT == 1 || (BAL && HD == 256), "several column tiles: balanced form, head dimension 256");
     constexpr int kM = HD / 32;   // QK operands (32 elements each) per row
     constexpr int kH = HD / 128;  // 128-element halves of a row
     static_assert(K8 || KVF == TQ::kStorageFormat, "16-bit pages are read in the query type");
