@@ -2716,13 +2716,16 @@ static size_t scratch_bytes_for(int local_kv_heads, int total_tokens, int num_re
         if (bal > bytes) bytes = bal;
     }
     // verify batches: several column tiles per workgroup, several tiles per request (the query tokens
-    // taken as spread evenly over the requests)
-    const int q_len = max_q_len > 0 ? max_q_len : (total_tokens + num_reqs - 1) / num_reqs;
-    const BalShape shape = balanced_shape(q_len, q_group, 2);
-    if (shape.tiles <= kBalMaxTiles) {
-        const size_t prows = bal_partial_row(balanced_groups(q_subgroups) + num_reqs * shape.tiles, kv_subs, 0, 16 * shape.nt, 0);
-        const size_t bal = partial_bytes((long long)prows, 1) + (size_t)total_tokens * 16;
-        if (bal > bytes) bytes = bal;
+    // taken as spread evenly over the requests; no plan without a request)
+    if (num_reqs >= 1) {
+        const int q_len = max_q_len > 0 ? max_q_len : (int)(((long long)total_tokens + num_reqs - 1) / num_reqs);
+        const BalShape shape = balanced_shape(q_len, q_group, 2);
+        if (shape.tiles <= kBalMaxTiles) {
+            const size_t prows =
+                bal_partial_row(balanced_groups(q_subgroups) + num_reqs * shape.tiles, kv_subs, 0, 16 * shape.nt, 0);
+            const size_t bal = partial_bytes((long long)prows, 1) + (size_t)total_tokens * 16;
+            if (bal > bytes) bytes = bal;
+        }
     }
     return bytes;
 }
