@@ -37,10 +37,12 @@ def test_rows_verify_many_requests(fmt, dtype, n):
     _check(fmt, dtype, 64, seq, [1 + (i % 6) for i in range(n)], 413, scratch=SCRATCH, q_heads=16)
 
 
-@pytest.mark.parametrize("scratch", [2 << 20, 8 << 20])
+@pytest.mark.parametrize("scratch", [2 << 20, 7 << 20, 8 << 20])
 def test_rows_verify_small_scratch(scratch):
-    """Fewer pieces where the scratch cannot hold the records of all of them, or the plain form."""
+    """20 requests in 8 MiB: 106 of the plan's 128 shares.  7 MiB would hold 90: the chunk grid.  Three requests are
+    on the grid with any scratch."""
     _check(FMT_FP8, DT_F16, 64, [3000, 900, 2000], [4, 4, 4], 414, scratch=scratch, q_heads=16)
+    _check(FMT_FP8, DT_F16, 64, [30 + 61 * ((i * 7) % 20) for i in range(20)], [4] * 20, 419, scratch=scratch, q_heads=16)
 
 
 @pytest.mark.parametrize("fmt", [FMT_FP8, FMT_Q8_0])
@@ -58,3 +60,23 @@ def test_rows_verify_either_side_of_the_grid_rule(fmt, dtype, n):
     longer requests, for which the plan cuts pieces of 4 units and of more."""
     for seq in ([130, 40, 300, 90, 17][:n], [2600, 900, 4000, 31, 1500][:n]):
         _check(fmt, dtype, 16, seq, [4] * n, 417, scratch=SCRATCH, q_heads=16)
+
+
+@pytest.mark.parametrize("fmt,dtype", [(FMT_Q8_0, DT_F16), (FMT_BF16, DT_BF16)])
+@pytest.mark.parametrize("n,q", [(200, 1), (235, 1), (60, 4), (110, 4)])
+def test_rows_large_batches_in_8mib_keep_a_workgroup_per_tile(fmt, dtype, n, q):
+    """8 MiB hold the records of 52, 17, 66 or 16 shares of these batches: they run as one workgroup per tile, the
+    scratch stays untouched and the bits are those of a call without scratch."""
+    import gpu_harness as G
+    from cases import make_case
+
+    seq = [10 + 23 * ((i * 5) % 7) for i in range(n)]
+    pool, bt, k, v, qb, aq, ctx = make_case(fmt, 16, seq, [q] * n, 418, dtype, q_heads=16)
+    hb = oracle.HostBatch(aq, seq, bt, context_lens_before=ctx)
+    dpool = G.DevPool(pool)
+    dpool.upload()
+    rc0, plain, _ = G.dev_attention(dpool, hb, qb, dtype, 16)
+    rc1, got, ws = G.dev_attention(dpool, hb, qb, dtype, 16, scratch_bytes=8 << 20)
+    assert rc0 == 0 and rc1 == 0
+    assert bool((ws == 0x5A).all()), "the scratch was used"
+    assert got.tobytes() == plain.tobytes()

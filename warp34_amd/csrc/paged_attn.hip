@@ -2184,13 +2184,19 @@ static int launch_rows_balanced(const warp34_exec* ex, const warp34_attention_ba
         const long long tiles16 = ((long long)batch->total_tokens * P.q_group + 15) / 16 * P.q_subgroups;
         if (HD != kHeadDim || tiles16 <= kRowsGridTiles) return -1;
     }
-    // fewer shares where the scratch cannot hold the records of all of them
+    // Fewer shares where the scratch cannot hold the records of all of them, down to three quarters; with less
+    // room the chunk grid, whose workgroups grow with the batch, leaves fewer compute units idle.  8 MiB, two kv
+    // heads, Q8_0, chunk grid against plan: 150 decode requests (102 shares) of 1000 keys 45.4 against 46.3 us,
+    // of 1K to 9K 194 against 140; 175 (77 shares) 46 against 61, 202 against 187; 200 (52 shares) 47 against 93, 226 against 296;
+    // 235 (17 shares) 54 against 308, 262 against 1046.  20 requests x 4 tokens (106 shares) on 300 to 3000 keys 29.2 against 31.1,
+    // on 3K to 16K 93 against 60; 60 x 4 (66 shares) on 300 to 3000 keys 54 against 66.
     const long long entries = (long long)batch->num_reqs * tiles;
     const size_t slot_bytes = partial_bytes((long long)kv_subs * 16 * nt, 1), table_bytes = (size_t)batch->total_tokens * 16;
     if (ex->scratch_size < table_bytes) return -1;
     const long long room = (long long)((ex->scratch_size - table_bytes) / slot_bytes) - entries;
-    const int groups = (int)(room < balanced_groups(P.q_subgroups) ? room : balanced_groups(P.q_subgroups));
-    if (groups < 16) return -1;
+    const int all_groups = balanced_groups(P.q_subgroups);
+    const int groups = (int)(room < all_groups ? room : all_groups);
+    if (groups < 1 || 4 * groups < 3 * all_groups) return -1;
     const size_t prows = (size_t)(groups + entries) * kv_subs * 16 * nt;
     P.piece_cost = kRowsPieceCost;
     if (nt * tiles > 1) P.min_upc = kMinUnitsPerWidePiece;
