@@ -310,8 +310,10 @@ int warp34_qsa_sparse_paged_attn_hadamard_f16(
  * >= 8 MiB (op_paged_attn.cu:1301-1304); provided so a host can size ex->scratch. */
 size_t warp34_paged_attention_scratch_bytes(int total_tokens, int num_q_heads, int max_seq_len);
 /* The same for a known layout and request count: the exact figure the launchers use (the form
- * above does not know local_kv_heads and returns the largest need over all layouts).
- * num_reqs < 0: unknown, total_tokens is assumed.  No counterpart in the reference. */
+ * above does not know local_kv_heads and returns the largest need over all layouts), with the query
+ * tokens taken as spread evenly over the requests (a batch in which one request has many more than the
+ * others may run with fewer shares).  num_reqs < 0: unknown, total_tokens is assumed.  No counterpart
+ * in the reference. */
 size_t warp34_paged_attention_scratch_bytes_for_layout(const warp34_kv_layer_layout* layout, int total_tokens,
                                                        int num_reqs, int num_q_heads, int max_seq_len);
 

@@ -80,3 +80,25 @@ def test_rows_large_batches_in_8mib_keep_a_workgroup_per_tile(fmt, dtype, n, q):
     assert rc0 == 0 and rc1 == 0
     assert bool((ws == 0x5A).all()), "the scratch was used"
     assert got.tobytes() == plain.tobytes()
+
+
+@pytest.mark.parametrize("fmt,dtype", [(FMT_Q8_0, DT_F16), (FMT_BF16, DT_BF16)])
+@pytest.mark.parametrize("n,q", [(1, 1), (1, 4), (5, 4), (3, 16), (40, 1), (40, 4)])
+def test_rows_scratch_of_the_queried_size_splits_fully(fmt, dtype, n, q):
+    """The bits of a call with the scratch the query names are those of a call with 64 MiB."""
+    import ctypes as C
+
+    import gpu_harness as G
+    from cases import make_case
+
+    seq = [16 + 131 * ((i * 5) % 9) for i in range(n)]
+    pool, bt, k, v, qb, aq, ctx = make_case(fmt, 16, seq, [q] * n, 420, dtype, q_heads=16)
+    hb = oracle.HostBatch(aq, seq, bt, context_lens_before=ctx)
+    dpool = G.DevPool(pool)
+    dpool.upload()
+    L = dpool.layout()
+    need = G.lib().warp34_paged_attention_scratch_bytes_for_layout(C.byref(L), n * q, n, 16, max(seq))
+    rc0, want, _ = G.dev_attention(dpool, hb, qb, dtype, 16, scratch_bytes=SCRATCH)
+    rc1, got, _ = G.dev_attention(dpool, hb, qb, dtype, 16, scratch_bytes=need)
+    assert rc0 == 0 and rc1 == 0
+    assert got.tobytes() == want.tobytes()

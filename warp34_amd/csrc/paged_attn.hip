@@ -2153,37 +2153,47 @@ static int launch_tq4(const warp34_exec* ex, const warp34_kv_layer_layout* layou
 // Most tiles per request that the balanced plan takes: with more, the 128-row tile kernel or one
 // workgroup per tile is the better shape.
 constexpr int kBalMaxTiles = 16;
-// Column tiles per workgroup (nt) and tiles per request of a balanced batch whose requests have up to
-// q_len query tokens: as many column tiles as a request's query columns fill, up to max_nt.
+// Column tiles per workgroup (nt) and tiles per request of a balanced batch over row-format pages whose
+// requests have up to q_len query tokens; no tiles: the batch is not for the plan.  Two column tiles where a
+// request has more than 16 query columns; rotated 8-bit values (a second value operand: accumulator
+// registers) stay with one, and head dimension 128 takes the plan with one tile per request only.
 struct BalShape {
     int nt, tok_tile, tiles;
 };
-static BalShape balanced_shape(int q_len, int q_group, int max_nt) {
-    const long long cols = (long long)q_len * q_group;
+static BalShape rows_balanced_shape(int num_reqs, int total_tokens, int q_len, int q_group, int q_subgroups, bool vres,
+                                    int head_dim) {
+    const BalShape none{0, 0, 0};
+    if (num_reqs < 1 || q_len < 1 || total_tokens > 65535) return none;
     BalShape s;
-    s.nt = cols > 16 && max_nt >= 2 ? 2 : 1;
+    s.nt = (long long)q_len * q_group > 16 && !vres && head_dim == kHeadDim ? 2 : 1;
     s.tok_tile = 16 * s.nt / q_group;
-    s.tiles = (q_len + s.tok_tile - 1) / s.tok_tile;
+    const long long tiles = ((long long)q_len + s.tok_tile - 1) / s.tok_tile;
+    if (tiles > kBalMaxTiles || (num_reqs == 1 && s.nt == 1 && tiles == 1)) return none;
+    s.tiles = (int)tiles;
+    if (s.nt * s.tiles > 1) {
+        const long long tiles16 = ((long long)total_tokens * q_group + 15) / 16 * q_subgroups;
+        if (head_dim != kHeadDim || tiles16 <= kRowsGridTiles) return none;
+    }
     return s;
+}
+// rotated 8-bit value rows
+static bool rows_vres(const warp34_kv_layer_layout* l) {
+    return (l->v_format == WARP34_KV_FORMAT_FP8_E4M3 || l->v_format == WARP34_KV_FORMAT_Q8_0) &&
+           l->v_transform == WARP34_KV_TRANSFORM_RADEMACHER_WHT256;
 }
 
 // Balanced decode / verify over row-format pages; -1: the batch is not for it.
-// Two column tiles where a request has more than 16 query columns; rotated 8-bit values (a second value
-// operand) stay with one (accumulator registers).
 template <typename TQ, int KVF, bool VRES, int HD>
 static int launch_rows_balanced(const warp34_exec* ex, const warp34_attention_batch* batch, AttnParams P, int kv_subs,
                                 int force_single, hipStream_t stream) {
-    if (force_single || batch->max_q_len <= 0 || batch->sliding_window > 0 || batch->valid_token_mask != nullptr ||
-        ex->scratch_ptr == 0 || (ex->scratch_ptr & 15u) != 0u || batch->total_tokens > 65535)
+    if (force_single || batch->sliding_window > 0 || batch->valid_token_mask != nullptr || ex->scratch_ptr == 0 ||
+        (ex->scratch_ptr & 15u) != 0u)
         return -1;
-    const BalShape shape = balanced_shape(batch->max_q_len, P.q_group, VRES ? 1 : 2);
+    const BalShape shape =
+        rows_balanced_shape(batch->num_reqs, batch->total_tokens, batch->max_q_len, P.q_group, P.q_subgroups, VRES, HD);
     const int nt = shape.nt, tiles = shape.tiles;
+    if (tiles < 1) return -1;
     P.tok_tile = shape.tok_tile;
-    if (tiles > kBalMaxTiles || (batch->num_reqs == 1 && nt == 1 && tiles == 1)) return -1;
-    if (nt * tiles > 1) {
-        const long long tiles16 = ((long long)batch->total_tokens * P.q_group + 15) / 16 * P.q_subgroups;
-        if (HD != kHeadDim || tiles16 <= kRowsGridTiles) return -1;
-    }
     // Fewer shares where the scratch cannot hold the records of all of them, down to three quarters; with less
     // room the chunk grid, whose workgroups grow with the batch, leaves fewer compute units idle.  8 MiB, two kv
     // heads, Q8_0, chunk grid against plan: 150 decode requests (102 shares) of 1000 keys 45.4 against 46.3 us,
@@ -2479,7 +2489,7 @@ static int attention_entry(const warp34_exec* ex, const warp34_kv_layer_layout* 
                                (long long)batch->total_tokens * num_q_heads >= 128ll * kPfRows;
         if ((force_tile || (!force && many_rows)) && prefill_tq4_applicable(layout, batch, num_q_heads))
             return launch_prefill_tq4<TQ, WARP34_KV_FORMAT_FP8_E4M3>(ex, layout, batch, q, out, num_q_heads, gate);
-        if (layout->v_transform == WARP34_KV_TRANSFORM_RADEMACHER_WHT256)
+        if (rows_vres(layout))
             return launch_rows<TQ, WARP34_KV_FORMAT_FP8_E4M3, true>(ex, layout, batch, q, out, num_q_heads, force_single, gate);
         return launch_rows<TQ, WARP34_KV_FORMAT_FP8_E4M3>(ex, layout, batch, q, out, num_q_heads, force_single, gate);
     }
@@ -2489,7 +2499,7 @@ static int attention_entry(const warp34_exec* ex, const warp34_kv_layer_layout* 
                                (long long)batch->total_tokens * num_q_heads >= 128ll * kPfRows;
         if ((force_tile || (!force && many_rows)) && prefill_tq4_applicable(layout, batch, num_q_heads))
             return launch_prefill_tq4<TQ, WARP34_KV_FORMAT_Q8_0>(ex, layout, batch, q, out, num_q_heads, gate);
-        if (layout->v_transform == WARP34_KV_TRANSFORM_RADEMACHER_WHT256)
+        if (rows_vres(layout))
             return launch_rows<TQ, WARP34_KV_FORMAT_Q8_0, true>(ex, layout, batch, q, out, num_q_heads, force_single, gate);
         return launch_rows<TQ, WARP34_KV_FORMAT_Q8_0>(ex, layout, batch, q, out, num_q_heads, force_single, gate);
     }
@@ -2674,15 +2684,15 @@ extern "C" int warp34_paged_attention_f16_force_kernel_for_test(
 }
 
 // Scratch that lets a batch split fully, computed the way the launchers compute it.
-// q_group / q_subgroups as in launch_tq4 / launch_rows; local_kv_heads <= 0: not known, take the
-// largest need over all layouts with this many q heads.
-static size_t scratch_bytes_for(int local_kv_heads, int total_tokens, int num_reqs, int num_q_heads,
-                                int max_seq_len, int max_q_len = 0) {
+// q_group / q_subgroups as in launch_tq4 / launch_rows; layout null: not known, take the largest need over
+// all layouts with this many q heads.  num_reqs < 0: not known, as many as tokens.
+static size_t scratch_bytes_for(const warp34_kv_layer_layout* layout, int total_tokens, int num_reqs, int num_q_heads,
+                                int max_seq_len) {
     if (total_tokens <= 0 || num_q_heads <= 0) return 0;
     int q_group = 1, q_subgroups = 1, kv_subs = num_q_heads;  // the bound when the layout is unknown
     int tok_tile = 16;
-    if (local_kv_heads > 0 && num_q_heads % local_kv_heads == 0) {
-        const int gqa = num_q_heads / local_kv_heads;
+    if (layout && layout->local_kv_heads > 0 && num_q_heads % layout->local_kv_heads == 0) {
+        const int gqa = num_q_heads / layout->local_kv_heads;
         q_group = gqa;
         if (q_group > 16) {
             for (int d = 16; d >= 1; --d)
@@ -2692,10 +2702,10 @@ static size_t scratch_bytes_for(int local_kv_heads, int total_tokens, int num_re
                 }
         }
         q_subgroups = gqa / q_group;
-        kv_subs = local_kv_heads * q_subgroups;
+        kv_subs = layout->local_kv_heads * q_subgroups;
         tok_tile = 16 / q_group < 1 ? 1 : 16 / q_group;
     }
-    const int tiles = (total_tokens + tok_tile - 1) / tok_tile;
+    const int tiles = (int)(((long long)total_tokens + tok_tile - 1) / tok_tile);
     long long want = kTargetWorkgroupsPerHead / ((long long)tiles * q_subgroups);
     if (want > kMaxChunksCap) want = kMaxChunksCap;
     if (max_seq_len > 0) {
@@ -2704,47 +2714,47 @@ static size_t scratch_bytes_for(int local_kv_heads, int total_tokens, int num_re
         if (bound < want) want = bound;
     }
     size_t bytes = want >= 2 ? partial_bytes((long long)total_tokens * num_q_heads, (int)want) : 0;
-    // verify batches over long contexts may take the shared-prefix pass: its partial slots sit
+    // TQ4 verify batches over long contexts may take the shared-prefix pass: its partial slots sit
     // behind the split-K ones, and a header behind the records
-    if (want >= 2 && total_tokens >= 16 && (num_reqs < 0 || num_reqs >= 4) && max_seq_len >= 8 * kSpMinTokens &&
-        (max_q_len <= 0 || (max_q_len >= 2 && max_q_len <= kPfRows / q_group)) && (q_group & (q_group - 1)) == 0) {
+    if ((!layout || is_tq4(layout)) && want >= 2 && total_tokens >= 16 && (num_reqs < 0 || num_reqs >= 4) &&
+        max_seq_len >= 8 * kSpMinTokens && (q_group & (q_group - 1)) == 0) {
         const int parts = shared_prefix_parts(total_tokens, q_group, q_subgroups);
         if ((int)want + parts <= kMergeGroups * kMergeMaxPerGroup)
             bytes = partial_bytes((long long)total_tokens * num_q_heads, (int)want + parts) + sizeof(SpHeader);
     }
-    // balanced decode: (shares + requests) partial slots of 16 columns per (kv head, q subgroup)
-    // and the per-token table
-    // (only batches in which no request has more than one tile take it; max_q_len <= 0: not known)
+    // The balanced plan: (shares + entries) partial slots of 16 columns per column tile and (kv head, q
+    // subgroup), and the per-token table.
+    const auto plan = [&](long long entries, int nt) {
+        const size_t slots = (size_t)(balanced_groups(q_subgroups) + entries) * kv_subs * 16 * nt;
+        const size_t need = partial_bytes((long long)slots, 1) + (size_t)total_tokens * 16;
+        if (need > bytes) bytes = need;
+    };
     if (num_reqs < 0 || num_reqs > total_tokens) num_reqs = total_tokens;
-    if (num_reqs >= 2 && max_q_len <= tok_tile) {
-        const size_t prows = bal_partial_row(balanced_groups(q_subgroups) + num_reqs, kv_subs, 0, 16, 0);
-        const size_t bal = partial_bytes((long long)prows, 1) + (size_t)total_tokens * 16;
-        if (bal > bytes) bytes = bal;
-    }
-    // verify batches: several column tiles per workgroup, several tiles per request (the query tokens
-    // taken as spread evenly over the requests; no plan without a request)
-    if (num_reqs >= 1) {
-        const int q_len = max_q_len > 0 ? max_q_len : (int)(((long long)total_tokens + num_reqs - 1) / num_reqs);
-        const BalShape shape = balanced_shape(q_len, q_group, 2);
-        if (shape.tiles <= kBalMaxTiles) {
-            const size_t prows =
-                bal_partial_row(balanced_groups(q_subgroups) + num_reqs * shape.tiles, kv_subs, 0, 16 * shape.nt, 0);
-            const size_t bal = partial_bytes((long long)prows, 1) + (size_t)total_tokens * 16;
-            if (bal > bytes) bytes = bal;
-        }
+    // one tile per request (decode steps; not with more tokens than that many tiles hold)
+    if (num_reqs >= 2 && total_tokens <= 65535 && total_tokens <= (long long)num_reqs * tok_tile) plan(num_reqs, 1);
+    if (!layout) {
+        // one q head per kv head: two column tiles from 17 tokens per request on, at most an entry per 16 tokens
+        if (total_tokens > 16 * kRowsGridTiles && total_tokens <= 65535) plan(total_tokens / 16, 2);
+    } else if (is_kv16(layout, WARP34_KV_FORMAT_FP16) || is_kv16(layout, WARP34_KV_FORMAT_BF16) ||
+               is_kv8(layout, WARP34_KV_FORMAT_FP8_E4M3) || is_kv8(layout, WARP34_KV_FORMAT_Q8_0)) {
+        // row formats: several tiles or column tiles per request (the tokens taken as spread evenly)
+        const int q_len = num_reqs > 0 ? (int)(((long long)total_tokens + num_reqs - 1) / num_reqs) : 0;
+        const BalShape shape = rows_balanced_shape(num_reqs, total_tokens, q_len, q_group, q_subgroups, rows_vres(layout),
+                                                   layout->head_dim);
+        if (shape.nt * shape.tiles > 1) plan((long long)num_reqs * shape.tiles, shape.nt);
     }
     return bytes;
 }
 
 extern "C" size_t warp34_paged_attention_scratch_bytes(int total_tokens, int num_q_heads, int max_seq_len) {
-    return scratch_bytes_for(0, total_tokens, -1, num_q_heads, max_seq_len);
+    return scratch_bytes_for(nullptr, total_tokens, -1, num_q_heads, max_seq_len);
 }
 
 extern "C" size_t warp34_paged_attention_scratch_bytes_for_layout(const warp34_kv_layer_layout* layout,
                                                                   int total_tokens, int num_reqs, int num_q_heads,
                                                                   int max_seq_len) {
     if (!layout) return 0;
-    return scratch_bytes_for(layout->local_kv_heads, total_tokens, num_reqs, num_q_heads, max_seq_len);
+    return scratch_bytes_for(layout, total_tokens, num_reqs, num_q_heads, max_seq_len);
 }
 
 // op_qsa.cu:1711-1730
