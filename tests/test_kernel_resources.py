@@ -1,0 +1,42 @@
+"""What the built library's kernel descriptors say: the row-format attention kernels keep everything in registers.
+A reload from scratch memory waits for the row loads in flight as well, which the kernels place their own waits for."""
+import os
+import re
+import struct
+import subprocess
+
+import pytest
+
+READELF = "/opt/rocm/llvm/bin/llvm-readelf"
+
+
+def kernel_scratch_bytes(tmp_path):
+    """{kernel name: bytes of scratch memory per lane} of the gfx950 code objects inside the library."""
+    from warp34_amd import ffi
+
+    data = open(ffi.LIB_PATH, "rb").read()
+    found, at, n = {}, data.find(b"__CLANG_OFFLOAD_BUNDLE__"), 0
+    while at >= 0:
+        pos = at + 32
+        for _ in range(struct.unpack_from("<Q", data, at + 24)[0]):
+            offset, size, name_len = struct.unpack_from("<QQQ", data, pos)
+            triple = data[pos + 24:pos + 24 + name_len]
+            pos += 24 + name_len
+            if b"gfx950" not in triple or not size:
+                continue
+            path = os.path.join(str(tmp_path), "%d.o" % n)
+            n += 1
+            with open(path, "wb") as f:
+                f.write(data[at + offset:at + offset + size])
+            notes = subprocess.run([READELF, "--notes", path], stdout=subprocess.PIPE, text=True, check=True).stdout
+            for name, scratch in re.findall(r"\.name: +(_Z\S+)\n(?:.*\n)*?.*\.private_segment_fixed_size: (\d+)", notes):
+                found[name] = int(scratch)
+        at = data.find(b"__CLANG_OFFLOAD_BUNDLE__", at + 24)
+    return found
+
+
+@pytest.mark.skipif(not os.path.exists(READELF), reason="no llvm-readelf")
+def test_row_format_kernels_do_not_spill(tmp_path):
+    kernels = {k: v for k, v in kernel_scratch_bytes(tmp_path).items() if "paged_attn_rows" in k}
+    assert len(kernels) >= 20, sorted(kernels)
+    assert {k: v for k, v in kernels.items() if v} == {}

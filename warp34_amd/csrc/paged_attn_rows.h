@@ -189,7 +189,12 @@ __device__ __forceinline__ void rows_tile(const AttnParams& P, uint8_t* smem, co
     constexpr int kWaves = kKv16Waves;
     constexpr int kRowBytes = M::kRowBytes;
 
-    const int tid = (int)threadIdx.x;
+    int tid = (int)threadIdx.x;
+    // The next piece works its lane values out again: the compiler kept addresses and the sign bits of the query
+    // rotation in registers across the pieces, which the loop over the keys then did not have.  Q8_0 with two
+    // column tiles: 256 registers and 10 spilled, reloaded behind the first row loads and waiting for them;
+    // now 246 and none, 20 requests x 4 tokens on 3K to 16K keys 57.1 -> 52.5 us.
+    if constexpr (BAL) asm volatile("" : "+v"(tid));
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n = lane & 15;
@@ -268,8 +273,8 @@ __device__ __forceinline__ void rows_tile(const AttnParams& P, uint8_t* smem, co
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
         const int tok = tok0 + div_q_group(nt * 16 + n, P);
-        tok_ok[nt] = tok < B.total_tokens &&
-                     (B.valid_token_mask == nullptr || B.valid_token_mask[min(tok, B.total_tokens - 1)] != 0);
+        tok_ok[nt] = tok < B.total_tokens && (BAL || B.valid_token_mask == nullptr ||
+                                              B.valid_token_mask[min(tok, B.total_tokens - 1)] != 0);
     }
     int tile_tokens = rq_end - tok0;
     if (tile_tokens > P.tok_tile) tile_tokens = P.tok_tile;
@@ -289,7 +294,8 @@ __device__ __forceinline__ void rows_tile(const AttnParams& P, uint8_t* smem, co
         col_ok[nt] = false;
         ok_mask[nt] = 0u;
     }
-    const bool simple = B.valid_token_mask == nullptr && B.sliding_window <= 0;
+    // (a balanced batch has neither, see launch_rows_balanced)
+    const bool simple = BAL || (B.valid_token_mask == nullptr && B.sliding_window <= 0);
     auto column_info = [&](bool accumulate) {
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) {
@@ -301,7 +307,7 @@ __device__ __forceinline__ void rows_tile(const AttnParams& P, uint8_t* smem, co
             int mx = (B.mask_mode == WARP34_ATTN_MASK_NONCAUSAL_WINDOW) ? seq_after - 1 : ctx_before + q_off;
             if (mx >= seq_after) mx = seq_after - 1;
             int mn = 0;
-            if (B.sliding_window > 0) mn = max(0, ctx_before + q_off - B.sliding_window + 1);
+            if (!BAL && B.sliding_window > 0) mn = max(0, ctx_before + q_off - B.sliding_window + 1);
             col_ok[nt] = ok;
             col_lo[nt] = ok ? mn : 0;
             col_hi[nt] = ok ? mx : -1;
@@ -597,7 +603,7 @@ __device__ __forceinline__ void rows_tile(const AttnParams& P, uint8_t* smem, co
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     const int pos = pos0 + 4 * b + i;
-                    const bool vis = col_ok[nt] && pos >= col_lo[nt] && pos <= col_hi[nt];
+                    const bool vis = (BAL || pos >= col_lo[nt]) && pos <= col_hi[nt];  // (dead columns: col_hi = -1)
                     sc[i] = vis ? sc[i] : kNegBig;
                 }
             }
@@ -848,7 +854,7 @@ __device__ __forceinline__ void rows_tile(const AttnParams& P, uint8_t* smem, co
         for (int k = 0; k < NT; ++k) {
             if (k != nt) continue;  // wave-uniform
             live = ok_mask[k];
-            if (col_ok[k]) {
+            if ((live >> n) & 1u) {
                 float* c = region + n * kColStride;
 #pragma unroll
                 for (int h = 0; h < kH; ++h)
