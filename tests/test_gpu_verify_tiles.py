@@ -102,3 +102,49 @@ def test_rows_scratch_of_the_queried_size_splits_fully(fmt, dtype, n, q):
     rc1, got, _ = G.dev_attention(dpool, hb, qb, dtype, 16, scratch_bytes=need)
     assert rc0 == 0 and rc1 == 0
     assert got.tobytes() == want.tobytes()
+
+
+@pytest.mark.parametrize("fmt,dtype", ROWS)
+@pytest.mark.parametrize("seq,q", [([200, 31, 224, 17, 9], [4, 4, 4, 4, 4]), ([40 + 9 * (i % 20) for i in range(20)], [4] * 20),
+                                   ([60 + 41 * (i % 5) for i in range(64)], [3] * 64), ([224, 130, 33], [16, 16, 9])])
+def test_rows_short_batches_do_not_depend_on_the_sequence_bound(fmt, dtype, seq, q):
+    """No request above 224 keys: on the chunk grid where the host's bound says so, as pieces of 16 columns where the
+    plan finds it out; the same bits, and the oracle's answer."""
+    import gpu_harness as G
+    from cases import make_case
+
+    pool, bt, k, v, qb, aq, ctx = make_case(fmt, 16, seq, q, 421, dtype, q_heads=16)
+    hb = oracle.HostBatch(aq, seq, bt, context_lens_before=ctx)
+    dpool = G.DevPool(pool)
+    dpool.upload()
+    outs = []
+    for bound in (None, 224, 225, 4096, 131072):
+        rc, out, _ = G.dev_attention(dpool, hb, qb, dtype, 16, scratch_bytes=SCRATCH, max_seq_len=bound)
+        assert rc == 0
+        outs.append(out)
+    assert all(o.tobytes() == outs[0].tobytes() for o in outs[1:])
+    want = oracle.paged_attention(pool, hb, qb, dtype, 16, n_threads=4)
+    G.assert_close(outs[0], dtype, want, what="short batch", scale=G.channel_scale(v, dtype, hb, 16))
+
+
+@pytest.mark.parametrize("fmt,dtype", [(FMT_Q8_0, DT_F16), (FMT_BF16, DT_BF16)])
+def test_rows_short_batches_with_idle_requests(fmt, dtype):
+    """20 requests of up to 900 keys, more than 64 tiles of 16 columns among them, masked requests left untouched;
+    and the same lengths eight times over, which is no short batch any more."""
+    import gpu_harness as G
+    from cases import make_case
+
+    for scale, n, q in ((1, 20, 4), (8, 20, 4), (1, 30, 6), (1, 21, 9)):
+        seq = [16 + scale * (37 + 97 * ((i * 7) % 9)) for i in range(n)]
+        mask = [0 if i % 6 == 5 else 1 for i in range(n)]
+        pool, bt, k, v, qb, aq, ctx = make_case(fmt, 64, seq, [q] * n, 422, dtype, q_heads=16)
+        hb = oracle.HostBatch(aq, seq, bt, context_lens_before=ctx, valid_req_mask=mask)
+        dpool = G.DevPool(pool)
+        dpool.upload()
+        rc, got, _ = G.dev_attention(dpool, hb, qb, dtype, 16, scratch_bytes=SCRATCH)
+        assert rc == 0
+        live = np.repeat(np.array(mask), q) != 0
+        assert bool((got[~live] == 0x5500).all()), "masked requests were written"
+        want = oracle.paged_attention(pool, hb, qb, dtype, 16, n_threads=4)
+        G.assert_close(got[live], dtype, want[live], what="short batch, masked requests x%d" % scale,
+                       scale=G.channel_scale(v, dtype, hb, 16)[live])

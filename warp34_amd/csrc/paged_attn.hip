@@ -38,6 +38,7 @@
 //
 // MFMA use: v_mfma_f32_16x16x32_f16.  A = K rows (QK) or V^T (PV) so that every lane owns one
 // query column: softmax state and the O rescale are per-lane scalars.
+#include <algorithm>
 #include <atomic>
 #include <type_traits>
 
@@ -102,7 +103,7 @@ struct AttnParams {
     int tiles_by_request;  // 1: blockIdx.z is a request (no request has more than one tile)
     int rot_q;             // K rows are stored rotated (WHT-256 transform): rotate the query rows
     int rot_out;           // V rows are stored rotated: rotate the output back
-    int32_t* bal_table;    // balanced decode: per query token {first partial slot, pieces, token of the tile, -}
+    int32_t* bal_table;    // balanced decode: per query token {first partial slot, pieces, token of the tile, columns (0: bal_cols)}
     int bal_tiles;         // balanced decode: tiles per request (a bound; the plan's entries are request x tile)
     int bal_aligned;       // balanced decode: no piece boundary inside a workgroup's share (few entries)
     int piece_cost;        // balanced decode: what starting a piece costs, in units
@@ -110,9 +111,17 @@ struct AttnParams {
     uint32_t block_magic;  // floor(2^32 / block_size), see div_block
     uint32_t q_group_magic;  // see div_q_group
     const uint16_t* gate;  // fp16 [tokens, q heads, 256] or null: out = fp16(out) * sigmoid(gate)
-    // chunk geometry of a tile whose keys are exactly [0, max_seq_len): worked out on the host, so a
-    // request that is as long as the host's bound needs no division on the device
-    int spec_units, spec_upc, spec_chunks;
+    union {  // (a longer argument block costs every kernel's start: 12 bytes more, a bf16 decode step 0.2 us of 20)
+        // chunk geometry of a tile whose keys are exactly [0, max_seq_len): worked out on the host, so a
+        // request that is as long as the host's bound needs no division on the device
+        struct {
+            int spec_units, spec_upc, spec_chunks;
+        };
+        // balanced verify: a batch of up to short_units units runs as tiles of 16 columns (bal_short_piece); -1: none does
+        struct {
+            int short_units, short_tiles, short_tok_tile;
+        };
+    };
     // Partial records: part_stride slots per output row.  Slots [0, max_chunks) belong to the
     // split-K chunks of the decode kernels; a shared-prefix pass (tile kernel over the keys every
     // request of the batch has in common) owns slots [pf_slot_base, pf_slot_base + pf_split), and
@@ -346,6 +355,8 @@ __device__ __forceinline__ constexpr int tq4_pv_elem(int h, int j, int r) {
     return 8 * r - 4 + j;
 }
 
+// Smallest chunk: 256 tokens, one unit per wave.  7 to 12 % faster than 16 at 16K-32K keys, same as 4
+constexpr int kMinUnitsPerChunk = 8;
 constexpr int kMergeGroups = 16;
 constexpr int kMergeMaxPerGroup = 16;  // at most 256 partials per row
 
@@ -382,19 +393,19 @@ struct BalReq {  // entry base + lane of a group of 64
     int cost;  // units + P.piece_cost, 0 for an entry without work
     int live;  // has query tokens and is not masked
 };
-__device__ __forceinline__ BalReq bal_load_req(const AttnParams& P, int e) {
+__device__ __forceinline__ BalReq bal_load_req(const AttnParams& P, int tiles, int tok_tile, int e) {
     const warp34_attention_batch& B = P.B;
     BalReq q{0, 0, 0, 0, 0, 0, 0, 0, 0};
-    const int r = P.bal_tiles == 1 ? e : small_div(e, P.bal_tiles);
+    const int r = tiles == 1 ? e : small_div(e, tiles);
     if (r >= B.num_reqs) return q;
     q.lo = B.query_start_loc[r];
     q.hi = B.query_start_loc[r + 1];
     q.sa = B.seq_lens_after[r];
     const int q_len = q.hi - q.lo;
     q.cb = B.context_lens_before != nullptr ? B.context_lens_before[r] : q.sa - q_len;
-    const int first = (e - r * P.bal_tiles) * P.tok_tile;  // the tile's first token inside the request
+    const int first = (e - r * tiles) * tok_tile;  // the tile's first token inside the request
     q.t_lo = min(q.lo + first, max(q.lo, q.hi));
-    q.t_hi = min(q.lo + first + P.tok_tile, max(q.lo, q.hi));
+    q.t_hi = min(q.lo + first + tok_tile, max(q.lo, q.hi));
     const bool live = q.t_hi > q.t_lo && (B.valid_req_mask == nullptr || B.valid_req_mask[r] != 0);
     int last = (B.mask_mode == WARP34_ATTN_MASK_NONCAUSAL_WINDOW) ? q.sa - 1 : q.cb + (q.t_hi - q.lo) - 1;
     if (last >= q.sa) last = q.sa - 1;
@@ -424,7 +435,7 @@ __device__ __forceinline__ int bal_share(int total, int groups, int min_share) {
 // `req`, the piece number `slot` (partials of a tile occupy consecutive slots) and the number of
 // pieces the tile is cut into.
 struct BalItem {
-    int req, tile, rq_start, rq_end, seq_after, ctx_before;
+    int req, tile, tok_tile, rq_start, rq_end, seq_after, ctx_before;
     int u_begin, u_end, n_chunks, slot;
 };
 
@@ -1393,18 +1404,105 @@ __global__ __launch_bounds__(kTq4Waves * 64, 1) void paged_attn_tq4_kernel(const
     }
 }
 
+// The argument block once more, from the kernel's argument segment: a second body of a kernel that reads its
+// arguments here leaves the scalar registers of the first alone (shared, the scalars of both are loaded at
+// the kernel's start and spilled).
+__device__ __forceinline__ AttnParams kernel_params_again() {
+    typedef const __attribute__((address_space(4))) AttnParams* Args;
+    Args args = (Args)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(args));
+    return *(const AttnParams*)args;
+}
+
+// A batch of two column tiles that has little to read (P.short_units): its tiles have 16 columns, and every entry (at
+// most 128) is cut into equal pieces of its own, so that a workgroup has at most one.  The second column tile costs 5 us
+// per piece (query table, merge of the waves), the second piece of a share 8; reading the keys once for both
+// tiles repays neither here.  The plan decides by the lengths it finds, not by the host's bound.  us, before the plan ->
+// one plan for all -> now: 20 requests x 4 tokens over Q8_0 on 600 keys 31.5 -> 27.7 -> 18.4, on 1000 33.3 -> 28.4 ->
+// 21.3; 40 x 4 on 1000 26.2 -> 32.2 -> 27.6; bf16 10 x 4 on 1000 23.4 -> 20.1 -> 18.0.  Longer batches: no change.
+template <typename TileFn>
+__device__ __forceinline__ void bal_short_piece(const AttnParams& P, TileFn&& tile) {
+    const int lane = (int)threadIdx.x & 63;
+    const int groups = (int)gridDim.x, wg = (int)blockIdx.x;
+    const int entries = P.B.num_reqs * P.short_tiles;
+    const BalReq q0 = bal_load_req(P, P.short_tiles, P.short_tok_tile, lane);
+    const BalReq q1 = bal_load_req(P, P.short_tiles, P.short_tok_tile, 64 + lane);
+    const auto record = [&](int tok, int first, int pieces, int tok_of_tile) {
+        if (tok < P.B.total_tokens) *reinterpret_cast<int4*>(P.bal_table + 4 * (size_t)tok) = int4{first, pieces, tok_of_tile, 16};
+    };
+    const auto record_idle = [&](const BalReq& q, int e) {  // as in bal_for_each_piece
+        if (e >= entries) return;
+        if (q.units == 0) {
+            for (int t = q.t_lo; t < q.t_hi; ++t) record(t, 0, q.live ? 0 : -1, 0);
+        }
+        if (e == entries - 1) {
+            for (int t = max(q.hi, 0); t < P.B.total_tokens; ++t) record(t, 0, -1, 0);
+        }
+    };
+    if (wg == 0 && blockIdx.y == 0 && threadIdx.x < 64) {
+        record_idle(q0, lane);
+        record_idle(q1, 64 + lane);
+    }
+    int longest = bal_share(__builtin_amdgcn_readlane(wave_incl_scan(q0.units + q1.units), 63), groups, kMinUnitsPerChunk);
+    int pieces0, pieces1, incl0, incl1;
+    for (;;) {  // as in bal_for_each_piece
+        pieces0 = q0.units > 0 ? fast_div(q0.units + longest - 1, longest) : 0;
+        pieces1 = q1.units > 0 ? fast_div(q1.units + longest - 1, longest) : 0;
+        incl0 = wave_incl_scan(pieces0);
+        incl1 = __builtin_amdgcn_readlane(incl0, 63) + wave_incl_scan(pieces1);
+        const int n = __builtin_amdgcn_readlane(incl1, 63);
+        if (n <= groups) break;
+        longest += fast_div(longest * (n - groups), groups) + 1;
+    }
+    unsigned long long hits = __ballot(pieces0 > 0 && wg < incl0);
+    const bool second = hits == 0ull;
+    if (second) hits = __ballot(pieces1 > 0 && wg < incl1);
+    if (hits == 0ull) return;
+    const int src = __builtin_ctzll(hits);
+    // (lane values picked one by one: a copy of the struct, first or second, would go through memory)
+    const auto pick = [&](int a, int b) {
+        return second ? __builtin_amdgcn_readlane(b, src) : __builtin_amdgcn_readlane(a, src);
+    };
+    const int n_pieces = pick(pieces0, pieces1), first = pick(incl0, incl1) - n_pieces, units = pick(q0.units, q1.units);
+    const int per_piece = fast_div(units + n_pieces - 1, n_pieces);
+    const int entry = second ? 64 + src : src;
+    BalItem it;
+    it.req = small_div(entry, P.short_tiles);
+    it.tile = entry - it.req * P.short_tiles;
+    it.tok_tile = P.short_tok_tile;
+    it.rq_start = pick(q0.lo, q1.lo);
+    it.rq_end = pick(q0.hi, q1.hi);
+    it.seq_after = pick(q0.sa, q1.sa);
+    it.ctx_before = pick(q0.cb, q1.cb);
+    it.u_begin = (wg - first) * per_piece;
+    it.u_end = min(it.u_begin + per_piece, units);
+    it.n_chunks = n_pieces;
+    it.slot = wg;
+    const int tok = pick(q0.t_lo, q1.t_lo) + (int)threadIdx.x;
+    if (wg == first && blockIdx.y == 0 && tok < pick(q0.t_hi, q1.t_hi)) record(tok, first, n_pieces, (int)threadIdx.x);
+    tile(it);
+}
+
 // Balanced decode: grid = (groups, kv head x q subgroup).  Every wave computes the plan (the
 // loads are the same addresses in every wave of the chip and stay in cache) and calls
 // tile(piece) for the pieces of its workgroup's share, in order.
-template <typename TileFn>
-__device__ __forceinline__ void bal_for_each_piece(const AttnParams& P, TileFn&& tile) {
+// SHORT: a batch that turns out short is left to short_batch().
+template <bool SHORT, typename TileFn, typename ShortFn>
+__device__ __forceinline__ void bal_for_each_piece(const AttnParams& P, TileFn&& tile, ShortFn&& short_batch) {
     const int lane = (int)threadIdx.x & 63;
     const int entries = P.B.num_reqs * P.bal_tiles;
     // the first 64 entries are loaded once: their lane values serve the total and the search for
     // the first piece (most workgroups have exactly one piece, most batches at most 64 entries)
-    const BalReq q0 = bal_load_req(P, lane);
+    const BalReq q0 = bal_load_req(P, P.bal_tiles, P.tok_tile, lane);
     const int incl0 = wave_incl_scan(q0.cost);
     int total = __builtin_amdgcn_readlane(incl0, 63);
+    if constexpr (SHORT) {
+        // (a batch that may be short has at most 64 entries)
+        if (total - P.piece_cost * (int)__popcll(__ballot(q0.units > 0)) <= P.short_units) {  // uniform for the grid
+            short_batch();
+            return;
+        }
+    }
     // wave 0 of workgroup (0, 0) records the tokens no workgroup will work on
     const bool recorder = blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x < 64;
     auto record_idle = [&](const BalReq& q, int e) {
@@ -1420,11 +1518,12 @@ __device__ __forceinline__ void bal_for_each_piece(const AttnParams& P, TileFn&&
     };
     record_idle(q0, lane);
     for (int base = 64; base < entries; base += 64) {
-        const BalReq q = bal_load_req(P, base + lane);
+        const BalReq q = bal_load_req(P, P.bal_tiles, P.tok_tile, base + lane);
         record_idle(q, base + lane);
         total += __builtin_amdgcn_readlane(wave_incl_scan(q.cost), 63);
     }
     BalItem it{};
+    it.tok_tile = P.tok_tile;
     int my_begin = 0, my_end = 0, piece_end = 0;  // (aligned: the one piece ends the share)
     int share = 1;
     if (P.bal_aligned) {  // uniform for the grid; at most 64 entries
@@ -1454,8 +1553,9 @@ __device__ __forceinline__ void bal_for_each_piece(const AttnParams& P, TileFn&&
         it.rq_end = __builtin_amdgcn_readlane(q0.hi, src);
         it.seq_after = __builtin_amdgcn_readlane(q0.sa, src);
         it.ctx_before = __builtin_amdgcn_readlane(q0.cb, src);
-        // (equal pieces; rounding up may leave the last ones without units, they still write a record)
-        it.u_begin = min(((int)blockIdx.x - first) * per_piece, e_units);
+        // equal pieces, none without units: n_pieces = ceil(e_units / share), so per_piece <= share and
+        // (n_pieces - 1) * per_piece < e_units
+        it.u_begin = ((int)blockIdx.x - first) * per_piece;
         it.u_end = min(it.u_begin + per_piece, e_units);
         it.n_chunks = n_pieces;
         it.slot = (int)blockIdx.x;
@@ -1510,7 +1610,7 @@ __device__ __forceinline__ void bal_for_each_piece(const AttnParams& P, TileFn&&
     };
     auto find_next = [&]() -> bool {
         while (base < entries && before < my_end) {
-            const BalReq q = bal_load_req(P, base + lane);
+            const BalReq q = bal_load_req(P, P.bal_tiles, P.tok_tile, base + lane);
             if (scan_group(q, wave_incl_scan(q.cost))) return true;
         }
         return false;
@@ -1530,10 +1630,11 @@ __global__ __launch_bounds__(kTq4Waves * 64, 1) void paged_attn_tq4_balanced_ker
     extern __shared__ __align__(16) uint8_t smem[];
     // the pair table survives a piece (the merge regions lie in the staging areas): built once
     bool first = true;
-    bal_for_each_piece(P, [&](const BalItem& it) {
+    const auto piece = [&](const BalItem& it) {
         tq4_tile<TQ, true>(P, smem, it, first);
         first = false;
-    });
+    };
+    bal_for_each_piece<false>(P, piece, [] {});
 }
 
 // Merge for the balanced decode kernel: one workgroup of GROUPS waves per (token, q head) row; wave g
@@ -1564,8 +1665,9 @@ __global__ __launch_bounds__(GROUPS * 64) void balanced_merge_kernel(const AttnP
     }
     const int kv_sub = small_div(head, P.q_group);  // = kv_head * q_subgroups + subgroup
     const int col = entry.z * P.q_group + (head - kv_sub * P.q_group);
-    const size_t prow0 = bal_partial_row(entry.x, kv_subs, kv_sub, P.bal_cols, col);
-    const size_t pstride = (size_t)kv_subs * P.bal_cols;  // partial rows between consecutive slots
+    const int cols = entry.w != 0 ? entry.w : P.bal_cols;
+    const size_t prow0 = bal_partial_row(entry.x, kv_subs, kv_sub, cols, col);
+    const size_t pstride = (size_t)kv_subs * cols;  // partial rows between consecutive slots
     if (tid < n_chunks && tid < kSlots) s_rec[tid] = *reinterpret_cast<const f4*>(P.part_ml + (prow0 + tid * pstride) * 4);
     f4 a[kMergeMaxPerGroup];
     auto load_slices = [&](int first) {
@@ -1769,8 +1871,6 @@ namespace w34 {
 
 // ---- host side ---------------------------------------------------------------------------------
 constexpr int kMaxChunksCap = 256;
-// 256 tokens, one unit per wave: 7 to 12 % faster than 16 at 16K-32K keys, same as 4
-constexpr int kMinUnitsPerChunk = 8;
 // Cost of starting a piece of a balanced batch, in units of streaming: TQ4 builds its table and
 // rotates the queries first.
 constexpr int kTq4PieceCost = 32;
@@ -1788,6 +1888,23 @@ constexpr int kMinUnitsPerWidePiece = 4;
 // against 24.2 us, eight of 16 on 4000 39.7 against 44.2, but four of 16 on 2K to 5K keys 31.8 against 30.9 and
 // twelve of 8 on 8000 55.0 against 50.2.  (Counts of tiles, not lengths: results do not depend on max_seq_len.)
 constexpr int kRowsGridTiles = 8;
+// Short batches (bal_short_piece): key and value rows of up to this many bytes per kv head, each counted once, for
+// batches whose entries are cut into pieces of their own anyway and for others (whose workgroups mostly have
+// two pieces).  Tiles of 16 against 32 columns, us: few entries, Q8_0 5 x 4 tokens on 800 to 8000 keys (12 MB) 21.2 against
+// 22.0, 5 x 8 (24 MB) 27.4 against 25.0, bf16 10 x 4 on 2000 (21 MB) equal; others, Q8_0 20 x 4 on 2000 (22 MB) 26.7
+// against 29.4, 32 x 4 on 300 to 3000 (29 MB) 36.6 against 32.9, bf16 20 x 4 on 1000 (21 MB) 23.3 against 29.5, on 300 to 3000
+// (34 MB) 34.5 against 31.4.
+constexpr int kShortBytesFew = 16 << 20;
+constexpr int kShortBytes = 24 << 20;
+constexpr int kShortMaxEntries = 128;  // of 16 columns: two per lane
+// Up to here the chunk grid has one chunk per tile and its merge is not launched; a short batch whose requests
+// are no longer has one piece per tile of the same 16 columns, and the bits are the same (5 x 4 tokens on 200 keys:
+// 11.4 against 13.6 us).
+constexpr int kShortGridKeys = (kMinUnitsPerChunk - 1) * kUnit;
+// The most units that 64 entries of kShortGridKeys have make a short batch in every format.
+static_assert(kShortMaxEntries / 2 * (kMinUnitsPerChunk - 1) <= kShortBytes / (64 * 2 * kHeadDim) &&
+                  16 * (kMinUnitsPerChunk - 1) <= kShortBytesFew / (64 * 2 * kHeadDim),
+              "the chunk grid stands in for short batches only");
 // Split geometry is sized for the layout the path is built for, two kv heads per device: 128
 // chunks (or shares) per kv head.  The counts below depend on the batch and on gqa only, never
 // on local_kv_heads: a rank that holds one kv head of a sharded model computes every row with
@@ -2217,6 +2334,17 @@ static int launch_rows_balanced(const warp34_exec* ex, const warp34_attention_ba
     P.bal_tiles = tiles;
     P.bal_cols = 16 * nt;
     P.bal_aligned = balanced_aligned(entries, groups);
+    P.short_units = -1;
+    if (nt == 2) {
+        const int tok16 = 16 / P.q_group, tiles16 = (batch->max_q_len + tok16 - 1) / tok16;
+        if (entries <= kShortMaxEntries / 2 && (long long)batch->num_reqs * tiles16 <= std::min(groups, kShortMaxEntries)) {
+            // (no entry has two pieces, on either path one workgroup does the same arithmetic: launch shape only)
+            if (batch->max_seq_len > 0 && batch->max_seq_len <= kShortGridKeys) return -1;
+            P.short_units = (P.bal_aligned ? kShortBytesFew : kShortBytes) / (4 * RowsLds<KVF, HD>::kHalf);
+            P.short_tiles = tiles16;
+            P.short_tok_tile = tok16;
+        }
+    }
     const auto launch = [&](auto column_tiles) -> int {
         constexpr int NT = decltype(column_tiles)::value;
         constexpr int smem = rows_smem_bytes<KVF, HD>(NT);

@@ -214,8 +214,9 @@ __device__ __forceinline__ void rows_tile(const AttnParams& P, uint8_t* smem, co
     // after it.  Rotated queries and several tiles go through the LDS table below.
     const bool rot_q = K8 && P.rot_q != 0;  // workgroup-uniform
     const bool q_direct = NT == 1 && !rot_q;
-    const int tok_guess = BAL ? item.rq_start + item.tile * P.tok_tile
-                              : min(P.tiles_by_request ? tile_z : tile_z * P.tok_tile, B.total_tokens - 1);
+    const int tok_tile = BAL ? item.tok_tile : P.tok_tile;
+    const int tok_guess = BAL ? item.rq_start + item.tile * tok_tile
+                              : min(P.tiles_by_request ? tile_z : tile_z * tok_tile, B.total_tokens - 1);
     u4 bq[kM];
     auto load_q = [&](int tokbase) {
         const int t = div_q_group(n, P);
@@ -256,7 +257,7 @@ __device__ __forceinline__ void rows_tile(const AttnParams& P, uint8_t* smem, co
     if (!ti.hit) return;  // no such tile, empty or masked request: outputs untouched
     const int req = ti.req, rq_start = ti.rq_start, rq_end = ti.rq_end;
     const int seq_after = ti.seq_after, ctx_before = ti.ctx_before;
-    const int tok0 = rq_start + ti.tile_in_req * P.tok_tile;
+    const int tok0 = rq_start + ti.tile_in_req * tok_tile;
     if (q_direct) {
         if (tok0 != tok_guess) load_q(tok0);  // wave-uniform, rare
         if constexpr (K8 && Q_BF16) {
@@ -277,7 +278,7 @@ __device__ __forceinline__ void rows_tile(const AttnParams& P, uint8_t* smem, co
                                               B.valid_token_mask[min(tok, B.total_tokens - 1)] != 0);
     }
     int tile_tokens = rq_end - tok0;
-    if (tile_tokens > P.tok_tile) tile_tokens = P.tok_tile;
+    if (tile_tokens > tok_tile) tile_tokens = tok_tile;
 
     // Column info (per lane = per query column: visible key range; tile-wide: union and intersection
     // of the ranges).  Without a token mask and a window the tile-wide values follow from scalars
@@ -908,7 +909,13 @@ __global__ __launch_bounds__(kKv16Waves * 64, 1) void paged_attn_rows_kernel(con
 template <typename TQ, int NT, int KVF, bool VRES, bool STREAM, int HD = kHeadDim>
 __global__ __launch_bounds__(kKv16Waves * 64, 1) void paged_attn_rows_balanced_kernel(const AttnParams P) {
     extern __shared__ __align__(16) uint8_t smem[];
-    bal_for_each_piece(P, [&](const BalItem& it) { rows_tile<TQ, NT, KVF, true, VRES, STREAM, HD>(P, smem, it); });
+    bal_for_each_piece<(NT > 1)>(
+        P, [&](const BalItem& it) { rows_tile<TQ, NT, KVF, true, VRES, STREAM, HD>(P, smem, it); },
+        [&] {
+            const AttnParams A = kernel_params_again();
+            // (several tiles per request: ordinary loads)
+            bal_short_piece(A, [&](const BalItem& it) { rows_tile<TQ, 1, KVF, true, VRES, false, HD>(A, smem, it); });
+        });
 }
 
 }  // namespace w34
