@@ -83,6 +83,24 @@ def test_rows_large_batches_in_8mib_keep_a_workgroup_per_tile(fmt, dtype, n, q):
 
 
 @pytest.mark.parametrize("fmt,dtype", [(FMT_Q8_0, DT_F16), (FMT_BF16, DT_BF16)])
+@pytest.mark.parametrize("lens", [37, 211])
+def test_rows_verify_in_8mib_keeps_the_plan_while_it_has_the_workgroups(fmt, dtype, lens):
+    """40 requests x 4 tokens: 86 shares for 80 tiles of 16 columns.  Short and longer batches."""
+    import gpu_harness as G
+    from cases import make_case
+
+    seq = [40 + lens * ((i * 7) % 11) for i in range(40)]
+    pool, bt, k, v, qb, aq, ctx = make_case(fmt, 64, seq, [4] * 40, 423, dtype, q_heads=16)
+    hb = oracle.HostBatch(aq, seq, bt, context_lens_before=ctx)
+    dpool = G.DevPool(pool)
+    dpool.upload()
+    rc, got, ws = G.dev_attention(dpool, hb, qb, dtype, 16, scratch_bytes=8 << 20)
+    assert rc == 0 and not bool((ws == 0x5A).all())
+    want = oracle.paged_attention(pool, hb, qb, dtype, 16, n_threads=4)
+    G.assert_close(got, dtype, want, what="40 x 4 in 8 MiB", scale=G.channel_scale(v, dtype, hb, 16))
+
+
+@pytest.mark.parametrize("fmt,dtype", [(FMT_Q8_0, DT_F16), (FMT_BF16, DT_BF16)])
 @pytest.mark.parametrize("n,q", [(1, 1), (1, 4), (5, 4), (3, 16), (40, 1), (40, 4)])
 def test_rows_scratch_of_the_queried_size_splits_fully(fmt, dtype, n, q):
     """The bits of a call with the scratch the query names are those of a call with 64 MiB."""

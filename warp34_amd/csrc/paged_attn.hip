@@ -2311,19 +2311,24 @@ static int launch_rows_balanced(const warp34_exec* ex, const warp34_attention_ba
     const int nt = shape.nt, tiles = shape.tiles;
     if (tiles < 1) return -1;
     P.tok_tile = shape.tok_tile;
-    // Fewer shares where the scratch cannot hold the records of all of them, down to three quarters; with less
-    // room the chunk grid, whose workgroups grow with the batch, leaves fewer compute units idle.  8 MiB, two kv
-    // heads, Q8_0, chunk grid against plan: 150 decode requests (102 shares) of 1000 keys 45.4 against 46.3 us,
-    // of 1K to 9K 194 against 140; 175 (77 shares) 46 against 61, 202 against 187; 200 (52 shares) 47 against 93, 226 against 296;
-    // 235 (17 shares) 54 against 308, 262 against 1046.  20 requests x 4 tokens (106 shares) on 300 to 3000 keys 29.2 against 31.1,
-    // on 3K to 16K 93 against 60; 60 x 4 (66 shares) on 300 to 3000 keys 54 against 66.
+    // Fewer shares where the scratch cannot hold the records of all of them, down to three quarters or to the
+    // workgroups that the chunk grid would launch; with less room the chunk grid, whose workgroups grow with the
+    // batch, leaves fewer compute units idle.  8 MiB, two kv heads, Q8_0, chunk grid against plan, us: 150 decode
+    // requests (102 shares) of 1000 keys 45 against 46, of 1K to 9K 194 against 140; 175 (77 shares) 46 against 61, 202 against
+    // 187; 200 (52 shares) 47 against 93, 226 against 296; 235 (17 shares) 54 against 308, 262 against 1046.  40 requests x 4
+    // tokens (86 shares, 80 tiles) on 1000 keys 24 against 27, on 300 to 3000 49 against 40, on 800 to 8000 112 against 67;
+    // 50 x 4 (76 shares, 100 tiles) on 1000 keys 25 against 38, on 300 to 3000 50 against 51; 60 x 4 (66 shares) 54 against 64.
     const long long entries = (long long)batch->num_reqs * tiles;
     const size_t slot_bytes = partial_bytes((long long)kv_subs * 16 * nt, 1), table_bytes = (size_t)batch->total_tokens * 16;
     if (ex->scratch_size < table_bytes) return -1;
     const long long room = (long long)((ex->scratch_size - table_bytes) / slot_bytes) - entries;
     const int all_groups = balanced_groups(P.q_subgroups);
     const int groups = (int)(room < all_groups ? room : all_groups);
-    if (groups < 1 || 4 * groups < 3 * all_groups) return -1;
+    const int tok16 = 16 / P.q_group, tiles16 = (batch->max_q_len + tok16 - 1) / tok16;
+    if (groups < 1 || (4 * groups < 3 * all_groups &&
+                       groups < (long long)batch->num_reqs * tiles16 *
+                                    choose_max_chunks(ex, batch->total_tokens, P.num_q_heads, tok16, P.q_subgroups)))
+        return -1;
     const size_t prows = (size_t)(groups + entries) * kv_subs * 16 * nt;
     P.piece_cost = kRowsPieceCost;
     if (nt * tiles > 1) P.min_upc = kMinUnitsPerWidePiece;
@@ -2336,7 +2341,6 @@ static int launch_rows_balanced(const warp34_exec* ex, const warp34_attention_ba
     P.bal_aligned = balanced_aligned(entries, groups);
     P.short_units = -1;
     if (nt == 2) {
-        const int tok16 = 16 / P.q_group, tiles16 = (batch->max_q_len + tok16 - 1) / tok16;
         if (entries <= kShortMaxEntries / 2 && (long long)batch->num_reqs * tiles16 <= std::min(groups, kShortMaxEntries)) {
             // (no entry has two pieces, on either path one workgroup does the same arithmetic: launch shape only)
             if (batch->max_seq_len > 0 && batch->max_seq_len <= kShortGridKeys) return -1;
