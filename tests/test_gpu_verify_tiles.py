@@ -166,3 +166,10 @@ def test_rows_short_batches_with_idle_requests(fmt, dtype):
         want = oracle.paged_attention(pool, hb, qb, dtype, 16, n_threads=4)
         G.assert_close(got[live], dtype, want[live], what="short batch, masked requests x%d" % scale,
                        scale=G.channel_scale(v, dtype, hb, 16)[live])
+
+
+@pytest.mark.parametrize("n", [2, 3, 4, 7])
+def test_rows_decode_head_dim_128_either_side_of_the_grid_rule(n):
+    """Up to three requests on the chunk grid, more on the plan."""
+    _check(FMT_BF16, DT_BF16, 16, [1500, 37, 4000, 700, 16, 2100, 330][:n], [1] * n, 424, scratch=SCRATCH, q_heads=16, kv_heads=4,
+           head_dim=128)

@@ -66,6 +66,7 @@ def test_decode_batches_of_every_format_and_verify_batches_of_row_formats():
         assert query(32, 32, 30000, fmt) == plan(32, 32)
         assert query(32, 16, 30000, fmt) == max(plan(32, 16), chunks(32, 8))
     assert query(4, 4, 2000, "bf16", q_heads=4, kv_heads=2, head_dim=128) == max(plan(4, 4), chunks(4, 8, 4))
+    assert query(3, 3, 2000, "bf16", q_heads=4, kv_heads=2, head_dim=128) == chunks(3, 8, 4)
     for fmt in ("q8_0", "fp8", "bf16", "fp16"):
         assert query(20, 5, 21000, fmt) == plan(20, 5, 32)
         assert query(64, 16, 262144, fmt) == plan(64, 16, 32)

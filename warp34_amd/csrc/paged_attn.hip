@@ -1891,19 +1891,26 @@ constexpr int kMaxChunksCap = 256;
 // rotates the queries first.
 constexpr int kTq4PieceCost = 32;
 constexpr int kRowsPieceCost = 16;
-// Smallest piece where a request has several tiles or column tiles.  It counts for short requests only: a
-// layer's step of 12 requests x 4 tokens on 270 to 800 keys (Q8_0) 34.8 us with 16, 28.6 with 8, 26.8 with 4
-// (31.3 on the chunk grid of one-tile workgroups before); at 7K to 19K keys the same.
+// Smallest piece where a request has several tiles or column tiles and the batch is no short one (bal_short_piece).
+// It counts where few keys meet many shares: Q8_0, 100 requests x 4 tokens on 200 keys 29.5 us with 4, 32.1 with 8, 36.7
+// with 16; rotated Q8_0, 5 x 4 on 600 keys 14.9, 17.0, 17.3.  On longer contexts the same.
 constexpr int kMinUnitsPerWidePiece = 4;
 // A batch whose requests have several tiles goes to the chunk grid instead while it has no more 16-column
-// tiles than this per kv head: the plan, the table and the merge of wider pieces cost 4 to 9 us of a call,
-// which reading the keys once for two tiles repays from there on.  Layer steps over Q8_0 pages, chunk
-// grid against plan: 4 requests x 4 tokens (8 tiles) on 2000 keys 23.0 against 26.8 us, on 16000 keys 35.5 against 36.8;
-// 5 x 4 (10 tiles) on 7K to 19K keys 46.2 against 40.2; 12 x 4 on 800 keys 23.4 against 26.8, on 3000 (16 x 4) the same.
-// At head dimension 128 every such batch does: half the bytes per tile.  Three draft blocks of 8 tokens on 2000 keys 17.4
-// against 24.2 us, eight of 16 on 4000 39.7 against 44.2, but four of 16 on 2K to 5K keys 31.8 against 30.9 and
-// twelve of 8 on 8000 55.0 against 50.2.  (Counts of tiles, not lengths: results do not depend on max_seq_len.)
+// tiles than this per kv head: the plan, the table and the merge launch cost 1 to 2 us of a call.  Layer steps over
+// Q8_0 pages (contexts from a third of the length up), chunk grid against plan, us: 4 requests x 4 tokens (8 tiles) on
+// 2000 keys 23.4 against 24.1, on 16000 32.5 against 34.5; 5 x 4 (10 tiles) on 2000 23.6 against 24.3, on 19000 37.6
+// against 37.2; 12 x 4 on 800 23.8 against 24.4; 16 x 4 on 3000 31.6 against 31.4; 30 x 4 on 2000 38.9 against 39.7.  The
+// line lies where the longest contexts turn (attention alone, 10 x 4 on 3K to 16K 54 against 35, 20 x 4 93 against 53).
+// (Counts of tiles, not lengths: results do not depend on max_seq_len.)
+// At head dimension 128 every such batch goes there: the plan has one column tile at that size (with two the merge of
+// the waves outweighs the keys read once more) and is nowhere ahead.  Draft blocks, layer steps: 3 x 8 on 2000 keys
+// 17.4 against 18.9, 4 x 16 on 9000 32.3 against 36.7, 12 x 8 on 8000 55 against 60, 16 x 16 on 16000 150.6 against 150.5.
 constexpr int kRowsGridTiles = 8;
+// A decode batch at head dimension 128 (four q heads per kv head) goes to the chunk grid up to this many requests.
+// Chunk grid against plan, four kv heads, us: 2 requests of 1000 keys 10.2 against 13.0, of 3K to 16K 11.6 against 15.0, of 5K to
+// 60K 24.2 against 24.4; 3 requests 10.5 against 13.3, 17.9 against 20.7, 41 against 35; 4 requests 11.8 against 13.5, 24.1
+// against 23.2, 59 against 45; 6 requests 11.7 against 13.6, 38 against 29.
+constexpr int kRowsGridRequests128 = 3;
 // Short batches (bal_short_piece): key and value rows of up to this many bytes per kv head, each counted once, for
 // batches whose entries are cut into pieces of their own anyway and for others (whose workgroups mostly have
 // two pieces).  Tiles of 16 against 32 columns, us: few entries, Q8_0 5 x 4 tokens on 800 to 8000 keys (12 MB) 21.2 against
@@ -2015,7 +2022,9 @@ static int balanced_aligned(long long entries, int groups) {
 // a long sequence in flight at once; from 32 rows per kv head on the workgroups are many and the
 // partials of a row few, and four waves per row start sooner (two kv heads, 80 rows of 25 partials: 6.9 ->
 // 5.2 us; 512 rows: 8.9 -> 5.8; four kv heads, 1 024 rows of ten: 11.5 -> 4.9; but 16 rows of 128
-// partials: 5.2 -> 6.8).  Rows per kv head, not rows: a rank with one kv head adds in the same order.
+// partials: 5.2 -> 6.8).  At the line, one request of 4 tokens (32 rows): 64 partials, 32 768 keys, whole call 23.2 us with
+// sixteen waves, 23.6 with four; 6 partials, 1500 keys, 16.9 and 16.7.  24 rows of 64 partials: 21.3 and 21.7; 64 rows of 32:
+// 28.4 and 28.4.  Rows per kv head, not rows: a rank with one kv head adds in the same order.
 static bool merge_small_groups(const AttnParams& P) { return (long long)P.B.total_tokens * P.gqa >= 32; }
 
 template <typename TQ, int HD>
@@ -2306,6 +2315,8 @@ static BalShape rows_balanced_shape(int num_reqs, int total_tokens, int q_len, i
     if (s.nt * s.tiles > 1) {
         const long long tiles16 = ((long long)total_tokens * q_group + 15) / 16 * q_subgroups;
         if (head_dim != kHeadDim || tiles16 <= kRowsGridTiles) return none;
+    } else if (head_dim != kHeadDim && num_reqs <= kRowsGridRequests128) {
+        return none;
     }
     return s;
 }
@@ -2878,19 +2889,20 @@ static size_t scratch_bytes_for(const warp34_kv_layer_layout* layout, int total_
         if (need > bytes) bytes = need;
     };
     if (num_reqs < 0 || num_reqs > total_tokens) num_reqs = total_tokens;
-    // one tile per request (decode steps; not with more tokens than that many tiles hold)
-    if (num_reqs >= 2 && total_tokens <= 65535 && total_tokens <= (long long)num_reqs * tok_tile) plan(num_reqs, 1);
-    if (!layout) {
-        // one q head per kv head: two column tiles from 17 tokens per request on, at most an entry per 16 tokens
-        if (total_tokens > 16 * kRowsGridTiles && total_tokens <= 65535) plan(total_tokens / 16, 2);
-    } else if (is_kv16(layout, WARP34_KV_FORMAT_FP16) || is_kv16(layout, WARP34_KV_FORMAT_BF16) ||
-               is_kv8(layout, WARP34_KV_FORMAT_FP8_E4M3) || is_kv8(layout, WARP34_KV_FORMAT_Q8_0)) {
-        // row formats: several tiles or column tiles per request (the tokens taken as spread evenly)
+    if (layout && (is_kv16(layout, WARP34_KV_FORMAT_FP16) || is_kv16(layout, WARP34_KV_FORMAT_BF16) ||
+                   is_kv8(layout, WARP34_KV_FORMAT_FP8_E4M3) || is_kv8(layout, WARP34_KV_FORMAT_Q8_0))) {
+        // row formats: as launch_rows_balanced (the tokens taken as spread evenly over the requests)
         const int q_len = num_reqs > 0 ? (int)(((long long)total_tokens + num_reqs - 1) / num_reqs) : 0;
         const BalShape shape = rows_balanced_shape(num_reqs, total_tokens, q_len, q_group, q_subgroups, rows_vres(layout),
                                                    layout->head_dim);
-        if (shape.nt * shape.tiles > 1) plan((long long)num_reqs * shape.tiles, shape.nt);
+        if (shape.tiles > 0) plan((long long)num_reqs * shape.tiles, shape.nt);
+        return bytes;
     }
+    // one tile per request (decode steps; not with more tokens than that many tiles hold)
+    if (num_reqs >= 2 && total_tokens <= 65535 && total_tokens <= (long long)num_reqs * tok_tile) plan(num_reqs, 1);
+    // layout not known, one q head per kv head: two column tiles from 17 tokens per request on, at most an entry
+    // per 16 tokens
+    if (!layout && total_tokens > 16 * kRowsGridTiles && total_tokens <= 65535) plan(total_tokens / 16, 2);
     return bytes;
 }
 
