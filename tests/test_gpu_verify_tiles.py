@@ -128,10 +128,24 @@ def test_rows_scratch_of_the_queried_size_splits_fully(fmt, dtype, n, q):
 def test_rows_short_batches_do_not_depend_on_the_sequence_bound(fmt, dtype, seq, q):
     """No request above 224 keys: on the chunk grid where the host's bound says so, as pieces of 16 columns where the
     plan finds it out; the same bits, and the oracle's answer."""
+    _short_batch(fmt, dtype, seq, q)
+
+
+@pytest.mark.parametrize("fmt", [FMT_FP8, FMT_Q8_0])
+def test_rows_short_batches_of_rotated_rows(fmt):
+    """One column tile, 40 and 60 entries; few enough entries keep the plan with any bound."""
+    for seq, q in (([40 + 9 * (i % 20) for i in range(20)], [4] * 20), ([31, 224, 100, 60, 17] * 3, [7] * 15), ([200] * 5, [4] * 5)):
+        _short_batch(fmt, DT_F16, seq, q, xf=XF_WHT256, plain_excess=4e-4)
+    seq = [16 + 37 * ((i * 7) % 20) for i in range(20)]
+    _check(fmt, DT_F16, 16, seq, [4] * 20, 425, scratch=SCRATCH, q_heads=16, xf=XF_WHT256, plain_excess=4e-4)
+    _check(fmt, DT_F16, 16, [9 * s for s in seq], [4] * 20, 426, scratch=SCRATCH, q_heads=16, xf=XF_WHT256, plain_excess=4e-4)
+
+
+def _short_batch(fmt, dtype, seq, q, xf=None, plain_excess=0.0):
     import gpu_harness as G
     from cases import make_case
 
-    pool, bt, k, v, qb, aq, ctx = make_case(fmt, 16, seq, q, 421, dtype, q_heads=16)
+    pool, bt, k, v, qb, aq, ctx = make_case(fmt, 16, seq, q, 421, dtype, q_heads=16, xf=xf)
     hb = oracle.HostBatch(aq, seq, bt, context_lens_before=ctx)
     dpool = G.DevPool(pool)
     dpool.upload()
@@ -142,7 +156,7 @@ def test_rows_short_batches_do_not_depend_on_the_sequence_bound(fmt, dtype, seq,
         outs.append(out)
     assert all(o.tobytes() == outs[0].tobytes() for o in outs[1:])
     want = oracle.paged_attention(pool, hb, qb, dtype, 16, n_threads=4)
-    G.assert_close(outs[0], dtype, want, what="short batch", scale=G.channel_scale(v, dtype, hb, 16))
+    G.assert_close(outs[0], dtype, want, what="short batch", scale=G.channel_scale(v, dtype, hb, 16), plain_excess=plain_excess)
 
 
 @pytest.mark.parametrize("fmt,dtype", [(FMT_Q8_0, DT_F16), (FMT_BF16, DT_BF16)])

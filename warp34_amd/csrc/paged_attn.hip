@@ -1425,7 +1425,7 @@ __device__ __forceinline__ AttnParams kernel_params_again() {
     return *(const AttnParams*)args;
 }
 
-// A batch of two column tiles that has little to read (P.short_units): its tiles have 16 columns, and every entry (at
+// A batch of wide or several tiles that has little to read (P.short_units): its tiles have 16 columns, and every entry (at
 // most 128) is cut into equal pieces of its own, so that a workgroup has at most one.  The second column tile costs 5 us
 // per piece (query table, merge of the waves), the second piece of a share 8; reading the keys once for both
 // tiles repays neither here.  The plan decides by the lengths it finds, not by the host's bound.  us, before the plan ->
@@ -2367,7 +2367,7 @@ static int launch_rows_balanced(const warp34_exec* ex, const warp34_attention_ba
     P.bal_cols = 16 * nt;
     P.bal_aligned = balanced_aligned(entries, groups);
     P.short_units = -1;
-    if (nt == 2) {
+    if (nt == 2 || (VRES && tiles > 1 && !P.bal_aligned)) {
         if (entries <= kShortMaxEntries / 2 && (long long)batch->num_reqs * tiles16 <= std::min(groups, kShortMaxEntries)) {
             // (no entry has two pieces, on either path one workgroup does the same arithmetic: launch shape only)
             if (batch->max_seq_len > 0 && batch->max_seq_len <= kShortGridKeys) return -1;

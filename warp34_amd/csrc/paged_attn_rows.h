@@ -909,7 +909,7 @@ __global__ __launch_bounds__(kKv16Waves * 64, 1) void paged_attn_rows_kernel(con
 template <typename TQ, int NT, int KVF, bool VRES, bool STREAM, int HD = kHeadDim>
 __global__ __launch_bounds__(kKv16Waves * 64, 1) void paged_attn_rows_balanced_kernel(const AttnParams P) {
     extern __shared__ __align__(16) uint8_t smem[];
-    bal_for_each_piece<(NT > 1)>(
+    bal_for_each_piece<(NT > 1 || (VRES && !STREAM))>(
         P, [&](const BalItem& it) { rows_tile<TQ, NT, KVF, true, VRES, STREAM, HD>(P, smem, it); },
         [&] {
             const AttnParams A = kernel_params_again();
