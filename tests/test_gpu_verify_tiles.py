@@ -187,3 +187,54 @@ def test_rows_decode_head_dim_128_either_side_of_the_grid_rule(n):
     """Up to three requests on the chunk grid, more on the plan."""
     _check(FMT_BF16, DT_BF16, 16, [1500, 37, 4000, 700, 16, 2100, 330][:n], [1] * n, 424, scratch=SCRATCH, q_heads=16, kv_heads=4,
            head_dim=128)
+
+
+def test_rows_verify_graph_serves_short_and_long_batches():
+    """One captured verify step of 20 requests x 4 tokens; the lengths on the device change between replays from
+    a short batch to a long one and back.  Every replay gives the bits of an eager call."""
+    import torch
+
+    import gpu_harness as G
+    from cases import make_case
+
+    n = 20
+    long = [1400 - 3 * i for i in range(n)]
+    pool, bt, k, v, qb, aq, ctx = make_case(FMT_BF16, 64, long, [4] * n, 427, DT_BF16, q_heads=16)
+    hb = oracle.HostBatch(aq, long, bt, context_lens_before=ctx)
+    dpool = G.DevPool(pool)
+    dpool.upload()
+    L = dpool.layout()
+    db = G.DevBatch(hb, max_seq_len=8192)
+    B = db.struct()
+    lens = {"long": long, "short": [90 + 17 * (i % 13) for i in range(n)], "mixed": [90 if i % 2 else s for i, s in enumerate(long)]}
+    q = G.to_dev(qb)
+    out = torch.zeros((4 * n, 16, 256), dtype=torch.int16, device=G.DEV)
+    ws = torch.zeros(SCRATCH, dtype=torch.uint8, device=G.DEV)
+
+    def set_lengths(name):
+        s = np.array(lens[name], dtype=np.int32)
+        db.t["seq"].copy_(torch.from_numpy(s))
+        db.t["ctx"].copy_(torch.from_numpy(s - 4))
+
+    def call():
+        import ctypes as C
+
+        from warp34_amd import ffi
+        ex = ffi.Warp34Exec(torch.cuda.current_stream().cuda_stream, ws.data_ptr(), ws.numel(), 0)
+        assert G.lib().warp34_paged_attention_bf16(C.byref(ex), C.byref(L), C.byref(B), G.ptr(q), G.ptr(out), 16) == 0
+
+    want = {}
+    for name in lens:
+        set_lengths(name)
+        call()
+        torch.cuda.synchronize()
+        want[name] = out.clone()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        call()
+    for name in ("short", "long", "mixed", "short", "long"):
+        set_lengths(name)
+        out.fill_(0)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want[name]), name
