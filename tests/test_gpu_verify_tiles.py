@@ -238,3 +238,13 @@ def test_rows_verify_graph_serves_short_and_long_batches():
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, want[name]), name
+
+
+@pytest.mark.parametrize("fmt,dtype", [(FMT_Q8_0, DT_F16), (FMT_BF16, DT_BF16)])
+@pytest.mark.parametrize("q_heads", [4, 10, 12, 20, 40, 64])
+def test_rows_short_batches_other_group_sizes(fmt, dtype, q_heads):
+    """2 to 32 q heads per kv head: groups that do not fill a tile of 16 columns, two q subgroups."""
+    n = 24
+    _check(fmt, dtype, 16, [30 + 53 * ((i * 7) % 12) for i in range(n)], [4 + 5 * (i % 2) for i in range(n)], 428, scratch=SCRATCH,
+           q_heads=q_heads)
+    _check(fmt, dtype, 16, [100 + 9 * (i % 14) for i in range(n)], [9] * n, 429, scratch=SCRATCH, q_heads=q_heads)

@@ -1915,7 +1915,7 @@ constexpr int kRowsGridRequests128 = 3;
 // batches whose entries are cut into pieces of their own anyway and for others (whose workgroups mostly have
 // two pieces).  Tiles of 16 against 32 columns, us: few entries, Q8_0 5 x 4 tokens on 800 to 8000 keys (12 MB) 21.2 against
 // 22.0, 5 x 8 (24 MB) 27.4 against 25.0, bf16 10 x 4 on 2000 (21 MB) equal; others, Q8_0 20 x 4 on 2000 (22 MB) 26.7
-// against 29.4, 32 x 4 on 300 to 3000 (29 MB) 36.6 against 32.9, bf16 20 x 4 on 1000 (21 MB) 23.3 against 29.5, on 300 to 3000
+// against 29.4, 32 x 4 on 300 to 3000 (29 MB) 36.6 against 32.9, bf16 20 x 4 on 1000 (21 MB) 24.4 against 29.5, on 300 to 3000
 // (34 MB) 34.5 against 31.4.
 constexpr int kShortBytesFew = 16 << 20;
 constexpr int kShortBytes = 24 << 20;
