@@ -182,9 +182,10 @@ int warp34_paged_attention_bf16(const warp34_exec* ex, const warp34_kv_layer_lay
                                 const void* q_in, void* attn_out, int num_q_heads); /* warp34_cuda.h:366-367 */
 
 /* Test-only kernel selector (op_paged_attn.cu:1451-1519): use_64q == 0 runs the decode / verify
- * kernel as a single pass (no split, scratch untouched), any other value the 128-row MFMA tile
- * kernel (when the layout admits it: a power-of-two number of q heads per kv head; otherwise as 0).
- * Both compute the same function, with different summation orders. */
+ * kernel as a single pass (no split, scratch untouched), any other value the MFMA tile kernels
+ * (when the layout admits them: a power-of-two number of q heads per kv head; otherwise as 0), 2 the
+ * 256-row one for TQ4 pages too, whatever the number of tiles (its bits are those of the 128-row one).
+ * All compute the same function, the first with another summation order. */
 int warp34_paged_attention_f16_force_kernel_for_test(
     const warp34_exec* ex, const warp34_kv_layer_layout* layout,
     const warp34_attention_batch* batch,

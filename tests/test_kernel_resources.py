@@ -1,4 +1,4 @@
-"""What the built library's kernel descriptors say: the row-format attention kernels keep everything in registers.
+"""What the built library's kernel descriptors say: the row-format attention and the prefill kernels keep everything in registers.
 A reload from scratch memory waits for the row loads in flight as well, which the kernels place their own waits for."""
 import os
 import re
@@ -39,4 +39,11 @@ def kernel_scratch_bytes(tmp_path):
 def test_row_format_kernels_do_not_spill(tmp_path):
     kernels = {k: v for k, v in kernel_scratch_bytes(tmp_path).items() if "paged_attn_rows" in k}
     assert len(kernels) >= 20, sorted(kernels)
+    assert {k: v for k, v in kernels.items() if v} == {}
+
+
+@pytest.mark.skipif(not os.path.exists(READELF), reason="no llvm-readelf")
+def test_prefill_kernels_do_not_spill(tmp_path):
+    kernels = {k: v for k, v in kernel_scratch_bytes(tmp_path).items() if "paged_prefill" in k}
+    assert len(kernels) >= 16, sorted(kernels)
     assert {k: v for k, v in kernels.items() if v} == {}

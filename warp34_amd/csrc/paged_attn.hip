@@ -1880,6 +1880,7 @@ __global__ __launch_bounds__(GROUPS * 64) void split_merge_kernel(const float* p
 
 #include "paged_attn_rows.h"
 #include "paged_prefill_tq4.h"
+#include "paged_prefill_wide.h"
 #include "qsa_sparse_tq4.h"
 #include "qsa_sparse_rows.h"
 
@@ -2244,11 +2245,10 @@ static int launch_tq4(const warp34_exec* ex, const warp34_kv_layer_layout* layou
             T.tok_tile = kPfRows / q_group;
             T.key_floor = nullptr;
             const int pf_tiles = (batch->total_tokens + T.tok_tile - 1) / T.tok_tile;
-            using PfL = PfLds<WARP34_KV_FORMAT_TQ4>;
-            rc = ensure_dynamic_lds(paged_prefill_tq4_kernel<TQ, WARP34_KV_FORMAT_TQ4, false, true, true>, PfL::kSmem, true);
+                        rc = ensure_dynamic_lds(paged_prefill_tq4_kernel<TQ, true>, kPfSmem, true);
             if (rc) return rc;
-            hipLaunchKernelGGL((paged_prefill_tq4_kernel<TQ, WARP34_KV_FORMAT_TQ4, false, true, true>),
-                               dim3((unsigned)(pf_tiles * parts), (unsigned)kv_subs, 1u), dim3(12 * 64), PfL::kSmem,
+            hipLaunchKernelGGL((paged_prefill_tq4_kernel<TQ, true>),
+                               dim3((unsigned)(pf_tiles * parts), (unsigned)kv_subs, 1u), dim3(12 * 64), kPfSmem,
                                stream, T);
             rc = (int)hipGetLastError();
             if (rc) return rc;
@@ -2464,8 +2464,7 @@ static int launch_rows(const warp34_exec* ex, const warp34_kv_layer_layout* layo
     return P.max_chunks > 1 ? launch_split_merge<TQ, false, HD>(P, P.max_chunks, 1.0f, stream) : 0;
 }
 
-// Chunked prefill over TQ4 pages: one workgroup per (128-row query tile, kv head x q subgroup,
-// request); no split (a prefill batch has thousands of tiles).
+// Chunked prefill: no split over the keys (a prefill batch has hundreds of tiles).
 static bool prefill_tq4_applicable(const warp34_kv_layer_layout* layout, const warp34_attention_batch* batch,
                                    int num_q_heads) {
     const int gqa = num_q_heads / layout->local_kv_heads;
@@ -2483,7 +2482,7 @@ static bool prefill_tq4_applicable(const warp34_kv_layer_layout* layout, const w
 template <typename TQ, int KVF>
 static int launch_prefill_tq4(const warp34_exec* ex, const warp34_kv_layer_layout* layout,
                               const warp34_attention_batch* batch, const void* q, void* out, int num_q_heads,
-                              const void* gate) {
+                              const void* gate, bool force_wide) {
     AttnParams P{};
     P.L = *layout;
     P.B = *batch;
@@ -2506,37 +2505,46 @@ static int launch_prefill_tq4(const warp34_exec* ex, const warp34_kv_layer_layou
     P.q_group = q_group;
     P.q_group_magic = q_group_magic_for(q_group);
     P.q_subgroups = P.gqa / q_group;
-    P.tok_tile = kPfRows / q_group;
     P.max_chunks = 1;
     P.min_upc = kMinUnitsPerChunk;
-    const int tiles = (batch->max_q_len + P.tok_tile - 1) / P.tok_tile;
-    const dim3 grid((unsigned)tiles, (unsigned)(layout->local_kv_heads * P.q_subgroups), (unsigned)batch->num_reqs);
     P.rot_q = layout->k_transform == WARP34_KV_TRANSFORM_RADEMACHER_WHT256 ? 1 : 0;
     P.rot_out = layout->v_transform == WARP34_KV_TRANSFORM_RADEMACHER_WHT256 ? 1 : 0;
+    const int kv_subs = layout->local_kv_heads * P.q_subgroups;
+    if constexpr (KVF == WARP34_KV_FORMAT_TQ4) {
+        // 128-row tiles on twelve waves (eight multiply, four dequantise) take 0.57 of the time of a 256-row tile, the
+        // wide kernel's half tiles 0.65.  us, 128-row tiles / wide: 128 tiles of 256 rows 140 / 161, 206 303 / 301, 230 514 / 539,
+        // 256 795 / 764, 318 1 287 / 1 240, 640 2 182 / 2 007, 850 3 098 / 2 813.
+        const long long wide = ((long long)batch->total_tokens * q_group / pw_rows(2) + (batch->num_reqs + 1) / 2) * kv_subs;
+        if (wide < kPwTq4Tiles && !force_wide) {
+            P.tok_tile = kPfRows / q_group;
+            const dim3 grid((unsigned)((batch->max_q_len + P.tok_tile - 1) / P.tok_tile), (unsigned)kv_subs, (unsigned)batch->num_reqs);
+            const int rc = ensure_dynamic_lds(paged_prefill_tq4_kernel<TQ, false>, kPfSmem, true);
+            if (rc) return rc;
+            hipLaunchKernelGGL((paged_prefill_tq4_kernel<TQ, false>), grid, dim3(12 * 64), kPfSmem, (hipStream_t)ex->stream, P);
+            return (int)hipGetLastError();
+        }
+    }
+    P.tok_tile = pw_rows(2) / q_group;
+    P.bal_tiles = (batch->max_q_len + P.tok_tile - 1) / P.tok_tile;
+    // (the last round's cut tiles: fewer than kPwCus / 2 workgroups more)
+    const long long wgs = (long long)P.bal_tiles * kv_subs * batch->num_reqs + kPwCus / 2;
+    if (wgs > 0x7fffffffll) return (int)hipErrorNotSupported;
+    const dim3 grid((unsigned)std::min<long long>(wgs, 1 << 20), (unsigned)((wgs + (1 << 20) - 1) >> 20));
     constexpr bool k8bit = KVF == WARP34_KV_FORMAT_FP8_E4M3 || KVF == WARP34_KV_FORMAT_Q8_0;
-    int rc;
     if constexpr (k8bit) {
         if (P.rot_out) {  // rotated 8-bit value rows: codes in the value tile, block scales in the weights
-            rc = ensure_dynamic_lds(paged_prefill_tq4_kernel<TQ, KVF, true>, PfLds<KVF>::kSmem, true);
+            const int rc = ensure_dynamic_lds(paged_prefill_wide_kernel<TQ, KVF, true>, pw_smem<KVF>(), true);
             if (rc) return rc;
-            hipLaunchKernelGGL((paged_prefill_tq4_kernel<TQ, KVF, true>), grid, dim3(kPfWaves * 64), PfLds<KVF>::kSmem,
+            hipLaunchKernelGGL((paged_prefill_wide_kernel<TQ, KVF, true>), grid, dim3(kPfWaves * 64), pw_smem<KVF>(),
                                (hipStream_t)ex->stream, P);
             return (int)hipGetLastError();
         }
     }
-    if constexpr (KVF == WARP34_KV_FORMAT_TQ4) {  // twelve waves: eight multiply, four dequantise
-        rc = ensure_dynamic_lds(paged_prefill_tq4_kernel<TQ, KVF, false, true>, PfLds<KVF>::kSmem, true);
-        if (rc) return rc;
-        hipLaunchKernelGGL((paged_prefill_tq4_kernel<TQ, KVF, false, true>), grid, dim3(12 * 64), PfLds<KVF>::kSmem,
-                           (hipStream_t)ex->stream, P);
-        return (int)hipGetLastError();
-    } else {
-        rc = ensure_dynamic_lds(paged_prefill_tq4_kernel<TQ, KVF, false>, PfLds<KVF>::kSmem, true);
-        if (rc) return rc;
-        hipLaunchKernelGGL((paged_prefill_tq4_kernel<TQ, KVF, false>), grid, dim3(kPfWaves * 64), PfLds<KVF>::kSmem,
-                           (hipStream_t)ex->stream, P);
-        return (int)hipGetLastError();
-    }
+    const int rc = ensure_dynamic_lds(paged_prefill_wide_kernel<TQ, KVF, false>, pw_smem<KVF>(), true);
+    if (rc) return rc;
+    hipLaunchKernelGGL((paged_prefill_wide_kernel<TQ, KVF, false>), grid, dim3(kPfWaves * 64), pw_smem<KVF>(),
+                       (hipStream_t)ex->stream, P);
+    return (int)hipGetLastError();
 }
 
 static bool is_kv16(const warp34_kv_layer_layout* l, int format) {
@@ -2607,9 +2615,9 @@ static int attention_entry(const warp34_exec* ex, const warp34_kv_layer_layout* 
                            const warp34_attention_batch* batch, const void* q, void* out, int num_q_heads,
                            int force, const void* gate = nullptr) {
     // force (the test selector): 0 = the dispatch below, 1 = the decode / verify kernel as a single
-    // pass, 2 = the 128-row tile kernel (where the batch shape admits it, else as 1)
+    // pass, 2 = the tile kernels (where the batch shape admits them, else as 1), 3 = as 2, TQ4 pages on the wide one
     const int force_single = force != 0 ? 1 : 0;
-    const bool force_tile = force == 2;
+    const bool force_tile = force == 2 || force == 3, force_wide = force == 3;
     if (layout->local_kv_heads <= 0 || num_q_heads % layout->local_kv_heads != 0 || batch->num_reqs <= 0 ||
         !batch->query_start_loc || !batch->seq_lens_after || !batch->block_tables ||
         batch->max_blocks_per_req <= 0 || batch->sliding_window < 0 ||
@@ -2623,7 +2631,7 @@ static int attention_entry(const warp34_exec* ex, const warp34_kv_layer_layout* 
         const bool many_rows = batch->max_q_len >= 32 &&
                                (long long)batch->total_tokens * num_q_heads >= 128ll * kPfRows;
         if ((force_tile || (!force && many_rows)) && prefill_tq4_applicable(layout, batch, num_q_heads))
-            return launch_prefill_tq4<TQ, WARP34_KV_FORMAT_TQ4>(ex, layout, batch, q, out, num_q_heads, gate);
+            return launch_prefill_tq4<TQ, WARP34_KV_FORMAT_TQ4>(ex, layout, batch, q, out, num_q_heads, gate, force_wide);
         return launch_tq4<TQ>(ex, layout, batch, q, out, num_q_heads, force_single, gate);
     }
     // 16-bit pages: the storage type must be the query type (FP16 pages with the f16 entry
@@ -2637,7 +2645,7 @@ static int attention_entry(const warp34_exec* ex, const warp34_kv_layer_layout* 
         if (layout->head_dim == 128)
             return launch_rows<TQ, TQ::kStorageFormat, false, 128>(ex, layout, batch, q, out, num_q_heads, force_single, gate);
         if ((force_tile || (!force && many_rows)) && prefill_tq4_applicable(layout, batch, num_q_heads))
-            return launch_prefill_tq4<TQ, TQ::kStorageFormat>(ex, layout, batch, q, out, num_q_heads, gate);
+            return launch_prefill_tq4<TQ, TQ::kStorageFormat>(ex, layout, batch, q, out, num_q_heads, gate, force_wide);
         return launch_rows<TQ, TQ::kStorageFormat>(ex, layout, batch, q, out, num_q_heads, force_single, gate);
     }
     // 8-bit pages (the tail layers of the default TQ4 policy, cache.rs:87-109)
@@ -2647,7 +2655,7 @@ static int attention_entry(const warp34_exec* ex, const warp34_kv_layer_layout* 
         const bool many_rows = batch->max_q_len >= 32 &&
                                (long long)batch->total_tokens * num_q_heads >= 128ll * kPfRows;
         if ((force_tile || (!force && many_rows)) && prefill_tq4_applicable(layout, batch, num_q_heads))
-            return launch_prefill_tq4<TQ, WARP34_KV_FORMAT_FP8_E4M3>(ex, layout, batch, q, out, num_q_heads, gate);
+            return launch_prefill_tq4<TQ, WARP34_KV_FORMAT_FP8_E4M3>(ex, layout, batch, q, out, num_q_heads, gate, force_wide);
         if (rows_vres(layout))
             return launch_rows<TQ, WARP34_KV_FORMAT_FP8_E4M3, true>(ex, layout, batch, q, out, num_q_heads, force_single, gate);
         return launch_rows<TQ, WARP34_KV_FORMAT_FP8_E4M3>(ex, layout, batch, q, out, num_q_heads, force_single, gate);
@@ -2657,7 +2665,7 @@ static int attention_entry(const warp34_exec* ex, const warp34_kv_layer_layout* 
         const bool many_rows = batch->max_q_len >= 32 &&
                                (long long)batch->total_tokens * num_q_heads >= 128ll * kPfRows;
         if ((force_tile || (!force && many_rows)) && prefill_tq4_applicable(layout, batch, num_q_heads))
-            return launch_prefill_tq4<TQ, WARP34_KV_FORMAT_Q8_0>(ex, layout, batch, q, out, num_q_heads, gate);
+            return launch_prefill_tq4<TQ, WARP34_KV_FORMAT_Q8_0>(ex, layout, batch, q, out, num_q_heads, gate, force_wide);
         if (rows_vres(layout))
             return launch_rows<TQ, WARP34_KV_FORMAT_Q8_0, true>(ex, layout, batch, q, out, num_q_heads, force_single, gate);
         return launch_rows<TQ, WARP34_KV_FORMAT_Q8_0>(ex, layout, batch, q, out, num_q_heads, force_single, gate);
@@ -2838,8 +2846,8 @@ extern "C" int warp34_paged_attention_f16_force_kernel_for_test(
     if (rc) return rc;
     if (batch->total_tokens <= 0 || num_q_heads <= 0) return 0;
     // the reference's selector picks the 16-row kernel (0) or one of its 64 / 128-row prefill kernels;
-    // here: the decode / verify kernel as a single pass, or the 128-row tile kernel
-    return attention_entry<F16>(ex, layout, batch, q_in, attn_out, num_q_heads, use_64q == 0 ? 1 : 2);
+    // here: the decode / verify kernel as a single pass, the tile kernels, or (2) the 256-row one for TQ4 pages too
+    return attention_entry<F16>(ex, layout, batch, q_in, attn_out, num_q_heads, use_64q == 0 ? 1 : use_64q == 2 ? 3 : 2);
 }
 
 // Scratch that lets a batch split fully, computed the way the launchers compute it.
