@@ -8,7 +8,7 @@
 // counterpart in the reference; its result equals operator + warp34_kv_cache_write_strided bit
 // for bit (the same row encoders).
 //
-// Mapping: one workgroup (4 waves) per token.  The last wave computes the token's sine / cosine
+// Mapping: one workgroup (4 waves) per token, or several with one item per wave (kFqSpreadTokens).  The last wave computes the token's sine / cosine
 // values (they depend on the token's three positions and on the pair index only, not on the
 // head) in double precision and leaves them in LDS, fp16-rounded as the reference does, while
 // the other waves normalise their first rows.  Every wave takes items in turn, one item per wave, the two 32-lane halves of the wave each
@@ -30,6 +30,11 @@
 namespace w34 {
 
 constexpr int kFqMaxPairs = 128;  // rotary_dim / 2
+// Up to this many tokens a token's items go to several workgroups, one item per wave (a wave's items in turn are
+// a chain of memory round trips, and the K / V items came last).  us, one workgroup per token / spread, 16 q + 2 kv heads, TQ4:
+// 1 token 7.0 / 5.0, 64 7.5 / 5.5, 256 8.5 / 6.8, 512 10.1 / 9.9, 1 024 12.2 / 15.0; 32 + 4 heads: 1 token 9.0 / 5.3, 256 11.6 / 10.0,
+// 512 17.1 / 16.3, 1 024 18.2 / 23.0; Q8_0 alike.
+constexpr int kFqSpreadTokens = 256;
 
 struct FusedQkParams {
     const uint16_t* q_gate_in;
@@ -50,6 +55,7 @@ struct FusedQkParams {
     float inv_freq[kFqMaxPairs];
 };
 
+template <bool SPREAD>
 __global__ __launch_bounds__(256) void fused_qk_norm_rope_gate_kernel(const FusedQkParams P) {
     __shared__ float s_cos[kFqMaxPairs], s_sin[kFqMaxPairs];
     __shared__ __align__(16) uint16_t s_row[4][2][256];
@@ -89,7 +95,9 @@ __global__ __launch_bounds__(256) void fused_qk_norm_rope_gate_kernel(const Fuse
     uint16_t* row = s_row[wave][half_id];
     const bool owns_vec = 8 * l32 < hd;
 
-    for (int it = wave; it < n_items; it += 4) {  // wave-uniform
+    // SPREAD: three items per workgroup, one per wave, beside the wave of the sine / cosine values
+    const int first = SPREAD ? (wave == 3 ? n_items : 3 * (int)blockIdx.y + wave) : wave;
+    for (int it = first; it < n_items; it += SPREAD ? n_items : 4) {  // wave-uniform
         const bool is_q = it < q_items;
         const int kv_head = is_q ? 0 : it - q_items;
         const bool is_v_half = !is_q && half_id == 1;
@@ -256,8 +264,14 @@ static int launch_fused_qk(const warp34_exec* ex, const void* q_gate_in, const v
         const float pw = (float)std::pow((double)rope_theta, (double)expo);
         P.inv_freq[i] = 1.0f / pw;
     }
-    hipLaunchKernelGGL(fused_qk_norm_rope_gate_kernel, dim3((unsigned)num_tokens), dim3(256), 0,
-                       (hipStream_t)ex->stream, P);
+    const int items = (num_q_heads + 1) / 2 + num_kv_heads;
+    if (num_tokens <= kFqSpreadTokens) {
+        hipLaunchKernelGGL(fused_qk_norm_rope_gate_kernel<true>, dim3((unsigned)num_tokens, (unsigned)((items + 2) / 3)), dim3(256), 0,
+                           (hipStream_t)ex->stream, P);
+    } else {
+        hipLaunchKernelGGL(fused_qk_norm_rope_gate_kernel<false>, dim3((unsigned)num_tokens), dim3(256), 0,
+                           (hipStream_t)ex->stream, P);
+    }
     return (int)hipGetLastError();
 }
 
