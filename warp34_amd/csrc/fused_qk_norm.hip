@@ -8,8 +8,8 @@
 // counterpart in the reference; its result equals operator + warp34_kv_cache_write_strided bit
 // for bit (the same row encoders).
 //
-// Mapping: one workgroup (4 waves) per token, or several with one item per wave (kFqSpreadTokens).  The last wave computes the token's sine / cosine
-// values (they depend on the token's three positions and on the pair index only, not on the
+// Mapping: one workgroup (4 waves) per token, or several with one item per wave (kFqSpreadTokens).
+// The last wave computes the token's sine / cosine values (they depend on the token's three positions and on the pair index only, not on the
 // head) in double precision and leaves them in LDS, fp16-rounded as the reference does, while
 // the other waves normalise their first rows.  Every wave takes items in turn, one item per wave, the two 32-lane halves of the wave each
 // playing the part of the reference's vector lanes: a Q item is two Q heads, a KV item is one K
@@ -139,7 +139,7 @@ __global__ __launch_bounds__(256) void fused_qk_norm_rope_gate_kernel(const Fuse
         }
         const float sum_sq = half_wave_sum(acc, lane);
         const float mean = sum_sq / (float)hd + P.eps;
-        const float inv_rms = (float)(1.0 / sqrt((double)mean));
+        const float inv_rms = rsqrt_rn(mean);
         uint32_t nw[4];
 #pragma unroll
         for (int k = 0; k < 4; ++k) {

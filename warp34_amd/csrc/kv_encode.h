@@ -17,6 +17,22 @@
 
 namespace w34 {
 
+// (float)(1.0 / sqrt((double)x)) for a normal x: the hardware's reciprocal root (within 1 ulp) and one second-order
+// correction in double precision, 8 double-precision instructions instead of 35 (the append of 4 096 tokens
+// 9.1 -> 8.8 us).  1 / sqrt(x) of a float x is never nearer than 2^-51.7 (relative) to the middle of two floats, and
+// over all significands of two binades and starting values up to 2 ulp off both forms round to the same float
+// (checked on the host).
+__device__ __forceinline__ float rsqrt_rn_normal(float x) {
+    const double y = (double)__builtin_amdgcn_rsqf(x);
+    const double r = __builtin_fma(-(y * y), (double)x, 1.0);
+    return (float)__builtin_fma(y, r * __builtin_fma(r, 0.375, 0.5), y);
+}
+// the same for every x
+__device__ __forceinline__ float rsqrt_rn(float x) {
+    if (x >= 1.17549435e-38f && x <= 3.402823466e38f) return rsqrt_rn_normal(x);
+    return (float)(1.0 / sqrt((double)x));
+}
+
 // 32-lane xor butterfly sum, offsets 16,8,4,2,1 (tq4_kv_common.cuh:54-60); cross-lane moves are
 // DPP / lane-swap VALU operations (lane_xor), not LDS permutes.
 __device__ __forceinline__ float half_wave_sum(float v, int lane) {
@@ -113,34 +129,44 @@ __device__ __forceinline__ float row_sum_of_groups(float s, int lane) {
 }
 
 // Codes of a lane's eight elements -- the number of boundaries below the value (op_kv_cache.cu:186-189) --
-// and their centroids.  Binary search over the sorted boundaries in heap order: node 1 is the middle, the
-// children of node k are 2 k and 2 k + 1, and node 16 + code is what the search ends at, so the node
-// number is both the next lane to fetch from and, in the end, the code.  `tab_b`, `tab_c` hold threshold
-// node / centroid i in every lane with lane % 16 == i (ds_bpermute: no memory access).  The first two thresholds
-// are selected between constants.  `at` is four times the node, the byte address ds_bpermute takes.
-// Instruction-bound; a search by indices worked out from the code needs an index per level and three fetches per
-// element instead of two: 4 096 tokens x 2 heads of K and V, 9.9 us a call with it, 9.7 with this.
-__device__ __forceinline__ int tq4_heap_boundary(int lane) {
-    const int k = (lane & 15) > 0 ? (lane & 15) : 1;
-    const int level = 31 - __builtin_clz(k);
-    return __float_as_int(kBoundaries[((2 * (k - (1 << level)) + 1) << (3 - level)) - 1]);
+// and their centroids.  64 equal cells of 1 / 120.25 around zero, of which no one holds two boundaries and no boundary is
+// within a quarter of a cell of an edge: the cell of u (rounded as it may be) names the one boundary u has to be
+// compared with and the code below it.  The cell tables are held across the lanes and fetched with ds_bpermute
+// (no memory access); what the first two fetches give is the lane of the third, 16 + code.
+// Instruction-bound: 4 096 tokens x 2 heads of K and V, us a call: 9.7 with a binary search (two thresholds by selection, two
+// fetched), 9.1 with this.
+constexpr float kCellsPerUnit = 120.25f, kCellOfZero = 31.5f;
+constexpr uint64_t tq4_cells_with_boundary() {
+    uint64_t cells = 0;
+    for (int k = 0; k < 15; ++k) cells |= 1ull << (int)(kBoundaries[k] * kCellsPerUnit + kCellOfZero);
+    return cells;
 }
-__device__ __forceinline__ void tq4_codes(const float (&v)[8], float inv_norm, int tab_b, int tab_c, uint32_t& halves_lo,
+static_assert(__builtin_popcountll(tq4_cells_with_boundary()) == 15, "every boundary in a cell of its own");
+struct Tq4Tables {  // lane i: of cell i the boundary in it (or +inf) and 4 (16 + number of boundaries below it); centroid i % 16
+    int boundary, at, centroid;
+};
+__device__ __forceinline__ Tq4Tables tq4_tables(int lane) {
+    constexpr uint64_t kCells = tq4_cells_with_boundary();
+    const int below = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(kCells >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)kCells, 0u));
+    const bool has = (kCells >> lane) & 1ull;
+    const float boundary = kBoundaries[below < 15 ? below : 14];
+    return Tq4Tables{has ? __float_as_int(boundary) : 0x7F800000, 4 * (16 + below), __float_as_int(kCentroids[lane & 15])};
+}
+__device__ __forceinline__ void tq4_codes(const float (&v)[8], float inv_norm, const Tq4Tables& tab, uint32_t& halves_lo,
                                           uint32_t& halves_hi, float (&c)[8]) {
     int at[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
         const float u = v[j] * inv_norm;
-        const bool upper = u > kBoundaries[7];
-        const float t1 = upper ? kBoundaries[11] : kBoundaries[3];
-        int a = (upper ? 24 : 16) + ((u > t1) ? 4 : 0);
-#pragma unroll
-        for (int lvl = 2; lvl < 4; ++lvl) {
-            const float t = __int_as_float(__builtin_amdgcn_ds_bpermute(a, tab_b));
-            a = 2 * a + ((u > t) ? 4 : 0);
-        }
-        at[j] = a;  // 4 (16 + code)
-        c[j] = __int_as_float(__builtin_amdgcn_ds_bpermute(a, tab_c));
+        // four times the cell: the byte address ds_bpermute takes, which ignores its two low bits.  The conversion
+        // saturates, NaN to 0 (a NaN is above no boundary).
+        uint32_t cell;
+        asm("v_cvt_u32_f32 %0, %1" : "=v"(cell) : "v"(__builtin_fmaf(u, 4.0f * kCellsPerUnit, 4.0f * kCellOfZero)));
+        cell = cell < 255u ? cell : 255u;
+        const float t = __int_as_float(__builtin_amdgcn_ds_bpermute((int)cell, tab.boundary));
+        const int below = __builtin_amdgcn_ds_bpermute((int)cell, tab.at);
+        at[j] = below + ((u > t) ? 4 : 0);  // 4 (16 + code)
+        c[j] = __int_as_float(__builtin_amdgcn_ds_bpermute(at[j], tab.centroid));
     }
     // nibble pairs (even element low), two bytes per half: 4 (code bytes) + what the sixteens add up to
     constexpr int kSixteens = 64 * (1 + 16) * (1 + 256);
@@ -154,20 +180,19 @@ __device__ __forceinline__ void tq4_codes(const float (&v)[8], float inv_norm, i
 // scale block, lanes 16-31 the second: one instruction stream computes both norms and scales.
 __device__ __forceinline__ void tq4_encode_row(float (&v)[8], int lane, uint8_t* row) {
     const int l32 = lane & 31;
-    const int tab_b = tq4_heap_boundary(lane);
-    const int tab_c = __float_as_int(kCentroids[lane & 15]);
+    const Tq4Tables tab = tq4_tables(lane);
     sign_wht256(v, lane);
 
     float p[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) p[j] = v[j] * v[j];
     const float s_sq = row_sum_of_groups(group32_sums(p, lane), lane);
-    const float rs = (float)(1.0 / sqrt((double)s_sq));
-    const float inv_norm = (s_sq > 1e-20f) ? (0.7071067811865475f * rs) : 0.0f;
+    // (an infinite sum has the reciprocal root 0)
+    const float inv_norm = (s_sq > 1e-20f && s_sq <= 3.402823466e38f) ? (0.7071067811865475f * rsqrt_rn_normal(s_sq)) : 0.0f;
 
     float c[8];
     uint32_t lo, hi;
-    tq4_codes(v, inv_norm, tab_b, tab_c, lo, hi, c);
+    tq4_codes(v, inv_norm, tab, lo, hi, c);
     // byte m of a 64-byte block holds elements 2m (low nibble) and 2m + 1 (high nibble):
     // elements 8 l32 .. + 7 are bytes 4 (l32 % 16) .. + 3 of block l32 / 16
     uint8_t* wdst = row + 66 * (l32 >> 4) + 2 + 4 * (l32 & 15);
@@ -203,8 +228,7 @@ __device__ __forceinline__ float block128_sum(const float (&p)[8], int lane) {
 
 __device__ __forceinline__ void tq4_encode_row_plain(const float (&v)[8], int lane, uint8_t* row) {
     const int l32 = lane & 31;
-    const int tab_b = tq4_heap_boundary(lane);
-    const int tab_c = __float_as_int(kCentroids[lane & 15]);
+    const Tq4Tables tab = tq4_tables(lane);
     float p[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) p[j] = v[j] * v[j];
@@ -212,7 +236,7 @@ __device__ __forceinline__ void tq4_encode_row_plain(const float (&v)[8], int la
     const float inv_norm = (norm_x > 1e-12f) ? (0.7071067811865475f / norm_x) : 0.0f;
     float c[8];
     uint32_t lo, hi;
-    tq4_codes(v, inv_norm, tab_b, tab_c, lo, hi, c);
+    tq4_codes(v, inv_norm, tab, lo, hi, c);
     // ("q = b + 1 for the last boundary b below u" over ascending boundaries = the number of boundaries below u)
     uint8_t* wdst = row + 66 * (l32 >> 4) + 2 + 4 * (l32 & 15);
     *reinterpret_cast<uint16_t*>(wdst) = (uint16_t)lo;

@@ -92,7 +92,7 @@ __global__ __launch_bounds__(256) void qk_norm_rope_kernel(const NormRopeParams 
     float s = ((sq[0] + sq[4]) + (sq[2] + sq[6])) + ((sq[1] + sq[5]) + (sq[3] + sq[7]));
     s = half_wave_sum(s, lane);
     const float mean = s / (float)dim + P.eps;
-    const float inv = (float)(1.0 / sqrt((double)mean));
+    const float inv = rsqrt_rn(mean);
 
     // rotated values of this lane: out[c] and out[half + c] for c = l32, l32 + 32, ... < half
     float lo[4], hi[4];
