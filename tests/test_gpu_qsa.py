@@ -254,3 +254,27 @@ def test_argument_checks_and_unsupported_formats():
     rc = G.lib().warp34_qsa_sparse_paged_attn_f16(C.byref(ex), G.ptr(t), None, C.byref(L), G.ptr(t), G.ptr(t),
                                                   G.ptr(t), G.ptr(t), None, G.ptr(out), 0, 8, 4, 0.0625)
     assert rc == 0
+
+
+@pytest.mark.parametrize("block_size", [16, 48])
+@pytest.mark.parametrize("heads", [1, 8, 9, 16])
+@pytest.mark.parametrize("scratch", [0, SCRATCH])
+def test_lists_of_every_length_against_the_capacity(block_size, heads, scratch):
+    """Lists from empty to the full 600 groups (75 units: without a split a wave has up to ten, the entries of eight are
+    held at a time), which start elsewhere than the capacity says; pages that are no power of two; one, eight,
+    nine and sixteen q heads on one kv head (eight columns a pass in the sum over the waves); skipped groups; the last keys
+    behind the position."""
+    rng = np.random.default_rng(19)
+    seq, select_k = 3001, 600
+    lengths = [600, 0, 1, 8, 9, 63, 64, 65, 511, 513, 577, 599]
+    pool, bt, k, v, _, _, _ = make_case(FMT_TQ4, block_size, [seq], [1], 671, DT_F16, kv_heads=1)
+    n_tok = len(lengths)
+    q = oracle.fill_normal(n_tok * heads * 256, 672, DT_F16).reshape(n_tok, heads, 256)
+    sel_phys, sel_log, num_sel = _selection(bt, seq, block_size, n_tok, select_k, rng)
+    num_sel[:] = lengths
+    sel_phys[0, rng.permutation(select_k)[:40]] = -1
+    for t in range(n_tok):
+        sel_phys[t, num_sel[t]:] = 0x7fffff
+    seq_pos = np.full(n_tok, seq - 1, dtype=np.int32)
+    seq_pos[9] = 1500
+    _check(pool, v, q, sel_phys, sel_log, num_sel, seq_pos, heads, scratch=scratch, what="list lengths")

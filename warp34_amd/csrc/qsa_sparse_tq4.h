@@ -4,9 +4,14 @@
 // The streaming core is the one of the dense TQ4 decode kernel (pair table in LDS, S^T = K Q'^T
 // and O^T += V^T P^T on v_mfma_f32_16x16x32_f16, one query column per lane); what differs is where
 // the keys come from.  A 32-token unit is eight selected groups; a group is four consecutive rows
-// of one page, 528 bytes = 33 16-byte pieces, so a unit is still 4 x 132 pieces per K and V and
-// lands in LDS in the layout the core expects.  Only the piece addresses change: they are
-// per-lane (group id -> page, row) instead of a wave-uniform run base.
+// of one page, 528 bytes = 33 16-byte pieces: one LDS-direct load of 33 lanes from a wave-uniform address, and the unit
+// lies in LDS in the layout the core expects.
+// What bounds it: two dependent memory round trips (the list, the rows), the table and one or two units per
+// wave for a small batch; the instructions of the unit for a large one (eight units a wave).  Hence: the list entries
+// of eight units in one load, K rows asked for before V rows and the next unit's before this one's products, table reads
+// a batch ahead of the MFMAs, one barrier before the loop and one behind it.  us a call, 513 groups, against rows through
+// registers, K and V waited for together, two barriers on either side: 16 tokens 19.6 -> 17.4, 64 30.6 -> 25.8, 256
+// 85 -> 66; 16 tokens x 64 groups 12.6 -> 11.2.
 //
 //   grid  = (query tokens, kv heads x q subgroups, splits), block = 8 waves
 //   split = an equal share of the token's units; every split writes an (m, l) record (l = 0
@@ -20,12 +25,12 @@
 namespace w34 {
 
 constexpr int kQsaWaves = 8;
-constexpr int kQsaLoopBytes = kLutBytes + kQsaWaves * kStageTq4;
-constexpr int kQsaColStride = 260;
-constexpr int kQsaRegion = 16 * kQsaColStride;  // floats per wave
-constexpr int kQsaMergeBytes = kQsaWaves * kQsaRegion * 4;
-constexpr int kQsaMlBytes = (kQsaWaves + 1) * 16 * 2 * 4;
-constexpr int kQsaSmem = (kQsaLoopBytes > kQsaMergeBytes ? kQsaLoopBytes : kQsaMergeBytes) + kQsaMlBytes;
+// LDS: the pair table, the waves' staging areas (after the loop: merge regions), the query rows, (m, l) of the waves
+constexpr int kQsaQStride = 264;
+constexpr int kQsaQBase = kLutBytes + kQsaWaves * kStageTq4;
+constexpr int kQsaMlBase = kQsaQBase + 16 * kQsaQStride * 2;
+constexpr int kQsaSmem = kQsaMlBase + kQsaWaves * 16 * 2 * 4;
+constexpr int kQsaGroupBytes = 4 * kTq4RowBytes;  // 33 pieces of 16 bytes
 constexpr int kQsaMaxSplits = 16;
 
 struct QsaParams {
@@ -114,21 +119,23 @@ __global__ __launch_bounds__(kQsaWaves * 64, 1) void qsa_sparse_tq4_kernel(const
     const int q_head_base = kv_head * P.gqa + (kv_sub - kv_head * P.q_subgroups) * P.q_group;
 
     // ---- this token's list ------------------------------------------------------------------------
-    // The counts and the list entries of this wave's first unit are requested together: the first
-    // unit is guessed from the list's capacity (exact when the list is full, the common case) and
-    // fetched again when the guess is wrong, so the guess changes the latency only.
+    // The counts and the list entries of this wave's first eight units (lane l: group l & 7 of unit l >> 3) are requested
+    // together: where the wave's units start is guessed from the list's capacity (exact when the list is full, the
+    // common case) and the entries are fetched again when the guess is wrong, so the guess changes the latency only.
     const int32_t* tok_phys = P.sel_phys + (size_t)tok * P.select_k;
     const int32_t* tok_log = P.sel_log + (size_t)tok * P.select_k;
     const int upc_guess = fast_div(((P.select_k + 7) >> 3) + P.n_splits - 1, P.n_splits);
     const int unit_guess = split * upc_guess + wave;
-    int spec_id = -1, spec_lg = 0;
-    {
-        const int gi = unit_guess * 8 + (lane & 7);
-        if (gi < P.select_k) {
-            spec_id = tok_phys[gi];
-            spec_lg = tok_log[gi];
+    int list_id = -1, list_lg = 0;
+    auto load_list = [&](int first_unit, int end) {
+        const int gi = (first_unit + kQsaWaves * (lane >> 3)) * 8 + (lane & 7);
+        list_id = -1, list_lg = 0;
+        if (gi < end) {
+            list_id = tok_phys[gi];
+            list_lg = tok_log[gi];
         }
-    }
+    };
+    load_list(unit_guess, P.select_k);
     int a_live = 1, a_sel = P.num_sel[tok], a_pos = P.seq_pos[tok];  // one vector load each, no scalar-cache trip
     if (P.valid_token_mask != nullptr) a_live = (int)P.valid_token_mask[tok];
 
@@ -168,86 +175,58 @@ __global__ __launch_bounds__(kQsaWaves * 64, 1) void qsa_sparse_tq4_kernel(const
     const uint8_t* k_base = reinterpret_cast<const uint8_t*>((uintptr_t)L.k_base) + (size_t)kv_head * L.k_head_stride_bytes;
     const uint8_t* v_base = reinterpret_cast<const uint8_t*>((uintptr_t)L.v_base) + (size_t)kv_head * L.v_head_stride_bytes;
     uint8_t* stage = stage_all + wave * kStageTq4;
-    // Piece p of a 16-row run belongs to group p / 33 of the run's four groups.  Lane l carries
-    // pieces l and 64 + l of every run; lanes 0-15 also carry the tail pieces 128 + (l & 3) of run
-    // l >> 2.
-    const int pa_g = lane / 33, pa_o = lane - 33 * pa_g;
-    const int pb_g = (64 + lane) / 33, pb_o = 64 + lane - 33 * pb_g;
-    const int pt_o = 29 + (lane & 3);  // pieces 128-131 are pieces 29-32 of group 3
-    u4 pf[9];
-    // lane l holds group (l & 7) of a unit: physical id (or -1) and first key position (or a
-    // position that is never visible)
-    auto load_groups = [&](int unit, int& id_vec, int& pos_vec) {
-        const int gi = unit * 8 + (lane & 7);
-        int id = -1, lg = 0;
-        if (gi < n_sel) {
-            id = tok_phys[gi];
-            lg = tok_log[gi];
-        }
-        id_vec = id;
-        pos_vec = id >= 0 ? 4 * lg : 0x3fffffff;
-    };
-    // Base of a group's four rows in the K and the V slab.  The ids come out of readlane, so this
-    // is scalar arithmetic; a skipped group reads group 0 of page 0: any TQ4 bytes dequantise to
+    const uint32_t stage_addr = (uint32_t)(kLutBytes + wave * kStageTq4);
+    // Of this lane's entry of the list: byte offsets of the group's rows in the K and the V slab, and its first key position
+    // (or a position that is never visible).  A skipped group reads group 0 of page 0: any TQ4 bytes dequantise to
     // finite values, and every key of such a group is masked.
-    auto group_base = [&](int id, const uint8_t*& kp, const uint8_t*& vp) {
-        const int gid = id >= 0 ? id : 0;
+    uint64_t k_off = 0, v_off = 0;
+    int pos_vec = 0x3fffffff;
+    auto locate_list = [&](int first_unit) {
+        const int gi = (first_unit + kQsaWaves * (lane >> 3)) * 8 + (lane & 7);
+        const bool skip = gi >= n_sel || list_id < 0;
+        const int gid = skip ? 0 : list_id;
         // pages of 2^k tokens (the usual case): shift and mask
         const int pg = P.gpp_shift >= 0 ? gid >> P.gpp_shift : gid / P.groups_per_page;
-        const int row = (gid - pg * P.groups_per_page) * 4;
-        kp = k_base + (size_t)pg * L.k_page_stride_bytes + (size_t)row * L.k_token_stride_bytes;
-        vp = v_base + (size_t)pg * L.v_page_stride_bytes + (size_t)row * L.v_token_stride_bytes;
+        const uint32_t row = (uint32_t)(gid - pg * P.groups_per_page) * 4u;
+        k_off = (uint64_t)(uint32_t)pg * L.k_page_stride_bytes + (uint64_t)row * L.k_token_stride_bytes;
+        v_off = (uint64_t)(uint32_t)pg * L.v_page_stride_bytes + (uint64_t)row * L.v_token_stride_bytes;
+        pos_vec = skip ? 0x3fffffff : 4 * list_lg;
     };
-    auto issue_loads = [&](int id_vec) {
-        const uint8_t *kt[2], *vt[2];
+    // The K or the V rows of the wave's unit j: eight LDS-direct loads of one group each.
+    auto issue_loads = [&](int j, uint64_t off, const uint8_t* base, uint32_t lds) __attribute__((always_inline)) {
+        const uint32_t lane16 = 16u * (uint32_t)lane;
+        if (lane < kQsaGroupBytes / 16) {
 #pragma unroll
-        for (int hr = 0; hr < 2; ++hr) {  // rows 0-15 / 16-31 of the unit = groups 0-3 / 4-7
-            const uint8_t *kg[4], *vg[4];
-#pragma unroll
-            for (int gi = 0; gi < 4; ++gi) group_base(__builtin_amdgcn_readlane(id_vec, 4 * hr + gi), kg[gi], vg[gi]);
-            // piece lane: group 0 or 1; piece 64 + lane: group 1, 2 or 3
-            const uint8_t* ka = (pa_g == 0 ? kg[0] : kg[1]) + 16 * pa_o;
-            const uint8_t* va = (pa_g == 0 ? vg[0] : vg[1]) + 16 * pa_o;
-            const uint8_t* kb = (pb_g == 1 ? kg[1] : pb_g == 2 ? kg[2] : kg[3]) + 16 * pb_o;
-            const uint8_t* vb = (pb_g == 1 ? vg[1] : pb_g == 2 ? vg[2] : vg[3]) + 16 * pb_o;
-            pf[2 * hr] = *(global_cu4*)ka;
-            pf[2 * hr + 1] = *(global_cu4*)kb;
-            pf[4 + 2 * hr] = *(global_cu4*)va;
-            pf[4 + 2 * hr + 1] = *(global_cu4*)vb;
-            kt[hr] = kg[3];
-            vt[hr] = vg[3];
-        }
-        {
-            const int r = (lane >> 2) & 3;  // run: K rows 0-15, K rows 16-31, V rows 0-15, V rows 16-31
-            const uint8_t* base = r == 0 ? kt[0] : r == 1 ? kt[1] : r == 2 ? vt[0] : vt[1];
-            pf[8] = *(global_cu4*)(base + 16 * pt_o);
+            for (int gi = 0; gi < 8; ++gi) {
+                const int at = 8 * (j & 7) + gi;
+                const uint64_t o = ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(off >> 32), at) << 32) |
+                                   (uint32_t)__builtin_amdgcn_readlane((int)off, at);
+                asm volatile(
+                    "s_mov_b32 m0, %2\n\ts_nop 0\n\t"
+                    "global_load_lds_dwordx4 %0, %1"
+                    :
+                    : "v"(lane16), "s"(base + o), "s"(lds + gi * kQsaGroupBytes)
+                    : "memory");
+            }
         }
     };
-    auto commit_loads = [&]() {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            *reinterpret_cast<u4*>(stage + r * kRunBytes + 16 * lane) = pf[2 * r];
-            *reinterpret_cast<u4*>(stage + r * kRunBytes + 1024 + 16 * lane) = pf[2 * r + 1];
-        }
-        if (lane < 16) *reinterpret_cast<u4*>(stage + (lane >> 2) * kRunBytes + 2048 + 16 * (lane & 3)) = pf[8];
-    };
+    auto issue_k = [&](int j) __attribute__((always_inline)) { issue_loads(j, k_off, k_base, stage_addr); };
+    auto issue_v = [&](int j) __attribute__((always_inline)) { issue_loads(j, v_off, v_base, stage_addr + 2 * kRunBytes); };
+    constexpr int kLoads = 8;  // load instructions of a unit's K (or V) rows
 
-    int unit = cu_first + wave;
-    int id_vec = -1, pos_vec = 0x3fffffff;
-    if (unit < cu_end) {
-        if (unit == unit_guess) {  // wave-uniform
-            const bool in_list = unit * 8 + (lane & 7) < n_sel;
-            id_vec = in_list ? spec_id : -1;
-            pos_vec = id_vec >= 0 ? 4 * spec_lg : 0x3fffffff;
-        } else {
-            load_groups(unit, id_vec, pos_vec);
-        }
-    }
-    issue_loads(id_vec);  // harmless for a wave without work
+    const int unit0 = cu_first + wave;
+    if (unit0 != unit_guess) load_list(unit0, n_sel);  // wave-uniform
+    locate_list(unit0);
+    // (the compiler's own loads end here, where they have landed: a wait for one of them behind the rows, which return in
+    // order, would wait for the rows too)
+#pragma unroll
+    for (int c = 0; c < kColsPerWave; ++c) asm volatile("" ::"v"(q_raw[c].x), "v"(q_raw[c].y));
+    asm volatile("" ::"v"(pos_vec));
+    if (unit0 < cu_end) issue_k(0);
 
     // ---- rotated, scaled fp16 queries to LDS, then the B operands of the QK MFMAs -----------------
-    constexpr int kQStride = 264;
-    _Float16* qlds = reinterpret_cast<_Float16*>(stage_all);
+    constexpr int kQStride = kQsaQStride;
+    _Float16* qlds = reinterpret_cast<_Float16*>(smem + kQsaQBase);
     const float q_scale = P.sm_scale * kLog2e * kLutInvGain;
 #pragma unroll
     for (int c = 0; c < kColsPerWave; ++c) {
@@ -264,7 +243,8 @@ __global__ __launch_bounds__(kQsaWaves * 64, 1) void qsa_sparse_tq4_kernel(const
         packed.y = pack_h2(qv[2] * q_scale, qv[3] * q_scale);
         *reinterpret_cast<uint2*>(qlds + col * kQStride + 4 * lane) = packed;
     }
-    __syncthreads();
+    if (unit0 < cu_end) issue_v(0);
+    __syncthreads();  // the table and the query rows are complete
     h8 bq[9];
     {
         const int kb = 8 * (b & 1) + 4 * (b >> 1);
@@ -285,7 +265,6 @@ __global__ __launch_bounds__(kQsaWaves * 64, 1) void qsa_sparse_tq4_kernel(const
 #pragma unroll
         for (int m = 0; m < 4; ++m) bq[5 + m] = *reinterpret_cast<const h8*>(qrow + 256 + 16 * (kb + m));
     }
-    __syncthreads();  // qlds is dead, the staging area may be overwritten; the table is complete
 
     const uint32_t lut_lane = (uint32_t)lane << 2;
     const bool col_ok = n < P.q_group;
@@ -298,51 +277,61 @@ __global__ __launch_bounds__(kQsaWaves * 64, 1) void qsa_sparse_tq4_kernel(const
 
     // One 32-token unit.  gp0 / gp1: first key position of the groups that hold this lane's key
     // slots 0-3 / 4-7 (group 4 (b & 1) + (b >> 1), and that group + 2).
-    auto process_unit = [&](int gp0, int gp1, const bool MASKED) {
+    auto process_unit = [&](int gp0, int gp1, const bool MASKED, const bool HAS_NEXT, int j_next) {
         const uint8_t* k_rows = stage;
         const uint8_t* v_rows = stage + 2 * kRunBytes;
+        wait_vm<kLoads>();  // the K rows have landed (the V rows may still be on their way)
         float sc[8];
-        uint32_t kw[2][9], ks0[2][4], ks16[2][4];
+        uint32_t kw[2][9], ks[2][4];
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
             const int arow = unit_token(s, n >> 2, n & 3);
             const uint32_t* row32 = reinterpret_cast<const uint32_t*>(k_rows + arow * kTq4RowBytes);
 #pragma unroll
             for (int mf = 0; mf < 9; ++mf) kw[s][mf] = row32[tq4_qk_dword(mf < 5 ? 0 : 1, mf < 5 ? mf : mf - 5, b)];
+            // (the two scales of a token in one register: lane n reads token n & 3, see the dense kernel)
+            const uint32_t* r32 = reinterpret_cast<const uint32_t*>(k_rows + unit_token(s, b, n & 3) * kTq4RowBytes);
+            const uint32_t mine = __builtin_amdgcn_perm(r32[16], r32[0], 0x07060100u);
+            ks[s][0] = row_bcast<0>(mine);
+            ks[s][1] = row_bcast<1>(mine);
+            ks[s][2] = row_bcast<2>(mine);
+            ks[s][3] = row_bcast<3>(mine);
+        }
+        wait_lds_reads();
+        if (HAS_NEXT) issue_k(j_next);
+        // six batches of three operands, the table reads of a batch in front of the MFMAs of the one before
+        constexpr int kQkOrder[9] = {0, 5, 1, 6, 2, 7, 3, 8, 4};
+        f4 s_acc[2][2];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const uint32_t* r32 = reinterpret_cast<const uint32_t*>(k_rows + unit_token(s, b, i) * kTq4RowBytes);
-                ks0[s][i] = r32[0];
-                ks16[s][i] = r32[16];
+        for (int s = 0; s < 2; ++s) s_acc[s][0] = s_acc[s][1] = f4{0.f, 0.f, 0.f, 0.f};
+        u4 qa[2][3];
+        auto qk_reads = [&](int bt, u4 (&a)[3]) __attribute__((always_inline)) {
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                const uint32_t w = kw[bt / 3][kQkOrder[3 * (bt % 3) + k]];
+                a[k][0] = lut_read(w, lut_lane, 0x0c0c0400u);
+                a[k][1] = lut_read(w, lut_lane, 0x0c0c0500u);
+                a[k][2] = lut_read(w, lut_lane, 0x0c0c0600u);
+                a[k][3] = lut_read(w, lut_lane, 0x0c0c0700u);
+            }
+        };
+        qk_reads(0, qa[0]);
+#pragma unroll
+        for (int bt = 0; bt < 6; ++bt) {
+            if (bt + 1 < 6) qk_reads(bt + 1, qa[(bt + 1) & 1]);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                const int mf = kQkOrder[3 * (bt % 3) + k];
+                f4& acc = s_acc[bt / 3][mf < 5 ? 0 : 1];
+                acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, qa[bt & 1][k]), bq[mf], acc, 0, 0, 0);
             }
         }
-        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int s = 0; s < 2; ++s) {
-            u4 a[9];
-#pragma unroll
-            for (int mf = 0; mf < 9; ++mf) {
-                const uint32_t w = kw[s][mf];
-                a[mf][0] = lut_read(w, lut_lane, 0x0c0c0400u);
-                a[mf][1] = lut_read(w, lut_lane, 0x0c0c0500u);
-                a[mf][2] = lut_read(w, lut_lane, 0x0c0c0600u);
-                a[mf][3] = lut_read(w, lut_lane, 0x0c0c0700u);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-            f4 s_acc[2] = {f4{0.f, 0.f, 0.f, 0.f}, f4{0.f, 0.f, 0.f, 0.f}};
-#pragma unroll
-            for (int m = 0; m < 5; ++m) {
-#pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    if (h == 1 && m == 4) continue;
-                    const int mf = h == 0 ? m : 5 + m;
-                    s_acc[h] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, a[mf]), bq[mf], s_acc[h], 0, 0, 0);
-                }
-            }
+        for (int s = 0; s < 2; ++s)
 #pragma unroll
             for (int i = 0; i < 4; ++i)
-                sc[4 * s + i] = half_lo_to_f32(ks0[s][i]) * s_acc[0][i] + half_hi_to_f32(ks16[s][i]) * s_acc[1][i];
-        }
+                sc[4 * s + i] = __builtin_fmaf(s_acc[s][1][i], half_hi_to_f32(ks[s][i]), mul_by_half_lo(s_acc[s][0][i], ks[s][i]));
         if (MASKED) {
 #pragma unroll
             for (int t = 0; t < 8; ++t) {
@@ -350,16 +339,42 @@ __global__ __launch_bounds__(kQsaWaves * 64, 1) void qsa_sparse_tq4_kernel(const
                 sc[t] = (col_ok && pos <= seq_pos) ? sc[t] : kNegBig;
             }
         }
-        uint32_t vd0[8], vd16[8], vwr[8], vw1[8];
-#pragma unroll
-        for (int t = 0; t < 8; ++t) {
-            const int trow = unit_token(t >> 2, b, t & 3);
-            const uint32_t* row32 = reinterpret_cast<const uint32_t*>(v_rows + trow * kTq4RowBytes);
-            vd0[t] = row32[0];
-            vd16[t] = row32[16];
-            vwr[t] = row32[n];
-            vw1[t] = row32[17 + n];
+        if (HAS_NEXT) {
+            wait_vm<kLoads>();  // the V rows have landed; the next K rows may be on their way
+        } else {
+            wait_vm<0>();
         }
+        // Per token: the two scales in one register, the dword of the first half-row that holds this lane's codes (dword n; for
+        // n = 0 codes 0-3 and 124-127 out of dwords 0 and 16) and that of the second; lane n reads dwords 0 and 16
+        // of token n & 7 and hands the scales and the n = 0 column round inside its row of lanes (as in the dense kernel,
+        // the volatile read and its LDS-typed address too).
+        uint32_t vsc[8], vw[2][8];
+        {
+            const uint32_t* r32 = reinterpret_cast<const uint32_t*>(v_rows + unit_token((n >> 2) & 1, b, n & 3) * kTq4RowBytes);
+            const uint32_t d0 = r32[0], d16 = r32[16];
+            const uint32_t mine_sc = __builtin_amdgcn_perm(d16, d0, 0x07060100u);
+            const uint32_t mine_c0 = __builtin_amdgcn_alignbit(d16, d0, 16);
+            uint32_t c0[8];
+            vsc[0] = row_bcast<0>(mine_sc); c0[0] = row_bcast<0>(mine_c0);
+            vsc[1] = row_bcast<1>(mine_sc); c0[1] = row_bcast<1>(mine_c0);
+            vsc[2] = row_bcast<2>(mine_sc); c0[2] = row_bcast<2>(mine_c0);
+            vsc[3] = row_bcast<3>(mine_sc); c0[3] = row_bcast<3>(mine_c0);
+            vsc[4] = row_bcast<4>(mine_sc); c0[4] = row_bcast<4>(mine_c0);
+            vsc[5] = row_bcast<5>(mine_sc); c0[5] = row_bcast<5>(mine_c0);
+            vsc[6] = row_bcast<6>(mine_sc); c0[6] = row_bcast<6>(mine_c0);
+            vsc[7] = row_bcast<7>(mine_sc); c0[7] = row_bcast<7>(mine_c0);
+#pragma unroll
+            for (int t = 0; t < 8; ++t) {
+                const int row = unit_token(t >> 2, b, t & 3) * kTq4RowBytes;
+                typedef __attribute__((address_space(3))) const volatile uint32_t lds_vol_u32;
+                const uint32_t first_half =
+                    *reinterpret_cast<lds_vol_u32*>((uintptr_t)(stage_addr + (uint32_t)(2 * kRunBytes + row + 4 * n)));
+                vw[0][t] = n == 0 ? c0[t] : first_half;
+                vw[1][t] = reinterpret_cast<const uint32_t*>(v_rows + row)[17 + n];
+            }
+        }
+        wait_lds_reads();
+        if (HAS_NEXT) issue_v(j_next);
         float p[8];
         {
             float mx = fmaxf(fmaxf(fmaxf(sc[0], sc[1]), fmaxf(sc[2], sc[3])), fmaxf(fmaxf(sc[4], sc[5]), fmaxf(sc[6], sc[7])));
@@ -384,113 +399,96 @@ __global__ __launch_bounds__(kQsaWaves * 64, 1) void qsa_sparse_tq4_kernel(const
                     for (int j = 0; j < 8; ++j) o_acc[h][j] *= alpha;
             }
         }
+        // probability times the half-row scale of the value row, as a high and a low fp16 operand (split_h2): one rounding
+        // would be shared by the whole scale block.  (Masked tokens have p == 0; a garbage scale must not reach the weights.)
+        if (MASKED) {
+#pragma unroll
+            for (int t = 0; t < 8; ++t) vsc[t] = p[t] > 0.f ? vsc[t] : 0u;
+        }
+        u4 ph[2], pl[2];
+        uint32_t lo[2][4], hi[2][4];
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-            // probability times the half-row scale of the value row, as a high and a low fp16
-            // operand (split_h2): one rounding would be shared by the whole scale block
-            uint32_t pb_hi[4], pb_lo[4];
-            {
-                float w[8];
+            float w[8];
 #pragma unroll
-                for (int t = 0; t < 8; ++t) w[t] = p[t] * (h == 0 ? half_lo_to_f32(vd0[t]) : half_hi_to_f32(vd16[t]));
-                if (MASKED) {
-#pragma unroll
-                    for (int t = 0; t < 8; ++t) w[t] = p[t] > 0.f ? w[t] : 0.f;
-                }
-#pragma unroll
-                for (int k = 0; k < 4; ++k) split_h2(w[2 * k], w[2 * k + 1], pb_hi[k], pb_lo[k]);
-            }
-            uint32_t lo[4], hi[4];
+            for (int t = 0; t < 8; ++t) w[t] = h == 0 ? mul_by_half_lo(p[t], vsc[t]) : mul_by_half_hi(p[t], vsc[t]);
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
-                uint32_t wa, wb;
-                if (h == 0) {
-                    const uint32_t xa = __builtin_amdgcn_alignbit(vd16[2 * k], vd0[2 * k], 16);
-                    const uint32_t xb = __builtin_amdgcn_alignbit(vd16[2 * k + 1], vd0[2 * k + 1], 16);
-                    wa = n == 0 ? xa : vwr[2 * k];
-                    wb = n == 0 ? xb : vwr[2 * k + 1];
-                } else {
-                    wa = vw1[2 * k];
-                    wb = vw1[2 * k + 1];
-                }
-                lo[k] = (wa & 0x0F0F0F0Fu) | ((wb << 4) & 0xF0F0F0F0u);
-                hi[k] = ((wa >> 4) & 0x0F0F0F0Fu) | (wb & 0xF0F0F0F0u);
+                uint32_t whi, wlo;
+                split_h2(w[2 * k], w[2 * k + 1], whi, wlo);
+                ph[h][k] = whi;
+                pl[h][k] = wlo;
+                const uint32_t wa = vw[h][2 * k], wb = vw[h][2 * k + 1];
+                lo[h][k] = (wa & 0x0F0F0F0Fu) | ((wb << 4) & 0xF0F0F0F0u);
+                hi[h][k] = ((wa >> 4) & 0x0F0F0F0Fu) | (wb & 0xF0F0F0F0u);
             }
-            u4 a[8];
+        }
+        settle(ph[0], ph[1], pl[0], pl[1]);
+        // four batches of four value tiles, the table reads of a batch in front of the MFMAs of the one before
+        u4 va[2][4];
+        auto pv_reads = [&](int bt, u4 (&a)[4]) __attribute__((always_inline)) {
 #pragma unroll
-            for (int j = 0; j < 8; ++j) {
+            for (int jj = 0; jj < 4; ++jj) {
+                const int j = 4 * (bt & 1) + jj;
 #pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    const uint32_t src = (j & 1) ? hi[k] : lo[k];
-                    const uint32_t sel = 0x0c0c0400u + ((uint32_t)(j >> 1) << 8);
-                    a[j][k] = lut_read(src, lut_lane, sel);
-                }
+                for (int k = 0; k < 4; ++k)
+                    a[jj][k] = lut_read((j & 1) ? hi[bt >> 1][k] : lo[bt >> 1][k], lut_lane, 0x0c0c0400u + ((uint32_t)(j >> 1) << 8));
             }
+        };
+        pv_reads(0, va[0]);
+#pragma unroll
+        for (int bt = 0; bt < 4; ++bt) {
+            if (bt + 1 < 4) pv_reads(bt + 1, va[(bt + 1) & 1]);
             __builtin_amdgcn_sched_barrier(0);
-            u4 ph = {pb_hi[0], pb_hi[1], pb_hi[2], pb_hi[3]};
-            u4 pl = {pb_lo[0], pb_lo[1], pb_lo[2], pb_lo[3]};
-            settle(ph, pl);
 #pragma unroll
-            for (int j = 0; j < 8; ++j)
-                o_acc[h][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, a[j]),
-                                                                    __builtin_bit_cast(h8, ph), o_acc[h][j], 0, 0, 0);
+            for (int part = 0; part < 2; ++part)  // (a pass of its own: a tile's two MFMAs are not back to back)
 #pragma unroll
-            for (int j = 0; j < 8; ++j)  // (a pass of its own: a tile's two MFMAs are not back to back)
-                o_acc[h][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, a[j]),
-                                                                    __builtin_bit_cast(h8, pl), o_acc[h][j], 0, 0, 0);
+                for (int jj = 0; jj < 4; ++jj) {
+                    f4& o = o_acc[bt >> 1][4 * (bt & 1) + jj];
+                    o = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, va[bt & 1][jj]),
+                                                              __builtin_bit_cast(h8, part ? pl[bt >> 1] : ph[bt >> 1]), o, 0, 0, 0);
+                }
         }
     };
 
-    while (unit < cu_end) {
-        commit_loads();
-        const int cur_pos_vec = pos_vec;
+    int unit = unit0;
+    for (int j = 0; unit < cu_end; ++j) {
         const int next_unit = unit + kQsaWaves;
-        if (next_unit < cu_end) {
-            load_groups(next_unit, id_vec, pos_vec);
-            issue_loads(id_vec);
-        }
-        const int ga = 4 * (b & 1) + (b >> 1);
-        const int gp0 = __shfl(cur_pos_vec, ga, 64);
-        const int gp1 = __shfl(cur_pos_vec, ga + 2, 64);
+        const int ga = 8 * (j & 7) + 4 * (b & 1) + (b >> 1);
+        const int gp0 = __shfl(pos_vec, ga, 64);
+        const int gp1 = __shfl(pos_vec, ga + 2, 64);
         // interior unit: all eight groups present and wholly in front of the token's position
-        const bool interior = __ballot(lane < 8 && cur_pos_vec + 3 > seq_pos) == 0ull;
-        process_unit(gp0, gp1, !interior);
+        const bool interior = __ballot((lane >> 3) == (j & 7) && pos_vec + 3 > seq_pos) == 0ull;
+        if ((j & 7) == 7 && next_unit < cu_end) {  // the next eight units' entries
+            load_list(next_unit, n_sel);
+            locate_list(next_unit);
+            asm volatile("" ::"v"(pos_vec));
+        }
+        process_unit(gp0, gp1, !interior, next_unit < cu_end, j + 1);
         unit = next_unit;
     }
 
     // ---- merge the waves' states through LDS (layout as in the dense kernel) -------------------------
+    // (one barrier: every wave leaves its state in its own staging area, the adding wave weighs them)
     l_run = sum_over_rows(l_run);
-    float* xbuf = reinterpret_cast<float*>(smem);
-    float* mlbuf = reinterpret_cast<float*>(smem + (kQsaSmem - kQsaMlBytes));
+    constexpr int kRegion = 8 * kMergeColStride;
+    static_assert(kRegion * 4 == kStageTq4, "a wave's merge region is its own staging area");
+    float* xbuf = reinterpret_cast<float*>(stage_all);
+    float* tbuf = reinterpret_cast<float*>(smem) + wave * 256;  // the table is dead behind the barrier
+    float* mlbuf = reinterpret_cast<float*>(smem + kQsaMlBase);
     if (b == 0) {
         mlbuf[(wave * 16 + n) * 2 + 0] = m_run;
         mlbuf[(wave * 16 + n) * 2 + 1] = l_run;
     }
-    __syncthreads();  // every wave is done with the table and with its staging area
-    {
-        float mt = kNegBig;
+    auto store_region = [&](int half) {
+        if ((n >> 3) != half || !col_ok) return;
+        float* c = xbuf + wave * kRegion + (n & 7) * kMergeColStride;
 #pragma unroll
-        for (int w = 0; w < kQsaWaves; ++w) mt = fmaxf(mt, mlbuf[(w * 16 + n) * 2]);
-        float lt = 0.f;
+        for (int h = 0; h < 2; ++h)
 #pragma unroll
-        for (int w = 0; w < kQsaWaves; ++w)
-            lt += mlbuf[(w * 16 + n) * 2 + 1] * __builtin_amdgcn_exp2f(mlbuf[(w * 16 + n) * 2] - mt);
-        const float wgt = __builtin_amdgcn_exp2f(m_run - mt);
-        float* c = xbuf + wave * kQsaRegion + n * kQsaColStride;
-        if (col_ok) {
-#pragma unroll
-            for (int h = 0; h < 2; ++h)
-#pragma unroll
-                for (int j = 0; j < 8; ++j) *reinterpret_cast<f4*>(c + ((h * 8 + j) * 4 + b) * 4) = o_acc[h][j] * wgt;
-        }
-        float* mltot = mlbuf + kQsaWaves * 16 * 2;
-        if (wave == 0 && b == 0) {
-            mltot[n * 2 + 0] = mt;
-            mltot[n * 2 + 1] = lt;
-        }
-    }
-    __syncthreads();
-    const float* mltot = mlbuf + kQsaWaves * 16 * 2;
+            for (int j = 0; j < 8; ++j) *reinterpret_cast<f4*>(c + ((h * 8 + j) * 4 + b) * 4) = o_acc[h][j];
+    };
+    store_region(0);
 
     int merge_slot[4];  // region slot of element 4 lane + k (inverse of tq4_pv_elem)
 #pragma unroll
@@ -508,19 +506,43 @@ __global__ __launch_bounds__(kQsaWaves * 64, 1) void qsa_sparse_tq4_kernel(const
         }
         merge_slot[k] = ((h * 8 + j) * 4 + (r >> 2)) * 4 + (r & 3);
     }
-    for (int col = wave; col < P.q_group; col += kQsaWaves) {
+    static_assert(kQsaWaves == 8, "a wave adds up one column of a pass");
+    __syncthreads();
+#pragma unroll 1
+    for (int half = 0; half < 2; ++half) {
+        if (8 * half >= P.q_group) break;  // the same in every wave
+        if (half == 1) {
+            __syncthreads();  // the first pass has read the regions
+            store_region(1);
+            __syncthreads();
+        }
+        const int col = 8 * half + wave;
+        if (col >= P.q_group) continue;
         const size_t row = (size_t)tok * P.num_q_heads + (size_t)(q_head_base + col);
         uint2 g = {0u, 0u};
         if (P.n_splits == 1) g = qsa_load_gate(P.gate, row, lane);
-        float v[4] = {0.f, 0.f, 0.f, 0.f};
+        float mw[kQsaWaves], lw[kQsaWaves];
 #pragma unroll
         for (int w = 0; w < kQsaWaves; ++w) {
-            const float* c = xbuf + w * kQsaRegion + col * kQsaColStride;
-#pragma unroll
-            for (int k = 0; k < 4; ++k) v[k] += c[merge_slot[k]];
+            const f2 r = *reinterpret_cast<const f2*>(mlbuf + (w * 16 + col) * 2);
+            mw[w] = r[0];
+            lw[w] = r[1];
         }
-        const float m_col = mltot[col * 2 + 0];
-        const float l_col = mltot[col * 2 + 1];
+        float m_col = kNegBig, l_col = 0.f;
+#pragma unroll
+        for (int w = 0; w < kQsaWaves; ++w) m_col = fmaxf(m_col, mw[w]);
+        f4 tot = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int w = 0; w < kQsaWaves; ++w) {
+            const float wgt = __builtin_amdgcn_exp2f(mw[w] - m_col);
+            l_col += lw[w] * wgt;
+            tot += *reinterpret_cast<const f4*>(xbuf + w * kRegion + wave * kMergeColStride + 4 * lane) * wgt;
+        }
+        // into the element order of the head dimension (the reads follow the write of the same wave in LDS order)
+        *reinterpret_cast<f4*>(tbuf + 4 * lane) = tot;
+        float v[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) v[k] = tbuf[merge_slot[k]];
         if (P.n_splits > 1) {
             const size_t prow = row * P.n_splits + split;
             *reinterpret_cast<f4*>(P.part_acc + prow * kHeadDim + 4 * lane) = f4{v[0], v[1], v[2], v[3]};
