@@ -288,6 +288,9 @@ __device__ __forceinline__ void settle(u4& a, u4& b, u4& c, u4& d) {
 __device__ __forceinline__ void settle(u2v (&a)[8]) {
     asm("s_nop 1" : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]), "+v"(a[4]), "+v"(a[5]), "+v"(a[6]), "+v"(a[7]));
 }
+__device__ __forceinline__ void settle(u4 (&a)[8]) {
+    asm("s_nop 1" : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]), "+v"(a[4]), "+v"(a[5]), "+v"(a[6]), "+v"(a[7]));
+}
 // a * (fp16 half of w) as one mixed-precision FMA that reads the half in place (v_fma_mix_f32 with
 // a zero addend; written as an fma so that the compiler forms it and places the wait states that
 // separate it from the instruction that produced a).  A product of -0 comes out as +0.

@@ -332,12 +332,12 @@ __global__ __launch_bounds__(kKv16Waves * 64, 1) void qsa_sparse_rows_kernel(con
 #pragma unroll
         for (int h = 0; h < 2; ++h)
 #pragma unroll
-            for (int j = 0; j < 8; ++j) o_acc[h][j] = mfma_x16<false>(a_v[h][j], pb, o_acc[h][j]);
+            for (int j = 0; j < 8; ++j) o_acc[h][j] = mfma_x16(a_v[h][j], pb, o_acc[h][j]);
         if constexpr (VRES) {
 #pragma unroll
             for (int h = 0; h < 2; ++h)
 #pragma unroll
-                for (int j = 0; j < 8; ++j) o_acc[h][j] = mfma_x16<false>(a_vr[h][j], pb, o_acc[h][j]);
+                for (int j = 0; j < 8; ++j) o_acc[h][j] = mfma_x16(a_vr[h][j], pb, o_acc[h][j]);
         }
     };
 
