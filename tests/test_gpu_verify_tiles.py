@@ -252,9 +252,10 @@ def test_rows_short_batches_other_group_sizes(fmt, dtype, q_heads):
 
 @pytest.mark.parametrize("fmt,dtype,heads,head_dim", [(FMT_TQ4, DT_F16, 2, 256), (FMT_Q8_0, DT_F16, 2, 256), (FMT_BF16, DT_BF16, 4, 128)])
 @pytest.mark.parametrize("seq,q", [([900, 900, 900], [16, 16, 16]), ([900, 60, 1500], [1, 3, 16]), ([40, 2500, 300], [16, 1, 2]),
-                                   ([700, 33], [5, 5]), ([1800], [16]), ([64, 900, 500, 200], [0, 7, 0, 7])])
+                                   ([700, 33], [5, 5]), ([1800], [16]), ([64, 900, 500, 200], [0, 7, 0, 7]),
+                                   ([30 + 11 * (i % 17) for i in range(70)], [1 + (i * 5) % 6 for i in range(70)])])
 def test_grid_of_several_tiles_per_request(fmt, dtype, heads, head_dim, seq, q):
     """The grid's bound (as many tiles for every request as the longest has, or one more per request than the tokens
     fill): all requests full, only the first or only the last, none; and the request guessed from the tile number right,
-    wrong, and behind the last."""
+    wrong, and behind the last; more requests than a wave looks up at a time."""
     _check(fmt, dtype, 16, seq, q, 431, scratch=SCRATCH, q_heads=16, kv_heads=heads, head_dim=head_dim)

@@ -460,10 +460,55 @@ struct TileInfo {
     bool hit;
     int req, rq_start, rq_end, seq_after, ctx_before, tile_in_req;
 };
-__device__ __forceinline__ TileInfo locate_tile(const AttnParams& P, int tile_z, int lane) {
+// what the lookup reads of request base + lane
+struct TileReq {
+    int lo, hi, sa, cb, rm;
+};
+__device__ __forceinline__ TileReq load_tile_req(const AttnParams& P, int base, int lane) {
+    const warp34_attention_batch& B = P.B;
+    const int r = base + lane;
+    const bool inb = r < B.num_reqs;
+    TileReq q;
+    q.lo = inb ? B.query_start_loc[r] : 0;
+    q.hi = inb ? B.query_start_loc[r + 1] : 0;
+    q.sa = inb ? B.seq_lens_after[r] : 0;
+    q.cb = (inb && B.context_lens_before != nullptr) ? B.context_lens_before[r] : 0;
+    q.rm = (inb && B.valid_req_mask != nullptr) ? (int)B.valid_req_mask[r] : 1;
+    return q;
+}
+// Tile tile_z by the requests' tile counts; q: the first 64 requests (load_tile_req), which a kernel with other work to do meanwhile
+// asks for ahead.  The sum over the lanes by DPP moves; by LDS permutes, with the requests asked for here: us a call, 4 tokens each,
+// Q8_0 1 request on 16 000 keys 18.8 -> 18.3, TQ4 20.0 -> 19.5, 1 on 1 000 16.6 -> 16.2.
+__device__ __forceinline__ TileInfo locate_tile_of(const AttnParams& P, int tile_z, int lane, TileReq q) {
     const warp34_attention_batch& B = P.B;
     TileInfo t{false, -1, 0, 0, 0, 0, 0};
+    int tiles_before = 0;
+    for (int base = 0; base < B.num_reqs; base += 64) {
+        if (base > 0) q = load_tile_req(P, base, lane);
+        const int cnt = q.hi > q.lo ? fast_div(q.hi - q.lo + P.tok_tile - 1, P.tok_tile) : 0;
+        const int incl = wave_incl_scan(cnt);
+        const int first = tiles_before + incl - cnt;
+        const unsigned long long hits = __ballot(cnt > 0 && tile_z >= first && tile_z < first + cnt);
+        if (hits != 0ull) {
+            const int src = __builtin_ctzll(hits);
+            t.req = base + src;
+            t.rq_start = __builtin_amdgcn_readlane(q.lo, src);
+            t.rq_end = __builtin_amdgcn_readlane(q.hi, src);
+            t.seq_after = __builtin_amdgcn_readlane(q.sa, src);
+            t.ctx_before = B.context_lens_before != nullptr ? __builtin_amdgcn_readlane(q.cb, src)
+                                                            : t.seq_after - (t.rq_end - t.rq_start);
+            t.tile_in_req = tile_z - __builtin_amdgcn_readlane(first, src);
+            t.hit = __builtin_amdgcn_readlane(q.rm, src) != 0;
+            return t;
+        }
+        tiles_before += __builtin_amdgcn_readlane(incl, 63);
+    }
+    return t;
+}
+__device__ __forceinline__ TileInfo locate_tile(const AttnParams& P, int tile_z, int lane) {
+    const warp34_attention_batch& B = P.B;
     if (P.tiles_by_request) {
+        TileInfo t{false, -1, 0, 0, 0, 0, 0};
         t.req = tile_z;
         const int lo = B.query_start_loc[tile_z];
         const int hi = B.query_start_loc[tile_z + 1];
@@ -478,39 +523,7 @@ __device__ __forceinline__ TileInfo locate_tile(const AttnParams& P, int tile_z,
         t.hit = __builtin_amdgcn_readfirstlane(rm) != 0 && t.rq_end > t.rq_start;
         return t;
     }
-    int tiles_before = 0;
-    for (int base = 0; base < B.num_reqs; base += 64) {
-        const int r = base + lane;
-        const bool inb = r < B.num_reqs;
-        const int lo = inb ? B.query_start_loc[r] : 0;
-        const int hi = inb ? B.query_start_loc[r + 1] : 0;
-        const int sa = inb ? B.seq_lens_after[r] : 0;
-        const int cb = (inb && B.context_lens_before != nullptr) ? B.context_lens_before[r] : 0;
-        const int rm = (inb && B.valid_req_mask != nullptr) ? (int)B.valid_req_mask[r] : 1;
-        const int cnt = hi > lo ? fast_div(hi - lo + P.tok_tile - 1, P.tok_tile) : 0;
-        int incl = cnt;
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-            const int up = __shfl_up(incl, off, 64);
-            if (lane >= off) incl += up;
-        }
-        const int first = tiles_before + incl - cnt;
-        const unsigned long long hits = __ballot(cnt > 0 && tile_z >= first && tile_z < first + cnt);
-        if (hits != 0ull) {
-            const int src = __builtin_ctzll(hits);
-            t.req = base + src;
-            t.rq_start = __builtin_amdgcn_readlane(lo, src);
-            t.rq_end = __builtin_amdgcn_readlane(hi, src);
-            t.seq_after = __builtin_amdgcn_readlane(sa, src);
-            t.ctx_before = B.context_lens_before != nullptr ? __builtin_amdgcn_readlane(cb, src)
-                                                            : t.seq_after - (t.rq_end - t.rq_start);
-            t.tile_in_req = tile_z - __builtin_amdgcn_readlane(first, src);
-            t.hit = __builtin_amdgcn_readlane(rm, src) != 0;
-            return t;
-        }
-        tiles_before += __builtin_amdgcn_readlane(incl, 63);
-    }
-    return t;
+    return locate_tile_of(P, tile_z, lane, load_tile_req(P, 0, lane));
 }
 
 // LDS-direct loads (gfx950): each active lane's 16 bytes go from global memory straight to LDS at
@@ -601,6 +614,7 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
     int req = -1, rq_start = 0, rq_end = 0, seq_after = 0, ctx_before = 0, tile_in_req = 0;
     int spec_slot_base = -1, spec_vec = -1;
     int a_lo = 0, a_hi = 0, a_sa = 0, a_cb = 0, a_rm = 0;
+    TileReq a_req;  // several tiles per request: as a_*, of request `lane`
     if constexpr (BAL) {
         req = item.req;
         rq_start = item.rq_start;
@@ -614,12 +628,13 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
         spec_slot_base = div_block(item.u_begin * kUnit, P);
         const int slot = spec_slot_base + lane;
         if (slot < B.max_blocks_per_req) spec_vec = B.block_tables[(size_t)req * B.max_blocks_per_req + slot];
-    } else if (P.tiles_by_request) {
-        req = tile_z;  // < num_reqs by the launch geometry
+    } else {
+        // a request by the launch geometry, or the guess that all requests have as many tiles as the longest
+        req = P.tiles_by_request ? tile_z : min(fast_div(tile_z, P.bal_tiles), B.num_reqs - 1);
         // Speculative block-table load, in flight together with the request's lengths: it
         // assumes that the request's length is the host's bound max_seq_len.  When the guess is
         // wrong the ids are fetched again below, so it changes the latency only, never the result.
-        if (B.sliding_window <= 0 && B.max_seq_len > 0) {
+        if (!SP && B.sliding_window <= 0 && B.max_seq_len > 0) {
             spec_slot_base = div_block(chunk * P.spec_upc * kUnit, P);
             const int slot = spec_slot_base + lane;
             if (slot < B.max_blocks_per_req)
@@ -628,20 +643,15 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
         // one vector load per array (all lanes the same address), no scalar-cache round trip;
         // the values are made scalar after the table has been built, so that the build overlaps
         // the round trip
-        a_lo = B.query_start_loc[req];
-        a_hi = B.query_start_loc[req + 1];
-        a_sa = B.seq_lens_after[req];
-        a_cb = B.context_lens_before != nullptr ? B.context_lens_before[req] : 0;
-        a_rm = B.valid_req_mask != nullptr ? (int)B.valid_req_mask[req] : 1;
-    } else {
-        const TileInfo ti = locate_tile(P, tile_z, lane);
-        req = ti.req;
-        rq_start = ti.rq_start;
-        rq_end = ti.rq_end;
-        seq_after = ti.seq_after;
-        ctx_before = ti.ctx_before;
-        tile_in_req = ti.tile_in_req;
-        req_hit = ti.hit;
+        if (P.tiles_by_request) {
+            a_lo = B.query_start_loc[req];
+            a_hi = B.query_start_loc[req + 1];
+            a_sa = B.seq_lens_after[req];
+            a_cb = B.context_lens_before != nullptr ? B.context_lens_before[req] : 0;
+            a_rm = B.valid_req_mask != nullptr ? (int)B.valid_req_mask[req] : 1;
+        } else {
+            a_req = load_tile_req(P, 0, lane);
+        }
     }
     // While the request's lengths are on their way: the raw query rows of this wave's columns and
     // the table.  The first token of the tile is guessed (exact when every request has a whole
@@ -699,6 +709,17 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
         ctx_before = B.context_lens_before != nullptr ? __builtin_amdgcn_readfirstlane(a_cb)
                                                       : seq_after - (rq_end - rq_start);
         req_hit = __builtin_amdgcn_readfirstlane(a_rm) != 0 && rq_end > rq_start;
+    }
+    if (!BAL && !P.tiles_by_request) {
+        const TileInfo ti = locate_tile_of(P, tile_z, lane, a_req);
+        if (ti.req != req) spec_slot_base = -1;
+        req = ti.req;
+        rq_start = ti.rq_start;
+        rq_end = ti.rq_end;
+        seq_after = ti.seq_after;
+        ctx_before = ti.ctx_before;
+        tile_in_req = ti.tile_in_req;
+        req_hit = ti.hit;
     }
     if (!req_hit) return;  // no such tile, empty or masked request: outputs untouched
     const int tok0 = rq_start + tile_in_req * P.tok_tile;
@@ -2245,6 +2266,7 @@ static int launch_tq4(const warp34_exec* ex, const warp34_kv_layer_layout* layou
             P.part_stride = stride;
             P.pf_split = parts;
             P.pf_slot_base = P.max_chunks;
+            P.bal_tiles = tiles_per_request_bound(*batch, P);
             P.part_ml = P.part_acc + (size_t)rows * stride * kHeadDim;
             SpHeader* hdr = reinterpret_cast<SpHeader*>(P.part_ml + (size_t)rows * stride * 4);
             P.key_floor = &hdr->floor;
@@ -2299,6 +2321,7 @@ static int launch_tq4(const warp34_exec* ex, const warp34_kv_layer_layout* layou
             return launch_balanced_merge<TQ, kHeadDim>(P, kv_subs, kLutInvGain, stream);
         }
     }
+    P.bal_tiles = tiles_per_request_bound(*batch, P);
     rc = ensure_dynamic_lds(paged_attn_tq4_kernel<TQ, 1>, smem_bytes_for(1), true);
     if (rc) return rc;
     hipLaunchKernelGGL((paged_attn_tq4_kernel<TQ, 1>), grid, dim3(waves_for(1) * 64), smem_bytes_for(1), stream, P);
