@@ -337,6 +337,22 @@ __device__ __forceinline__ uint32_t lut_read(uint32_t code_word, uint32_t lut_la
     return *reinterpret_cast<lds_cu32*>((uintptr_t)addr);
 }
 
+// The pair table, by 512 threads: entry e = (gain*centroid[e & 15], gain*centroid[e >> 4]) as packed fp16, 64 copies of 4 bytes.
+// Thread t writes the 16-byte slots t + 512 i (conflict-free), i.e. entries (t >> 4) + 32 i:
+// their low code (t >> 4) & 15 is the thread's own, their high code (t >> 8) + 2 i is the
+// same in the whole wave.  Lane j < 16 computes centroid j once; everything else is lane
+// traffic, so the build costs a few dozen instructions per wave.
+__device__ __forceinline__ void build_pair_table(uint8_t* smem, int tid, int lane, int wave) {
+    const uint32_t c_bits = (uint32_t)F16::from_f32(kLutGain * centroid_of_code(lane & 15));
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_ds_bpermute(((tid >> 4) & 15) << 2, (int)c_bits);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)c_bits, (wave >> 2) + 2 * i);
+        const uint32_t v = lo | (hi << 16);
+        *reinterpret_cast<u4*>(smem + (tid + 512 * i) * 16) = u4{v, v, v, v};
+    }
+}
+
 // element index (0..255) of nibble i of aligned dword D of a TQ4 row, -1 for scale nibbles
 __device__ __forceinline__ constexpr int tq4_dword_elem(int D, int i) {
     if (D == 0) return i >= 4 ? i - 4 : -1;
@@ -686,11 +702,7 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
     load_tok_ok(tok_guess);
 
     if (build_table) {
-        // entry e = (gain*centroid[e & 15], gain*centroid[e >> 4]) as packed fp16, 64 copies of 4 bytes.
-        // Thread t writes the 16-byte slots t + 512 i (conflict-free), i.e. entries (t >> 4) + 32 i:
-        // their low code (t >> 4) & 15 is the thread's own, their high code (t >> 8) + 2 i is the
-        // same in the whole wave.  Lane j < 16 computes centroid j once; everything else is lane
-        // traffic, so the build costs a few dozen instructions per wave.
+        // (build_pair_table's text: as a call, one request on 1 200 keys takes 13.4 us instead of 12.8)
         static_assert(kWaves == 8, "table build: 512 threads");
         const uint32_t c_bits = (uint32_t)F16::from_f32(kLutGain * centroid_of_code(lane & 15));
         const uint32_t lo = (uint32_t)__builtin_amdgcn_ds_bpermute(((tid >> 4) & 15) << 2, (int)c_bits);

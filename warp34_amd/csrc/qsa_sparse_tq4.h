@@ -11,7 +11,8 @@
 // of eight units in one load, K rows asked for before V rows and the next unit's before this one's products, table reads
 // a batch ahead of the MFMAs, one barrier before the loop and one behind it.  us a call, 513 groups, against rows through
 // registers, K and V waited for together, two barriers on either side: 16 tokens 19.6 -> 17.4, 64 30.6 -> 25.8, 256
-// 85 -> 66; 16 tokens x 64 groups 12.6 -> 11.2.
+// 85 -> 66; 16 tokens x 64 groups 12.6 -> 11.2; with the table written without bank conflicts (build_pair_table; 16 bytes every 128
+// before) 16.7, 25.7, 67 and 9.8.
 //
 //   grid  = (query tokens, kv heads x q subgroups, splits), block = 8 waves
 //   split = an equal share of the token's units; every split writes an (m, l) record (l = 0
@@ -151,15 +152,7 @@ __global__ __launch_bounds__(kQsaWaves * 64, 1) void qsa_sparse_tq4_kernel(const
             q_raw[c] = *reinterpret_cast<const uint2*>(qrow + 4 * lane);
         }
     }
-    {
-        // entry e = (gain * centroid[e & 15], gain * centroid[e >> 4]) as packed fp16, 64 copies
-        const int e = tid >> 1;
-        const uint32_t v = pack_h2(kLutGain * centroid_of_code(e & 15), kLutGain * centroid_of_code(e >> 4));
-        u4 vv = {v, v, v, v};
-        u4* dst = reinterpret_cast<u4*>(smem + e * 256 + (tid & 1) * 128);
-#pragma unroll
-        for (int k = 0; k < 8; ++k) dst[k] = vv;
-    }
+    build_pair_table(smem, tid, lane, wave);
 
     int n_sel = __builtin_amdgcn_readfirstlane(a_live) != 0 ? __builtin_amdgcn_readfirstlane(a_sel) : 0;
     if (n_sel > P.select_k) n_sel = P.select_k;
