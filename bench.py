@@ -73,13 +73,13 @@ PROFILED_TRAFFIC = {
     "fp8_decode_b32_ctx1k_64k": (1_162_710_000, "profiles/paged_attn_rows_fp8_decode_b32_ctx1k_64k.txt"),
     "fp8_decode_b1_ctx131072": (140_900_000, "profiles/paged_attn_rows_fp8_decode_b1_ctx131072.txt"),
     "q8_0_decode_b1_ctx131072": (145_110_000, "profiles/paged_attn_rows_q8_0_decode_b1_ctx131072.txt"),
-    # (the four kernels of the shared-prefix path together: probe 0.27 + tile 144.87 + decode 535.49 + merge 39.06 MB)
-    "tq4_verify_16x4_ctx262144_shared200k": (719_690_000, "profiles/paged_attn_tq4_verify_16x4_ctx262144_shared200k.txt"),
-    "tq4_prefill_8x2048_ctx16384": (1_119_610_000, "profiles/paged_prefill_tq4_8x2048_ctx16384.txt"),
-    "tq4_qsa_sparse_16x513_ctx131072": (23_400_000, "profiles/qsa_sparse_tq4_16x513_ctx131072.txt"),
+    # (the four kernels of the shared-prefix path together: probe 0.27 + tile 144.89 + decode 535.52 + merge 39.06 MB)
+    "tq4_verify_16x4_ctx262144_shared200k": (719_740_000, "profiles/paged_attn_tq4_verify_16x4_ctx262144_shared200k.txt"),
+    "tq4_prefill_8x2048_ctx16384": (567_780_000, "profiles/paged_prefill_tq4_8x2048_ctx16384.txt"),
+    "tq4_qsa_sparse_16x513_ctx131072": (23_340_000, "profiles/qsa_sparse_tq4_16x513_ctx131072.txt"),
     "tq4_norm_rope_append_8192": (182_920_000, "profiles/qk_norm_rope_tq4_append_8192.txt"),
-    "tq4_fused_qk_gate_append_8192": (289_660_000, "profiles/fused_qk_norm_rope_gate_tq4_append_8192.txt"),
-    "tq4_append_4096": (10_880_000, "profiles/kv_append_tq4_4096.txt"),
+    "tq4_fused_qk_gate_append_8192": (289_740_000, "profiles/fused_qk_norm_rope_gate_tq4_append_8192.txt"),
+    "tq4_append_4096": (10_800_000, "profiles/kv_append_tq4_4096.txt"),
 }
 SHARED_PREFIX = {"tq4_verify_16x4_ctx262144_shared200k": 200000}
 VERIFY_Q = {"tq4_verify_16x4_ctx262144_shared200k": 4}
@@ -368,7 +368,7 @@ def run_prefill(args, torch, lib, ffi, layers, ctx, n_layers, pool_pages, fmt):
         "roofline": {"bound": "mfma", "achieved": round(tf_attn, 1), "peak": peak, "unit": "TFLOP/s",
                      "frac": round(tf_attn / peak, 4), "traffic": PROFILED_TRAFFIC.get(args.workload, (None, None))[0],
                      "traffic_source": PROFILED_TRAFFIC.get(args.workload, (None, None))[1],
-                     "kernel": "paged_prefill_tq4_kernel (attention-only launches)",
+                     "kernel": "paged_prefill_wide_kernel (attention-only launches)",
                      "avg_launch_us": round(ms_attn * 1e3, 1)},
     }))
 

@@ -2678,7 +2678,7 @@ static int attention_entry(const warp34_exec* ex, const warp34_kv_layer_layout* 
     if (is_tq4(layout)) {
         if (!tq4_geometry_ok(layout, q) || (((uintptr_t)out) & 7u) != 0) return (int)hipErrorNotSupported;
         // Many query rows per request and enough tiles to fill the chip: the tile kernel shares
-        // every dequantised key block between 128 query rows.
+        // every dequantised key block between 256 (or 128) query rows.
         const bool many_rows = batch->max_q_len >= 32 &&
                                (long long)batch->total_tokens * num_q_heads >= 128ll * kPfRows;
         if ((force_tile || (!force && many_rows)) && prefill_tq4_applicable(layout, batch, num_q_heads))
