@@ -1,12 +1,15 @@
 """What the built library's kernel descriptors say: the row-format attention and the prefill kernels keep everything in registers.
-A reload from scratch memory waits for the row loads in flight as well, which the kernels place their own waits for."""
+A reload from scratch memory waits for the row loads in flight as well, which the kernels place their own waits for.  And what the
+compiler makes of device helpers whose instructions have waiting times."""
 import os
 import re
+import shutil
 import struct
 import subprocess
 
 import pytest
 
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 READELF = "/opt/rocm/llvm/bin/llvm-readelf"
 
 
@@ -47,3 +50,26 @@ def test_prefill_kernels_do_not_spill(tmp_path):
     kernels = {k: v for k, v in kernel_scratch_bytes(tmp_path).items() if "paged_prefill" in k}
     assert len(kernels) >= 16, sorted(kernels)
     assert {k: v for k, v in kernels.items() if v} == {}
+
+
+def assembly(tmp_path, source):
+    path = os.path.join(str(tmp_path), "probe.hip")
+    with open(path, "w") as f:
+        f.write('#include "%s"\n%s' % (os.path.join(ROOT, "warp34_amd", "csrc", "kv_common.h"), source))
+    cmd = ["hipcc", "-O3", "-std=c++17", "--offload-arch=gfx950", "--cuda-device-only", "-S", "-o", "-", path]
+    text = subprocess.run(cmd, stdout=subprocess.PIPE, text=True, check=True).stdout
+    lines = [line.split(";")[0].strip() for line in text.splitlines()]
+    return [line for line in lines if re.match(r"[a-z]+_", line)]
+
+
+@pytest.mark.skipif(shutil.which("hipcc") is None, reason="no hipcc")
+def test_product_of_a_weight_waits_for_its_exponential(tmp_path):
+    code = assembly(tmp_path, """
+        __global__ void weight(float* p, const float* d) {
+            const int i = threadIdx.x;
+            const float scale = d[i], score = p[i] * scale;
+            p[i] = w34::mul_legacy(__builtin_amdgcn_exp2f(score), scale);
+        }""")
+    at = next(i for i, line in enumerate(code) if line.startswith("v_exp_f32"))
+    use = next(i for i, line in enumerate(code) if line.startswith("v_mul_legacy_f32"))
+    assert use > at + 1, code[at:use + 1]

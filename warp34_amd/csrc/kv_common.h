@@ -56,6 +56,11 @@ __device__ __forceinline__ float apply_sign(float v, int i) {
     return __uint_as_float(__float_as_uint(v) ^ (((sign_word(i >> 5) >> (i & 31)) & 1u) << 31));
 }
 
+// a * b with 0 times anything = 0: the scale of a row that a column does not see may be anything.  (The compiler's own
+// instruction and not an assembly statement: a vector instruction may read the result of a transcendental one a wait state later
+// at the earliest, which is not kept in front of assembly, and the weights come straight from exp.)
+__device__ float mul_legacy(float a, float b) __asm("llvm.amdgcn.fmul.legacy");
+
 constexpr int kHeadDim = 256;
 constexpr int kTq4RowBytes = 132;   // 2 x (fp16 scale + 64 bytes of nibbles), tq4_kv_common.cuh:21-26
 constexpr int kTq4RowDwords = 33;

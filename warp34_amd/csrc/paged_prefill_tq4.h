@@ -63,13 +63,6 @@ __device__ __forceinline__ float max2(float a, float b) {  // (see max3)
     asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
     return r;
 }
-// a * b with 0 times anything = 0: the scale of a row that a column does not see may be anything.  (a must not come
-// straight from a transcendental instruction: the compiler places no wait states in front of an assembly statement.)
-__device__ __forceinline__ float mul_legacy(float a, float b) {
-    float r;
-    asm("v_mul_legacy_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
-    return r;
-}
 // High and low fp16 operands of the weights p0 d0 | p1 d1 (see split_h2).  (v_fma_mix_f32 and v_cvt_pk_f16_f32 issue every
 // 4 cycles, v_fma_mixlo_f16 / mixhi every 8.)
 __device__ __forceinline__ void weight_h2(float p0, float p1, float d0, float d1, uint32_t& hi, uint32_t& lo) {
