@@ -1,0 +1,102 @@
+"""Batches whose requests differ: what the kernels pay for them, as ratios of times of two batches on the same card, and the results of
+the routes that only such batches take."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import oracle
+from oracle import DT_BF16, DT_F16, FMT_BF16, FMT_FP16, FMT_FP8, FMT_Q8_0, FMT_TQ4
+
+pytestmark = pytest.mark.gpu
+
+ROW_BYTES = {FMT_TQ4: lambda hd: 132, FMT_FP8: lambda hd: 264, FMT_Q8_0: lambda hd: 272, FMT_FP16: lambda hd: 2 * hd,
+             FMT_BF16: lambda hd: 2 * hd}
+
+
+class Batch:
+    """One attention call over empty pages, which take as long as full ones."""
+
+    def __init__(self, fmt, seqs, news, q_heads=16, kv_heads=2, head_dim=256, both_ways=False, block=64):
+        import torch
+
+        from warp34_amd import ffi
+
+        dev = "cuda:0"
+        self.lib = ffi.load()
+        tok = ROW_BYTES[fmt](head_dim)
+        pages = [(s + block - 1) // block for s in seqs]
+        table = np.zeros((len(seqs), max(pages)), np.int32)
+        order = np.random.default_rng(7).permutation(sum(pages)).astype(np.int32)
+        at = 0
+        for r, n in enumerate(pages):
+            table[r, :n] = order[at:at + n]
+            at += n
+        starts = np.concatenate([[0], np.cumsum(news)]).astype(np.int32)
+        n = int(starts[-1])
+        keep = [torch.zeros(sum(pages) * kv_heads * block * tok, dtype=torch.uint8, device=dev) for _ in range(2)]
+        keep += [torch.from_numpy(a).to(dev) for a in (table, starts, np.array(seqs, np.int32),
+                                                       np.array(seqs, np.int32) - np.array(news, np.int32))]
+        k, v, tab, qsl, seq, ctx = keep
+        dtype = torch.bfloat16 if fmt == FMT_BF16 else torch.float16
+        q, out = (torch.zeros((n, q_heads, head_dim), dtype=dtype, device=dev) for _ in range(2))
+        strides = (kv_heads * block * tok, block * tok, tok)
+        xf = oracle.XF_WHT256 if fmt == FMT_TQ4 else oracle.XF_IDENTITY
+        layout = ffi.Warp34KvLayerLayout(k.data_ptr(), v.data_ptr(), *strides, *strides, 0, 0, kv_heads, head_dim, block, fmt, fmt,
+                                         xf, xf, 0)
+        mask = ffi.WARP34_ATTN_MASK_NONCAUSAL_WINDOW if both_ways else ffi.WARP34_ATTN_MASK_CAUSAL
+        batch = ffi.Warp34AttentionBatch(qsl.data_ptr(), ctx.data_ptr(), seq.data_ptr(), tab.data_ptr(), None, None, None, len(seqs), n,
+                                         table.shape[1], max(news), max(seqs), mask, 0, head_dim ** -0.5, 0)
+        need = self.lib.warp34_paged_attention_scratch_bytes_for_layout(C.byref(layout), n, len(seqs), q_heads, max(seqs))
+        scratch = torch.zeros(max(need, 8 << 20), dtype=torch.uint8, device=dev)
+        ex = ffi.Warp34Exec(torch.cuda.current_stream().cuda_stream, scratch.data_ptr(), scratch.numel(), 0)
+        self.keep = (keep, q, out, layout, batch, scratch, ex)
+        call = self.lib.warp34_paged_attention_bf16 if fmt == FMT_BF16 else self.lib.warp34_paged_attention_f16
+        self.args = (call, C.byref(ex), C.byref(layout), C.byref(batch), q.data_ptr(), out.data_ptr(), q_heads)
+
+    def __call__(self):
+        assert self.args[0](*self.args[1:]) == 0
+
+
+def times(*batches, rounds=15, calls=10):
+    """Least microseconds a call of each, measured in turn."""
+    import torch
+
+    best = [float("inf")] * len(batches)
+    start, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+    for _ in range(rounds):
+        for i, b in enumerate(batches):
+            b()
+            start.record()
+            for _ in range(calls):
+                b()
+            end.record()
+            torch.cuda.synchronize()
+            best[i] = min(best[i], start.elapsed_time(end) / calls * 1e3)
+    print("us a call:", ["%.1f" % t for t in best], flush=True)
+    return best
+
+
+@pytest.mark.parametrize("fmt", [FMT_TQ4, FMT_FP8, FMT_Q8_0, FMT_FP16, FMT_BF16])
+def test_tile_of_few_rows_costs_less_than_a_whole_one(fmt):
+    """Requests of 80 and of 256 query rows, one tile of 256 each: 0.75 of the time."""
+    short, whole = times(Batch(fmt, [400] * 64, [40] * 64, kv_heads=8), Batch(fmt, [400] * 64, [128] * 64, kv_heads=8))
+    assert short < 0.88 * whole
+
+
+@pytest.mark.parametrize("fmt", [FMT_FP8, FMT_Q8_0, FMT_FP16, FMT_BF16])
+def test_short_last_tiles_of_many_requests(fmt):
+    """A whole tile and one of a few rows each, more requests than a wave has lanes: less than two whole tiles on every part of the chip."""
+    ragged, whole = times(Batch(fmt, [1000] * 150, [33] * 150), Batch(fmt, [1000] * 150, [64] * 150))
+    assert ragged < 0.94 * whole
+
+
+@pytest.mark.parametrize("fmt,dtype", [(FMT_TQ4, DT_F16), (FMT_Q8_0, DT_F16), (FMT_FP8, DT_F16), (FMT_BF16, DT_BF16)])
+@pytest.mark.parametrize("n,q_heads,longest", [(9, 4, 128), (70, 4, 129), (66, 16, 33), (70, 16, 64)])
+def test_many_short_requests(fmt, dtype, n, q_heads, longest):
+    """Tiles of one row up to whole ones, one or two a request, at most and more than 64 requests."""
+    from test_gpu_prefill_wide import WIDE, _run
+
+    q_lens = [1 + (r * 37) % longest for r in range(n - 2)] + [longest, longest // 2]
+    _run(fmt, dtype, 16, [q + 30 + 5 * r for r, q in enumerate(q_lens)], q_lens, 1901 + longest, q_heads=q_heads, keep=0.3,
+         force=WIDE if dtype == DT_F16 else None)

@@ -748,7 +748,16 @@ __device__ __forceinline__ void pw_tile(const AttnParams& P, uint8_t* smem, int 
 // other.  A last, partly filled round of workgroups over the kPwCus CUs would cost as much as a full one: as many of its tiles as
 // there are CUs left over are cut into two tiles of 128 rows, which take about 0.65 of the time of a whole one (Q8_0 0.73, FP8
 // and FP16 0.69, TQ4 and BF16 0.63): the longest ones while the batch fits one round (they end last), else the shortest ones (they
-// start last).  More than 64 requests: whole tiles in grid order.
+// start last).
+// A tile whose request ends inside its first half runs as one of 128 rows: the other half's products would be those of dead
+// columns.  us a layer step, 128-row tiles of their own kernel / whole tiles only / this: 32 requests x 40 tokens, two q heads
+// per kv head, on 240 to 940 keys: Q8_0 90 / 109 / 86, FP8 86 / 105 / 82, FP16 84 / 99 / 77; 300 x 33 to 60 733 / 920 / 700.
+// More than 64 requests: no ranks.  The workgroups of a request one after the other, its last tile first, which share its keys;
+// but by tile index, all requests' first tiles first, where a request's tiles would meet the same parts of the chip over and over
+// (workgroups go round 8 XCDs and their shader engines): with two tiles, one whole and one short, half of the XCDs get the whole
+// ones only; with 24 and more a shader engine keeps seeing the same index, behind the end of most requests.  us, the former order /
+// the latter: Q8_0 100 x 33 to 48 tokens, eight q heads per kv head, 213 / 183, bf16 128 x 129, two q heads, 869 / 816, Q8_0
+// 70 x 100 to 1 000 (32 tiles) 2 440 / 1 697; 80 x 20 to 300 (10 tiles) on 1 500 to 5 200 keys 1 389 / 1 512.
 constexpr int kPwCus = 256;
 constexpr int kPwTq4Tiles = 250;  // TQ4 pages: from this many 256-row tiles on (see launch_prefill_tq4)
 template <typename TQ, int KVF, bool VF>
@@ -788,17 +797,27 @@ __global__ __launch_bounds__(kPfWaves * 64, 1) void paged_prefill_wide_kernel(co
         req = t.req;
         tile = t.tile;
     } else {
-        const int per_req = tiles_x * kv_subs;
-        req = wg / per_req;
-        if (req >= P.B.num_reqs) return;
-        const int in_req = wg - req * per_req;
-        kv_sub = in_req / tiles_x;
-        tile = tiles_x - 1 - (in_req - kv_sub * tiles_x);
+        const int per_req = tiles_x * kv_subs, per_tile = P.B.num_reqs * kv_subs;
+        if (tiles_x <= 2 || tiles_x >= 24) {
+            tile = wg / per_tile;
+            if (tile >= tiles_x) return;
+            const int at = wg - tile * per_tile;
+            req = at / kv_subs;
+            kv_sub = at - req * kv_subs;
+        } else {
+            req = wg / per_req;
+            if (req >= P.B.num_reqs) return;
+            const int in_req = wg - req * per_req;
+            kv_sub = in_req / tiles_x;
+            tile = tiles_x - 1 - (in_req - kv_sub * tiles_x);
+        }
     }
-    if (half < 0) {
-        pw_tile<TQ, KVF, 2, VF>(P, smem, req, kv_sub, tile * P.tok_tile, P.tok_tile);
+    const int half_tok = P.tok_tile >> 1, tok0 = tile * P.tok_tile + (half > 0 ? half_tok : 0);
+    const int left = P.B.query_start_loc[req + 1] - P.B.query_start_loc[req] - tok0;
+    if (half < 0 && left > half_tok) {
+        pw_tile<TQ, KVF, 2, VF>(P, smem, req, kv_sub, tok0, P.tok_tile);
     } else {
-        pw_tile<TQ, KVF, 1, VF>(P, smem, req, kv_sub, tile * P.tok_tile + half * (P.tok_tile >> 1), P.tok_tile >> 1);
+        pw_tile<TQ, KVF, 1, VF>(P, smem, req, kv_sub, tok0, half_tok);
     }
 }
 
