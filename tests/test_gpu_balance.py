@@ -91,6 +91,14 @@ def test_short_last_tiles_of_many_requests(fmt):
     assert ragged < 0.94 * whole
 
 
+@pytest.mark.parametrize("n,q,more", [(12, 8, 13), (9, 16, 11)])
+def test_draft_blocks_in_an_odd_number_of_chunks(n, q, more):
+    """Draft blocks cut into 5 (3) chunks, and more requests cut into 4 (2) of them: the tiles of a request, which read the same keys, are
+    on one XCD with either number, and the time goes with the keys (0.88 and 0.75; on two XCDs 1.5 and 0.98)."""
+    odd, even = times(*(Batch(FMT_BF16, [8000] * r, [q] * r, kv_heads=4, head_dim=128, both_ways=True) for r in (n, more)))
+    assert odd < 0.95 * even
+
+
 @pytest.mark.parametrize("fmt,dtype", [(FMT_TQ4, DT_F16), (FMT_Q8_0, DT_F16), (FMT_FP8, DT_F16), (FMT_BF16, DT_BF16)])
 @pytest.mark.parametrize("n,q_heads,longest", [(9, 4, 128), (70, 4, 129), (66, 16, 33), (70, 16, 64)])
 def test_many_short_requests(fmt, dtype, n, q_heads, longest):

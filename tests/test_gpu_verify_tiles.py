@@ -259,3 +259,36 @@ def test_grid_of_several_tiles_per_request(fmt, dtype, heads, head_dim, seq, q):
     fill): all requests full, only the first or only the last, none; and the request guessed from the tile number right,
     wrong, and behind the last; more requests than a wave looks up at a time."""
     _check(fmt, dtype, 16, seq, q, 431, scratch=SCRATCH, q_heads=16, kv_heads=heads, head_dim=head_dim)
+
+
+@pytest.mark.parametrize("fmt,dtype,q_heads,kv_heads,head_dim,seq,q", [
+    # 7 chunks x 4 heads, 9 requests of two tiles; 3 x 3; 1 x 4 (no split)
+    (FMT_BF16, DT_BF16, 16, 4, 128, [2000 + 131 * i for i in range(9)], [8] * 9),
+    (FMT_BF16, DT_BF16, 12, 3, 128, [900 + 257 * i for i in range(9)], [16] * 9),
+    (FMT_FP16, DT_F16, 16, 4, 128, [20 + 31 * (i % 7) for i in range(30)], [16] * 30),
+    # requests with fewer tiles than the longest, none at all; two q subgroups (20 q heads per kv head)
+    (FMT_BF16, DT_BF16, 16, 4, 128, [1500] * 8 + [70], [16, 16, 9, 16, 16, 0, 16, 16, 13]),
+    (FMT_BF16, DT_BF16, 40, 2, 128, [900, 40, 1300, 700, 2100], [5] * 5),
+    # head dimension 256: 21 chunks x 2 heads, 63 x 2
+    (FMT_Q8_0, DT_F16, 16, 2, 256, [6000, 900, 6000], [4] * 3),
+    (FMT_FP8, DT_F16, 16, 2, 256, [16000], [4]),
+    (FMT_BF16, DT_BF16, 8, 1, 256, [9000, 40, 9000], [4, 3, 4]),
+])
+def test_chunk_grid_by_groups_of_keys(fmt, dtype, q_heads, kv_heads, head_dim, seq, q):
+    """Workgroups that are not a multiple of eight a tile go by the keys they share; the bits are those of launch order, where a batch
+    without a bound on its requests' tokens stays."""
+    import gpu_harness as G
+    from cases import make_case
+
+    pool, bt, k, v, qb, aq, ctx = make_case(fmt, 16, seq, q, 432, dtype, kv_heads=kv_heads, q_heads=q_heads, head_dim=head_dim)
+    hb = oracle.HostBatch(aq, seq, bt, context_lens_before=ctx, mask_mode=1 if head_dim == 128 else 0)
+    dpool = G.DevPool(pool)
+    dpool.upload()
+    outs = []
+    for bound in (None, 0):
+        rc, out, _ = G.dev_attention(dpool, hb, qb, dtype, q_heads, scratch_bytes=SCRATCH, max_q_len=bound)
+        assert rc == 0
+        outs.append(out)
+    assert outs[0].tobytes() == outs[1].tobytes()
+    want = oracle.paged_attention(pool, hb, qb, dtype, q_heads, n_threads=4)
+    G.assert_close(outs[0], dtype, want, what="groups of keys", scale=G.channel_scale(v, dtype, hb, q_heads))

@@ -77,6 +77,7 @@ __host__ __device__ constexpr int smem_bytes_for(int nt) {
 }
 static_assert(merge_floats_for(1) * 4 <= waves_for(1) * kStageTq4, "merge regions alias the staging areas only");
 static_assert(smem_bytes_for(1) <= 160 * 1024, "decode LDS budget");
+constexpr int kXcds = 8;  // workgroups go round them in launch order
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kNegBig = -1.0e30f;  // "minus infinity" that stays finite under subtraction
 // The table holds fp16(kLutGain * centroid); the gain is divided out of the query (K side)
@@ -107,7 +108,10 @@ struct AttnParams {
     int bal_tiles;         // tiles per request (a bound); balanced decode: the plan's entries are request x tile
     int bal_aligned;       // balanced decode: no piece boundary inside a workgroup's share (few entries)
     int piece_cost;        // balanced decode: what starting a piece costs, in units
-    int bal_cols;          // columns of a partial slot: 16 x column tiles of the kernel
+    union {
+        int bal_cols;      // balanced decode: columns of a partial slot, 16 x column tiles of the kernel
+        int key_groups;    // row formats, chunk grid: see rows_key_groups
+    };
     uint32_t block_magic;  // floor(2^32 / block_size), see div_block
     uint32_t q_group_magic;  // see div_q_group
     const uint16_t* gate;  // fp16 [tokens, q heads, 256] or null: out = fp16(out) * sigmoid(gate)
@@ -2445,6 +2449,23 @@ static int launch_rows_balanced(const warp34_exec* ex, const warp34_attention_ba
     return launch(std::integral_constant<int, 1>{});
 }
 
+// Groups of keys (request x kv head x chunk) of a chunk grid whose workgroups go by them (rows_by_keys), 0: in launch order, chunk by
+// chunk, head by head, tile by tile.  Launch order puts the tiles of a request on one XCD where a tile's workgroups are a multiple of
+// eight; else two or more XCDs fetch the same keys, and two workgroups on a CU wait for them together.  us a layer step, launch order /
+// by groups, bf16 draft blocks (four kv heads), contexts from an eighth of the length up: 9 x 16 tokens (3 chunks) on 16 000 keys 82.3 /
+// 65.7, 9 x 8 (7) 64.6 / 46.4, 12 x 8 (5) 85.4 / 58.5, on 6 000 42.2 / 31.8; head dimension 256, 3 x 4 (21) on 3 000 to 16 000, bf16 24.8 /
+// 20.0, Q8_0 26.2 / 24.9, 1 x 4 (63) on 16 000 20.2 / 16.8.  Where launch order does as well the arithmetic costs 0.1 to 0.3 (4 x 16 on
+// 2 000 keys, 8 chunks, 17.6 / 17.9), and with fewer than kKeyGroupsFrom workgroups there is nothing to gain (Q8_0, 3 x 4: 132 of them, on
+// 2 900 keys, 20.1 / 20.3; 204, on 4 100, 21.2 / 21.0; 252, on 6 000, 22.9 / 22.0).
+// (A batch with fewer tiles than its requests could have stays in launch order: many groups would have no tile.)
+constexpr int kKeyGroupsFrom = 192;
+static int rows_key_groups(const warp34_attention_batch& B, const AttnParams& P, int kv_subs, int grid_z) {
+    const int per_tile = P.max_chunks * kv_subs;
+    if (P.bal_tiles < 2 || per_tile % kXcds == 0 || grid_z != (long long)B.num_reqs * P.bal_tiles) return 0;
+    const long long groups = (long long)B.num_reqs * per_tile;
+    return groups * P.bal_tiles >= kKeyGroupsFrom && groups <= 65535ll * kXcds ? (int)groups : 0;
+}
+
 // VRES: value rows stored rotated in an 8-bit format (residual operand, see rows_tile)
 template <typename TQ, int KVF, bool VRES = false, int HD = kHeadDim>
 static int launch_rows(const warp34_exec* ex, const warp34_kv_layer_layout* layout,
@@ -2500,12 +2521,14 @@ static int launch_rows(const warp34_exec* ex, const warp34_kv_layer_layout* layo
     P.rot_out = layout->v_transform == WARP34_KV_TRANSFORM_RADEMACHER_WHT256 ? 1 : 0;
     const int grid_z = tiles_bound(*batch, P);
     const int kv_subs = layout->local_kv_heads * P.q_subgroups;
-    const dim3 grid((unsigned)grid_x, (unsigned)kv_subs, (unsigned)grid_z);
+    dim3 grid((unsigned)grid_x, (unsigned)kv_subs, (unsigned)grid_z);
     hipStream_t stream = (hipStream_t)ex->stream;
     int rc;
     rc = launch_rows_balanced<TQ, KVF, VRES, HD>(ex, batch, P, kv_subs, force_single, stream);
     if (rc >= 0) return rc;
     P.bal_tiles = tiles_per_request_bound(*batch, P);
+    P.key_groups = rows_key_groups(*batch, P, kv_subs, grid_z);
+    if (P.key_groups > 0) grid = dim3((unsigned)(kXcds * P.bal_tiles), (unsigned)((P.key_groups + kXcds - 1) / kXcds));
     constexpr int smem = rows_smem_bytes<KVF, HD>(1);
     rc = ensure_dynamic_lds(paged_attn_rows_kernel<TQ, KVF, VRES, HD>, smem, true);
     if (rc) return rc;

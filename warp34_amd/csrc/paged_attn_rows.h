@@ -125,12 +125,29 @@ template <int KVF, int HD>
 __host__ __device__ constexpr int rows_ml_offset(int nt) {
     // One tile of 16-bit rows has its query operands in registers from the start.  At head dimension 128 a workgroup then takes 77 KB
     // and two share a CU: a batch over four kv heads (512 workgroups) runs in one round.  us: 4 x 16 draft tokens on 1 000 / 4 000 /
-    // 16 000 keys 14.6 / 24.3 / 53.8 -> 13.3 / 19.7 / 48.0, 8 x 8 14.6 / 29.8 / 64.7 -> 14.0 / 23.7 / 59.8.
+    // 16 000 keys 14.6 / 24.3 / 53.8 -> 13.3 / 19.7 / 48.0, 8 x 8 14.6 / 29.8 / 64.7 -> 14.0 / 23.7 / 59.8.  A layer step, contexts from
+    // an eighth of the length up, against one workgroup per CU: 8 x 16 on 6 000 32.8 -> 28.0, 12 x 16 on 16 000 101 -> 84, 15 x 16 142 -> 138
+    // (with the tiles of a request on one XCD, see rows_key_groups: on two, 9 x 16 on 16 000 73.9 -> 82.5, 7 x 8 50.0 -> 53.3).
     return rows_q_offset<KVF, HD>() + (nt == 1 && !RowsLds<KVF, HD>::k8 ? 0 : nt * (HD / 32) * 1024);
 }
 template <int KVF, int HD>
 __host__ __device__ constexpr int rows_smem_bytes(int nt) {
     return rows_ml_offset<KVF, HD>(nt) + kKv16Waves * nt * 16 * 2 * 4;
+}
+
+// Chunk grid, P.key_groups > 0: a workgroup's tile, kv head and chunk.  The tiles of a request read the same keys, and workgroups
+// go round the XCDs in launch order: blockIdx.x = 8 x tile of the request + XCD, blockIdx.y = a group of keys (request x kv head x
+// chunk) of each XCD, so that an XCD's L2 takes a group's keys in once.  False: no such group.
+__device__ __forceinline__ bool rows_by_keys(const AttnParams& P, int& tile_z, int& kv_sub, int& chunk) {
+    const int group = kXcds * (int)blockIdx.y + ((int)blockIdx.x & (kXcds - 1));
+    if (group >= P.key_groups) return false;
+    const int kv_subs = P.L.local_kv_heads * P.q_subgroups;
+    const int req_head = small_div(group, P.max_chunks);
+    const int req = small_div(req_head, kv_subs);
+    chunk = group - req_head * P.max_chunks;
+    kv_sub = req_head - req * kv_subs;
+    tile_z = req * P.bal_tiles + ((int)blockIdx.x >> 3);
+    return true;
 }
 
 // One LDS-direct load instruction: lane l's 16 bytes from base + voffset + IMM to lds_addr + IMM + 16 l.
@@ -205,11 +222,13 @@ __device__ __forceinline__ void rows_tile(const AttnParams& P, uint8_t* smem, co
     const warp34_kv_layer_layout& L = P.L;
     const warp34_attention_batch& B = P.B;
 
-    const int tile_z = BAL ? item.req : (int)blockIdx.z;  // tile index (see locate_tile)
-    const int kv_sub = (int)blockIdx.y;
+    int tile_z = BAL ? item.req : (int)blockIdx.z;  // tile index (see locate_tile)
+    int kv_sub = (int)blockIdx.y, chunk = BAL ? 0 : (int)blockIdx.x;
+    if constexpr (!BAL && !STREAM) {
+        if (P.key_groups > 0 && !rows_by_keys(P, tile_z, kv_sub, chunk)) return;
+    }
     const int kv_head = small_div(kv_sub, P.q_subgroups);
     const int q_head_base = kv_head * P.gqa + (kv_sub - kv_head * P.q_subgroups) * P.q_group;
-    const int chunk = BAL ? 0 : (int)blockIdx.x;
 
     // Query rows in MFMA B layout: lane (n, b) holds Q[column n][32 m + 8 b .. + 7] for m = 0..kM-1.
     // One tile of un-rotated queries comes straight from global memory into registers; the first
