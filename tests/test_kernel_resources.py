@@ -73,3 +73,21 @@ def test_product_of_a_weight_waits_for_its_exponential(tmp_path):
     at = next(i for i, line in enumerate(code) if line.startswith("v_exp_f32"))
     use = next(i for i, line in enumerate(code) if line.startswith("v_mul_legacy_f32"))
     assert use > at + 1, code[at:use + 1]
+
+
+@pytest.mark.skipif(shutil.which("hipcc") is None, reason="no hipcc")
+@pytest.mark.parametrize("cells_per_unit,holds", [("120.25f", True), ("121.0f", False), ("118.0f", False), ("208.0f", False)])
+def test_code_cells_keep_the_boundaries_from_their_edges(tmp_path, cells_per_unit, holds):
+    """Sizes of the encoders' cells with every boundary in a cell of its own, but some nearer than a quarter of a cell to its edge (with
+    208 also in the first cell), do not compile."""
+    csrc = os.path.join(ROOT, "warp34_amd", "csrc")
+    with open(os.path.join(csrc, "kv_encode.h")) as f:
+        text, n = re.subn(r"kCellsPerUnit = [0-9.]+f", "kCellsPerUnit = " + cells_per_unit, f.read())
+    assert n == 1
+    path = os.path.join(str(tmp_path), "probe.hip")
+    with open(path, "w") as f:
+        f.write(text.replace("#pragma once", ""))
+    cmd = ["hipcc", "-std=c++17", "--offload-arch=gfx950", "--cuda-device-only", "-fsyntax-only", "-I", csrc, path]
+    p = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    assert (p.returncode == 0) == holds, p.stdout
+    assert holds or "away from its edges" in p.stdout

@@ -176,7 +176,16 @@ constexpr uint64_t tq4_cells_with_boundary() {
     for (int k = 0; k < 15; ++k) cells |= 1ull << (int)(kBoundaries[k] * kCellsPerUnit + kCellOfZero);
     return cells;
 }
-static_assert(__builtin_popcountll(tq4_cells_with_boundary()) == 15, "every boundary in a cell of its own");
+// Where u is rounded across the edge of a cell, both cells give the same code only while no boundary is near the edge; the first and the
+// last cell also take what saturates (and NaN), so they hold none.
+constexpr bool tq4_boundaries_inside_cells() {
+    for (int k = 0; k < 15; ++k) {
+        const float at = kBoundaries[k] * kCellsPerUnit + kCellOfZero, in_cell = at - (float)(int)at;
+        if (!(at >= 1.0f && at < 63.0f && in_cell >= 0.25f && in_cell <= 0.75f)) return false;
+    }
+    return __builtin_popcountll(tq4_cells_with_boundary()) == 15;
+}
+static_assert(tq4_boundaries_inside_cells(), "every boundary in a cell of its own, away from its edges");
 struct Tq4Tables {  // lane i: of cell i the boundary in it (or +inf) and 4 (16 + number of boundaries below it); centroid i % 16
     int boundary, at, centroid;
 };
