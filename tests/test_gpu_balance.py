@@ -99,6 +99,13 @@ def test_draft_blocks_in_an_odd_number_of_chunks(n, q, more):
     assert odd < 0.95 * even
 
 
+@pytest.mark.parametrize("fmt", [FMT_BF16, FMT_Q8_0])
+def test_one_request_of_many_tiles_uses_the_whole_chip(fmt):
+    """One request with the tiles of eight: the same products (1.0; on one XCD 6)."""
+    one, eight = times(Batch(fmt, [4473], [952], q_heads=8, kv_heads=1), Batch(fmt, [4473] * 8, [119] * 8, q_heads=8, kv_heads=1))
+    assert one < 1.5 * eight
+
+
 @pytest.mark.parametrize("fmt,dtype", [(FMT_TQ4, DT_F16), (FMT_Q8_0, DT_F16), (FMT_FP8, DT_F16), (FMT_BF16, DT_BF16)])
 @pytest.mark.parametrize("n,q_heads,longest", [(9, 4, 128), (70, 4, 129), (66, 16, 33), (70, 16, 64)])
 def test_many_short_requests(fmt, dtype, n, q_heads, longest):

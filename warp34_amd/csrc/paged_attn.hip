@@ -2458,12 +2458,18 @@ static int launch_rows_balanced(const warp34_exec* ex, const warp34_attention_ba
 // 2 000 keys, 8 chunks, 17.6 / 17.9), and with fewer than kKeyGroupsFrom workgroups there is nothing to gain (Q8_0, 3 x 4: 132 of them, on
 // 2 900 keys, 20.1 / 20.3; 204, on 4 100, 21.2 / 21.0; 252, on 6 000, 22.9 / 22.0).
 // (A batch with fewer tiles than its requests could have stays in launch order: many groups would have no tile.)
+// The XCDs have to get about as much each: nearly as many groups, and each request on all of them or, from 80 groups of at least four a
+// request on, many requests.  One request of 951 tokens (476 tiles of one kv head) is one group: 103 us in launch order, 694 on one XCD.
 constexpr int kKeyGroupsFrom = 192;
+constexpr int kKeyGroupsOfManyRequests = 80;
 static int rows_key_groups(const warp34_attention_batch& B, const AttnParams& P, int kv_subs, int grid_z) {
     const int per_tile = P.max_chunks * kv_subs;
     if (P.bal_tiles < 2 || per_tile % kXcds == 0 || grid_z != (long long)B.num_reqs * P.bal_tiles) return 0;
     const long long groups = (long long)B.num_reqs * per_tile;
-    return groups * P.bal_tiles >= kKeyGroupsFrom && groups <= 65535ll * kXcds ? (int)groups : 0;
+    const long long on_an_xcd = (groups + kXcds - 1) / kXcds;
+    if (8 * kXcds * on_an_xcd > 9 * groups) return 0;
+    if (per_tile < kXcds && (per_tile < kXcds / 2 || groups < kKeyGroupsOfManyRequests)) return 0;
+    return groups * P.bal_tiles >= kKeyGroupsFrom && on_an_xcd <= 65535 ? (int)groups : 0;
 }
 
 // VRES: value rows stored rotated in an 8-bit format (residual operand, see rows_tile)
