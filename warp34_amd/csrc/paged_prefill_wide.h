@@ -758,7 +758,56 @@ __device__ __forceinline__ void pw_tile(const AttnParams& P, uint8_t* smem, int 
 // ones only; with 24 and more a shader engine keeps seeing the same index, behind the end of most requests.  us, the former order /
 // the latter: Q8_0 100 x 33 to 48 tokens, eight q heads per kv head, 213 / 183, bf16 128 x 129, two q heads, 869 / 816, Q8_0
 // 70 x 100 to 1 000 (32 tiles) 2 440 / 1 697; 80 x 20 to 300 (10 tiles) on 1 500 to 5 200 keys 1 389 / 1 512.
+// Requests of different lengths: whole tiles of the longest would be the batch's time, so they are cut too (pw_long_tiles).
 constexpr int kPwCus = 256;
+// What a tile of a request takes, in units of its length (pf_longest_first): lane r holds request r.
+struct PwRequest {
+    int first, count;  // lengths first + 1 .. first + count
+    // tiles of at least this length, and what they take
+    __device__ __forceinline__ int from(int length) const { return max(0, min(count, first + count + 1 - length)); }
+    __device__ __forceinline__ float work(int n) const { return (float)n * ((float)(first + count) - 0.5f * (float)(n - 1)); }
+};
+// How many tiles, of the longest, are cut into halves because the others would be done long before them: all that are longer than
+// three quarters of the longest, if there are few enough for their halves to run at once, and if by list scheduling (a tile
+// begins when what comes before it, spread over the CUs, is done; a half takes 0.7) the batch then ends before the longest whole tile
+// would.  us, whole tiles only / this: four requests of 1 024 tokens, eight q heads per kv head, one on 16 000 keys and three on 2 000:
+// FP8 871 / 686, Q8_0 961 / 797, FP16 810 / 682, BF16 1 023 / 750.
+__device__ __forceinline__ int pw_long_tiles(const AttnParams& P, int lane, int kv_subs, int tiles) {
+    const warp34_attention_batch& B = P.B;
+    if (B.num_reqs < 2 || B.sliding_window > 0 || B.mask_mode == WARP34_ATTN_MASK_NONCAUSAL_WINDOW) return 0;
+    PwRequest mine{0, 0};
+    if (lane < B.num_reqs && (B.valid_req_mask == nullptr || B.valid_req_mask[lane] != 0)) {
+        const int q_len = B.query_start_loc[lane + 1] - B.query_start_loc[lane];
+        const int ctx = B.context_lens_before != nullptr ? B.context_lens_before[lane] : B.seq_lens_after[lane] - q_len;
+        mine.count = q_len > 0 ? (q_len + P.tok_tile - 1) / P.tok_tile : 0;
+        mine.first = ctx > 0 ? ctx / P.tok_tile : 0;
+    }
+    int longest = mine.count > 0 ? mine.first + mine.count : 0;
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) longest = max(longest, __shfl_xor(longest, off, 64));
+    longest = __builtin_amdgcn_readfirstlane(longest);
+    const int cut_from = longest - (longest >> 2) + 1;
+    // up to and with the shortest tile of this lane's request: workgroups, what they take, the batch's cut tiles
+    int before = 0, cut = 0;
+    float work = 0.0f;
+    for (int r = 0; r < B.num_reqs; ++r) {
+        const PwRequest other{__builtin_amdgcn_readlane(mine.first, r), __builtin_amdgcn_readlane(mine.count, r)};
+        const int n = other.from(mine.first + 1), n_cut = other.from(cut_from), halved = min(n, n_cut);
+        before += n + halved;
+        work += other.work(n) + 0.4f * other.work(halved);
+        cut += n_cut;
+    }
+    cut = __builtin_amdgcn_readfirstlane(cut) * kv_subs;
+    if (cut > kPwCus / 2 || cut >= tiles) return 0;
+    float end = 0.0f;
+    if (mine.count > 0) {
+        const float own = (float)(mine.first + 1);
+        end = before * kv_subs > kPwCus ? work * (float)kv_subs / (float)kPwCus + own : own;
+    }
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) end = fmaxf(end, __shfl_xor(end, off, 64));
+    return __ballot(end < 0.95f * (float)longest) != 0ull ? cut : 0;
+}
 constexpr int kPwTq4Tiles = 250;  // TQ4 pages: from this many 256-row tiles on (see launch_prefill_tq4)
 template <typename TQ, int KVF, bool VF>
 __global__ __launch_bounds__(kPfWaves * 64, 1) void paged_prefill_wide_kernel(const AttnParams P) {
@@ -780,10 +829,13 @@ __global__ __launch_bounds__(kPfWaves * 64, 1) void paged_prefill_wide_kernel(co
             tiles = __builtin_amdgcn_readfirstlane(tiles) * kv_subs;
         }
         const int last = tiles % kPwCus;
-        const int cut = min(last, last == 0 ? 0 : kPwCus - last);
+        const int spare = min(last, last == 0 ? 0 : kPwCus - last);
+        const int longest = tiles > kPwCus / 2 ? pw_long_tiles(P, (int)threadIdx.x & 63, kv_subs, tiles) : 0;
+        const bool from_front = tiles < kPwCus || longest > 0;
+        const int cut = longest == 0 ? spare : tiles < kPwCus ? max(longest, spare) : longest;
         if (wg >= tiles + cut) return;
         int at = wg;  // the tile
-        if (tiles < kPwCus) {
+        if (from_front) {
             if (wg < 2 * cut) at = wg >> 1, half = wg & 1;
             else at = wg - cut;
         } else if (wg >= tiles - cut) {
