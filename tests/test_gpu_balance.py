@@ -99,6 +99,15 @@ def test_draft_blocks_in_an_odd_number_of_chunks(n, q, more):
     assert odd < 0.95 * even
 
 
+def test_long_draft_blocks_do_not_share_a_cu():
+    """Twelve draft blocks, 384 workgroups: the long requests at the places whose workgroups would share CUs, and none of them there."""
+    long, short = 12000, 2000
+    apart = [long] * 4 + [short] * 4 + [short] * 4
+    meet = [long] * 2 + [short] * 6 + [long] * 2 + [short] * 2
+    a, b = times(*(Batch(FMT_BF16, s, [16] * 12, kv_heads=4, head_dim=128, both_ways=True) for s in (apart, meet)))
+    assert max(a, b) < 1.08 * min(a, b)
+
+
 @pytest.mark.parametrize("fmt", [FMT_BF16, FMT_Q8_0])
 def test_one_request_of_many_tiles_uses_the_whole_chip(fmt):
     """One request with the tiles of eight: the same products (1.0; on one XCD 6)."""

@@ -269,14 +269,18 @@ def test_grid_of_several_tiles_per_request(fmt, dtype, heads, head_dim, seq, q):
     # requests with fewer tiles than the longest, none at all; two q subgroups (20 q heads per kv head)
     (FMT_BF16, DT_BF16, 16, 4, 128, [1500] * 8 + [70], [16, 16, 9, 16, 16, 0, 16, 16, 13]),
     (FMT_BF16, DT_BF16, 40, 2, 128, [900, 40, 1300, 700, 2100], [5] * 5),
+    # by length, eight requests in the first round (launch order, 8 a tile; equal lengths, a request without tokens) and ten (by keys)
+    (FMT_BF16, DT_BF16, 16, 4, 128, [2100, 300, 2100, 90, 1500, 16, 700, 2100, 40, 1100, 1900, 333], [16] * 12),
+    (FMT_FP16, DT_F16, 16, 4, 128, [2001 - 170 * i for i in range(11)], [16, 3, 16, 16, 0, 16, 16, 16, 16, 9, 16]),
+    (FMT_BF16, DT_BF16, 12, 3, 128, [90, 4000, 3100, 16, 800, 2222, 60, 4000, 1000], [16] * 9),
     # head dimension 256: 21 chunks x 2 heads, 63 x 2
     (FMT_Q8_0, DT_F16, 16, 2, 256, [6000, 900, 6000], [4] * 3),
     (FMT_FP8, DT_F16, 16, 2, 256, [16000], [4]),
     (FMT_BF16, DT_BF16, 8, 1, 256, [9000, 40, 9000], [4, 3, 4]),
 ])
 def test_chunk_grid_by_groups_of_keys(fmt, dtype, q_heads, kv_heads, head_dim, seq, q):
-    """Workgroups that are not a multiple of eight a tile go by the keys they share; the bits are those of launch order, where a batch
-    without a bound on its requests' tokens stays."""
+    """Workgroups that are not a multiple of eight a tile go by the keys they share, long requests at head dimension 128 by length; the
+    bits are those of launch order, where a batch without a bound on its requests' tokens stays."""
     import gpu_harness as G
     from cases import make_case
 

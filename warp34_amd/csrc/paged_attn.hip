@@ -78,6 +78,7 @@ __host__ __device__ constexpr int smem_bytes_for(int nt) {
 static_assert(merge_floats_for(1) * 4 <= waves_for(1) * kStageTq4, "merge regions alias the staging areas only");
 static_assert(smem_bytes_for(1) <= 160 * 1024, "decode LDS budget");
 constexpr int kXcds = 8;  // workgroups go round them in launch order
+constexpr int kChipCus = 256;
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kNegBig = -1.0e30f;  // "minus infinity" that stays finite under subtraction
 // The table holds fp16(kLutGain * centroid); the gain is divided out of the query (K side)
@@ -106,7 +107,10 @@ struct AttnParams {
     int rot_out;           // V rows are stored rotated: rotate the output back
     int32_t* bal_table;    // balanced decode: per query token {first partial slot, pieces, token of the tile, columns (0: bal_cols)}
     int bal_tiles;         // tiles per request (a bound); balanced decode: the plan's entries are request x tile
-    int bal_aligned;       // balanced decode: no piece boundary inside a workgroup's share (few entries)
+    union {
+        int bal_aligned;    // balanced decode: no piece boundary inside a workgroup's share (few entries)
+        int first_round;    // row formats, chunk grid: see rows_first_round
+    };
     int piece_cost;        // balanced decode: what starting a piece costs, in units
     union {
         int bal_cols;      // balanced decode: columns of a partial slot, 16 x column tiles of the kernel
@@ -2001,7 +2005,7 @@ static int choose_max_chunks(const warp34_exec* ex, int total_tokens, int num_q_
 // device d is configured.  Kernels that address their dequantisation table absolutely
 // (lds_base_zero) also have their static LDS size checked here: it must be zero, so that the
 // dynamic block starts at LDS address 0.
-constexpr int kLdsRecordSlots = 96;
+constexpr int kLdsRecordSlots = 128;
 static std::atomic<const void*> g_lds_fn[kLdsRecordSlots];
 static std::atomic<unsigned long long> g_lds_devs[kLdsRecordSlots];
 
@@ -2472,6 +2476,23 @@ static int rows_key_groups(const warp34_attention_batch& B, const AttnParams& P,
     return groups * P.bal_tiles >= kKeyGroupsFrom && on_an_xcd <= 65535 ? (int)groups : 0;
 }
 
+// Chunk grid at head dimension 128, more workgroups than CUs but no more than two on each: the requests go by length
+// (rows_longest_first); returned is how many the first round of workgroups takes, 0: in their own order.  us a layer step, bf16 draft blocks,
+// mean of six sets of contexts from an eighth of the length up, one workgroup per CU / two in the requests' order / two by length:
+// up to 14 000 keys 9 x 16 tokens 72.2 / 57.0 / 50.6, 12 x 16 86.2 / 74.9 / 65.5, 15 x 16 105 / 90.7 / 74.3, 13 x 8 58.0 / 55.4 / 50.0,
+// 16 x 8 69.4 / 66.5 / 58.4; up to 5 000 12 x 16 45.4 / 39.9 / 37.3.  (The longest first all through: 52.2, 67.4, 80.4, 51.7, 63.2; 37.8.)
+// Single sets in the requests' order were up to 18 % slower than one per CU (12 x 16, 88.9 / 105).  From kLongestFirstKeys keys a
+// workgroup on: the lengths are asked for before anything else, and with shorter chunks that costs what it gains (4 x 16 up to 5 000,
+// 8 chunks, 22.8 / 22.9; 4 x 8, 16 chunks, 20.1 / 20.5; 6 x 8 up to 14 000, 10 chunks, 31.6 / 30.9).
+constexpr int kLongestFirstKeys = 1000;
+static int rows_first_round(const warp34_attention_batch& B, const AttnParams& P, int kv_subs, int grid_z) {
+    const long long per_req = (long long)P.max_chunks * kv_subs * P.bal_tiles, wgs = per_req * B.num_reqs;
+    if (P.bal_tiles < 2 || B.num_reqs < 2 || B.num_reqs > 64 || grid_z != (long long)B.num_reqs * P.bal_tiles || B.sliding_window > 0 ||
+        wgs <= kChipCus || wgs > 2 * kChipCus || B.max_seq_len < (long long)kLongestFirstKeys * P.max_chunks)
+        return 0;
+    return std::max(1, (int)(kChipCus / per_req));
+}
+
 // VRES: value rows stored rotated in an 8-bit format (residual operand, see rows_tile)
 template <typename TQ, int KVF, bool VRES = false, int HD = kHeadDim>
 static int launch_rows(const warp34_exec* ex, const warp34_kv_layer_layout* layout,
@@ -2534,11 +2555,14 @@ static int launch_rows(const warp34_exec* ex, const warp34_kv_layer_layout* layo
     if (rc >= 0) return rc;
     P.bal_tiles = tiles_per_request_bound(*batch, P);
     P.key_groups = rows_key_groups(*batch, P, kv_subs, grid_z);
+    P.first_round = HD != kHeadDim ? rows_first_round(*batch, P, kv_subs, grid_z) : 0;
     if (P.key_groups > 0) grid = dim3((unsigned)(kXcds * P.bal_tiles), (unsigned)((P.key_groups + kXcds - 1) / kXcds));
     constexpr int smem = rows_smem_bytes<KVF, HD>(1);
-    rc = ensure_dynamic_lds(paged_attn_rows_kernel<TQ, KVF, VRES, HD>, smem, true);
+    const auto kernel = P.key_groups > 0 || P.first_round > 0 ? paged_attn_rows_mapped_kernel<TQ, KVF, VRES, HD>
+                                                              : paged_attn_rows_kernel<TQ, KVF, VRES, HD>;
+    rc = ensure_dynamic_lds(kernel, smem, true);
     if (rc) return rc;
-    hipLaunchKernelGGL((paged_attn_rows_kernel<TQ, KVF, VRES, HD>), grid, dim3(kKv16Waves * 64), smem, stream, P);
+    hipLaunchKernelGGL(kernel, grid, dim3(kKv16Waves * 64), smem, stream, P);
     rc = (int)hipGetLastError();
     if (rc) return rc;
     return P.max_chunks > 1 ? launch_split_merge<TQ, false, HD>(P, P.max_chunks, 1.0f, stream) : 0;

@@ -8,10 +8,11 @@
 //   * S^T = K Q^T: A operand = 16 K rows read from LDS, B operand = the query rows, loaded
 //     once in MFMA layout.  8-bit codes are widened to fp16 in registers (exact) and the fp32
 //     block scales are applied to per-block partial scores, so K is never rounded;
-//   * O^T += V^T P^T with 16x16x16 MFMAs: each lane reads the 8-element slice of its 4 tokens
+//   * O^T += V^T P^T over the 16 keys of a half: each lane reads the 8-element slice of its 4 tokens
 //     and transposes the 4x8 block in registers.  8-bit V is dequantised to fp16(d * code)
-//     on the way, which is what the reference stages (op_paged_attn.cu:59-105);
-//   * BF16 storage: P is split into a bf16 high and low part (two MFMAs) so that the 8-bit
+//     on the way, which is what the reference stages (op_paged_attn.cu:59-105).  16x16x16 MFMAs, or where
+//     an operand has two parts 16x16x32 ones, whose upper 16 keys are the second part;
+//   * BF16 storage: P is split into a bf16 high and low part (over the same value rows) so that the 8-bit
 //     mantissa of bf16 does not limit the accuracy of the weighted sum;
 //   * 8-bit layers may be stored rotated (WHT256 transform): the query rows are then rotated
 //     once per tile and the output is rotated back once (op_kv_cache.cu:443-451,763-783).
@@ -22,7 +23,6 @@
 namespace w34 {
 
 typedef _Float16 h4 __attribute__((ext_vector_type(4)));
-typedef short s4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
 
 constexpr int kKv16Waves = 8;
@@ -150,6 +150,24 @@ __device__ __forceinline__ bool rows_by_keys(const AttnParams& P, int& tile_z, i
     return true;
 }
 
+// Chunk grid, P.first_round > 0: the tile of a workgroup where the requests go by length: the longest in the first round of
+// workgroups, one per CU, longest first; the others, which share the CUs with them, shortest first, so that the shortest meets the
+// longest.  In the requests' own order two long ones may meet on a CU and are done long after the others.  Lane r holds request r,
+// at most 64.
+__device__ __forceinline__ int rows_longest_first(const AttnParams& P, int lane, int tile_z) {
+    const int n = P.B.num_reqs;
+    const int place = small_div(tile_z, P.bal_tiles);
+    const int len = lane < n ? P.B.seq_lens_after[lane] : 0;
+    int longer = 0;  // requests before this lane's
+    for (int r = 0; r < n; ++r) {
+        const int other = __builtin_amdgcn_readlane(len, r);
+        longer += other > len || (other == len && r < lane) ? 1 : 0;
+    }
+    const int want = place < P.first_round ? place : n - 1 - (place - P.first_round);
+    const unsigned long long mine = __ballot(lane < n && longer == want);
+    return (int)__builtin_ctzll(mine) * P.bal_tiles + (tile_z - place * P.bal_tiles);
+}
+
 // One LDS-direct load instruction: lane l's 16 bytes from base + voffset + IMM to lds_addr + IMM + 16 l.
 template <bool STREAM, int IMM>
 __device__ __forceinline__ void lds_load_piece(uint32_t voffset, const uint8_t* sbase, uint32_t lds_addr) {
@@ -185,15 +203,16 @@ __device__ __forceinline__ void lds_load_half(uint32_t voffset, const uint8_t* s
 // streaming, and the merge of the waves (2.3 us per tile).
 // BAL: the tile and its unit range come from `item` (balanced decode, see bal_for_each_piece)
 // instead of blockIdx.
-// VRES (8-bit rows stored rotated): the value operand fp16(d * code) is followed by a second
-// operand holding its rounding residual, and every P V tile takes a second MFMA.  A scale block
+// VRES (8-bit rows stored rotated): the value operand is fp16(d * code) and, as the upper 16 keys of the
+// same MFMA with the same weights, its rounding residual.  A scale block
 // of a rotated row with large entries holds few distinct codes, so part of the fp16 rounding of
 // d * code is common to the block, and the inverse rotation of the finished row would gather
 // that common part into a single channel.
 // HD: the head dimension, 256 or -- 16-bit rows only (op_kv_cache.cu:1227) -- 128.  At 128 a row is
 // one 128-element half: four QK operands instead of eight, eight value tiles instead of sixteen,
 // and lanes 0-31 carry a finished row.  The split-K partial records keep their 256-float stride.
-template <typename TQ, int NT, int KVF, bool BAL, bool VRES = false, bool STREAM = BAL, int HD = kHeadDim>
+// MAPPED: chunk grid whose workgroups go by keys or by length (rows_by_keys, rows_longest_first), else in launch order.
+template <typename TQ, int NT, int KVF, bool BAL, bool VRES = false, bool STREAM = BAL, int HD = kHeadDim, bool MAPPED = false>
 __device__ __forceinline__ void rows_tile(const AttnParams& P, uint8_t* smem, const BalItem& item) {
     static_assert(!VRES || KVF == WARP34_KV_FORMAT_FP8_E4M3 || KVF == WARP34_KV_FORMAT_Q8_0, "residual operand: 8-bit rows");
     using M = RowsLds<KVF, HD>;
@@ -224,8 +243,11 @@ __device__ __forceinline__ void rows_tile(const AttnParams& P, uint8_t* smem, co
 
     int tile_z = BAL ? item.req : (int)blockIdx.z;  // tile index (see locate_tile)
     int kv_sub = (int)blockIdx.y, chunk = BAL ? 0 : (int)blockIdx.x;
-    if constexpr (!BAL && !STREAM) {
+    if constexpr (MAPPED) {
         if (P.key_groups > 0 && !rows_by_keys(P, tile_z, kv_sub, chunk)) return;
+        if constexpr (HD != kHeadDim) {
+            if (P.first_round > 0) tile_z = rows_longest_first(P, lane, tile_z);
+        }
     }
     const int kv_head = small_div(kv_sub, P.q_subgroups);
     const int q_head_base = kv_head * P.gqa + (kv_sub - kv_head * P.q_subgroups) * P.q_group;
@@ -925,6 +947,13 @@ __global__ __launch_bounds__(kKv16Waves * 64, 1) void paged_attn_rows_kernel(con
     } else {
         rows_tile<TQ, 1, KVF, false, VRES, false, HD>(P, smem, BalItem{});
     }
+}
+// The chunk grid by keys or by length.  (A kernel of its own: with the order worked out in the other, or a third body in it, chunks of 130 tokens
+// over bf16 pages, which stay in launch order, took 4 to 5 % longer with the same instructions in the loop: 67.9 -> 71.8 us.)
+template <typename TQ, int KVF, bool VRES, int HD = kHeadDim>
+__global__ __launch_bounds__(kKv16Waves * 64, 1) void paged_attn_rows_mapped_kernel(const AttnParams P) {
+    extern __shared__ __align__(16) uint8_t smem[];
+    rows_tile<TQ, 1, KVF, false, VRES, false, HD, true>(P, smem, BalItem{});
 }
 
 template <typename TQ, int NT, int KVF, bool VRES, bool STREAM, int HD = kHeadDim>

@@ -759,7 +759,7 @@ __device__ __forceinline__ void pw_tile(const AttnParams& P, uint8_t* smem, int 
 // the latter: Q8_0 100 x 33 to 48 tokens, eight q heads per kv head, 213 / 183, bf16 128 x 129, two q heads, 869 / 816, Q8_0
 // 70 x 100 to 1 000 (32 tiles) 2 440 / 1 697; 80 x 20 to 300 (10 tiles) on 1 500 to 5 200 keys 1 389 / 1 512.
 // Requests of different lengths: whole tiles of the longest would be the batch's time, so they are cut too (pw_long_tiles).
-constexpr int kPwCus = 256;
+constexpr int kPwCus = kChipCus;
 // What a tile of a request takes, in units of its length (pf_longest_first): lane r holds request r.
 struct PwRequest {
     int first, count;  // lengths first + 1 .. first + count
