@@ -2302,7 +2302,7 @@ static int launch_tq4(const warp34_exec* ex, const warp34_kv_layer_layout* layou
             T.tok_tile = kPfRows / q_group;
             T.key_floor = nullptr;
             const int pf_tiles = (batch->total_tokens + T.tok_tile - 1) / T.tok_tile;
-                        rc = ensure_dynamic_lds(paged_prefill_tq4_kernel<TQ, true>, kPfSmem, true);
+            rc = ensure_dynamic_lds(paged_prefill_tq4_kernel<TQ, true>, kPfSmem, true);
             if (rc) return rc;
             hipLaunchKernelGGL((paged_prefill_tq4_kernel<TQ, true>),
                                dim3((unsigned)(pf_tiles * parts), (unsigned)kv_subs, 1u), dim3(12 * 64), kPfSmem,
@@ -2630,7 +2630,7 @@ static int launch_prefill_tq4(const warp34_exec* ex, const warp34_kv_layer_layou
     }
     P.tok_tile = pw_rows(2) / q_group;
     P.bal_tiles = (batch->max_q_len + P.tok_tile - 1) / P.tok_tile;
-    // (the last round's cut tiles: fewer than kPwCus / 2 workgroups more)
+    // (the last round's cut tiles: at most kPwCus / 2 workgroups more)
     const long long wgs = (long long)P.bal_tiles * kv_subs * batch->num_reqs + kPwCus / 2;
     if (wgs > 0x7fffffffll) return (int)hipErrorNotSupported;
     const dim3 grid((unsigned)std::min<long long>(wgs, 1 << 20), (unsigned)((wgs + (1 << 20) - 1) >> 20));
