@@ -1948,13 +1948,16 @@ constexpr int kMinUnitsPerWidePiece = 4;
 // line lies where the longest contexts turn (attention alone, 10 x 4 on 3K to 16K 54 against 35, 20 x 4 93 against 53).
 // (Counts of tiles, not lengths: results do not depend on max_seq_len.)
 // At head dimension 128 every such batch goes there: the plan has one column tile at that size (with two the merge of
-// the waves outweighs the keys read once more) and is nowhere ahead.  Draft blocks, layer steps: 3 x 8 on 2000 keys
-// 17.4 against 18.9, 4 x 16 on 9000 32.3 against 36.7, 12 x 8 on 8000 55 against 60, 16 x 16 on 16000 150.6 against 150.5.
+// the waves outweighs the keys read once more) and is nowhere ahead.  Draft blocks, layer steps, contexts from an eighth of the length
+// up: 3 x 8 on 2000 keys 16.2 against 19.8, 4 x 16 on 9000 24.3 against 34.2, 12 x 8 on 8000 32.9 against 44.6, 9 x 16 on 16000 69.6
+// against 103, 16 x 16 99 against 174; 8 x 16 on 6000 each 45.7 against 51.1.
 constexpr int kRowsGridTiles = 8;
 // A decode batch at head dimension 128 (four q heads per kv head) goes to the chunk grid up to this many requests.
 // Chunk grid against plan, four kv heads, us: 2 requests of 1000 keys 10.2 against 13.0, of 3K to 16K 11.6 against 15.0, of 5K to
 // 60K 24.2 against 24.4; 3 requests 10.5 against 13.3, 17.9 against 20.7, 41 against 35; 4 requests 11.8 against 13.5, 24.1
 // against 23.2, 59 against 45; 6 requests 11.7 against 13.6, 38 against 29.
+// (Those with one workgroup per CU.  With two, layer steps: 2 requests of 1000 keys 14.5 against 19.3, of 3K to 16K 16.0 against 20.4, of 5K to
+// 60K 25.1 against 25.1; 3 requests 14.7 against 19.5, 21.0 against 21.6, 40.4 against 37.0.)
 constexpr int kRowsGridRequests128 = 3;
 // Short batches (bal_short_piece): key and value rows of up to this many bytes per kv head, each counted once, for
 // batches whose entries are cut into pieces of their own anyway and for others (whose workgroups mostly have
