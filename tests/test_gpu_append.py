@@ -261,3 +261,35 @@ def test_write_argument_validation():
     assert l.warp34_kv_cache_write_strided_bf16(C.byref(ex), C.byref(L), C.byref(B), G.ptr(k), G.ptr(k), 100) == inval
     gk, gv = dpool.download()
     assert not gk.any() and not gv.any()
+
+
+@pytest.mark.parametrize("in_dtype", [DT_BF16, DT_F16])
+@pytest.mark.parametrize("k_row,v_row", [
+    ((FMT_TQ4, XF_WHT256), (FMT_TQ4, XF_IDENTITY)), ((FMT_TQ4, XF_IDENTITY), (FMT_TQ4, XF_WHT256)),
+    ((FMT_Q8_0, XF_WHT256), (FMT_Q8_0, XF_IDENTITY)), ((FMT_FP8, XF_IDENTITY), (FMT_Q8_0, XF_IDENTITY)),
+    ((FMT_TQ4, XF_WHT256), (FMT_FP8, XF_IDENTITY)), ((FMT_FP16, XF_IDENTITY), (FMT_TQ4, XF_IDENTITY)),
+])
+def test_k_and_v_rows_of_different_kinds(k_row, v_row, in_dtype):
+    """K and V slabs that differ in transform or format: each holds the rows of a layout of its own kind."""
+    import gpu_harness as G
+
+    n, bs = 77, 16
+    pages = (n + bs - 1) // bs + 1
+    bt = oracle.permutation(pages, 17)[:pages - 1].reshape(1, -1)
+    hb = oracle.HostBatch([0, n], [n], bt, context_lens_before=[0], write_slot_mapping=oracle.slot_mapping(bt[0], 0, n, bs))
+    k, v = (oracle.fill_kv_rows(n, 2, 256, seed, in_dtype, 3) for seed in (41, 42))
+    k_pool, v_pool = (oracle.HostPool(pages, 2, 256, bs, *row) for row in (k_row, v_row))
+    for pool in (k_pool, v_pool):
+        oracle.kv_cache_write(pool, hb, k, v, in_dtype)
+    k_dev, v_dev = G.DevPool(k_pool), G.DevPool(v_pool)
+    mixed, v_lay = k_dev.layout(), v_dev.layout()
+    for field, _ in mixed._fields_:
+        if field.startswith("v_"):
+            setattr(mixed, field, getattr(v_lay, field))
+    rc = G.dev_write(k_dev, hb, k, v, in_dtype, layout=mixed)
+    if in_dtype == DT_BF16 and k_row[0] != v_row[0] and FMT_TQ4 in (k_row[0], v_row[0]):
+        assert rc != 0  # the bf16 entry point takes TQ4 pages for both slabs or for neither
+        return
+    assert rc == 0
+    assert k_dev.download()[0].tobytes() == k_pool.k.tobytes()
+    assert v_dev.download()[1].tobytes() == v_pool.v.tobytes()

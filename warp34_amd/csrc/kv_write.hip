@@ -21,7 +21,10 @@ namespace w34 {
 // lanes 0-31 write K, lanes 32-63 write V.  Everything up to the row addresses is the same for
 // the whole wave and is kept in scalar registers (block_magic = floor(2^32 / block_size): the
 // page of a slot without a division).
-template <typename TIn>
+// MIXED: the layout's K and V rows differ in format or transform.  The encoders fetch their tables from all 64 lanes, so both
+// halves of a wave have to go through the same one: blockIdx.z is 0 for K and 1 for V, both halves encode that row, and the
+// first one stores it.
+template <typename TIn, bool MIXED>
 __global__ __launch_bounds__(256) void kv_append_kernel(warp34_kv_layer_layout L,
                                                         warp34_attention_batch B,
                                                         const uint16_t* __restrict__ k_in,
@@ -45,7 +48,8 @@ __global__ __launch_bounds__(256) void kv_append_kernel(warp34_kv_layer_layout L
     const int off = slot - page * L.block_size;
 
     const int lane = lane_id();
-    const int is_v = lane >> 5;
+    const int half = lane >> 5;
+    const int is_v = MIXED ? (int)blockIdx.z : half;
     const int l32 = lane & 31;
     const int format = is_v ? L.v_format : L.k_format;
     const uint64_t k_dst = L.k_base + (uint64_t)page * L.k_page_stride_bytes + (uint64_t)head * L.k_head_stride_bytes +
@@ -61,7 +65,7 @@ __global__ __launch_bounds__(256) void kv_append_kernel(warp34_kv_layer_layout L
     if (format == WARP34_KV_FORMAT_FP8_E4M3 || format == WARP34_KV_FORMAT_Q8_0) {
         // host side guarantees head_dim == 256 and 4-byte aligned rows
         float v[8];
-        uint8_t* row = rows[wave][is_v];
+        uint8_t* row = rows[wave][half];
         const int n_dwords = format == WARP34_KV_FORMAT_FP8_E4M3 ? 66 : 68;
         const uint16_t* src8 = src + 8 * l32;
         if ((reinterpret_cast<uintptr_t>(src8) & 15u) == 0) {
@@ -86,6 +90,7 @@ __global__ __launch_bounds__(256) void kv_append_kernel(warp34_kv_layer_layout L
         __atomic_signal_fence(__ATOMIC_SEQ_CST);
         __builtin_amdgcn_wave_barrier();
         __atomic_signal_fence(__ATOMIC_SEQ_CST);
+        if (MIXED && half != 0) return;
         const uint32_t* r32 = reinterpret_cast<const uint32_t*>(row);
         uint32_t* d32 = reinterpret_cast<uint32_t*>(dst);
         d32[l32] = r32[l32];
@@ -119,7 +124,7 @@ __global__ __launch_bounds__(256) void kv_append_kernel(warp34_kv_layer_layout L
         }
         // the row is assembled in LDS and leaves with one 32-bit store per lane (16-bit stores
         // when the destination is only 2-byte aligned, which is all the row format promises)
-        uint8_t* row = rows[wave][is_v];
+        uint8_t* row = rows[wave][half];
         if (rotated) {
             tq4_encode_row(v, lane, row);
         } else {
@@ -128,6 +133,7 @@ __global__ __launch_bounds__(256) void kv_append_kernel(warp34_kv_layer_layout L
         __atomic_signal_fence(__ATOMIC_SEQ_CST);
         __builtin_amdgcn_wave_barrier();
         __atomic_signal_fence(__ATOMIC_SEQ_CST);
+        if (MIXED && half != 0) return;
         if (L.head_dim == 256 && (reinterpret_cast<uintptr_t>(dst) & 3u) == 0) {
             const uint32_t* r32 = reinterpret_cast<const uint32_t*>(row);
             uint32_t* d32 = reinterpret_cast<uint32_t*>(dst);
@@ -145,6 +151,7 @@ __global__ __launch_bounds__(256) void kv_append_kernel(warp34_kv_layer_layout L
     }
     // 16-bit storage formats: plain copy when the storage type is the source type,
     // otherwise convert through fp32 (op_kv_cache.cu:18-31).
+    if (MIXED && half != 0) return;
     uint16_t* d16 = reinterpret_cast<uint16_t*>(dst);
     const bool same = (format == TIn::kStorageFormat);
     for (int c = l32; c < L.head_dim; c += 32) {
@@ -165,15 +172,18 @@ static inline uint32_t append_block_magic(int block_size) {
 template <typename TIn>
 static int launch_append(const warp34_exec* ex, const warp34_kv_layer_layout* layout,
                          const warp34_attention_batch* batch, const void* k_in, const void* v_in,
-                         int k_row_stride, int v_row_stride) {
-    const dim3 grid((unsigned)((batch->total_tokens + 3) / 4), (unsigned)layout->local_kv_heads);
-    const int check_req = (batch->valid_req_mask != nullptr && batch->query_start_loc != nullptr &&
-                           batch->num_reqs > 0)
-                              ? 1
-                              : 0;
-    hipLaunchKernelGGL((kv_append_kernel<TIn>), grid, dim3(256), 0, (hipStream_t)ex->stream,
-                       *layout, *batch, (const uint16_t*)k_in, (const uint16_t*)v_in, k_row_stride,
-                       v_row_stride, check_req, append_block_magic(layout->block_size));
+                         int k_row_stride, int v_row_stride, int check_req) {
+    const bool mixed = layout->k_format != layout->v_format || layout->k_transform != layout->v_transform;
+    const dim3 grid((unsigned)((batch->total_tokens + 3) / 4), (unsigned)layout->local_kv_heads, mixed ? 2u : 1u);
+    if (mixed) {
+        hipLaunchKernelGGL((kv_append_kernel<TIn, true>), grid, dim3(256), 0, (hipStream_t)ex->stream, *layout, *batch,
+                           (const uint16_t*)k_in, (const uint16_t*)v_in, k_row_stride, v_row_stride, check_req,
+                           append_block_magic(layout->block_size));
+    } else {
+        hipLaunchKernelGGL((kv_append_kernel<TIn, false>), grid, dim3(256), 0, (hipStream_t)ex->stream, *layout, *batch,
+                           (const uint16_t*)k_in, (const uint16_t*)v_in, k_row_stride, v_row_stride, check_req,
+                           append_block_magic(layout->block_size));
+    }
     return (int)hipGetLastError();
 }
 
@@ -205,7 +215,11 @@ extern "C" int warp34_kv_cache_write_strided(const warp34_exec* ex, const warp34
         return (int)hipErrorNotSupported;
     }
     if (!rows_aligned_for_write(layout)) return (int)hipErrorInvalidValue;
-    return launch_append<F16>(ex, layout, batch, k_in, v_in, k_row_stride, v_row_stride);
+    const int check_req = (batch->valid_req_mask != nullptr && batch->query_start_loc != nullptr &&
+                           batch->num_reqs > 0)
+                              ? 1
+                              : 0;
+    return launch_append<F16>(ex, layout, batch, k_in, v_in, k_row_stride, v_row_stride, check_req);
 }
 
 // op_kv_cache.cu:852-858
@@ -249,11 +263,7 @@ extern "C" int warp34_kv_cache_write_strided_bf16(const warp34_exec* ex,
     }
     if (!batch->total_tokens) return 0;
     // the reference's bf16 writer always resolves the owning request (op_kv_cache.cu:803-807)
-    const dim3 grid((unsigned)((batch->total_tokens + 3) / 4), (unsigned)layout->local_kv_heads);
-    hipLaunchKernelGGL((kv_append_kernel<BF16>), grid, dim3(256), 0, (hipStream_t)ex->stream,
-                       *layout, *batch, (const uint16_t*)k, (const uint16_t*)v, row_stride_elems,
-                       row_stride_elems, 1, append_block_magic(layout->block_size));
-    return (int)hipGetLastError();
+    return launch_append<BF16>(ex, layout, batch, k, v, row_stride_elems, row_stride_elems, 1);
 }
 
 // op_kv_cache.cu:1185-1190
