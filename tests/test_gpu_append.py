@@ -293,3 +293,30 @@ def test_k_and_v_rows_of_different_kinds(k_row, v_row, in_dtype):
     assert rc == 0
     assert k_dev.download()[0].tobytes() == k_pool.k.tobytes()
     assert v_dev.download()[1].tobytes() == v_pool.v.tobytes()
+
+
+@pytest.mark.parametrize("n_reqs", [1, 64, 65, 200])
+def test_owning_request_among_many(n_reqs):
+    """The bf16 entry point writes a token only if a live request owns it: empty requests, masked ones, and tokens behind the last."""
+    import gpu_harness as G
+
+    rng = np.random.default_rng(n_reqs)
+    lens = rng.integers(0, 4, n_reqs)
+    lens[0] = 3
+    qsl = np.concatenate([[0], np.cumsum(lens)])
+    n = int(qsl[-1]) + 5  # five tokens of no request
+    rmask = (rng.random(n_reqs) < 0.7).astype(np.uint8)
+    pages = (n + 15) // 16
+    bt = np.arange(pages, dtype=np.int32).reshape(1, -1)
+    k, v = (oracle.fill_kv_rows(n, 1, 256, seed, DT_BF16, 3) for seed in (51, 52))
+    pool = oracle.HostPool(pages, 1, 256, 16, FMT_TQ4, XF_WHT256)
+    hb = oracle.HostBatch(qsl, [n] * n_reqs, np.repeat(bt, n_reqs, axis=0), write_slot_mapping=oracle.slot_mapping(bt[0], 0, n, 16),
+                          valid_req_mask=rmask, total_tokens=n)
+    oracle.kv_cache_write(pool, hb, k, v, DT_BF16)
+    written = pool.k.reshape(-1, 132)[:n].any(axis=1)
+    owner = np.searchsorted(qsl, np.arange(n), side="right") - 1
+    assert (written == ((owner < n_reqs) & (rmask[np.minimum(owner, n_reqs - 1)] != 0))).all()
+    dev = G.DevPool(pool)
+    assert G.dev_write(dev, hb, k, v, DT_BF16) == 0
+    gk, gv = dev.download()
+    assert gk.tobytes() == pool.k.tobytes() and gv.tobytes() == pool.v.tobytes()

@@ -100,3 +100,20 @@ def test_producer_on_both_sides_of_the_token_limit(n, qh, kh, fmt):
     assert q.tobytes() == want_q.tobytes() and ko.tobytes() == want_k.tobytes() and g.tobytes() == want_g.tobytes()
     gk, gv = dev.download()
     assert gk.tobytes() == pool.k.tobytes() and gv.tobytes() == pool.v.tobytes()
+
+
+def test_rows_on_both_sides_of_the_short_transform():
+    """Rows whose sum of squares sends a wave to the exact transform beside rows that stay on the short one: energies around 1e-15 / 256 and
+    around the largest finite sum of 16-fold values, zeros, subnormal elements, single elements."""
+    rng = np.random.default_rng(11)
+    rows = [rng.standard_normal(256) * 10.0 ** e for e in np.concatenate([np.arange(-10.6, -9.2, 0.05), np.arange(16.4, 18.4, 0.1)])]
+    for e in (-38, -30, -20, 0):
+        row = rng.standard_normal(256)
+        row[rng.permutation(256)[:200]] *= 10.0 ** e
+        rows += [row, np.where(np.arange(256) < 128, row, 0.0)]
+    for i in range(16):
+        spike = np.zeros(256)
+        spike[17 * i] = 2.0 ** (i - 8)
+        rows.append(spike)
+    rows.append(np.zeros(256))
+    _append_equals_oracle(rng.permutation(np.stack(rows)).astype(np.float32), DT_BF16, XF_WHT256)

@@ -106,6 +106,32 @@ def test_dense_wrapper_equals_strided():
             assert g.reshape(w.shape).tobytes() == w.tobytes()
 
 
+@pytest.mark.parametrize("theta,top", [(THETA, 2 ** 31 - 1), (10000.0, 2 ** 20), (0.5, 262143), (1.0e-9, 2 ** 31 - 1)])
+def test_angles_of_any_size(theta, top):
+    """Sines and cosines of angles up to the largest position, and above it where the base is below 1."""
+    n, qh, kh, hd, rot = 512, 1, 1, 256, 64
+    qg, k, qw, kw = _inputs(n, qh, kh, hd, 23)
+    pos = np.random.default_rng(24).integers(0, top, size=(3, n), endpoint=True).astype(np.int32)
+    pos[:, 0] = top
+    want = oracle.fused_qk_rmsnorm_rope_gate_f16(qg, k, qw, kw, pos, qh, kh, hd, rot, MROPE, theta, EPS)
+    rc, got = _dev_operator(qg, k, qw, kw, pos, qh, kh, hd, rot, theta=theta)
+    assert rc == 0
+    for g, w in zip(got, want):
+        assert g.reshape(w.shape).tobytes() == w.tobytes()
+
+
+@pytest.mark.parametrize("n,qh,kh", [(1, 4095, 1), (2, 4096, 3), (1, 1, 1024)])
+def test_head_counts_on_both_sides_of_the_packed_argument(n, qh, kh):
+    hd, rot = 64, 32
+    qg, k, qw, kw = _inputs(n, qh, kh, hd, 25)
+    pos = _positions(n, 26)
+    want = oracle.fused_qk_rmsnorm_rope_gate_f16(qg, k, qw, kw, pos, qh, kh, hd, rot, (6, 5, 5), THETA, EPS)
+    rc, got = _dev_operator(qg, k, qw, kw, pos, qh, kh, hd, rot, mrope=(6, 5, 5))
+    assert rc == 0
+    for g, w in zip(got, want):
+        assert g.reshape(w.shape).tobytes() == w.tobytes()
+
+
 def _dev_fused_write(dpool, qg, k, v, qw, kw, pos, slots, qh, kh, hd, rot, mask=None, with_k_out=True, layout=None):
     import torch
     import gpu_harness as G

@@ -19,15 +19,17 @@ COMMON = ["-O3", "-std=c++17", "-fPIC", "-Wall", "-Wno-unused-function"]
 # packed fp32 VALU forms are kept out of every device object
 DEVICE = ["--offload-arch=" + ARCH, "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 
+# leading scalar kernel arguments are preloaded into SGPRs at wave launch (gfx950 feature;
+# firmware without it runs the compatibility prologue the compiler emits)
+PRELOAD = ["-mllvm", "-amdgpu-kernarg-preload-count=14"]
+
 SOURCES = [
     # (path, extra flags)
-    (os.path.join(CSRC, "kv_write.hip"), ["-ffp-contract=off"]),
+    (os.path.join(CSRC, "kv_write.hip"), ["-ffp-contract=off"] + PRELOAD),
     (os.path.join(CSRC, "qk_norm_rope.hip"), ["-ffp-contract=off"]),
     (os.path.join(CSRC, "attn_output_gate.hip"), ["-ffp-contract=off"]),
     (os.path.join(CSRC, "fused_qk_norm.hip"), ["-ffp-contract=off"]),
-    # leading scalar kernel arguments are preloaded into SGPRs at wave launch (gfx950 feature;
-    # firmware without it runs the compatibility prologue the compiler emits)
-    (os.path.join(CSRC, "paged_attn.hip"), ["-mllvm", "-amdgpu-kernarg-preload-count=12"]),
+    (os.path.join(CSRC, "paged_attn.hip"), PRELOAD),
     (os.path.join(CSRC, "runtime.hip"), []),
     (os.path.join(HOST, "kv_host.cpp"), []),
     (os.path.join(HOST, "prefix_cache.cpp"), []),

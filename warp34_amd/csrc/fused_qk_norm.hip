@@ -23,6 +23,7 @@
 // fp32 in source order; the eight squares of a lane added in order, then the 32-lane xor
 // butterfly 16,8,4,2,1; rsqrt, powf, sinf, cosf = the double-precision result rounded once to
 // fp32 (theta^(2i/rotary) on the host, it does not depend on the token); fp16 RNE.
+#include <algorithm>
 #include <cmath>
 
 #include "kv_encode.h"
@@ -38,66 +39,116 @@ constexpr int kFqSpreadTokens = 256;
 
 struct FusedQkParams {
     const uint16_t* q_gate_in;
-    const uint16_t* k_in;
-    const uint16_t* v_in;  // cache write only
     const uint16_t* qw;
-    const uint16_t* kw;
-    const int32_t* positions;
     const uint8_t* mask;
     uint16_t* q_out;
     uint16_t* k_out;  // may be null when the cache is written
     uint16_t* gate_out;
     const int32_t* write_slot_mapping;  // null: no cache write
     warp34_kv_layer_layout L;
-    int num_tokens, pos_plane_stride, q_heads, kv_heads, head_dim, rotary_dim, s1, s2;
-    int q_stride, k_stride, v_stride;
+    int num_tokens, q_stride, q_heads, kv_heads;
     float eps;
     float inv_freq[kFqMaxPairs];
 };
 
-template <bool SPREAD>
-__global__ __launch_bounds__(256) void fused_qk_norm_rope_gate_kernel(const FusedQkParams P) {
+// sin and cos of an angle of at most 2^31 in double precision, rounded to fp32: the multiple of pi / 2 is taken off in two parts
+// (the product of the first is exact inside the fma: an angle has 24 bits, the multiple 31), the rest, within pi / 4, goes
+// through the Taylor series to r^15 and r^16 (remainders below 5e-17).  Within an ulp of double precision, as the library's
+// functions are, which need 87 registers and 4 times the instructions for angles of any size.
+__device__ __forceinline__ void sin_cos_rounded(float angle, float& s, float& c) {
+    const double x = (double)angle, n = __builtin_rint(x * 0.636619772367581343);  // 2 / pi
+    const double r = __builtin_fma(-n, 6.12323399573676604e-17, __builtin_fma(-n, 1.57079632679489656, x));
+    const double r2 = r * r;
+    double ps = -1.0 / 1307674368000.0;
+    ps = __builtin_fma(ps, r2, 1.0 / 6227020800.0);
+    ps = __builtin_fma(ps, r2, -1.0 / 39916800.0);
+    ps = __builtin_fma(ps, r2, 1.0 / 362880.0);
+    ps = __builtin_fma(ps, r2, -1.0 / 5040.0);
+    ps = __builtin_fma(ps, r2, 1.0 / 120.0);
+    ps = __builtin_fma(ps, r2, -1.0 / 6.0);
+    const double sine = __builtin_fma(r * r2, ps, r);
+    double pc = 1.0 / 20922789888000.0;
+    pc = __builtin_fma(pc, r2, -1.0 / 87178291200.0);
+    pc = __builtin_fma(pc, r2, 1.0 / 479001600.0);
+    pc = __builtin_fma(pc, r2, -1.0 / 3628800.0);
+    pc = __builtin_fma(pc, r2, 1.0 / 40320.0);
+    pc = __builtin_fma(pc, r2, -1.0 / 720.0);
+    pc = __builtin_fma(pc, r2, 1.0 / 24.0);
+    pc = __builtin_fma(pc, r2, -0.5);
+    const double cosine = __builtin_fma(pc, r2, 1.0);
+    const int q = (int)n;
+    const double a = (q & 1) ? cosine : sine, b = (q & 1) ? sine : cosine;
+    s = (float)((q & 2) ? -a : a);
+    c = (float)(((q + 1) & 2) ? -b : b);
+}
+
+// Three small numbers in one kernel argument
+struct FqPacked {
+    __host__ static uint32_t of(int a, int b, int c) { return (uint32_t)a | (uint32_t)b << 12 | (uint32_t)c << 22; }
+    __device__ static int a(uint32_t x) { return (int)(x & 4095u); }
+    __device__ static int b(uint32_t x) { return (int)(x >> 12 & 1023u); }
+    __device__ static int c(uint32_t x) { return (int)(x >> 22); }
+};
+// A small batch is a chain of memory round trips.  The leading arguments are in scalar registers when a wave starts: the sine / cosine
+// values and the K / V items, the longest parts, ask for their data at once instead of behind the argument block; slot and
+// block arrive meanwhile, and what an item's end uses is requested with its row.
+// heads: q heads, kv heads, head size; rot: rotary pairs, sections 1 and 2 of the three position planes
+// ROTATED_TQ4: pages of that kind only.  ANY: angles above 2^31 (a base below 1), head counts that `heads` cannot hold.
+template <bool SPREAD, bool ROTATED_TQ4, bool ANY>
+__global__ __launch_bounds__(256) void fused_qk_norm_rope_gate_kernel(
+    const int32_t* __restrict__ positions, const uint16_t* __restrict__ k_in, const uint16_t* __restrict__ v_in,
+    const uint16_t* __restrict__ kw, int k_stride, int v_stride, int pos_plane_stride, uint32_t heads, uint32_t rot, const FusedQkParams P) {
     __shared__ float s_cos[kFqMaxPairs], s_sin[kFqMaxPairs];
     __shared__ __align__(16) uint16_t s_row[4][2][256];
     __shared__ __align__(8) uint8_t s_enc[4][2][272];
     const int tok = (int)blockIdx.x;
-    if (P.mask != nullptr && P.mask[tok] == 0) return;
-    const int wave = (int)(threadIdx.x >> 6);
-    const int lane = lane_id();
-    const int half_id = lane >> 5;
-    const int l32 = lane & 31;
-    const int hd = P.head_dim, half_rot = P.rotary_dim >> 1;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int q_heads = ANY ? P.q_heads : FqPacked::a(heads), kv_heads = ANY ? P.kv_heads : FqPacked::b(heads), hd = FqPacked::c(heads);
+    const int half_rot = FqPacked::a(rot), s1 = FqPacked::b(rot), s2 = FqPacked::c(rot);
+    const int q_items = (q_heads + 1) >> 1;
+    const int n_items = q_items + kv_heads;
 
     // The token's sine / cosine values: the last wave computes them (it has the fewest items),
     // the others go ahead with the first half of their first item and meet it at the barrier
     // in front of the first rotation.
     if (wave == 3) {
-        for (int i = lane; i < half_rot; i += 64) {
+        for (int i = lane_id(); i < half_rot; i += 64) {
             int plane = 0;
-            if ((i % 3) == 1 && i < P.s1 * 3) {
+            if ((i % 3) == 1 && i < s1 * 3) {
                 plane = 1;
-            } else if ((i % 3) == 2 && i < P.s2 * 3) {
+            } else if ((i % 3) == 2 && i < s2 * 3) {
                 plane = 2;
             }
-            const float pos = (float)P.positions[(size_t)plane * P.pos_plane_stride + tok];
+            const float pos = (float)positions[(size_t)plane * pos_plane_stride + tok];
             const float angle = pos * P.inv_freq[i];
-            s_sin[i] = F16::to_f32(F16::from_f32_of_fp32_result((float)sin((double)angle)));
-            s_cos[i] = F16::to_f32(F16::from_f32_of_fp32_result((float)cos((double)angle)));
+            float sine, cosine;
+            if constexpr (ANY) {
+                sine = (float)sin((double)angle);
+                cosine = (float)cos((double)angle);
+            } else {
+                sin_cos_rounded(angle, sine, cosine);
+            }
+            s_sin[i] = F16::to_f32(F16::from_f32_of_fp32_result(sine));
+            s_cos[i] = F16::to_f32(F16::from_f32_of_fp32_result(cosine));
+        }
+        if (P.mask != nullptr && P.mask[tok] == 0) return;  // (behind the requests, as in the other waves)
+        if (SPREAD) {
+            __syncthreads();
+            return;
         }
     }
     bool trig_ready = false;  // wave-uniform: this wave has passed the barrier behind the sine / cosine values
 
-    const bool to_cache_any = P.write_slot_mapping != nullptr;
-    const int slot = to_cache_any ? P.write_slot_mapping[tok] : -1;
-    const bool to_cache = slot >= 0;  // uniform
-    const int q_items = (P.q_heads + 1) >> 1;
-    const int n_items = q_items + P.kv_heads;
-    uint16_t* row = s_row[wave][half_id];
-    const bool owns_vec = 8 * l32 < hd;
-
     // SPREAD: three items per workgroup, one per wave, beside the wave of the sine / cosine values
-    const int first = SPREAD ? (wave == 3 ? n_items : 3 * (int)blockIdx.y + wave) : wave;
+    const int first = SPREAD ? 3 * (int)blockIdx.y + wave : wave;
+    int slot = -1;
     for (int it = first; it < n_items; it += SPREAD ? n_items : 4) {  // wave-uniform
+        // (the lane and what follows from it are worked out for each item: kept, they cost 25 registers and two waves a SIMD)
+        int lane = lane_id();
+        asm volatile("" : "+v"(lane));
+        const int half_id = lane >> 5, l32 = lane & 31;
+        uint16_t* row = s_row[wave][half_id];
+        const bool owns_vec = 8 * l32 < hd;
         const bool is_q = it < q_items;
         const int kv_head = is_q ? 0 : it - q_items;
         const bool is_v_half = !is_q && half_id == 1;
@@ -106,25 +157,37 @@ __global__ __launch_bounds__(256) void fused_qk_norm_rope_gate_kernel(const Fuse
         // a half without a head of its own (the second half of the last Q item when q_heads is odd,
         // the second half of a KV item when no V row is encoded) works on a row it may read and
         // stores nothing.
-        const bool has_head = is_q ? q_head < P.q_heads : (!is_v_half || to_cache);
-        if (is_q && q_head >= P.q_heads) q_head = P.q_heads - 1;
+        const bool has_head = q_head < q_heads;  // (of a Q item)
+        if (q_head >= q_heads) q_head = q_heads - 1;
         const uint16_t* src;
-        const uint16_t* w = is_q ? P.qw : P.kw;
         if (is_q) {
             src = P.q_gate_in + (size_t)tok * P.q_stride + (size_t)q_head * 2 * hd;
-        } else if (is_v_half && to_cache) {
-            src = P.v_in + (size_t)tok * P.v_stride + (size_t)kv_head * hd;
+        } else if (is_v_half && v_in != nullptr) {
+            src = v_in + (size_t)tok * v_stride + (size_t)kv_head * hd;
         } else {
-            src = P.k_in + (size_t)tok * P.k_stride + (size_t)kv_head * hd;
+            src = k_in + (size_t)tok * k_stride + (size_t)kv_head * hd;
         }
+        const uint16_t* w = is_q ? P.qw : kw;
 
         // ---- sum of squares and normalisation: lane t owns elements 8t .. 8t+7 ----
         uint4 raw = {0u, 0u, 0u, 0u};
         uint4 wraw = {0u, 0u, 0u, 0u};
+        // what the item's end uses: the gate of a Q item, the encoder's lane entry of a KV item
+        uint4 late0 = {0u, 0u, 0u, 0u}, late1 = {0u, 0u, 0u, 0u};
         if (owns_vec) {
             raw = *reinterpret_cast<const uint4*>(src + 8 * l32);
             wraw = *reinterpret_cast<const uint4*>(w + 8 * l32);
+            if (is_q) late0 = *reinterpret_cast<const uint4*>(src + hd + 8 * l32);
         }
+        if (!is_q) {
+            late0 = tq4_lane_entry(lane)[0];
+            late1 = tq4_lane_entry(lane)[1];
+        }
+        if (SPREAD || it == first) {  // (behind the requests of the first row)
+            if (P.mask != nullptr && P.mask[tok] == 0) return;
+            if (P.write_slot_mapping != nullptr) slot = P.write_slot_mapping[tok];
+        }
+        const bool to_cache = slot >= 0;  // uniform
         // (halves taken out and put together with shifts: indexing the vectors through a pointer
         // would move them to scratch memory)
         const uint32_t rw[4] = {raw.x, raw.y, raw.z, raw.w};
@@ -180,14 +243,13 @@ __global__ __launch_bounds__(256) void fused_qk_norm_rope_gate_kernel(const Fuse
         // ---- outputs ----
         if (is_q) {
             if (has_head && owns_vec) {
-                *reinterpret_cast<uint4*>(P.q_out + ((size_t)tok * P.q_heads + q_head) * hd + 8 * l32) =
+                *reinterpret_cast<uint4*>(P.q_out + ((size_t)tok * q_heads + q_head) * hd + 8 * l32) =
                     *reinterpret_cast<const uint4*>(row + 8 * l32);
-                *reinterpret_cast<uint4*>(P.gate_out + ((size_t)tok * P.q_heads + q_head) * hd + 8 * l32) =
-                    *reinterpret_cast<const uint4*>(src + hd + 8 * l32);
+                *reinterpret_cast<uint4*>(P.gate_out + ((size_t)tok * q_heads + q_head) * hd + 8 * l32) = late0;
             }
         } else {
             if (!is_v_half && P.k_out != nullptr && owns_vec) {
-                *reinterpret_cast<uint4*>(P.k_out + ((size_t)tok * P.kv_heads + kv_head) * hd + 8 * l32) =
+                *reinterpret_cast<uint4*>(P.k_out + ((size_t)tok * kv_heads + kv_head) * hd + 8 * l32) =
                     *reinterpret_cast<const uint4*>(row + 8 * l32);
             }
             if (to_cache) {
@@ -207,8 +269,8 @@ __global__ __launch_bounds__(256) void fused_qk_norm_rope_gate_kernel(const Fuse
                         v[2 * j + 1] = F16::to_f32((uint16_t)(w[j] >> 16));
                     }
                 }
-                encode_store_row(v, is_v_half ? P.L.v_format : P.L.k_format, is_v_half ? P.L.v_transform : P.L.k_transform,
-                                 lane, s_enc[wave][half_id], dst);
+                encode_store_row<ROTATED_TQ4>(v, is_v_half ? P.L.v_format : P.L.k_format, is_v_half ? P.L.v_transform : P.L.k_transform,
+                                 lane, tq4_lane_of(late0, late1), s_enc[wave][half_id], dst);
             }
         }
         // the next item of this wave overwrites the row buffer
@@ -235,12 +297,8 @@ static int launch_fused_qk(const warp34_exec* ex, const void* q_gate_in, const v
         return (int)hipErrorNotSupported;
     }
     FusedQkParams P{};
-    P.q_gate_in = (const uint16_t*)q_gate_in;
-    P.k_in = (const uint16_t*)k_in;
-    P.v_in = (const uint16_t*)v_in;
     P.qw = (const uint16_t*)q_norm_w;
-    P.kw = (const uint16_t*)k_norm_w;
-    P.positions = positions;
+    P.q_gate_in = (const uint16_t*)q_gate_in;
     P.mask = valid_token_mask;
     P.q_out = (uint16_t*)q_out;
     P.k_out = (uint16_t*)k_out;
@@ -248,29 +306,35 @@ static int launch_fused_qk(const warp34_exec* ex, const void* q_gate_in, const v
     P.write_slot_mapping = write_slot_mapping;
     if (layout != nullptr) P.L = *layout;
     P.num_tokens = num_tokens;
-    P.pos_plane_stride = pos_plane_stride;
+    P.q_stride = q_gate_row_stride;
     P.q_heads = num_q_heads;
     P.kv_heads = num_kv_heads;
-    P.head_dim = head_dim;
-    P.rotary_dim = rotary_dim;
-    P.s1 = mrope_s1;
-    P.s2 = mrope_s2;
-    P.q_stride = q_gate_row_stride;
-    P.k_stride = k_row_stride;
-    P.v_stride = v_row_stride;
     P.eps = rms_eps;
+    bool any = num_q_heads >= 4096 || num_kv_heads >= 1024;
     for (int i = 0; i < rotary_dim / 2; ++i) {
         const float expo = (float)(2 * i) / (float)rotary_dim;
         const float pw = (float)std::pow((double)rope_theta, (double)expo);
         P.inv_freq[i] = 1.0f / pw;
+        any = any || !(P.inv_freq[i] <= 1.0f);  // (a position is below 2^31)
     }
+    // sections behind the last pair, and none (a pair i takes the plane of i % 3 below 3 s)
+    const int s1 = std::max(0, std::min(mrope_s1, kFqMaxPairs)), s2 = std::max(0, std::min(mrope_s2, kFqMaxPairs));
     const int items = (num_q_heads + 1) / 2 + num_kv_heads;
-    if (num_tokens <= kFqSpreadTokens) {
-        hipLaunchKernelGGL(fused_qk_norm_rope_gate_kernel<true>, dim3((unsigned)num_tokens, (unsigned)((items + 2) / 3)), dim3(256), 0,
-                           (hipStream_t)ex->stream, P);
+    const bool spread = num_tokens <= kFqSpreadTokens;
+    const dim3 grid((unsigned)num_tokens, spread ? (unsigned)((items + 2) / 3) : 1u);
+    const auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, dim3(256), 0, (hipStream_t)ex->stream, positions, (const uint16_t*)k_in, (const uint16_t*)v_in,
+                           (const uint16_t*)k_norm_w, k_row_stride, v_row_stride, pos_plane_stride,
+                           FqPacked::of(num_q_heads & 4095, num_kv_heads & 1023, head_dim), FqPacked::of(rotary_dim / 2, s1, s2), P);
+    };
+    const bool rotated_tq4 = layout != nullptr && layout->k_format == WARP34_KV_FORMAT_TQ4 &&  // (V rows: the same, see the entry point)
+                             layout->k_transform == WARP34_KV_TRANSFORM_RADEMACHER_WHT256;
+    if (any) {
+        spread ? launch(fused_qk_norm_rope_gate_kernel<true, false, true>) : launch(fused_qk_norm_rope_gate_kernel<false, false, true>);
+    } else if (rotated_tq4) {
+        spread ? launch(fused_qk_norm_rope_gate_kernel<true, true, false>) : launch(fused_qk_norm_rope_gate_kernel<false, true, false>);
     } else {
-        hipLaunchKernelGGL(fused_qk_norm_rope_gate_kernel<false>, dim3((unsigned)num_tokens), dim3(256), 0,
-                           (hipStream_t)ex->stream, P);
+        spread ? launch(fused_qk_norm_rope_gate_kernel<true, false, false>) : launch(fused_qk_norm_rope_gate_kernel<false, false, false>);
     }
     return (int)hipGetLastError();
 }

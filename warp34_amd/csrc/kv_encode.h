@@ -91,16 +91,8 @@ __device__ __forceinline__ void wht_lane_stage16(float& a, float& b) {
     b = __uint_as_float(o[1]);
 }
 
-// sign[i] * x[i], then the 256-point Walsh-Hadamard transform with the 1/16 scale on the last
-// stage; v[j] = x[8 l32 + j] on entry and y[8 l32 + j] on return.
-__device__ __forceinline__ void sign_wht256(float (&v)[8], int lane) {
-    const int l32 = lane & 31;
-    {
-        const uint32_t sb = sign_word(l32 >> 2) >> (8 * (l32 & 3));
-#pragma unroll
-        for (int j = 0; j < 8; ++j) v[j] = __uint_as_float(__float_as_uint(v[j]) ^ (((sb >> j) & 1u) << 31));
-    }
-    // stages 1, 2, 4: registers
+// stages 1, 2, 4 of the 256-point Walsh-Hadamard transform: registers
+__device__ __forceinline__ void wht_register_stages(float (&v)[8]) {
 #pragma unroll
     for (int j = 0; j < 8; j += 2) {
         const float a = v[j], b = v[j + 1];
@@ -122,6 +114,10 @@ __device__ __forceinline__ void sign_wht256(float (&v)[8], int lane) {
         v[i] = a + b;
         v[i + 4] = a - b;
     }
+}
+// The transform with the 1/16 scale on the last stage; v[j] = x[8 l32 + j] on entry and y[8 l32 + j] on return.
+__device__ __forceinline__ void wht256(float (&v)[8], int lane) {
+    wht_register_stages(v);
     // stages 8 .. 128: lanes (each stage over all eight registers: independent instructions
     // between a write and the cross-lane read of it)
     const uint32_t f1 = (uint32_t)(lane & 1) << 31, f2 = (uint32_t)(lane & 2) << 30, f8 = (uint32_t)(lane & 8) << 28;
@@ -139,15 +135,69 @@ __device__ __forceinline__ void sign_wht256(float (&v)[8], int lane) {
         v[j + 1] *= 0.0625f;
     }
 }
+// sign[i] * x[i], then the transform
+__device__ __forceinline__ void sign_wht256(float (&v)[8], int lane) {
+    const int l32 = lane & 31;
+    const uint32_t sb = sign_word(l32 >> 2) >> (8 * (l32 & 3));
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = __uint_as_float(__float_as_uint(v[j]) ^ (((sb >> j) & 1u) << 31));
+    wht256(v, lane);
+}
+// Sixteen times the transform, negated in the lanes where wht256_flipped() says so: a lane stage is then one instruction a value,
+// x +- x[lane ^ H] (the exact form's difference is x[lane ^ H] - x in the lanes with bit H set, the same but for its sign).  A
+// zero may have the other sign than the exact form's.
+__device__ __forceinline__ constexpr bool wht256_flipped(int lane) { return __builtin_popcount(lane & 11) & 1; }
+__device__ __forceinline__ void wht256_times16_flipped(float (&v)[8], int lane) {
+    wht_register_stages(v);
+    const float s1 = (lane & 1) ? -1.0f : 1.0f, s2 = (lane & 2) ? -1.0f : 1.0f, s8 = (lane & 8) ? -1.0f : 1.0f;
+    // (a value is read across lanes two instructions behind its write at the earliest)
+    asm("s_nop 1\n\t"
+        "v_fmac_f32_dpp %0, %0, %8 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %1, %1, %8 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %2, %2, %8 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %3, %3, %8 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %4, %4, %8 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %5, %5, %8 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %6, %6, %8 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %7, %7, %8 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %0, %0, %9 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %1, %1, %9 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %2, %2, %9 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %3, %3, %9 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %4, %4, %9 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %5, %5, %9 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %6, %6, %9 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %7, %7, %9 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+        "s_nop 1"
+        : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]), "+v"(v[6]), "+v"(v[7])
+        : "v"(s1), "v"(s2));
+    wht_lane_stage4(v);
+    asm("s_nop 1\n\t"
+        "v_fmac_f32_dpp %0, %0, %8 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %1, %1, %8 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %2, %2, %8 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %3, %3, %8 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %4, %4, %8 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %5, %5, %8 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %6, %6, %8 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %7, %7, %8 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+        "s_nop 1"
+        : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]), "+v"(v[6]), "+v"(v[7])
+        : "v"(s8));
+#pragma unroll
+    for (int j = 0; j < 8; j += 2) wht_lane_stage16(v[j], v[j + 1]);
+}
 
 // sums of the eight 32-element groups: lanes 4 g .. 4 g + 3 receive the sum of group g, added
-// in the order of the 32-lane butterfly (element e with e ^ 16, then ^ 8, ^ 4, ^ 2, ^ 1)
+// in the order of the 32-lane butterfly (element e with e ^ 16, then ^ 8, ^ 4, ^ 2, ^ 1).  FLIPPED: of values negated in the lanes
+// of wht256_flipped(), where lane ^ 2 and lane ^ 1 are the other way; the sums come out negated in the same lanes.
+template <bool FLIPPED = false>
 __device__ __forceinline__ float group32_sums(const float (&p)[8], int lane) {
     float t[8];
 #pragma unroll
-    for (int r = 0; r < 8; ++r) t[r] = p[r] + lane_xor<2>(p[r], lane);
+    for (int r = 0; r < 8; ++r) t[r] = FLIPPED ? lane_xor<2>(p[r], lane) - p[r] : p[r] + lane_xor<2>(p[r], lane);
 #pragma unroll
-    for (int r = 0; r < 8; ++r) t[r] = t[r] + lane_xor<1>(t[r], lane);
+    for (int r = 0; r < 8; ++r) t[r] = FLIPPED ? lane_xor<1>(t[r], lane) - t[r] : t[r] + lane_xor<1>(t[r], lane);
     const float a0 = t[0] + t[4], a1 = t[1] + t[5], a2 = t[2] + t[6], a3 = t[3] + t[7];
     const float b0 = a0 + a2, b1 = a1 + a3;
     return b0 + b1;
@@ -186,31 +236,60 @@ constexpr bool tq4_boundaries_inside_cells() {
     return __builtin_popcountll(tq4_cells_with_boundary()) == 15;
 }
 static_assert(tq4_boundaries_inside_cells(), "every boundary in a cell of its own, away from its edges");
-struct Tq4Tables {  // lane i: of cell i the boundary in it (or +inf) and 4 (16 + number of boundaries below it); centroid i % 16
-    int boundary, at, centroid;
+// What a lane of the encoder holds throughout, from one table of constants (two loads that are on their way beside those of the
+// row; worked out, 45 vector instructions of a wave's 433).
+struct __attribute__((aligned(16))) Tq4Lane {
+    uint32_t sign[4];  // of elements 8 l32 + 2 k (bit 15) and + 2 k + 1 (bit 31): the signs of the rotation, set where negative
+    float boundary;    // lane i: of cell i the boundary in it (or +inf)
+    int at;            // 4 (16 + number of boundaries below cell i)
+    float centroid;    // i % 16
+    float scale;       // 1/16, negated in the lanes of wht256_flipped()
 };
-__device__ __forceinline__ Tq4Tables tq4_tables(int lane) {
+struct Tq4LaneTable {
+    Tq4Lane lane[64];
+};
+constexpr Tq4LaneTable make_tq4_lane_table() {
+    Tq4LaneTable t{};
     constexpr uint64_t kCells = tq4_cells_with_boundary();
-    const int below = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(kCells >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)kCells, 0u));
-    const bool has = (kCells >> lane) & 1ull;
-    const float boundary = kBoundaries[below < 15 ? below : 14];
-    return Tq4Tables{has ? __float_as_int(boundary) : 0x7F800000, 4 * (16 + below), __float_as_int(kCentroids[lane & 15])};
+    int below = 0;
+    for (int i = 0; i < 64; ++i) {
+        Tq4Lane& l = t.lane[i];
+        for (int k = 0; k < 4; ++k) {
+            const int e = 8 * (i & 31) + 2 * k;
+            const uint32_t even = kSignMask[e >> 5] >> (e & 31) & 1u, odd = kSignMask[(e + 1) >> 5] >> ((e + 1) & 31) & 1u;
+            l.sign[k] = even << 15 | odd << 31;
+        }
+        const bool has = (kCells >> i) & 1u;
+        l.boundary = has ? kBoundaries[below] : __builtin_inff();
+        l.at = 4 * (16 + below);
+        below += has ? 1 : 0;
+        l.centroid = kCentroids[i & 15];
+        l.scale = wht256_flipped(i) ? -0.0625f : 0.0625f;
+    }
+    return t;
 }
-__device__ __forceinline__ void tq4_codes(const float (&v)[8], float inv_norm, const Tq4Tables& tab, uint32_t& halves_lo,
+__device__ __constant__ constexpr Tq4LaneTable kTq4LaneTable = make_tq4_lane_table();
+__device__ __forceinline__ const uint4* tq4_lane_entry(int lane) { return reinterpret_cast<const uint4*>(&kTq4LaneTable.lane[lane]); }
+__device__ __forceinline__ Tq4Lane tq4_lane_of(const uint4 a, const uint4 b) {  // the entry's two halves
+    return Tq4Lane{{a.x, a.y, a.z, a.w}, __uint_as_float(b.x), (int)b.y, __uint_as_float(b.z), __uint_as_float(b.w)};
+}
+__device__ __forceinline__ Tq4Lane tq4_lane(int lane) {
+    const uint4* src = tq4_lane_entry(lane);
+    return tq4_lane_of(src[0], src[1]);
+}
+__device__ __forceinline__ void tq4_codes(const float (&v)[8], float inv_norm, const Tq4Lane& tab, uint32_t& halves_lo,
                                           uint32_t& halves_hi, float (&c)[8]) {
     int at[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
         const float u = v[j] * inv_norm;
-        // four times the cell: the byte address ds_bpermute takes, which ignores its two low bits.  The conversion
-        // saturates, NaN to 0 (a NaN is above no boundary).
-        uint32_t cell;
-        asm("v_cvt_u32_f32 %0, %1" : "=v"(cell) : "v"(__builtin_fmaf(u, 4.0f * kCellsPerUnit, 4.0f * kCellOfZero)));
-        cell = cell < 255u ? cell : 255u;
-        const float t = __int_as_float(__builtin_amdgcn_ds_bpermute((int)cell, tab.boundary));
+        // four times the cell: the byte address ds_bpermute takes, which ignores its two low bits.  The conversion saturates at 0 and
+        // 255, NaN to 0 (a NaN is above no boundary); whether it rounds or truncates is an eighth of a cell.
+        const uint32_t cell = __builtin_amdgcn_cvt_pk_u8_f32(__builtin_fmaf(u, 4.0f * kCellsPerUnit, 4.0f * kCellOfZero), 0u, 0u);
+        const float t = __int_as_float(__builtin_amdgcn_ds_bpermute((int)cell, __float_as_int(tab.boundary)));
         const int below = __builtin_amdgcn_ds_bpermute((int)cell, tab.at);
         at[j] = below + ((u > t) ? 4 : 0);  // 4 (16 + code)
-        c[j] = __int_as_float(__builtin_amdgcn_ds_bpermute(at[j], tab.centroid));
+        c[j] = __int_as_float(__builtin_amdgcn_ds_bpermute(at[j], __float_as_int(tab.centroid)));
     }
     // nibble pairs (even element low), two bytes per half: 4 (code bytes) + what the sixteens add up to
     constexpr int kSixteens = 64 * (1 + 16) * (1 + 256);
@@ -219,13 +298,19 @@ __device__ __forceinline__ void tq4_codes(const float (&v)[8], float inv_norm, c
     halves_hi = (uint32_t)(p2 + 256 * p3 - kSixteens) >> 2;
 }
 
-// TQ4 encode of one 256-wide row, v[j] = x[8 l32 + j] (op_kv_cache.cu:152-218).  The 132 row
+// TQ4 encode of one 256-wide row, v[j] = sign * x[8 l32 + j] (op_kv_cache.cu:152-218).  The 132 row
 // bytes are assembled in `row` (LDS, private to this half-wave).  Lanes 0-15 hold the first
 // scale block, lanes 16-31 the second: one instruction stream computes both norms and scales.
-__device__ __forceinline__ void tq4_encode_row(float (&v)[8], int lane, uint8_t* row) {
+__device__ __forceinline__ void tq4_store_codes(uint8_t* row, int l32, uint32_t lo, uint32_t hi) {
+    // byte m of a 64-byte block holds elements 2m (low nibble) and 2m + 1 (high nibble):
+    // elements 8 l32 .. + 7 are bytes 4 (l32 % 16) .. + 3 of block l32 / 16
+    uint8_t* wdst = row + 66 * (l32 >> 4) + 2 + 4 * (l32 & 15);
+    *reinterpret_cast<uint16_t*>(wdst) = (uint16_t)lo;
+    *reinterpret_cast<uint16_t*>(wdst + 2) = (uint16_t)hi;
+}
+__device__ __forceinline__ void tq4_encode_row_exact(float (&v)[8], int lane, const Tq4Lane& tab, uint8_t* row) {
     const int l32 = lane & 31;
-    const Tq4Tables tab = tq4_tables(lane);
-    sign_wht256(v, lane);
+    wht256(v, lane);
 
     float p[8];
 #pragma unroll
@@ -237,11 +322,7 @@ __device__ __forceinline__ void tq4_encode_row(float (&v)[8], int lane, uint8_t*
     float c[8];
     uint32_t lo, hi;
     tq4_codes(v, inv_norm, tab, lo, hi, c);
-    // byte m of a 64-byte block holds elements 2m (low nibble) and 2m + 1 (high nibble):
-    // elements 8 l32 .. + 7 are bytes 4 (l32 % 16) .. + 3 of block l32 / 16
-    uint8_t* wdst = row + 66 * (l32 >> 4) + 2 + 4 * (l32 & 15);
-    *reinterpret_cast<uint16_t*>(wdst) = (uint16_t)lo;
-    *reinterpret_cast<uint16_t*>(wdst + 2) = (uint16_t)hi;
+    tq4_store_codes(row, l32, lo, hi);
 
     float pv[8], pc[8];
 #pragma unroll
@@ -250,6 +331,46 @@ __device__ __forceinline__ void tq4_encode_row(float (&v)[8], int lane, uint8_t*
         pc[j] = c[j] * c[j];
     }
     const float vc_dot = row_sum_of_groups(group32_sums(pv, lane), lane);
+    const float c_sq = row_sum_of_groups(group32_sums(pc, lane), lane);
+    if ((l32 & 15) == 0) {
+        const float d = (c_sq > 1e-10f) ? (vc_dot / c_sq) : 0.0f;
+        *reinterpret_cast<uint16_t*>(row + 66 * (l32 >> 4)) = F16::from_f32(d);
+    }
+}
+// The same bytes at 55 instructions less: the transform's shorter form, whose values y are 16 v, some of them negated.  Powers of two and
+// signs go through products and sums unchanged while nothing is infinite and nothing that counts is subnormal; rows for which
+// that is not so (by their sum of squares) take the exact form, all rows of a wave together.
+__device__ __forceinline__ void tq4_encode_row(const float (&x)[8], int lane, const Tq4Lane& tab, uint8_t* row) {
+    const int l32 = lane & 31;
+    float v[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = x[j];
+    wht256_times16_flipped(v, lane);
+
+    float p[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) p[j] = v[j] * v[j];
+    const float s_sq256 = row_sum_of_groups(group32_sums(p, lane), lane);
+    if (__builtin_expect(__ballot(!(s_sq256 >= 1e-15f && s_sq256 <= 3.402823466e38f)) != 0ull, 0)) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = x[j];
+        tq4_encode_row_exact(v, lane, tab, row);
+        return;
+    }
+    const float inv_norm = 0.7071067811865475f * rsqrt_rn_normal(s_sq256 * 0.00390625f);
+
+    float c[8];
+    uint32_t lo, hi;
+    tq4_codes(v, inv_norm * tab.scale, tab, lo, hi, c);
+    tq4_store_codes(row, l32, lo, hi);
+
+    float pv[8], pc[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        pv[j] = v[j] * c[j];
+        pc[j] = c[j] * c[j];
+    }
+    const float vc_dot = row_sum_of_groups(group32_sums<true>(pv, lane) * tab.scale, lane);
     const float c_sq = row_sum_of_groups(group32_sums(pc, lane), lane);
     if ((l32 & 15) == 0) {
         const float d = (c_sq > 1e-10f) ? (vc_dot / c_sq) : 0.0f;
@@ -270,9 +391,8 @@ __device__ __forceinline__ float block128_sum(const float (&p)[8], int lane) {
     return t + lane_xor<4>(t, lane);
 }
 
-__device__ __forceinline__ void tq4_encode_row_plain(const float (&v)[8], int lane, uint8_t* row) {
+__device__ __forceinline__ void tq4_encode_row_plain(const float (&v)[8], int lane, const Tq4Lane& tab, uint8_t* row) {
     const int l32 = lane & 31;
-    const Tq4Tables tab = tq4_tables(lane);
     float p[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) p[j] = v[j] * v[j];
@@ -282,9 +402,7 @@ __device__ __forceinline__ void tq4_encode_row_plain(const float (&v)[8], int la
     uint32_t lo, hi;
     tq4_codes(v, inv_norm, tab, lo, hi, c);
     // ("q = b + 1 for the last boundary b below u" over ascending boundaries = the number of boundaries below u)
-    uint8_t* wdst = row + 66 * (l32 >> 4) + 2 + 4 * (l32 & 15);
-    *reinterpret_cast<uint16_t*>(wdst) = (uint16_t)lo;
-    *reinterpret_cast<uint16_t*>(wdst + 2) = (uint16_t)hi;
+    tq4_store_codes(row, l32, lo, hi);
 
     float pv[8], pc[8];
 #pragma unroll
@@ -374,22 +492,30 @@ __device__ __forceinline__ void q8_encode_row(const float (&v)[8], int lane, uin
 // (op_kv_cache.cu:36-44,71-99: the same scale and code arithmetic; max is order-free).  The
 // caller guarantees what the append entry points check: head_dim 256, TQ4 with WHT256, 8-bit
 // rows 4-byte aligned.
-__device__ __forceinline__ void encode_store_row(float (&v)[8], int format, int transform, int lane,
+// tab: tq4_lane(lane) for TQ4 rows, requested well before (not looked at otherwise).
+// ROTATED_TQ4: the caller knows that the row is one; a kernel that holds this form alone needs fewer registers.
+template <bool ROTATED_TQ4 = false>
+__device__ __forceinline__ void encode_store_row(float (&v)[8], int format, int transform, int lane, const Tq4Lane& tab,
                                                  uint8_t* row, uint8_t* dst) {
     const int l32 = lane & 31;
-    if (format == WARP34_KV_FORMAT_FP16 || format == WARP34_KV_FORMAT_BF16) {
-        if (dst == nullptr) return;
-        uint16_t* d16 = reinterpret_cast<uint16_t*>(dst) + 8 * l32;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) d16[j] = (format == WARP34_KV_FORMAT_BF16) ? BF16::from_f32(v[j]) : F16::from_f32(v[j]);
-        return;
-    }
     int n_dwords = 33;
-    if (format == WARP34_KV_FORMAT_TQ4) {
-        if (transform == WARP34_KV_TRANSFORM_RADEMACHER_WHT256) {
-            tq4_encode_row(v, lane, row);
+    if constexpr (!ROTATED_TQ4) {
+        if (format == WARP34_KV_FORMAT_FP16 || format == WARP34_KV_FORMAT_BF16) {
+            if (dst == nullptr) return;
+            uint16_t* d16 = reinterpret_cast<uint16_t*>(dst) + 8 * l32;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) d16[j] = (format == WARP34_KV_FORMAT_BF16) ? BF16::from_f32(v[j]) : F16::from_f32(v[j]);
+            return;
+        }
+    }
+    if (ROTATED_TQ4 || format == WARP34_KV_FORMAT_TQ4) {
+        if (ROTATED_TQ4 || transform == WARP34_KV_TRANSFORM_RADEMACHER_WHT256) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                v[j] = __uint_as_float(__float_as_uint(v[j]) ^ ((j & 1 ? tab.sign[j >> 1] : tab.sign[j >> 1] << 16) & 0x80000000u));
+            tq4_encode_row(v, lane, tab, row);
         } else {
-            tq4_encode_row_plain(v, lane, row);
+            tq4_encode_row_plain(v, lane, tab, row);
         }
     } else {
         if (transform == WARP34_KV_TRANSFORM_RADEMACHER_WHT256) sign_wht256(v, lane);

@@ -81,6 +81,9 @@ __global__ __launch_bounds__(256) void qk_norm_rope_kernel(const NormRopeParams 
     uint16_t* src = row_base + (size_t)(is_v_half ? P.q_heads + P.kv_heads + kv_head : head) * dim;
     const uint16_t* w = is_q ? P.qw : P.kw;
 
+    Tq4Lane tab{};
+    if (to_cache && P.L.k_format == WARP34_KV_FORMAT_TQ4) tab = tq4_lane(lane);  // (used by the row encoder)
+
     // sum of squares, element c = l32 + 32 k in register k (op_dflash2.cu:362-380)
     float raw[8], sq[8];
 #pragma unroll
@@ -153,7 +156,7 @@ __global__ __launch_bounds__(256) void qk_norm_rope_kernel(const NormRopeParams 
 #pragma unroll
             for (int j = 0; j < 8; ++j) v[j] = is_v_half ? raw[j] : (j < 4 ? lo[j & 3] : hi[j & 3]);
             strided_to_consecutive(v, lane, xpose_lds[wave][half_id]);
-            encode_store_row(v, format, transform, lane, row_lds, dst);
+            encode_store_row(v, format, transform, lane, tab, row_lds, dst);
         }
         return;
     }
