@@ -164,3 +164,41 @@ def test_argument_validation():
         assert rc == inval
     gk, gv = dpool.download()
     assert not gk.any() and not gv.any()
+
+
+@pytest.mark.parametrize("dim,q_heads,kv_heads,rows", [(128, 16, 4, 64), (128, 3, 1, 5), (96, 4, 2, 9), (64, 2, 2, 3)])
+def test_bf16_pages_at_smaller_head_sizes(dim, q_heads, kv_heads, rows):
+    """The fused write to BF16 pages: rotated K rows and V rows in the pages, Q in its buffer, the packed rows as they were."""
+    import gpu_harness as G
+
+    qkv, qw, kw, pos, table = _case(rows, 15, dim, q_heads, kv_heads)
+    pos[rows // 2] = -1
+    slots = np.random.default_rng(16).permutation(6 * 16)[:rows].astype(np.int32)
+    slots[0] = -1  # this row's K is rotated in place
+    want, want_q = oracle.qk_norm_rope_bf16(qkv.copy(), pos, qw, kw, table, q_heads, kv_heads, dim, 1e-6,
+                                            q_out=np.full((rows, q_heads * dim), 0x7E7E, np.uint16))
+    pool = oracle.HostPool(6, kv_heads, dim, 16, FMT_BF16, XF_IDENTITY)
+    dpool = G.DevPool(pool)
+    rc, got, got_q = _dev_call("warp34_dflash_qk_norm_rope_kv_write_bf16_f32_table", qkv, pos, qw, kw, table, q_heads, kv_heads, dim,
+                               1e-6, q_out=np.full((rows, q_heads * dim), 0x7E7E, np.uint16), dpool=dpool, slots=slots)
+    assert rc == 0 and got_q.tobytes() == want_q.tobytes()
+    k_cols = slice(q_heads * dim, (q_heads + kv_heads) * dim)
+    expect = qkv.copy()
+    expect[0, k_cols] = want[0, k_cols]
+    assert got.tobytes() == expect.tobytes()
+    k_page, v_page = (x.view(np.uint16).reshape(6, kv_heads, 16, dim) for x in (pool.k, pool.v))
+    for r in range(1, rows):
+        if r != rows // 2:
+            k_page[slots[r] // 16, :, slots[r] % 16] = want[r, k_cols].reshape(kv_heads, dim)
+            v_page[slots[r] // 16, :, slots[r] % 16] = qkv[r, (q_heads + kv_heads) * dim:].reshape(kv_heads, dim)
+    gk, gv = dpool.download()
+    assert gk.tobytes() == pool.k.tobytes() and gv.tobytes() == pool.v.tobytes()
+
+
+def test_more_items_than_the_float_quotient_divides():
+    """Rows of many small heads: items on both sides of 2^21."""
+    dim, q_heads, kv_heads, rows = 2, 128, 64, 33000
+    qkv, qw, kw, pos, table = _case(rows, 17, dim, q_heads, kv_heads)
+    want, _ = oracle.qk_norm_rope_bf16(qkv.copy(), pos, qw, kw, table, q_heads, kv_heads, dim, 1e-6)
+    rc, got, _ = _dev_call("warp34_dflash_qk_norm_rope_bf16_f32_table", qkv, pos, qw, kw, table, q_heads, kv_heads, dim, 1e-6)
+    assert rc == 0 and got.tobytes() == want.tobytes()

@@ -20,49 +20,58 @@
 namespace w34 {
 
 struct NormRopeParams {
-    uint16_t* qkv;         // [rows, (q_heads + 2 kv_heads) * dim] bf16
     uint16_t* q_out;       // [rows, q_heads * dim] or null (Q in place)
-    const int32_t* positions;
-    const uint16_t* qw;
-    const uint16_t* kw;
     const void* table;     // [table_rows, dim]: cos (dim/2) | sin (dim/2)
-    const int32_t* write_slot_mapping;  // null: no cache write
     warp34_kv_layer_layout L;
-    int rows, q_heads, kv_heads, dim, table_rows;
+    int table_rows;
     float eps;
 };
 
-// D256: head size 256 known at compile time (no bounds tests, the second pass reuses the
-// values of the first instead of loading them again).
-template <bool TABLE_F32, bool D256>
-__global__ __launch_bounds__(256) void qk_norm_rope_kernel(const NormRopeParams P) {
-    __shared__ __align__(8) uint8_t rows_lds[4][2][272];
-    __shared__ __align__(16) float xpose_lds[4][2][256];  // register layout of the rotation -> the encoder's
-    const int wave = (int)(threadIdx.x >> 6);
+// A call over a few rows is a chain of memory round trips: the leading arguments are in scalar registers when a wave starts, so
+// position, slot, row and weights are asked for at once, and the table's row as soon as the position is there (before: arguments,
+// position, row, weights and table, for head sizes other than 256 the row a second time).  us: four draft blocks of sixteen
+// tokens over 16 + 4 heads of 128, with their attention, 24.1 before / 21.7 a layer; 8 192 tokens over 16 + 2 heads of 256 to
+// rotated TQ4 pages 40.8 / 36.2.
+// HD: the head size where it is known at compile time (256 or 128: no bounds tests, the second pass reuses the values of the
+// first), else 0.  PAGES: what the rows may go to besides q_out and the packed rows.
+enum NormRopePages { kBf16Pages, kRotatedTq4Pages, kQuantisedPages };
+template <bool TABLE_F32, int HD, NormRopePages PAGES>
+__global__ __launch_bounds__(256) void qk_norm_rope_kernel(const int32_t* __restrict__ positions, const int32_t* __restrict__ slots,
+                                                           uint16_t* qkv,  // [rows, (q_heads + 2 kv_heads) * dim] bf16
+                                                           const uint16_t* __restrict__ qw, const uint16_t* __restrict__ kw, int rows,
+                                                           int q_heads, int kv_heads, int dim_arg, const NormRopeParams P) {
+    constexpr bool QUANT = PAGES != kBf16Pages;
+    static_assert(!QUANT || HD == 256, "quantised pages: head size 256");
+    __shared__ __align__(8) uint8_t rows_lds[QUANT ? 4 : 1][2][272];
+    __shared__ __align__(16) float xpose_lds[QUANT ? 4 : 1][2][256];  // register layout of the rotation -> the encoder's
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int lane = lane_id();
     const int half_id = lane >> 5;
     const int l32 = lane & 31;
     // Items are ordered KV items of all rows first, then the Q items: the long items (norm +
     // two row encodes) start first and every workgroup holds items of one kind.
-    const int q_items = (P.q_heads + 1) >> 1;
-    const long long item = (long long)blockIdx.x * 4 + wave;
-    const long long n_kv_items = (long long)P.rows * P.kv_heads;
+    const int q_items = (q_heads + 1) >> 1;
     int row, it;
-    if (item < n_kv_items) {
-        row = (int)(item / P.kv_heads);
-        it = q_items + (int)(item - (long long)row * P.kv_heads);
-    } else {
-        const long long qi = item - n_kv_items;
-        row = q_items > 0 ? (int)(qi / q_items) : P.rows;
-        it = q_items > 0 ? (int)(qi - (long long)row * q_items) : 0;
+    {
+        const long long n_kv_items = (long long)rows * kv_heads, item = (long long)blockIdx.x * 4 + wave;
+        const bool kv = item < n_kv_items;
+        const long long n = kv ? item : item - n_kv_items;
+        const int per_row = kv ? kv_heads : q_items;
+        if (n < (1 << 21) && per_row > 0) {  // (uniform: exact by the float quotient and one correction)
+            row = __builtin_amdgcn_readfirstlane((int)((float)(int)n * __builtin_amdgcn_rcpf((float)per_row)));
+            const int r = (int)n - row * per_row;
+            row += r >= per_row ? 1 : r < 0 ? -1 : 0;
+        } else {
+            row = per_row > 0 ? (int)(n / per_row) : rows;
+        }
+        if (row >= rows) return;
+        it = (int)(n - (long long)row * per_row) + (kv ? q_items : 0);
     }
-    if (row >= P.rows) return;
-    const int pos = P.positions[row];
-    if (pos < 0 || pos >= P.table_rows) return;  // op_dflash2.cu:356
+    const int pos = positions[row];
 
-    const int dim = D256 ? 256 : P.dim, half = dim >> 1;
-    const size_t row_elems = (size_t)(P.q_heads + 2 * P.kv_heads) * dim;
-    uint16_t* row_base = P.qkv + (size_t)row * row_elems;
+    const int dim = HD ? HD : dim_arg, half = dim >> 1;
+    const size_t row_elems = (size_t)(q_heads + 2 * kv_heads) * dim;
+    uint16_t* row_base = qkv + (size_t)row * row_elems;
 
     // Both halves of the wave run the same instruction stream (the cross-lane steps want the
     // whole wave): the half without a head of its own (the V half of a KV item, the second half
@@ -70,26 +79,61 @@ __global__ __launch_bounds__(256) void qk_norm_rope_kernel(const NormRopeParams 
     const bool is_q = it < q_items;
     const bool is_v_half = !is_q && half_id == 1;
     const int kv_head = is_q ? 0 : it - q_items;
-    int head = is_q ? 2 * it + half_id : P.q_heads + kv_head;
-    const bool has_head = is_q ? head < P.q_heads : !is_v_half;
-    if (is_q && head >= P.q_heads) head = P.q_heads - 1;
-    const int slot = (!is_q && P.write_slot_mapping != nullptr) ? P.write_slot_mapping[row] : -1;
-    const bool to_cache = slot >= 0;  // wave-uniform
-    uint8_t* row_lds = rows_lds[wave][half_id];
+    int head = is_q ? 2 * it + half_id : q_heads + kv_head;
+    const bool has_head = is_q ? head < q_heads : !is_v_half;
+    if (is_q && head >= q_heads) head = q_heads - 1;
 
     // V half: its "head" is the V row of the kv head (read-only)
-    uint16_t* src = row_base + (size_t)(is_v_half ? P.q_heads + P.kv_heads + kv_head : head) * dim;
-    const uint16_t* w = is_q ? P.qw : P.kw;
-
-    Tq4Lane tab{};
-    if (to_cache && P.L.k_format == WARP34_KV_FORMAT_TQ4) tab = tq4_lane(lane);  // (used by the row encoder)
+    uint16_t* src = row_base + (size_t)(is_v_half ? q_heads + kv_heads + kv_head : head) * dim;
+    const uint16_t* w = is_q ? qw : kw;
 
     // sum of squares, element c = l32 + 32 k in register k (op_dflash2.cu:362-380)
-    float raw[8], sq[8];
+    constexpr int kPairs = HD ? HD / 64 : 4;  // pairs (c, half + c) of a lane
+    uint16_t raw16[8], w16[2 * kPairs];
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
         const int c = l32 + 32 * k;
-        raw[k] = (D256 || c < dim) ? BF16::to_f32(src[c]) : 0.0f;
+        raw16[k] = (HD ? c < HD : c < dim) ? src[c] : (uint16_t)0;
+    }
+#pragma unroll
+    for (int k = 0; k < kPairs; ++k) {
+        const int c = l32 + 32 * k;
+        w16[k] = w16[kPairs + k] = 0;
+        if (HD || c < half) {
+            w16[k] = w[c];
+            w16[kPairs + k] = w[half + c];
+        }
+    }
+    const int slot = (!is_q && slots != nullptr) ? slots[row] : -1;
+    // (the compiler would load these only where they are used, behind the checks)
+    asm volatile("" ::"s"(pos), "s"(P.table), "s"(P.table_rows), "s"(P.q_out), "s"(P.L.k_base), "s"(P.L.v_base), "s"(P.L.k_page_stride_bytes),
+                 "s"(P.L.k_head_stride_bytes), "s"(P.L.k_token_stride_bytes), "s"(P.L.block_size));
+    const bool to_cache = slot >= 0;  // wave-uniform
+    if (pos < 0 || pos >= P.table_rows) return;  // op_dflash2.cu:356
+    float cosine[kPairs], sine[kPairs];
+#pragma unroll
+    for (int k = 0; k < kPairs; ++k) {
+        const int c = l32 + 32 * k;
+        cosine[k] = sine[k] = 0.0f;
+        if (HD || c < half) {
+            if constexpr (TABLE_F32) {
+                const float* t = reinterpret_cast<const float*>(P.table) + (size_t)pos * dim;
+                cosine[k] = t[c];
+                sine[k] = t[half + c];
+            } else {
+                const uint16_t* t = reinterpret_cast<const uint16_t*>(P.table) + (size_t)pos * dim;
+                cosine[k] = BF16::to_f32(t[c]);
+                sine[k] = BF16::to_f32(t[half + c]);
+            }
+        }
+    }
+    Tq4Lane tab{};
+    if (QUANT && to_cache && (PAGES == kRotatedTq4Pages || P.L.k_format == WARP34_KV_FORMAT_TQ4)) tab = tq4_lane(lane);  // (used by the row encoder)
+
+    float raw[8], sq[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        raw[k] = BF16::to_f32(raw16[k]);
         sq[k] = raw[k] * raw[k];
     }
     float s = ((sq[0] + sq[4]) + (sq[2] + sq[6])) + ((sq[1] + sq[5]) + (sq[3] + sq[7]));
@@ -98,27 +142,17 @@ __global__ __launch_bounds__(256) void qk_norm_rope_kernel(const NormRopeParams 
     const float inv = rsqrt_rn(mean);
 
     // rotated values of this lane: out[c] and out[half + c] for c = l32, l32 + 32, ... < half
-    float lo[4], hi[4];
+    float lo[kPairs], hi[kPairs];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
+    for (int k = 0; k < kPairs; ++k) {
         const int c = l32 + 32 * k;
         lo[k] = hi[k] = 0.0f;
-        if (D256 || c < half) {
-            const float x_lo = D256 ? raw[k] : BF16::to_f32(src[c]);
-            const float x_hi = D256 ? raw[k + 4] : BF16::to_f32(src[half + c]);
-            const float a = BF16::to_f32(BF16::from_f32(x_lo * inv * BF16::to_f32(w[c])));
-            const float b = BF16::to_f32(BF16::from_f32(x_hi * inv * BF16::to_f32(w[half + c])));
-            float cosine, sine;
-            if constexpr (TABLE_F32) {
-                const float* t = reinterpret_cast<const float*>(P.table) + (size_t)pos * dim;
-                cosine = t[c];
-                sine = t[half + c];
-            } else {
-                const uint16_t* t = reinterpret_cast<const uint16_t*>(P.table) + (size_t)pos * dim;
-                cosine = BF16::to_f32(t[c]);
-                sine = BF16::to_f32(t[half + c]);
-            }
-            const float ac = a * cosine, bs = b * sine, bc = b * cosine, as = a * sine;
+        if (HD || c < half) {
+            const float x_lo = raw[k];  // element l32 + 32 k, of every head size
+            const float x_hi = HD ? raw[(k + kPairs) & 7] : BF16::to_f32(src[half + c]);
+            const float a = BF16::to_f32(BF16::from_f32(x_lo * inv * BF16::to_f32(w16[k])));
+            const float b = BF16::to_f32(BF16::from_f32(x_hi * inv * BF16::to_f32(w16[kPairs + k])));
+            const float ac = a * cosine[k], bs = b * sine[k], bc = b * cosine[k], as = a * sine[k];
             lo[k] = BF16::to_f32(BF16::from_f32(ac - bs));
             hi[k] = BF16::to_f32(BF16::from_f32(bc + as));
         }
@@ -132,23 +166,7 @@ __global__ __launch_bounds__(256) void qk_norm_rope_kernel(const NormRopeParams 
                        (size_t)page * (is_v_half ? P.L.v_page_stride_bytes : P.L.k_page_stride_bytes) +
                        (size_t)kv_head * (is_v_half ? P.L.v_head_stride_bytes : P.L.k_head_stride_bytes) +
                        (size_t)off * (is_v_half ? P.L.v_token_stride_bytes : P.L.k_token_stride_bytes);
-        const int format = is_v_half ? P.L.v_format : P.L.k_format;
-        const int transform = is_v_half ? P.L.v_transform : P.L.k_transform;
-        if (format == WARP34_KV_FORMAT_BF16) {  // both slabs are BF16 (host check)
-            uint16_t* d16 = reinterpret_cast<uint16_t*>(dst);
-            if (is_v_half) {
-                for (int c = l32; c < dim; c += 32) d16[c] = src[c];
-            } else {
-#pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    const int c = l32 + 32 * k;
-                    if (D256 || c < half) {
-                        d16[c] = BF16::from_f32(lo[k]);
-                        d16[half + c] = BF16::from_f32(hi[k]);
-                    }
-                }
-            }
-        } else {
+        if constexpr (QUANT) {
             // Quantised pages: head_dim 256, K and V in the same format and transform (host
             // check), so both halves take the same path through the encoder.  Element
             // l32 + 32 j is lo[j] for j < 4 and hi[j - 4] above.
@@ -156,16 +174,34 @@ __global__ __launch_bounds__(256) void qk_norm_rope_kernel(const NormRopeParams 
 #pragma unroll
             for (int j = 0; j < 8; ++j) v[j] = is_v_half ? raw[j] : (j < 4 ? lo[j & 3] : hi[j & 3]);
             strided_to_consecutive(v, lane, xpose_lds[wave][half_id]);
-            encode_store_row(v, format, transform, lane, tab, row_lds, dst);
+            encode_store_row<PAGES == kRotatedTq4Pages>(v, P.L.k_format, P.L.k_transform, lane, tab, rows_lds[wave][half_id], dst);
+        } else {  // both slabs are BF16 (host check)
+            uint16_t* d16 = reinterpret_cast<uint16_t*>(dst);
+            if (is_v_half) {
+#pragma unroll
+                for (int k = 0; k < 8; ++k) {
+                    const int c = l32 + 32 * k;
+                    if (HD ? c < HD : c < dim) d16[c] = raw16[k];
+                }
+            } else {
+#pragma unroll
+                for (int k = 0; k < kPairs; ++k) {
+                    const int c = l32 + 32 * k;
+                    if (HD || c < half) {
+                        d16[c] = BF16::from_f32(lo[k]);
+                        d16[half + c] = BF16::from_f32(hi[k]);
+                    }
+                }
+            }
         }
         return;
     }
     if (!has_head) return;
-    uint16_t* dst = (is_q && P.q_out != nullptr) ? P.q_out + ((size_t)row * P.q_heads + head) * dim : src;
+    uint16_t* dst = (is_q && P.q_out != nullptr) ? P.q_out + ((size_t)row * q_heads + head) * dim : src;
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
+    for (int k = 0; k < kPairs; ++k) {
         const int c = l32 + 32 * k;
-        if (D256 || c < half) {
+        if (HD || c < half) {
             dst[c] = BF16::from_f32(lo[k]);
             dst[half + c] = BF16::from_f32(hi[k]);
         }
@@ -186,26 +222,26 @@ static int launch_norm_rope(const warp34_exec* ex, void* qkv, void* q_out, const
                             const int32_t* write_slot_mapping, int rows, int q_heads, int kv_heads, int dim,
                             int table_rows, float eps) {
     NormRopeParams P{};
-    P.qkv = (uint16_t*)qkv;
     P.q_out = (uint16_t*)q_out;
-    P.positions = positions;
-    P.qw = (const uint16_t*)qw;
-    P.kw = (const uint16_t*)kw;
     P.table = table;
-    P.write_slot_mapping = write_slot_mapping;
     if (layout != nullptr) P.L = *layout;
-    P.rows = rows;
-    P.q_heads = q_heads;
-    P.kv_heads = kv_heads;
-    P.dim = dim;
     P.table_rows = table_rows;
     P.eps = eps;
     const long long items = (long long)rows * ((q_heads + 1) / 2 + kv_heads);
     const unsigned grid = (unsigned)((items + 3) / 4);
-    if (dim == 256) {
-        hipLaunchKernelGGL((qk_norm_rope_kernel<TABLE_F32, true>), dim3(grid), dim3(256), 0, (hipStream_t)ex->stream, P);
+    const auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), 0, (hipStream_t)ex->stream, positions, write_slot_mapping, (uint16_t*)qkv,
+                           (const uint16_t*)qw, (const uint16_t*)kw, rows, q_heads, kv_heads, dim, P);
+    };
+    if (layout != nullptr && layout->k_format != WARP34_KV_FORMAT_BF16) {
+        const bool rotated_tq4 = layout->k_format == WARP34_KV_FORMAT_TQ4 && layout->k_transform == WARP34_KV_TRANSFORM_RADEMACHER_WHT256;
+        rotated_tq4 ? launch(qk_norm_rope_kernel<TABLE_F32, 256, kRotatedTq4Pages>) : launch(qk_norm_rope_kernel<TABLE_F32, 256, kQuantisedPages>);
+    } else if (dim == 256) {
+        launch(qk_norm_rope_kernel<TABLE_F32, 256, kBf16Pages>);
+    } else if (dim == 128) {
+        launch(qk_norm_rope_kernel<TABLE_F32, 128, kBf16Pages>);
     } else {
-        hipLaunchKernelGGL((qk_norm_rope_kernel<TABLE_F32, false>), dim3(grid), dim3(256), 0, (hipStream_t)ex->stream, P);
+        launch(qk_norm_rope_kernel<TABLE_F32, 0, kBf16Pages>);
     }
     return (int)hipGetLastError();
 }
