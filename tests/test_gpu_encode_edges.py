@@ -68,7 +68,8 @@ def test_rows_at_the_ends_of_the_energy_range(xf):
     _append_equals_oracle(np.stack(rows).astype(np.float32), DT_BF16, xf)
 
 
-@pytest.mark.parametrize("n,qh,kh", [(1, 16, 2), (2, 1, 1), (3, 5, 3), (255, 6, 1), (256, 3, 2), (257, 3, 2), (258, 6, 1)])
+@pytest.mark.parametrize("n,qh,kh", [(1, 16, 2), (2, 1, 1), (3, 5, 3), (255, 6, 1), (256, 3, 2), (257, 3, 2), (258, 6, 1),
+                                     (512, 3, 2), (513, 6, 1)])
 @pytest.mark.parametrize("fmt", [FMT_TQ4, FMT_Q8_0])
 def test_producer_on_both_sides_of_the_token_limit(n, qh, kh, fmt):
     import gpu_harness as G

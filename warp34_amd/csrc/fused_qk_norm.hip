@@ -33,9 +33,9 @@ namespace w34 {
 constexpr int kFqMaxPairs = 128;  // rotary_dim / 2
 // Up to this many tokens a token's items go to several workgroups, one item per wave (a wave's items in turn are
 // a chain of memory round trips, and the K / V items came last).  us, one workgroup per token / spread, 16 q + 2 kv heads, TQ4:
-// 1 token 7.0 / 5.0, 64 7.5 / 5.5, 256 8.5 / 6.8, 512 10.1 / 9.9, 1 024 12.2 / 15.0; 32 + 4 heads: 1 token 9.0 / 5.3, 256 11.6 / 10.0,
-// 512 17.1 / 16.3, 1 024 18.2 / 23.0; Q8_0 alike.
-constexpr int kFqSpreadTokens = 256;
+// 64 tokens 5.9 / 5.0, 256 6.5 / 5.0, 384 7.7 / 5.8, 512 8.2 / 6.9, 768 9.1 / 8.9, 1 024 10.0 / 10.5; Q8_0 512 7.6 / 6.7, 768 8.4 / 8.6;
+// 32 + 4 heads: 384 10.7 / 9.0, 512 11.1 / 10.3, 768 13.2 / 13.7.
+constexpr int kFqSpreadTokens = 512;
 
 struct FusedQkParams {
     const uint16_t* q_gate_in;

@@ -2816,28 +2816,19 @@ static int launch_qsa_sparse(const warp34_exec* ex, const void* q, const void* g
     if (gate != nullptr && (((uintptr_t)gate) & 7u) != 0) return (int)hipErrorNotSupported;
     QsaParams P{};
     P.L = *layout;
-    P.q = (const uint16_t*)q;
     P.gate = (const uint16_t*)gate;
     P.out = (uint16_t*)out;
-    P.sel_phys = selected_phys_blocks;
-    P.sel_log = selected_logical_blocks;
-    P.num_sel = num_selected_blocks;
-    P.seq_pos = token_seq_pos;
     P.valid_token_mask = valid_token_mask;
-    P.num_tokens = num_tokens;
-    P.num_q_heads = local_q_heads;
-    P.gqa = local_q_heads / layout->local_kv_heads;
-    int q_group = P.gqa;
+    const int gqa = local_q_heads / layout->local_kv_heads;
+    int q_group = gqa;
     if (q_group > 16) {
         for (int d = 16; d >= 1; --d)
-            if (P.gqa % d == 0) {
+            if (gqa % d == 0) {
                 q_group = d;
                 break;
             }
     }
-    P.q_group = q_group;
-    P.q_subgroups = P.gqa / q_group;
-    P.select_k = select_k_blocks;
+    const int q_subgroups = gqa / q_group;
     P.groups_per_page = layout->block_size / 4;
     P.gpp_shift = -1;
     for (int k = 0; k < 30; ++k)
@@ -2847,7 +2838,7 @@ static int launch_qsa_sparse(const warp34_exec* ex, const void* q, const void* g
     P.out_scale = form == kFormTq4 ? kLutInvGain : 1.0f;
     P.rot_q = layout->k_transform == WARP34_KV_TRANSFORM_RADEMACHER_WHT256 ? 1 : 0;
     P.rot_out = layout->v_transform == WARP34_KV_TRANSFORM_RADEMACHER_WHT256 ? 1 : 0;
-    const int kv_subs = layout->local_kv_heads * P.q_subgroups;
+    const int kv_subs = layout->local_kv_heads * q_subgroups;
     // work items of a token: 32-key units (TQ4) or 16-key halves (row formats), one per wave and turn
     const int max_units = form == kFormTq4 ? (select_k_blocks + 7) / 8 : (select_k_blocks + 3) / 4;
     long long want = 256ll / ((long long)num_tokens * kv_subs);
@@ -2857,27 +2848,30 @@ static int launch_qsa_sparse(const warp34_exec* ex, const void* q, const void* g
     if (want < 1) want = 1;
     const size_t rows = (size_t)num_tokens * local_q_heads;
     const size_t need = rows * (size_t)want * (kHeadDim + 4) * sizeof(float);
-    P.n_splits = (want > 1 && ex->scratch_ptr != 0 && (ex->scratch_ptr & 15u) == 0u && ex->scratch_size >= need)
-                     ? (int)want
-                     : 1;
-    if (P.n_splits > 1) {
+    const int n_splits = (want > 1 && ex->scratch_ptr != 0 && (ex->scratch_ptr & 15u) == 0u && ex->scratch_size >= need) ? (int)want : 1;
+    if (n_splits > 1) {
         P.part_acc = reinterpret_cast<float*>((uintptr_t)ex->scratch_ptr);
-        P.part_ml = P.part_acc + rows * P.n_splits * kHeadDim;
+        P.part_ml = P.part_acc + rows * n_splits * kHeadDim;
     }
+    const uint32_t shape = QsaShape::pack(q_group, n_splits, q_subgroups);
+    const int guess = (max_units + n_splits - 1) / n_splits;
     hipStream_t stream = (hipStream_t)ex->stream;
-    const dim3 grid((unsigned)num_tokens, (unsigned)kv_subs, (unsigned)P.n_splits);
+    const dim3 grid((unsigned)num_tokens, (unsigned)kv_subs, (unsigned)n_splits);
     int rc;
     auto launch_rows_form = [&](auto kernel) {
         const int smem = kv16_smem_bytes(1);
         int r = ensure_dynamic_lds(kernel, smem);
         if (r) return r;
-        hipLaunchKernelGGL(kernel, grid, dim3(kKv16Waves * 64), smem, stream, P);
+        hipLaunchKernelGGL(kernel, grid, dim3(kKv16Waves * 64), smem, stream, selected_phys_blocks, selected_logical_blocks,
+                           num_selected_blocks, token_seq_pos, (const uint16_t*)q, select_k_blocks, guess, shape, local_q_heads, P);
         return (int)hipGetLastError();
     };
     if (form == kFormTq4) {
         rc = ensure_dynamic_lds(qsa_sparse_tq4_kernel, kQsaSmem, true);
         if (rc) return rc;
-        hipLaunchKernelGGL(qsa_sparse_tq4_kernel, grid, dim3(kQsaWaves * 64), kQsaSmem, stream, P);
+        hipLaunchKernelGGL(qsa_sparse_tq4_kernel, grid, dim3(kQsaWaves * 64), kQsaSmem, stream, selected_phys_blocks,
+                           selected_logical_blocks, num_selected_blocks, token_seq_pos, (const uint16_t*)q, select_k_blocks, guess, shape,
+                           local_q_heads, P);
         rc = (int)hipGetLastError();
     } else if (form == WARP34_KV_FORMAT_FP16) {
         rc = launch_rows_form(qsa_sparse_rows_kernel<WARP34_KV_FORMAT_FP16>);
@@ -2889,8 +2883,9 @@ static int launch_qsa_sparse(const warp34_exec* ex, const void* q, const void* g
                        : launch_rows_form(qsa_sparse_rows_kernel<WARP34_KV_FORMAT_Q8_0, false>);
     }
     if (rc) return rc;
-    if (P.n_splits > 1) {
-        hipLaunchKernelGGL(qsa_sparse_merge_kernel, dim3((unsigned)rows), dim3(64), 0, stream, P);
+    if (n_splits > 1) {
+        hipLaunchKernelGGL(qsa_sparse_merge_kernel, dim3((unsigned)rows), dim3(64), 0, stream, P.part_ml, P.part_acc, P.gate, P.out, n_splits,
+                           P.rot_out, P.had64, P.out_scale);
         rc = (int)hipGetLastError();
     }
     return rc;

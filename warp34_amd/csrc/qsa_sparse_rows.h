@@ -13,7 +13,7 @@ namespace w34 {
 // VRES (8-bit value rows stored rotated): a second operand with the rounding residuals of
 // fp16(d * code) and a second MFMA per P V tile, as in rows_tile.
 template <int KVF, bool VRES = false>
-__global__ __launch_bounds__(kKv16Waves * 64, 1) void qsa_sparse_rows_kernel(const QsaParams P) {
+__global__ __launch_bounds__(kKv16Waves * 64, 1) void qsa_sparse_rows_kernel(QSA_LEAD, const QsaParams P) {
     static_assert(!VRES || KVF == WARP34_KV_FORMAT_FP8_E4M3 || KVF == WARP34_KV_FORMAT_Q8_0, "residual operand: 8-bit rows");
     constexpr bool K8 = KVF == WARP34_KV_FORMAT_FP8_E4M3 || KVF == WARP34_KV_FORMAT_Q8_0;
     constexpr bool FP8 = KVF == WARP34_KV_FORMAT_FP8_E4M3;
@@ -32,32 +32,34 @@ __global__ __launch_bounds__(kKv16Waves * 64, 1) void qsa_sparse_rows_kernel(con
     const int tok = (int)blockIdx.x;
     const int kv_sub = (int)blockIdx.y;
     const int split = (int)blockIdx.z;
-    const int kv_head = fast_div(kv_sub, P.q_subgroups);
-    const int q_head_base = kv_head * P.gqa + (kv_sub - kv_head * P.q_subgroups) * P.q_group;
-    const bool col_ok = n < P.q_group;
+    const QsaShape S(shape);
+    const int kv_head = fast_div(kv_sub, S.q_subgroups);
+    const int q_head_base = kv_sub * S.q_group;  // (a kv head's q heads are its subgroups')
+    const bool col_ok = n < S.q_group;
 
     // ---- this token's list: counts and the entries of this wave's first half together (the first
     // half is guessed from the list's capacity and fetched again when the guess is wrong) ----
-    const int32_t* tok_phys = P.sel_phys + (size_t)tok * P.select_k;
-    const int32_t* tok_log = P.sel_log + (size_t)tok * P.select_k;
-    const int hpc_guess = fast_div(((P.select_k + 3) >> 2) + P.n_splits - 1, P.n_splits);
-    const int half_guess = split * hpc_guess + wave;
+    const int32_t* tok_phys = sel_phys + (size_t)tok * select_k;
+    const int32_t* tok_log = sel_log + (size_t)tok * select_k;
+    const int half_guess = split * guess + wave;
     int spec_id = -1, spec_lg = 0;
     {
         const int gi = half_guess * 4 + (lane & 3);
-        if (gi < P.select_k) {
+        if (gi < select_k) {
             spec_id = tok_phys[gi];
             spec_lg = tok_log[gi];
         }
     }
-    int a_live = 1, a_sel = P.num_sel[tok], a_pos = P.seq_pos[tok];
+    const int a_sel = num_sel[tok], a_pos = seq_pos_of[tok];
+    qsa_have_arguments(P);
+    int a_live = 1;
     if (P.valid_token_mask != nullptr) a_live = (int)P.valid_token_mask[tok];
 
     // ---- query rows in MFMA B layout: lane (n, b) holds Q[column n][32 m + 8 b .. + 7] ----
     u4 bq[8];
     const bool rot_q = K8 && P.rot_q != 0;  // workgroup-uniform
     if (!rot_q) {
-        const uint16_t* qrow = P.q + ((size_t)tok * P.num_q_heads + (size_t)(q_head_base + min(n, P.q_group - 1))) * kHeadDim;
+        const uint16_t* qrow = q_in + ((size_t)tok * num_q_heads + (size_t)(q_head_base + min(n, S.q_group - 1))) * kHeadDim;
 #pragma unroll
         for (int m = 0; m < 8; ++m) bq[m] = *reinterpret_cast<const u4*>(qrow + 32 * m + 8 * b);
     } else {
@@ -66,7 +68,7 @@ __global__ __launch_bounds__(kKv16Waves * 64, 1) void qsa_sparse_rows_kernel(con
         constexpr int kQStride = 264;  // halves
         _Float16* qlds = reinterpret_cast<_Float16*>(smem);
         for (int col = wave; col < 16; col += kWaves) {
-            const uint16_t* qrow = P.q + ((size_t)tok * P.num_q_heads + (size_t)(q_head_base + min(col, P.q_group - 1))) * kHeadDim;
+            const uint16_t* qrow = q_in + ((size_t)tok * num_q_heads + (size_t)(q_head_base + min(col, S.q_group - 1))) * kHeadDim;
             const uint2 raw = *reinterpret_cast<const uint2*>(qrow + 4 * lane);
             float v[4] = {F16::to_f32((uint16_t)(raw.x & 0xFFFFu)), F16::to_f32((uint16_t)(raw.x >> 16)),
                           F16::to_f32((uint16_t)(raw.y & 0xFFFFu)), F16::to_f32((uint16_t)(raw.y >> 16))};
@@ -89,11 +91,11 @@ __global__ __launch_bounds__(kKv16Waves * 64, 1) void qsa_sparse_rows_kernel(con
     }
 
     int n_sel = __builtin_amdgcn_readfirstlane(a_live) != 0 ? __builtin_amdgcn_readfirstlane(a_sel) : 0;
-    if (n_sel > P.select_k) n_sel = P.select_k;
+    if (n_sel > select_k) n_sel = select_k;
     if (n_sel < 0) n_sel = 0;
     const int seq_pos = __builtin_amdgcn_readfirstlane(a_pos);
     const int n_halves = (n_sel + 3) >> 2;
-    const int hpc = fast_div(n_halves + P.n_splits - 1, P.n_splits);
+    const int hpc = fast_div(n_halves + S.n_splits - 1, S.n_splits);
     const int ch_first = split * hpc;
     int ch_end = ch_first + hpc;
     if (ch_end > n_halves) ch_end = n_halves;
@@ -409,10 +411,10 @@ __global__ __launch_bounds__(kKv16Waves * 64, 1) void qsa_sparse_rows_kernel(con
         const int h = e >> 7, r = (e >> 3) & 15, j = e & 7;
         merge_slot[k] = ((h * 8 + j) * 4 + (r >> 2)) * 4 + (r & 3);
     }
-    for (int col = wave; col < P.q_group; col += kWaves) {
-        const size_t row = (size_t)tok * P.num_q_heads + (size_t)(q_head_base + col);
+    for (int col = wave; col < S.q_group; col += kWaves) {
+        const size_t row = (size_t)tok * num_q_heads + (size_t)(q_head_base + col);
         uint2 g = {0u, 0u};
-        if (P.n_splits == 1) g = qsa_load_gate(P.gate, row, lane);
+        if (S.n_splits == 1) g = qsa_load_gate(P.gate, row, lane);
         float v[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int w = 0; w < kWaves; ++w) {
@@ -422,8 +424,8 @@ __global__ __launch_bounds__(kKv16Waves * 64, 1) void qsa_sparse_rows_kernel(con
         }
         const float m_col = mltot[col * 2 + 0];
         const float l_col = mltot[col * 2 + 1];
-        if (P.n_splits > 1) {
-            const size_t prow = row * P.n_splits + split;
+        if (S.n_splits > 1) {
+            const size_t prow = row * S.n_splits + split;
             *reinterpret_cast<f4*>(P.part_acc + prow * kHeadDim + 4 * lane) = f4{v[0], v[1], v[2], v[3]};
             if (lane == 0) *reinterpret_cast<f4*>(P.part_ml + prow * 4) = f4{m_col, l_col, 0.f, 0.f};
         } else {

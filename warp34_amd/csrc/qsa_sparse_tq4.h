@@ -36,17 +36,12 @@ constexpr int kQsaMaxSplits = 16;
 
 struct QsaParams {
     warp34_kv_layer_layout L;
-    const uint16_t* q;
     const uint16_t* gate;  // may be null
     uint16_t* out;
-    const int32_t* sel_phys;
-    const int32_t* sel_log;
-    const int32_t* num_sel;
-    const int32_t* seq_pos;
     const uint8_t* valid_token_mask;  // may be null
     float* part_acc;  // [rows][n_splits][256]
     float* part_ml;   // [rows][n_splits][4]: m, l, -, -
-    int num_tokens, num_q_heads, gqa, q_group, q_subgroups, select_k, n_splits, had64;
+    int had64;
     int groups_per_page;
     int gpp_shift;  // log2(groups_per_page), or -1 when it is not a power of two
     float sm_scale;
@@ -54,6 +49,25 @@ struct QsaParams {
     int rot_q;        // row-format form: K rows are stored rotated, rotate the query rows
     int rot_out;      // V rows are stored rotated: rotate the finished row back
 };
+
+// Leading arguments of the two attention kernels: in scalar registers when a wave starts, so the list, its counts and the query rows are
+// asked for at once (behind the argument block: 16 tokens of 513 groups, TQ4, 16.5 us a call instead of 15.8).
+#define QSA_LEAD                                                                                                                  \
+    const int32_t *__restrict__ sel_phys, const int32_t *__restrict__ sel_log, const int32_t *__restrict__ num_sel,               \
+        const int32_t *__restrict__ seq_pos_of, const uint16_t *__restrict__ q_in, int select_k, int guess, uint32_t shape, int num_q_heads
+// shape: q_group (5 bits), splits (5 bits), q_subgroups.  guess: units (halves) of a split of a full list.
+struct QsaShape {
+    int q_group, n_splits, q_subgroups;
+    __host__ static uint32_t pack(int q_group, int n_splits, int q_subgroups) { return (uint32_t)(q_group | n_splits << 5 | q_subgroups << 10); }
+    __device__ explicit QsaShape(uint32_t x) : q_group((int)(x & 31u)), n_splits((int)(x >> 5 & 31u)), q_subgroups((int)(x >> 10)) {}
+};
+static_assert(kQsaMaxSplits < 32, "splits in five bits");
+// (the compiler would load the rest of the arguments where they are used; here they are on their way beside the list)
+__device__ __forceinline__ void qsa_have_arguments(const QsaParams& P) {
+    asm volatile("" ::"s"(P.L.k_base), "s"(P.L.v_base), "s"(P.L.k_page_stride_bytes), "s"(P.L.v_page_stride_bytes), "s"(P.L.k_head_stride_bytes),
+                 "s"(P.L.v_head_stride_bytes), "s"(P.L.k_token_stride_bytes), "s"(P.L.v_token_stride_bytes), "s"(P.valid_token_mask),
+                 "s"(P.groups_per_page), "s"(P.gpp_shift), "s"(P.sm_scale));
+}
 
 // The end of a row: v = element 4 lane + k of the normalised sum in the rotated domain.
 __device__ __forceinline__ uint2 qsa_load_gate(const uint16_t* gate, size_t row, int lane) {
@@ -100,7 +114,7 @@ __device__ __forceinline__ void qsa_finish_row(float (&v)[4], int lane, size_t r
     *reinterpret_cast<uint2*>(out + row * kHeadDim + 4 * lane) = o;
 }
 
-__global__ __launch_bounds__(kQsaWaves * 64, 1) void qsa_sparse_tq4_kernel(const QsaParams P) {
+__global__ __launch_bounds__(kQsaWaves * 64, 1) void qsa_sparse_tq4_kernel(QSA_LEAD, const QsaParams P) {
     extern __shared__ __align__(16) uint8_t smem[];
     // lut_read() addresses the table absolutely: the dynamic block starts at LDS address 0 because
     // the kernel has no static LDS (checked on the host before the first launch)
@@ -116,17 +130,17 @@ __global__ __launch_bounds__(kQsaWaves * 64, 1) void qsa_sparse_tq4_kernel(const
     const int tok = (int)blockIdx.x;
     const int kv_sub = (int)blockIdx.y;
     const int split = (int)blockIdx.z;
-    const int kv_head = fast_div(kv_sub, P.q_subgroups);
-    const int q_head_base = kv_head * P.gqa + (kv_sub - kv_head * P.q_subgroups) * P.q_group;
+    const QsaShape S(shape);
+    const int kv_head = fast_div(kv_sub, S.q_subgroups);
+    const int q_head_base = kv_sub * S.q_group;  // (a kv head's q heads are its subgroups')
 
     // ---- this token's list ------------------------------------------------------------------------
     // The counts and the list entries of this wave's first eight units (lane l: group l & 7 of unit l >> 3) are requested
     // together: where the wave's units start is guessed from the list's capacity (exact when the list is full, the
     // common case) and the entries are fetched again when the guess is wrong, so the guess changes the latency only.
-    const int32_t* tok_phys = P.sel_phys + (size_t)tok * P.select_k;
-    const int32_t* tok_log = P.sel_log + (size_t)tok * P.select_k;
-    const int upc_guess = fast_div(((P.select_k + 7) >> 3) + P.n_splits - 1, P.n_splits);
-    const int unit_guess = split * upc_guess + wave;
+    const int32_t* tok_phys = sel_phys + (size_t)tok * select_k;
+    const int32_t* tok_log = sel_log + (size_t)tok * select_k;
+    const int unit_guess = split * guess + wave;
     int list_id = -1, list_lg = 0;
     auto load_list = [&](int first_unit, int end) {
         const int gi = (first_unit + kQsaWaves * (lane >> 3)) * 8 + (lane & 7);
@@ -136,9 +150,8 @@ __global__ __launch_bounds__(kQsaWaves * 64, 1) void qsa_sparse_tq4_kernel(const
             list_lg = tok_log[gi];
         }
     };
-    load_list(unit_guess, P.select_k);
-    int a_live = 1, a_sel = P.num_sel[tok], a_pos = P.seq_pos[tok];  // one vector load each, no scalar-cache trip
-    if (P.valid_token_mask != nullptr) a_live = (int)P.valid_token_mask[tok];
+    load_list(unit_guess, select_k);
+    const int a_sel = num_sel[tok], a_pos = seq_pos_of[tok];
 
     // ---- query rows of this wave's columns (column c = q head q_head_base + c, c < q_group) ----------
     constexpr int kColsPerWave = 16 / kQsaWaves;
@@ -147,19 +160,22 @@ __global__ __launch_bounds__(kQsaWaves * 64, 1) void qsa_sparse_tq4_kernel(const
     for (int c = 0; c < kColsPerWave; ++c) {
         const int col = wave + c * kQsaWaves;
         q_raw[c] = uint2{0u, 0u};
-        if (col < P.q_group) {
-            const uint16_t* qrow = P.q + ((size_t)tok * P.num_q_heads + (size_t)(q_head_base + col)) * kHeadDim;
+        if (col < S.q_group) {
+            const uint16_t* qrow = q_in + ((size_t)tok * num_q_heads + (size_t)(q_head_base + col)) * kHeadDim;
             q_raw[c] = *reinterpret_cast<const uint2*>(qrow + 4 * lane);
         }
     }
+    qsa_have_arguments(P);
+    int a_live = 1;
+    if (P.valid_token_mask != nullptr) a_live = (int)P.valid_token_mask[tok];
     build_pair_table(smem, tid, lane, wave);
 
     int n_sel = __builtin_amdgcn_readfirstlane(a_live) != 0 ? __builtin_amdgcn_readfirstlane(a_sel) : 0;
-    if (n_sel > P.select_k) n_sel = P.select_k;
+    if (n_sel > select_k) n_sel = select_k;
     if (n_sel < 0) n_sel = 0;
     const int seq_pos = __builtin_amdgcn_readfirstlane(a_pos);
     const int n_units = (n_sel + 7) >> 3;
-    const int upc = fast_div(n_units + P.n_splits - 1, P.n_splits);
+    const int upc = fast_div(n_units + S.n_splits - 1, S.n_splits);
     const int cu_first = split * upc;
     int cu_end = cu_first + upc;
     if (cu_end > n_units) cu_end = n_units;
@@ -226,7 +242,7 @@ __global__ __launch_bounds__(kQsaWaves * 64, 1) void qsa_sparse_tq4_kernel(const
         const int col = wave + c * kQsaWaves;
         float qv[4] = {F16::to_f32((uint16_t)(q_raw[c].x & 0xFFFFu)), F16::to_f32((uint16_t)(q_raw[c].x >> 16)),
                        F16::to_f32((uint16_t)(q_raw[c].y & 0xFFFFu)), F16::to_f32((uint16_t)(q_raw[c].y >> 16))};
-        if (col < P.q_group) {  // wave-uniform; dead columns stay zero
+        if (col < S.q_group) {  // wave-uniform; dead columns stay zero
 #pragma unroll
             for (int k = 0; k < 4; ++k) qv[k] = apply_sign(qv[k], 4 * lane + k);
             wht256_wave(qv, lane);
@@ -260,7 +276,7 @@ __global__ __launch_bounds__(kQsaWaves * 64, 1) void qsa_sparse_tq4_kernel(const
     }
 
     const uint32_t lut_lane = (uint32_t)lane << 2;
-    const bool col_ok = n < P.q_group;
+    const bool col_ok = n < S.q_group;
     f4 o_acc[2][8];
     float m_run = kNegBig, l_run = 0.f;
 #pragma unroll
@@ -503,17 +519,17 @@ __global__ __launch_bounds__(kQsaWaves * 64, 1) void qsa_sparse_tq4_kernel(const
     __syncthreads();
 #pragma unroll 1
     for (int half = 0; half < 2; ++half) {
-        if (8 * half >= P.q_group) break;  // the same in every wave
+        if (8 * half >= S.q_group) break;  // the same in every wave
         if (half == 1) {
             __syncthreads();  // the first pass has read the regions
             store_region(1);
             __syncthreads();
         }
         const int col = 8 * half + wave;
-        if (col >= P.q_group) continue;
-        const size_t row = (size_t)tok * P.num_q_heads + (size_t)(q_head_base + col);
+        if (col >= S.q_group) continue;
+        const size_t row = (size_t)tok * num_q_heads + (size_t)(q_head_base + col);
         uint2 g = {0u, 0u};
-        if (P.n_splits == 1) g = qsa_load_gate(P.gate, row, lane);
+        if (S.n_splits == 1) g = qsa_load_gate(P.gate, row, lane);
         float mw[kQsaWaves], lw[kQsaWaves];
 #pragma unroll
         for (int w = 0; w < kQsaWaves; ++w) {
@@ -536,8 +552,8 @@ __global__ __launch_bounds__(kQsaWaves * 64, 1) void qsa_sparse_tq4_kernel(const
         float v[4];
 #pragma unroll
         for (int k = 0; k < 4; ++k) v[k] = tbuf[merge_slot[k]];
-        if (P.n_splits > 1) {
-            const size_t prow = row * P.n_splits + split;
+        if (S.n_splits > 1) {
+            const size_t prow = row * S.n_splits + split;
             *reinterpret_cast<f4*>(P.part_acc + prow * kHeadDim + 4 * lane) = f4{v[0], v[1], v[2], v[3]};
             if (lane == 0) *reinterpret_cast<f4*>(P.part_ml + prow * 4) = f4{m_col, l_col, 0.f, 0.f};
         } else {
@@ -553,20 +569,23 @@ __global__ __launch_bounds__(kQsaWaves * 64, 1) void qsa_sparse_tq4_kernel(const
     }
 }
 
-// One wave per (token, q head) row: lane s holds the record of split s (n_splits <= 16).
-__global__ __launch_bounds__(64) void qsa_sparse_merge_kernel(const QsaParams P) {
+// One wave per (token, q head) row: lane s holds the record of split s (n_splits <= 16).  All arguments are in scalar registers when a
+// wave starts: records, sums and gate are asked for at once.
+__global__ __launch_bounds__(64) void qsa_sparse_merge_kernel(const float* __restrict__ part_ml, const float* __restrict__ part_acc,
+                                                              const uint16_t* __restrict__ gate, uint16_t* __restrict__ out, int n_splits,
+                                                              int rot_out, int had64, float out_scale) {
     const int lane = (int)threadIdx.x;
     const size_t row = (size_t)blockIdx.x;
-    const float* ml = P.part_ml + row * P.n_splits * 4;
-    const float* acc = P.part_acc + row * P.n_splits * kHeadDim;
+    const float* ml = part_ml + row * n_splits * 4;
+    const float* acc = part_acc + row * n_splits * kHeadDim;
     f4 rec = {kNegBig, 0.f, 0.f, 0.f};
-    if (lane < P.n_splits) rec = *reinterpret_cast<const f4*>(ml + 4 * lane);
-    const uint2 g = qsa_load_gate(P.gate, row, lane);
+    if (lane < n_splits) rec = *reinterpret_cast<const f4*>(ml + 4 * lane);
+    const uint2 g = qsa_load_gate(gate, row, lane);
     f4 a[kQsaMaxSplits];
 #pragma unroll
     for (int s = 0; s < kQsaMaxSplits; ++s) {
         a[s] = f4{0.f, 0.f, 0.f, 0.f};
-        if (s < P.n_splits) a[s] = *reinterpret_cast<const f4*>(acc + (size_t)s * kHeadDim + 4 * lane);
+        if (s < n_splits) a[s] = *reinterpret_cast<const f4*>(acc + (size_t)s * kHeadDim + 4 * lane);
     }
     float m_tot = rec[1] > 0.f ? rec[0] : kNegBig;
     m_tot = fmaxf(m_tot, lane_xor<1>(m_tot, lane));
@@ -580,20 +599,20 @@ __global__ __launch_bounds__(64) void qsa_sparse_merge_kernel(const QsaParams P)
     for (int s = 0; s < kQsaMaxSplits; ++s) {
         const float ws = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w_my), s));
         const float ls = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(rec[1]), s));
-        if (s < P.n_splits && ws > 0.f) {  // wave-uniform
+        if (s < n_splits && ws > 0.f) {  // wave-uniform
             l_tot += ls * ws;
 #pragma unroll
             for (int k = 0; k < 4; ++k) v[k] += a[s][k] * ws;
         }
     }
     if (!(l_tot > 0.f)) {  // masked token or no visible key: a row of (positive) zeros
-        *reinterpret_cast<uint2*>(P.out + row * kHeadDim + 4 * lane) = uint2{0u, 0u};
+        *reinterpret_cast<uint2*>(out + row * kHeadDim + 4 * lane) = uint2{0u, 0u};
         return;
     }
-    const float inv = P.out_scale / l_tot;
+    const float inv = out_scale / l_tot;
 #pragma unroll
     for (int k = 0; k < 4; ++k) v[k] *= inv;
-    qsa_finish_row(v, lane, row, P.rot_out != 0, P.gate != nullptr, g, P.had64 != 0, P.out);
+    qsa_finish_row(v, lane, row, rot_out != 0, gate != nullptr, g, had64 != 0, out);
 }
 
 }  // namespace w34
