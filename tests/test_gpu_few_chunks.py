@@ -1,0 +1,40 @@
+"""Contexts of few chunks: shorter chunks, and a merge of one wave per row, against the oracle at the lengths where the number of chunks and
+the form of the merge change; and, with a bound on the length under which the merge of several waves runs, the same bytes."""
+import numpy as np
+import pytest
+
+import oracle
+from cases import make_case
+from oracle import DT_BF16, DT_F16, FMT_BF16, FMT_FP8, FMT_Q8_0, FMT_TQ4
+
+pytestmark = pytest.mark.gpu
+SCRATCH = 64 << 20
+UNIT = 32
+
+
+@pytest.mark.parametrize("fmt,dtype,head_dim", [(FMT_TQ4, DT_F16, 256), (FMT_TQ4, DT_BF16, 256), (FMT_Q8_0, DT_F16, 256),
+                                                (FMT_FP8, DT_BF16, 256), (FMT_BF16, DT_BF16, 128)])
+@pytest.mark.parametrize("units", [8, 9, 32, 33, 64, 65, 96, 128, 129, 200, 257])
+def test_lengths_at_which_the_chunks_change(fmt, dtype, head_dim, units):
+    """One token (rows summed in the order of sixteen waves) and four (of four), a whole last unit and one key in it."""
+    import gpu_harness as G
+
+    q_heads, kv_heads = 16, 2 if head_dim == 256 else 4
+    for q_len, seq in ((1, units * UNIT), (4, (units - 1) * UNIT + 1)):
+        pool, bt, k, v, q, aq, ctx = make_case(fmt, 64, [seq], [q_len], 2300 + units, dtype, kv_heads=kv_heads, q_heads=q_heads,
+                                               head_dim=head_dim)
+        mask = np.ones(q_len, dtype=np.uint8)
+        if q_len > 1:
+            mask[1] = 0
+        hb = oracle.HostBatch(aq, [seq], bt, context_lens_before=ctx, valid_token_mask=mask)
+        want = oracle.paged_attention(pool, hb, q, dtype, q_heads)
+        dpool = G.DevPool(pool)
+        dpool.upload()
+        rc, got, _ = G.dev_attention(dpool, hb, q, dtype, q_heads, scratch_bytes=SCRATCH)
+        assert rc == 0
+        live = mask != 0
+        assert (got[~live] == 0x5500).all()
+        G.assert_close(got[live], dtype, want[live], what="fmt=%d seq=%d q=%d" % (fmt, seq, q_len),
+                       scale=G.channel_scale(v, dtype, hb, q_heads)[live])
+        rc, wide, _ = G.dev_attention(dpool, hb, q, dtype, q_heads, scratch_bytes=SCRATCH, max_seq_len=131072)
+        assert rc == 0 and wide.tobytes() == got.tobytes()

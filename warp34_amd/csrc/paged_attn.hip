@@ -211,11 +211,22 @@ __host__ inline uint32_t q_group_magic_for(int q_group) { return (65536u + (uint
 struct ChunkGeom {
     int u_first, n_units, upc, n_chunks;
 };
-__device__ __forceinline__ ChunkGeom chunk_geom(int u_lo, int u_hi, int max_chunks, int min_upc) {
+// Chunks of n_units units, `whole` of them of the usual least length.  Up to `few` chunks (kFewChunks*) they are shorter: four units are one
+// for the first wave of every SIMD, which then shares its issue slots with nobody, and one half unit per wave of a row format.
+constexpr int kShortChunkUnits = 4;
+__host__ __device__ constexpr int chunk_count(int n_units, int whole, int few) {
+    const int quick = (n_units + kShortChunkUnits - 1) / kShortChunkUnits;
+    return whole <= 1 || whole >= few ? whole : quick < few ? quick : few;
+}
+// us a layer step of one request, chunks of eight units / of four (merged by one wave per row on both sides): TQ4, 1 token on 600 keys
+// 17.3 / 16.8, on 2 500 17.5 / 17.1, 4 tokens on 5 000 with 40 chunks 21.2 / 21.5; Q8_0 1 200 17.3 / 16.6, 5 000 18.3 / 17.3; FP16 2 500 17.0 / 15.6, 10 000
+// with 79 chunks 18.4 / 18.8.
+constexpr int kFewChunksTq4 = 24, kFewChunksRows = 32;
+__device__ __forceinline__ ChunkGeom chunk_geom(int u_lo, int u_hi, int max_chunks, int min_upc, int few) {
     ChunkGeom g;
     g.u_first = u_lo >> 5;
     g.n_units = (u_hi >= u_lo) ? ((u_hi >> 5) - g.u_first + 1) : 0;
-    int nc = fast_div(g.n_units + min_upc - 1, min_upc);
+    int nc = chunk_count(g.n_units, fast_div(g.n_units + min_upc - 1, min_upc), few);
     if (nc > max_chunks) nc = max_chunks;
     if (nc < 1) nc = 1;
     g.upc = fast_div(g.n_units + nc - 1, nc);
@@ -385,6 +396,7 @@ __device__ __forceinline__ constexpr int tq4_pv_elem(int h, int j, int r) {
 // Smallest chunk: 256 tokens, one unit per wave.  7 to 12 % faster than 16 at 16K-32K keys, same as 4
 constexpr int kMinUnitsPerChunk = 8;
 constexpr int kMergeGroups = 16;
+constexpr int kMergeFew = 32;  // up to this many chunks: one wave per row (split_merge_few_kernel)
 constexpr int kMergeMaxPerGroup = 16;  // at most 256 partials per row
 
 // ---- balanced decode ----------------------------------------------------------------------------
@@ -836,7 +848,7 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
         if (u_lo == 0 && B.max_seq_len > 0 && u_hi == B.max_seq_len - 1) {
             g = ChunkGeom{0, P.spec_units, P.spec_upc, P.spec_chunks};  // as long as the host's bound
         } else {
-            g = chunk_geom(u_lo, u_hi, P.max_chunks, P.min_upc);
+            g = chunk_geom(u_lo, u_hi, P.max_chunks, P.min_upc, kFewChunksTq4);
         }
         if (chunk >= g.n_chunks) return;
         cu_first = g.u_first + chunk * g.upc;
@@ -1920,6 +1932,84 @@ __global__ __launch_bounds__(GROUPS * 64) void split_merge_kernel(const float* p
     store_out_row<TQ, HD>(P, row, lane, o);
 }
 
+// The same for rows of at most SLOTS chunks: one wave per row, which holds all of its records' slices; the records reach the other lanes
+// through scalar registers, no LDS and no barrier.  The sums are those of ORDER waves (split_merge_kernel<.., ORDER>) added up in its order: every
+// bit is the same.
+template <typename TQ, int HD, int SLOTS, int ORDER>
+__global__ __launch_bounds__(64) void split_merge_few_kernel(const float* part_acc_in, const float* part_ml_in, int max_chunks_in,
+                                                             int num_q_heads_in, const AttnParams P, float out_scale, int rotate) {
+    static_assert(SLOTS <= 64, "one record per lane");
+    const int lane = (int)threadIdx.x;
+    const int tok = (int)blockIdx.y;
+    const warp34_attention_batch& B = P.B;
+    const size_t row = (size_t)tok * num_q_heads_in + blockIdx.x;
+    const float* ml = part_ml_in + row * max_chunks_in * 4;
+    const float* acc = part_acc_in + row * max_chunks_in * kHeadDim;
+    f4 rec = {kNegBig, 0.f, 0.f, 0.f};
+    if (lane < max_chunks_in) rec = *reinterpret_cast<const f4*>(ml + 4 * lane);
+    f4 a[SLOTS];
+#pragma unroll
+    for (int s = 0; s < SLOTS; ++s) {
+        a[s] = f4{0.f, 0.f, 0.f, 0.f};
+        if (s < max_chunks_in && (HD == 256 || 4 * lane < HD)) a[s] = *reinterpret_cast<const f4*>(acc + (size_t)s * kHeadDim + 4 * lane);
+    }
+    bool ok = B.valid_token_mask == nullptr || B.valid_token_mask[tok] != 0;
+    bool found = false;
+    for (int base = 0; base < B.num_reqs && !found; base += 64) {
+        const int r = base + lane;
+        const bool inb = r < B.num_reqs;
+        const int lo = inb ? B.query_start_loc[r] : 0x7fffffff;
+        const int hi = inb ? B.query_start_loc[r + 1] : -0x7fffffff;
+        const int rm = (inb && B.valid_req_mask != nullptr) ? (int)B.valid_req_mask[r] : 1;
+        const unsigned long long hits = __ballot(inb && tok >= lo && tok < hi);
+        if (hits != 0ull) {
+            found = true;
+            ok = ok && __builtin_amdgcn_readlane(rm, __builtin_ctzll(hits)) != 0;
+        }
+    }
+    if (!ok || !found) return;  // masked row: output untouched
+    const int n_chunks = min((int)__int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(rec[2]))), max_chunks_in);
+    const bool mine = lane < n_chunks && rec[1] > 0.f;
+    float m_tot = mine ? fmaxf(rec[0], kNegBig) : kNegBig;
+    m_tot = fmaxf(m_tot, lane_xor<1>(m_tot, lane));
+    m_tot = fmaxf(m_tot, lane_xor<2>(m_tot, lane));
+    m_tot = fmaxf(m_tot, lane_xor<4>(m_tot, lane));
+    m_tot = fmaxf(m_tot, lane_xor<8>(m_tot, lane));
+    m_tot = fmaxf(m_tot, lane_xor<16>(m_tot, lane));
+    m_tot = fmaxf(m_tot, lane_xor<32>(m_tot, lane));
+    const float w = mine ? __builtin_amdgcn_exp2f(rec[0] - m_tot) : 0.f, l = rec[1];
+    const unsigned long long live = __ballot(mine);
+    f4 v[ORDER];
+    float l_part[ORDER];
+#pragma unroll
+    for (int g = 0; g < ORDER; ++g) v[g] = f4{0.f, 0.f, 0.f, 0.f}, l_part[g] = 0.f;
+#pragma unroll
+    for (int s = 0; s < SLOTS; ++s) {
+        if ((live >> s) & 1ull) {  // uniform
+            const float ws = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), s));
+            const float ls = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(l), s));
+            l_part[s % ORDER] = __builtin_fmaf(ls, ws, l_part[s % ORDER]);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) v[s % ORDER][k] = __builtin_fmaf(a[s][k], ws, v[s % ORDER][k]);
+        }
+    }
+    f4 tot = {0.f, 0.f, 0.f, 0.f};
+    float l_tot = 0.f;
+#pragma unroll
+    for (int g = 0; g < ORDER; ++g) {
+        tot += v[g];
+        l_tot += l_part[g];
+    }
+    const float inv = l_tot > 0.f ? out_scale / l_tot : 0.f;
+    float o[4] = {tot[0] * inv, tot[1] * inv, tot[2] * inv, tot[3] * inv};
+    if (rotate) {
+        wht256_wave(o, lane);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) o[k] = apply_sign(o[k], 4 * lane + k);
+    }
+    store_out_row<TQ, HD>(P, row, lane, o);
+}
+
 }  // namespace w34
 
 #include "paged_attn_rows.h"
@@ -2090,6 +2180,22 @@ static int launch_balanced_merge(const AttnParams& P, int kv_subs, float out_sca
 template <typename TQ, bool SP, int HD>
 static int launch_split_merge(const AttnParams& P, int slots, float out_scale, hipStream_t stream) {
     const dim3 grid((unsigned)P.num_q_heads, (unsigned)P.B.total_tokens);
+    if constexpr (!SP) {
+        const auto few = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, grid, dim3(64), 0, stream, (const float*)P.part_acc, (const float*)P.part_ml, slots, P.num_q_heads, P,
+                               out_scale, P.rot_out);
+            return (int)hipGetLastError();
+        };
+        if (slots <= kMergeFew) {
+            if (merge_small_groups(P))
+                return slots <= 8    ? few(split_merge_few_kernel<TQ, HD, 8, 4>)
+                       : slots <= 16 ? few(split_merge_few_kernel<TQ, HD, 16, 4>)
+                                     : few(split_merge_few_kernel<TQ, HD, kMergeFew, 4>);
+            return slots <= 8    ? few(split_merge_few_kernel<TQ, HD, 8, kMergeGroups>)
+                   : slots <= 16 ? few(split_merge_few_kernel<TQ, HD, 16, kMergeGroups>)
+                                 : few(split_merge_few_kernel<TQ, HD, kMergeFew, kMergeGroups>);
+        }
+    }
     if (merge_small_groups(P)) {
         hipLaunchKernelGGL((split_merge_kernel<TQ, SP, HD, 4>), grid, dim3(4 * 64), 0, stream, (const float*)P.part_acc,
                            (const float*)P.part_ml, slots, P.num_q_heads, P, out_scale, P.rot_out);
@@ -2114,11 +2220,11 @@ static int tiles_bound(const warp34_attention_batch& B, const AttnParams& P) {
     return (int)(B.max_q_len > 0 && by_requests < by_tokens ? by_requests : by_tokens);
 }
 
-// P.spec_* = chunk_geom(0, max_seq_len - 1, P.max_chunks, P.min_upc), worked out on the host
-static void fill_spec_geometry(AttnParams& P, int max_seq_len) {
+// P.spec_* = chunk_geom(0, max_seq_len - 1, P.max_chunks, P.min_upc, few), worked out on the host
+static void fill_spec_geometry(AttnParams& P, int max_seq_len, int few) {
     if (max_seq_len <= 0) return;
     P.spec_units = ((max_seq_len - 1) >> 5) + 1;
-    int nc = (P.spec_units + P.min_upc - 1) / P.min_upc;
+    int nc = chunk_count(P.spec_units, (P.spec_units + P.min_upc - 1) / P.min_upc, few);
     if (nc > P.max_chunks) nc = P.max_chunks;
     if (nc < 1) nc = 1;
     P.spec_upc = (P.spec_units + nc - 1) / nc;
@@ -2258,7 +2364,7 @@ static int launch_tq4(const warp34_exec* ex, const warp34_kv_layer_layout* layou
     int grid_x = P.max_chunks;
     if (batch->max_seq_len > 0) {
         const int units = (batch->max_seq_len + kUnit - 1) / kUnit + 1;
-        const int bound = (units + P.min_upc - 1) / P.min_upc;
+        const int bound = chunk_count(units, (units + P.min_upc - 1) / P.min_upc, kFewChunksTq4);
         if (bound < grid_x) grid_x = bound < 1 ? 1 : bound;
     }
     // No tile has more chunks than that: the cap is lowered to it, which changes no chunk (a
@@ -2266,7 +2372,7 @@ static int launch_tq4(const warp34_exec* ex, const warp34_kv_layer_layout* layou
     // the merge kernel loads ahead of knowing the count, as small as the bound allows.
     P.max_chunks = grid_x;
     P.part_stride = grid_x;
-    fill_spec_geometry(P, batch->max_seq_len);
+    fill_spec_geometry(P, batch->max_seq_len, kFewChunksTq4);
     if (P.max_chunks > 1) {
         uint8_t* ws = reinterpret_cast<uint8_t*>((uintptr_t)ex->scratch_ptr);
         P.part_acc = reinterpret_cast<float*>(ws);
@@ -2532,7 +2638,7 @@ static int launch_rows(const warp34_exec* ex, const warp34_kv_layer_layout* layo
     int grid_x = P.max_chunks;
     if (batch->max_seq_len > 0) {
         const int units = (batch->max_seq_len + kUnit - 1) / kUnit + 1;
-        const int bound = (units + P.min_upc - 1) / P.min_upc;
+        const int bound = chunk_count(units, (units + P.min_upc - 1) / P.min_upc, kFewChunksRows);
         if (bound < grid_x) grid_x = bound < 1 ? 1 : bound;
     }
     // No tile has more chunks than that: the cap is lowered to it, which changes no chunk (a
@@ -2540,7 +2646,7 @@ static int launch_rows(const warp34_exec* ex, const warp34_kv_layer_layout* layo
     // the merge kernel loads ahead of knowing the count, as small as the bound allows.
     P.max_chunks = grid_x;
     P.part_stride = grid_x;
-    fill_spec_geometry(P, batch->max_seq_len);
+    fill_spec_geometry(P, batch->max_seq_len, kFewChunksRows);
     if (P.max_chunks > 1) {
         uint8_t* ws = reinterpret_cast<uint8_t*>((uintptr_t)ex->scratch_ptr);
         P.part_acc = reinterpret_cast<float*>(ws);
