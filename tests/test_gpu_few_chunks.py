@@ -1,11 +1,11 @@
-"""Contexts of few chunks: shorter chunks, and a merge of one wave per row, against the oracle at the lengths where the number of chunks and
+"""Contexts and batches of few chunks: shorter chunks, and a merge of one wave per row, against the oracle at the lengths where the number of chunks and
 the form of the merge change; and, with a bound on the length under which the merge of several waves runs, the same bytes."""
 import numpy as np
 import pytest
 
 import oracle
 from cases import make_case
-from oracle import DT_BF16, DT_F16, FMT_BF16, FMT_FP8, FMT_Q8_0, FMT_TQ4
+from oracle import DT_BF16, DT_F16, FMT_BF16, FMT_FP16, FMT_FP8, FMT_Q8_0, FMT_TQ4, XF_IDENTITY, XF_WHT256
 
 pytestmark = pytest.mark.gpu
 SCRATCH = 64 << 20
@@ -38,3 +38,36 @@ def test_lengths_at_which_the_chunks_change(fmt, dtype, head_dim, units):
                        scale=G.channel_scale(v, dtype, hb, q_heads)[live])
         rc, wide, _ = G.dev_attention(dpool, hb, q, dtype, q_heads, scratch_bytes=SCRATCH, max_seq_len=131072)
         assert rc == 0 and wide.tobytes() == got.tobytes()
+
+
+@pytest.mark.parametrize("fmt,dtype,xf", [(FMT_TQ4, DT_BF16, None), (FMT_Q8_0, DT_F16, XF_IDENTITY), (FMT_Q8_0, DT_F16, XF_WHT256),
+                                          (FMT_FP16, DT_F16, None)])
+@pytest.mark.parametrize("reqs,longest", [(2, 1024), (2, 1025), (16, 128), (16, 129), (17, 180), (17, 181), (64, 48), (64, 49), (65, 20)])
+def test_decode_batches_on_either_side_of_the_grid_rule(fmt, dtype, xf, reqs, longest):
+    """Chunk grid and plan give the same bytes for a batch that the chunk grid may serve: which of them runs follows from the host's bound on
+    the lengths (units of the longest request times requests: 2 048, from 17 requests on 3 072).  A request without a key and a
+    masked one among the others."""
+    import gpu_harness as G
+
+    rng = np.random.default_rng(reqs * 1000 + longest)
+    seq = [int(x) for x in rng.integers(1, longest * UNIT if reqs == 2 else max(2, longest * UNIT // 4), reqs)]
+    seq[-1] = longest * UNIT
+    q_heads = 16 if reqs < 17 else 8
+    pool, bt, k, v, q, aq, ctx = make_case(fmt, 16, seq, [1] * reqs, 2400 + reqs, dtype, q_heads=q_heads, xf=xf)
+    mask = np.ones(reqs, dtype=np.uint8)
+    if reqs > 2:
+        mask[1] = 0
+    hb = oracle.HostBatch(aq, seq, bt, context_lens_before=ctx, valid_req_mask=mask)
+    want = oracle.paged_attention(pool, hb, q, dtype, q_heads, n_threads=8)
+    dpool = G.DevPool(pool)
+    dpool.upload()
+    outs = []
+    for bound in (max(seq), max(seq) + 40 * UNIT, 131072):
+        rc, got, _ = G.dev_attention(dpool, hb, q, dtype, q_heads, scratch_bytes=SCRATCH, max_seq_len=bound)
+        assert rc == 0
+        assert (got[mask == 0] == 0x5500).all()
+        outs.append(got.tobytes())
+    live = mask != 0
+    G.assert_close(got[live], dtype, want[live], what="fmt=%d reqs=%d longest=%d units" % (fmt, reqs, longest),
+                   scale=G.channel_scale(v, dtype, hb, q_heads)[live], plain_excess=4e-4 if xf == XF_WHT256 else 0.0)
+    assert outs[0] == outs[1] == outs[2]

@@ -129,6 +129,10 @@ struct AttnParams {
         struct {
             int short_units, short_tiles, short_tok_tile;
         };
+        // balanced decode: the chunk grid's cap on chunks per request, for batches it may serve (grid_decode_units); 0: none
+        struct {
+            int grid_chunks;
+        };
     };
     // Partial records: part_stride slots per output row.  Slots [0, max_chunks) belong to the
     // split-K chunks of the decode kernels; a shared-prefix pass (tile kernel over the keys every
@@ -424,6 +428,16 @@ constexpr int kMergeMaxPerGroup = 16;  // at most 256 partials per row
 __host__ __device__ __forceinline__ size_t bal_partial_row(int slot, int kv_subs, int kv_sub, int cols, int col) {
     return ((size_t)slot * kv_subs + kv_sub) * cols + col;
 }
+
+// A decode batch (kGridDecodeReqs requests at most, one q subgroup) whose longest request times the number of requests is at most this
+// many units is cut as the chunk grid cuts it, 128 / requests chunks each at most, and the chunk grid runs instead of the plan where the host's
+// bound on the lengths says as much: the plan and the merge's table cost 2 to 3 us of a call, one request's chunks being longer
+// than a share costs less.  us a layer, attention alone, plan / chunk grid: TQ4, 2 requests of 1 600 to 16 000 keys 16.1 / 14.2, 8 of 400 to 4 000
+// 15.4 / 13.2, 16 of 400 to 4 000 17.4 / 15.2, 32 of 200 to 2 000 18.2 / 16.2, 32 of 300 to 3 000 25.0 / 18.8; Q8_0, 8 of 400 to 4 000 14.0 / 12.6, 24 of
+// 266 to 2 666 20.1 / 18.2.  Beyond the line, lengths from a tenth up: 10 of up to 9 600 TQ4 18.7 / 19.7, Q8_0 20.3 / 21.8, 12 of up to 10 666 23.1 /
+// 25.3.  More than 16 requests (shares that cross from one into the next): later, 48 of up to 2 000 TQ4 25.0 / 20.6, Q8_0 23.3 / 24.0.
+constexpr int kGridDecodeReqs = 64;
+__host__ __device__ constexpr int grid_decode_units(int reqs) { return reqs <= 16 ? 2048 : 3072; }
 
 struct BalReq {  // entry base + lane of a group of 64
     int lo, hi;          // query tokens of the request
@@ -1559,7 +1573,8 @@ __device__ __forceinline__ void bal_short_piece(const AttnParams& P, TileFn&& ti
 // loads are the same addresses in every wave of the chip and stay in cache) and calls
 // tile(piece) for the pieces of its workgroup's share, in order.
 // SHORT: a batch that turns out short is left to short_batch().
-template <bool SHORT, typename TileFn, typename ShortFn>
+// FEW: chunk_count's line for the format.
+template <bool SHORT, int FEW, typename TileFn, typename ShortFn>
 __device__ __forceinline__ void bal_for_each_piece(const AttnParams& P, TileFn&& tile, ShortFn&& short_batch) {
     const int lane = (int)threadIdx.x & 63;
     const int entries = P.B.num_reqs * P.bal_tiles;
@@ -1598,19 +1613,28 @@ __device__ __forceinline__ void bal_for_each_piece(const AttnParams& P, TileFn&&
     it.tok_tile = P.tok_tile;
     int my_begin = 0, my_end = 0, piece_end = 0;  // (aligned: the one piece ends the share)
     int share = 1;
-    if (P.bal_aligned) {  // uniform for the grid; at most 64 entries
+    // a batch that the chunk grid serves where the host's bound says so: its chunks, so that the bits do not depend on the bound
+    bool as_grid = false;
+    if constexpr (!SHORT) as_grid = P.grid_chunks > 0 && __ballot(q0.units * P.B.num_reqs > grid_decode_units(P.B.num_reqs)) == 0ull;
+    const bool aligned = P.bal_aligned || as_grid;
+    if (aligned) {  // uniform for the grid; at most 64 entries
         // Units per piece: the smallest count found by a few steps from below for which the pieces fit
         // the grid.  (Every wave of the chip computes the same numbers.)
         const int groups = (int)gridDim.x;
         const int units = __builtin_amdgcn_readlane(wave_incl_scan(q0.units), 63);
         int pieces, incl;
-        share = bal_share(units, groups, P.min_upc);
-        for (;;) {
-            pieces = q0.units > 0 ? fast_div(q0.units + share - 1, share) : 0;
+        if (as_grid) {
+            pieces = q0.units > 0 ? chunk_geom(0, 32 * q0.units - 1, P.grid_chunks, P.min_upc, FEW).n_chunks : 0;
             incl = wave_incl_scan(pieces);
-            const int n = __builtin_amdgcn_readlane(incl, 63);
-            if (n <= groups) break;
-            share += fast_div(share * (n - groups), groups) + 1;
+        } else {
+            share = bal_share(units, groups, P.min_upc);
+            for (;;) {
+                pieces = q0.units > 0 ? fast_div(q0.units + share - 1, share) : 0;
+                incl = wave_incl_scan(pieces);
+                const int n = __builtin_amdgcn_readlane(incl, 63);
+                if (n <= groups) break;
+                share += fast_div(share * (n - groups), groups) + 1;
+            }
         }
         const unsigned long long hits = __ballot(pieces > 0 && (int)blockIdx.x < incl);
         if (hits == 0ull) return;
@@ -1687,7 +1711,7 @@ __device__ __forceinline__ void bal_for_each_piece(const AttnParams& P, TileFn&&
         }
         return false;
     };
-    bool have = P.bal_aligned || scan_group(q0, incl0);
+    bool have = aligned || scan_group(q0, incl0);
     if (!have) have = find_next();
     while (have) {
         tile(it);
@@ -1706,7 +1730,7 @@ __global__ __launch_bounds__(kTq4Waves * 64, 1) void paged_attn_tq4_balanced_ker
         tq4_tile<TQ, true>(P, smem, it, first);
         first = false;
     };
-    bal_for_each_piece<false>(P, piece, [] {});
+    bal_for_each_piece<false, kFewChunksTq4>(P, piece, [] {});
 }
 
 // Merge for the balanced decode kernel: one workgroup of GROUPS waves per (token, q head) row; wave g
@@ -2143,6 +2167,17 @@ static bool balanced_decode_applicable(const warp34_exec* ex, const warp34_atten
            batch->valid_token_mask == nullptr && batch->total_tokens <= 65535 && ex->scratch_ptr != 0 && (ex->scratch_ptr & 15u) == 0u;
 }
 // shares of a balanced decode batch per (kv head, q subgroup): a function of gqa only
+// The chunk grid's cap on chunks per request of a decode batch that it may serve in the plan's place (grid_decode_units): one round of
+// workgroups; 0: not such a batch.
+static int decode_grid_chunks(const warp34_exec* ex, const warp34_attention_batch* batch, int num_q_heads, int q_subgroups) {
+    if (q_subgroups != 1 || batch->num_reqs < 2 || batch->num_reqs > kGridDecodeReqs) return 0;
+    const int chunks = kTargetWorkgroupsPerHead / batch->num_reqs;
+    return partial_bytes((long long)batch->total_tokens * num_q_heads, chunks) <= ex->scratch_size ? chunks : 0;
+}
+static bool decode_on_grid(const warp34_attention_batch* batch, int chunks) {
+    return chunks > 0 && batch->max_seq_len > 0 &&
+           ((long long)batch->max_seq_len + kUnit - 1) / kUnit * batch->num_reqs <= grid_decode_units(batch->num_reqs);
+}
 static int balanced_groups(int q_subgroups) {
     int groups = kTargetWorkgroupsPerHead / (q_subgroups > 0 ? q_subgroups : 1);
     if (groups > kMergeGroups * kMergeMaxPerGroup - 1) groups = kMergeGroups * kMergeMaxPerGroup - 1;
@@ -2355,8 +2390,18 @@ static int launch_tq4(const warp34_exec* ex, const warp34_kv_layer_layout* layou
                       layout->v_page_stride_bytes <= 0xFFFFFFFFull)
                          ? 1
                          : 0;
-    P.max_chunks = force_single ? 1 : choose_max_chunks(ex, batch->total_tokens, num_q_heads, P.tok_tile,
-                                                        P.q_subgroups);
+    P.tiles_by_request = (batch->max_q_len > 0 && batch->max_q_len <= P.tok_tile) ? 1 : 0;
+    const int kv_subs = layout->local_kv_heads * P.q_subgroups;
+    // decode batches: the plan's records and table fit
+    const int plan_groups = balanced_groups(P.q_subgroups);
+    const size_t plan_rows = bal_partial_row(plan_groups + batch->num_reqs, kv_subs, 0, 16, 0);
+    const bool plan = balanced_decode_applicable(ex, batch, P.tiles_by_request, force_single) &&
+                      partial_bytes((long long)plan_rows, 1) + (size_t)batch->total_tokens * 16 <= ex->scratch_size;
+    const int decode_chunks = plan ? decode_grid_chunks(ex, batch, num_q_heads, P.q_subgroups) : 0;
+    const bool on_grid = decode_on_grid(batch, decode_chunks);
+    P.max_chunks = force_single ? 1
+                   : on_grid    ? decode_chunks
+                                : choose_max_chunks(ex, batch->total_tokens, num_q_heads, P.tok_tile, P.q_subgroups);
     P.part_acc = nullptr;
     P.part_ml = nullptr;
     const long long rows = (long long)batch->total_tokens * num_q_heads;
@@ -2378,9 +2423,7 @@ static int launch_tq4(const warp34_exec* ex, const warp34_kv_layer_layout* layou
         P.part_acc = reinterpret_cast<float*>(ws);
         P.part_ml = P.part_acc + (size_t)rows * P.max_chunks * kHeadDim;
     }
-    P.tiles_by_request = (batch->max_q_len > 0 && batch->max_q_len <= P.tok_tile) ? 1 : 0;
     const int grid_z = tiles_bound(*batch, P);
-    const int kv_subs = layout->local_kv_heads * P.q_subgroups;
     const dim3 grid((unsigned)grid_x, (unsigned)kv_subs, (unsigned)grid_z);
     hipStream_t stream = (hipStream_t)ex->stream;
     int rc;
@@ -2429,26 +2472,23 @@ static int launch_tq4(const warp34_exec* ex, const warp34_kv_layer_layout* layou
     }
     // Decode batches of several requests: equal shares of the batch's units per workgroup
     // instead of per-request chunks (the requests' lengths are unknown to the host and differ).
-    if (balanced_decode_applicable(ex, batch, P.tiles_by_request, force_single)) {
-        const int groups = balanced_groups(P.q_subgroups);
-        const size_t prows = bal_partial_row(groups + batch->num_reqs, kv_subs, 0, 16, 0);
-        if (partial_bytes((long long)prows, 1) + (size_t)batch->total_tokens * 16 <= ex->scratch_size) {
-            P.part_acc = reinterpret_cast<float*>((uintptr_t)ex->scratch_ptr);
-            P.part_ml = P.part_acc + prows * kHeadDim;
-            P.bal_table = reinterpret_cast<int32_t*>(P.part_ml + prows * 4);
-            P.max_chunks = groups + 1;
-            P.bal_tiles = 1;
-            P.bal_cols = 16;
-            P.piece_cost = kTq4PieceCost;
-            P.bal_aligned = balanced_aligned(batch->num_reqs, groups);
-            rc = ensure_dynamic_lds(paged_attn_tq4_balanced_kernel<TQ>, smem_bytes_for(1), true);
-            if (rc) return rc;
-            hipLaunchKernelGGL((paged_attn_tq4_balanced_kernel<TQ>), dim3((unsigned)groups, (unsigned)kv_subs),
-                               dim3(waves_for(1) * 64), smem_bytes_for(1), stream, P);
-            rc = (int)hipGetLastError();
-            if (rc) return rc;
-            return launch_balanced_merge<TQ, kHeadDim>(P, kv_subs, kLutInvGain, stream);
-        }
+    if (plan && !on_grid) {
+        P.part_acc = reinterpret_cast<float*>((uintptr_t)ex->scratch_ptr);
+        P.part_ml = P.part_acc + plan_rows * kHeadDim;
+        P.bal_table = reinterpret_cast<int32_t*>(P.part_ml + plan_rows * 4);
+        P.max_chunks = plan_groups + 1;
+        P.bal_tiles = 1;
+        P.bal_cols = 16;
+        P.piece_cost = kTq4PieceCost;
+        P.bal_aligned = balanced_aligned(batch->num_reqs, plan_groups);
+        P.grid_chunks = decode_chunks;
+        rc = ensure_dynamic_lds(paged_attn_tq4_balanced_kernel<TQ>, smem_bytes_for(1), true);
+        if (rc) return rc;
+        hipLaunchKernelGGL((paged_attn_tq4_balanced_kernel<TQ>), dim3((unsigned)plan_groups, (unsigned)kv_subs),
+                           dim3(waves_for(1) * 64), smem_bytes_for(1), stream, P);
+        rc = (int)hipGetLastError();
+        if (rc) return rc;
+        return launch_balanced_merge<TQ, kHeadDim>(P, kv_subs, kLutInvGain, stream);
     }
     P.bal_tiles = tiles_per_request_bound(*batch, P);
     rc = ensure_dynamic_lds(paged_attn_tq4_kernel<TQ, 1>, smem_bytes_for(1), true);
@@ -2496,7 +2536,7 @@ static bool rows_vres(const warp34_kv_layer_layout* l) {
 // Balanced decode / verify over row-format pages; -1: the batch is not for it.
 template <typename TQ, int KVF, bool VRES, int HD>
 static int launch_rows_balanced(const warp34_exec* ex, const warp34_attention_batch* batch, AttnParams P, int kv_subs,
-                                int force_single, hipStream_t stream) {
+                                int force_single, hipStream_t stream, int* grid_chunks) {
     if (force_single || batch->sliding_window > 0 || batch->valid_token_mask != nullptr || ex->scratch_ptr == 0 ||
         (ex->scratch_ptr & 15u) != 0u)
         return -1;
@@ -2534,6 +2574,14 @@ static int launch_rows_balanced(const warp34_exec* ex, const warp34_attention_ba
     P.bal_cols = 16 * nt;
     P.bal_aligned = balanced_aligned(entries, groups);
     P.short_units = -1;
+    if (HD == kHeadDim && nt * tiles == 1 && groups == all_groups) {
+        const int chunks = decode_grid_chunks(ex, batch, P.num_q_heads, P.q_subgroups);
+        if (decode_on_grid(batch, chunks)) {
+            *grid_chunks = chunks;
+            return -1;
+        }
+        P.grid_chunks = chunks;
+    }
     if (nt == 2 || (VRES && tiles > 1 && !P.bal_aligned)) {
         if (entries <= kShortMaxEntries / 2 && (long long)batch->num_reqs * tiles16 <= std::min(groups, kShortMaxEntries)) {
             // (no entry has two pieces, on either path one workgroup does the same arithmetic: launch shape only)
@@ -2630,8 +2678,18 @@ static int launch_rows(const warp34_exec* ex, const warp34_kv_layer_layout* layo
     P.tok_tile = 16 / q_group;  // one N tile
     if (P.tok_tile < 1) P.tok_tile = 1;
     P.min_upc = kMinUnitsPerChunk;
-    P.max_chunks = force_single ? 1 : choose_max_chunks(ex, batch->total_tokens, num_q_heads, P.tok_tile,
-                                                        P.q_subgroups);
+    P.tiles_by_request = (batch->max_q_len > 0 && batch->max_q_len <= P.tok_tile) ? 1 : 0;
+    P.rot_q = layout->k_transform == WARP34_KV_TRANSFORM_RADEMACHER_WHT256 ? 1 : 0;
+    P.rot_out = layout->v_transform == WARP34_KV_TRANSFORM_RADEMACHER_WHT256 ? 1 : 0;
+    const int grid_z = tiles_bound(*batch, P);
+    const int kv_subs = layout->local_kv_heads * P.q_subgroups;
+    hipStream_t stream = (hipStream_t)ex->stream;
+    int rc, decode_chunks = 0;
+    rc = launch_rows_balanced<TQ, KVF, VRES, HD>(ex, batch, P, kv_subs, force_single, stream, &decode_chunks);
+    if (rc >= 0) return rc;
+    P.max_chunks = force_single        ? 1
+                   : decode_chunks > 0 ? decode_chunks
+                                       : choose_max_chunks(ex, batch->total_tokens, num_q_heads, P.tok_tile, P.q_subgroups);
     P.part_acc = nullptr;
     P.part_ml = nullptr;
     const long long rows = (long long)batch->total_tokens * num_q_heads;
@@ -2652,16 +2710,7 @@ static int launch_rows(const warp34_exec* ex, const warp34_kv_layer_layout* layo
         P.part_acc = reinterpret_cast<float*>(ws);
         P.part_ml = P.part_acc + (size_t)rows * P.max_chunks * kHeadDim;
     }
-    P.tiles_by_request = (batch->max_q_len > 0 && batch->max_q_len <= P.tok_tile) ? 1 : 0;
-    P.rot_q = layout->k_transform == WARP34_KV_TRANSFORM_RADEMACHER_WHT256 ? 1 : 0;
-    P.rot_out = layout->v_transform == WARP34_KV_TRANSFORM_RADEMACHER_WHT256 ? 1 : 0;
-    const int grid_z = tiles_bound(*batch, P);
-    const int kv_subs = layout->local_kv_heads * P.q_subgroups;
     dim3 grid((unsigned)grid_x, (unsigned)kv_subs, (unsigned)grid_z);
-    hipStream_t stream = (hipStream_t)ex->stream;
-    int rc;
-    rc = launch_rows_balanced<TQ, KVF, VRES, HD>(ex, batch, P, kv_subs, force_single, stream);
-    if (rc >= 0) return rc;
     P.bal_tiles = tiles_per_request_bound(*batch, P);
     P.key_groups = rows_key_groups(*batch, P, kv_subs, grid_z);
     P.first_round = HD != kHeadDim ? rows_first_round(*batch, P, kv_subs, grid_z) : 0;

@@ -877,7 +877,10 @@ __device__ __forceinline__ void rows_tile(const AttnParams& P, uint8_t* smem, co
         } else {
             const float inv = l_col > 0.f ? 1.0f / l_col : 0.f;
 #pragma unroll
-            for (int k = 0; k < 4; ++k) v[k] *= inv;
+            for (int k = 0; k < 4; ++k) {
+                v[k] *= inv;
+                asm("" : "+v"(v[k]));  // rounded before the conversion to fp16, as where a merge kernel finishes the row
+            }
             if (K8 && P.rot_out) {  // rotated V rows: one inverse rotation of the finished row
                 wht256_wave(v, lane);
 #pragma unroll
@@ -959,7 +962,7 @@ __global__ __launch_bounds__(kKv16Waves * 64, 1) void paged_attn_rows_mapped_ker
 template <typename TQ, int NT, int KVF, bool VRES, bool STREAM, int HD = kHeadDim>
 __global__ __launch_bounds__(kKv16Waves * 64, 1) void paged_attn_rows_balanced_kernel(const AttnParams P) {
     extern __shared__ __align__(16) uint8_t smem[];
-    bal_for_each_piece<(NT > 1 || (VRES && !STREAM))>(
+    bal_for_each_piece<(NT > 1 || (VRES && !STREAM)), kFewChunksRows>(
         P, [&](const BalItem& it) { rows_tile<TQ, NT, KVF, true, VRES, STREAM, HD>(P, smem, it); },
         [&] {
             const AttnParams A = kernel_params_again();
