@@ -116,3 +116,30 @@ def test_tq4_scales_of_unseen_rows(bits):
             assert rc == 0
             outs.append(got[:-1].tobytes())
     assert all(o == outs[0] for o in outs)
+
+
+@pytest.mark.parametrize("xf", [XF_WHT256, XF_IDENTITY])
+def test_tq4_value_scales_that_leave_no_room_above_one(xf):
+    """Value scales of 3 000 in every third token: a probability of more than 21 times such a scale is no fp16 number, so a running maximum
+    that lags behind the scores would overflow there.  Tiles of both sizes, the same bytes."""
+    import gpu_harness as G
+
+    seq, ql = [700, 333], [300, 333]
+    pool, bt, k, v, q, aq, ctx = make_case(FMT_TQ4, 64, seq, ql, 1801, DT_F16, q_heads=16, xf=xf, v_xf=xf)
+    rows = pool.v.reshape(-1, pool.kv_heads, pool.block_size, pool.tok).view(np.uint16)
+    assert np.shares_memory(rows, pool.v)
+    rows[:, :, ::3, [0, 33]] = np.float16(3000.0).view(np.uint16)
+    hb = oracle.HostBatch(aq, seq, bt, context_lens_before=ctx)
+    want = oracle.paged_attention(pool, hb, q, DT_F16, 16, n_threads=8)
+    dpool = G.DevPool(pool)
+    dpool.upload()
+    outs = []
+    for force in (1, WIDE):
+        rc, got, _ = G.dev_attention(dpool, hb, q, DT_F16, 16, force_kernel=force)
+        assert rc == 0
+        outs.append(got)
+    assert outs[0].tobytes() == outs[1].tobytes()
+    out = oracle.bits_to_f32(outs[0], DT_F16).astype(np.float64)
+    assert np.isfinite(out).all()
+    # the scores' error, 2e-3 of the largest value scale, and the output's rounding
+    assert (np.abs(out - want) <= 1e-2 * np.abs(want) + 2e-3 * 3000.0).all()

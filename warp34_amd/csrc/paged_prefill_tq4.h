@@ -46,6 +46,17 @@ static_assert(kPfSmem >= PfLds<WARP34_KV_FORMAT_TQ4>::kEpilogue && kPfSmem <= 16
 static_assert(PfLds<WARP34_KV_FORMAT_TQ4>::kRaw == kStageTq4, "TQ4 raw unit");
 static_assert(kPfWaves * 16 * 264 * 2 <= 2 * kPfDeqBytes, "query staging must fit in the dequant buffers");
 
+// Weights of two operands (TQ4, BF16): a column's running maximum is raised only by scores that exceed it by more than this (log2 domain), so
+// a probability may be up to 2^8; its operands keep 22 (16) bits of it whatever its size, the sums are fp32.  Raising multiplies 64 sums per column
+// tile, and of the first units nearly every one raises the maximum of some column of a wave.  TQ4 value scales ride on the probabilities: in a
+// unit with a larger one than kPfSlackScale, where the weight could leave fp16's range, and where a column does not see the whole unit (what lies
+// behind the sequence must not matter), the maximum is exact.  Per column, so that tiles of either size give the same bits.  (One fp16
+// operand: exact as well, the largest probability is then 1 and rounds to itself; with the slack FP16 and Q8_0 batches came out 6 % further from 64
+// bits, 3.24e-4 for 3.05e-4.)  us, maximum
+// raised by every unit that exceeds it / now: 16 requests of 256 tokens on 2 048 keys BF16 224 / 199, TQ4 261 / 247, 4 of 700 on 6 000 BF16 507 / 459,
+// TQ4 634 / 618, 8 of 2 048 on 16 384 TQ4 6 261 / 6 185.
+constexpr float kPfSlack = 8.0f, kPfSlackScale = 255.0f;
+
 typedef __attribute__((address_space(3))) uint32_t lds_u32;
 
 // 16x16x32 MFMA on fp16 or bf16 operands given as raw bits
@@ -500,13 +511,18 @@ __global__ __launch_bounds__(12 * 64, 1) void paged_prefill_tq4_kernel(const Att
                 score[t] = (col_ok && pos >= col_lo && pos <= col_hi) ? score[t] : kNegBig;
             }
         }
-        // online softmax, log2 domain; key slot j of this lane = token 16 (j >> 2) + 4 b + (j & 3).  Few units raise a
-        // maximum (one in eight of a 16 000 token prefix): the others need no exchange between lanes.
+        // online softmax, log2 domain; key slot j of this lane = token 16 (j >> 2) + 4 b + (j & 3).  See kPfSlack.
         const float mx = max3(max3(max3(score[0], score[1], score[2]), score[3], score[4]), score[5], max2(score[6], score[7]));
-        if (!started || __ballot(mx > 0.f) != 0ull) {
+        float slack = kPfSlack;
+        if (__ballot(mx > 0.f) != 0ull) {  // one value scale of the unit per lane
+            const bool large = __ballot(!(fabsf(sc[64 + lane]) <= kPfSlackScale)) != 0ull;
+            slack = large || (MASKED && !(t0 >= col_lo && t0 + kUnit - 1 <= col_hi)) ? 0.f : kPfSlack;
+        }
+        const bool raise = !started || __ballot(mx > slack) != 0ull;
+        if (raise) {
             const float m = max_over_rows(mx);
             const bool empty = !(sum_over_rows(l_run) > 0.f);
-            const float up = empty ? (m > 0.5f * kNegBig ? m : 0.f) : fmaxf(m, 0.f);
+            const float up = empty ? (m > 0.5f * kNegBig ? m : 0.f) : m > slack ? m : 0.f;
             const float alpha = empty ? 1.f : __builtin_amdgcn_exp2f(-up);
             m_run += up;
             l_run *= alpha;
