@@ -400,8 +400,9 @@ __global__ __launch_bounds__(kQsaWaves * 64, 1) void qsa_sparse_tq4_kernel(QSA_L
             }
 #pragma unroll
             for (int t = 0; t < 8; ++t) psum += p[t];
+            const bool scale = alpha != 1.0f && l_run != 0.f;  // (without a weight so far the sums are zero)
             l_run = l_run * alpha + psum;
-            if (__ballot(alpha != 1.0f) != 0ull) {
+            if (__ballot(scale) != 0ull) {
 #pragma unroll
                 for (int h = 0; h < 2; ++h)
 #pragma unroll
