@@ -132,3 +132,30 @@ def test_many_short_requests(fmt, dtype, n, q_heads, longest):
     q_lens = [1 + (r * 37) % longest for r in range(n - 2)] + [longest, longest // 2]
     _run(fmt, dtype, 16, [q + 30 + 5 * r for r, q in enumerate(q_lens)], q_lens, 1901 + longest, q_heads=q_heads, keep=0.3,
          force=WIDE if dtype == DT_F16 else None)
+
+
+@pytest.mark.parametrize("fmt", [FMT_Q8_0, FMT_FP8])
+@pytest.mark.parametrize("reqs,idle", [(2, 2), (5, 5), (64, 64), (70, 64), (70, 70)])
+def test_idle_requests_over_rotated_8bit_values_and_many_query_heads(fmt, reqs, idle):
+    """32 query heads on one kv head, decode: the first requests (all that the plan looks at first, or all there are) masked, then without keys.
+    Masked rows stay as they were, rows without keys are zero, the others are the oracle's."""
+    import gpu_harness as G
+    from cases import make_case
+
+    seq = [20 + 37 * (r % 5) for r in range(reqs)]
+    pool, bt, k, v, q, aq, ctx = make_case(fmt, 16, seq, [1] * reqs, 2500 + reqs, DT_F16, kv_heads=1, q_heads=32, xf=oracle.XF_WHT256)
+    dpool = G.DevPool(pool)
+    dpool.upload()
+    live = np.arange(reqs) >= idle
+    for masked in (True, False):
+        lens = seq if masked else [s if on else 0 for s, on in zip(seq, live)]
+        hb = oracle.HostBatch(aq, lens, bt, context_lens_before=[max(0, s - 1) for s in lens],
+                              valid_req_mask=live.astype(np.uint8) if masked else None)
+        want = oracle.paged_attention(pool, hb, q, DT_F16, 32)
+        rc, got, _ = G.dev_attention(dpool, hb, q, DT_F16, 32, scratch_bytes=64 << 20, max_seq_len=max(seq))
+        assert rc == 0
+        assert (got[~live] == (0x5500 if masked else 0)).all()
+        if live.any():
+            full = oracle.HostBatch(aq, seq, bt, context_lens_before=ctx)
+            G.assert_close(got[live], DT_F16, want[live], what="fmt=%d reqs=%d idle=%d" % (fmt, reqs, idle),
+                           scale=G.channel_scale(v, DT_F16, full, 32)[live], plain_excess=4e-4)

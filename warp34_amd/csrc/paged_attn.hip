@@ -129,10 +129,6 @@ struct AttnParams {
         struct {
             int short_units, short_tiles, short_tok_tile;
         };
-        // balanced decode: the chunk grid's cap on chunks per request, for batches it may serve (grid_decode_units); 0: none
-        struct {
-            int grid_chunks;
-        };
     };
     // Partial records: part_stride slots per output row.  Slots [0, max_chunks) belong to the
     // split-K chunks of the decode kernels; a shared-prefix pass (tile kernel over the keys every
@@ -145,6 +141,9 @@ struct AttnParams {
     // 32) and both page strides fit 32 bits, so a unit's four runs follow from ONE block-table entry
     // and two 32 x 32-bit products
     int unit_in_page;
+    // Balanced decode: the chunk grid's cap on chunks per request, for batches it may serve (grid_decode_units); 0: none.  (A word of its own: a
+    // launch may take a kernel that reads short_units.)
+    int grid_chunks;
 };
 
 // A finished output row leaves the kernels here: lane l holds channels 4 l .. 4 l + 3.  With a gate
@@ -2239,7 +2238,6 @@ static bool balanced_decode_applicable(const warp34_exec* ex, const warp34_atten
     return tiles_by_request && batch->num_reqs >= 2 && !force_single && batch->sliding_window <= 0 &&
            batch->valid_token_mask == nullptr && batch->total_tokens <= 65535 && ex->scratch_ptr != 0 && (ex->scratch_ptr & 15u) == 0u;
 }
-// shares of a balanced decode batch per (kv head, q subgroup): a function of gqa only
 // The chunk grid's cap on chunks per request of a decode batch that it may serve in the plan's place (grid_decode_units): one round of
 // workgroups; 0: not such a batch.
 static int decode_grid_chunks(const warp34_exec* ex, const warp34_attention_batch* batch, int num_q_heads, int q_subgroups) {
@@ -2251,6 +2249,7 @@ static bool decode_on_grid(const warp34_attention_batch* batch, int chunks) {
     return chunks > 0 && batch->max_seq_len > 0 &&
            ((long long)batch->max_seq_len + kUnit - 1) / kUnit * batch->num_reqs <= grid_decode_units(batch->num_reqs);
 }
+// shares of a balanced decode batch per (kv head, q subgroup): a function of gqa only
 static int balanced_groups(int q_subgroups) {
     int groups = kTargetWorkgroupsPerHead / (q_subgroups > 0 ? q_subgroups : 1);
     if (groups > kMergeGroups * kMergeMaxPerGroup - 1) groups = kMergeGroups * kMergeMaxPerGroup - 1;
