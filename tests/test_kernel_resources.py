@@ -13,12 +13,12 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 READELF = "/opt/rocm/llvm/bin/llvm-readelf"
 
 
-def kernel_scratch_bytes(tmp_path):
-    """{kernel name: bytes of scratch memory per lane} of the gfx950 code objects inside the library."""
+def code_objects(tmp_path):
+    """Paths of the gfx950 code objects inside the library."""
     from warp34_amd import ffi
 
     data = open(ffi.LIB_PATH, "rb").read()
-    found, at, n = {}, data.find(b"__CLANG_OFFLOAD_BUNDLE__"), 0
+    paths, at = [], data.find(b"__CLANG_OFFLOAD_BUNDLE__")
     while at >= 0:
         pos = at + 32
         for _ in range(struct.unpack_from("<Q", data, at + 24)[0]):
@@ -27,14 +27,35 @@ def kernel_scratch_bytes(tmp_path):
             pos += 24 + name_len
             if b"gfx950" not in triple or not size:
                 continue
-            path = os.path.join(str(tmp_path), "%d.o" % n)
-            n += 1
-            with open(path, "wb") as f:
+            paths.append(os.path.join(str(tmp_path), "%d.o" % len(paths)))
+            with open(paths[-1], "wb") as f:
                 f.write(data[at + offset:at + offset + size])
-            notes = subprocess.run([READELF, "--notes", path], stdout=subprocess.PIPE, text=True, check=True).stdout
-            for name, scratch in re.findall(r"\.name: +(_Z\S+)\n(?:.*\n)*?.*\.private_segment_fixed_size: (\d+)", notes):
-                found[name] = int(scratch)
         at = data.find(b"__CLANG_OFFLOAD_BUNDLE__", at + 24)
+    return paths
+
+
+def readelf(*args):
+    return subprocess.run([READELF, *args], stdout=subprocess.PIPE, text=True, check=True).stdout
+
+
+def kernel_scratch_bytes(tmp_path):
+    """{kernel name: bytes of scratch memory per lane}"""
+    found = {}
+    for path in code_objects(tmp_path):
+        for name, scratch in re.findall(r"\.name: +(_Z\S+)\n(?:.*\n)*?.*\.private_segment_fixed_size: (\d+)", readelf("--notes", path)):
+            found[name] = int(scratch)
+    return found
+
+
+def kernel_preload_dwords(tmp_path):
+    """{kernel name: dwords of its arguments that are in scalar registers when a wave starts}"""
+    found = {}
+    for path in code_objects(tmp_path):
+        data = open(path, "rb").read()
+        text = readelf("--sections", "--symbols", "--wide", path)
+        addr, offset = (int(x, 16) for x in re.search(r"\.rodata +PROGBITS +(\w+) +(\w+)", text).groups())
+        for value, name in re.findall(r"^ *\d+: (\w+) +64 OBJECT .* (\S+)\.kd$", text, re.M):
+            found[name] = struct.unpack_from("<H", data, int(value, 16) - addr + offset + 58)[0] & 127  # kernarg_preload_spec_length
     return found
 
 
@@ -50,6 +71,16 @@ def test_prefill_kernels_do_not_spill(tmp_path):
     kernels = {k: v for k, v in kernel_scratch_bytes(tmp_path).items() if "paged_prefill" in k}
     assert len(kernels) >= 16, sorted(kernels)
     assert {k: v for k, v in kernels.items() if v} == {}
+
+
+@pytest.mark.skipif(not os.path.exists(READELF), reason="no llvm-readelf")
+@pytest.mark.parametrize("part,dwords", [("kv_append_kernel", 14), ("fused_qk_norm_rope_gate_kernel", 13), ("qk_norm_rope_kernel", 14),
+                                         ("balanced_merge_kernel", 10), ("split_merge_few_kernel", 6), ("qsa_sparse_", 11)])
+def test_leading_arguments_are_preloaded(tmp_path, part, dwords):
+    """Kernels whose first requests wait for nothing but their arguments."""
+    kernels = {k: v for k, v in kernel_preload_dwords(tmp_path).items() if part in k and (part != "qk_norm_rope_kernel" or "fused" not in k)}
+    assert kernels
+    assert {k: v for k, v in kernels.items() if v < dwords} == {}
 
 
 def assembly(tmp_path, source):

@@ -26,9 +26,9 @@ PRELOAD = ["-mllvm", "-amdgpu-kernarg-preload-count=14"]
 SOURCES = [
     # (path, extra flags)
     (os.path.join(CSRC, "kv_write.hip"), ["-ffp-contract=off"] + PRELOAD),
-    (os.path.join(CSRC, "qk_norm_rope.hip"), ["-ffp-contract=off"]),
+    (os.path.join(CSRC, "qk_norm_rope.hip"), ["-ffp-contract=off"] + PRELOAD),
     (os.path.join(CSRC, "attn_output_gate.hip"), ["-ffp-contract=off"]),
-    (os.path.join(CSRC, "fused_qk_norm.hip"), ["-ffp-contract=off"]),
+    (os.path.join(CSRC, "fused_qk_norm.hip"), ["-ffp-contract=off"] + PRELOAD),
     (os.path.join(CSRC, "paged_attn.hip"), PRELOAD),
     (os.path.join(CSRC, "runtime.hip"), []),
     (os.path.join(HOST, "kv_host.cpp"), []),

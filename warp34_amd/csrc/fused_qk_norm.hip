@@ -91,7 +91,8 @@ struct FqPacked {
 };
 // A small batch is a chain of memory round trips.  The leading arguments are in scalar registers when a wave starts: the sine / cosine
 // values and the K / V items, the longest parts, ask for their data at once instead of behind the argument block; slot and
-// block arrive meanwhile, and what an item's end uses is requested with its row.
+// block arrive meanwhile, and what an item's end uses is requested with its row.  (us, 16 + 2 heads, arguments loaded / preloaded:
+// TQ4 1 token 3.40 / 3.35, 512 7.39 / 7.19, 8 192 60.1 / 59.9; FP16 512 6.69 / 6.36; 32 + 4 heads, FP8, 256 tokens 7.87 / 7.58.)
 // heads: q heads, kv heads, head size; rot: rotary pairs, sections 1 and 2 of the three position planes
 // ROTATED_TQ4: pages of that kind only.  ANY: angles above 2^31 (a base below 1), head counts that `heads` cannot hold.
 template <bool SPREAD, bool ROTATED_TQ4, bool ANY>
