@@ -42,11 +42,12 @@ def test_lengths_at_which_the_chunks_change(fmt, dtype, head_dim, units):
 
 @pytest.mark.parametrize("fmt,dtype,xf", [(FMT_TQ4, DT_BF16, None), (FMT_Q8_0, DT_F16, XF_IDENTITY), (FMT_Q8_0, DT_F16, XF_WHT256),
                                           (FMT_FP16, DT_F16, None)])
-@pytest.mark.parametrize("reqs,longest", [(2, 1024), (2, 1025), (16, 128), (16, 129), (17, 180), (17, 181), (64, 48), (64, 49), (65, 20)])
+@pytest.mark.parametrize("reqs,longest", [(2, 1024), (2, 1025), (16, 128), (16, 129), (17, 180), (17, 181), (64, 48), (64, 49), (65, 20),
+                                            (2, 512), (2, 513), (12, 80), (12, 81), (16, 64), (16, 65), (17, 120), (17, 121), (64, 32), (64, 33)])
 def test_decode_batches_on_either_side_of_the_grid_rule(fmt, dtype, xf, reqs, longest):
     """Chunk grid and plan give the same bytes for a batch that the chunk grid may serve: which of them runs follows from the host's bound on
-    the lengths (units of the longest request times requests: 2 048, from 17 requests on 3 072).  A request without a key and a
-    masked one among the others."""
+    the lengths (units of the longest request: 8 x (128 / requests); from 17 requests on, times requests, 3 072, row formats 2 048).  A
+    masked request among the others."""
     import gpu_harness as G
 
     rng = np.random.default_rng(reqs * 1000 + longest)

@@ -94,3 +94,21 @@ def test_kernels_of_the_plan_get_the_numbers_that_they_read(recorder):
             else:
                 assert grid_chunks == 0 or (q_subgroups == 1 and 1 < grid_chunks and grid_chunks * c["reqs"] <= grid), (c, name)
     assert len(seen) == 4
+
+
+def test_short_decode_batches_on_the_grid_keep_the_chunks_of_the_plan(recorder):
+    """Up to 16 requests a batch runs on the chunk grid only where the cap leaves the longest request chunks of eight units, the plan's least; with more
+    requests up to 3 072 units (row formats: 2 048) for all of them at the longest one's length."""
+    units = (1, 8, 40, 42, 43, 48, 49, 62, 63, 64, 65, 72, 73, 80, 81, 120, 121, 180, 181, 256, 257, 512, 513, 1024)
+    cases = [case(fmt, reqs, 1, 32 * u, xf=xf) for fmt, xf in (("tq4", 1), ("q8_0", 0), ("fp8", 1), ("bf16", 0))
+             for reqs in (2, 4, 12, 13, 14, 16, 17, 33, 48, 64, 65) for u in units]
+    for c, (_, (run,)) in zip(cases, recorder(cases)):
+        u = c["max_seq"] // 32
+        if c["reqs"] <= 16:
+            grid = u <= 8 * (128 // c["reqs"])
+        else:
+            grid = c["reqs"] <= 64 and u * c["reqs"] <= (3072 if c["fmt"] == "tq4" else 2048)
+        assert ("balanced_kernel" not in run[0][0]) == grid, c
+        if grid and c["reqs"] <= 16:
+            shape = run[0][1]
+            assert shape[0] * 8 >= u, c

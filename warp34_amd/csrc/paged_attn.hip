@@ -141,7 +141,7 @@ struct AttnParams {
     // 32) and both page strides fit 32 bits, so a unit's four runs follow from ONE block-table entry
     // and two 32 x 32-bit products
     int unit_in_page;
-    // Balanced decode: the chunk grid's cap on chunks per request, for batches it may serve (grid_decode_units); 0: none.  (A word of its own: a
+    // Balanced decode: the chunk grid's cap on chunks per request, for batches it may serve (grid_decode_serves); 0: none.  (A word of its own: a
     // launch may take a kernel that reads short_units.)
     int grid_chunks;
 };
@@ -465,15 +465,23 @@ __host__ __device__ __forceinline__ size_t bal_partial_row(int slot, int kv_subs
     return ((size_t)slot * kv_subs + kv_sub) * cols + col;
 }
 
-// A decode batch (kGridDecodeReqs requests at most, one q subgroup) whose longest request times the number of requests is at most this
-// many units is cut as the chunk grid cuts it, 128 / requests chunks each at most, and the chunk grid runs instead of the plan where the host's
-// bound on the lengths says as much: the plan and the merge's table cost 2 to 3 us of a call, one request's chunks being longer
-// than a share costs less.  us a layer, attention alone, plan / chunk grid: TQ4, 2 requests of 1 600 to 16 000 keys 16.1 / 14.2, 8 of 400 to 4 000
-// 15.4 / 13.2, 16 of 400 to 4 000 17.4 / 15.2, 32 of 200 to 2 000 18.2 / 16.2, 32 of 300 to 3 000 25.0 / 18.8; Q8_0, 8 of 400 to 4 000 14.0 / 12.6, 24 of
-// 266 to 2 666 20.1 / 18.2.  Beyond the line, lengths from a tenth up: 10 of up to 9 600 TQ4 18.7 / 19.7, Q8_0 20.3 / 21.8, 12 of up to 10 666 23.1 /
-// 25.3.  More than 16 requests (shares that cross from one into the next): later, 48 of up to 2 000 TQ4 25.0 / 20.6, Q8_0 23.3 / 24.0.
-constexpr int kGridDecodeReqs = 64;
-__host__ __device__ constexpr int grid_decode_units(int reqs) { return reqs <= 16 ? 2048 : 3072; }
+// A decode batch (kGridDecodeReqs requests at most, one q subgroup) whose longest request is at most this many units is cut as the chunk grid cuts
+// it, 128 / requests chunks each at most, and the chunk grid runs instead of the plan where the host's bound on the lengths says as
+// much: the plan and the merge's table cost 2 to 3 us of a call.  Under a looser bound the plan runs and cuts the same way.  So a batch must not
+// lose by the cut, whatever its lengths are:
+// - Up to 16 requests (kAlignedReqs) the plan would cut a long request among short ones into pieces of kMinUnitsPerChunk.  A chunk is no longer
+//   than that while the cap does not bind.  us a layer, attention alone, plan's own cut / this cut under the exact bound / under a loose one,
+//   one long request and the others of one unit: TQ4 16 of up to 64 units 14.3 / 11.9 / 13.5, 12 of 80 14.3 / 12.0 / 13.7, 12 of 85 (ten chunks of nine
+//   units) 14.3 / 14.1 / 15.5, 16 of 128 14.6 / 14.6 / 16.3; Q8_0 16 of 64 13.8 / 12.5 / 13.3, of 128 14.4 / 16.1 / 17.2; BF16 4 of 256 15.4 / 14.1 / 15.3, of
+//   512 16.8 / 19.0 / 20.3.  All of the same length: TQ4 16 of 64 15.9 / 13.1 / 14.6, of 128 19.2 / 16.4 / 17.8, BF16 16 of 64 19.7 / 17.7 / 18.9.
+// - With more requests the plan's shares cross from one into the next, which costs it 5 us more: `many` units in all.  TQ4 24 of 128, one long
+//   23.7 / 18.7 / 20.4, all 26.0 / 21.0 / 22.3, 64 of 48 23.9 / 17.1 / 18.3.  Row formats turn earlier: BF16 33 of 62 22.5 / 18.8 / 20.3, of 77 22.6 / 21.6 / 23.2,
+//   48 of 53 22.4 / 22.3 / 23.8; Q8_0 48 of 42 21.1 / 18.1 / 19.2, of 53 21.1 / 20.8 / 22.0.
+constexpr int kGridDecodeReqs = 64, kAlignedReqs = 16;
+constexpr int kGridUnitsTq4 = 3072, kGridUnitsRows = 2048;  // many
+__host__ __device__ constexpr bool grid_decode_serves(long long longest, int reqs, int chunks, int many) {
+    return reqs <= kAlignedReqs ? longest <= (long long)kMinUnitsPerChunk * chunks : longest * reqs <= many;
+}
 
 struct BalReq {  // entry base + lane of a group of 64
     int lo, hi;          // query tokens of the request
@@ -1609,8 +1617,8 @@ __device__ __forceinline__ void bal_short_piece(const AttnParams& P, TileFn&& ti
 // loads are the same addresses in every wave of the chip and stay in cache) and calls
 // tile(piece) for the pieces of its workgroup's share, in order.
 // SHORT: a batch that turns out short is left to short_batch().
-// FEW: chunk_count's line for the format.
-template <bool SHORT, int FEW, typename TileFn, typename ShortFn>
+// FEW, MANY: chunk_count's and grid_decode_serves' lines for the format.
+template <bool SHORT, int FEW, int MANY, typename TileFn, typename ShortFn>
 __device__ __forceinline__ void bal_for_each_piece(const AttnParams& P, TileFn&& tile, ShortFn&& short_batch) {
     const int lane = (int)threadIdx.x & 63;
     const int entries = P.B.num_reqs * P.bal_tiles;
@@ -1651,7 +1659,7 @@ __device__ __forceinline__ void bal_for_each_piece(const AttnParams& P, TileFn&&
     int share = 1;
     // a batch that the chunk grid serves where the host's bound says so: its chunks, so that the bits do not depend on the bound
     bool as_grid = false;
-    if constexpr (!SHORT) as_grid = P.grid_chunks > 0 && __ballot(q0.units * P.B.num_reqs > grid_decode_units(P.B.num_reqs)) == 0ull;
+    if constexpr (!SHORT) as_grid = P.grid_chunks > 0 && __ballot(!grid_decode_serves(q0.units, P.B.num_reqs, P.grid_chunks, MANY)) == 0ull;
     const bool aligned = P.bal_aligned || as_grid;
     if (aligned) {  // uniform for the grid; at most 64 entries
         // Units per piece: the smallest count found by a few steps from below for which the pieces fit
@@ -1766,7 +1774,7 @@ __global__ __launch_bounds__(kTq4Waves * 64, 1) void paged_attn_tq4_balanced_ker
         tq4_tile<TQ, true>(P, smem, it, first);
         first = false;
     };
-    bal_for_each_piece<false, kFewChunksTq4>(P, piece, [] {});
+    bal_for_each_piece<false, kFewChunksTq4, kGridUnitsTq4>(P, piece, [] {});
 }
 
 // One wave adds up the slices of a row's n_chunks chunks (at most SLOTS; lane s holds the record of chunk s), in the order in which ORDER waves
@@ -2238,16 +2246,16 @@ static bool balanced_decode_applicable(const warp34_exec* ex, const warp34_atten
     return tiles_by_request && batch->num_reqs >= 2 && !force_single && batch->sliding_window <= 0 &&
            batch->valid_token_mask == nullptr && batch->total_tokens <= 65535 && ex->scratch_ptr != 0 && (ex->scratch_ptr & 15u) == 0u;
 }
-// The chunk grid's cap on chunks per request of a decode batch that it may serve in the plan's place (grid_decode_units): one round of
+// The chunk grid's cap on chunks per request of a decode batch that it may serve in the plan's place (grid_decode_serves): one round of
 // workgroups; 0: not such a batch.
 static int decode_grid_chunks(const warp34_exec* ex, const warp34_attention_batch* batch, int num_q_heads, int q_subgroups) {
     if (q_subgroups != 1 || batch->num_reqs < 2 || batch->num_reqs > kGridDecodeReqs) return 0;
     const int chunks = kTargetWorkgroupsPerHead / batch->num_reqs;
     return partial_bytes((long long)batch->total_tokens * num_q_heads, chunks) <= ex->scratch_size ? chunks : 0;
 }
-static bool decode_on_grid(const warp34_attention_batch* batch, int chunks) {
+static bool decode_on_grid(const warp34_attention_batch* batch, int chunks, int many) {
     return chunks > 0 && batch->max_seq_len > 0 &&
-           ((long long)batch->max_seq_len + kUnit - 1) / kUnit * batch->num_reqs <= grid_decode_units(batch->num_reqs);
+           grid_decode_serves(((long long)batch->max_seq_len + kUnit - 1) / kUnit, batch->num_reqs, chunks, many);
 }
 // shares of a balanced decode batch per (kv head, q subgroup): a function of gqa only
 static int balanced_groups(int q_subgroups) {
@@ -2468,7 +2476,7 @@ static int launch_tq4(const warp34_exec* ex, const warp34_kv_layer_layout* layou
     const bool plan = balanced_decode_applicable(ex, batch, P.tiles_by_request, force_single) &&
                       partial_bytes((long long)plan_rows, 1) + (size_t)batch->total_tokens * 16 <= ex->scratch_size;
     const int decode_chunks = plan ? decode_grid_chunks(ex, batch, num_q_heads, P.q_subgroups) : 0;
-    const bool on_grid = decode_on_grid(batch, decode_chunks);
+    const bool on_grid = decode_on_grid(batch, decode_chunks, kGridUnitsTq4);
     P.max_chunks = force_single ? 1
                    : on_grid    ? decode_chunks
                                 : choose_max_chunks(ex, batch->total_tokens, num_q_heads, P.tok_tile, P.q_subgroups);
@@ -2646,7 +2654,7 @@ static int launch_rows_balanced(const warp34_exec* ex, const warp34_attention_ba
     P.short_units = -1;
     if (HD == kHeadDim && nt * tiles == 1 && groups == all_groups) {
         const int chunks = decode_grid_chunks(ex, batch, P.num_q_heads, P.q_subgroups);
-        if (decode_on_grid(batch, chunks)) {
+        if (decode_on_grid(batch, chunks, kGridUnitsRows)) {
             *grid_chunks = chunks;
             return -1;
         }

@@ -964,7 +964,7 @@ __global__ __launch_bounds__(kKv16Waves * 64, 1) void paged_attn_rows_mapped_ker
 template <typename TQ, int NT, int KVF, bool VRES, bool STREAM, int HD = kHeadDim>
 __global__ __launch_bounds__(kKv16Waves * 64, 1) void paged_attn_rows_balanced_kernel(const AttnParams P) {
     extern __shared__ __align__(16) uint8_t smem[];
-    bal_for_each_piece<(NT > 1 || (VRES && !STREAM)), kFewChunksRows>(
+    bal_for_each_piece<(NT > 1 || (VRES && !STREAM)), kFewChunksRows, kGridUnitsRows>(
         P, [&](const BalItem& it) { rows_tile<TQ, NT, KVF, true, VRES, STREAM, HD>(P, smem, it); },
         [&] {
             const AttnParams A = kernel_params_again();
