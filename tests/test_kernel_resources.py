@@ -74,6 +74,14 @@ def test_prefill_kernels_do_not_spill(tmp_path):
 
 
 @pytest.mark.skipif(not os.path.exists(READELF), reason="no llvm-readelf")
+def test_sparse_kernels_do_not_spill(tmp_path):
+    """Two registers of the Q8_0 form with rotated values excepted, which is faster with them there."""
+    kernels = {k: v for k, v in kernel_scratch_bytes(tmp_path).items() if "qsa_sparse" in k}
+    assert len(kernels) == 7, sorted(kernels)
+    assert {k: v for k, v in kernels.items() if v > (12 if "rows_kernelILi3ELb1E" in k else 0)} == {}
+
+
+@pytest.mark.skipif(not os.path.exists(READELF), reason="no llvm-readelf")
 @pytest.mark.parametrize("part,dwords", [("kv_append_kernel", 14), ("fused_qk_norm_rope_gate_kernel", 13), ("qk_norm_rope_kernel", 14),
                                          ("balanced_merge_kernel", 10), ("split_merge_few_kernel", 6), ("qsa_sparse_", 11)])
 def test_leading_arguments_are_preloaded(tmp_path, part, dwords):

@@ -159,9 +159,15 @@ __global__ __launch_bounds__(kKv16Waves * 64, 1) void qsa_sparse_rows_kernel(QSA
     auto commit_half = [&](int pos_vec, bool edge) {
         uint8_t* k_rows = stage;
         uint8_t* v_rows = stage + 16 * kRowStride;
+        int at = lane;
+        // (FP8: rows and columns of the pieces are worked out for each half; kept across the loop, they put 25 registers into scratch
+        // memory.  us a call, 513 groups, kept / now: 1 token 14.8 / 14.0, 16 21.0 / 17.9, 64 36.9 / 33.6, 16 with 200 groups 14.8 / 12.6; rotated
+        // rows 16 20.4 / 19.2.  Q8_0 rows have one division, which costs more than the registers: 16 18.0 / 18.5,
+        // with rotated values, where two of them are in scratch memory, 19.8 / 20.3.)
+        if constexpr (FP8) asm volatile("" : "+v"(at));
 #pragma unroll
         for (int i = 0; i < kLoads; ++i) {
-            const int c = lane + 64 * i;
+            const int c = at + 64 * i;
             if (kPieces % 64 != 0 && c >= kPieces) break;
             u4 kv = pf[i], vv = pf[kLoads + i];
             if constexpr (FP8) {
