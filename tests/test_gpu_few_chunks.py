@@ -1,5 +1,7 @@
 """Contexts and batches of few chunks: shorter chunks, and a merge of one wave per row, against the oracle at the lengths where the number of chunks and
 the form of the merge change; and, with a bound on the length under which the merge of several waves runs, the same bytes."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -38,6 +40,24 @@ def test_lengths_at_which_the_chunks_change(fmt, dtype, head_dim, units):
                        scale=G.channel_scale(v, dtype, hb, q_heads)[live])
         rc, wide, _ = G.dev_attention(dpool, hb, q, dtype, q_heads, scratch_bytes=SCRATCH, max_seq_len=131072)
         assert rc == 0 and wide.tobytes() == got.tobytes()
+
+
+@pytest.mark.parametrize("fmt,dtype", [(FMT_TQ4, DT_BF16), (FMT_Q8_0, DT_F16)])
+@pytest.mark.parametrize("q_len,seq", [(1, 300), (1, 1200), (4, 1200), (4, 5000), (1, 9000)])
+def test_queried_scratch_gives_the_bytes_of_a_large_one(fmt, dtype, q_len, seq):
+    import gpu_harness as G
+
+    pool, bt, k, v, q, aq, ctx = make_case(fmt, 64, [seq], [q_len], 2600 + seq, dtype)
+    hb = oracle.HostBatch(aq, [seq], bt, context_lens_before=ctx)
+    dpool = G.DevPool(pool)
+    dpool.upload()
+    need = G.lib().warp34_paged_attention_scratch_bytes_for_layout(C.byref(dpool.layout()), q_len, 1, 16, seq)
+    outs = []
+    for scratch in (need, SCRATCH):
+        rc, got, _ = G.dev_attention(dpool, hb, q, dtype, 16, scratch_bytes=scratch, max_seq_len=seq)
+        assert rc == 0
+        outs.append(got.tobytes())
+    assert outs[0] == outs[1]
 
 
 @pytest.mark.parametrize("fmt,dtype,xf", [(FMT_TQ4, DT_BF16, None), (FMT_Q8_0, DT_F16, XF_IDENTITY), (FMT_Q8_0, DT_F16, XF_WHT256),

@@ -112,3 +112,14 @@ def test_short_decode_batches_on_the_grid_keep_the_chunks_of_the_plan(recorder):
         if grid and c["reqs"] <= 16:
             shape = run[0][1]
             assert shape[0] * 8 >= u, c
+
+
+def test_queried_scratch_gives_the_launches_of_a_large_one(recorder):
+    """What the size query answers is what the launchers want: same kernels, grids and numbers of chunks as with 64 MiB."""
+    cases = [case(fmt, reqs, q_len, max_seq, q_heads, kv_heads, head_dim, xf, scratch=("queried", 64 << 20))
+             for fmt, xf, q_heads, kv_heads, head_dim in (("tq4", 1, 16, 2, 256), ("tq4", 1, 32, 4, 256), ("q8_0", 0, 16, 2, 256), ("q8_0", 1, 8, 1, 256),
+                                                          ("fp8", 0, 32, 1, 256), ("bf16", 0, 16, 2, 256), ("bf16", 0, 16, 4, 128))
+             for reqs, q_len in ((1, 1), (1, 2), (1, 4), (1, 7), (1, 16), (2, 1), (3, 4), (16, 1), (40, 1))
+             for max_seq in (1, 100, 224, 257, 600, 768, 769, 1000, 1200, 2500, 5000, 6144, 8192, 8193, 10000, 32000, 131072)]
+    for c, (need, (queried, large)) in zip(cases, recorder(cases)):
+        assert queried == large, (c, need)

@@ -36,9 +36,9 @@ def query(tokens, reqs, max_seq, fmt="tq4", q_heads=16, kv_heads=2, head_dim=256
 
 @pytest.mark.parametrize("fmt", ["tq4", "q8_0"])
 def test_request_counts_outside_the_batch(fmt):
-    """4 tokens, 16 query rows per kv head: five chunks of a request of 1000 keys fit their minimum of 8 units, no
+    """4 tokens, 16 query rows per kv head: a request of 1000 keys (33 units counted) has nine chunks of four units, no
     request means no plan; a negative count and one above the tokens stand for one token per request."""
-    assert query(4, 0, 1000, fmt) == 4 * 16 * 5 * RECORD
+    assert query(4, 0, 1000, fmt) == 4 * 16 * 9 * RECORD
     assert query(4, -1, 1000, fmt) == query(4, 4, 1000, fmt) == query(4, 9, 1000, fmt)
 
 
@@ -65,8 +65,8 @@ def test_decode_batches_of_every_format_and_verify_batches_of_row_formats():
     for fmt in ("tq4", "q8_0", "bf16"):
         assert query(32, 32, 30000, fmt) == plan(32, 32)
         assert query(32, 16, 30000, fmt) == max(plan(32, 16), chunks(32, 8))
-    assert query(4, 4, 2000, "bf16", q_heads=4, kv_heads=2, head_dim=128) == max(plan(4, 4), chunks(4, 8, 4))
-    assert query(3, 3, 2000, "bf16", q_heads=4, kv_heads=2, head_dim=128) == chunks(3, 8, 4)
+    assert query(4, 4, 2000, "bf16", q_heads=4, kv_heads=2, head_dim=128) == max(plan(4, 4), chunks(4, 16, 4))
+    assert query(3, 3, 2000, "bf16", q_heads=4, kv_heads=2, head_dim=128) == chunks(3, 16, 4)
     for fmt in ("q8_0", "fp8", "bf16", "fp16"):
         assert query(20, 5, 21000, fmt) == plan(20, 5, 32)
         assert query(64, 16, 262144, fmt) == plan(64, 16, 32)

@@ -2182,18 +2182,25 @@ static size_t partial_bytes(long long rows, int max_chunks) {
     return (size_t)rows * (size_t)max_chunks * (kHeadDim + 4) * sizeof(float);
 }
 
-// Cap on chunks per tile: a function of total_tokens (tiles), gqa (q subgroups per kv head) and
-// the scratch size only.
-static int choose_max_chunks(const warp34_exec* ex, int total_tokens, int num_q_heads, int tok_tile,
-                             int q_subgroups) {
+// Cap on chunks per tile: a function of total_tokens (tiles), gqa (q subgroups per kv head) and, with too little of it, the scratch and
+// the heads.  Then as many as it holds and the chip takes in one round (two kv heads: all), so that scratch for n chunks gives n, or the
+// target halved until it fits.  us, scratch by the size query, halved / now: one token of 16 + 2 heads, 1 200 keys, TQ4 13.3 / 11.2 (eight of ten chunks), Q8_0
+// 12.4 / 10.7, 10 000 keys TQ4 15.2 / 12.9 (64 of 79).  What halving is for: 8 MiB, 4 tokens of 32 + 4 heads on 32 000 keys, 63 chunks / 32: TQ4 35.6 / 26.8,
+// Q8_0 35.6 / 28.6; 64 + 8 heads, 31 / 16: 48.6 / 36.0.
+static long long one_round(long long tiles, int kv_subs) { return 2 * kTargetWorkgroupsPerHead / (tiles * kv_subs); }
+static int choose_max_chunks(const warp34_exec* ex, int total_tokens, int num_q_heads, int tok_tile, int q_subgroups, int kv_subs) {
     if (ex->scratch_ptr == 0 || (ex->scratch_ptr & 15u) != 0u) return 1;
     const int tiles = (total_tokens + tok_tile - 1) / tok_tile;
     const long long per_chunk = (long long)(tiles > 0 ? tiles : 1) * (q_subgroups > 0 ? q_subgroups : 1);
     int want = (int)(kTargetWorkgroupsPerHead / per_chunk);
     if (want > kMaxChunksCap) want = kMaxChunksCap;
     if (want < 2) return 1;
-    const long long rows = (long long)total_tokens * num_q_heads;
-    while (want > 1 && partial_bytes(rows, want) > ex->scratch_size) want >>= 1;
+    const size_t one = partial_bytes((long long)total_tokens * num_q_heads, 1);
+    if (one > 0 && ex->scratch_size / one < (size_t)want) {
+        const int fit = (int)(ex->scratch_size / one);
+        while (want > fit) want >>= 1;
+        want = std::max(want, (int)std::min<long long>(fit, one_round(tiles, kv_subs)));
+    }
     return want < 2 ? 1 : want;
 }
 
@@ -2479,7 +2486,7 @@ static int launch_tq4(const warp34_exec* ex, const warp34_kv_layer_layout* layou
     const bool on_grid = decode_on_grid(batch, decode_chunks, kGridUnitsTq4);
     P.max_chunks = force_single ? 1
                    : on_grid    ? decode_chunks
-                                : choose_max_chunks(ex, batch->total_tokens, num_q_heads, P.tok_tile, P.q_subgroups);
+                                : choose_max_chunks(ex, batch->total_tokens, num_q_heads, P.tok_tile, P.q_subgroups, kv_subs);
     P.part_acc = nullptr;
     P.part_ml = nullptr;
     const long long rows = (long long)batch->total_tokens * num_q_heads;
@@ -2639,7 +2646,7 @@ static int launch_rows_balanced(const warp34_exec* ex, const warp34_attention_ba
     const int tok16 = 16 / P.q_group, tiles16 = (batch->max_q_len + tok16 - 1) / tok16;
     if (groups < 1 || (4 * groups < 3 * all_groups &&
                        groups < (long long)batch->num_reqs * tiles16 *
-                                    choose_max_chunks(ex, batch->total_tokens, P.num_q_heads, tok16, P.q_subgroups)))
+                                    choose_max_chunks(ex, batch->total_tokens, P.num_q_heads, tok16, P.q_subgroups, kv_subs)))
         return -1;
     const size_t prows = (size_t)(groups + entries) * kv_subs * 16 * nt;
     P.piece_cost = kRowsPieceCost;
@@ -2767,7 +2774,7 @@ static int launch_rows(const warp34_exec* ex, const warp34_kv_layer_layout* layo
     if (rc >= 0) return rc;
     P.max_chunks = force_single        ? 1
                    : decode_chunks > 0 ? decode_chunks
-                                       : choose_max_chunks(ex, batch->total_tokens, num_q_heads, P.tok_tile, P.q_subgroups);
+                                       : choose_max_chunks(ex, batch->total_tokens, num_q_heads, P.tok_tile, P.q_subgroups, kv_subs);
     P.part_acc = nullptr;
     P.part_ml = nullptr;
     const long long rows = (long long)batch->total_tokens * num_q_heads;
@@ -3193,6 +3200,7 @@ static size_t scratch_bytes_for(const warp34_kv_layer_layout* layout, int total_
     if (total_tokens <= 0 || num_q_heads <= 0) return 0;
     int q_group = 1, q_subgroups = 1, kv_subs = num_q_heads;  // the bound when the layout is unknown
     int tok_tile = 16;
+    const int few = layout && is_tq4(layout) ? kFewChunksTq4 : kFewChunksRows;  // (the larger one when the layout is unknown)
     if (layout && layout->local_kv_heads > 0 && num_q_heads % layout->local_kv_heads == 0) {
         const int gqa = num_q_heads / layout->local_kv_heads;
         q_group = gqa;
@@ -3212,8 +3220,15 @@ static size_t scratch_bytes_for(const warp34_kv_layer_layout* layout, int total_
     if (want > kMaxChunksCap) want = kMaxChunksCap;
     if (max_seq_len > 0) {
         const int units = (max_seq_len + kUnit - 1) / kUnit + 1;
-        const int bound = (units + kMinUnitsPerChunk - 1) / kMinUnitsPerChunk;
-        if (bound < want) want = bound;
+        const long long full = want;
+        want = std::min<long long>(want, chunk_count(units, (units + kMinUnitsPerChunk - 1) / kMinUnitsPerChunk, few));
+        // (the first of full, full / 2, ... that is enough is at most 2 want - 1)
+        if (!layout) want = std::min(full, 2 * want - 1);
+        else if (want > one_round(tiles, kv_subs)) {
+            long long halved = full;
+            while (halved / 2 >= want) halved /= 2;
+            want = halved;
+        }
     }
     size_t bytes = want >= 2 ? partial_bytes((long long)total_tokens * num_q_heads, (int)want) : 0;
     // TQ4 verify batches over long contexts may take the shared-prefix pass: its partial slots sit
