@@ -123,3 +123,14 @@ def test_queried_scratch_gives_the_launches_of_a_large_one(recorder):
              for max_seq in (1, 100, 224, 257, 600, 768, 769, 1000, 1200, 2500, 5000, 6144, 8192, 8193, 10000, 32000, 131072)]
     for c, (need, (queried, large)) in zip(cases, recorder(cases)):
         assert queried == large, (c, need)
+
+
+def test_merge_of_one_wave_up_to_sixteen_chunks(recorder):
+    cases = [case(fmt, 1, q_len, 32 * units) for fmt in ("tq4", "q8_0", "bf16") for q_len in (1, 2, 4, 8) for units in range(8, 300, 7)]
+    forms = set()
+    for c, (_, (run,)) in zip(cases, recorder(cases)):
+        if len(run) == 2:
+            name, (_, _, _, _, slots), _ = run[1]
+            assert ("split_merge_few_kernel" in name) == (slots <= 16), (c, name, slots)
+            forms.add(slots <= 16)
+    assert len(forms) == 2

@@ -436,7 +436,10 @@ __device__ __forceinline__ constexpr int tq4_pv_elem(int h, int j, int r) {
 // Smallest chunk: 256 tokens, one unit per wave.  7 to 12 % faster than 16 at 16K-32K keys, same as 4
 constexpr int kMinUnitsPerChunk = 8;
 constexpr int kMergeGroups = 16;
-constexpr int kMergeFew = 32;  // up to this many chunks: one wave per row (split_merge_few_kernel)
+// Up to this many chunks one wave per row adds them up (split_merge_few_kernel).  us a call, sixteen waves / one: nine to sixteen chunks, one request of 2 000 keys
+// TQ4 11.7 / 11.3, Q8_0 11.2 / 10.8, of 1 000 16 tokens BF16 13.0 / 12.4; twenty and more TQ4 3 500 keys 12.4 / 12.6, 8 000 12.8 / 13.2, Q8_0 5 000 12.2 / 12.5, 8 000
+// 13.7 / 14.0; from 32 rows per kv head on (four waves) the same.
+constexpr int kMergeFew = 16;
 constexpr int kMergeMaxPerGroup = 16;  // at most 256 partials per row
 
 // ---- balanced decode ----------------------------------------------------------------------------
@@ -2308,12 +2311,9 @@ static int launch_split_merge(const AttnParams& P, int slots, float out_scale, h
         };
         if (slots <= kMergeFew) {
             if (merge_small_groups(P))
-                return slots <= 8    ? few(split_merge_few_kernel<TQ, HD, 8, 4>)
-                       : slots <= 16 ? few(split_merge_few_kernel<TQ, HD, 16, 4>)
-                                     : few(split_merge_few_kernel<TQ, HD, kMergeFew, 4>);
-            return slots <= 8    ? few(split_merge_few_kernel<TQ, HD, 8, kMergeGroups>)
-                   : slots <= 16 ? few(split_merge_few_kernel<TQ, HD, 16, kMergeGroups>)
-                                 : few(split_merge_few_kernel<TQ, HD, kMergeFew, kMergeGroups>);
+                return slots <= 8 ? few(split_merge_few_kernel<TQ, HD, 8, 4>) : few(split_merge_few_kernel<TQ, HD, kMergeFew, 4>);
+            return slots <= 8 ? few(split_merge_few_kernel<TQ, HD, 8, kMergeGroups>)
+                              : few(split_merge_few_kernel<TQ, HD, kMergeFew, kMergeGroups>);
         }
     }
     if (merge_small_groups(P)) {
