@@ -134,3 +134,16 @@ def test_merge_of_one_wave_up_to_sixteen_chunks(recorder):
             assert ("split_merge_few_kernel" in name) == (slots <= 16), (c, name, slots)
             forms.add(slots <= 16)
     assert len(forms) == 2
+
+
+def test_shorter_chunks_take_no_second_round(recorder):
+    """A call that fits the chip (256 workgroups) with chunks of eight units does so with shorter ones, up to eight kv heads; at one kv head as at
+    eight the same number of chunks."""
+    cases = [case(fmt, 1, q_len, 32 * units, 8 * kv_heads, kv_heads, head_dim, xf)
+             for fmt, xf, head_dim in (("tq4", 1, 256), ("q8_0", 0, 256), ("bf16", 0, 128)) for q_len in (1, 2, 4, 6, 8, 12, 16)
+             for units in (9, 15, 19, 30, 47, 63, 94, 120, 188) for kv_heads in (1, 2, 4, 8)]
+    chunks = {}
+    for c, (_, (run,)) in zip(cases, recorder(cases)):
+        n, whole, tiles = run[0][2][0], (c["max_seq"] // 32 + 1 + 7) // 8, (c["q_len"] * 8 + 15) // 16
+        assert n * tiles * c["kv_heads"] <= max(256, min(whole, 128 // tiles) * tiles * c["kv_heads"]), c
+        assert chunks.setdefault((c["fmt"], c["q_len"], c["max_seq"]), n) == n, c

@@ -101,7 +101,10 @@ struct AttnParams {
     int q_subgroups;  // gqa / q_group
     int tok_tile;     // query tokens per tile
     int max_chunks;   // cap on chunks per tile (1 = no split, scratch untouched)
-    int min_upc;      // minimum units per chunk
+    union {  // (in the place of one: as a word further on, 0.1 us of a 12.5 us call)
+        int min_upc;      // balanced decode: minimum units per piece
+        int few_chunks;   // chunk grid: chunk_count's line (few_chunks_of)
+    };
     int tiles_by_request;  // 1: blockIdx.z is a request (no request has more than one tile)
     int rot_q;             // K rows are stored rotated (WHT-256 transform): rotate the query rows
     int rot_out;           // V rows are stored rotated: rotate the output back
@@ -214,22 +217,43 @@ __host__ inline uint32_t q_group_magic_for(int q_group) { return (65536u + (uint
 struct ChunkGeom {
     int u_first, n_units, upc, n_chunks;
 };
-// Chunks of n_units units, `whole` of them of the usual least length.  Up to `few` chunks (kFewChunks*) they are shorter: four units are one
+// Smallest chunk: 256 tokens, one unit per wave.  7 to 12 % faster than 16 at 16K-32K keys, same as 4
+constexpr int kMinUnitsPerChunk = 8;
+// Split geometry is sized for the layout the path is built for, two kv heads per device: 128
+// chunks (or shares) per kv head.  The counts below depend on the batch and on gqa only, never
+// on local_kv_heads: a rank that holds one kv head of a sharded model computes every row with
+// the same chunks, in the same order, as a rank that holds all of them (bit-identical outputs
+// under head sharding, op_paged_attn.cu:1301-1304), at the price of half-filled compute units
+// on such a rank.
+constexpr int kTargetWorkgroupsPerHead = 128;
+// Chunks of n_units units.  Up to `few` chunks (kFewChunks*) they are shorter: four units are one
 // for the first wave of every SIMD, which then shares its issue slots with nobody, and one half unit per wave of a row format.
 constexpr int kShortChunkUnits = 4;
-__host__ __device__ constexpr int chunk_count(int n_units, int whole, int few) {
-    const int quick = (n_units + kShortChunkUnits - 1) / kShortChunkUnits;
+__host__ __device__ constexpr int chunk_count(int n_units, int few) {
+    const int whole = (n_units + kMinUnitsPerChunk - 1) / kMinUnitsPerChunk, quick = (n_units + kShortChunkUnits - 1) / kShortChunkUnits;
     return whole <= 1 || whole >= few ? whole : quick < few ? quick : few;
 }
 // us a layer step of one request, chunks of eight units / of four (merged by one wave per row on both sides): TQ4, 1 token on 600 keys
 // 17.3 / 16.8, on 2 500 17.5 / 17.1, 4 tokens on 5 000 with 40 chunks 21.2 / 21.5; Q8_0 1 200 17.3 / 16.6, 5 000 18.3 / 17.3; FP16 2 500 17.0 / 15.6, 10 000
 // with 79 chunks 18.4 / 18.8.
 constexpr int kFewChunksTq4 = 24, kFewChunksRows = 32;
-__device__ __forceinline__ ChunkGeom chunk_geom(int u_lo, int u_hi, int max_chunks, int min_upc, int few) {
+// More workgroups than the chip takes in one round cost more than shorter ones give, so all tiles of a kv head together have at most this many shorter
+// chunks: 256 workgroups with eight kv heads.  (The count must not depend on the kv heads: a rank that holds some of them has the chunks of all.)  us, chunks of
+// eight units / of four without a limit / with it: 32 + 4 heads, TQ4 16 tokens on 3 000 keys 17.5 / 27.0 / 16.6, 8 on 6 000 17.7 / 27.2 / 16.9, 4 requests of 750 to 3 000
+// 17.2 / 20.5 / 13.6; Q8_0 16 on 3 000 15.9 / 22.8 / 15.1; 64 + 8 heads, TQ4 4 on 6 000 17.8 / 27.0 / 17.1.  What it costs two kv heads: TQ4 16 tokens on
+// 1 500 keys 16.2 / 14.5 / 15.0, 8 requests of 375 to 1 500 14.7 / 12.2 / 12.9, Q8_0 14.7 / 11.7 / 13.1 (64 in all would give half of that back, and eight kv heads as slow
+// as without a limit); others within 1 %.
+constexpr int kShortWorkgroupsPerHead = 32;
+static_assert(kTargetWorkgroupsPerHead % kShortWorkgroupsPerHead == 0, "few_chunks_of: target = 128 / tiles");
+__host__ __device__ constexpr int few_chunks_of(int few, int target) {
+    const int share = target / (kTargetWorkgroupsPerHead / kShortWorkgroupsPerHead);
+    return share < few ? share : few;
+}
+__device__ __forceinline__ ChunkGeom chunk_geom(int u_lo, int u_hi, int max_chunks, int few) {
     ChunkGeom g;
     g.u_first = u_lo >> 5;
     g.n_units = (u_hi >= u_lo) ? ((u_hi >> 5) - g.u_first + 1) : 0;
-    int nc = chunk_count(g.n_units, fast_div(g.n_units + min_upc - 1, min_upc), few);
+    int nc = chunk_count(g.n_units, few);
     if (nc > max_chunks) nc = max_chunks;
     if (nc < 1) nc = 1;
     g.upc = fast_div(g.n_units + nc - 1, nc);
@@ -433,8 +457,6 @@ __device__ __forceinline__ constexpr int tq4_pv_elem(int h, int j, int r) {
     return 8 * r - 4 + j;
 }
 
-// Smallest chunk: 256 tokens, one unit per wave.  7 to 12 % faster than 16 at 16K-32K keys, same as 4
-constexpr int kMinUnitsPerChunk = 8;
 constexpr int kMergeGroups = 16;
 // Up to this many chunks one wave per row adds them up (split_merge_few_kernel).  us a call, sixteen waves / one: nine to sixteen chunks, one request of 2 000 keys
 // TQ4 11.7 / 11.3, Q8_0 11.2 / 10.8, of 1 000 16 tokens BF16 13.0 / 12.4; twenty and more TQ4 3 500 keys 12.4 / 12.6, 8 000 12.8 / 13.2, Q8_0 5 000 12.2 / 12.5, 8 000
@@ -909,7 +931,7 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
         if (u_lo == 0 && B.max_seq_len > 0 && u_hi == B.max_seq_len - 1) {
             g = ChunkGeom{0, P.spec_units, P.spec_upc, P.spec_chunks};  // as long as the host's bound
         } else {
-            g = chunk_geom(u_lo, u_hi, P.max_chunks, P.min_upc, kFewChunksTq4);
+            g = chunk_geom(u_lo, u_hi, P.max_chunks, P.few_chunks);
         }
         if (chunk >= g.n_chunks) return;
         cu_first = g.u_first + chunk * g.upc;
@@ -1671,7 +1693,7 @@ __device__ __forceinline__ void bal_for_each_piece(const AttnParams& P, TileFn&&
         const int units = __builtin_amdgcn_readlane(wave_incl_scan(q0.units), 63);
         int pieces, incl;
         if (as_grid) {
-            pieces = q0.units > 0 ? chunk_geom(0, 32 * q0.units - 1, P.grid_chunks, P.min_upc, FEW).n_chunks : 0;
+            pieces = q0.units > 0 ? chunk_geom(0, 32 * q0.units - 1, P.grid_chunks, few_chunks_of(FEW, P.grid_chunks)).n_chunks : 0;
             incl = wave_incl_scan(pieces);
         } else {
             share = bal_share(units, groups, P.min_upc);
@@ -2173,14 +2195,6 @@ constexpr int kShortGridKeys = (kMinUnitsPerChunk - 1) * kUnit;
 static_assert(kShortMaxEntries / 2 * (kMinUnitsPerChunk - 1) <= kShortBytes / (64 * 2 * kHeadDim) &&
                   16 * (kMinUnitsPerChunk - 1) <= kShortBytesFew / (64 * 2 * kHeadDim),
               "the chunk grid stands in for short batches only");
-// Split geometry is sized for the layout the path is built for, two kv heads per device: 128
-// chunks (or shares) per kv head.  The counts below depend on the batch and on gqa only, never
-// on local_kv_heads: a rank that holds one kv head of a sharded model computes every row with
-// the same chunks, in the same order, as a rank that holds all of them (bit-identical outputs
-// under head sharding, op_paged_attn.cu:1301-1304), at the price of half-filled compute units
-// on such a rank.
-constexpr int kTargetWorkgroupsPerHead = 128;
-
 static size_t partial_bytes(long long rows, int max_chunks) {
     return (size_t)rows * (size_t)max_chunks * (kHeadDim + 4) * sizeof(float);
 }
@@ -2191,12 +2205,13 @@ static size_t partial_bytes(long long rows, int max_chunks) {
 // 12.4 / 10.7, 10 000 keys TQ4 15.2 / 12.9 (64 of 79).  What halving is for: 8 MiB, 4 tokens of 32 + 4 heads on 32 000 keys, 63 chunks / 32: TQ4 35.6 / 26.8,
 // Q8_0 35.6 / 28.6; 64 + 8 heads, 31 / 16: 48.6 / 36.0.
 static long long one_round(long long tiles, int kv_subs) { return 2 * kTargetWorkgroupsPerHead / (tiles * kv_subs); }
+static int chunk_target(long long tiles, int q_subgroups) {
+    return (int)std::min<long long>(kMaxChunksCap, kTargetWorkgroupsPerHead / (std::max(tiles, 1ll) * std::max(q_subgroups, 1)));
+}
 static int choose_max_chunks(const warp34_exec* ex, int total_tokens, int num_q_heads, int tok_tile, int q_subgroups, int kv_subs) {
     if (ex->scratch_ptr == 0 || (ex->scratch_ptr & 15u) != 0u) return 1;
     const int tiles = (total_tokens + tok_tile - 1) / tok_tile;
-    const long long per_chunk = (long long)(tiles > 0 ? tiles : 1) * (q_subgroups > 0 ? q_subgroups : 1);
-    int want = (int)(kTargetWorkgroupsPerHead / per_chunk);
-    if (want > kMaxChunksCap) want = kMaxChunksCap;
+    int want = chunk_target(tiles, q_subgroups);
     if (want < 2) return 1;
     const size_t one = partial_bytes((long long)total_tokens * num_q_heads, 1);
     if (one > 0 && ex->scratch_size / one < (size_t)want) {
@@ -2340,11 +2355,11 @@ static int tiles_bound(const warp34_attention_batch& B, const AttnParams& P) {
     return (int)(B.max_q_len > 0 && by_requests < by_tokens ? by_requests : by_tokens);
 }
 
-// P.spec_* = chunk_geom(0, max_seq_len - 1, P.max_chunks, P.min_upc, few), worked out on the host
-static void fill_spec_geometry(AttnParams& P, int max_seq_len, int few) {
+// P.spec_* = chunk_geom(0, max_seq_len - 1, P.max_chunks, P.few_chunks), worked out on the host
+static void fill_spec_geometry(AttnParams& P, int max_seq_len) {
     if (max_seq_len <= 0) return;
     P.spec_units = ((max_seq_len - 1) >> 5) + 1;
-    int nc = chunk_count(P.spec_units, (P.spec_units + P.min_upc - 1) / P.min_upc, few);
+    int nc = chunk_count(P.spec_units, P.few_chunks);
     if (nc > P.max_chunks) nc = P.max_chunks;
     if (nc < 1) nc = 1;
     P.spec_upc = (P.spec_units + nc - 1) / nc;
@@ -2470,7 +2485,6 @@ static int launch_tq4(const warp34_exec* ex, const warp34_kv_layer_layout* layou
     const int nt = 1;
     P.tok_tile = (16 * nt) / q_group;
     if (P.tok_tile < 1) P.tok_tile = 1;
-    P.min_upc = kMinUnitsPerChunk;
     P.unit_in_page = (layout->block_size % kUnit == 0 && layout->k_page_stride_bytes <= 0xFFFFFFFFull &&
                       layout->v_page_stride_bytes <= 0xFFFFFFFFull)
                          ? 1
@@ -2491,10 +2505,12 @@ static int launch_tq4(const warp34_exec* ex, const warp34_kv_layer_layout* layou
     P.part_ml = nullptr;
     const long long rows = (long long)batch->total_tokens * num_q_heads;
     // grid.x: chunks that can exist given the host's upper bound on the sequence length
+    const long long tok_tiles = ((long long)batch->total_tokens + P.tok_tile - 1) / P.tok_tile;
+    P.few_chunks = few_chunks_of(kFewChunksTq4, on_grid ? decode_chunks : chunk_target(tok_tiles, P.q_subgroups));
     int grid_x = P.max_chunks;
     if (batch->max_seq_len > 0) {
         const int units = (batch->max_seq_len + kUnit - 1) / kUnit + 1;
-        const int bound = chunk_count(units, (units + P.min_upc - 1) / P.min_upc, kFewChunksTq4);
+        const int bound = chunk_count(units, P.few_chunks);
         if (bound < grid_x) grid_x = bound < 1 ? 1 : bound;
     }
     // No tile has more chunks than that: the cap is lowered to it, which changes no chunk (a
@@ -2502,7 +2518,7 @@ static int launch_tq4(const warp34_exec* ex, const warp34_kv_layer_layout* layou
     // the merge kernel loads ahead of knowing the count, as small as the bound allows.
     P.max_chunks = grid_x;
     P.part_stride = grid_x;
-    fill_spec_geometry(P, batch->max_seq_len, kFewChunksTq4);
+    fill_spec_geometry(P, batch->max_seq_len);
     if (P.max_chunks > 1) {
         uint8_t* ws = reinterpret_cast<uint8_t*>((uintptr_t)ex->scratch_ptr);
         P.part_acc = reinterpret_cast<float*>(ws);
@@ -2565,6 +2581,7 @@ static int launch_tq4(const warp34_exec* ex, const warp34_kv_layer_layout* layou
         P.bal_tiles = 1;
         P.bal_cols = 16;
         P.piece_cost = kTq4PieceCost;
+        P.min_upc = kMinUnitsPerChunk;
         P.bal_aligned = balanced_aligned(batch->num_reqs, plan_groups);
         P.grid_chunks = decode_chunks;
         rc = ensure_dynamic_lds(paged_attn_tq4_balanced_kernel<TQ>, smem_bytes_for(1), true);
@@ -2778,10 +2795,12 @@ static int launch_rows(const warp34_exec* ex, const warp34_kv_layer_layout* layo
     P.part_acc = nullptr;
     P.part_ml = nullptr;
     const long long rows = (long long)batch->total_tokens * num_q_heads;
+    const long long tok_tiles = ((long long)batch->total_tokens + P.tok_tile - 1) / P.tok_tile;
+    P.few_chunks = few_chunks_of(kFewChunksRows, decode_chunks > 0 ? decode_chunks : chunk_target(tok_tiles, P.q_subgroups));
     int grid_x = P.max_chunks;
     if (batch->max_seq_len > 0) {
         const int units = (batch->max_seq_len + kUnit - 1) / kUnit + 1;
-        const int bound = chunk_count(units, (units + P.min_upc - 1) / P.min_upc, kFewChunksRows);
+        const int bound = chunk_count(units, P.few_chunks);
         if (bound < grid_x) grid_x = bound < 1 ? 1 : bound;
     }
     // No tile has more chunks than that: the cap is lowered to it, which changes no chunk (a
@@ -2789,7 +2808,7 @@ static int launch_rows(const warp34_exec* ex, const warp34_kv_layer_layout* layo
     // the merge kernel loads ahead of knowing the count, as small as the bound allows.
     P.max_chunks = grid_x;
     P.part_stride = grid_x;
-    fill_spec_geometry(P, batch->max_seq_len, kFewChunksRows);
+    fill_spec_geometry(P, batch->max_seq_len);
     if (P.max_chunks > 1) {
         uint8_t* ws = reinterpret_cast<uint8_t*>((uintptr_t)ex->scratch_ptr);
         P.part_acc = reinterpret_cast<float*>(ws);
@@ -3216,28 +3235,27 @@ static size_t scratch_bytes_for(const warp34_kv_layer_layout* layout, int total_
         tok_tile = 16 / q_group < 1 ? 1 : 16 / q_group;
     }
     const int tiles = (int)(((long long)total_tokens + tok_tile - 1) / tok_tile);
-    long long want = kTargetWorkgroupsPerHead / ((long long)tiles * q_subgroups);
-    if (want > kMaxChunksCap) want = kMaxChunksCap;
+    const int full = chunk_target(tiles, q_subgroups);
+    int want = full;
     if (max_seq_len > 0) {
         const int units = (max_seq_len + kUnit - 1) / kUnit + 1;
-        const long long full = want;
-        want = std::min<long long>(want, chunk_count(units, (units + kMinUnitsPerChunk - 1) / kMinUnitsPerChunk, few));
+        want = std::min(want, chunk_count(units, few_chunks_of(few, full)));
         // (the first of full, full / 2, ... that is enough is at most 2 want - 1)
         if (!layout) want = std::min(full, 2 * want - 1);
         else if (want > one_round(tiles, kv_subs)) {
-            long long halved = full;
+            int halved = full;
             while (halved / 2 >= want) halved /= 2;
             want = halved;
         }
     }
-    size_t bytes = want >= 2 ? partial_bytes((long long)total_tokens * num_q_heads, (int)want) : 0;
+    size_t bytes = want >= 2 ? partial_bytes((long long)total_tokens * num_q_heads, want) : 0;
     // TQ4 verify batches over long contexts may take the shared-prefix pass: its partial slots sit
     // behind the split-K ones, and a header behind the records
     if ((!layout || is_tq4(layout)) && want >= 2 && total_tokens >= 16 && (num_reqs < 0 || num_reqs >= 4) &&
         max_seq_len >= 8 * kSpMinTokens && (q_group & (q_group - 1)) == 0) {
         const int parts = shared_prefix_parts(total_tokens, q_group, q_subgroups);
-        if ((int)want + parts <= kMergeGroups * kMergeMaxPerGroup)
-            bytes = partial_bytes((long long)total_tokens * num_q_heads, (int)want + parts) + sizeof(SpHeader);
+        if (want + parts <= kMergeGroups * kMergeMaxPerGroup)
+            bytes = partial_bytes((long long)total_tokens * num_q_heads, want + parts) + sizeof(SpHeader);
     }
     // The balanced plan: (shares + entries) partial slots of 16 columns per column tile and (kv head, q
     // subgroup), and the per-token table.

@@ -418,7 +418,7 @@ __device__ __forceinline__ void rows_tile(const AttnParams& P, uint8_t* smem, co
         if (u_lo == 0 && B.max_seq_len > 0 && u_hi == B.max_seq_len - 1) {
             g = ChunkGeom{0, P.spec_units, P.spec_upc, P.spec_chunks};  // as long as the host's bound
         } else {
-            g = chunk_geom(u_lo, u_hi, P.max_chunks, P.min_upc, kFewChunksRows);
+            g = chunk_geom(u_lo, u_hi, P.max_chunks, P.few_chunks);
         }
         if (chunk >= g.n_chunks) return;
         cu_first = g.u_first + chunk * g.upc;
