@@ -47,6 +47,15 @@ def kernel_scratch_bytes(tmp_path):
     return found
 
 
+def kernel_scalar_spills(tmp_path):
+    """{kernel name: scalar registers that are kept in lanes of vector registers}"""
+    found = {}
+    for path in code_objects(tmp_path):
+        for name, spills in re.findall(r"\.name: +(_Z\S+)\n(?:.*\n)*?.*\.sgpr_spill_count: (\d+)", readelf("--notes", path)):
+            found[name] = int(spills)
+    return found
+
+
 def kernel_preload_dwords(tmp_path):
     """{kernel name: dwords of its arguments that are in scalar registers when a wave starts}"""
     found = {}
@@ -71,6 +80,14 @@ def test_prefill_kernels_do_not_spill(tmp_path):
     kernels = {k: v for k, v in kernel_scratch_bytes(tmp_path).items() if "paged_prefill" in k}
     assert len(kernels) >= 16, sorted(kernels)
     assert {k: v for k, v in kernels.items() if v} == {}
+
+
+@pytest.mark.skipif(not os.path.exists(READELF), reason="no llvm-readelf")
+def test_wide_pieces_of_8bit_rows_keep_their_scalars(tmp_path):
+    """Two column tiles: a kernel that has to bring 110 scalars and more back starts a microsecond later."""
+    kernels = {k: v for k, v in kernel_scalar_spills(tmp_path).items() if re.search(r"rows_balanced_kernel.*Li2ELi[34]E", k)}
+    assert len(kernels) == 8, sorted(kernels)
+    assert {k: v for k, v in kernels.items() if v >= 100} == {}
 
 
 @pytest.mark.skipif(not os.path.exists(READELF), reason="no llvm-readelf")

@@ -266,11 +266,18 @@ __device__ __forceinline__ ChunkGeom chunk_geom(int u_lo, int u_hi, int max_chun
 // The 256-point WHT of finished rows and queries: 60 instructions a row (128 with an exchange, two sums and a select per value and lane stage).
 // A prefill wave rotates 64 rows: 16 requests of 256 tokens on 512 keys 116.6 / 107.7 us, 2 of 250 on 1 000 46.9 / 45.3.
 // One lane stage, H = 1, 2 or 8: lanes with bit H clear take v + v[lane ^ H], the others v[lane ^ H] - v.
-template <int H>
+// SELECT: the same by both results and a choice, twelve instructions more in all and no sign to keep.  For the two-column-tile form of 8-bit rows: with
+// the signs it spills 30 to 50 more scalars, also where nothing is rotated.  us a call, signs / choice: Q8_0 5 requests x 4 tokens on 2 000 keys 17.3 / 16.1, 24 tokens
+// on 240 keys 14.3 / 13.0, FP8 16.4 / 15.8, 13.5 / 12.7.  The other forms are as fast with the signs or faster (rotated FP8, 8 x 8 tokens on 240 keys 14.4 / 14.8).
+template <int H, bool SELECT = false>
 __device__ __forceinline__ void wht_stage(float (&v)[4], int lane) {
     const uint32_t flip = (lane & H) ? 0x80000000u : 0u;
 #pragma unroll
-    for (int k = 0; k < 4; ++k) v[k] = lane_xor<H>(v[k], lane) + __uint_as_float(__float_as_uint(v[k]) ^ flip);
+    for (int k = 0; k < 4; ++k) {
+        const float o = lane_xor<H>(v[k], lane);
+        if constexpr (SELECT) v[k] = (lane & H) ? o - v[k] : v[k] + o;
+        else v[k] = o + __uint_as_float(__float_as_uint(v[k]) ^ flip);
+    }
 }
 // H = 4: the sum in the groups of four lanes with the bit clear, the difference in the others.  (The compiler does not see that the statement
 // reads across lanes: the waits stand in it.)
@@ -308,6 +315,7 @@ __device__ __forceinline__ void wht_stage_pair(float& a, float& b) {
 }
 
 // 256-point WHT over one wave: element e = 4*lane + k, scaled by 1/16.
+template <bool SELECT = false>
 __device__ __forceinline__ void wht256_wave(float (&v)[4], int lane) {
     {
         const float a0 = v[0] + v[1], a1 = v[0] - v[1], a2 = v[2] + v[3], a3 = v[2] - v[3];
@@ -316,10 +324,10 @@ __device__ __forceinline__ void wht256_wave(float (&v)[4], int lane) {
         v[2] = a0 - a2;
         v[3] = a1 - a3;
     }
-    wht_stage<1>(v, lane);
-    wht_stage<2>(v, lane);
+    wht_stage<1, SELECT>(v, lane);
+    wht_stage<2, SELECT>(v, lane);
     wht_stage4(v);
-    wht_stage<8>(v, lane);
+    wht_stage<8, SELECT>(v, lane);
     wht_stage_pair<16>(v[0], v[1]);
     wht_stage_pair<16>(v[2], v[3]);
     wht_stage_pair<32>(v[0], v[1]);

@@ -813,7 +813,7 @@ __device__ __forceinline__ void rows_tile(const AttnParams& P, uint8_t* smem, co
                 if (rot_q) {
 #pragma unroll
                     for (int k = 0; k < 4; ++k) v[k] = apply_sign(v[k], 4 * lane + k);
-                    wht256_wave(v, lane);
+                    wht256_wave<NT == 2>(v, lane);
                 }
                 packed.x = pack_h2(v[0], v[1]);
                 packed.y = pack_h2(v[2], v[3]);
@@ -884,7 +884,7 @@ __device__ __forceinline__ void rows_tile(const AttnParams& P, uint8_t* smem, co
                 asm("" : "+v"(v[k]));  // rounded before the conversion to fp16, as where a merge kernel finishes the row
             }
             if (K8 && P.rot_out) {  // rotated V rows: one inverse rotation of the finished row
-                wht256_wave(v, lane);
+                wht256_wave<NT == 2>(v, lane);
 #pragma unroll
                 for (int k = 0; k < 4; ++k) v[k] = apply_sign(v[k], 4 * lane + k);
             }
