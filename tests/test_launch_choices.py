@@ -125,23 +125,25 @@ def test_queried_scratch_gives_the_launches_of_a_large_one(recorder):
         assert queried == large, (c, need)
 
 
-def test_merge_of_one_wave_up_to_sixteen_chunks(recorder):
-    cases = [case(fmt, 1, q_len, 32 * units) for fmt in ("tq4", "q8_0", "bf16") for q_len in (1, 2, 4, 8) for units in range(8, 300, 7)]
+def test_merge_of_one_wave(recorder):
+    """In the place of sixteen waves up to 16 chunks, of four (from 32 rows per kv head on) up to 32."""
+    cases = [case(fmt, 1, q_len, 32 * units) for fmt in ("tq4", "q8_0", "bf16") for q_len in (1, 2, 3, 4, 8) for units in range(8, 300, 7)]
     forms = set()
     for c, (_, (run,)) in zip(cases, recorder(cases)):
         if len(run) == 2:
             name, (_, _, _, _, slots), _ = run[1]
-            assert ("split_merge_few_kernel" in name) == (slots <= 16), (c, name, slots)
-            forms.add(slots <= 16)
-    assert len(forms) == 2
+            few = 32 if c["q_len"] * 8 >= 32 else 16
+            assert ("split_merge_few_kernel" in name) == (slots <= few), (c, name, slots)
+            forms.add((few, slots <= few))
+    assert len(forms) == 4
 
 
 def test_shorter_chunks_take_no_second_round(recorder):
-    """A call that fits the chip (256 workgroups) with chunks of eight units does so with shorter ones, up to eight kv heads; at one kv head as at
-    eight the same number of chunks."""
+    """A call that fits the chip (256 workgroups) with chunks of eight units does so with shorter ones, up to four kv heads; at one kv head as at
+    four the same number of chunks."""
     cases = [case(fmt, 1, q_len, 32 * units, 8 * kv_heads, kv_heads, head_dim, xf)
              for fmt, xf, head_dim in (("tq4", 1, 256), ("q8_0", 0, 256), ("bf16", 0, 128)) for q_len in (1, 2, 4, 6, 8, 12, 16)
-             for units in (9, 15, 19, 30, 47, 63, 94, 120, 188) for kv_heads in (1, 2, 4, 8)]
+             for units in (9, 15, 19, 30, 47, 63, 94, 120, 188) for kv_heads in (1, 2, 4)]
     chunks = {}
     for c, (_, (run,)) in zip(cases, recorder(cases)):
         n, whole, tiles = run[0][2][0], (c["max_seq"] // 32 + 1 + 7) // 8, (c["q_len"] * 8 + 15) // 16

@@ -238,12 +238,12 @@ __host__ __device__ constexpr int chunk_count(int n_units, int few) {
 // with 79 chunks 18.4 / 18.8.
 constexpr int kFewChunksTq4 = 24, kFewChunksRows = 32;
 // More workgroups than the chip takes in one round cost more than shorter ones give, so all tiles of a kv head together have at most this many shorter
-// chunks: 256 workgroups with eight kv heads.  (The count must not depend on the kv heads: a rank that holds some of them has the chunks of all.)  us, chunks of
+// chunks: 256 workgroups with four kv heads.  (The count must not depend on the kv heads: a rank that holds some of them has the chunks of all.)  us, chunks of
 // eight units / of four without a limit / with it: 32 + 4 heads, TQ4 16 tokens on 3 000 keys 17.5 / 27.0 / 16.6, 8 on 6 000 17.7 / 27.2 / 16.9, 4 requests of 750 to 3 000
-// 17.2 / 20.5 / 13.6; Q8_0 16 on 3 000 15.9 / 22.8 / 15.1; 64 + 8 heads, TQ4 4 on 6 000 17.8 / 27.0 / 17.1.  What it costs two kv heads: TQ4 16 tokens on
-// 1 500 keys 16.2 / 14.5 / 15.0, 8 requests of 375 to 1 500 14.7 / 12.2 / 12.9, Q8_0 14.7 / 11.7 / 13.1 (64 in all would give half of that back, and eight kv heads as slow
-// as without a limit); others within 1 %.
-constexpr int kShortWorkgroupsPerHead = 32;
+// 17.2 / 20.5 / 13.6; Q8_0 16 on 3 000 15.9 / 22.8 / 15.1.  What it costs two kv heads: TQ4 8 requests of 375 to 1 500 keys 14.7 / 12.2 / 12.9, Q8_0 14.7 / 11.7 / 12.0,
+// BF16 10 of 402 to 1 592 16.4 / 12.7 / 14.1.  Half the limit spares eight kv heads the second round as well (TQ4 4 tokens of 64 + 8 heads on 6 000 keys 17.8 / 27.0 / 27.3,
+// with half 17.1), but takes back a third of what one and two kv heads gain where it binds (Q8_0 7 requests of 507 to 1 705, 8 + 1 heads, 14.2 / 11.1 / 11.5, with half 12.8).
+constexpr int kShortWorkgroupsPerHead = 64;
 static_assert(kTargetWorkgroupsPerHead % kShortWorkgroupsPerHead == 0, "few_chunks_of: target = 128 / tiles");
 __host__ __device__ constexpr int few_chunks_of(int few, int target) {
     const int share = target / (kTargetWorkgroupsPerHead / kShortWorkgroupsPerHead);
@@ -466,10 +466,11 @@ __device__ __forceinline__ constexpr int tq4_pv_elem(int h, int j, int r) {
 }
 
 constexpr int kMergeGroups = 16;
-// Up to this many chunks one wave per row adds them up (split_merge_few_kernel).  us a call, sixteen waves / one: nine to sixteen chunks, one request of 2 000 keys
-// TQ4 11.7 / 11.3, Q8_0 11.2 / 10.8, of 1 000 16 tokens BF16 13.0 / 12.4; twenty and more TQ4 3 500 keys 12.4 / 12.6, 8 000 12.8 / 13.2, Q8_0 5 000 12.2 / 12.5, 8 000
-// 13.7 / 14.0; from 32 rows per kv head on (four waves) the same.
-constexpr int kMergeFew = 16;
+// Up to this many chunks one wave per row adds them up (split_merge_few_kernel); kMergeFewRows where it stands for four waves, not sixteen
+// (merge_small_groups).  us a call, sixteen waves / one: nine to sixteen chunks, one request of 2 000 keys TQ4 11.7 / 11.3, Q8_0 11.2 / 10.8, of 1 000
+// 16 tokens BF16 13.0 / 12.4; twenty and more TQ4 3 500 keys 12.4 / 12.6, 8 000 12.8 / 13.2, Q8_0 5 000 12.2 / 12.5, 8 000 13.7 / 14.0.  Four waves / one, 21
+// chunks: TQ4 6 requests x 4 tokens on 8 000 keys, 8 + 2 heads, 22.3 / 21.5; of 32 rows the same.
+constexpr int kMergeFew = 16, kMergeFewRows = 32;
 constexpr int kMergeMaxPerGroup = 16;  // at most 256 partials per row
 
 // ---- balanced decode ----------------------------------------------------------------------------
@@ -2332,9 +2333,11 @@ static int launch_split_merge(const AttnParams& P, int slots, float out_scale, h
                                out_scale, P.rot_out);
             return (int)hipGetLastError();
         };
-        if (slots <= kMergeFew) {
+        if (slots <= (merge_small_groups(P) ? kMergeFewRows : kMergeFew)) {
             if (merge_small_groups(P))
-                return slots <= 8 ? few(split_merge_few_kernel<TQ, HD, 8, 4>) : few(split_merge_few_kernel<TQ, HD, kMergeFew, 4>);
+                return slots <= 8           ? few(split_merge_few_kernel<TQ, HD, 8, 4>)
+                       : slots <= kMergeFew ? few(split_merge_few_kernel<TQ, HD, kMergeFew, 4>)
+                                            : few(split_merge_few_kernel<TQ, HD, kMergeFewRows, 4>);
             return slots <= 8 ? few(split_merge_few_kernel<TQ, HD, 8, kMergeGroups>)
                               : few(split_merge_few_kernel<TQ, HD, kMergeFew, kMergeGroups>);
         }
