@@ -57,7 +57,6 @@ typedef uint32_t u2v __attribute__((ext_vector_type(2)));
 // LDS holds the table, eight staging areas, the query operand table and the (m, l) tables:
 // 142 KB of 160 KB, one workgroup per CU
 constexpr int kTq4Waves = 8;
-__host__ __device__ constexpr int waves_for(int nt) { return nt == 1 ? kTq4Waves : 4; }
 constexpr int kUnit = 32;             // tokens per wave iteration
 constexpr int kLutBytes = 256 * 256;  // 256 entries x 64 lane replicas x 4 B
 constexpr int kRunBytes = 16 * kTq4RowBytes;  // 16 rows = 2112 B = 132 16-byte pieces
@@ -65,18 +64,17 @@ constexpr int kStageTq4 = 4 * kRunBytes;      // K rows 0-31 then V rows 0-31: 8
 // column stride of a merge region in dwords: 1 056 bytes, a stride at which 128-bit accesses of
 // eight columns do not collide (measured; 1 040 bytes cost 40 % more)
 constexpr int kMergeColStride = 264;
-__host__ __device__ constexpr int merge_floats_for(int nt) {  // one region of 8 columns per wave
-    return waves_for(nt) * (nt * 8 * kMergeColStride);
-}
-constexpr int kQopBytes = 16 * 4 * 9 * 16;  // query operand table: 16 columns x 4 k-blocks x 9 operands
+constexpr int kMergeFloats = kTq4Waves * 8 * kMergeColStride;  // one region of 8 columns per wave
+constexpr int kQopBytes = 16 * 4 * 9 * 16;  // query operand table of a column tile: 16 columns x 4 k-blocks x 9 operands
+// nt: column tiles of a workgroup
 __host__ __device__ constexpr int ml_offset_for(int nt) {  // (m, l) tables of the merge: behind everything the loop uses
-    return kLutBytes + waves_for(nt) * kStageTq4 + kQopBytes;
+    return kLutBytes + kTq4Waves * kStageTq4 + nt * kQopBytes;
 }
 __host__ __device__ constexpr int smem_bytes_for(int nt) {
-    return ml_offset_for(nt) + (waves_for(nt) + 1) * nt * 16 * 2 * 4;
+    return ml_offset_for(nt) + (kTq4Waves + 1) * nt * 16 * 2 * 4;
 }
-static_assert(merge_floats_for(1) * 4 <= waves_for(1) * kStageTq4, "merge regions alias the staging areas only");
-static_assert(smem_bytes_for(1) <= 160 * 1024, "decode LDS budget");
+static_assert(kMergeFloats * 4 <= kTq4Waves * kStageTq4, "merge regions alias the staging areas only");
+static_assert(smem_bytes_for(2) <= 160 * 1024, "decode LDS budget");
 constexpr int kXcds = 8;  // workgroups go round them in launch order
 constexpr int kChipCus = 256;
 constexpr float kLog2e = 1.4426950408889634f;
@@ -422,6 +420,7 @@ __device__ __forceinline__ float sum_over_rows(float x) {
 // Table lookup: the dequantisation table sits at LDS address 0 (it is the start of the dynamic
 // LDS block and the kernel has no static LDS), so the v_perm_b32 result IS the address.
 typedef __attribute__((address_space(3))) const uint32_t lds_cu32;
+typedef __attribute__((address_space(3))) const h8 lds_ch8;
 typedef __attribute__((address_space(1))) const u4 global_cu4;
 __device__ __forceinline__ uint32_t lut_read(uint32_t code_word, uint32_t lut_lane, uint32_t sel) {
     const uint32_t addr = __builtin_amdgcn_perm(code_word, lut_lane, sel);
@@ -711,7 +710,8 @@ __device__ __forceinline__ void wait_lds_reads() { asm volatile("s_waitcnt lgkmc
 // K rows 0-31, then V rows 0-31, 132 bytes each (four runs of 16 rows = 2112 bytes).
 // SP: the keys below *P.key_floor belong to a shared-prefix pass (see AttnParams); a separate
 // instantiation, so that the plain form carries no trace of it.
-template <typename TQ, bool BAL, bool SP = false, bool STREAM = BAL>
+// NT: column tiles of 16 (two: batches with neither a token mask nor a window).
+template <typename TQ, bool BAL, bool SP = false, bool STREAM = BAL, int NT = 1>
 __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, const BalItem& item, bool build_table) {
     static_assert(!(SP && BAL), "shared-prefix pass: split-K form only");
     constexpr int kWaves = kTq4Waves;
@@ -730,11 +730,11 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
     // every workgroup that is launched has work.  When no request can have more than one tile
     // (max_q_len <= tok_tile, e.g. decode) tile z is request z; otherwise the tile is located
     // with a prefix sum over the requests' tile counts.
-    const int tile_z = BAL ? item.req : (int)blockIdx.z;
+    const int tile_z = BAL || SP ? item.req : (int)blockIdx.z;
     const int kv_sub = (int)blockIdx.y;
     const int kv_head = small_div(kv_sub, P.q_subgroups);
     const int q_head_base = kv_head * P.gqa + (kv_sub - kv_head * P.q_subgroups) * P.q_group;
-    const int chunk = BAL ? 0 : (int)blockIdx.x;
+    const int chunk = BAL ? 0 : SP ? item.slot : (int)blockIdx.x;
 
     // The request lookup goes first: its loads head the longest dependency chain of the prologue
     // (lengths -> chunk geometry -> page ids -> the first K / V loads).
@@ -786,7 +786,7 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
     // number of tiles); a wrong guess is corrected after the lookup.
     const int tok_guess = BAL ? item.rq_start + item.tile * P.tok_tile
                               : min(P.tiles_by_request ? tile_z : tile_z * P.tok_tile, B.total_tokens - 1);
-    constexpr int kColsPerWave = (16 + kWaves - 1) / kWaves;
+    constexpr int kColsPerWave = (16 * NT + kWaves - 1) / kWaves;
     uint2 q_raw[kColsPerWave];
     auto load_q = [&](int tokbase) {
 #pragma unroll
@@ -795,7 +795,7 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
             const int t = div_q_group(col, P);
             const int a = col - t * P.q_group;
             q_raw[c] = uint2{0u, 0u};
-            if (col < 16 && tokbase + t < B.total_tokens) {
+            if (col < 16 * NT && tokbase + t < B.total_tokens) {
                 const uint16_t* qrow =
                     P.q + ((size_t)(tokbase + t) * P.num_q_heads + (size_t)(q_head_base + a)) * kHeadDim;
                 q_raw[c] = *reinterpret_cast<const uint2*>(qrow + 4 * lane);
@@ -804,13 +804,15 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
     };
     load_q(tok_guess);
     // validity of the token of this lane's column
-    bool tok_ok;
+    bool tok_ok = false;
     auto load_tok_ok_col = [&](int tokbase, int column) {
         const int tok = tokbase + div_q_group(column, P);
         tok_ok = tok < B.total_tokens &&
                  (B.valid_token_mask == nullptr || B.valid_token_mask[min(tok, B.total_tokens - 1)] != 0);
     };
-    auto load_tok_ok = [&](int tokbase) { load_tok_ok_col(tokbase, n); };
+    auto load_tok_ok = [&](int tokbase) {
+        if constexpr (NT == 1) load_tok_ok_col(tokbase, n);
+    };
     load_tok_ok(tok_guess);
 
     if (build_table) {
@@ -860,7 +862,7 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
     // carry the LOW-order fp16 part of the value weights where columns 0-7 carry the high-order
     // part, so one MFMA per value tile does the work of two.  The two halves are added up before
     // the waves merge.
-    const bool pack = tile_tokens * P.q_group <= 8;  // wave-uniform
+    const bool pack = NT == 1 && tile_tokens * P.q_group <= 8;  // wave-uniform
     const int ncol = pack ? (n & 7) : n;             // the query column this lane works for
     if (pack && ncol != n) load_tok_ok_col(tok0, ncol);
 
@@ -871,14 +873,29 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
     // intersection the first one's), and the per-lane part waits until the first loads are out.
     int col_lo = 0, col_hi = -1;
     bool col_ok = false;
+    int col_hi2 = -1;  // (two column tiles) of column 16 + n
+    bool col_ok2 = false;
     int u_lo = 0x7fffffff, u_hi = -1;  // union of the visible ranges
     int i_lo = 0, i_hi = 0x7fffffff;   // intersection of the visible ranges
     uint32_t ok_mask = 0u;             // bit c: column c is live (wave-uniform)
-    const bool simple = B.valid_token_mask == nullptr && B.sliding_window <= 0;
+    const bool simple = NT > 1 || (B.valid_token_mask == nullptr && B.sliding_window <= 0);
     // keys below the floor were handled by the shared-prefix pass (a multiple of the unit size)
     int key_floor = 0;
     if constexpr (SP) key_floor = __builtin_amdgcn_readfirstlane(*P.key_floor);
     auto column_info = [&](bool accumulate) {
+        if constexpr (NT > 1) {
+            auto last = [&](int col, bool& ok) {
+                const int t = div_q_group(col, P), tok = tok0 + t;
+                ok = t < tile_tokens && tok < B.total_tokens;
+                const int mx = B.mask_mode == WARP34_ATTN_MASK_NONCAUSAL_WINDOW ? seq_after - 1 : ctx_before + tok - rq_start;
+                return ok ? min(mx, seq_after - 1) : -1;
+            };
+            col_lo = key_floor;
+            col_hi = last(n, col_ok);
+            col_hi2 = last(16 + n, col_ok2);
+            ok_mask = (uint32_t)(__ballot(col_ok) & 0xFFFFull) | (uint32_t)(__ballot(col_ok2) & 0xFFFFull) << 16;
+            return;
+        }
         const int t = div_q_group(ncol, P);
         const int tok = tok0 + t;
         const bool ok = t < tile_tokens && tok_ok;
@@ -1096,12 +1113,12 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
         q_mf = D == 16 ? 4 : (D < 16 ? (Dh & 3) : 5 + (Dh & 3));
         q_half = half;
     }
-    static_assert(kColsPerWave == 2 && kWaves == 8, "a packed tile's mirror column col + 8 belongs to the wave of col");
+    static_assert(kColsPerWave == 2 * NT && kWaves == 8, "a packed tile's mirror column col + 8 belongs to the wave of col");
     uint2 packed_prev = {0u, 0u};
 #pragma unroll
     for (int c = 0; c < kColsPerWave; ++c) {
         const int col = wave + c * kWaves;
-        if (col < 16) {  // wave-uniform
+        if (col < 16 * NT) {  // wave-uniform
             float q_rot[4];
             q_rot[0] = TQ::to_f32((uint16_t)(q_raw[c].x & 0xFFFFu));
             q_rot[1] = TQ::to_f32((uint16_t)(q_raw[c].x >> 16));
@@ -1150,9 +1167,12 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
     // ---- per-wave state -----------------------------------------------------------------------
     const uint32_t lut_lane = (uint32_t)lane << 2;  // byte 0 of every table address
     const uint8_t* my_qop = qop + (size_t)(n * 4 + b) * 144;
+    const uint32_t qop_lane = (uint32_t)(kLutBytes + kWaves * kStageTq4 + (n * 4 + b) * 144);  // its LDS address
     h8 bq[9];  // the query operands of this lane stay in registers
+    if constexpr (NT == 1) {
 #pragma unroll
-    for (int mf = 0; mf < 9; ++mf) bq[mf] = *reinterpret_cast<const h8*>(my_qop + 16 * mf);
+        for (int mf = 0; mf < 9; ++mf) bq[mf] = *reinterpret_cast<const h8*>(my_qop + 16 * mf);
+    }
 
     f4 o_acc[2][8];
     float m_run = kNegBig, l_run = 0.f;
@@ -1160,6 +1180,15 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
     for (int h = 0; h < 2; ++h)
 #pragma unroll
         for (int j = 0; j < 8; ++j) o_acc[h][j] = f4{0.f, 0.f, 0.f, 0.f};
+    // (two column tiles) the second one's
+    f4 o_acc2[2][8];
+    float m_run2 = kNegBig, l_run2 = 0.f;
+    if constexpr (NT > 1) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int j = 0; j < 8; ++j) o_acc2[h][j] = f4{0.f, 0.f, 0.f, 0.f};
+    }
 
     // rows of the staging area: K rows 0-31, then V rows 0-31, 132 bytes each
     const uint8_t* ka_lo = stage + unit_token(0, n >> 2, n & 3) * kTq4RowBytes;  // A row of sub-tile 0; sub-tile 1: + 8 rows
@@ -1200,6 +1229,8 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
         // table reads of batch k + 1 are requested before the MFMAs of batch k are issued, so the
         // wave does not sit out the LDS latency of every batch.
         constexpr int kQkOrder[9] = {0, 5, 1, 6, 2, 7, 3, 8, 4};
+        float sc[8], sc2[8];
+        if constexpr (NT == 1) {
         f4 s_acc[2][2];
 #pragma unroll
         for (int s = 0; s < 2; ++s) s_acc[s][0] = s_acc[s][1] = f4{0.f, 0.f, 0.f, 0.f};
@@ -1230,18 +1261,62 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
             }
         }
         // rows 4b+i of the result are tokens unit_token(s, b, i); apply the K scales
-        float sc[8];
 #pragma unroll
         for (int s = 0; s < 2; ++s)
 #pragma unroll
             for (int i = 0; i < 4; ++i)
                 sc[4 * s + i] = __builtin_fmaf(s_acc[s][1][i], half_hi_to_f32(ksc[s][i]), mul_by_half_lo(s_acc[s][0][i], ksc[s][i]));
+        } else {
+            // Nine steps of one operand each: eight table reads and the operands of both column tiles (from LDS: with
+            // 128 accumulators they do not fit the registers) a step ahead, four MFMAs.
+            f4 s_acc[2][2][2];  // [column tile][sub-tile][half row]
+#pragma unroll
+            for (int g2 = 0; g2 < 2; ++g2)
+#pragma unroll
+                for (int s = 0; s < 2; ++s) s_acc[g2][s][0] = s_acc[g2][s][1] = f4{0.f, 0.f, 0.f, 0.f};
+            u4 ka[2][2];
+            h8 qb[2][2];
+            auto reads = [&](int st, u4 (&a)[2], h8 (&q)[2]) {
+                const int mf = kQkOrder[st];
+#pragma unroll
+                for (int s = 0; s < 2; ++s) {
+                    const uint32_t w = kw[s][mf];
+                    a[s][0] = lut_read(w, lut_lane, 0x0c0c0400u);
+                    a[s][1] = lut_read(w, lut_lane, 0x0c0c0500u);
+                    a[s][2] = lut_read(w, lut_lane, 0x0c0c0600u);
+                    a[s][3] = lut_read(w, lut_lane, 0x0c0c0700u);
+                }
+#pragma unroll
+                for (int g2 = 0; g2 < 2; ++g2) q[g2] = *reinterpret_cast<lds_ch8*>((uintptr_t)(qop_lane + (uint32_t)(g2 * kQopBytes + 16 * mf)));
+            };
+            reads(0, ka[0], qb[0]);
+#pragma unroll
+            for (int st = 0; st < 9; ++st) {
+                if (st + 1 < 9) reads(st + 1, ka[(st + 1) & 1], qb[(st + 1) & 1]);
+                __builtin_amdgcn_sched_barrier(0);
+                const int h = kQkOrder[st] < 5 ? 0 : 1;
+#pragma unroll
+                for (int s = 0; s < 2; ++s)
+#pragma unroll
+                    for (int g2 = 0; g2 < 2; ++g2)
+                        s_acc[g2][s][h] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, ka[st & 1][s]), qb[st & 1][g2],
+                                                                                s_acc[g2][s][h], 0, 0, 0);
+            }
+#pragma unroll
+            for (int s = 0; s < 2; ++s)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    sc[4 * s + i] = __builtin_fmaf(s_acc[0][s][1][i], half_hi_to_f32(ksc[s][i]), mul_by_half_lo(s_acc[0][s][0][i], ksc[s][i]));
+                    sc2[4 * s + i] = __builtin_fmaf(s_acc[1][s][1][i], half_hi_to_f32(ksc[s][i]), mul_by_half_lo(s_acc[1][s][0][i], ksc[s][i]));
+                }
+        }
         if (MASKED) {
 #pragma unroll
             for (int t = 0; t < 8; ++t) {
                 const int pos = t0 + unit_token(t >> 2, b, t & 3);
                 const bool vis = col_ok && pos >= col_lo && pos <= col_hi;
                 sc[t] = vis ? sc[t] : kNegBig;
+                if constexpr (NT > 1) sc2[t] = pos >= col_lo && pos <= col_hi2 ? sc2[t] : kNegBig;
             }
         }
 
@@ -1289,6 +1364,96 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
         wait_lds_reads();
         if (HAS_NEXT) issue_v();
 
+        if constexpr (NT > 1) {
+            float p[8], p2[8];
+            auto softmax = [&](float (&x)[8], float (&pr)[8], float& m, float& l, f4 (&o)[2][8]) __attribute__((always_inline)) {
+                float mx = fmaxf(max3(x[0], x[1], x[2]), max3(x[3], x[4], max3(x[5], x[6], x[7])));
+                mx = max_over_rows(mx);
+                const float m_new = fmaxf(m, mx);
+                const float alpha = __builtin_amdgcn_exp2f(m - m_new);
+                m = m_new;
+#pragma unroll
+                for (int t = 0; t < 8; ++t) pr[t] = __builtin_amdgcn_exp2f(x[t] - m_new);
+                if (MASKED) {
+#pragma unroll
+                    for (int t = 0; t < 8; ++t) pr[t] = x[t] > 0.5f * kNegBig ? pr[t] : 0.f;
+                }
+                float psum = 0.f;
+#pragma unroll
+                for (int t = 0; t < 8; ++t) psum += pr[t];
+                l = l * alpha + psum;
+                if (__ballot(alpha != 1.0f) != 0ull) {
+#pragma unroll
+                    for (int h = 0; h < 2; ++h)
+#pragma unroll
+                        for (int j = 0; j < 8; ++j) o[h][j] *= alpha;
+                }
+            };
+            softmax(sc, p, m_run, l_run, o_acc);
+            softmax(sc2, p2, m_run2, l_run2, o_acc2);
+            if (MASKED) {
+                // (a token masked for one column tile only keeps its scales, which are those of a real row)
+#pragma unroll
+                for (int t = 0; t < 8; ++t) vsc[t] = p[t] > 0.f || p2[t] > 0.f ? vsc[t] : 0u;
+            }
+            // Eight batches of two value tiles: eight table reads a batch ahead, eight MFMAs (high and low weights of two column tiles).
+            // The weights and code words of a half row are made in front of its batches.
+            u4 va[2][2];
+            uint32_t lo[4], hi[4];
+            u4 ph[2], pl[2];
+            auto words = [&](int h) __attribute__((always_inline)) {
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    const uint32_t wa = vw[h][2 * k], wb = vw[h][2 * k + 1];
+                    lo[k] = (wa & 0x0F0F0F0Fu) | ((wb << 4) & 0xF0F0F0F0u);
+                    hi[k] = ((wa >> 4) & 0x0F0F0F0Fu) | (wb & 0xF0F0F0F0u);
+                }
+            };
+            auto weights = [&](int h) __attribute__((always_inline)) {
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    auto w = [&](const float (&pr)[8], int t) { return h == 0 ? mul_by_half_lo(pr[t], vsc[t]) : mul_by_half_hi(pr[t], vsc[t]); };
+                    uint32_t whi, wlo;
+                    split_h2(w(p, 2 * k), w(p, 2 * k + 1), whi, wlo);
+                    ph[0][k] = whi, pl[0][k] = wlo;
+                    split_h2(w(p2, 2 * k), w(p2, 2 * k + 1), whi, wlo);
+                    ph[1][k] = whi, pl[1][k] = wlo;
+                }
+                settle(ph[0], ph[1], pl[0], pl[1]);
+            };
+            auto pv_reads = [&](int bt, u4 (&a)[2]) __attribute__((always_inline)) {
+#pragma unroll
+                for (int jj = 0; jj < 2; ++jj)
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) a[jj][k] = lut_read(jj ? hi[k] : lo[k], lut_lane, 0x0c0c0400u + ((uint32_t)(bt & 3) << 8));
+            };
+            words(0);
+            pv_reads(0, va[0]);
+            weights(0);
+#pragma unroll
+            for (int bt = 0; bt < 8; ++bt) {
+                const int h = bt >> 2;
+                if (bt == 3) words(1);
+                if (bt + 1 < 8) pv_reads(bt + 1, va[(bt + 1) & 1]);
+                if (bt == 4) weights(1);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int jj = 0; jj < 2; ++jj) {
+                    const int j = 2 * (bt & 3) + jj;
+                    const h8 av = __builtin_bit_cast(h8, va[bt & 1][jj]);
+                    o_acc[h][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, __builtin_bit_cast(h8, ph[0]), o_acc[h][j], 0, 0, 0);
+                    o_acc2[h][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, __builtin_bit_cast(h8, ph[1]), o_acc2[h][j], 0, 0, 0);
+                }
+#pragma unroll
+                for (int jj = 0; jj < 2; ++jj) {
+                    const int j = 2 * (bt & 3) + jj;
+                    const h8 av = __builtin_bit_cast(h8, va[bt & 1][jj]);
+                    o_acc[h][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, __builtin_bit_cast(h8, pl[0]), o_acc[h][j], 0, 0, 0);
+                    o_acc2[h][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, __builtin_bit_cast(h8, pl[1]), o_acc2[h][j], 0, 0, 0);
+                }
+            }
+            return;
+        } else {
         // ---- online softmax (log2 domain), per lane = per query column --------------------
         float p[8];
         {
@@ -1382,6 +1547,7 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
                 }
             }
         }
+        }
     };
 
     for (int j = 0; unit < cu_end; ++j) {
@@ -1423,13 +1589,14 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
 
     // ---- combine the per-lane partial sums of l over the four k-block lanes of a column ------
     l_run = sum_over_rows(l_run);
+    if constexpr (NT > 1) l_run2 = sum_over_rows(l_run2);
 
     // ---- merge the waves' states through LDS ---------------------------------------------------
     // Every wave publishes (m, l) and its O, as it stands, in its own region -- its own staging area,
     // which nobody else touches, so the stores need not wait for the other waves -- and after ONE
     // barrier wave c adds up column c of the eight regions, each weighted by 2^(m_w - m_tot), in wave
     // order.  A region holds eight columns: a tile with live columns in both halves (more than
-    // eight columns, never a decode step) takes a second pass.
+    // eight columns, never a decode step) takes a second pass, two column tiles take up to four.
     // Region layout: column stride kMergeColStride dwords; inside a column the four values a lane
     // holds for one MFMA result (rows 4b..4b+3 of (h, j)) are contiguous at ((h*8 + j)*4 + b)*4,
     // so a lane stores them with one 128-bit write and the adding wave reads one 128-bit piece per
@@ -1442,11 +1609,16 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
     float* xbuf = reinterpret_cast<float*>(stage_all);
     float* tbuf = reinterpret_cast<float*>(qop) + wave * 256;
     // [kWaves][16][2]: in an area of its own, a wave publishes its state while others are still in their loops
-    float* mlbuf = reinterpret_cast<float*>(smem + ml_offset_for(1));
-    static_assert(kWaves * kRegion == merge_floats_for(1), "merge layout");
+    float* mlbuf = reinterpret_cast<float*>(smem + ml_offset_for(NT));
+    static_assert(kWaves * kRegion == kMergeFloats, "merge layout");
+    constexpr int kCols = 16 * NT;
     if (b == 0) {
-        mlbuf[(wave * 16 + n) * 2 + 0] = m_run;
-        mlbuf[(wave * 16 + n) * 2 + 1] = l_run;
+        mlbuf[(wave * kCols + n) * 2 + 0] = m_run;
+        mlbuf[(wave * kCols + n) * 2 + 1] = l_run;
+        if constexpr (NT > 1) {
+            mlbuf[(wave * kCols + 16 + n) * 2 + 0] = m_run2;
+            mlbuf[(wave * kCols + 16 + n) * 2 + 1] = l_run2;
+        }
     }
     auto store_region = [&](int half) {
         float* c = xbuf + wave * kRegion + (n & 7) * kColStride;
@@ -1466,7 +1638,8 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
         }
     };
     const bool live0 = (ok_mask & 0xFFu) != 0u, live1 = (ok_mask >> 8) != 0u;  // the same in every wave
-    store_region(live0 ? 0 : 1);
+    // (two column tiles: a live column is in the first eight, the tile's live ones lie without a gap from column 0 on)
+    store_region(NT > 1 || live0 ? 0 : 1);
 
     int merge_slot[4];  // region slot of element 4*lane + k (inverse of tq4_pv_elem)
 #pragma unroll
@@ -1486,20 +1659,45 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
     }
     __syncthreads();  // every wave is done with the table, and the regions of the first pass are there
 #pragma unroll 1
-    for (int half = 0; half < 2; ++half) {
-        if (!(half ? live1 : live0)) continue;
-        if (half == 1 && live0) {
-            __syncthreads();  // the first pass has read the regions
-            store_region(1);
-            __syncthreads();
+    for (int half = 0; half < 2 * NT; ++half) {
+        if constexpr (NT > 1) {
+            if (((ok_mask >> (8 * half)) & 0xFFu) == 0u) break;
+            if (half > 0) {
+                __syncthreads();  // the pass before has read the regions
+                if (half == 2) {  // on to the second column tile
+                    col_ok = col_ok2;
+#pragma unroll
+                    for (int h = 0; h < 2; ++h)
+#pragma unroll
+                        for (int j = 0; j < 8; ++j) o_acc[h][j] = o_acc2[h][j];
+                }
+                store_region(half & 1);
+                __syncthreads();
+            }
+        } else {
+            if (!(half ? live1 : live0)) continue;
+            if (half == 1 && live0) {
+                __syncthreads();  // the first pass has read the regions
+                store_region(1);
+                __syncthreads();
+            }
         }
         const int col = 8 * half + wave;
         if (wave < 8 && ((ok_mask >> col) & 1u)) {
+            size_t old_row = 0;
+            f4 old_acc, old_rec;
+            if constexpr (NT > 1) {
+                const int t = div_q_group(col, P);
+                old_row = ((size_t)(tok0 + t) * P.num_q_heads + (size_t)(q_head_base + col - t * P.q_group)) * P.part_stride +
+                          (size_t)(P.pf_slot_base + chunk);
+                old_acc = *reinterpret_cast<const f4*>(P.part_acc + old_row * kHeadDim + 4 * lane);
+                old_rec = *reinterpret_cast<const f4*>(P.part_ml + old_row * 4);
+            }
             // state of the column in the eight waves (the same addresses in every lane)
             float mw[kWaves], lw[kWaves];
 #pragma unroll
             for (int w = 0; w < kWaves; ++w) {
-                const f2 r = *reinterpret_cast<const f2*>(mlbuf + (w * 16 + col) * 2);
+                const f2 r = *reinterpret_cast<const f2*>(mlbuf + (w * kCols + col) * 2);
                 mw[w] = r[0];
                 lw[w] = r[1];
             }
@@ -1522,8 +1720,21 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
             const int t = div_q_group(col, P);
             const int a = col - t * P.q_group;
             const size_t row = (size_t)(tok0 + t) * P.num_q_heads + (size_t)(q_head_base + a);
-            if (BAL ? item.n_chunks > 1 : P.max_chunks > 1) {
+            if (NT > 1 || (BAL ? item.n_chunks > 1 : P.max_chunks > 1)) {
                 // un-normalised, rotated, still carrying the table gain; the merge kernel finishes
+                if constexpr (NT > 1) {
+                    // The chunk joins a record of the shared prefix (asked for ahead of the sums above); the row has no other
+                    // chunk records, which the first one of them says.
+                    const float m = fmaxf(m_col, old_rec[0]);
+                    const float w_new = __builtin_amdgcn_exp2f(m_col - m), w_old = __builtin_amdgcn_exp2f(old_rec[0] - m);
+                    float* dst = P.part_acc + old_row * kHeadDim;
+                    *reinterpret_cast<f4*>(dst + 4 * lane) = f4{v[0], v[1], v[2], v[3]} * w_new + old_acc * w_old;
+                    if (lane == 0) {
+                        *reinterpret_cast<f4*>(P.part_ml + old_row * 4) = f4{m, l_col * w_new + old_rec[1] * w_old, old_rec[2], 0.f};
+                        if (chunk == 0) *reinterpret_cast<f4*>(P.part_ml + row * P.part_stride * 4) = f4{kNegBig, 0.f, 0.f, 0.f};
+                    }
+                    continue;
+                }
                 const size_t prow = BAL ? bal_partial_row(item.slot, (int)gridDim.y, kv_sub, 16, col)
                                         : row * (SP ? P.part_stride : P.max_chunks) + chunk;
                 float* dst = P.part_acc + prow * kHeadDim;
@@ -1548,18 +1759,41 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
     }
 }
 
-template <typename TQ, int NT, bool SP = false>
+template <typename TQ, bool SP = false>
 __global__ __launch_bounds__(kTq4Waves * 64, 1) void paged_attn_tq4_kernel(const AttnParams P) {
-    static_assert(NT == 1, "one 16-column tile per workgroup");
     extern __shared__ __align__(16) uint8_t smem[];
     // lut_read() addresses the table absolutely: the dynamic block starts at LDS address 0 because
     // the kernel has no static LDS (checked on the host before the first launch)
     // decode steps (no request has more than one tile): every key is read by one workgroup only,
     // the loads carry the streaming hint; one body per kind of load
+    BalItem item{};
+    if constexpr (SP) item.req = (int)blockIdx.z, item.slot = (int)blockIdx.x;
     if (!SP && P.tiles_by_request != 0 && P.q_subgroups == 1) {  // uniform for the grid
-        tq4_tile<TQ, false, SP, true>(P, smem, BalItem{}, true);
+        tq4_tile<TQ, false, SP, true>(P, smem, item, true);
     } else {
-        tq4_tile<TQ, false, SP, false>(P, smem, BalItem{}, true);
+        tq4_tile<TQ, false, SP, false>(P, smem, item, true);
+    }
+}
+
+// The private rest of a verify batch with more than 16 query columns per request and kv head: both column tiles in one workgroup, so that
+// a key is looked up once for 32 columns (a wave's unit: 465 vector instructions and 100 MFMAs, one tile 330 and 50).  Issue bounds it, so the loads keep their
+// plain form: with the streaming hint 3 % slower.  `wide` holds the geometry of that form, whose chunks join the prefix's records, for which there is room
+// whatever their number; with nothing shared, `P`, that of the plain path, whose bits the batch then has.  us, 16 requests x 4 tokens on 262 144 keys, 200 000 of
+// them shared, one column tile / two: whole call 524 / 486, on another box 534 / 512; this kernel 177 / 147.
+template <typename TQ>
+__global__ __launch_bounds__(kTq4Waves * 64, 1) void paged_attn_tq4_private_kernel(int chunks, int tiles, int wide_chunks, int wide_tiles,
+                                                                                   const AttnParams P, const AttnParams wide) {
+    extern __shared__ __align__(16) uint8_t smem[];
+    const int wg = (int)blockIdx.x;
+    BalItem item{};
+    if (__builtin_amdgcn_readfirstlane(*P.key_floor) != 0) {
+        item.req = wg / wide_chunks;
+        item.slot = wg - item.req * wide_chunks;
+        if (item.req < wide_tiles) tq4_tile<TQ, false, true, false, 2>(wide, smem, item, true);
+    } else {
+        item.req = wg / chunks;
+        item.slot = wg - item.req * chunks;
+        if (item.req < tiles) tq4_tile<TQ, false, true, false, 1>(P, smem, item, true);
     }
 }
 
@@ -2490,11 +2724,8 @@ static int launch_tq4(const warp34_exec* ex, const warp34_kv_layer_layout* layou
     P.q_group = q_group;
     P.q_group_magic = q_group_magic_for(q_group);
     P.q_subgroups = P.gqa / q_group;
-    // One N tile (16 query columns) per workgroup, also for verify batches: the two-tile variant
-    // (4 waves, 32 columns) halves the key reads but runs at half the occupancy and measured
-    // slower (2.04 ms against 1.64 ms on 16 requests x 4 query tokens at 262 144 keys).
-    const int nt = 1;
-    P.tok_tile = (16 * nt) / q_group;
+    // One column tile (16 query columns) per workgroup; two behind a shared prefix (paged_attn_tq4_private_kernel).
+    P.tok_tile = 16 / q_group;
     if (P.tok_tile < 1) P.tok_tile = 1;
     P.unit_in_page = (layout->block_size % kUnit == 0 && layout->k_page_stride_bytes <= 0xFFFFFFFFull &&
                       layout->v_page_stride_bytes <= 0xFFFFFFFFull)
@@ -2573,10 +2804,24 @@ static int launch_tq4(const warp34_exec* ex, const warp34_kv_layer_layout* layou
                                stream, T);
             rc = (int)hipGetLastError();
             if (rc) return rc;
-            rc = ensure_dynamic_lds(paged_attn_tq4_kernel<TQ, 1, true>, smem_bytes_for(1), true);
-            if (rc) return rc;
-            hipLaunchKernelGGL((paged_attn_tq4_kernel<TQ, 1, true>), grid, dim3(waves_for(1) * 64), smem_bytes_for(1),
-                               stream, P);
+            if (batch->max_q_len * q_group > 16 && 32 % q_group == 0) {
+                AttnParams W = P;
+                W.tok_tile = 32 / q_group;
+                W.tiles_by_request = batch->max_q_len <= W.tok_tile ? 1 : 0;
+                W.bal_tiles = tiles_per_request_bound(*batch, W);
+                // a chunk joins the record of the prefix's part with its number
+                W.max_chunks = std::max(1, std::min(parts, chunk_target(((long long)batch->total_tokens + W.tok_tile - 1) / W.tok_tile, W.q_subgroups)));
+                const int tiles = tiles_bound(*batch, W);
+                rc = ensure_dynamic_lds(paged_attn_tq4_private_kernel<TQ>, smem_bytes_for(2), true);
+                if (rc) return rc;
+                const long long wgs = std::max((long long)grid_x * grid_z, (long long)W.max_chunks * tiles);
+                hipLaunchKernelGGL(paged_attn_tq4_private_kernel<TQ>, dim3((unsigned)wgs, (unsigned)kv_subs), dim3(kTq4Waves * 64),
+                                   smem_bytes_for(2), stream, grid_x, grid_z, W.max_chunks, tiles, P, W);
+            } else {
+                rc = ensure_dynamic_lds(paged_attn_tq4_kernel<TQ, true>, smem_bytes_for(1), true);
+                if (rc) return rc;
+                hipLaunchKernelGGL((paged_attn_tq4_kernel<TQ, true>), grid, dim3(kTq4Waves * 64), smem_bytes_for(1), stream, P);
+            }
             rc = (int)hipGetLastError();
             if (rc) return rc;
             return launch_split_merge<TQ, true, kHeadDim>(P, stride, kLutInvGain, stream);
@@ -2598,15 +2843,15 @@ static int launch_tq4(const warp34_exec* ex, const warp34_kv_layer_layout* layou
         rc = ensure_dynamic_lds(paged_attn_tq4_balanced_kernel<TQ>, smem_bytes_for(1), true);
         if (rc) return rc;
         hipLaunchKernelGGL((paged_attn_tq4_balanced_kernel<TQ>), dim3((unsigned)plan_groups, (unsigned)kv_subs),
-                           dim3(waves_for(1) * 64), smem_bytes_for(1), stream, P);
+                           dim3(kTq4Waves * 64), smem_bytes_for(1), stream, P);
         rc = (int)hipGetLastError();
         if (rc) return rc;
         return launch_balanced_merge<TQ, kHeadDim>(P, kv_subs, kLutInvGain, stream);
     }
     P.bal_tiles = tiles_per_request_bound(*batch, P);
-    rc = ensure_dynamic_lds(paged_attn_tq4_kernel<TQ, 1>, smem_bytes_for(1), true);
+    rc = ensure_dynamic_lds(paged_attn_tq4_kernel<TQ>, smem_bytes_for(1), true);
     if (rc) return rc;
-    hipLaunchKernelGGL((paged_attn_tq4_kernel<TQ, 1>), grid, dim3(waves_for(1) * 64), smem_bytes_for(1), stream, P);
+    hipLaunchKernelGGL(paged_attn_tq4_kernel<TQ>, grid, dim3(kTq4Waves * 64), smem_bytes_for(1), stream, P);
     rc = (int)hipGetLastError();
     if (rc) return rc;
     return P.max_chunks > 1 ? launch_split_merge<TQ, false, kHeadDim>(P, P.max_chunks, kLutInvGain, stream) : 0;

@@ -27,7 +27,6 @@ namespace w34 {
 // Query rows of a workgroup with NC column tiles of 16 per wave
 constexpr int pw_rows(int nc) { return kPfWaves * 16 * nc; }
 
-typedef __attribute__((address_space(3))) const h8 lds_ch8;
 typedef __attribute__((address_space(3))) const f4 lds_cf4;
 typedef __attribute__((address_space(3))) const f2 lds_cf2;
 typedef __attribute__((address_space(3))) u2v lds_u2;
