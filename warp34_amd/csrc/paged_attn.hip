@@ -65,7 +65,7 @@ constexpr int kStageTq4 = 4 * kRunBytes;      // K rows 0-31 then V rows 0-31: 8
 // eight columns do not collide (measured; 1 040 bytes cost 40 % more)
 constexpr int kMergeColStride = 264;
 constexpr int kMergeFloats = kTq4Waves * 8 * kMergeColStride;  // one region of 8 columns per wave
-constexpr int kQopBytes = 16 * 4 * 9 * 16;  // query operand table of a column tile: 16 columns x 4 k-blocks x 9 operands
+constexpr int kQopBytes = 16 * 4 * 9 * 16;  // query operand table of a column tile: 16 columns x 4 k-blocks x 8 operands, 144 bytes apart
 // nt: column tiles of a workgroup
 __host__ __device__ constexpr int ml_offset_for(int nt) {  // (m, l) tables of the merge: behind everything the loop uses
     return kLutBytes + kTq4Waves * kStageTq4 + nt * kQopBytes;
@@ -85,6 +85,18 @@ constexpr float kNegBig = -1.0e30f;  // "minus infinity" that stays finite under
 // the accuracy of the scores.
 constexpr float kLutGain = 1.908032f;
 constexpr float kLutInvGain = 1.0f / kLutGain;
+
+// Weights of two operands (TQ4, BF16): a column's running maximum is raised only by scores that exceed it by more than this (log2 domain), so
+// a probability may be up to 2^8; its operands keep 22 (16) bits of it whatever its size, the sums are fp32.  Raising multiplies 64 sums per column
+// tile, and of the first units nearly every one raises the maximum of some column of a wave.  TQ4 value scales ride on the probabilities: in a
+// unit with a larger one than kPfSlackScale, where the weight could leave fp16's range, and where a column does not see the whole unit (what lies
+// behind the sequence must not matter), the maximum is exact.  Per column, so that tiles of either size give the same bits.  (One fp16
+// operand: exact as well, the largest probability is then 1 and rounds to itself; with the slack FP16 and Q8_0 batches came out 6 % further from 64
+// bits, 3.24e-4 for 3.05e-4.)  us, maximum
+// raised by every unit that exceeds it / now: 16 requests of 256 tokens on 2 048 keys BF16 224 / 199, TQ4 261 / 247, 4 of 700 on 6 000 BF16 507 / 459,
+// TQ4 634 / 618, 8 of 2 048 on 16 384 TQ4 6 261 / 6 185.
+constexpr float kPfSlack = 8.0f, kPfSlackScale = 255.0f;
+constexpr uint32_t kSlackScaleBits = 0x5BF8u;  // kPfSlackScale in fp16
 
 struct AttnParams {
     warp34_kv_layer_layout L;
@@ -370,15 +382,20 @@ __device__ __forceinline__ void split_h2(float a, float b, uint32_t& hi, uint32_
 // An MFMA may read a register two wait states after a vector instruction has written it.  The compiler
 // keeps that distance for its own instructions but does not see through an assembly statement, so
 // the low-order operands pass through settle() on their way to the MFMAs.
-__device__ __forceinline__ void settle(u4& a, u4& b) { asm("s_nop 1" : "+v"(a), "+v"(b)); }
-__device__ __forceinline__ void settle(u4& a, u4& b, u4& c, u4& d) {
-    asm("s_nop 1" : "+v"(a), "+v"(b), "+v"(c), "+v"(d));
-}
 __device__ __forceinline__ void settle(u2v (&a)[8]) {
     asm("s_nop 1" : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]), "+v"(a[4]), "+v"(a[5]), "+v"(a[6]), "+v"(a[7]));
 }
 __device__ __forceinline__ void settle(u4 (&a)[8]) {
     asm("s_nop 1" : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]), "+v"(a[4]), "+v"(a[5]), "+v"(a[6]), "+v"(a[7]));
+}
+// The same for the weights of TQ4 rows, where issue and not registers is short: v_fma_mix_f32 and v_cvt_pk_f16_f32 issue every 4 cycles, v_fma_mixlo_f16 /
+// mixhi, which do both, every 8.  (Written as fma, the compiler widens the halves with instructions of their own.)
+__device__ __forceinline__ void split_weights(float a, float b, uint32_t& hi, uint32_t& lo) {
+    hi = pack_h2(a, b);
+    float r0, r1;
+    asm("v_fma_mix_f32 %0, %1, 1.0, -%2 op_sel:[0,0,0] op_sel_hi:[0,0,1]" : "=v"(r0) : "v"(a), "v"(hi));
+    asm("v_fma_mix_f32 %0, %1, 1.0, -%2 op_sel:[0,0,1] op_sel_hi:[0,0,1]" : "=v"(r1) : "v"(b), "v"(hi));
+    lo = pack_h2(r0, r1);
 }
 // a * (fp16 half of w) as one mixed-precision FMA that reads the half in place (v_fma_mix_f32 with
 // a zero addend; written as an fma so that the compiler forms it and places the wait states that
@@ -388,6 +405,11 @@ __device__ __forceinline__ float mul_by_half_lo(float a, uint32_t w) {
 }
 __device__ __forceinline__ float mul_by_half_hi(float a, uint32_t w) {
     return __builtin_fmaf(a, (float)__builtin_bit_cast(_Float16, (uint16_t)(w >> 16)), 0.0f);
+}
+// the larger ones of two pairs of 16-bit numbers
+__device__ __forceinline__ uint32_t max_u16x2(uint32_t a, uint32_t b) {
+    typedef uint16_t us2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(us2, a), __builtin_bit_cast(us2, b)));
 }
 // maximum of three finite values in one instruction (fmaxf would first quiet each operand); the
 // operands must come from ordinary vector instructions: the compiler places no wait states in
@@ -450,12 +472,16 @@ __device__ __forceinline__ constexpr int tq4_dword_elem(int D, int i) {
     if (D == 16) return i < 4 ? 124 + i : -1;
     return 128 + 8 * (D - 17) + i;
 }
-// dword read by k-block bk for QK MFMA m of half h (h=0: m 0..4, h=1: m 0..3).  The k-blocks of
+// dword read by k-block bk for QK MFMA m (0..3) of half h.  The k-blocks of
 // lanes 0-31 (bk 0,1) sit 8 dwords apart, which keeps the 32 simultaneous reads on 32 banks.
+// Dword 0 holds four codes behind a scale and dword 16 four in front of one: the two make one operand of eight codes
+// (tq4_fuse; a fifth MFMA for dword 16 alone and its four look-ups before).
 __device__ __forceinline__ constexpr int tq4_qk_dword(int h, int m, int bk) {
-    const int base = 8 * (bk & 1) + 4 * (bk >> 1);
-    if (h == 0) return m < 4 ? base + m : 16;
-    return 17 + base + m;
+    return (h == 0 ? 0 : 17) + 8 * (bk & 1) + 4 * (bk >> 1) + m;
+}
+// The code dword of the lanes with first: elements 0..3 and 124..127; the others: dword d as it is.
+__device__ __forceinline__ uint32_t tq4_fuse(uint32_t d16, uint32_t d, bool first) {
+    return __builtin_amdgcn_alignbit(d16, d, first ? 16u : 0u);
 }
 // element index of V^T row r, nibble j, half h (PV MFMA output row -> head dimension)
 __device__ __forceinline__ constexpr int tq4_pv_elem(int h, int j, int r) {
@@ -1086,11 +1112,10 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
     if (simple) column_info(false);
 
     // ---- prologue: the query operand table ---------------------------------------------------------
-    // B operands of the QK MFMAs, nine per lane (five for the first half-row, four for the second),
-    // in the order the loop reads them: slot (n, b) holds 9 x 16 bytes.  Operand (h, m) of k-block
-    // b pairs with row dword D = tq4_qk_dword(h, m, b); its eight elements (tq4_dword_elem) are
-    // contiguous in the query row: dword D < 16 covers elements 8 D - 4 .. 8 D + 3 (the first four
-    // are scale nibbles for D = 0 and stay zero), dword 16 elements 124 .. 127 and zeros, dword
+    // B operands of the QK MFMAs, eight per lane (four for either half-row), in the order the loop reads
+    // them: slot (n, b) holds 8 x 16 bytes.  Operand (h, m) of k-block b pairs with row dword D =
+    // tq4_qk_dword(h, m, b); its eight elements (tq4_dword_elem) are contiguous in the query row: dword
+    // D < 16 covers elements 8 D - 4 .. 8 D + 3 (D = 0: 0 .. 3 and 124 .. 127, see tq4_fuse), dword
     // 17 + k elements 128 + 8 k .. 128 + 8 k + 7.  A lane of the rotating wave holds elements
     // 4 lane .. 4 lane + 3 of its column, i.e. one half of one operand, and writes it there.
     // All the constant factors of the scores (softmax scale, log2 e, 1 / table gain) go into Q'.
@@ -1099,19 +1124,11 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
     // where this lane's four elements go: operand (k-block, mf) and which half of it
     int q_kb, q_mf, q_half;
     {
-        int D, half;
-        if (lane < 32) {
-            D = (lane + 1) >> 1;
-            half = (lane & 1) ? 0 : 1;
-        } else {
-            D = 17 + ((lane - 32) >> 1);
-            half = lane & 1;
-        }
-        const int Dh = D < 17 ? D : D - 17;  // dword inside its half-row
-        const int grp = (Dh >> 2) & 3;       // 4-dword group -> k-block (groups 1 and 2 swapped)
-        q_kb = D == 16 ? 0 : (grp == 1 ? 2 : grp == 2 ? 1 : grp);
-        q_mf = D == 16 ? 4 : (D < 16 ? (Dh & 3) : 5 + (Dh & 3));
-        q_half = half;
+        const int i = lane < 31 ? lane + 1 : lane == 31 ? 1 : lane - 32;  // half operand in its half-row, two per dword (D = 0: lanes 0 and 31)
+        const int Dh = i >> 1, grp = Dh >> 2;                               // dword inside its half-row, 4-dword group
+        q_kb = grp == 1 ? 2 : grp == 2 ? 1 : grp;                           // groups 1 and 2 swapped
+        q_mf = (Dh & 3) + (lane < 32 ? 0 : 4);
+        q_half = lane == 0 ? 0 : i & 1;
     }
     static_assert(kColsPerWave == 2 * NT && kWaves == 8, "a packed tile's mirror column col + 8 belongs to the wave of col");
     uint2 packed_prev = {0u, 0u};
@@ -1140,19 +1157,6 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
             packed_prev = packed;
             uint8_t* slot0 = qop + (size_t)(col * 4) * 144;
             *reinterpret_cast<uint2*>(slot0 + q_kb * 144 + q_mf * 16 + q_half * 8) = packed;
-            // the parts no element maps to: the scale nibbles of dword 0 (k-block 0, operand 0,
-            // first half), the second half of operand 4 in k-block 0, operand 4 of k-blocks 1-3
-            if (lane < 8) {
-                int zkb, zoff;
-                if (lane == 0) {
-                    zkb = 0; zoff = 0;
-                } else if (lane == 1) {
-                    zkb = 0; zoff = 4 * 16 + 8;
-                } else {
-                    zkb = 1 + (lane - 2) / 2; zoff = 4 * 16 + 8 * ((lane - 2) & 1);
-                }
-                *reinterpret_cast<uint2*>(slot0 + zkb * 144 + zoff) = uint2{0u, 0u};
-            }
         }
     }
     // The V half of the first unit is requested only now, about 1 us after its K half.  At one
@@ -1168,21 +1172,23 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
     const uint32_t lut_lane = (uint32_t)lane << 2;  // byte 0 of every table address
     const uint8_t* my_qop = qop + (size_t)(n * 4 + b) * 144;
     const uint32_t qop_lane = (uint32_t)(kLutBytes + kWaves * kStageTq4 + (n * 4 + b) * 144);  // its LDS address
-    h8 bq[9];  // the query operands of this lane stay in registers
+    h8 bq[8];  // the query operands of this lane stay in registers
     if constexpr (NT == 1) {
 #pragma unroll
-        for (int mf = 0; mf < 9; ++mf) bq[mf] = *reinterpret_cast<const h8*>(my_qop + 16 * mf);
+        for (int mf = 0; mf < 8; ++mf) bq[mf] = *reinterpret_cast<const h8*>(my_qop + 16 * mf);
     }
 
+    // Until every column has a maximum (`started`) the running maximum of a column without visible keys is 0 and its sum 0.
+    bool started = false;
     f4 o_acc[2][8];
-    float m_run = kNegBig, l_run = 0.f;
+    float m_run = 0.f, l_run = 0.f;
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll
         for (int j = 0; j < 8; ++j) o_acc[h][j] = f4{0.f, 0.f, 0.f, 0.f};
     // (two column tiles) the second one's
     f4 o_acc2[2][8];
-    float m_run2 = kNegBig, l_run2 = 0.f;
+    float m_run2 = 0.f, l_run2 = 0.f;
     if constexpr (NT > 1) {
 #pragma unroll
         for (int h = 0; h < 2; ++h)
@@ -1205,12 +1211,13 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
     auto process_unit = [&](int t0, const bool MASKED, const bool HAS_NEXT) {
         // ---- raw K dwords and K scales -------------------------------------------------------------
         wait_vm<kLoadsPerHalf>();  // this unit's K half has landed (its V half may still be in flight)
-        uint32_t kw[2][9], ksc[2][4];
+        uint32_t kw[2][8], ksc[2][4];
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
             const uint32_t* row32 = reinterpret_cast<const uint32_t*>(ka_lo + s * 8 * kTq4RowBytes);
 #pragma unroll
-            for (int mf = 0; mf < 9; ++mf) kw[s][mf] = row32[tq4_qk_dword(mf < 5 ? 0 : 1, mf < 5 ? mf : mf - 5, b)];
+            for (int mf = 0; mf < 8; ++mf) kw[s][mf] = row32[tq4_qk_dword(mf >> 2, mf & 3, b)];
+            kw[s][0] = tq4_fuse(row32[16], kw[s][0], b == 0);
             // The two scales of token unit_token(s, b, i) in one register, d0 | d1 << 16.  The 16
             // lanes of a row need the same four tokens: lane n reads token n & 3 and the values
             // are handed round inside the row.
@@ -1225,21 +1232,26 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
         if (HAS_NEXT) issue_k();  // nk was located by the caller
 
         // ---- S^T = K Q'^T for the two 16-key sub-tiles ------------------------------------------
-        // Six batches of three operands (twelve table reads, three MFMAs), software-pipelined: the
+        // Eight batches of two operands (eight table reads, two MFMAs), software-pipelined: the
         // table reads of batch k + 1 are requested before the MFMAs of batch k are issued, so the
         // wave does not sit out the LDS latency of every batch.
-        constexpr int kQkOrder[9] = {0, 5, 1, 6, 2, 7, 3, 8, 4};
+        constexpr int kQkOrder[8] = {0, 4, 1, 5, 2, 6, 3, 7};
+        // (log2 domain) minus the running maximum: the sum of the scaled partial scores of a token's half rows starts there
+        auto score = [](const f4 (&part)[2], int i, uint32_t scales, float m) __attribute__((always_inline)) {
+            return __builtin_fmaf(part[1][i], half_hi_to_f32(scales), __builtin_fmaf(part[0][i], half_lo_to_f32(scales), -m));
+        };
+        constexpr int kQkBatch = 2, kQkBatches = 16 / kQkBatch;
         float sc[8], sc2[8];
         if constexpr (NT == 1) {
         f4 s_acc[2][2];
 #pragma unroll
         for (int s = 0; s < 2; ++s) s_acc[s][0] = s_acc[s][1] = f4{0.f, 0.f, 0.f, 0.f};
-        u4 qa[2][3];
-        auto qk_reads = [&](int bt, u4 (&a)[3]) {
-            const int s = bt / 3;
+        u4 qa[2][kQkBatch];
+        auto qk_reads = [&](int bt, u4 (&a)[kQkBatch]) {
 #pragma unroll
-            for (int k = 0; k < 3; ++k) {
-                const uint32_t w = kw[s][kQkOrder[3 * (bt % 3) + k]];
+            for (int k = 0; k < kQkBatch; ++k) {
+                const int at = kQkBatch * bt + k;
+                const uint32_t w = kw[at >> 3][kQkOrder[at & 7]];
                 a[k][0] = lut_read(w, lut_lane, 0x0c0c0400u);
                 a[k][1] = lut_read(w, lut_lane, 0x0c0c0500u);
                 a[k][2] = lut_read(w, lut_lane, 0x0c0c0600u);
@@ -1248,14 +1260,12 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
         };
         qk_reads(0, qa[0]);
 #pragma unroll
-        for (int bt = 0; bt < 6; ++bt) {
-            if (bt + 1 < 6) qk_reads(bt + 1, qa[(bt + 1) & 1]);
+        for (int bt = 0; bt < kQkBatches; ++bt) {
+            if (bt + 1 < kQkBatches) qk_reads(bt + 1, qa[(bt + 1) & 1]);
             __builtin_amdgcn_sched_barrier(0);
-            const int s = bt / 3;
 #pragma unroll
-            for (int k = 0; k < 3; ++k) {
-                const int mf = kQkOrder[3 * (bt % 3) + k];
-                const int h = mf < 5 ? 0 : 1;
+            for (int k = 0; k < kQkBatch; ++k) {
+                const int at = kQkBatch * bt + k, s = at >> 3, mf = kQkOrder[at & 7], h = mf >> 2;
                 s_acc[s][h] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, qa[bt & 1][k]), bq[mf],
                                                                     s_acc[s][h], 0, 0, 0);
             }
@@ -1265,9 +1275,9 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
         for (int s = 0; s < 2; ++s)
 #pragma unroll
             for (int i = 0; i < 4; ++i)
-                sc[4 * s + i] = __builtin_fmaf(s_acc[s][1][i], half_hi_to_f32(ksc[s][i]), mul_by_half_lo(s_acc[s][0][i], ksc[s][i]));
+                sc[4 * s + i] = score(s_acc[s], i, ksc[s][i], m_run);
         } else {
-            // Nine steps of one operand each: eight table reads and the operands of both column tiles (from LDS: with
+            // Eight steps of one operand each: eight table reads and the operands of both column tiles (from LDS: with
             // 128 accumulators they do not fit the registers) a step ahead, four MFMAs.
             f4 s_acc[2][2][2];  // [column tile][sub-tile][half row]
 #pragma unroll
@@ -1291,10 +1301,10 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
             };
             reads(0, ka[0], qb[0]);
 #pragma unroll
-            for (int st = 0; st < 9; ++st) {
-                if (st + 1 < 9) reads(st + 1, ka[(st + 1) & 1], qb[(st + 1) & 1]);
+            for (int st = 0; st < 8; ++st) {
+                if (st + 1 < 8) reads(st + 1, ka[(st + 1) & 1], qb[(st + 1) & 1]);
                 __builtin_amdgcn_sched_barrier(0);
-                const int h = kQkOrder[st] < 5 ? 0 : 1;
+                const int h = kQkOrder[st] >> 2;
 #pragma unroll
                 for (int s = 0; s < 2; ++s)
 #pragma unroll
@@ -1306,8 +1316,8 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
             for (int s = 0; s < 2; ++s)
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    sc[4 * s + i] = __builtin_fmaf(s_acc[0][s][1][i], half_hi_to_f32(ksc[s][i]), mul_by_half_lo(s_acc[0][s][0][i], ksc[s][i]));
-                    sc2[4 * s + i] = __builtin_fmaf(s_acc[1][s][1][i], half_hi_to_f32(ksc[s][i]), mul_by_half_lo(s_acc[1][s][0][i], ksc[s][i]));
+                    sc[4 * s + i] = score(s_acc[0][s], i, ksc[s][i], m_run);
+                    sc2[4 * s + i] = score(s_acc[1][s], i, ksc[s][i], m_run2);
                 }
         }
         if (MASKED) {
@@ -1332,65 +1342,66 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
         uint32_t vsc[8], vw[2][8];
         {
             // lane n reads dwords 0 and 16 of token n & 7 (of the eight this row of lanes works on)
-            // and hands the scale pair and the n = 0 column round inside the row
+            // and hands the scale pair round inside the row
             const uint32_t* r32 = reinterpret_cast<const uint32_t*>(vt_n);
-            const uint32_t d0 = r32[0], d16 = r32[16];
-            const uint32_t mine_sc = __builtin_amdgcn_perm(d16, d0, 0x07060100u);
-            const uint32_t mine_c0 = __builtin_amdgcn_alignbit(d16, d0, 16);
-            uint32_t c0[8];
-            vsc[0] = row_bcast<0>(mine_sc); c0[0] = row_bcast<0>(mine_c0);
-            vsc[1] = row_bcast<1>(mine_sc); c0[1] = row_bcast<1>(mine_c0);
-            vsc[2] = row_bcast<2>(mine_sc); c0[2] = row_bcast<2>(mine_c0);
-            vsc[3] = row_bcast<3>(mine_sc); c0[3] = row_bcast<3>(mine_c0);
-            vsc[4] = row_bcast<4>(mine_sc); c0[4] = row_bcast<4>(mine_c0);
-            vsc[5] = row_bcast<5>(mine_sc); c0[5] = row_bcast<5>(mine_c0);
-            vsc[6] = row_bcast<6>(mine_sc); c0[6] = row_bcast<6>(mine_c0);
-            vsc[7] = row_bcast<7>(mine_sc); c0[7] = row_bcast<7>(mine_c0);
+            const uint32_t mine_sc = __builtin_amdgcn_perm(r32[16], r32[0], 0x07060100u);
+            vsc[0] = row_bcast<0>(mine_sc);
+            vsc[1] = row_bcast<1>(mine_sc);
+            vsc[2] = row_bcast<2>(mine_sc);
+            vsc[3] = row_bcast<3>(mine_sc);
+            vsc[4] = row_bcast<4>(mine_sc);
+            vsc[5] = row_bcast<5>(mine_sc);
+            vsc[6] = row_bcast<6>(mine_sc);
+            vsc[7] = row_bcast<7>(mine_sc);
 #pragma unroll
             for (int t = 0; t < 8; ++t) {
-                const uint32_t* row32 = reinterpret_cast<const uint32_t*>(vt_lo + (8 * (t >> 2) + (t & 3)) * kTq4RowBytes);
-                // (lane n = 0 reads dword 0 and drops it; the read is volatile so that it stays one
-                // unconditional instruction instead of a branch around the lanes with n = 0, and goes
-                // through an LDS-typed address: a volatile read through a generic pointer would be a
-                // FLAT load, which completes out of order with the LDS-direct loads and would break
-                // the hand-placed vmcnt waits)
-                typedef __attribute__((address_space(3))) const volatile uint32_t lds_vol_u32;
-                const uint32_t first_half = *reinterpret_cast<lds_vol_u32*>(
-                    (uintptr_t)(vt_lo_addr + (uint32_t)((8 * (t >> 2) + (t & 3)) * kTq4RowBytes + 4 * n)));
-                vw[0][t] = n == 0 ? c0[t] : first_half;
-                vw[1][t] = row32[17 + n];
+                // (dwords 16 + n and 17 + n by one instruction; the former counts for n = 0 only)
+                const uint32_t* row32 = reinterpret_cast<const uint32_t*>(vt_lo + (8 * (t >> 2) + (t & 3)) * kTq4RowBytes) + n;
+                vw[0][t] = tq4_fuse(row32[16], row32[0], n == 0);
+                vw[1][t] = row32[17];
             }
         }
         wait_lds_reads();
         if (HAS_NEXT) issue_v();
 
-        if constexpr (NT > 1) {
-            float p[8], p2[8];
-            auto softmax = [&](float (&x)[8], float (&pr)[8], float& m, float& l, f4 (&o)[2][8]) __attribute__((always_inline)) {
-                float mx = fmaxf(max3(x[0], x[1], x[2]), max3(x[3], x[4], max3(x[5], x[6], x[7])));
-                mx = max_over_rows(mx);
-                const float m_new = fmaxf(m, mx);
-                const float alpha = __builtin_amdgcn_exp2f(m - m_new);
-                m = m_new;
+        // ---- online softmax (log2 domain), per lane = per query column: scores -> probabilities ----
+        // A column's maximum stays where it is until a unit exceeds it by kPfSlack: most units need no exchange between lanes
+        // and leave the sums alone, and a probability of up to 2^8 keeps its 22 bits.  us, this, eight instead of nine operands (tq4_fuse) and split_weights, before /
+        // now: one token on 131 072 keys 26.5 / 25.9 a layer, eight layers of one on 1 200 126.3 / 124.2, 32 requests of 1 000 to 64 000 125.4 / 124.2.  Exact where that could leave fp16's range, and where the
+        // column does not see the whole unit (what lies behind the sequence must not matter).
+        auto softmax = [&](float (&x)[8], float& m, float& l, f4 (&o)[2][8], int last) __attribute__((always_inline)) {
+            const float mx = fmaxf(max3(x[0], x[1], x[2]), max3(x[3], x[4], max3(x[5], x[6], x[7])));
+            if (!started || __ballot(mx > 0.f) != 0ull) {
+                uint32_t d = 0;  // the largest scales
 #pragma unroll
-                for (int t = 0; t < 8; ++t) pr[t] = __builtin_amdgcn_exp2f(x[t] - m_new);
-                if (MASKED) {
+                for (int t = 0; t < 8; ++t) d = max_u16x2(d, vsc[t] & 0x7FFF7FFFu);
+                const bool large = __ballot((d & 0xFFFFu) > kSlackScaleBits || (d >> 16) > kSlackScaleBits) != 0ull;
+                const float slack = large || (MASKED && !(t0 >= col_lo && t0 + kUnit - 1 <= last)) ? 0.f : kPfSlack;
+                if (!started || __ballot(mx > slack) != 0ull) {
+                    const float top = max_over_rows(mx);
+                    const bool empty = !(sum_over_rows(l) > 0.f);
+                    const float up = empty ? (top > 0.5f * kNegBig ? top : 0.f) : top > slack ? top : 0.f;
+                    const float alpha = empty ? 1.f : __builtin_amdgcn_exp2f(-up);
+                    m += up;
+                    l *= alpha;
 #pragma unroll
-                    for (int t = 0; t < 8; ++t) pr[t] = x[t] > 0.5f * kNegBig ? pr[t] : 0.f;
-                }
-                float psum = 0.f;
-#pragma unroll
-                for (int t = 0; t < 8; ++t) psum += pr[t];
-                l = l * alpha + psum;
-                if (__ballot(alpha != 1.0f) != 0ull) {
+                    for (int t = 0; t < 8; ++t) x[t] -= up;
 #pragma unroll
                     for (int h = 0; h < 2; ++h)
 #pragma unroll
                         for (int j = 0; j < 8; ++j) o[h][j] *= alpha;
                 }
-            };
-            softmax(sc, p, m_run, l_run, o_acc);
-            softmax(sc2, p2, m_run2, l_run2, o_acc2);
+            }
+#pragma unroll
+            for (int t = 0; t < 8; ++t) x[t] = __builtin_amdgcn_exp2f(x[t]);
+            l += ((x[0] + x[1]) + (x[2] + x[3])) + ((x[4] + x[5]) + (x[6] + x[7]));
+        };
+        softmax(sc, m_run, l_run, o_acc, col_hi);
+        if constexpr (NT > 1) softmax(sc2, m_run2, l_run2, o_acc2, col_hi2);
+        started = started || !MASKED;
+        float(&p)[8] = sc;
+        if constexpr (NT > 1) {
+            float(&p2)[8] = sc2;
             if (MASKED) {
                 // (a token masked for one column tile only keeps its scales, which are those of a real row)
 #pragma unroll
@@ -1414,12 +1425,11 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
                 for (int k = 0; k < 4; ++k) {
                     auto w = [&](const float (&pr)[8], int t) { return h == 0 ? mul_by_half_lo(pr[t], vsc[t]) : mul_by_half_hi(pr[t], vsc[t]); };
                     uint32_t whi, wlo;
-                    split_h2(w(p, 2 * k), w(p, 2 * k + 1), whi, wlo);
+                    split_weights(w(p, 2 * k), w(p, 2 * k + 1), whi, wlo);
                     ph[0][k] = whi, pl[0][k] = wlo;
-                    split_h2(w(p2, 2 * k), w(p2, 2 * k + 1), whi, wlo);
+                    split_weights(w(p2, 2 * k), w(p2, 2 * k + 1), whi, wlo);
                     ph[1][k] = whi, pl[1][k] = wlo;
                 }
-                settle(ph[0], ph[1], pl[0], pl[1]);
             };
             auto pv_reads = [&](int bt, u4 (&a)[2]) __attribute__((always_inline)) {
 #pragma unroll
@@ -1454,37 +1464,9 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
             }
             return;
         } else {
-        // ---- online softmax (log2 domain), per lane = per query column --------------------
-        float p[8];
-        {
-            float mx = fmaxf(max3(sc[0], sc[1], sc[2]), max3(sc[3], sc[4], max3(sc[5], sc[6], sc[7])));
-            mx = max_over_rows(mx);
-            const float m_new = fmaxf(m_run, mx);
-            const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
-            m_run = m_new;
-            float psum = 0.f;
-            // (the MASKED tests sit outside the unrolled loops: one wave-uniform branch per block
-            // instead of one per element, and the eight exponentials can overlap)
-#pragma unroll
-            for (int t = 0; t < 8; ++t) p[t] = __builtin_amdgcn_exp2f(sc[t] - m_new);
-            if (MASKED) {
-#pragma unroll
-                for (int t = 0; t < 8; ++t) p[t] = sc[t] > 0.5f * kNegBig ? p[t] : 0.f;
-            }
-#pragma unroll
-            for (int t = 0; t < 8; ++t) psum += p[t];
-            l_run = l_run * alpha + psum;
-            if (__ballot(alpha != 1.0f) != 0ull) {
-#pragma unroll
-                for (int h = 0; h < 2; ++h)
-#pragma unroll
-                    for (int j = 0; j < 8; ++j) o_acc[h][j] *= alpha;
-            }
-        }
-
         // ---- O^T += V^T P^T ------------------------------------------------------------------
         // weights of each half: probability times the half-row scale of the value row, as a high
-        // and a low fp16 operand (split_h2)
+        // and a low fp16 operand (split_weights)
         if (MASKED) {
             // masked tokens have p == 0; their scale pair is zeroed so that a garbage scale (rows
             // beyond the sequence end) cannot inject NaN into the weights
@@ -1501,7 +1483,7 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
                 uint32_t whi, wlo;
-                split_h2(w[2 * k], w[2 * k + 1], whi, wlo);
+                split_weights(w[2 * k], w[2 * k + 1], whi, wlo);
                 ph[h][k] = (pack && (n & 8)) ? wlo : whi;  // packed: the mirror columns take the low-order part
                 pl[h][k] = wlo;
                 const uint32_t wa = vw[h][2 * k], wb = vw[h][2 * k + 1];
@@ -1510,7 +1492,6 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
                 hi[h][k] = ((wa >> 4) & 0x0F0F0F0Fu) | (wb & 0xF0F0F0F0u);
             }
         }
-        settle(ph[0], ph[1], pl[0], pl[1]);
         // four batches of four value tiles (16 table reads, eight MFMAs), pipelined like the QK batches
         u4 va[2][4];
         auto pv_reads = [&](int bt, u4 (&a)[4]) {
@@ -1589,7 +1570,11 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
 
     // ---- combine the per-lane partial sums of l over the four k-block lanes of a column ------
     l_run = sum_over_rows(l_run);
-    if constexpr (NT > 1) l_run2 = sum_over_rows(l_run2);
+    if (l_run == 0.f) m_run = kNegBig;  // (no visible key: must not set the column's maximum)
+    if constexpr (NT > 1) {
+        l_run2 = sum_over_rows(l_run2);
+        if (l_run2 == 0.f) m_run2 = kNegBig;
+    }
 
     // ---- merge the waves' states through LDS ---------------------------------------------------
     // Every wave publishes (m, l) and its O, as it stands, in its own region -- its own staging area,

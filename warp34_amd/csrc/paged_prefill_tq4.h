@@ -46,17 +46,6 @@ static_assert(kPfSmem >= PfLds<WARP34_KV_FORMAT_TQ4>::kEpilogue && kPfSmem <= 16
 static_assert(PfLds<WARP34_KV_FORMAT_TQ4>::kRaw == kStageTq4, "TQ4 raw unit");
 static_assert(kPfWaves * 16 * 264 * 2 <= 2 * kPfDeqBytes, "query staging must fit in the dequant buffers");
 
-// Weights of two operands (TQ4, BF16): a column's running maximum is raised only by scores that exceed it by more than this (log2 domain), so
-// a probability may be up to 2^8; its operands keep 22 (16) bits of it whatever its size, the sums are fp32.  Raising multiplies 64 sums per column
-// tile, and of the first units nearly every one raises the maximum of some column of a wave.  TQ4 value scales ride on the probabilities: in a
-// unit with a larger one than kPfSlackScale, where the weight could leave fp16's range, and where a column does not see the whole unit (what lies
-// behind the sequence must not matter), the maximum is exact.  Per column, so that tiles of either size give the same bits.  (One fp16
-// operand: exact as well, the largest probability is then 1 and rounds to itself; with the slack FP16 and Q8_0 batches came out 6 % further from 64
-// bits, 3.24e-4 for 3.05e-4.)  us, maximum
-// raised by every unit that exceeds it / now: 16 requests of 256 tokens on 2 048 keys BF16 224 / 199, TQ4 261 / 247, 4 of 700 on 6 000 BF16 507 / 459,
-// TQ4 634 / 618, 8 of 2 048 on 16 384 TQ4 6 261 / 6 185.
-constexpr float kPfSlack = 8.0f, kPfSlackScale = 255.0f;
-
 typedef __attribute__((address_space(3))) uint32_t lds_u32;
 
 // 16x16x32 MFMA on fp16 or bf16 operands given as raw bits
@@ -74,16 +63,9 @@ __device__ __forceinline__ float max2(float a, float b) {  // (see max3)
     asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
     return r;
 }
-// High and low fp16 operands of the weights p0 d0 | p1 d1 (see split_h2).  (v_fma_mix_f32 and v_cvt_pk_f16_f32 issue every
-// 4 cycles, v_fma_mixlo_f16 / mixhi every 8.)
+// High and low fp16 operands of the weights p0 d0 | p1 d1
 __device__ __forceinline__ void weight_h2(float p0, float p1, float d0, float d1, uint32_t& hi, uint32_t& lo) {
-    const float w0 = mul_legacy(p0, d0), w1 = mul_legacy(p1, d1);
-    const uint32_t h = pack_h2(w0, w1);
-    float r0, r1;  // (written as fma, the compiler widens the halves with instructions of their own)
-    asm("v_fma_mix_f32 %0, %1, 1.0, -%2 op_sel:[0,0,0] op_sel_hi:[0,0,1]" : "=v"(r0) : "v"(w0), "v"(h));
-    asm("v_fma_mix_f32 %0, %1, 1.0, -%2 op_sel:[0,0,1] op_sel_hi:[0,0,1]" : "=v"(r1) : "v"(w1), "v"(h));
-    hi = h;
-    lo = pack_h2(r0, r1);
+    split_weights(mul_legacy(p0, d0), mul_legacy(p1, d1), hi, lo);
 }
 
 // Which tile a workgroup takes: the n-th longest of the batch.  A causal tile's length is known up to a
@@ -543,7 +525,7 @@ __global__ __launch_bounds__(12 * 64, 1) void paged_prefill_tq4_kernel(const Att
         for (int h = 0; h < 2; ++h) {
             const f4 da = *reinterpret_cast<const f4*>(sc + 64 + 32 * h + 4 * b);
             const f4 db = *reinterpret_cast<const f4*>(sc + 64 + 32 * h + 16 + 4 * b);
-            // high and low fp16 operand (see split_h2): one rounding of p * d would be shared by the
+            // high and low fp16 operand (see split_weights): one rounding of p * d would be shared by the
             // whole 128-element scale block
 #pragma unroll
             for (int k = 0; k < 4; ++k) {

@@ -254,7 +254,7 @@ __global__ __launch_bounds__(kQsaWaves * 64, 1) void qsa_sparse_tq4_kernel(QSA_L
     }
     if (unit0 < cu_end) issue_v(0);
     __syncthreads();  // the table and the query rows are complete
-    h8 bq[9];
+    h8 bq[8];
     {
         const int kb = 8 * (b & 1) + 4 * (b >> 1);
         const uint8_t* qrow = reinterpret_cast<const uint8_t*>(qlds + n * kQStride);
@@ -262,17 +262,11 @@ __global__ __launch_bounds__(kQsaWaves * 64, 1) void qsa_sparse_tq4_kernel(QSA_L
         for (int m = 0; m < 4; ++m) {
             const int D = kb + m;
             u2v lo = *reinterpret_cast<const u2v*>(qrow + (D > 0 ? 16 * D - 8 : 0));
-            if (D == 0) lo = u2v{0u, 0u};
-            const u2v hi = *reinterpret_cast<const u2v*>(qrow + 16 * D);
+            u2v hi = *reinterpret_cast<const u2v*>(qrow + (D > 0 ? 16 * D : 248));  // (D = 0: see tq4_fuse)
             bq[m] = __builtin_bit_cast(h8, u4{lo[0], lo[1], hi[0], hi[1]});
         }
-        {
-            u2v lo = *reinterpret_cast<const u2v*>(qrow + 248);
-            if (b != 0) lo = u2v{0u, 0u};
-            bq[4] = __builtin_bit_cast(h8, u4{lo[0], lo[1], 0u, 0u});
-        }
 #pragma unroll
-        for (int m = 0; m < 4; ++m) bq[5 + m] = *reinterpret_cast<const h8*>(qrow + 256 + 16 * (kb + m));
+        for (int m = 0; m < 4; ++m) bq[4 + m] = *reinterpret_cast<const h8*>(qrow + 256 + 16 * (kb + m));
     }
 
     const uint32_t lut_lane = (uint32_t)lane << 2;
@@ -291,13 +285,14 @@ __global__ __launch_bounds__(kQsaWaves * 64, 1) void qsa_sparse_tq4_kernel(QSA_L
         const uint8_t* v_rows = stage + 2 * kRunBytes;
         wait_vm<kLoads>();  // the K rows have landed (the V rows may still be on their way)
         float sc[8];
-        uint32_t kw[2][9], ks[2][4];
+        uint32_t kw[2][8], ks[2][4];
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
             const int arow = unit_token(s, n >> 2, n & 3);
             const uint32_t* row32 = reinterpret_cast<const uint32_t*>(k_rows + arow * kTq4RowBytes);
 #pragma unroll
-            for (int mf = 0; mf < 9; ++mf) kw[s][mf] = row32[tq4_qk_dword(mf < 5 ? 0 : 1, mf < 5 ? mf : mf - 5, b)];
+            for (int mf = 0; mf < 8; ++mf) kw[s][mf] = row32[tq4_qk_dword(mf >> 2, mf & 3, b)];
+            kw[s][0] = tq4_fuse(row32[16], kw[s][0], b == 0);
             // (the two scales of a token in one register: lane n reads token n & 3, see the dense kernel)
             const uint32_t* r32 = reinterpret_cast<const uint32_t*>(k_rows + unit_token(s, b, n & 3) * kTq4RowBytes);
             const uint32_t mine = __builtin_amdgcn_perm(r32[16], r32[0], 0x07060100u);
@@ -308,16 +303,16 @@ __global__ __launch_bounds__(kQsaWaves * 64, 1) void qsa_sparse_tq4_kernel(QSA_L
         }
         wait_lds_reads();
         if (HAS_NEXT) issue_k(j_next);
-        // six batches of three operands, the table reads of a batch in front of the MFMAs of the one before
-        constexpr int kQkOrder[9] = {0, 5, 1, 6, 2, 7, 3, 8, 4};
+        // eight batches of two operands, the table reads of a batch in front of the MFMAs of the one before
+        constexpr int kQkOrder[8] = {0, 4, 1, 5, 2, 6, 3, 7};
         f4 s_acc[2][2];
 #pragma unroll
         for (int s = 0; s < 2; ++s) s_acc[s][0] = s_acc[s][1] = f4{0.f, 0.f, 0.f, 0.f};
-        u4 qa[2][3];
-        auto qk_reads = [&](int bt, u4 (&a)[3]) __attribute__((always_inline)) {
+        u4 qa[2][2];
+        auto qk_reads = [&](int bt, u4 (&a)[2]) __attribute__((always_inline)) {
 #pragma unroll
-            for (int k = 0; k < 3; ++k) {
-                const uint32_t w = kw[bt / 3][kQkOrder[3 * (bt % 3) + k]];
+            for (int k = 0; k < 2; ++k) {
+                const uint32_t w = kw[bt >> 2][kQkOrder[2 * (bt & 3) + k]];
                 a[k][0] = lut_read(w, lut_lane, 0x0c0c0400u);
                 a[k][1] = lut_read(w, lut_lane, 0x0c0c0500u);
                 a[k][2] = lut_read(w, lut_lane, 0x0c0c0600u);
@@ -326,13 +321,13 @@ __global__ __launch_bounds__(kQsaWaves * 64, 1) void qsa_sparse_tq4_kernel(QSA_L
         };
         qk_reads(0, qa[0]);
 #pragma unroll
-        for (int bt = 0; bt < 6; ++bt) {
-            if (bt + 1 < 6) qk_reads(bt + 1, qa[(bt + 1) & 1]);
+        for (int bt = 0; bt < 8; ++bt) {
+            if (bt + 1 < 8) qk_reads(bt + 1, qa[(bt + 1) & 1]);
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int k = 0; k < 3; ++k) {
-                const int mf = kQkOrder[3 * (bt % 3) + k];
-                f4& acc = s_acc[bt / 3][mf < 5 ? 0 : 1];
+            for (int k = 0; k < 2; ++k) {
+                const int mf = kQkOrder[2 * (bt & 3) + k];
+                f4& acc = s_acc[bt >> 2][mf >> 2];
                 acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, qa[bt & 1][k]), bq[mf], acc, 0, 0, 0);
             }
         }
@@ -353,33 +348,25 @@ __global__ __launch_bounds__(kQsaWaves * 64, 1) void qsa_sparse_tq4_kernel(QSA_L
         } else {
             wait_vm<0>();
         }
-        // Per token: the two scales in one register, the dword of the first half-row that holds this lane's codes (dword n; for
-        // n = 0 codes 0-3 and 124-127 out of dwords 0 and 16) and that of the second; lane n reads dwords 0 and 16
-        // of token n & 7 and hands the scales and the n = 0 column round inside its row of lanes (as in the dense kernel,
-        // the volatile read and its LDS-typed address too).
+        // Per token: the two scales in one register (lane n reads those of token n & 7 and hands them round inside its row of lanes),
+        // the dword of the first half-row that holds this lane's codes (dword n, see tq4_fuse) and that of the second.
         uint32_t vsc[8], vw[2][8];
         {
             const uint32_t* r32 = reinterpret_cast<const uint32_t*>(v_rows + unit_token((n >> 2) & 1, b, n & 3) * kTq4RowBytes);
-            const uint32_t d0 = r32[0], d16 = r32[16];
-            const uint32_t mine_sc = __builtin_amdgcn_perm(d16, d0, 0x07060100u);
-            const uint32_t mine_c0 = __builtin_amdgcn_alignbit(d16, d0, 16);
-            uint32_t c0[8];
-            vsc[0] = row_bcast<0>(mine_sc); c0[0] = row_bcast<0>(mine_c0);
-            vsc[1] = row_bcast<1>(mine_sc); c0[1] = row_bcast<1>(mine_c0);
-            vsc[2] = row_bcast<2>(mine_sc); c0[2] = row_bcast<2>(mine_c0);
-            vsc[3] = row_bcast<3>(mine_sc); c0[3] = row_bcast<3>(mine_c0);
-            vsc[4] = row_bcast<4>(mine_sc); c0[4] = row_bcast<4>(mine_c0);
-            vsc[5] = row_bcast<5>(mine_sc); c0[5] = row_bcast<5>(mine_c0);
-            vsc[6] = row_bcast<6>(mine_sc); c0[6] = row_bcast<6>(mine_c0);
-            vsc[7] = row_bcast<7>(mine_sc); c0[7] = row_bcast<7>(mine_c0);
+            const uint32_t mine_sc = __builtin_amdgcn_perm(r32[16], r32[0], 0x07060100u);
+            vsc[0] = row_bcast<0>(mine_sc);
+            vsc[1] = row_bcast<1>(mine_sc);
+            vsc[2] = row_bcast<2>(mine_sc);
+            vsc[3] = row_bcast<3>(mine_sc);
+            vsc[4] = row_bcast<4>(mine_sc);
+            vsc[5] = row_bcast<5>(mine_sc);
+            vsc[6] = row_bcast<6>(mine_sc);
+            vsc[7] = row_bcast<7>(mine_sc);
 #pragma unroll
             for (int t = 0; t < 8; ++t) {
-                const int row = unit_token(t >> 2, b, t & 3) * kTq4RowBytes;
-                typedef __attribute__((address_space(3))) const volatile uint32_t lds_vol_u32;
-                const uint32_t first_half =
-                    *reinterpret_cast<lds_vol_u32*>((uintptr_t)(stage_addr + (uint32_t)(2 * kRunBytes + row + 4 * n)));
-                vw[0][t] = n == 0 ? c0[t] : first_half;
-                vw[1][t] = reinterpret_cast<const uint32_t*>(v_rows + row)[17 + n];
+                const uint32_t* row32 = reinterpret_cast<const uint32_t*>(v_rows + unit_token(t >> 2, b, t & 3) * kTq4RowBytes) + n;
+                vw[0][t] = tq4_fuse(row32[16], row32[0], n == 0);
+                vw[1][t] = row32[17];
             }
         }
         wait_lds_reads();
@@ -409,7 +396,7 @@ __global__ __launch_bounds__(kQsaWaves * 64, 1) void qsa_sparse_tq4_kernel(QSA_L
                     for (int j = 0; j < 8; ++j) o_acc[h][j] *= alpha;
             }
         }
-        // probability times the half-row scale of the value row, as a high and a low fp16 operand (split_h2): one rounding
+        // probability times the half-row scale of the value row, as a high and a low fp16 operand (split_weights): one rounding
         // would be shared by the whole scale block.  (Masked tokens have p == 0; a garbage scale must not reach the weights.)
         if (MASKED) {
 #pragma unroll
@@ -425,7 +412,7 @@ __global__ __launch_bounds__(kQsaWaves * 64, 1) void qsa_sparse_tq4_kernel(QSA_L
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
                 uint32_t whi, wlo;
-                split_h2(w[2 * k], w[2 * k + 1], whi, wlo);
+                split_weights(w[2 * k], w[2 * k + 1], whi, wlo);
                 ph[h][k] = whi;
                 pl[h][k] = wlo;
                 const uint32_t wa = vw[h][2 * k], wb = vw[h][2 * k + 1];
@@ -433,7 +420,6 @@ __global__ __launch_bounds__(kQsaWaves * 64, 1) void qsa_sparse_tq4_kernel(QSA_L
                 hi[h][k] = ((wa >> 4) & 0x0F0F0F0Fu) | (wb & 0xF0F0F0F0u);
             }
         }
-        settle(ph[0], ph[1], pl[0], pl[1]);
         // four batches of four value tiles, the table reads of a batch in front of the MFMAs of the one before
         u4 va[2][4];
         auto pv_reads = [&](int bt, u4 (&a)[4]) __attribute__((always_inline)) {
