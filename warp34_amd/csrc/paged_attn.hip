@@ -346,16 +346,19 @@ __device__ __forceinline__ void wht256_wave(float (&v)[4], int lane) {
     for (int k = 0; k < 4; ++k) v[k] *= 0.0625f;
 }
 
-// centroid k as an immediate select chain (no constant-memory load on the critical path)
-__device__ __forceinline__ float centroid_imm(int k) {
-    const float m = (k & 4) ? ((k & 2) ? ((k & 1) ? 1.694104124e-1f : 1.285881878e-1f)
-                                       : ((k & 1) ? 1.006979993e-1f : 7.824930800e-2f))
-                            : ((k & 2) ? ((k & 1) ? 5.873210384e-2f : 4.094919437e-2f)
-                                       : ((k & 1) ? 2.420087619e-2f : 8.008373692e-3f));
-    return m;  // magnitude of centroid 8 + k; centroid[7 - k] = -m
+// Entry bits of a code: fp16(kLutGain * centroid), by two byte permutes over immediates (no constant-memory load on the critical path; a chain of selects
+// is sixty instructions with branches).  Magnitude k is that of centroids 8 + k and 7 - k.
+__host__ __device__ constexpr uint32_t centroid_bits_of(int code) { return __builtin_bit_cast(uint16_t, (_Float16)(kLutGain * kCentroids[code])); }
+__host__ __device__ constexpr uint32_t magnitude_bytes(int first, int shift) {  // byte `shift / 8` of four magnitudes
+    uint32_t r = 0;
+    for (int k = 0; k < 4; ++k) r |= (centroid_bits_of(8 + first + k) >> shift & 0xFFu) << (8 * k);
+    return r;
 }
-__device__ __forceinline__ float centroid_of_code(int code) {
-    return (code & 8) ? centroid_imm(code & 7) : -centroid_imm(7 - (code & 7));
+__device__ __forceinline__ uint32_t centroid_bits(uint32_t code) {
+    constexpr uint32_t lo0 = magnitude_bytes(0, 0), lo4 = magnitude_bytes(4, 0), hi0 = magnitude_bytes(0, 8), hi4 = magnitude_bytes(4, 8);
+    const bool negative = (code & 8u) == 0u;
+    const uint32_t k = (negative ? ~code : code) & 7u;
+    return __builtin_amdgcn_perm(lo4, lo0, k | 0x0c0c0c00u) | __builtin_amdgcn_perm(hi4, hi0, k << 8 | 0x0c0c000cu) | (negative ? 0x8000u : 0u);
 }
 
 __device__ __forceinline__ uint32_t pack_h2(float a, float b) {
@@ -452,15 +455,13 @@ __device__ __forceinline__ uint32_t lut_read(uint32_t code_word, uint32_t lut_la
 // The pair table, by 512 threads: entry e = (gain*centroid[e & 15], gain*centroid[e >> 4]) as packed fp16, 64 copies of 4 bytes.
 // Thread t writes the 16-byte slots t + 512 i (conflict-free), i.e. entries (t >> 4) + 32 i:
 // their low code (t >> 4) & 15 is the thread's own, their high code (t >> 8) + 2 i is the
-// same in the whole wave.  Lane j < 16 computes centroid j once; everything else is lane
-// traffic, so the build costs a few dozen instructions per wave.
-__device__ __forceinline__ void build_pair_table(uint8_t* smem, int tid, int lane, int wave) {
-    const uint32_t c_bits = (uint32_t)F16::from_f32(kLutGain * centroid_of_code(lane & 15));
-    const uint32_t lo = (uint32_t)__builtin_amdgcn_ds_bpermute(((tid >> 4) & 15) << 2, (int)c_bits);
+// same in the whole wave, one of two immediates.
+__device__ __forceinline__ void build_pair_table(uint8_t* smem, int tid, int wave) {
+    const uint32_t lo = centroid_bits((uint32_t)tid >> 4 & 15u);
+    const bool odd = (wave >> 2) != 0;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-        const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)c_bits, (wave >> 2) + 2 * i);
-        const uint32_t v = lo | (hi << 16);
+        const uint32_t v = lo | (odd ? centroid_bits_of(2 * i + 1) << 16 : centroid_bits_of(2 * i) << 16);
         *reinterpret_cast<u4*>(smem + (tid + 512 * i) * 16) = u4{v, v, v, v};
     }
 }
@@ -737,7 +738,9 @@ __device__ __forceinline__ void wait_lds_reads() { asm volatile("s_waitcnt lgkmc
 // SP: the keys below *P.key_floor belong to a shared-prefix pass (see AttnParams); a separate
 // instantiation, so that the plain form carries no trace of it.
 // NT: column tiles of 16 (two: batches with neither a token mask nor a window).
-template <typename TQ, bool BAL, bool SP = false, bool STREAM = BAL, int NT = 1>
+// PLAIN: split-K form of a batch whose requests have one tile of at most eight columns each, all q heads of a kv head in it, without masks and window, page
+// strides below 4 GiB (plain_decode): what follows from the host's bounds on it is worked out while the lengths travel.
+template <typename TQ, bool BAL, bool SP = false, bool STREAM = BAL, int NT = 1, bool PLAIN = false>
 __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, const BalItem& item, bool build_table) {
     static_assert(!(SP && BAL), "shared-prefix pass: split-K form only");
     constexpr int kWaves = kTq4Waves;
@@ -758,8 +761,8 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
     // with a prefix sum over the requests' tile counts.
     const int tile_z = BAL || SP ? item.req : (int)blockIdx.z;
     const int kv_sub = (int)blockIdx.y;
-    const int kv_head = small_div(kv_sub, P.q_subgroups);
-    const int q_head_base = kv_head * P.gqa + (kv_sub - kv_head * P.q_subgroups) * P.q_group;
+    const int kv_head = PLAIN ? kv_sub : small_div(kv_sub, P.q_subgroups);
+    const int q_head_base = PLAIN ? kv_sub * P.q_group : kv_head * P.gqa + (kv_sub - kv_head * P.q_subgroups) * P.q_group;
     const int chunk = BAL ? 0 : SP ? item.slot : (int)blockIdx.x;
 
     // The request lookup goes first: its loads head the longest dependency chain of the prologue
@@ -784,11 +787,11 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
         if (slot < B.max_blocks_per_req) spec_vec = B.block_tables[(size_t)req * B.max_blocks_per_req + slot];
     } else {
         // a request by the launch geometry, or the guess that all requests have as many tiles as the longest
-        req = P.tiles_by_request ? tile_z : min(fast_div(tile_z, P.bal_tiles), B.num_reqs - 1);
+        req = PLAIN || P.tiles_by_request ? tile_z : min(fast_div(tile_z, P.bal_tiles), B.num_reqs - 1);
         // Speculative block-table load, in flight together with the request's lengths: it
         // assumes that the request's length is the host's bound max_seq_len.  When the guess is
         // wrong the ids are fetched again below, so it changes the latency only, never the result.
-        if (!SP && B.sliding_window <= 0 && B.max_seq_len > 0) {
+        if (PLAIN || (!SP && B.sliding_window <= 0 && B.max_seq_len > 0)) {
             spec_slot_base = div_block(chunk * P.spec_upc * kUnit, P);
             const int slot = spec_slot_base + lane;
             if (slot < B.max_blocks_per_req)
@@ -797,7 +800,17 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
         // one vector load per array (all lanes the same address), no scalar-cache round trip;
         // the values are made scalar after the table has been built, so that the build overlaps
         // the round trip
-        if (P.tiles_by_request) {
+        if constexpr (PLAIN) {
+            // (a lane value in the index: the compiler would take scalar loads, whose wait is one for all of them and the arguments, in
+            // front of the query rows and the table)
+            int at = req;
+            asm volatile("" : "+v"(at));
+            a_lo = B.query_start_loc[at];
+            a_hi = B.query_start_loc[at + 1];
+            a_sa = B.seq_lens_after[at];
+            a_cb = B.context_lens_before[at];
+            a_rm = 1;
+        } else if (P.tiles_by_request) {
             a_lo = B.query_start_loc[req];
             a_hi = B.query_start_loc[req + 1];
             a_sa = B.seq_lens_after[req];
@@ -811,12 +824,12 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
     // the table.  The first token of the tile is guessed (exact when every request has a whole
     // number of tiles); a wrong guess is corrected after the lookup.
     const int tok_guess = BAL ? item.rq_start + item.tile * P.tok_tile
-                              : min(P.tiles_by_request ? tile_z : tile_z * P.tok_tile, B.total_tokens - 1);
+                              : min(PLAIN || P.tiles_by_request ? tile_z : tile_z * P.tok_tile, B.total_tokens - 1);
     constexpr int kColsPerWave = (16 * NT + kWaves - 1) / kWaves;
     uint2 q_raw[kColsPerWave];
     auto load_q = [&](int tokbase) {
 #pragma unroll
-        for (int c = 0; c < kColsPerWave; ++c) {
+        for (int c = 0; c < (PLAIN ? 1 : kColsPerWave); ++c) {
             const int col = wave + c * kWaves;
             const int t = div_q_group(col, P);
             const int a = col - t * P.q_group;
@@ -834,7 +847,7 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
     auto load_tok_ok_col = [&](int tokbase, int column) {
         const int tok = tokbase + div_q_group(column, P);
         tok_ok = tok < B.total_tokens &&
-                 (B.valid_token_mask == nullptr || B.valid_token_mask[min(tok, B.total_tokens - 1)] != 0);
+                 (PLAIN || B.valid_token_mask == nullptr || B.valid_token_mask[min(tok, B.total_tokens - 1)] != 0);
     };
     auto load_tok_ok = [&](int tokbase) {
         if constexpr (NT == 1) load_tok_ok_col(tokbase, n);
@@ -842,27 +855,37 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
     load_tok_ok(tok_guess);
 
     if (build_table) {
-        // (build_pair_table's text: as a call, one request on 1 200 keys takes 13.4 us instead of 12.8)
         static_assert(kWaves == 8, "table build: 512 threads");
-        const uint32_t c_bits = (uint32_t)F16::from_f32(kLutGain * centroid_of_code(lane & 15));
-        const uint32_t lo = (uint32_t)__builtin_amdgcn_ds_bpermute(((tid >> 4) & 15) << 2, (int)c_bits);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)c_bits, (wave >> 2) + 2 * i);
-            const uint32_t v = lo | (hi << 16);
-            *reinterpret_cast<u4*>(smem + (tid + 512 * i) * 16) = u4{v, v, v, v};
-        }
+        build_pair_table(smem, tid, wave);
     }
 
-    if (!BAL && P.tiles_by_request) {
+    // PLAIN: the first unit of this wave if the request is as long as the host's bound, its runs' places in the pages and the slabs
+    const int simd = wave & 3, wslot = wave >> 2;
+    uint32_t spec_in_page[2] = {0u, 0u};
+    int spec_rel[2] = {0, 0};
+    uint64_t k_slab = 0, v_slab = 0;
+    if constexpr (PLAIN) {
+        k_slab = L.k_base + (uint64_t)(uint32_t)kv_head * L.k_head_stride_bytes;
+        v_slab = L.v_base + (uint64_t)(uint32_t)kv_head * L.v_head_stride_bytes;
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+            const int pos = (chunk * P.spec_upc + 4 * wslot + simd) * kUnit + 16 * r;
+            const int slot = div_block(pos, P);
+            spec_rel[r] = slot - spec_slot_base;
+            spec_in_page[r] = (uint32_t)(pos - slot * L.block_size) * (uint32_t)kTq4RowBytes;
+            asm volatile("" : "+s"(spec_rel[r]), "+s"(spec_in_page[r]));
+        }
+        asm volatile("" : "+s"(k_slab), "+s"(v_slab));
+    }
+    if (!BAL && (PLAIN || P.tiles_by_request)) {
         rq_start = __builtin_amdgcn_readfirstlane(a_lo);
         rq_end = __builtin_amdgcn_readfirstlane(a_hi);
         seq_after = __builtin_amdgcn_readfirstlane(a_sa);
-        ctx_before = B.context_lens_before != nullptr ? __builtin_amdgcn_readfirstlane(a_cb)
-                                                      : seq_after - (rq_end - rq_start);
+        ctx_before = PLAIN || B.context_lens_before != nullptr ? __builtin_amdgcn_readfirstlane(a_cb)
+                                                               : seq_after - (rq_end - rq_start);
         req_hit = __builtin_amdgcn_readfirstlane(a_rm) != 0 && rq_end > rq_start;
     }
-    if (!BAL && !P.tiles_by_request) {
+    if (!BAL && !PLAIN && !P.tiles_by_request) {
         const TileInfo ti = locate_tile_of(P, tile_z, lane, a_req);
         if (ti.req != req) spec_slot_base = -1;
         req = ti.req;
@@ -888,7 +911,7 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
     // carry the LOW-order fp16 part of the value weights where columns 0-7 carry the high-order
     // part, so one MFMA per value tile does the work of two.  The two halves are added up before
     // the waves merge.
-    const bool pack = NT == 1 && tile_tokens * P.q_group <= 8;  // wave-uniform
+    const bool pack = PLAIN || (NT == 1 && tile_tokens * P.q_group <= 8);  // wave-uniform
     const int ncol = pack ? (n & 7) : n;             // the query column this lane works for
     if (pack && ncol != n) load_tok_ok_col(tok0, ncol);
 
@@ -904,7 +927,7 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
     int u_lo = 0x7fffffff, u_hi = -1;  // union of the visible ranges
     int i_lo = 0, i_hi = 0x7fffffff;   // intersection of the visible ranges
     uint32_t ok_mask = 0u;             // bit c: column c is live (wave-uniform)
-    const bool simple = NT > 1 || (B.valid_token_mask == nullptr && B.sliding_window <= 0);
+    const bool simple = PLAIN || NT > 1 || (B.valid_token_mask == nullptr && B.sliding_window <= 0);
     // keys below the floor were handled by the shared-prefix pass (a multiple of the unit size)
     int key_floor = 0;
     if constexpr (SP) key_floor = __builtin_amdgcn_readfirstlane(*P.key_floor);
@@ -926,10 +949,10 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
         const int tok = tok0 + t;
         const bool ok = t < tile_tokens && tok_ok;
         const int q_off = tok - rq_start;
-        int mx = (B.mask_mode == WARP34_ATTN_MASK_NONCAUSAL_WINDOW) ? seq_after - 1 : ctx_before + q_off;
+        int mx = (!PLAIN && B.mask_mode == WARP34_ATTN_MASK_NONCAUSAL_WINDOW) ? seq_after - 1 : ctx_before + q_off;
         if (mx >= seq_after) mx = seq_after - 1;
         int mn = key_floor;
-        if (B.sliding_window > 0) mn = max(key_floor, ctx_before + q_off - B.sliding_window + 1);
+        if (!PLAIN && B.sliding_window > 0) mn = max(key_floor, ctx_before + q_off - B.sliding_window + 1);
         col_ok = ok;
         col_lo = ok ? mn : 0;
         col_hi = ok ? mx : -1;
@@ -946,7 +969,7 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
     if (simple) {
         if (tok0 >= B.total_tokens) return;  // no live column
         const int q_off0 = tok0 - rq_start;
-        const bool window = B.mask_mode == WARP34_ATTN_MASK_NONCAUSAL_WINDOW;
+        const bool window = !PLAIN && B.mask_mode == WARP34_ATTN_MASK_NONCAUSAL_WINDOW;
         int hi_first = window ? seq_after - 1 : ctx_before + q_off0;
         int hi_last = window ? seq_after - 1 : ctx_before + q_off0 + tile_tokens - 1;
         if (hi_first >= seq_after) hi_first = seq_after - 1;
@@ -974,6 +997,7 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
 
     ChunkGeom g;
     int cu_first, cu_end;
+    bool as_guessed = false;
     if constexpr (BAL) {
         // the plan counted the units of [0, u_hi]: the batch has no window and no token mask
         g = ChunkGeom{0, (u_hi >> 5) + 1, 0, item.n_chunks};
@@ -982,6 +1006,7 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
     } else {
         if (u_lo == 0 && B.max_seq_len > 0 && u_hi == B.max_seq_len - 1) {
             g = ChunkGeom{0, P.spec_units, P.spec_upc, P.spec_chunks};  // as long as the host's bound
+            as_guessed = true;
         } else {
             g = chunk_geom(u_lo, u_hi, P.max_chunks, P.few_chunks);
         }
@@ -992,10 +1017,15 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
     }
 
     // ---- staging machinery ----------------------------------------------------------------------
-    const uint8_t* k_base = reinterpret_cast<const uint8_t*>((uintptr_t)L.k_base) +
-                            (size_t)kv_head * L.k_head_stride_bytes;
-    const uint8_t* v_base = reinterpret_cast<const uint8_t*>((uintptr_t)L.v_base) +
-                            (size_t)kv_head * L.v_head_stride_bytes;
+    const uint8_t* k_base;
+    const uint8_t* v_base;
+    if constexpr (PLAIN) {
+        k_base = reinterpret_cast<const uint8_t*>((uintptr_t)k_slab);
+        v_base = reinterpret_cast<const uint8_t*>((uintptr_t)v_slab);
+    } else {
+        k_base = reinterpret_cast<const uint8_t*>((uintptr_t)L.k_base) + (size_t)kv_head * L.k_head_stride_bytes;
+        v_base = reinterpret_cast<const uint8_t*>((uintptr_t)L.v_base) + (size_t)kv_head * L.v_head_stride_bytes;
+    }
     const uint32_t stage_addr = (uint32_t)(kLutBytes + wave * kStageTq4);  // LDS byte address (the block starts at 0)
     uint8_t* stage = stage_all + wave * kStageTq4;
 
@@ -1060,6 +1090,12 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
             }
             const int32_t pg = __builtin_amdgcn_readlane(page_vec, rel);
             const bool live = pos <= u_hi && pos + 15 >= u_lo && pg >= 0;
+            if constexpr (PLAIN) {
+                const uint64_t tok_off = (uint64_t)((uint32_t)in_page * (uint32_t)kTq4RowBytes);
+                nk[gidx] = k_base + (live ? (uint64_t)(uint32_t)pg * (uint32_t)L.k_page_stride_bytes + tok_off : 0);
+                nv[gidx] = v_base + (live ? (uint64_t)(uint32_t)pg * (uint32_t)L.v_page_stride_bytes + tok_off : 0);
+                continue;
+            }
             const size_t koff = live ? (size_t)pg * L.k_page_stride_bytes + (size_t)in_page * L.k_token_stride_bytes : 0;
             const size_t voff = live ? (size_t)pg * L.v_page_stride_bytes + (size_t)in_page * L.v_token_stride_bytes : 0;
             nk[gidx] = k_base + koff;
@@ -1089,7 +1125,6 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
     // on every run and under every page permutation.  The rule deals the units to the four
     // SIMDs in turn and, inside a SIMD, to its waves in turn (wave w runs on SIMD w mod 4): with
     // a wave count that is not a multiple of four the SIMDs still get equal shares.
-    const int simd = wave & 3, wslot = wave >> 2;
     const int simd_waves = (kWaves - simd + 3) / 4;
     auto nth_unit = [&](int j) -> int { return cu_first + 4 * (wslot + simd_waves * j) + simd; };
 
@@ -1104,9 +1139,19 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
     // order, so a wait for them placed behind those loads would wait for the K / V data as well:
     // the (empty) statement makes the compiler finish its own loads here, where they have long landed.
 #pragma unroll
-    for (int c = 0; c < kColsPerWave; ++c) asm volatile("" ::"v"(q_raw[c].x), "v"(q_raw[c].y));
+    for (int c = 0; c < (PLAIN ? 1 : kColsPerWave); ++c) asm volatile("" ::"v"(q_raw[c].x), "v"(q_raw[c].y));
     if (unit < cu_end) {
-        locate_unit(unit);
+        if (PLAIN && as_guessed) {  // (spec_rel < 64: the first eight units of a chunk, 256 tokens of pages of 16 and more)
+#pragma unroll
+            for (int r = 0; r < 2; ++r) {
+                const int32_t pg = __builtin_amdgcn_readlane(page_vec, spec_rel[r]);
+                const bool live = unit * kUnit + 16 * r <= u_hi && pg >= 0;
+                nk[r] = k_base + (live ? (uint64_t)(uint32_t)pg * (uint32_t)L.k_page_stride_bytes + spec_in_page[r] : 0);
+                nv[r] = v_base + (live ? (uint64_t)(uint32_t)pg * (uint32_t)L.v_page_stride_bytes + spec_in_page[r] : 0);
+            }
+        } else {
+            locate_unit(unit);
+        }
         issue_k();  // (its V half follows below, behind the query operands)
     }
     if (simple) column_info(false);
@@ -1760,14 +1805,24 @@ __global__ __launch_bounds__(kTq4Waves * 64, 1) void paged_attn_tq4_kernel(const
     }
 }
 
+// Decode steps without masks, see plain_decode; the bits of the general kernel.  What bounds a short one is the chain lengths - addresses - first rows: device
+// timestamps, one token on 1 200 keys, from the wave's entry: lengths there 1.16 us, addresses 1.72, first rows asked for 2.17 in the general kernel, most of it
+// scalar instructions, which eight waves issue one after the other.  us, general / this: one token on 1 200 keys, eight layers with their producers, 124.2 / 115.2, one on
+// 131 072, four layers, 92.0 / 88.8.
+template <typename TQ>
+__global__ __launch_bounds__(kTq4Waves * 64, 1) void paged_attn_tq4_plain_kernel(const AttnParams P) {
+    extern __shared__ __align__(16) uint8_t smem[];
+    tq4_tile<TQ, false, false, true, 1, true>(P, smem, BalItem{}, true);
+}
+
 // The private rest of a verify batch with more than 16 query columns per request and kv head: both column tiles in one workgroup, so that
 // a key is looked up once for 32 columns (a wave's unit: 465 vector instructions and 100 MFMAs, one tile 330 and 50).  Issue bounds it, so the loads keep their
 // plain form: with the streaming hint 3 % slower.  `wide` holds the geometry of that form, whose chunks join the prefix's records, for which there is room
 // whatever their number; with nothing shared, `P`, that of the plain path, whose bits the batch then has.  us, 16 requests x 4 tokens on 262 144 keys, 200 000 of
 // them shared, one column tile / two: whole call 524 / 486, on another box 534 / 512; this kernel 177 / 147.
 template <typename TQ>
-__global__ __launch_bounds__(kTq4Waves * 64, 1) void paged_attn_tq4_private_kernel(int chunks, int tiles, int wide_chunks, int wide_tiles,
-                                                                                   const AttnParams P, const AttnParams wide) {
+__global__ __launch_bounds__(kTq4Waves * 64, 1) void paged_attn_tq4_private_kernel(const AttnParams P, const AttnParams wide, int chunks, int tiles,
+                                                                                   int wide_chunks, int wide_tiles) {
     extern __shared__ __align__(16) uint8_t smem[];
     const int wg = (int)blockIdx.x;
     BalItem item{};
@@ -2683,6 +2738,14 @@ static int shared_prefix_parts(int total_tokens, int q_group, int q_subgroups) {
     return parts < 1 ? 1 : (parts > 32 ? 32 : parts);
 }
 
+// Batches for the kernel that knows this of them.
+static bool plain_decode(const AttnParams& P) {
+    const warp34_attention_batch& B = P.B;
+    return P.tiles_by_request != 0 && P.q_subgroups == 1 && B.max_q_len * P.q_group <= 8 && B.max_seq_len > 0 && B.sliding_window <= 0 && B.mask_mode == WARP34_ATTN_MASK_CAUSAL &&
+           B.valid_token_mask == nullptr && B.valid_req_mask == nullptr && B.context_lens_before != nullptr &&
+           P.L.k_page_stride_bytes <= 0xFFFFFFFFull && P.L.v_page_stride_bytes <= 0xFFFFFFFFull;
+}
+
 template <typename TQ>
 static int launch_tq4(const warp34_exec* ex, const warp34_kv_layer_layout* layout,
                       const warp34_attention_batch* batch, const void* q, void* out, int num_q_heads,
@@ -2801,7 +2864,7 @@ static int launch_tq4(const warp34_exec* ex, const warp34_kv_layer_layout* layou
                 if (rc) return rc;
                 const long long wgs = std::max((long long)grid_x * grid_z, (long long)W.max_chunks * tiles);
                 hipLaunchKernelGGL(paged_attn_tq4_private_kernel<TQ>, dim3((unsigned)wgs, (unsigned)kv_subs), dim3(kTq4Waves * 64),
-                                   smem_bytes_for(2), stream, grid_x, grid_z, W.max_chunks, tiles, P, W);
+                                   smem_bytes_for(2), stream, P, W, grid_x, grid_z, W.max_chunks, tiles);
             } else {
                 rc = ensure_dynamic_lds(paged_attn_tq4_kernel<TQ, true>, smem_bytes_for(1), true);
                 if (rc) return rc;
@@ -2834,9 +2897,10 @@ static int launch_tq4(const warp34_exec* ex, const warp34_kv_layer_layout* layou
         return launch_balanced_merge<TQ, kHeadDim>(P, kv_subs, kLutInvGain, stream);
     }
     P.bal_tiles = tiles_per_request_bound(*batch, P);
-    rc = ensure_dynamic_lds(paged_attn_tq4_kernel<TQ>, smem_bytes_for(1), true);
+    const auto kernel = plain_decode(P) ? paged_attn_tq4_plain_kernel<TQ> : paged_attn_tq4_kernel<TQ>;
+    rc = ensure_dynamic_lds(kernel, smem_bytes_for(1), true);
     if (rc) return rc;
-    hipLaunchKernelGGL(paged_attn_tq4_kernel<TQ>, grid, dim3(kTq4Waves * 64), smem_bytes_for(1), stream, P);
+    hipLaunchKernelGGL(kernel, grid, dim3(kTq4Waves * 64), smem_bytes_for(1), stream, P);
     rc = (int)hipGetLastError();
     if (rc) return rc;
     return P.max_chunks > 1 ? launch_split_merge<TQ, false, kHeadDim>(P, P.max_chunks, kLutInvGain, stream) : 0;

@@ -175,7 +175,7 @@ __global__ __launch_bounds__(12 * 64, 1) void paged_prefill_tq4_kernel(const Att
     // ---- the pair table (64 lane replicas, as in the decode kernel) ----
     if (tid < kPfWaves * 64) {
         const int e = tid >> 1;
-        const uint32_t v = pack_h2(kLutGain * centroid_of_code(e & 15), kLutGain * centroid_of_code(e >> 4));
+        const uint32_t v = centroid_bits((uint32_t)e & 15u) | centroid_bits((uint32_t)e >> 4) << 16;
         u4 vv = {v, v, v, v};
         u4* dst = reinterpret_cast<u4*>(smem + e * 256 + (tid & 1) * 128);
 #pragma unroll

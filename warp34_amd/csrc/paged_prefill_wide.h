@@ -130,7 +130,7 @@ __device__ __forceinline__ void pw_tile(const AttnParams& P, uint8_t* smem, int 
     // ---- the pair table (64 lane replicas, as in the decode kernel) ----
     if (TQ4F) {
         const int e = tid >> 1;
-        const uint32_t v = pack_h2(kLutGain * centroid_of_code(e & 15), kLutGain * centroid_of_code(e >> 4));
+        const uint32_t v = centroid_bits((uint32_t)e & 15u) | centroid_bits((uint32_t)e >> 4) << 16;
         u4 vv = {v, v, v, v};
         u4* dst = reinterpret_cast<u4*>(smem + e * 256 + (tid & 1) * 128);
 #pragma unroll

@@ -168,7 +168,7 @@ __global__ __launch_bounds__(kQsaWaves * 64, 1) void qsa_sparse_tq4_kernel(QSA_L
     qsa_have_arguments(P);
     int a_live = 1;
     if (P.valid_token_mask != nullptr) a_live = (int)P.valid_token_mask[tok];
-    build_pair_table(smem, tid, lane, wave);
+    build_pair_table(smem, tid, wave);
 
     int n_sel = __builtin_amdgcn_readfirstlane(a_live) != 0 ? __builtin_amdgcn_readfirstlane(a_sel) : 0;
     if (n_sel > select_k) n_sel = select_k;
