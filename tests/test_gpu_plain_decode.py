@@ -5,7 +5,7 @@ import pytest
 
 import oracle
 from cases import make_case
-from oracle import DT_BF16, DT_F16, FMT_TQ4
+from oracle import DT_BF16, DT_F16, FMT_BF16, FMT_FP16, FMT_FP8, FMT_Q8_0, FMT_TQ4
 
 pytestmark = pytest.mark.gpu
 
@@ -43,3 +43,39 @@ def test_bytes_of_the_general_kernel(case, dtype):
     assert outs[0].tobytes() == outs[1].tobytes()
     want = oracle.paged_attention(pool, hb, q, dtype, q_heads)
     G.assert_close(outs[0], dtype, want, what="plain decode", scale=G.channel_scale(v, dtype, hb, q_heads))
+
+
+# format, type, head dimension, then as above, and the mask mode (1: the tokens of a draft block see each other both ways)
+ROWS = [
+    (FMT_Q8_0, DT_F16, 256, 16, 2, 16, [1200], [1], 0, 0),
+    (FMT_Q8_0, DT_BF16, 256, 64, 2, 16, [1200], [1], 5000, 0),
+    (FMT_Q8_0, DT_F16, 256, 112, 1, 8, [1], [1], 0, 0),
+    (FMT_FP8, DT_F16, 256, 48, 2, 16, [769], [1], 770, 0),
+    (FMT_FP8, DT_BF16, 256, 16, 4, 4, [700, 9, 2500, 64], [1, 0, 1, 1], 10000, 0),
+    (FMT_Q8_0, DT_F16, 256, 16, 2, 16, [2000], [4], 0, 0),               # two tiles
+    (FMT_FP8, DT_F16, 256, 64, 1, 16, [300, 1000, 77], [3, 5, 1], 0, 0),  # tiles of one token, not as many in every request
+    (FMT_FP16, DT_F16, 256, 16, 2, 16, [1700], [3], 0, 0),
+    (FMT_BF16, DT_BF16, 256, 64, 2, 16, [500, 1030], [4, 2], 2000, 0),
+    (FMT_BF16, DT_BF16, 128, 16, 4, 16, [700, 500], [16, 16], 0, 1),
+    (FMT_BF16, DT_BF16, 128, 16, 4, 16, [65, 300, 17], [8, 16, 5], 0, 1),
+    (FMT_FP16, DT_F16, 128, 32, 2, 8, [900], [6], 901, 0),
+]
+
+
+@pytest.mark.parametrize("case", range(len(ROWS)))
+def test_row_formats(case):
+    import gpu_harness as G
+
+    fmt, dtype, head_dim, block, kv_heads, q_heads, seqs, q_lens, bound, mask_mode = ROWS[case]
+    pool, bt, k, v, q, aq, ctx = make_case(fmt, block, seqs, q_lens, 3200 + case, dtype, kv_heads=kv_heads, q_heads=q_heads, head_dim=head_dim)
+    hb = oracle.HostBatch(aq, seqs, bt, context_lens_before=ctx, mask_mode=mask_mode)
+    dpool = G.DevPool(pool)
+    dpool.upload()
+    outs = []
+    for batch in (hb, oracle.HostBatch(aq, seqs, bt, mask_mode=mask_mode)):
+        rc, got, _ = G.dev_attention(dpool, batch, q, dtype, q_heads, scratch_bytes=64 << 20, max_seq_len=bound or None)
+        assert rc == 0
+        outs.append(got)
+    assert outs[0].tobytes() == outs[1].tobytes()
+    want = oracle.paged_attention(pool, hb, q, dtype, q_heads)
+    G.assert_close(outs[0], dtype, want, what="plain rows", scale=G.channel_scale(v, dtype, hb, q_heads), plain_excess=0.0 if fmt in (FMT_FP16, FMT_BF16) else 4e-4)

@@ -618,6 +618,8 @@ struct TileInfo {
 struct TileReq {
     int lo, hi, sa, cb, rm;
 };
+// PLAIN: the batch has context_lens_before and no request mask
+template <bool PLAIN = false>
 __device__ __forceinline__ TileReq load_tile_req(const AttnParams& P, int base, int lane) {
     const warp34_attention_batch& B = P.B;
     const int r = base + lane;
@@ -626,19 +628,20 @@ __device__ __forceinline__ TileReq load_tile_req(const AttnParams& P, int base, 
     q.lo = inb ? B.query_start_loc[r] : 0;
     q.hi = inb ? B.query_start_loc[r + 1] : 0;
     q.sa = inb ? B.seq_lens_after[r] : 0;
-    q.cb = (inb && B.context_lens_before != nullptr) ? B.context_lens_before[r] : 0;
-    q.rm = (inb && B.valid_req_mask != nullptr) ? (int)B.valid_req_mask[r] : 1;
+    q.cb = (inb && (PLAIN || B.context_lens_before != nullptr)) ? B.context_lens_before[r] : 0;
+    q.rm = (inb && !PLAIN && B.valid_req_mask != nullptr) ? (int)B.valid_req_mask[r] : 1;
     return q;
 }
 // Tile tile_z by the requests' tile counts; q: the first 64 requests (load_tile_req), which a kernel with other work to do meanwhile
 // asks for ahead.  The sum over the lanes by DPP moves; by LDS permutes, with the requests asked for here: us a call, 4 tokens each,
 // Q8_0 1 request on 16 000 keys 18.8 -> 18.3, TQ4 20.0 -> 19.5, 1 on 1 000 16.6 -> 16.2.
+template <bool PLAIN = false>
 __device__ __forceinline__ TileInfo locate_tile_of(const AttnParams& P, int tile_z, int lane, TileReq q) {
     const warp34_attention_batch& B = P.B;
     TileInfo t{false, -1, 0, 0, 0, 0, 0};
     int tiles_before = 0;
     for (int base = 0; base < B.num_reqs; base += 64) {
-        if (base > 0) q = load_tile_req(P, base, lane);
+        if (base > 0) q = load_tile_req<PLAIN>(P, base, lane);
         const int cnt = q.hi > q.lo ? fast_div(q.hi - q.lo + P.tok_tile - 1, P.tok_tile) : 0;
         const int incl = wave_incl_scan(cnt);
         const int first = tiles_before + incl - cnt;
@@ -649,8 +652,8 @@ __device__ __forceinline__ TileInfo locate_tile_of(const AttnParams& P, int tile
             t.rq_start = __builtin_amdgcn_readlane(q.lo, src);
             t.rq_end = __builtin_amdgcn_readlane(q.hi, src);
             t.seq_after = __builtin_amdgcn_readlane(q.sa, src);
-            t.ctx_before = B.context_lens_before != nullptr ? __builtin_amdgcn_readlane(q.cb, src)
-                                                            : t.seq_after - (t.rq_end - t.rq_start);
+            t.ctx_before = PLAIN || B.context_lens_before != nullptr ? __builtin_amdgcn_readlane(q.cb, src)
+                                                                     : t.seq_after - (t.rq_end - t.rq_start);
             t.tile_in_req = tile_z - __builtin_amdgcn_readlane(first, src);
             t.hit = __builtin_amdgcn_readlane(q.rm, src) != 0;
             return t;
@@ -801,14 +804,10 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
         // the values are made scalar after the table has been built, so that the build overlaps
         // the round trip
         if constexpr (PLAIN) {
-            // (a lane value in the index: the compiler would take scalar loads, whose wait is one for all of them and the arguments, in
-            // front of the query rows and the table)
-            int at = req;
-            asm volatile("" : "+v"(at));
-            a_lo = B.query_start_loc[at];
-            a_hi = B.query_start_loc[at + 1];
-            a_sa = B.seq_lens_after[at];
-            a_cb = B.context_lens_before[at];
+            a_lo = B.query_start_loc[req];
+            a_hi = B.query_start_loc[req + 1];
+            a_sa = B.seq_lens_after[req];
+            a_cb = B.context_lens_before[req];
             a_rm = 1;
         } else if (P.tiles_by_request) {
             a_lo = B.query_start_loc[req];
@@ -1807,8 +1806,8 @@ __global__ __launch_bounds__(kTq4Waves * 64, 1) void paged_attn_tq4_kernel(const
 
 // Decode steps without masks, see plain_decode; the bits of the general kernel.  What bounds a short one is the chain lengths - addresses - first rows: device
 // timestamps, one token on 1 200 keys, from the wave's entry: lengths there 1.16 us, addresses 1.72, first rows asked for 2.17 in the general kernel, most of it
-// scalar instructions, which eight waves issue one after the other.  us, general / this: one token on 1 200 keys, eight layers with their producers, 124.2 / 115.2, one on
-// 131 072, four layers, 92.0 / 88.8.
+// scalar instructions, which eight waves issue one after the other.  us, general / this: one token on 1 200 keys, eight layers with their producers, 124.2 / 114.5, one on
+// 131 072, four layers, 99.6 / 95.3.
 template <typename TQ>
 __global__ __launch_bounds__(kTq4Waves * 64, 1) void paged_attn_tq4_plain_kernel(const AttnParams P) {
     extern __shared__ __align__(16) uint8_t smem[];
@@ -2738,13 +2737,19 @@ static int shared_prefix_parts(int total_tokens, int q_group, int q_subgroups) {
     return parts < 1 ? 1 : (parts > 32 ? 32 : parts);
 }
 
-// Batches for the kernel that knows this of them.
-static bool plain_decode(const AttnParams& P) {
+// Batches for the kernels that know this of them.
+static bool plain_batch(const AttnParams& P) {
     const warp34_attention_batch& B = P.B;
-    return P.tiles_by_request != 0 && P.q_subgroups == 1 && B.max_q_len * P.q_group <= 8 && B.max_seq_len > 0 && B.sliding_window <= 0 && B.mask_mode == WARP34_ATTN_MASK_CAUSAL &&
-           B.valid_token_mask == nullptr && B.valid_req_mask == nullptr && B.context_lens_before != nullptr &&
-           P.L.k_page_stride_bytes <= 0xFFFFFFFFull && P.L.v_page_stride_bytes <= 0xFFFFFFFFull;
+    return P.q_subgroups == 1 && B.max_seq_len > 0 && B.sliding_window <= 0 && B.valid_token_mask == nullptr && B.valid_req_mask == nullptr &&
+           B.context_lens_before != nullptr && P.L.k_page_stride_bytes <= 0xFFFFFFFFull && P.L.v_page_stride_bytes <= 0xFFFFFFFFull;
 }
+static bool plain_decode(const AttnParams& P) {
+    return plain_batch(P) && P.tiles_by_request != 0 && P.B.max_q_len * P.q_group <= 8 && P.B.mask_mode == WARP34_ATTN_MASK_CAUSAL;
+}
+// Row formats: 8-bit rows, and 16-bit rows of several tiles per request (one tile: within 1 %, the rows themselves are what takes the time).  us, general / plain: eight layers
+// of one token on 1 200 keys Q8_0 116.0 / 110.9, FP8 119.2 / 113.4, with their producers; four requests of 1 000 to 3 000 Q8_0 93.4 / 86.6; one token on 20 000 Q8_0
+// 120.9 / 113.6; 4 tokens on 2 000 Q8_0 127.8 / 121.1; five layers of 4 x 16 draft tokens 115.3 / 114.2.
+static bool plain_rows(const AttnParams& P) { return plain_batch(P) && P.key_groups == 0 && P.first_round == 0 && P.rot_q == 0; }
 
 template <typename TQ>
 static int launch_tq4(const warp34_exec* ex, const warp34_kv_layer_layout* layout,
@@ -3125,8 +3130,14 @@ static int launch_rows(const warp34_exec* ex, const warp34_kv_layer_layout* layo
     P.first_round = HD != kHeadDim ? rows_first_round(*batch, P, kv_subs, grid_z) : 0;
     if (P.key_groups > 0) grid = dim3((unsigned)(kXcds * P.bal_tiles), (unsigned)((P.key_groups + kXcds - 1) / kXcds));
     constexpr int smem = rows_smem_bytes<KVF, HD>(1);
-    const auto kernel = P.key_groups > 0 || P.first_round > 0 ? paged_attn_rows_mapped_kernel<TQ, KVF, VRES, HD>
-                                                              : paged_attn_rows_kernel<TQ, KVF, VRES, HD>;
+    auto kernel = P.key_groups > 0 || P.first_round > 0 ? paged_attn_rows_mapped_kernel<TQ, KVF, VRES, HD>
+                                                        : paged_attn_rows_kernel<TQ, KVF, VRES, HD>;
+    if constexpr (!VRES) {
+        if (plain_rows(P)) {
+            if (P.tiles_by_request == 0) kernel = paged_attn_rows_plain_kernel<TQ, KVF, HD, false>;
+            else if constexpr (RowsLds<KVF, HD>::k8) kernel = paged_attn_rows_plain_kernel<TQ, KVF, HD, true>;
+        }
+    }
     rc = ensure_dynamic_lds(kernel, smem, true);
     if (rc) return rc;
     hipLaunchKernelGGL(kernel, grid, dim3(kKv16Waves * 64), smem, stream, P);

@@ -212,7 +212,9 @@ __device__ __forceinline__ void lds_load_half(uint32_t voffset, const uint8_t* s
 // one 128-element half: four QK operands instead of eight, eight value tiles instead of sixteen,
 // and lanes 0-31 carry a finished row.  The split-K partial records keep their 256-float stride.
 // MAPPED: chunk grid whose workgroups go by keys or by length (rows_by_keys, rows_longest_first), else in launch order.
-template <typename TQ, int NT, int KVF, bool BAL, bool VRES = false, bool STREAM = BAL, int HD = kHeadDim, bool MAPPED = false>
+// PLAIN: chunk grid in launch order of a batch without masks and window, all q heads of a kv head in a tile, queries as given, page strides below 4 GiB
+// (plain_rows): what follows from the host's bounds on it is worked out while the lengths travel.  STREAM: and one tile per request.
+template <typename TQ, int NT, int KVF, bool BAL, bool VRES = false, bool STREAM = BAL, int HD = kHeadDim, bool MAPPED = false, bool PLAIN = false>
 __device__ __forceinline__ void rows_tile(const AttnParams& P, uint8_t* smem, const BalItem& item) {
     static_assert(!VRES || KVF == WARP34_KV_FORMAT_FP8_E4M3 || KVF == WARP34_KV_FORMAT_Q8_0, "residual operand: 8-bit rows");
     using M = RowsLds<KVF, HD>;
@@ -249,18 +251,18 @@ __device__ __forceinline__ void rows_tile(const AttnParams& P, uint8_t* smem, co
             if (P.first_round > 0) tile_z = rows_longest_first(P, lane, tile_z);
         }
     }
-    const int kv_head = small_div(kv_sub, P.q_subgroups);
-    const int q_head_base = kv_head * P.gqa + (kv_sub - kv_head * P.q_subgroups) * P.q_group;
+    const int kv_head = PLAIN ? kv_sub : small_div(kv_sub, P.q_subgroups);
+    const int q_head_base = PLAIN ? kv_sub * P.q_group : kv_head * P.gqa + (kv_sub - kv_head * P.q_subgroups) * P.q_group;
 
     // Query rows in MFMA B layout: lane (n, b) holds Q[column n][32 m + 8 b .. + 7] for m = 0..kM-1.
     // One tile of un-rotated queries comes straight from global memory into registers; the first
     // token of the tile is guessed so that these loads overlap the lookup, a wrong guess is corrected
     // after it.  Rotated queries and several tiles go through the LDS table below.
-    const bool rot_q = K8 && P.rot_q != 0;  // workgroup-uniform
+    const bool rot_q = !PLAIN && K8 && P.rot_q != 0;  // workgroup-uniform
     const bool q_direct = NT == 1 && !rot_q;
     const int tok_tile = BAL ? item.tok_tile : P.tok_tile;
     const int tok_guess = BAL ? item.rq_start + item.tile * tok_tile
-                              : min(P.tiles_by_request ? tile_z : tile_z * tok_tile, B.total_tokens - 1);
+                              : min((PLAIN ? STREAM : P.tiles_by_request != 0) ? tile_z : tile_z * tok_tile, B.total_tokens - 1);
     u4 bq[kM];
     auto load_q = [&](int tokbase) {
         const int t = div_q_group(n, P);
@@ -270,6 +272,20 @@ __device__ __forceinline__ void rows_tile(const AttnParams& P, uint8_t* smem, co
 #pragma unroll
         for (int m = 0; m < kM; ++m) bq[m] = *reinterpret_cast<const u4*>(qrow + 32 * m + 8 * b);
     };
+    // PLAIN: the lengths and the block-table slice are asked for first, the query rows behind them.
+    TileReq a_req{};
+    int spec_slot_base = -1, spec_vec = -1, req_guess = tile_z;
+    if constexpr (PLAIN) {
+        if constexpr (STREAM) {
+            a_req = TileReq{B.query_start_loc[tile_z], B.query_start_loc[tile_z + 1], B.seq_lens_after[tile_z], B.context_lens_before[tile_z], 1};
+        } else {
+            a_req = load_tile_req<true>(P, 0, lane);
+            req_guess = min(fast_div(tile_z, P.bal_tiles), B.num_reqs - 1);
+        }
+        spec_slot_base = div_block(chunk * P.spec_upc * kUnit, P);
+        const int slot = spec_slot_base + lane;
+        if (slot < B.max_blocks_per_req) spec_vec = B.block_tables[(size_t)req_guess * B.max_blocks_per_req + slot];
+    }
     if (q_direct) {
         load_q(tok_guess);
     } else {
@@ -281,8 +297,8 @@ __device__ __forceinline__ void rows_tile(const AttnParams& P, uint8_t* smem, co
     // request's length is the host's bound max_seq_len and, where a request may have several tiles, that all
     // requests have as many.  A wrong guess is fetched again below, so it changes the latency only, never the result.
     // (4 requests x 16 tokens on 1 000 keys, head dimension 128, with the producer: 18.5 -> 17.4 us a layer.)
-    int spec_slot_base = -1, spec_vec = -1, req_guess = tile_z;
-    if constexpr (BAL) {
+    if constexpr (PLAIN) {
+    } else if constexpr (BAL) {
         // the piece's first unit is known: its block-table slice is requested with the query rows
         spec_slot_base = div_block(item.u_begin * kUnit, P);
         const int slot = spec_slot_base + lane;
@@ -294,8 +310,26 @@ __device__ __forceinline__ void rows_tile(const AttnParams& P, uint8_t* smem, co
         if (slot < B.max_blocks_per_req)
             spec_vec = B.block_tables[(size_t)req_guess * B.max_blocks_per_req + slot];
     }
+    // PLAIN: the first half of this wave if the request is as long as the host's bound, its place in its page, and the slabs
+    uint32_t spec_in_page = 0;
+    int spec_rel = 0;
+    uint64_t k_slab = 0, v_slab = 0;
+    if constexpr (PLAIN) {
+        k_slab = L.k_base + (uint64_t)(uint32_t)kv_head * L.k_head_stride_bytes;
+        v_slab = L.v_base + (uint64_t)(uint32_t)kv_head * L.v_head_stride_bytes;
+        const int pos = chunk * P.spec_upc * kUnit + 16 * wave;
+        const int slot = div_block(pos, P);
+        spec_rel = slot - spec_slot_base;
+        spec_in_page = (uint32_t)(pos - slot * L.block_size) * (uint32_t)kRowBytes;
+        asm volatile("" : "+s"(spec_rel), "+s"(spec_in_page), "+s"(k_slab), "+s"(v_slab));
+    }
     TileInfo ti;
-    if constexpr (BAL) {
+    if constexpr (PLAIN && STREAM) {
+        const int lo = __builtin_amdgcn_readfirstlane(a_req.lo), hi = __builtin_amdgcn_readfirstlane(a_req.hi);
+        ti = TileInfo{hi > lo, tile_z, lo, hi, __builtin_amdgcn_readfirstlane(a_req.sa), __builtin_amdgcn_readfirstlane(a_req.cb), 0};
+    } else if constexpr (PLAIN) {
+        ti = locate_tile_of<true>(P, tile_z, lane, a_req);
+    } else if constexpr (BAL) {
         ti = TileInfo{true, item.req, item.rq_start, item.rq_end, item.seq_after, item.ctx_before, item.tile};
     } else {
         ti = locate_tile(P, tile_z, lane);
@@ -321,7 +355,7 @@ __device__ __forceinline__ void rows_tile(const AttnParams& P, uint8_t* smem, co
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
         const int tok = tok0 + div_q_group(nt * 16 + n, P);
-        tok_ok[nt] = tok < B.total_tokens && (BAL || B.valid_token_mask == nullptr ||
+        tok_ok[nt] = tok < B.total_tokens && (BAL || PLAIN || B.valid_token_mask == nullptr ||
                                               B.valid_token_mask[min(tok, B.total_tokens - 1)] != 0);
     }
     int tile_tokens = rq_end - tok0;
@@ -343,7 +377,7 @@ __device__ __forceinline__ void rows_tile(const AttnParams& P, uint8_t* smem, co
         ok_mask[nt] = 0u;
     }
     // (a balanced batch has neither, see launch_rows_balanced)
-    const bool simple = BAL || (B.valid_token_mask == nullptr && B.sliding_window <= 0);
+    const bool simple = BAL || PLAIN || (B.valid_token_mask == nullptr && B.sliding_window <= 0);
     auto column_info = [&](bool accumulate) {
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) {
@@ -355,7 +389,7 @@ __device__ __forceinline__ void rows_tile(const AttnParams& P, uint8_t* smem, co
             int mx = (B.mask_mode == WARP34_ATTN_MASK_NONCAUSAL_WINDOW) ? seq_after - 1 : ctx_before + q_off;
             if (mx >= seq_after) mx = seq_after - 1;
             int mn = 0;
-            if (!BAL && B.sliding_window > 0) mn = max(0, ctx_before + q_off - B.sliding_window + 1);
+            if (!BAL && !PLAIN && B.sliding_window > 0) mn = max(0, ctx_before + q_off - B.sliding_window + 1);
             col_ok[nt] = ok;
             col_lo[nt] = ok ? mn : 0;
             col_hi[nt] = ok ? mx : -1;
@@ -409,6 +443,7 @@ __device__ __forceinline__ void rows_tile(const AttnParams& P, uint8_t* smem, co
 
     ChunkGeom g;
     int cu_first, cu_end;
+    bool as_guessed = false;
     if constexpr (BAL) {
         // the plan counted the units of [0, u_hi]: the batch has no window and no token mask
         g = ChunkGeom{0, (u_hi >> 5) + 1, 0, item.n_chunks};
@@ -417,6 +452,7 @@ __device__ __forceinline__ void rows_tile(const AttnParams& P, uint8_t* smem, co
     } else {
         if (u_lo == 0 && B.max_seq_len > 0 && u_hi == B.max_seq_len - 1) {
             g = ChunkGeom{0, P.spec_units, P.spec_upc, P.spec_chunks};  // as long as the host's bound
+            as_guessed = true;
         } else {
             g = chunk_geom(u_lo, u_hi, P.max_chunks, P.few_chunks);
         }
@@ -427,10 +463,15 @@ __device__ __forceinline__ void rows_tile(const AttnParams& P, uint8_t* smem, co
     }
 
     // ---- staging: LDS-direct loads of half units, K and V one half ahead ------------------------------
-    const uint8_t* k_base = reinterpret_cast<const uint8_t*>((uintptr_t)L.k_base) +
-                            (size_t)kv_head * L.k_head_stride_bytes;
-    const uint8_t* v_base = reinterpret_cast<const uint8_t*>((uintptr_t)L.v_base) +
-                            (size_t)kv_head * L.v_head_stride_bytes;
+    const uint8_t* k_base;
+    const uint8_t* v_base;
+    if constexpr (PLAIN) {
+        k_base = reinterpret_cast<const uint8_t*>((uintptr_t)k_slab);
+        v_base = reinterpret_cast<const uint8_t*>((uintptr_t)v_slab);
+    } else {
+        k_base = reinterpret_cast<const uint8_t*>((uintptr_t)L.k_base) + (size_t)kv_head * L.k_head_stride_bytes;
+        v_base = reinterpret_cast<const uint8_t*>((uintptr_t)L.v_base) + (size_t)kv_head * L.v_head_stride_bytes;
+    }
     uint8_t* stage = smem + wave * M::kStage;
     const uint8_t* k_rows = stage;
     const uint8_t* v_rows = stage + M::kKeyBytes;
@@ -474,6 +515,12 @@ __device__ __forceinline__ void rows_tile(const AttnParams& P, uint8_t* smem, co
         }
         const int32_t pg = __builtin_amdgcn_readlane(page_vec, rel);
         const bool live = pos <= u_hi && pos + 15 >= u_lo && pg >= 0;
+        if constexpr (PLAIN) {
+            const uint32_t in_bytes = (uint32_t)in_page * (uint32_t)kRowBytes;
+            next_k = k_base + (live ? (uint64_t)(uint32_t)pg * (uint32_t)L.k_page_stride_bytes + in_bytes : 0);
+            next_v = v_base + (live ? (uint64_t)(uint32_t)pg * (uint32_t)L.v_page_stride_bytes + in_bytes : 0);
+            return;
+        }
         next_k = k_base + (live ? (size_t)pg * L.k_page_stride_bytes + (size_t)in_page * L.k_token_stride_bytes : 0);
         next_v = v_base + (live ? (size_t)pg * L.v_page_stride_bytes + (size_t)in_page * L.v_token_stride_bytes : 0);
     };
@@ -773,7 +820,13 @@ __device__ __forceinline__ void rows_tile(const AttnParams& P, uint8_t* smem, co
     asm volatile("" ::"v"(page_vec));
     auto first_rows = [&]() {
         if (hidx < h_end) {
-            locate_half(hidx);
+            if (PLAIN && as_guessed && slot_base == spec_slot_base && ti.req == req_guess) {  // (spec_rel < 64: eight halves from the chunk's start on)
+                const int32_t pg = __builtin_amdgcn_readlane(page_vec, spec_rel);
+                next_k = k_base + (pg >= 0 ? (uint64_t)(uint32_t)pg * (uint32_t)L.k_page_stride_bytes + spec_in_page : 0);
+                next_v = v_base + (pg >= 0 ? (uint64_t)(uint32_t)pg * (uint32_t)L.v_page_stride_bytes + spec_in_page : 0);
+            } else {
+                locate_half(hidx);
+            }
             issue_k();
             issue_v();
         }
@@ -952,6 +1005,12 @@ __global__ __launch_bounds__(kKv16Waves * 64, 1) void paged_attn_rows_kernel(con
     } else {
         rows_tile<TQ, 1, KVF, false, VRES, false, HD>(P, smem, BalItem{});
     }
+}
+// Without masks and windows, in launch order, see plain_rows; the bits of the kernel above.
+template <typename TQ, int KVF, int HD, bool ONE_TILE>
+__global__ __launch_bounds__(kKv16Waves * 64, 1) void paged_attn_rows_plain_kernel(const AttnParams P) {
+    extern __shared__ __align__(16) uint8_t smem[];
+    rows_tile<TQ, 1, KVF, false, false, ONE_TILE, HD, false, true>(P, smem, BalItem{});
 }
 // The chunk grid by keys or by length.  (A kernel of its own: with the order worked out in the other, or a third body in it, chunks of 130 tokens
 // over bf16 pages, which stay in launch order, took 4 to 5 % longer with the same instructions in the loop: 67.9 -> 71.8 us.)
