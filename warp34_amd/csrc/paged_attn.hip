@@ -491,6 +491,16 @@ __device__ __forceinline__ constexpr int tq4_pv_elem(int h, int j, int r) {
     return 8 * r - 4 + j;
 }
 
+// Elements 4 lane .. 4 lane + 3 in the order of the code dwords: twice the dword inside its half-row plus the half of it.  (Lanes 0 and 31, elements 0..3 and
+// 124..127, are the halves of the fused dword, see tq4_fuse.)
+__device__ __forceinline__ int tq4_half_dword(int lane) { return lane < 32 ? (lane == 0 || lane == 31 ? lane & 1 : lane + 1) : lane - 32; }
+// Merge regions: slot of element 4 lane; element 4 lane + k: + 16 k (inverse of tq4_pv_elem).  (Worked out element by element, with a branch for
+// each kind of lane, it was 150 instructions in front of the workgroup's barrier.)
+__device__ __forceinline__ int tq4_merge_slot(int lane) {
+    const int i = tq4_half_dword(lane), r = i >> 1;
+    return (((lane >> 5) * 8 + 4 * (i & 1)) * 4 + (r >> 2)) * 4 + (r & 3);
+}
+
 constexpr int kMergeGroups = 16;
 // Up to this many chunks one wave per row adds them up (split_merge_few_kernel); kMergeFewRows where it stands for four waves, not sixteen
 // (merge_small_groups).  us a call, sixteen waves / one: nine to sixteen chunks, one request of 2 000 keys TQ4 11.7 / 11.3, Q8_0 11.2 / 10.8, of 1 000
@@ -716,11 +726,11 @@ __device__ __forceinline__ void lds_load_run(uint32_t voffset, const uint8_t* sb
             : "memory");
     }
 }
-// lane L of every row of 16 lanes, in all lanes of that row (one VALU move)
 // value of the lane eight places on inside the row of 16 lanes (DPP row_ror:8)
 __device__ __forceinline__ float row_ror8(float v) {
     return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x128, 0xF, 0xF, true));
 }
+// lane L of every row of 16 lanes, in all lanes of that row (one VALU move)
 template <int L>
 __device__ __forceinline__ uint32_t row_bcast(uint32_t v) {
     return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x150 + L, 0xF, 0xF, true);  // row_newbcast:L
@@ -730,6 +740,35 @@ __device__ __forceinline__ void wait_vm() {
     asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory");
 }
 __device__ __forceinline__ void wait_lds_reads() { asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory"); }
+
+// Packed tile: columns n and n + 8 += each other (the high-order and the low-order share of the weights), in both lanes.  (The empty statement keeps the
+// sums here: moved behind a branch they would be an exchange and a sum.)
+__device__ __forceinline__ void add_mirror_columns(f4 (&o)[2][8]) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                float x = o[h][j][k];
+                x += row_ror8(x);
+                asm volatile("" : "+v"(x));
+                o[h][j][k] = x;
+            }
+}
+// ... and a column's values into its merge region: lane n < 8 the value tiles with even j, lane n + 8 those with odd j.  (The comments in assembly keep
+// the branches' stores apart: joined, they take an address inside the array, which then lies in scratch memory.)
+__device__ __forceinline__ void store_packed_column(float* c, const f4 (&o)[2][8], int n, int b) {
+    if (n < 8) {
+#pragma unroll
+        for (int t = 0; t < 16; t += 2) *reinterpret_cast<f4*>(c + (t * 4 + b) * 4) = o[t >> 3][t & 7];
+        asm volatile("; even tiles");
+    } else {
+#pragma unroll
+        for (int t = 1; t < 16; t += 2) *reinterpret_cast<f4*>(c + (t * 4 + b) * 4) = o[t >> 3][t & 7];
+        asm volatile("; odd tiles");
+    }
+}
 
 // The work of one workgroup on one tile.  BAL = false: the tile and the chunk come from
 // blockIdx (grid = chunks x (kv head, q subgroup) x tiles).  BAL = true: they come from `item`
@@ -1168,11 +1207,11 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
     // where this lane's four elements go: operand (k-block, mf) and which half of it
     int q_kb, q_mf, q_half;
     {
-        const int i = lane < 31 ? lane + 1 : lane == 31 ? 1 : lane - 32;  // half operand in its half-row, two per dword (D = 0: lanes 0 and 31)
+        const int i = tq4_half_dword(lane);
         const int Dh = i >> 1, grp = Dh >> 2;                               // dword inside its half-row, 4-dword group
         q_kb = grp == 1 ? 2 : grp == 2 ? 1 : grp;                           // groups 1 and 2 swapped
         q_mf = (Dh & 3) + (lane < 32 ? 0 : 4);
-        q_half = lane == 0 ? 0 : i & 1;
+        q_half = i & 1;
     }
     static_assert(kColsPerWave == 2 * NT && kWaves == 8, "a packed tile's mirror column col + 8 belongs to the wave of col");
     uint2 packed_prev = {0u, 0u};
@@ -1594,23 +1633,7 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
     __builtin_amdgcn_s_setprio(0);
     wait_vm<0>();  // nothing of this wave may still be on its way into LDS when the areas are reused
 
-    // ---- packed tile: column n += its mirror column n + 8 (the low-order share of the weights) ----
-    // Both lanes of a pair end up with sums, and both take part in the stores below: lane n < 8 keeps
-    // the value tiles with even j in the even slots, its mirror lane those with odd j.
-    if (pack) {
-        const bool upper = (n & 8) != 0;
-#pragma unroll
-        for (int h = 0; h < 2; ++h)
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    const float even = o_acc[h][2 * i][k], odd = o_acc[h][2 * i + 1][k];
-                    const float keep = upper ? odd : even;   // this lane's tile of the pair
-                    const float give = upper ? even : odd;   // what the mirror lane keeps
-                    o_acc[h][2 * i][k] = keep + row_ror8(give);
-                }
-    }
+    if (pack) add_mirror_columns(o_acc);
 
     // ---- combine the per-lane partial sums of l over the four k-block lanes of a column ------
     l_run = sum_over_rows(l_run);
@@ -1651,14 +1674,8 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
     }
     auto store_region = [&](int half) {
         float* c = xbuf + wave * kRegion + (n & 7) * kColStride;
-        if (pack) {  // (half 0) all 64 lanes store: eight tiles each, see above
-            if (col_ok) {
-#pragma unroll
-                for (int h = 0; h < 2; ++h)
-#pragma unroll
-                    for (int i = 0; i < 4; ++i)
-                        *reinterpret_cast<f4*>(c + ((h * 8 + 2 * i + (n >> 3)) * 4 + b) * 4) = o_acc[h][2 * i];
-            }
+        if (pack) {  // (half 0)
+            if (col_ok) store_packed_column(c, o_acc, n, b);
         } else if ((n >> 3) == half && col_ok) {  // dead columns are never read back
 #pragma unroll
             for (int h = 0; h < 2; ++h)
@@ -1670,26 +1687,11 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
     // (two column tiles: a live column is in the first eight, the tile's live ones lie without a gap from column 0 on)
     store_region(NT > 1 || live0 ? 0 : 1);
 
-    int merge_slot[4];  // region slot of element 4*lane + k (inverse of tq4_pv_elem)
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        const int e = 4 * lane + k;
-        int h, j, r;
-        if (e >= 128) {
-            h = 1; r = (e - 128) >> 3; j = e & 7;
-        } else if (e < 4) {
-            h = 0; r = 0; j = e;
-        } else if (e >= 124) {
-            h = 0; r = 0; j = e - 120;
-        } else {
-            h = 0; r = (e + 4) >> 3; j = (e + 4) & 7;
-        }
-        merge_slot[k] = ((h * 8 + j) * 4 + (r >> 2)) * 4 + (r & 3);
-    }
     __syncthreads();  // every wave is done with the table, and the regions of the first pass are there
 #pragma unroll 1
-    for (int half = 0; half < 2 * NT; ++half) {
-        if constexpr (NT > 1) {
+    for (int half = 0; half < (PLAIN ? 1 : 2 * NT); ++half) {
+        if constexpr (PLAIN) {
+        } else if constexpr (NT > 1) {
             if (((ok_mask >> (8 * half)) & 0xFFu) == 0u) break;
             if (half > 0) {
                 __syncthreads();  // the pass before has read the regions
@@ -1745,7 +1747,7 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
             // follow the write of the same wave in LDS order
             float v[4];
 #pragma unroll
-            for (int k = 0; k < 4; ++k) v[k] = tbuf[merge_slot[k]];
+            for (int k = 0; k < 4; ++k) v[k] = tbuf[tq4_merge_slot(lane) + 16 * k];
             const int t = div_q_group(col, P);
             const int a = col - t * P.q_group;
             const size_t row = (size_t)(tok0 + t) * P.num_q_heads + (size_t)(q_head_base + a);

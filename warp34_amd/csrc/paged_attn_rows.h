@@ -908,14 +908,9 @@ __device__ __forceinline__ void rows_tile(const AttnParams& P, uint8_t* smem, co
             mlbuf[(wave * NT * 16 + nt * 16 + n) * 2 + 1] = l_run[nt];
         }
     }
-    // element e = 128 h + 8 r + j sits in slot ((h*8 + j)*4 + (r >> 2))*4 + (r & 3)
-    int merge_slot[4];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        const int e = (4 * lane + k) & (HD - 1);  // (lanes beyond the row repeat its start and store nothing)
-        const int h = e >> 7, r = (e >> 3) & 15, j = e & 7;
-        merge_slot[k] = ((h * 8 + j) * 4 + (r >> 2)) * 4 + (r & 3);
-    }
+    // element e = 128 h + 8 r + j sits in slot ((h*8 + j)*4 + (r >> 2))*4 + (r & 3): of element 4 lane (the next ones: + 16 each)
+    const int merge_e = (4 * lane) & (HD - 1);  // (lanes beyond the row repeat its start and store nothing)
+    const int merge_slot = (((merge_e >> 7) * 8 + (merge_e & 7)) * 4 + (merge_e >> 5 & 3)) * 4 + (merge_e >> 3 & 3);
     // finishes column `col` from its sums v (element order of the head dimension) and its state
     auto finish_column = [&](int col, float (&v)[4], float m_col, float l_col) {
         const int t = div_q_group(col, P);
@@ -989,7 +984,7 @@ __device__ __forceinline__ void rows_tile(const AttnParams& P, uint8_t* smem, co
             *reinterpret_cast<f4*>(tbuf + 4 * lane) = tot;
             float v[4];  // the reads follow the write of the same wave in LDS order
 #pragma unroll
-            for (int k = 0; k < 4; ++k) v[k] = tbuf[merge_slot[k]];
+            for (int k = 0; k < 4; ++k) v[k] = tbuf[merge_slot + 16 * k];
             finish_column(nt * 16 + col, v, m_col, l_col);
         }
     }

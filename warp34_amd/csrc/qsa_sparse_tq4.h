@@ -237,9 +237,17 @@ __global__ __launch_bounds__(kQsaWaves * 64, 1) void qsa_sparse_tq4_kernel(QSA_L
     constexpr int kQStride = kQsaQStride;
     _Float16* qlds = reinterpret_cast<_Float16*>(smem + kQsaQBase);
     const float q_scale = P.sm_scale * kLog2e * kLutInvGain;
+    // up to eight columns: columns 8-15 repeat them and take the low-order part of the weights (see the dense kernel)
+    const bool pack = S.q_group <= 8;
+    static_assert(kQsaWaves == 8 && kColsPerWave == 2, "a packed tile's mirror column col + 8 belongs to the wave of col");
+    uint2 packed_prev = {0u, 0u};
 #pragma unroll
     for (int c = 0; c < kColsPerWave; ++c) {
         const int col = wave + c * kQsaWaves;
+        if (pack && c == 1) {
+            *reinterpret_cast<uint2*>(qlds + col * kQStride + 4 * lane) = packed_prev;
+            continue;
+        }
         float qv[4] = {F16::to_f32((uint16_t)(q_raw[c].x & 0xFFFFu)), F16::to_f32((uint16_t)(q_raw[c].x >> 16)),
                        F16::to_f32((uint16_t)(q_raw[c].y & 0xFFFFu)), F16::to_f32((uint16_t)(q_raw[c].y >> 16))};
         if (col < S.q_group) {  // wave-uniform; dead columns stay zero
@@ -251,6 +259,7 @@ __global__ __launch_bounds__(kQsaWaves * 64, 1) void qsa_sparse_tq4_kernel(QSA_L
         packed.x = pack_h2(qv[0] * q_scale, qv[1] * q_scale);
         packed.y = pack_h2(qv[2] * q_scale, qv[3] * q_scale);
         *reinterpret_cast<uint2*>(qlds + col * kQStride + 4 * lane) = packed;
+        packed_prev = packed;
     }
     if (unit0 < cu_end) issue_v(0);
     __syncthreads();  // the table and the query rows are complete
@@ -270,7 +279,7 @@ __global__ __launch_bounds__(kQsaWaves * 64, 1) void qsa_sparse_tq4_kernel(QSA_L
     }
 
     const uint32_t lut_lane = (uint32_t)lane << 2;
-    const bool col_ok = n < S.q_group;
+    const bool col_ok = (pack ? n & 7 : n) < S.q_group;
     f4 o_acc[2][8];
     float m_run = kNegBig, l_run = 0.f;
 #pragma unroll
@@ -413,7 +422,7 @@ __global__ __launch_bounds__(kQsaWaves * 64, 1) void qsa_sparse_tq4_kernel(QSA_L
             for (int k = 0; k < 4; ++k) {
                 uint32_t whi, wlo;
                 split_weights(w[2 * k], w[2 * k + 1], whi, wlo);
-                ph[h][k] = whi;
+                ph[h][k] = pack && (n & 8) ? wlo : whi;
                 pl[h][k] = wlo;
                 const uint32_t wa = vw[h][2 * k], wb = vw[h][2 * k + 1];
                 lo[h][k] = (wa & 0x0F0F0F0Fu) | ((wb << 4) & 0xF0F0F0F0u);
@@ -437,13 +446,15 @@ __global__ __launch_bounds__(kQsaWaves * 64, 1) void qsa_sparse_tq4_kernel(QSA_L
             if (bt + 1 < 4) pv_reads(bt + 1, va[(bt + 1) & 1]);
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int part = 0; part < 2; ++part)  // (a pass of its own: a tile's two MFMAs are not back to back)
+            for (int part = 0; part < 2; ++part) {  // (a pass of its own: a tile's two MFMAs are not back to back)
+                if (part == 1 && pack) continue;
 #pragma unroll
                 for (int jj = 0; jj < 4; ++jj) {
                     f4& o = o_acc[bt >> 1][4 * (bt & 1) + jj];
                     o = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, va[bt & 1][jj]),
                                                               __builtin_bit_cast(h8, part ? pl[bt >> 1] : ph[bt >> 1]), o, 0, 0, 0);
                 }
+            }
         }
     };
 
@@ -466,6 +477,7 @@ __global__ __launch_bounds__(kQsaWaves * 64, 1) void qsa_sparse_tq4_kernel(QSA_L
 
     // ---- merge the waves' states through LDS (layout as in the dense kernel) -------------------------
     // (one barrier: every wave leaves its state in its own staging area, the adding wave weighs them)
+    if (pack) add_mirror_columns(o_acc);
     l_run = sum_over_rows(l_run);
     constexpr int kRegion = 8 * kMergeColStride;
     static_assert(kRegion * 4 == kStageTq4, "a wave's merge region is its own staging area");
@@ -477,8 +489,12 @@ __global__ __launch_bounds__(kQsaWaves * 64, 1) void qsa_sparse_tq4_kernel(QSA_L
         mlbuf[(wave * 16 + n) * 2 + 1] = l_run;
     }
     auto store_region = [&](int half) {
-        if ((n >> 3) != half || !col_ok) return;
         float* c = xbuf + wave * kRegion + (n & 7) * kMergeColStride;
+        if (pack) {  // (half 0)
+            if (col_ok) store_packed_column(c, o_acc, n, b);
+            return;
+        }
+        if ((n >> 3) != half || !col_ok) return;
 #pragma unroll
         for (int h = 0; h < 2; ++h)
 #pragma unroll
@@ -486,22 +502,6 @@ __global__ __launch_bounds__(kQsaWaves * 64, 1) void qsa_sparse_tq4_kernel(QSA_L
     };
     store_region(0);
 
-    int merge_slot[4];  // region slot of element 4 lane + k (inverse of tq4_pv_elem)
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        const int e = 4 * lane + k;
-        int h, j, r;
-        if (e >= 128) {
-            h = 1; r = (e - 128) >> 3; j = e & 7;
-        } else if (e < 4) {
-            h = 0; r = 0; j = e;
-        } else if (e >= 124) {
-            h = 0; r = 0; j = e - 120;
-        } else {
-            h = 0; r = (e + 4) >> 3; j = (e + 4) & 7;
-        }
-        merge_slot[k] = ((h * 8 + j) * 4 + (r >> 2)) * 4 + (r & 3);
-    }
     static_assert(kQsaWaves == 8, "a wave adds up one column of a pass");
     __syncthreads();
 #pragma unroll 1
@@ -538,7 +538,7 @@ __global__ __launch_bounds__(kQsaWaves * 64, 1) void qsa_sparse_tq4_kernel(QSA_L
         *reinterpret_cast<f4*>(tbuf + 4 * lane) = tot;
         float v[4];
 #pragma unroll
-        for (int k = 0; k < 4; ++k) v[k] = tbuf[merge_slot[k]];
+        for (int k = 0; k < 4; ++k) v[k] = tbuf[tq4_merge_slot(lane) + 16 * k];
         if (S.n_splits > 1) {
             const size_t prow = row * S.n_splits + split;
             *reinterpret_cast<f4*>(P.part_acc + prow * kHeadDim + 4 * lane) = f4{v[0], v[1], v[2], v[3]};
