@@ -164,14 +164,15 @@ struct AttnParams {
 // output rounded to its 16-bit type and then passed through the gate operator's arithmetic
 // (ops/op_norms_rope_act.cu:742-759), so it has the bits of the two calls in sequence.
 // HD: the head dimension (lanes beyond a 128-element row store nothing).
-template <typename TQ, int HD = kHeadDim>
-__device__ __forceinline__ void store_out_row(const AttnParams& P, size_t row, int lane, const float (&o)[4]) {
+// gate_values: the row's, loaded here or asked for ahead (load_out_gate) by a kernel that waits for something else anyway.
+template <typename TQ, int HD, typename GateFn>
+__device__ __forceinline__ void store_out_row_by(const AttnParams& P, size_t row, int lane, const float (&o)[4], GateFn&& gate_values) {
     if (HD < 256 && 4 * lane >= HD) return;
     uint16_t h[4];
 #pragma unroll
     for (int k = 0; k < 4; ++k) h[k] = TQ::from_f32(o[k]);
     if (P.gate != nullptr) {
-        const uint2 g = *reinterpret_cast<const uint2*>(P.gate + row * HD + 4 * lane);
+        const uint2 g = gate_values();
         const uint16_t gb[4] = {(uint16_t)g.x, (uint16_t)(g.x >> 16), (uint16_t)g.y, (uint16_t)(g.y >> 16)};
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
@@ -182,6 +183,19 @@ __device__ __forceinline__ void store_out_row(const AttnParams& P, size_t row, i
     ob.x = (uint32_t)h[0] | ((uint32_t)h[1] << 16);
     ob.y = (uint32_t)h[2] | ((uint32_t)h[3] << 16);
     *reinterpret_cast<uint2*>(P.out + row * HD + 4 * lane) = ob;
+}
+template <typename TQ, int HD = kHeadDim>
+__device__ __forceinline__ void store_out_row(const AttnParams& P, size_t row, int lane, const float (&o)[4]) {
+    store_out_row_by<TQ, HD>(P, row, lane, o, [&] { return *reinterpret_cast<const uint2*>(P.gate + row * HD + 4 * lane); });
+}
+template <typename TQ, int HD = kHeadDim>
+__device__ __forceinline__ void store_out_row(const AttnParams& P, size_t row, int lane, const float (&o)[4], uint2 g) {
+    store_out_row_by<TQ, HD>(P, row, lane, o, [&] { return g; });
+}
+template <int HD = kHeadDim>
+__device__ __forceinline__ uint2 load_out_gate(const uint16_t* gate, size_t row, int lane) {
+    if (gate == nullptr || (HD < 256 && 4 * lane >= HD)) return uint2{0u, 0u};
+    return *reinterpret_cast<const uint2*>(gate + row * HD + 4 * lane);
 }
 
 
@@ -2135,7 +2149,8 @@ __device__ __forceinline__ f4 merge_slices(const f4& rec, int n_chunks, const f4
 template <typename TQ, int HD, int GROUPS>
 __global__ __launch_bounds__(GROUPS * 64) void balanced_merge_kernel(const int32_t* bal_table, const float* part_acc,
                                                                      const float* part_ml, int num_q_heads, int q_group, int kv_subs,
-                                                                     int bal_cols, const AttnParams P, float out_scale, int rotate) {
+                                                                     int bal_cols, const uint16_t* gate, const AttnParams P, float out_scale,
+                                                                     int rotate) {
     constexpr int kSlots = kMergeGroups * kMergeMaxPerGroup;  // partials of a row at most
     static_assert(GROUPS * 64 >= kSlots, "one record per thread");
     __shared__ f4 s_acc[GROUPS][64];
@@ -2148,12 +2163,17 @@ __global__ __launch_bounds__(GROUPS * 64) void balanced_merge_kernel(const int32
     // (the leading arguments repeat fields of P: preloaded, so that the table entry is asked for at once)
     const size_t row = (size_t)tok * num_q_heads + head;
     const int4 entry = *reinterpret_cast<const int4*>(bal_table + 4 * (size_t)tok);  // same address in every lane
+    uint2 g = {0u, 0u};
+    if (grp == 0) {
+        g = load_out_gate<HD>(gate, row, lane);
+        asm volatile("" ::"s"(P.out), "s"(P.gate), "s"(out_scale), "s"(rotate));  // (on their way beside the entry, not where they are used)
+    }
     const int kv_sub = small_div(head, q_group);  // = kv_head * q_subgroups + subgroup
     const int n_chunks = __builtin_amdgcn_readfirstlane(entry.y);
     if (n_chunks < 0 || n_chunks == 1) return;  // masked, or finished by the attention kernel
     if (n_chunks == 0) {                        // no visible key: zeros
         const float zero[4] = {0.f, 0.f, 0.f, 0.f};
-        if (grp == 0) store_out_row<TQ, HD>(P, row, lane, zero);
+        if (grp == 0) store_out_row<TQ, HD>(P, row, lane, zero, g);
         return;
     }
     const int col = entry.z * q_group + (head - kv_sub * q_group);
@@ -2180,7 +2200,7 @@ __global__ __launch_bounds__(GROUPS * 64) void balanced_merge_kernel(const int32
 #pragma unroll
             for (int k = 0; k < 4; ++k) o[k] = apply_sign(o[k], 4 * lane + k);
         }
-        store_out_row<TQ, HD>(P, row, lane, o);
+        store_out_row<TQ, HD>(P, row, lane, o, g);
         return;
     }
     if (tid < n_chunks && tid < kSlots) s_rec[tid] = *reinterpret_cast<const f4*>(part_ml + (prow0 + tid * pstride) * 4);
@@ -2244,8 +2264,32 @@ __global__ __launch_bounds__(GROUPS * 64) void balanced_merge_kernel(const int32
 #pragma unroll
         for (int k = 0; k < 4; ++k) o[k] = apply_sign(o[k], 4 * lane + k);
     }
-    store_out_row<TQ, HD>(P, row, lane, o);
+    store_out_row<TQ, HD>(P, row, lane, o, g);
 }
+
+// Does a row's token belong to a request, and is it to be computed?  Lane r looks at request r; the first 64 requests' tokens are asked for by the
+// constructor, together with what else the kernel needs: asked for one behind the other, and the gate behind the sums, they were three more round trips of
+// a kernel that consists of one (us, eight layers of one token on 1 200 keys 113.5 / 109.7, four of one on 32 768 bf16 keys 78.5 / 77.5).  (First match wins.)
+struct RowOwner {
+    int lo, hi;
+    __device__ __forceinline__ RowOwner(const int32_t* query_start_loc, int num_reqs, int lane) {
+        const int r = min(lane, num_reqs - 1);
+        lo = query_start_loc[r];
+        hi = query_start_loc[r + 1];
+    }
+    __device__ __forceinline__ bool live(const warp34_attention_batch& B, int tok, int lane) const {
+        if (B.valid_token_mask != nullptr && B.valid_token_mask[tok] == 0) return false;
+        for (int base = 0; base < B.num_reqs; base += 64) {
+            const int r = base + lane;
+            const bool inb = r < B.num_reqs;
+            const int first = base == 0 ? lo : inb ? B.query_start_loc[r] : 0;
+            const int end = base == 0 ? hi : inb ? B.query_start_loc[r + 1] : 0;
+            const unsigned long long hits = __ballot(inb && tok >= first && tok < end);
+            if (hits != 0ull) return B.valid_req_mask == nullptr || B.valid_req_mask[base + __builtin_ctzll(hits)] != 0;
+        }
+        return false;
+    }
+};
 
 // Merge of the split-K partials (op_paged_attn.cu:1132-1218): m_tot = max m_s,
 // w_s = 2^(m_s - m_tot), out = sum acc_s w_s / sum l_s w_s, then one inverse rotation.
@@ -2256,8 +2300,9 @@ __global__ __launch_bounds__(GROUPS * 64) void balanced_merge_kernel(const int32
 // loaded speculatively and the slots beyond the row's chunk count are discarded with selects.
 template <typename TQ, bool SP, int HD, int GROUPS>
 __global__ __launch_bounds__(GROUPS * 64) void split_merge_kernel(const float* part_acc_in, const float* part_ml_in,
-                                                                  int max_chunks_in, int num_q_heads_in, const AttnParams P,
-                                                                  float out_scale, int rotate) {
+                                                                  int max_chunks_in, int num_q_heads_in, const int32_t* query_start_loc,
+                                                                  const uint16_t* gate, int num_reqs, const AttnParams P, float out_scale,
+                                                                  int rotate) {
     constexpr int kSlots = kMergeGroups * kMergeMaxPerGroup;
     static_assert(GROUPS * 64 >= kSlots, "one record per thread");
     __shared__ f4 s_acc[GROUPS][64];
@@ -2269,8 +2314,7 @@ __global__ __launch_bounds__(GROUPS * 64) void split_merge_kernel(const float* p
     const int grp = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int tok = (int)blockIdx.y;
     const warp34_attention_batch& B = P.B;
-    // the leading arguments repeat P.part_acc / P.part_ml / P.max_chunks / P.num_q_heads: they are
-    // preloaded into scalar registers at wave launch, so the speculative loads below do not wait for
+    // the leading arguments repeat fields of P: they are preloaded into scalar registers at wave launch, so the loads below do not wait for
     // the kernel-argument fetch
     const size_t row = (size_t)tok * num_q_heads_in + blockIdx.x;
     const float* ml = part_ml_in + row * max_chunks_in * 4;
@@ -2291,23 +2335,13 @@ __global__ __launch_bounds__(GROUPS * 64) void split_merge_kernel(const float* p
         }
     };
     load_slices(0);
-    // row validity (wave 0): token mask and owning request, first match wins
+    uint2 g = {0u, 0u};
     if (grp == 0) {
-        bool ok = B.valid_token_mask == nullptr || B.valid_token_mask[tok] != 0;
-        bool found = false;
-        for (int base = 0; base < B.num_reqs && !found; base += 64) {
-            const int r = base + lane;
-            const bool inb = r < B.num_reqs;
-            const int lo = inb ? B.query_start_loc[r] : 0x7fffffff;
-            const int hi = inb ? B.query_start_loc[r + 1] : -0x7fffffff;
-            const int rm = (inb && B.valid_req_mask != nullptr) ? (int)B.valid_req_mask[r] : 1;
-            const unsigned long long hits = __ballot(inb && tok >= lo && tok < hi);
-            if (hits != 0ull) {
-                found = true;
-                ok = ok && __builtin_amdgcn_readlane(rm, __builtin_ctzll(hits)) != 0;
-            }
-        }
-        if (lane == 0) s_valid = (ok && found) ? 1 : 0;
+        const RowOwner owner(query_start_loc, num_reqs, lane);
+        g = load_out_gate<HD>(gate, row, lane);
+        asm volatile("" ::"s"(P.out), "s"(P.gate), "s"(out_scale), "s"(rotate));  // (on their way beside the slices, not where they are used)
+        const bool live = owner.live(B, tok, lane);
+        if (lane == 0) s_valid = live ? 1 : 0;
     }
     if (tid < kSlots) s_rec[tid] = rec;
     __syncthreads();
@@ -2372,14 +2406,15 @@ __global__ __launch_bounds__(GROUPS * 64) void split_merge_kernel(const float* p
 #pragma unroll
         for (int k = 0; k < 4; ++k) o[k] = apply_sign(o[k], 4 * lane + k);
     }
-    store_out_row<TQ, HD>(P, row, lane, o);
+    store_out_row<TQ, HD>(P, row, lane, o, g);
 }
 
 // The same for rows of at most SLOTS chunks: one wave per row, which holds all of its records' slices; the records reach the other lanes
 // through scalar registers, no LDS and no barrier.
 template <typename TQ, int HD, int SLOTS, int ORDER>
 __global__ __launch_bounds__(64) void split_merge_few_kernel(const float* part_acc_in, const float* part_ml_in, int max_chunks_in,
-                                                             int num_q_heads_in, const AttnParams P, float out_scale, int rotate) {
+                                                             int num_q_heads_in, const int32_t* query_start_loc, const uint16_t* gate,
+                                                             int num_reqs, const AttnParams P, float out_scale, int rotate) {
     static_assert(SLOTS <= 64, "one record per lane");
     const int lane = (int)threadIdx.x;
     const int tok = (int)blockIdx.y;
@@ -2395,21 +2430,10 @@ __global__ __launch_bounds__(64) void split_merge_few_kernel(const float* part_a
         a[s] = f4{0.f, 0.f, 0.f, 0.f};
         if (s < max_chunks_in && (HD == 256 || 4 * lane < HD)) a[s] = *reinterpret_cast<const f4*>(acc + (size_t)s * kHeadDim + 4 * lane);
     }
-    bool ok = B.valid_token_mask == nullptr || B.valid_token_mask[tok] != 0;
-    bool found = false;
-    for (int base = 0; base < B.num_reqs && !found; base += 64) {
-        const int r = base + lane;
-        const bool inb = r < B.num_reqs;
-        const int lo = inb ? B.query_start_loc[r] : 0x7fffffff;
-        const int hi = inb ? B.query_start_loc[r + 1] : -0x7fffffff;
-        const int rm = (inb && B.valid_req_mask != nullptr) ? (int)B.valid_req_mask[r] : 1;
-        const unsigned long long hits = __ballot(inb && tok >= lo && tok < hi);
-        if (hits != 0ull) {
-            found = true;
-            ok = ok && __builtin_amdgcn_readlane(rm, __builtin_ctzll(hits)) != 0;
-        }
-    }
-    if (!ok || !found) return;  // masked row: output untouched
+    const RowOwner owner(query_start_loc, num_reqs, lane);
+    const uint2 g = load_out_gate<HD>(gate, row, lane);
+    asm volatile("" ::"s"(P.out), "s"(P.gate), "s"(out_scale), "s"(rotate));  // (on their way beside the slices, not where they are used)
+    if (!owner.live(B, tok, lane)) return;  // masked row: output untouched
     const int n_chunks = min((int)__int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(rec[2]))), max_chunks_in);
     float l_tot;
     const f4 tot = merge_slices<SLOTS, ORDER>(rec, n_chunks, a, lane, l_tot);
@@ -2420,7 +2444,7 @@ __global__ __launch_bounds__(64) void split_merge_few_kernel(const float* part_a
 #pragma unroll
         for (int k = 0; k < 4; ++k) o[k] = apply_sign(o[k], 4 * lane + k);
     }
-    store_out_row<TQ, HD>(P, row, lane, o);
+    store_out_row<TQ, HD>(P, row, lane, o, g);
 }
 
 }  // namespace w34
@@ -2595,7 +2619,7 @@ static int launch_balanced_merge(const AttnParams& P, int kv_subs, float out_sca
     const int groups = merge_small_groups(P) ? 4 : kMergeGroups;
     const auto kernel = groups == 4 ? balanced_merge_kernel<TQ, HD, 4> : balanced_merge_kernel<TQ, HD, kMergeGroups>;
     hipLaunchKernelGGL(kernel, grid, dim3((unsigned)groups * 64), 0, stream, (const int32_t*)P.bal_table, (const float*)P.part_acc,
-                       (const float*)P.part_ml, P.num_q_heads, P.q_group, kv_subs, P.bal_cols, P, out_scale, P.rot_out);
+                       (const float*)P.part_ml, P.num_q_heads, P.q_group, kv_subs, P.bal_cols, P.gate, P, out_scale, P.rot_out);
     return (int)hipGetLastError();
 }
 
@@ -2604,8 +2628,8 @@ static int launch_split_merge(const AttnParams& P, int slots, float out_scale, h
     const dim3 grid((unsigned)P.num_q_heads, (unsigned)P.B.total_tokens);
     if constexpr (!SP) {
         const auto few = [&](auto kernel) {
-            hipLaunchKernelGGL(kernel, grid, dim3(64), 0, stream, (const float*)P.part_acc, (const float*)P.part_ml, slots, P.num_q_heads, P,
-                               out_scale, P.rot_out);
+            hipLaunchKernelGGL(kernel, grid, dim3(64), 0, stream, (const float*)P.part_acc, (const float*)P.part_ml, slots, P.num_q_heads,
+                               P.B.query_start_loc, P.gate, P.B.num_reqs, P, out_scale, P.rot_out);
             return (int)hipGetLastError();
         };
         if (slots <= (merge_small_groups(P) ? kMergeFewRows : kMergeFew)) {
@@ -2619,10 +2643,11 @@ static int launch_split_merge(const AttnParams& P, int slots, float out_scale, h
     }
     if (merge_small_groups(P)) {
         hipLaunchKernelGGL((split_merge_kernel<TQ, SP, HD, 4>), grid, dim3(4 * 64), 0, stream, (const float*)P.part_acc,
-                           (const float*)P.part_ml, slots, P.num_q_heads, P, out_scale, P.rot_out);
+                           (const float*)P.part_ml, slots, P.num_q_heads, P.B.query_start_loc, P.gate, P.B.num_reqs, P, out_scale, P.rot_out);
     } else {
         hipLaunchKernelGGL((split_merge_kernel<TQ, SP, HD, kMergeGroups>), grid, dim3(kMergeGroups * 64), 0, stream,
-                           (const float*)P.part_acc, (const float*)P.part_ml, slots, P.num_q_heads, P, out_scale, P.rot_out);
+                           (const float*)P.part_acc, (const float*)P.part_ml, slots, P.num_q_heads, P.B.query_start_loc, P.gate, P.B.num_reqs, P,
+                           out_scale, P.rot_out);
     }
     return (int)hipGetLastError();
 }
