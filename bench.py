@@ -66,17 +66,17 @@ WORKLOADS = {
 # be read from inside this process, so workloads without such a profile report null.
 PROFILED_TRAFFIC = {
     # workload: (HBM bytes per launch of the dominant kernel, the profile that holds the counter readings)
-    "tq4_decode_b1_ctx131072": (71_830_000, "profiles/paged_attn_tq4_decode_b1_ctx131072.txt"),
-    "tq4_decode_b8_ctx131072": (556_780_000, "profiles/paged_attn_tq4_decode_b8_ctx131072.txt"),
-    "tq4_decode_b32_ctx1k_64k": (584_030_000, "profiles/paged_attn_tq4_decode_b32_ctx1k_64k.txt"),
+    "tq4_decode_b1_ctx131072": (71_710_000, "profiles/paged_attn_tq4_decode_b1_ctx131072.txt"),
+    "tq4_decode_b8_ctx131072": (556_730_000, "profiles/paged_attn_tq4_decode_b8_ctx131072.txt"),
+    "tq4_decode_b32_ctx1k_64k": (583_940_000, "profiles/paged_attn_tq4_decode_b32_ctx1k_64k.txt"),
     "bf16_decode_b1_ctx32768": (69_530_000, "profiles/paged_attn_rows_bf16_decode_b1_ctx32768.txt"),
     "fp8_decode_b32_ctx1k_64k": (1_162_710_000, "profiles/paged_attn_rows_fp8_decode_b32_ctx1k_64k.txt"),
-    "fp8_decode_b1_ctx131072": (140_900_000, "profiles/paged_attn_rows_fp8_decode_b1_ctx131072.txt"),
-    "q8_0_decode_b1_ctx131072": (145_110_000, "profiles/paged_attn_rows_q8_0_decode_b1_ctx131072.txt"),
-    # (the four kernels of the shared-prefix path together: probe 0.27 + tile 144.89 + decode 535.52 + merge 39.06 MB)
-    "tq4_verify_16x4_ctx262144_shared200k": (719_740_000, "profiles/paged_attn_tq4_verify_16x4_ctx262144_shared200k.txt"),
+    "fp8_decode_b1_ctx131072": (140_820_000, "profiles/paged_attn_rows_fp8_decode_b1_ctx131072.txt"),
+    "q8_0_decode_b1_ctx131072": (145_020_000, "profiles/paged_attn_rows_q8_0_decode_b1_ctx131072.txt"),
+    # (the four kernels of the shared-prefix path together: probe 0.27 + tile 144.78 + private rest 547.70 + merge 39.04 MB)
+    "tq4_verify_16x4_ctx262144_shared200k": (731_790_000, "profiles/paged_attn_tq4_verify_16x4_ctx262144_shared200k.txt"),
     "tq4_prefill_8x2048_ctx16384": (567_780_000, "profiles/paged_prefill_tq4_8x2048_ctx16384.txt"),
-    "tq4_qsa_sparse_16x513_ctx131072": (23_340_000, "profiles/qsa_sparse_tq4_16x513_ctx131072.txt"),
+    "tq4_qsa_sparse_16x513_ctx131072": (23_330_000, "profiles/qsa_sparse_tq4_16x513_ctx131072.txt"),
     "tq4_norm_rope_append_8192": (182_920_000, "profiles/qk_norm_rope_tq4_append_8192.txt"),
     "tq4_fused_qk_gate_append_8192": (289_740_000, "profiles/fused_qk_norm_rope_gate_tq4_append_8192.txt"),
     "tq4_append_4096": (10_800_000, "profiles/kv_append_tq4_4096.txt"),
@@ -916,10 +916,11 @@ def run_workload(args, torch, lib, ffi, dev):
             "traffic_source": None if args.ctx else PROFILED_TRAFFIC.get(args.workload, (None, None))[1],
             "traffic_measured_in_this_run": False,
             "kernel": ("shared_prefix_probe_kernel + paged_prefill_tq4_kernel (shared pages, 32 parts) + "
-                       "paged_attn_tq4_kernel (private rest) + split_merge_kernel, all inside the timed launch")
+                       "paged_attn_tq4_private_kernel (private rest) + split_merge_kernel, all inside the timed launch")
                       if args.workload in SHARED_PREFIX else
                       "paged_attn_%s_kernel (+ merge kernel, both inside the timed launch)"
-                      % (("tq4" if fmt == "tq4" else "rows") + ("_balanced" if R > 1 and ql == 1 else "")),
+                      % (("tq4" if fmt == "tq4" else "rows") + ("_balanced" if R > 1 and ql == 1 else
+                                                                "_plain" if fmt in ("tq4", "fp8", "q8_0") else "")),
             "avg_launch_us": round(ms_per_step * 1e3, 3),
             "host_wall_us_per_step": round(t_wall / args.steps * 1e6, 2),
         },
