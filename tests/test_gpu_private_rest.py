@@ -5,7 +5,8 @@ import numpy as np
 import pytest
 
 import oracle
-from oracle import DT_BF16
+from cases import make_case
+from oracle import DT_BF16, FMT_TQ4
 
 pytestmark = pytest.mark.gpu
 
@@ -42,3 +43,42 @@ def test_private_rest_matches_oracle(name):
     assert rc == 0
     # another order of the same sums, unless nothing is shared
     assert (got.tobytes() == plain.tobytes()) == (shared == 0)
+
+
+def _small(block, q_lens, ctx, shared, seed, q_heads=16):
+    """A batch whose requests have their first `shared` keys in common, on a pool of the host."""
+    pool, bt, k, v, q, aq, before = make_case(FMT_TQ4, block, ctx, q_lens, seed, DT_BF16, q_heads=q_heads)
+    bt[1:, :shared // block] = bt[0, :shared // block]
+    hb = oracle.HostBatch(aq, ctx, bt, context_lens_before=before)
+    v_absmax = np.abs(oracle.bits_to_f32(v, DT_BF16)).max(axis=0)
+    return pool, hb, q, np.repeat(np.maximum(1.0, v_absmax), q_heads // 2, axis=0)[None]
+
+
+LONG = 40000  # a bound from which on the shared keys get a pass of their own
+
+
+@pytest.mark.parametrize("bits", [0x7C00, 0xFFFF])     # an infinite and a NaN scale
+@pytest.mark.parametrize("both_slabs", [False, True])  # the value rows, which leave the scores as they are, or the key rows too
+@pytest.mark.parametrize("token", [3, 2])              # both in the second column tile of a request, the first one has tokens 0 and 1
+def test_scales_of_unseen_rows(token, both_slabs, bits):
+    """The scales of a token's rows are not finite: the tokens in front of it, which do not see them, keep their bits."""
+    import gpu_harness as G
+
+    pool, hb, q, _ = _small(64, (4, 4, 4, 4), (4133, 4196, 4165, 4612), 4096, 1401)
+    outs = []
+    for poisoned in (False, True):
+        if poisoned:
+            for slab in (pool.k, pool.v) if both_slabs else (pool.v,):
+                rows = slab.reshape(-1, pool.kv_heads, pool.block_size, pool.tok).view(np.uint16)
+                assert np.shares_memory(rows, slab)
+                for r, pos in enumerate(hb.ctx + token):
+                    rows[hb.bt[r, pos // 64], :, pos % 64][:, [0, 33]] = bits
+        dpool = G.DevPool(pool)
+        dpool.upload()
+        rc, got, _ = G.dev_attention(dpool, hb, q, DT_BF16, 16, scratch_bytes=96 << 20, max_seq_len=LONG)
+        assert rc == 0
+        got = got.reshape(4, 4, 16, 256)
+        assert both_slabs or np.isnan(oracle.bits_to_f32(got[:, token:], DT_BF16)).all() == poisoned
+        outs.append(got[:, :token])
+    assert np.isfinite(oracle.bits_to_f32(outs[0], DT_BF16)).all()
+    assert np.array_equal(outs[0], outs[1])

@@ -1500,9 +1500,35 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
         if constexpr (NT > 1) {
             float(&p2)[8] = sc2;
             if (MASKED) {
-                // (a token masked for one column tile only keeps its scales, which are those of a real row)
+                // A token masked for one column tile only keeps its scales.  Where one is not finite, its product with that tile's weight of 0 would be
+                // NaN: what the columns that see the token get of it, NaN in all channels of the half row, goes to their sums here, and
+                // the scale counts as 0.  (A choice per tile in weights() instead, which few units need: whole call 508 / 513 us.)
+                uint32_t bad = 0;
 #pragma unroll
-                for (int t = 0; t < 8; ++t) vsc[t] = p[t] > 0.f || p2[t] > 0.f ? vsc[t] : 0u;
+                for (int t = 0; t < 8; ++t) {
+                    vsc[t] = p[t] > 0.f || p2[t] > 0.f ? vsc[t] : 0u;
+                    bad = max_u16x2(bad, vsc[t] & 0x7FFF7FFFu);
+                }
+                if (__ballot((bad & 0xFFFFu) >= 0x7C00u || (bad >> 16) >= 0x7C00u) != 0ull) {
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {
+                        const uint32_t exponent = 0x7C00u << (16 * h);
+                        float sees = 0.f, sees2 = 0.f;
+#pragma unroll
+                        for (int t = 0; t < 8; ++t) {
+                            const bool finite = (vsc[t] & exponent) != exponent;
+                            sees += finite ? 0.f : p[t];
+                            sees2 += finite ? 0.f : p2[t];
+                            vsc[t] &= finite ? 0xFFFFFFFFu : 0xFFFFu << (16 * (1 - h));
+                        }
+                        const float add = sum_over_rows(sees) == 0.f ? 0.f : __builtin_nanf(""), add2 = sum_over_rows(sees2) == 0.f ? 0.f : __builtin_nanf("");
+#pragma unroll
+                        for (int j = 0; j < 8; ++j) {
+                            o_acc[h][j] += add;
+                            o_acc2[h][j] += add2;
+                        }
+                    }
+                }
             }
             // Eight batches of two value tiles: eight table reads a batch ahead, eight MFMAs (high and low weights of two column tiles).
             // The weights and code words of a half row are made in front of its batches.
