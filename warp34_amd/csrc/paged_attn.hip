@@ -1275,8 +1275,9 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
         for (int mf = 0; mf < 8; ++mf) bq[mf] = *reinterpret_cast<const h8*>(my_qop + 16 * mf);
     }
 
-    // Until every column has a maximum (`started`) the running maximum of a column without visible keys is 0 and its sum 0.
-    bool started = false;
+    // Until every live column of the tile has a maximum (`started`) that of a column without one is 0, and so is its sum.  (A unit that it sees need
+    // not give it one: with infinite key scales its scores may all be minus infinity.)
+    bool started = false, started2 = false;
     f4 o_acc[2][8];
     float m_run = 0.f, l_run = 0.f;
 #pragma unroll
@@ -1466,18 +1467,19 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
         // and leave the sums alone, and a probability of up to 2^8 keeps its 22 bits.  us, this, eight instead of nine operands (tq4_fuse) and split_weights, before /
         // now: one token on 131 072 keys 26.5 / 25.9 a layer, eight layers of one on 1 200 126.3 / 124.2, 32 requests of 1 000 to 64 000 125.4 / 124.2.  Exact where that could leave fp16's range, and where the
         // column does not see the whole unit (what lies behind the sequence must not matter).
-        auto softmax = [&](float (&x)[8], float& m, float& l, f4 (&o)[2][8], int last) __attribute__((always_inline)) {
+        auto softmax = [&](float (&x)[8], float& m, float& l, f4 (&o)[2][8], int last, bool ok, bool& have) __attribute__((always_inline)) {
             const float mx = fmaxf(max3(x[0], x[1], x[2]), max3(x[3], x[4], max3(x[5], x[6], x[7])));
-            if (!started || __ballot(mx > 0.f) != 0ull) {
+            if (!have || __ballot(mx > 0.f) != 0ull) {
                 uint32_t d = 0;  // the largest scales
 #pragma unroll
                 for (int t = 0; t < 8; ++t) d = max_u16x2(d, vsc[t] & 0x7FFF7FFFu);
                 const bool large = __ballot((d & 0xFFFFu) > kSlackScaleBits || (d >> 16) > kSlackScaleBits) != 0ull;
                 const float slack = large || (MASKED && !(t0 >= col_lo && t0 + kUnit - 1 <= last)) ? 0.f : kPfSlack;
-                if (!started || __ballot(mx > slack) != 0ull) {
+                if (!have || __ballot(mx > slack) != 0ull) {
                     const float top = max_over_rows(mx);
-                    const bool empty = !(sum_over_rows(l) > 0.f);
-                    const float up = empty ? (top > 0.5f * kNegBig ? top : 0.f) : top > slack ? top : 0.f;
+                    const bool empty = !(sum_over_rows(l) > 0.f), any = top > 0.5f * kNegBig;
+                    have = __ballot(ok && empty && !any) == 0ull;
+                    const float up = empty ? (any ? top : 0.f) : top > slack ? top : 0.f;
                     const float alpha = empty ? 1.f : __builtin_amdgcn_exp2f(-up);
                     m += up;
                     l *= alpha;
@@ -1493,9 +1495,8 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
             for (int t = 0; t < 8; ++t) x[t] = __builtin_amdgcn_exp2f(x[t]);
             l += ((x[0] + x[1]) + (x[2] + x[3])) + ((x[4] + x[5]) + (x[6] + x[7]));
         };
-        softmax(sc, m_run, l_run, o_acc, col_hi);
-        if constexpr (NT > 1) softmax(sc2, m_run2, l_run2, o_acc2, col_hi2);
-        started = started || !MASKED;
+        softmax(sc, m_run, l_run, o_acc, col_hi, col_ok, started);
+        if constexpr (NT > 1) softmax(sc2, m_run2, l_run2, o_acc2, col_hi2, col_ok2, started2);
         float(&p)[8] = sc;
         if constexpr (NT > 1) {
             float(&p2)[8] = sc2;
