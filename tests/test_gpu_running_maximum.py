@@ -1,5 +1,5 @@
-"""The running maximum of the TQ4 decode and verify kernels, on rows that are made for it: every key is one row with a scale of its own, every
-query is that row, so a key's score is what its scale says; single pass, where a wave works on units 8, 16, ... units behind its first one."""
+"""The running maximum of the TQ4 kernels, on rows that are made for it: every key is one row with a scale of its own, every query is that
+row, so a key's score is what its scale says.  A wave of a decode kernel works on units 8, 16, ... units behind its first one."""
 import numpy as np
 import pytest
 
@@ -78,3 +78,22 @@ def test_units_without_weight_before_low_scores(form):
             want = oracle.paged_attention(pool, hb, q, DT_F16, HEADS, n_threads=oracle.hw_threads())
     for got in outs:
         G.assert_close(got, DT_F16, want, what=form)
+
+
+@pytest.mark.parametrize("force", [1, 2])  # tiles of 128 rows and of 256
+def test_prefill_units_without_weight_before_low_scores(force):
+    """The same for the tile kernels, whose waves work on all units of the request: the first two have scores of minus infinity."""
+    import gpu_harness as G
+
+    outs = []
+    for none in (-2000.0, -np.inf):
+        pool, hb, q = _pool(64, (400,), (200,), lambda pos: np.where(pos < 64, none, -300.0 - 0.1 * (pos % 7)))
+        dpool = G.DevPool(pool)
+        dpool.upload()
+        rc, got, _ = G.dev_attention(dpool, hb, q, DT_F16, HEADS, force_kernel=force)
+        assert rc == 0
+        outs.append(got)
+        if none > -np.inf:
+            want = oracle.paged_attention(pool, hb, q, DT_F16, HEADS, n_threads=oracle.hw_threads())
+    for got in outs:
+        G.assert_close(got, DT_F16, want, what="tiles %d" % force)

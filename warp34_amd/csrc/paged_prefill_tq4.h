@@ -377,7 +377,7 @@ __global__ __launch_bounds__(12 * 64, 1) void paged_prefill_tq4_kernel(const Att
     }
     // ---- per-wave attention state ----
     f4 o_acc[2][8];
-    // Until every column has a maximum (`started`) the running maximum of a column without visible keys is 0 and its sum 0.
+    // Until every live column has a maximum (`started`) that of a column without one is 0, and so is its sum (see the decode kernel).
     bool started = false;
     float m_run = 0.f, l_run = 0.f;
 #pragma unroll
@@ -503,8 +503,9 @@ __global__ __launch_bounds__(12 * 64, 1) void paged_prefill_tq4_kernel(const Att
         const bool raise = !started || __ballot(mx > slack) != 0ull;
         if (raise) {
             const float m = max_over_rows(mx);
-            const bool empty = !(sum_over_rows(l_run) > 0.f);
-            const float up = empty ? (m > 0.5f * kNegBig ? m : 0.f) : m > slack ? m : 0.f;
+            const bool empty = !(sum_over_rows(l_run) > 0.f), any = m > 0.5f * kNegBig;
+            if (!started) started = __ballot(col_ok && empty && !any) == 0ull;
+            const float up = empty ? (any ? m : 0.f) : m > slack ? m : 0.f;
             const float alpha = empty ? 1.f : __builtin_amdgcn_exp2f(-up);
             m_run += up;
             l_run *= alpha;
@@ -514,7 +515,6 @@ __global__ __launch_bounds__(12 * 64, 1) void paged_prefill_tq4_kernel(const Att
             for (int h = 0; h < 2; ++h)
 #pragma unroll
                 for (int j = 0; j < 8; ++j) o_acc[h][j] *= alpha;
-            started = started || !MASKED;
         }
         float p[8];
 #pragma unroll

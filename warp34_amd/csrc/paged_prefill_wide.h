@@ -514,7 +514,7 @@ __device__ __forceinline__ void pw_tile(const AttnParams& P, uint8_t* smem, int 
     auto read_v = [&](int at) __attribute__((always_inline)) {  // step at: channels 16 at ..
         vring[at % VRING] = pw_read_h8(v_at + at * 1024);
     };
-    // Until every column has a maximum (`started`) the running maximum of a column without visible keys is 0 and its sum 0.
+    // Until every live column has a maximum (`started`) that of a column without one is 0, and so is its sum (see the decode kernel).
     bool started = false;
     auto compute_unit = [&](int u, const bool masked, auto&& after_keys) __attribute__((always_inline)) {
         const int deqbuf = u & 1, t0 = (u_first + u) * kUnit;
@@ -598,9 +598,11 @@ __device__ __forceinline__ void pw_tile(const AttnParams& P, uint8_t* smem, int 
         }
         if (!started || (kLazy ? __ballot(mx[0] > slack[0] || mx[NC - 1] > slack[NC - 1])
                                : __ballot(max2(mx[0], mx[NC - 1]) > 0.f)) != 0ull) {
+            float least = -kNegBig;
 #pragma unroll
             for (int g = 0; g < NC; ++g) {
                 const float m = max_over_rows(mx[g]);
+                least = fminf(least, m);
                 const bool empty = !(sum_over_rows(l_run[g]) > 0.f);
                 const float up = empty ? (m > 0.5f * kNegBig ? m : 0.f) : !kLazy ? fmaxf(m, 0.f) : m > slack[g] ? m : 0.f;
                 const float alpha = empty ? 1.f : __builtin_amdgcn_exp2f(-up);
@@ -612,7 +614,7 @@ __device__ __forceinline__ void pw_tile(const AttnParams& P, uint8_t* smem, int 
 #pragma unroll
                     for (int j = 0; j < 8; ++j) o_acc[g][h][j] *= alpha;
             }
-            started = started || !masked;
+            started = started || (!masked && __ballot(!(least > 0.5f * kNegBig)) == 0ull);  // (a unit that every live column sees)
         }
 #pragma unroll
         for (int g = 0; g < NC; ++g) {
