@@ -82,3 +82,20 @@ def test_scales_of_unseen_rows(token, both_slabs, bits):
         outs.append(got[:, :token])
     assert np.isfinite(oracle.bits_to_f32(outs[0], DT_BF16)).all()
     assert np.array_equal(outs[0], outs[1])
+
+
+@pytest.mark.parametrize("q_lens,bounds", [((2,) * 8, (2, 3, 4, 16)), ((3, 1, 2, 2, 1, 3, 2, 2), (3, 4, 8)), ((4, 2, 4, 4, 4), (4, 5, 16))])
+def test_bytes_do_not_depend_on_the_token_bound(q_lens, bounds):
+    import gpu_harness as G
+
+    pool, hb, q, scale = _small(64, q_lens, [4200 + 97 * r for r in range(len(q_lens))], 4096, 1501)
+    dpool = G.DevPool(pool)
+    dpool.upload()
+    outs = []
+    for bound in bounds:
+        rc, got, _ = G.dev_attention(dpool, hb, q, DT_BF16, 16, scratch_bytes=96 << 20, max_seq_len=LONG, max_q_len=bound)
+        assert rc == 0
+        outs.append(got)
+    want = oracle.paged_attention(pool, hb, q, DT_BF16, 16, n_threads=oracle.hw_threads())
+    G.assert_close(outs[0], DT_BF16, want, what="bound %d" % bounds[0], scale=scale)
+    assert all(np.array_equal(got, outs[0]) for got in outs)

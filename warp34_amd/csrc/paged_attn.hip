@@ -2911,7 +2911,9 @@ static int launch_tq4(const warp34_exec* ex, const warp34_kv_layer_layout* layou
                                stream, T);
             rc = (int)hipGetLastError();
             if (rc) return rc;
-            if (batch->max_q_len * q_group > 16 && 32 % q_group == 0) {
+            // More than a column tile per request: by the number of tokens, not by the bound on a request's, on which no result may depend.  (q_group
+            // is a power of two, see shared_prefix_applicable: a tile holds whole tokens.)
+            if ((long long)batch->total_tokens * q_group > 16ll * batch->num_reqs) {
                 AttnParams W = P;
                 W.tok_tile = 32 / q_group;
                 W.tiles_by_request = batch->max_q_len <= W.tok_tile ? 1 : 0;
