@@ -99,3 +99,18 @@ def test_bytes_do_not_depend_on_the_token_bound(q_lens, bounds):
     want = oracle.paged_attention(pool, hb, q, DT_BF16, 16, n_threads=oracle.hw_threads())
     G.assert_close(outs[0], DT_BF16, want, what="bound %d" % bounds[0], scale=scale)
     assert all(np.array_equal(got, outs[0]) for got in outs)
+
+
+# pages of 16 keys (two per unit) and of 48 (units across their edges), the last of a request with one key and more; the shared keys end inside a page of 48
+@pytest.mark.parametrize("block,shared,ctx", [(16, 4096, (4113, 4129, 4100, 4611)), (48, 4176, (4225, 4181, 4300, 4801))])
+@pytest.mark.parametrize("q_lens", [(4, 4, 4, 4), (4, 0, 5, 7)])
+def test_other_page_sizes(block, shared, ctx, q_lens):
+    import gpu_harness as G
+
+    pool, hb, q, scale = _small(block, q_lens, ctx, shared, 1601)
+    dpool = G.DevPool(pool)
+    dpool.upload()
+    rc, got, _ = G.dev_attention(dpool, hb, q, DT_BF16, 16, scratch_bytes=96 << 20, max_seq_len=LONG)
+    assert rc == 0
+    want = oracle.paged_attention(pool, hb, q, DT_BF16, 16, n_threads=oracle.hw_threads())
+    G.assert_close(got, DT_BF16, want, what="pages of %d" % block, scale=scale)

@@ -97,3 +97,22 @@ def test_prefill_units_without_weight_before_low_scores(force):
             want = oracle.paged_attention(pool, hb, q, DT_F16, HEADS, n_threads=oracle.hw_threads())
     for got in outs:
         G.assert_close(got, DT_F16, want, what="tiles %d" % force)
+
+
+@pytest.mark.parametrize("form", sorted(FORMS))
+@pytest.mark.parametrize("lengths_before", [True, False])
+def test_value_scales_that_leave_no_room_above_one(form, lengths_before):
+    """Value scales of 3 000 in every third token and scores that rise by 6 from one unit of a wave to its next: with a maximum that stays where it
+    is, as it does for ordinary scales up to a rise of 8, a weight would be 64 x 3 000, which is no fp16 number."""
+    q_lens, seqs, shared, _, _ = FORMS[form]
+    pool, hb, q = _pool(64, seqs, q_lens, lambda pos: 6.0 * (pos // 256 + 1), shared)
+    rows = pool.v.reshape(-1, 64, pool.tok).view(np.uint16)
+    assert np.shares_memory(rows, pool.v)
+    rows[:, ::3, [0, 33]] = np.float16(3000.0).view(np.uint16)
+    want = oracle.paged_attention(pool, hb, q, DT_F16, HEADS, n_threads=oracle.hw_threads())
+    if not lengths_before:  # decode: the kernel that does not work ahead of them; a verify batch has no pass for shared keys
+        hb = oracle.HostBatch(hb.qsl, hb.seq, hb.bt)
+    out = oracle.bits_to_f32(_attend(pool, hb, q, form), DT_F16).astype(np.float64)
+    assert np.isfinite(out).all()
+    # the scores' error, 2e-3 of the largest value scale, and the output's rounding
+    assert (np.abs(out - want) <= 1e-2 * np.abs(want) + 2e-3 * 3000.0).all()
