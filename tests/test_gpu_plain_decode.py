@@ -79,3 +79,36 @@ def test_row_formats(case):
     assert outs[0].tobytes() == outs[1].tobytes()
     want = oracle.paged_attention(pool, hb, q, dtype, q_heads)
     G.assert_close(outs[0], dtype, want, what="plain rows", scale=G.channel_scale(v, dtype, hb, q_heads), plain_excess=0.0 if fmt in (FMT_FP16, FMT_BF16) else 4e-4)
+
+
+# Several requests of one tile each, on the chunk grid (test_launch_choices.py holds that these forms are): format, type, page size, kv heads, q heads, keys
+# and new tokens per request, bound on the keys (0: exact)
+ON_GRID = [
+    (FMT_TQ4, DT_F16, 32, 2, 16, [700, 9, 2500, 64], [1, 0, 1, 1], 8000),
+    (FMT_TQ4, DT_BF16, 16, 2, 16, [700, 9, 2500, 64], [1, 1, 0, 1], 0),
+    (FMT_TQ4, DT_F16, 64, 2, 4, [257, 5000, 31], [3, 4, 2], 10700),
+    (FMT_Q8_0, DT_F16, 16, 2, 16, [700, 9, 2500, 64], [1, 0, 1, 1], 8000),
+    (FMT_Q8_0, DT_BF16, 64, 1, 8, [300, 3000, 1, 2999], [0, 2, 1, 2], 0),
+    (FMT_FP8, DT_F16, 48, 4, 4, [700, 9, 2500, 64], [1, 0, 5, 16], 8192),
+    (FMT_FP8, DT_BF16, 16, 2, 16, [1200, 1201], [1, 1], 0),
+]
+
+
+@pytest.mark.parametrize("case", range(len(ON_GRID)))
+def test_several_requests(case):
+    import gpu_harness as G
+
+    fmt, dtype, block, kv_heads, q_heads, seqs, q_lens, bound = ON_GRID[case]
+    pool, bt, k, v, q, aq, ctx = make_case(fmt, block, seqs, q_lens, 3300 + case, dtype, kv_heads=kv_heads, q_heads=q_heads)
+    hb = oracle.HostBatch(aq, seqs, bt, context_lens_before=ctx)
+    dpool = G.DevPool(pool)
+    dpool.upload()
+    outs = []
+    for batch in (hb, oracle.HostBatch(aq, seqs, bt)):
+        rc, got, _ = G.dev_attention(dpool, batch, q, dtype, q_heads, scratch_bytes=64 << 20, max_seq_len=bound or None)
+        assert rc == 0
+        outs.append(got)
+    assert np.array_equal(outs[0], outs[1])
+    want = oracle.paged_attention(pool, hb, q, dtype, q_heads)
+    G.assert_close(outs[0], dtype, want, what="plain decode of several requests", scale=G.channel_scale(v, dtype, hb, q_heads),
+                   plain_excess=0.0 if fmt == FMT_TQ4 else 4e-4)

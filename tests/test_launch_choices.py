@@ -149,3 +149,17 @@ def test_shorter_chunks_take_no_second_round(recorder):
         n, whole, tiles = run[0][2][0], (c["max_seq"] // 32 + 1 + 7) // 8, (c["q_len"] * 8 + 15) // 16
         assert n * tiles * c["kv_heads"] <= max(256, min(whole, 128 // tiles) * tiles * c["kv_heads"]), c
         assert chunks.setdefault((c["fmt"], c["q_len"], c["max_seq"]), n) == n, c
+
+
+def test_batches_of_the_plain_kernels(recorder):
+    """The batches of several requests whose bytes are compared with the general kernels' run in the plain ones."""
+    from oracle import FMT_FP8, FMT_Q8_0
+    from test_gpu_plain_decode import ON_GRID
+
+    names = {FMT_Q8_0: "q8_0", FMT_FP8: "fp8"}
+    cases = [case(names.get(fmt, "tq4"), len(seqs), max(q_lens), bound or max(seqs), q_heads, kv_heads)
+             for fmt, _, _, kv_heads, q_heads, seqs, q_lens, bound in ON_GRID]
+    for c, (_, (run,)) in zip(cases, recorder(cases)):
+        assert ("paged_attn_tq4_plain_kernel" if c["fmt"] == "tq4" else "paged_attn_rows_plain_kernel") in run[0][0], (c, run[0][0])
+        if c["fmt"] != "tq4":  # one tile per request
+            assert re.search(r"plain_kernelI.*Lb1E", run[0][0]), run[0][0]
