@@ -108,6 +108,23 @@ def test_leading_arguments_are_preloaded(tmp_path, part, dwords):
     assert {k: v for k, v in kernels.items() if v < dwords} == {}
 
 
+@pytest.mark.skipif(not os.path.exists(READELF), reason="no llvm-readelf")
+@pytest.mark.parametrize("part,dwords", [("balanced_merge_kernel", 12), ("split_merge_few_kernel", 11), ("split_merge_kernel", 11)])
+def test_merges_have_all_of_their_leading_arguments(tmp_path, part, dwords):
+    """The requests' token ranges and the gate among them, which are asked for together with the slices."""
+    kernels = {k: v for k, v in kernel_preload_dwords(tmp_path).items() if re.search(r"w34\d+" + part + "I", k)}
+    assert len(kernels) >= 8, sorted(kernels)
+    assert {k: v for k, v in kernels.items() if v < dwords} == {}
+
+
+@pytest.mark.skipif(not os.path.exists(READELF), reason="no llvm-readelf")
+def test_tq4_decode_kernels_do_not_spill(tmp_path):
+    """Two column tiles hold 128 accumulators per lane; their stores must not turn into an address inside the array either."""
+    kernels = {k: v for k, v in kernel_scratch_bytes(tmp_path).items() if "paged_attn_tq4" in k}
+    assert len(kernels) == 10, sorted(kernels)
+    assert {k: v for k, v in kernels.items() if v} == {}
+
+
 def assembly(tmp_path, source):
     path = os.path.join(str(tmp_path), "probe.hip")
     with open(path, "w") as f:
