@@ -504,7 +504,7 @@ __global__ __launch_bounds__(12 * 64, 1) void paged_prefill_tq4_kernel(const Att
         if (raise) {
             const float m = max_over_rows(mx);
             const bool empty = !(sum_over_rows(l_run) > 0.f), any = m > 0.5f * kNegBig;
-            if (!started) started = __ballot(col_ok && empty && !any) == 0ull;
+            started = started || (!MASKED && __ballot(!any) == 0ull);  // (a unit that every live column sees)
             const float up = empty ? (any ? m : 0.f) : m > slack ? m : 0.f;
             const float alpha = empty ? 1.f : __builtin_amdgcn_exp2f(-up);
             m_run += up;
