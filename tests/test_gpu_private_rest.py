@@ -45,16 +45,40 @@ def test_private_rest_matches_oracle(name):
     assert (got.tobytes() == plain.tobytes()) == (shared == 0)
 
 
-def _small(block, q_lens, ctx, shared, seed, q_heads=16):
-    """A batch whose requests have their first `shared` keys in common, on a pool of the host."""
-    pool, bt, k, v, q, aq, before = make_case(FMT_TQ4, block, ctx, q_lens, seed, DT_BF16, q_heads=q_heads)
-    bt[1:, :shared // block] = bt[0, :shared // block]
-    hb = oracle.HostBatch(aq, ctx, bt, context_lens_before=before)
+LONG = 40000         # a bound from which on the shared keys get a pass of their own
+WIDE_UNITS = 6144    # units behind the prefix from which on both column tiles go to one workgroup
+
+
+def _long(block, q_lens, ctx, shared, seed, q_heads=16):
+    """Long requests over few pages: their last two and the first behind the shared ones are their own, the others any.  -> pool, batch, queries, scale, units behind the prefix (once per
+    column tile pair)"""
+    keys = 8192 // block * block
+    pool, pages, _, v, _, _, _ = make_case(FMT_TQ4, block, [keys], [1], seed, DT_BF16, q_heads=q_heads)
+    pages, rng = pages[0], np.random.default_rng(seed)
+    own, common = pages[:3 * len(ctx)].reshape(3, -1), pages[3 * len(ctx):]
+    bt = rng.choice(common, (len(ctx), max(ctx) // block + 1)).astype(np.int32)
+    bt[:, :shared // block] = bt[0, :shared // block]
+    bt[:, shared // block] = own[0]  # (the shared keys end here)
+    for r, n in enumerate(ctx):
+        last = (n - 1) // block
+        bt[r, last - 1:last + 1] = own[1:, r]
+    starts = np.concatenate([[0], np.cumsum(q_lens)]).astype(np.int32)
+    q = oracle.fill_normal(int(starts[-1]) * q_heads * 256, seed + 2, DT_BF16).reshape(-1, q_heads, 256)
+    hb = oracle.HostBatch(starts, ctx, bt, context_lens_before=[n - t for n, t in zip(ctx, q_lens)])
     v_absmax = np.abs(oracle.bits_to_f32(v, DT_BF16)).max(axis=0)
-    return pool, hb, q, np.repeat(np.maximum(1.0, v_absmax), q_heads // 2, axis=0)[None]
+    tok_tile, floor = 64 // q_heads, shared // block * block // 32
+    units = sum(-(-t // tok_tile) * ((n - 1) // 32 - floor + 1) for n, t in zip(ctx, q_lens) if t)
+    return pool, hb, q, np.repeat(np.maximum(1.0, v_absmax), q_heads // 2, axis=0)[None], units
 
 
-LONG = 40000  # a bound from which on the shared keys get a pass of their own
+def _attend(pool, hb, q, **bounds):
+    import gpu_harness as G
+
+    dpool = G.DevPool(pool)
+    dpool.upload()
+    rc, got, _ = G.dev_attention(dpool, hb, q, DT_BF16, q.shape[1], scratch_bytes=96 << 20, **bounds)
+    assert rc == 0
+    return got
 
 
 @pytest.mark.parametrize("bits", [0x7C00, 0xFFFF])     # an infinite and a NaN scale
@@ -62,9 +86,8 @@ LONG = 40000  # a bound from which on the shared keys get a pass of their own
 @pytest.mark.parametrize("token", [3, 2])              # both in the second column tile of a request, the first one has tokens 0 and 1
 def test_scales_of_unseen_rows(token, both_slabs, bits):
     """The scales of a token's rows are not finite: the tokens in front of it, which do not see them, keep their bits."""
-    import gpu_harness as G
-
-    pool, hb, q, _ = _small(64, (4, 4, 4, 4), (4133, 4196, 4165, 4612), 4096, 1401)
+    pool, hb, q, _, units = _long(64, (4,) * 8, [29000 + 37 * r for r in range(8)], 4096, 1401)
+    assert units >= WIDE_UNITS
     outs = []
     for poisoned in (False, True):
         if poisoned:
@@ -73,44 +96,39 @@ def test_scales_of_unseen_rows(token, both_slabs, bits):
                 assert np.shares_memory(rows, slab)
                 for r, pos in enumerate(hb.ctx + token):
                     rows[hb.bt[r, pos // 64], :, pos % 64][:, [0, 33]] = bits
-        dpool = G.DevPool(pool)
-        dpool.upload()
-        rc, got, _ = G.dev_attention(dpool, hb, q, DT_BF16, 16, scratch_bytes=96 << 20, max_seq_len=LONG)
-        assert rc == 0
-        got = got.reshape(4, 4, 16, 256)
+        got = _attend(pool, hb, q, max_seq_len=LONG).reshape(8, 4, 16, 256)
         assert both_slabs or np.isnan(oracle.bits_to_f32(got[:, token:], DT_BF16)).all() == poisoned
         outs.append(got[:, :token])
     assert np.isfinite(oracle.bits_to_f32(outs[0], DT_BF16)).all()
     assert np.array_equal(outs[0], outs[1])
 
 
-@pytest.mark.parametrize("q_lens,bounds", [((2,) * 8, (2, 3, 4, 16)), ((3, 1, 2, 2, 1, 3, 2, 2), (3, 4, 8)), ((4, 2, 4, 4, 4), (4, 5, 16))])
-def test_bytes_do_not_depend_on_the_token_bound(q_lens, bounds):
+@pytest.mark.parametrize("wide", [False, True])
+@pytest.mark.parametrize("q_lens,bounds", [((2,) * 8, (2, 3, 4, 16)), ((3, 1, 2, 2, 1, 3, 2, 2), (3, 4, 8)), ((4, 2, 4, 4, 4), (4, 5, 16)),
+                                           ((4, 4, 4, 0, 4), (4, 5))])
+def test_bytes_do_not_depend_on_the_bounds(q_lens, bounds, wide):
+    """A short rest and one of just as many units as two column tiles want."""
     import gpu_harness as G
 
-    pool, hb, q, scale = _small(64, q_lens, [4200 + 97 * r for r in range(len(q_lens))], 4096, 1501)
-    dpool = G.DevPool(pool)
-    dpool.upload()
-    outs = []
-    for bound in bounds:
-        rc, got, _ = G.dev_attention(dpool, hb, q, DT_BF16, 16, scratch_bytes=96 << 20, max_seq_len=LONG, max_q_len=bound)
-        assert rc == 0
-        outs.append(got)
+    tiles = sum(t > 0 for t in q_lens)
+    units = (WIDE_UNITS + tiles - 1) // tiles if wide else 30
+    pool, hb, q, scale, units = _long(64, q_lens, [4096 + 32 * units - r % 3 for r in range(len(q_lens))], 4096, 1501)
+    assert (units >= WIDE_UNITS) == wide
+    outs = [_attend(pool, hb, q, max_q_len=tokens, max_seq_len=keys) for tokens in bounds for keys in (LONG + 20000, 200000)]
     want = oracle.paged_attention(pool, hb, q, DT_BF16, 16, n_threads=oracle.hw_threads())
     G.assert_close(outs[0], DT_BF16, want, what="bound %d" % bounds[0], scale=scale)
     assert all(np.array_equal(got, outs[0]) for got in outs)
 
 
-# pages of 16 keys (two per unit) and of 48 (units across their edges), the last of a request with one key and more; the shared keys end inside a page of 48
-@pytest.mark.parametrize("block,shared,ctx", [(16, 4096, (4113, 4129, 4100, 4611)), (48, 4176, (4225, 4181, 4300, 4801))])
-@pytest.mark.parametrize("q_lens", [(4, 4, 4, 4), (4, 0, 5, 7)])
-def test_other_page_sizes(block, shared, ctx, q_lens):
+# pages of 16 keys (two per unit), of 48 (units across their edges) and of 64; the shared keys end inside a page of 48
+@pytest.mark.parametrize("block,shared", [(16, 4096), (48, 4176), (64, 4096)])
+@pytest.mark.parametrize("q_heads,q_lens,ctx", [(16, (4, 0, 5, 7, 8), (33000, 35001, 34015, 36001, 32912)), (32, (3, 5, 4, 5), (26017, 25002, 26000, 26001)),
+                                                (8, (9, 16, 7, 12), (34001, 33000, 37007, 35555))])
+def test_two_column_tiles(block, shared, q_heads, q_lens, ctx):
     import gpu_harness as G
 
-    pool, hb, q, scale = _small(block, q_lens, ctx, shared, 1601)
-    dpool = G.DevPool(pool)
-    dpool.upload()
-    rc, got, _ = G.dev_attention(dpool, hb, q, DT_BF16, 16, scratch_bytes=96 << 20, max_seq_len=LONG)
-    assert rc == 0
-    want = oracle.paged_attention(pool, hb, q, DT_BF16, 16, n_threads=oracle.hw_threads())
+    pool, hb, q, scale, units = _long(block, q_lens, ctx, shared, 1601, q_heads)
+    assert units >= WIDE_UNITS
+    got = _attend(pool, hb, q, max_seq_len=LONG)
+    want = oracle.paged_attention(pool, hb, q, DT_BF16, q_heads, n_threads=oracle.hw_threads())
     G.assert_close(got, DT_BF16, want, what="pages of %d" % block, scale=scale)

@@ -47,8 +47,8 @@ FORMS = {
     "decode": ((1,), (1300,), 0, 0, 0),
     "four tokens": ((4,), (1300,), 0, 0, 0),
     "balanced": ((1, 1, 1, 1), (16384, 9000, 12000, 300), 0, 0, 64 << 20),
-    # two column tiles, whose eight chunks are of two units a wave
-    "private rest": ((4,) * 16, (8192,) * 16, 4096, 40000, 96 << 20),
+    # two column tiles, whose eight chunks are of six units a wave
+    "private rest": ((4,) * 16, (16384,) * 16, 4096, 40000, 96 << 20),
 }
 
 
@@ -71,7 +71,7 @@ def test_units_without_weight_before_low_scores(form):
     q_lens, seqs, shared, _, _ = FORMS[form]
     outs = []
     for none in (-2000.0, -np.inf):
-        score = lambda pos: np.where((pos >= shared) & ((pos - shared) // 256 % 2 == 0) & (pos < shared + 4096), none, -300.0 - 0.1 * (pos % 7))
+        score = lambda pos: np.where((pos >= shared) & ((pos - shared) % 1536 < 256), none, -300.0 - 0.1 * (pos % 7))
         pool, hb, q = _pool(64, seqs, q_lens, score, shared)
         outs.append(_attend(pool, hb, q, form))
         if none > -np.inf:

@@ -791,8 +791,8 @@ __device__ __forceinline__ void store_packed_column(float* c, const f4 (&o)[2][8
 // LDS: [pair table 64 KB][kTq4Waves staging areas of 8448 B][query operand table 9216 B][(m, l) tables].
 // A staging area holds one 32-token unit as it lies in the pages, written by LDS-direct loads:
 // K rows 0-31, then V rows 0-31, 132 bytes each (four runs of 16 rows = 2112 bytes).
-// SP: the keys below *P.key_floor belong to a shared-prefix pass (see AttnParams); a separate
-// instantiation, so that the plain form carries no trace of it.
+// SP: the keys below `item.u_begin` belong to a shared-prefix pass (*P.key_floor, see AttnParams), tile and chunk are `item.req` and `item.slot`; a
+// separate instantiation, so that the plain form carries no trace of it.
 // NT: column tiles of 16 (two: batches with neither a token mask nor a window).
 // PLAIN: split-K form of a batch whose requests have one tile of at most eight columns each, all q heads of a kv head in it, without masks and window, page
 // strides below 4 GiB (plain_decode): what follows from the host's bounds on it is worked out while the lengths travel.
@@ -982,7 +982,7 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
     const bool simple = PLAIN || NT > 1 || (B.valid_token_mask == nullptr && B.sliding_window <= 0);
     // keys below the floor were handled by the shared-prefix pass (a multiple of the unit size)
     int key_floor = 0;
-    if constexpr (SP) key_floor = __builtin_amdgcn_readfirstlane(*P.key_floor);
+    if constexpr (SP) key_floor = item.u_begin;
     auto column_info = [&](bool accumulate) {
         if constexpr (NT > 1) {
             auto last = [&](int col, bool& ok) {
@@ -1839,7 +1839,7 @@ __global__ __launch_bounds__(kTq4Waves * 64, 1) void paged_attn_tq4_kernel(const
     // decode steps (no request has more than one tile): every key is read by one workgroup only,
     // the loads carry the streaming hint; one body per kind of load
     BalItem item{};
-    if constexpr (SP) item.req = (int)blockIdx.z, item.slot = (int)blockIdx.x;
+    if constexpr (SP) item.req = (int)blockIdx.z, item.slot = (int)blockIdx.x, item.u_begin = __builtin_amdgcn_readfirstlane(*P.key_floor);
     if (!SP && P.tiles_by_request != 0 && P.q_subgroups == 1) {  // uniform for the grid
         tq4_tile<TQ, false, SP, true>(P, smem, item, true);
     } else {
@@ -1857,18 +1857,30 @@ __global__ __launch_bounds__(kTq4Waves * 64, 1) void paged_attn_tq4_plain_kernel
     tq4_tile<TQ, false, false, true, 1, true>(P, smem, BalItem{}, true);
 }
 
+// What the probe of a shared prefix leaves for the kernels behind it.
+struct SpHeader {
+    int32_t floor;   // keys [0, floor) are the shared prefix
+    int32_t qsl[2];  // query_start_loc of the pseudo request: {0, total_tokens}
+    int32_t seq;     // its seq_lens_after (= floor)
+    int32_t ctx;     // its context_lens_before (= floor: every key visible to every token)
+    int32_t wide;    // the private rest is for two column tiles, see kWidePrivateUnits
+    int32_t pad[2];
+};
+
 // The private rest of a verify batch with more than 16 query columns per request and kv head: both column tiles in one workgroup, so that
 // a key is looked up once for 32 columns (a wave's unit: 465 vector instructions and 100 MFMAs, one tile 330 and 50).  Issue bounds it, so the loads keep their
 // plain form: with the streaming hint 3 % slower.  `wide` holds the geometry of that form, whose chunks join the prefix's records, for which there is room
-// whatever their number; with nothing shared, `P`, that of the plain path, whose bits the batch then has.  us, 16 requests x 4 tokens on 262 144 keys, 200 000 of
+// whatever their number; `P` that of the plain path, for a short rest (kWidePrivateUnits) and with nothing shared, where the batch has the plain path's bits.  us, 16 requests x 4 tokens on 262 144 keys, 200 000 of
 // them shared, one column tile / two: whole call 524 / 486, on another box 534 / 512; this kernel 177 / 147.
 template <typename TQ>
-__global__ __launch_bounds__(kTq4Waves * 64, 1) void paged_attn_tq4_private_kernel(const AttnParams P, const AttnParams wide, int chunks, int tiles,
-                                                                                   int wide_chunks, int wide_tiles) {
+__global__ __launch_bounds__(kTq4Waves * 64, 1) void paged_attn_tq4_private_kernel(const AttnParams P, const AttnParams wide, const SpHeader* hdr,
+                                                                                   int chunks, int tiles, int wide_chunks, int wide_tiles) {
     extern __shared__ __align__(16) uint8_t smem[];
     const int wg = (int)blockIdx.x;
     BalItem item{};
-    if (__builtin_amdgcn_readfirstlane(*P.key_floor) != 0) {
+    const int floor = hdr->floor, wide_rest = hdr->wide;
+    item.u_begin = __builtin_amdgcn_readfirstlane(floor);
+    if (__builtin_amdgcn_readfirstlane(wide_rest) != 0) {
         item.req = wg / wide_chunks;
         item.slot = wg - item.req * wide_chunks;
         if (item.req < wide_tiles) tq4_tile<TQ, false, true, false, 2>(wide, smem, item, true);
@@ -2711,29 +2723,34 @@ static void fill_spec_geometry(AttnParams& P, int max_seq_len) {
 // the pages that every request's block table holds at the same index and that lie below every
 // request's first query position (every query of the batch sees all of their keys).  It leaves
 // the length in tokens (a multiple of the unit; 0 below kSpMinTokens) and the descriptor of one
-// pseudo request -- all query tokens of the batch over exactly those keys -- in the header.
-struct SpHeader {
-    int32_t floor;   // keys [0, floor) are the shared prefix
-    int32_t qsl[2];  // query_start_loc of the pseudo request: {0, total_tokens}
-    int32_t seq;     // its seq_lens_after (= floor)
-    int32_t ctx;     // its context_lens_before (= floor: every key visible to every token)
-    int32_t pad[3];
-};
+// pseudo request -- all query tokens of the batch over exactly those keys -- in the header (SpHeader).
 constexpr int kSpMinTokens = 4096;
+// Units behind the prefix, counted once per column tile pair, from which on the private rest is for two column tiles.  A key is looked up once for both, but
+// the four columns of a wave are added up and joined to the records one after the other: about 6 us a call, which a short rest does not earn back.
+// Counted on the device from the lengths themselves, and not by the kv heads that a rank holds, so that results depend on neither the bounds nor
+// the sharding.  us a call, two kv heads of 8 query heads, one tile / two: 4 tokens each, 16 requests with 2 976 units in all 116.3 / 122.9, 8 with
+// 5 008 108.7 / 111.9, 4 with 7 680 84.1 / 81.8, 16 with 9 984 128.7 / 122.5; 8 requests of 8 tokens with 2 752 149.1 / 149.1, with 7 744 158.7 / 153.1.
+// What other numbers of kv heads give up for that: one, 8 x 4 tokens with 5 008 103.9 / 99.4; four, 6 x 4 with 1 872 118.8 / 126.9, 12 x 4 with 3 744 201.8 / 197.0.
+constexpr int kWidePrivateUnits = 6144;
 
-__global__ __launch_bounds__(1024) void shared_prefix_probe_kernel(const warp34_attention_batch B, int block_size,
+// wide_tok_tile: tokens of two column tiles
+__global__ __launch_bounds__(1024) void shared_prefix_probe_kernel(const warp34_attention_batch B, int block_size, int wide_tok_tile,
                                                                    SpHeader* hdr) {
-    __shared__ int s_first_diff, s_min_ctx;
+    __shared__ int s_first_diff, s_min_ctx, s_private;
     const int tid = (int)threadIdx.x;
     if (tid == 0) {
         s_first_diff = B.max_blocks_per_req;
         s_min_ctx = 0x7fffffff;
+        s_private = 0;
     }
     __syncthreads();
+    const auto tokens_of = [&](int r) { return B.query_start_loc[r + 1] - B.query_start_loc[r]; };
+    const auto context_of = [&](int r, int q_len) { return B.context_lens_before != nullptr ? B.context_lens_before[r] : B.seq_lens_after[r] - q_len; };
+    int my_q = 0, my_ctx = 0;  // of request tid
     for (int r = tid; r < B.num_reqs; r += 1024) {
-        const int q_len = B.query_start_loc[r + 1] - B.query_start_loc[r];
-        const int ctx = B.context_lens_before != nullptr ? B.context_lens_before[r] : B.seq_lens_after[r] - q_len;
+        const int q_len = tokens_of(r), ctx = context_of(r, q_len);
         atomicMin(&s_min_ctx, ctx < 0 ? 0 : ctx);
+        if (r == tid) my_q = q_len, my_ctx = ctx;
     }
     __syncthreads();
     int max_pages = s_min_ctx / block_size;  // pages that lie entirely below every first query position
@@ -2762,10 +2779,20 @@ __global__ __launch_bounds__(1024) void shared_prefix_probe_kernel(const warp34_
     }
     if (first_diff != 0x7fffffff) atomicMin(&s_first_diff, first_diff);
     __syncthreads();
+    const int pages = s_first_diff < max_pages ? s_first_diff : max_pages;
+    int floor = (pages * block_size) & ~(kUnit - 1);
+    if (floor < kSpMinTokens) floor = 0;
+    // units behind the prefix, one column tile pair's by one
+    int units = 0;
+    for (int r = tid; r < B.num_reqs; r += 1024) {
+        const int q_len = r == tid ? my_q : tokens_of(r), ctx = r == tid ? my_ctx : context_of(r, q_len);
+        const long long mine = (long long)((q_len + wide_tok_tile - 1) / wide_tok_tile) * (((ctx + q_len - 1) >> 5) - (floor >> 5) + 1);
+        units = (int)min((long long)kWidePrivateUnits, units + (q_len > 0 && mine > 0 ? mine : 0ll));
+    }
+    if (units > 0) atomicAdd(&s_private, units);
+    __syncthreads();
     if (tid == 0) {
-        const int pages = s_first_diff < max_pages ? s_first_diff : max_pages;
-        int floor = (pages * block_size) & ~(kUnit - 1);
-        if (floor < kSpMinTokens) floor = 0;
+        hdr->wide = floor != 0 && s_private >= kWidePrivateUnits ? 1 : 0;
         hdr->floor = floor;
         hdr->qsl[0] = 0;
         hdr->qsl[1] = B.total_tokens;
@@ -2892,7 +2919,7 @@ static int launch_tq4(const warp34_exec* ex, const warp34_kv_layer_layout* layou
             P.part_ml = P.part_acc + (size_t)rows * stride * kHeadDim;
             SpHeader* hdr = reinterpret_cast<SpHeader*>(P.part_ml + (size_t)rows * stride * 4);
             P.key_floor = &hdr->floor;
-            hipLaunchKernelGGL(shared_prefix_probe_kernel, dim3(1), dim3(1024), 0, stream, *batch, layout->block_size, hdr);
+            hipLaunchKernelGGL(shared_prefix_probe_kernel, dim3(1), dim3(1024), 0, stream, *batch, layout->block_size, 32 / q_group, hdr);
             rc = (int)hipGetLastError();
             if (rc) return rc;
             AttnParams T = P;  // the pseudo request of the header, 128-row tiles
@@ -2925,7 +2952,7 @@ static int launch_tq4(const warp34_exec* ex, const warp34_kv_layer_layout* layou
                 if (rc) return rc;
                 const long long wgs = std::max((long long)grid_x * grid_z, (long long)W.max_chunks * tiles);
                 hipLaunchKernelGGL(paged_attn_tq4_private_kernel<TQ>, dim3((unsigned)wgs, (unsigned)kv_subs), dim3(kTq4Waves * 64),
-                                   smem_bytes_for(2), stream, P, W, grid_x, grid_z, W.max_chunks, tiles);
+                                   smem_bytes_for(2), stream, P, W, (const SpHeader*)hdr, grid_x, grid_z, W.max_chunks, tiles);
             } else {
                 rc = ensure_dynamic_lds(paged_attn_tq4_kernel<TQ, true>, smem_bytes_for(1), true);
                 if (rc) return rc;
