@@ -21,7 +21,10 @@
  *     do not touch it;
  *   - every index array in warp34_attention_batch is a DEVICE pointer; the scalar
  *     fields max_q_len / max_seq_len / max_blocks_per_req are host-known upper bounds
- *     used only for launch geometry -- results do not depend on them;
+ *     used only for launch geometry.  They can choose between forms of the attention
+ *     kernels that add the same products in another order (a bound that lets a request
+ *     have several tiles of query tokens, the pass for shared prefixes), and change
+ *     nothing else in the results;
  *   - masked tokens / requests (valid_token_mask[tok]==0, valid_req_mask[req]==0,
  *     write slot < 0) write nothing and leave the output row untouched.
  */

@@ -53,9 +53,9 @@ typedef float f2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u2v __attribute__((ext_vector_type(2)));
 
-// waves per workgroup of the TQ4 decode kernel: eight, two per SIMD (up to 256 registers each); the
-// LDS holds the table, eight staging areas, the query operand table and the (m, l) tables:
-// 142 KB of 160 KB, one workgroup per CU
+// waves per workgroup of the TQ4 decode kernels: eight, two per SIMD (up to 256 registers each); the
+// LDS holds the table, eight staging areas, the query operand tables and the (m, l) tables, of 160 KB
+// 140 (one column tile) or 150 (two): one workgroup per CU
 constexpr int kTq4Waves = 8;
 constexpr int kUnit = 32;             // tokens per wave iteration
 constexpr int kLutBytes = 256 * 256;  // 256 entries x 64 lane replicas x 4 B
@@ -853,9 +853,8 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
             if (slot < B.max_blocks_per_req)
                 spec_vec = B.block_tables[(size_t)req * B.max_blocks_per_req + slot];
         }
-        // one vector load per array (all lanes the same address), no scalar-cache round trip;
-        // the values are made scalar after the table has been built, so that the build overlaps
-        // the round trip
+        // By requests: the same address in all lanes, so scalar loads, one per array and all on their way together with the block-table slice (in the
+        // row formats vector loads took 2 to 4 % longer).  By tiles: one request per lane.
         if constexpr (PLAIN) {
             a_lo = B.query_start_loc[req];
             a_hi = B.query_start_loc[req + 1];
@@ -1298,7 +1297,6 @@ __device__ __forceinline__ void tq4_tile(const AttnParams& P, uint8_t* smem, con
     const uint8_t* ka_lo = stage + unit_token(0, n >> 2, n & 3) * kTq4RowBytes;  // A row of sub-tile 0; sub-tile 1: + 8 rows
     const uint8_t* kt_lo = stage + unit_token(0, b, 0) * kTq4RowBytes;           // token of output row 4b; + 8 s + i rows
     const uint8_t* vt_lo = kt_lo + 2 * kRunBytes;
-    const uint32_t vt_lo_addr = stage_addr + (uint32_t)(2 * kRunBytes + unit_token(0, b, 0) * kTq4RowBytes);  // its LDS address
     const uint8_t* kt_n = kt_lo + (n & 3) * kTq4RowBytes;  // the token whose K scales this lane fetches (+ 8 s rows)
     const uint8_t* vt_n = vt_lo + (8 * ((n >> 2) & 1) + (n & 3)) * kTq4RowBytes;  // ... and V scales: token n & 7
 
@@ -1849,8 +1847,8 @@ __global__ __launch_bounds__(kTq4Waves * 64, 1) void paged_attn_tq4_kernel(const
 
 // Decode steps without masks, see plain_decode; the bits of the general kernel.  What bounds a short one is the chain lengths - addresses - first rows: device
 // timestamps, one token on 1 200 keys, from the wave's entry: lengths there 1.16 us, addresses 1.72, first rows asked for 2.17 in the general kernel, most of it
-// scalar instructions, which eight waves issue one after the other.  us, general / this: one token on 1 200 keys, eight layers with their producers, 124.2 / 114.5, one on
-// 131 072, four layers, 99.6 / 95.3.
+// scalar instructions, which eight waves issue one after the other.  us, general / this: one token on 1 200 keys, eight layers with their producers, 116.1 / 110.9, one on
+// 131 072, four layers, 101.9 / 98.4.
 template <typename TQ>
 __global__ __launch_bounds__(kTq4Waves * 64, 1) void paged_attn_tq4_plain_kernel(const AttnParams P) {
     extern __shared__ __align__(16) uint8_t smem[];
@@ -1868,7 +1866,7 @@ struct SpHeader {
 };
 
 // The private rest of a verify batch with more than 16 query columns per request and kv head: both column tiles in one workgroup, so that
-// a key is looked up once for 32 columns (a wave's unit: 465 vector instructions and 100 MFMAs, one tile 330 and 50).  Issue bounds it, so the loads keep their
+// a key is looked up once for 32 columns (a wave's unit: 465 vector instructions and 96 MFMAs, one tile 330 and 48).  Issue bounds it, so the loads keep their
 // plain form: with the streaming hint 3 % slower.  `wide` holds the geometry of that form, whose chunks join the prefix's records, for which there is room
 // whatever their number; `P` that of the plain path, for a short rest (kWidePrivateUnits) and with nothing shared, where the batch has the plain path's bits.  us, 16 requests x 4 tokens on 262 144 keys, 200 000 of
 // them shared, one column tile / two: whole call 524 / 486, on another box 534 / 512; this kernel 177 / 147.
