@@ -1,6 +1,6 @@
-"""The private rest of a verify batch behind a shared prefix, more than 16 query columns per request and kv head: two column tiles
-of a workgroup, whose sums join the records of the prefix's parts (no counterpart in the reference, which runs such a batch
-without any split, op_paged_attn.cu:1399-1415)."""
+"""The private rest of a verify batch behind a shared prefix, more than 16 query columns per request and kv head: one column tile per
+workgroup where it is short, else two, whose sums join the records of the prefix's parts (no counterpart in the reference, which
+runs such a batch without any split, op_paged_attn.cu:1399-1415)."""
 import numpy as np
 import pytest
 
@@ -71,12 +71,13 @@ def _long(block, q_lens, ctx, shared, seed, q_heads=16):
     return pool, hb, q, np.repeat(np.maximum(1.0, v_absmax), q_heads // 2, axis=0)[None], units
 
 
-def _attend(pool, hb, q, **bounds):
+def _attend(pool, hb, q, dpool=None, **over):
     import gpu_harness as G
 
-    dpool = G.DevPool(pool)
-    dpool.upload()
-    rc, got, _ = G.dev_attention(dpool, hb, q, DT_BF16, q.shape[1], scratch_bytes=96 << 20, **bounds)
+    if dpool is None:
+        dpool = G.DevPool(pool)
+        dpool.upload()
+    rc, got, _ = G.dev_attention(dpool, hb, q, DT_BF16, q.shape[1], scratch_bytes=96 << 20, **over)
     assert rc == 0
     return got
 
@@ -132,3 +133,21 @@ def test_two_column_tiles(block, shared, q_heads, q_lens, ctx):
     got = _attend(pool, hb, q, max_seq_len=LONG)
     want = oracle.paged_attention(pool, hb, q, DT_BF16, q_heads, n_threads=oracle.hw_threads())
     G.assert_close(got, DT_BF16, want, what="pages of %d" % block, scale=scale)
+
+
+def test_one_kv_head_gives_the_same_bytes():
+    """Whether the rest is for two column tiles does not depend on the kv heads that a rank holds."""
+    from test_gpu_head_sharding import _head_layout
+
+    import gpu_harness as G
+
+    for ctx in ((34017, 35001, 34000, 36001, 33912), (15017, 14001, 13015, 16001, 14912)):
+        pool, hb, q, _, units = _long(64, (4, 5, 4, 7, 8), ctx, 4096, 1701)
+        assert (units >= WIDE_UNITS) == (ctx[0] > 20000)
+        full = _attend(pool, hb, q, max_seq_len=LONG)
+        dpool = G.DevPool(pool)
+        dpool.upload()
+        for head in range(2):
+            q_h = np.ascontiguousarray(q[:, head * 8:(head + 1) * 8])
+            part = _attend(pool, hb, q_h, max_seq_len=LONG, dpool=dpool, layout=_head_layout(dpool, head))
+            assert np.array_equal(part, full[:, head * 8:(head + 1) * 8])
